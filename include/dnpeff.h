@@ -61,6 +61,13 @@ void* dnpeff_stream(void);
  * (cc/cuda_d_npeff/src/cuda/debugging/). */
 int dnpeff_device_memory(int64_t* free_bytes, int64_t* total_bytes);
 
+/* Gives back what the library keeps between calls: freed device blocks (at most 1 GiB of them, none
+ * larger than 256 MB, reused by later calls) and the pinned buffers that large copies to and from
+ * pageable memory go through (24 MB).  The blocks also go back when an allocation fails and before
+ * dnpeff_device_memory reports.  The reference allocates and frees per object and keeps nothing
+ * (cc/cuda_d_npeff/src/cuda/cuda_context.h:58-69). */
+int dnpeff_release_cached(void);
+
 /* The byte table behind the memory plan of dnpeff_nmf_create, computable without a GPU (capacity
  * planning, tests): for a matrix of n_rows x n_cols whose sparse part holds nnz_sparse entries
  * and whose dense head holds n_dense columns, at the given rank, with the tiled (1) or full-size

@@ -31,6 +31,7 @@ from .binding import (  # noqa: F401
     device_info,
     device_memory,
     plan_estimate,
+    release_cached,
     tuning_set,
     tuning_get,
     tuning_reset,

@@ -46,6 +46,7 @@ SIGNATURES = {
     "dnpeff_sync": (C.c_int, []),
     "dnpeff_stream": (_p, []),
     "dnpeff_device_memory": (C.c_int, [C.POINTER(_i64), C.POINTER(_i64)]),
+    "dnpeff_release_cached": (C.c_int, []),
     "dnpeff_tuning_set": (C.c_int, [C.c_char_p, _f64]),
     "dnpeff_tuning_get": (C.c_int, [C.c_char_p, C.POINTER(_f64)]),
     "dnpeff_plan_estimate": (C.c_int, [_i64, _i64, _i64, _i64, C.c_int, C.c_int, C.c_int, _i64, C.POINTER(_f64)]),
@@ -187,6 +188,11 @@ def plan_estimate(n_rows, n_cols, nnz_sparse, n_dense, rank, tiled, sweeps=True,
     return dict(zip(PLAN_FIELDS, [float(x) for x in out]))
 
 
+def release_cached():
+    """Gives back the device blocks and pinned buffers that the library keeps between calls."""
+    _check(lib.dnpeff_release_cached())
+
+
 def tuning_set(name: str, value: float):
     _check(lib.dnpeff_tuning_set(name.encode(), float(value)))
 
@@ -272,7 +278,7 @@ class DeviceArray:
         return d
 
     def numpy(self) -> np.ndarray:
-        out = np.zeros(self.shape, dtype=self.dtype)
+        out = np.empty(self.shape, dtype=self.dtype)
         _check(lib.dnpeff_dev_download(_ptr(out), self.ptr, self.nbytes))
         return out
 
@@ -460,14 +466,14 @@ class Csr:
 
     def download(self):
         n, _, z = self._shape3()
-        rowptr = np.zeros(n + 1, dtype=np.int64)
-        colind = np.zeros(z, dtype=np.int32)
-        vals = np.zeros(z, dtype=np.float32)
+        rowptr = np.empty(n + 1, dtype=np.int64)
+        colind = np.empty(z, dtype=np.int32)
+        vals = np.empty(z, dtype=np.float32)
         _check(lib.dnpeff_csr_download(self._h, _ptr(rowptr), _ptr(colind), _ptr(vals)))
         return rowptr, colind, vals
 
     def kept_indices(self):
-        out = np.zeros(self.n_cols, dtype=np.int32)
+        out = np.empty(self.n_cols, dtype=np.int32)
         _check(lib.dnpeff_csr_kept_indices(self._h, _ptr(out)))
         return out
 
@@ -647,13 +653,13 @@ class MuNmf:
 
     def loadWToHostSync(self) -> np.ndarray:
         """W as [n, r] row-major (after the reference's toRowMajor_inPlace)."""
-        W = np.zeros((self.n_rows, self.params.rank), dtype=np.float32)
+        W = np.empty((self.n_rows, self.params.rank), dtype=np.float32)
         _check(lib.dnpeff_nmf_get_W(self._h, _ptr(W)))
         return W
 
     def loadHToHostSync(self) -> np.ndarray:
         """H as [r, m] row-major (after the reference's toRowMajor_inPlace)."""
-        H = np.zeros((self.params.rank, self.n_cols), dtype=np.float32)
+        H = np.empty((self.params.rank, self.n_cols), dtype=np.float32)
         _check(lib.dnpeff_nmf_get_H(self._h, _ptr(H)))
         return H
 
@@ -743,7 +749,7 @@ class Learner:
         return history
 
     def GetOnHost_W(self) -> np.ndarray:
-        W = np.zeros((self.n_examples, self.n_components), dtype=np.float32)
+        W = np.empty((self.n_examples, self.n_components), dtype=np.float32)
         _check(lib.dnpeff_fit_get_W(self._h, _ptr(W)))
         return W
 

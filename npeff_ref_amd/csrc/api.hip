@@ -211,7 +211,7 @@ static int plan_matrix(dnpeff_csr* A, int rank, bool consume, bool* tiled) {
   const dnpeff_csr* S0 = sparse_part(A);
   // memory that the matrix structures may take: what is free now, plus what a consuming create
   // releases, plus what the structures hold already
-  double avail = (double)free_b;
+  double avail = (double)free_b + (double)pool_cached_bytes();
   if (consume && A->colind && A->vals) avail += 8.0 * (double)A->nnz;
   if (A->tail) {
     avail += (A->head.rm ? 8.0 : 4.0) * (double)A->head.n_pad * (double)A->head.n_d_pad;
@@ -367,7 +367,7 @@ DN_API int dnpeff_nmf_set_factors(dnpeff_nmf* nmf, const float* W_nr, const floa
   DN_CHECK(nmf != nullptr, "handle is NULL");
   DN_HIP(hipStreamSynchronize(stream()));
   if (W_nr)
-    DN_HIP(hipMemcpy(nmf->W, W_nr, sizeof(float) * nmf->n * nmf->r, hipMemcpyHostToDevice));
+    DN_HIP(copy_up(nmf->W, W_nr, sizeof(float) * nmf->n * nmf->r));
   if (H_rm) {
     nmf->gh_valid = false;
     nmf->nw_valid = false;
@@ -376,8 +376,11 @@ DN_API int dnpeff_nmf_set_factors(dnpeff_nmf* nmf, const float* W_nr, const floa
     const int64_t step = nmf->tiled ? nmf->tile_cols : nmf->m;
     for (int64_t c0 = 0; c0 < nmf->m; c0 += step) {
       const int64_t len = nmf->m - c0 < step ? nmf->m - c0 : step;
-      DN_HIP(hipMemcpy2D(nmf->S, sizeof(float) * len, H_rm + c0, sizeof(float) * nmf->m,
-                         sizeof(float) * len, (size_t)nmf->r, hipMemcpyHostToDevice));
+      if (len == nmf->m)
+        DN_HIP(copy_up(nmf->S, H_rm, sizeof(float) * len * nmf->r));
+      else
+        DN_HIP(hipMemcpy2D(nmf->S, sizeof(float) * len, H_rm + c0, sizeof(float) * nmf->m,
+                           sizeof(float) * len, (size_t)nmf->r, hipMemcpyHostToDevice));
       DN_TRY(launch_transpose(nmf->r, len, nmf->S, nmf->H + c0 * nmf->r));
       DN_HIP(hipStreamSynchronize(stream()));
     }
@@ -656,7 +659,7 @@ DN_API int dnpeff_nmf_get_W(dnpeff_nmf* nmf, float* W_nr) {
   clear_error();
   DN_CHECK(nmf && W_nr, "NULL argument");
   DN_HIP(hipStreamSynchronize(stream()));
-  DN_HIP(hipMemcpy(W_nr, nmf->W, sizeof(float) * nmf->n * nmf->r, hipMemcpyDeviceToHost));
+  DN_HIP(copy_down(W_nr, nmf->W, sizeof(float) * nmf->n * nmf->r));
   return 0;
 }
 
@@ -670,8 +673,11 @@ DN_API int dnpeff_nmf_get_H(dnpeff_nmf* nmf, float* H_rm) {
     const int64_t len = nmf->m - c0 < step ? nmf->m - c0 : step;
     DN_TRY(launch_transpose(len, nmf->r, nmf->H + c0 * nmf->r, nmf->S));
     DN_HIP(hipStreamSynchronize(stream()));
-    DN_HIP(hipMemcpy2D(H_rm + c0, sizeof(float) * nmf->m, nmf->S, sizeof(float) * len,
-                       sizeof(float) * len, (size_t)nmf->r, hipMemcpyDeviceToHost));
+    if (len == nmf->m)
+      DN_HIP(copy_down(H_rm, nmf->S, sizeof(float) * len * nmf->r));
+    else
+      DN_HIP(hipMemcpy2D(H_rm + c0, sizeof(float) * nmf->m, nmf->S, sizeof(float) * len,
+                         sizeof(float) * len, (size_t)nmf->r, hipMemcpyDeviceToHost));
   }
   return 0;
 }
@@ -768,7 +774,7 @@ DN_API int dnpeff_fit_set_W(dnpeff_fit* f, const float* W_nr) {
   clear_error();
   DN_CHECK(f && W_nr, "NULL argument");
   DN_HIP(hipStreamSynchronize(stream()));
-  DN_HIP(hipMemcpy(f->W, W_nr, sizeof(float) * f->n * f->r, hipMemcpyHostToDevice));
+  DN_HIP(copy_up(f->W, W_nr, sizeof(float) * f->n * f->r));
   f->whh_valid = false;
   return 0;
 }
@@ -818,7 +824,7 @@ DN_API int dnpeff_fit_get_W(dnpeff_fit* f, float* W_nr) {
   clear_error();
   DN_CHECK(f && W_nr, "NULL argument");
   DN_HIP(hipStreamSynchronize(stream()));
-  DN_HIP(hipMemcpy(W_nr, f->W, sizeof(float) * f->n * f->r, hipMemcpyDeviceToHost));
+  DN_HIP(copy_down(W_nr, f->W, sizeof(float) * f->n * f->r));
   return 0;
 }
 
@@ -826,7 +832,7 @@ DN_API int dnpeff_fit_get_products(dnpeff_fit* f, float* AH_nr, float* HH_rr, do
   clear_error();
   DN_CHECK(f != nullptr, "handle is NULL");
   DN_HIP(hipStreamSynchronize(stream()));
-  if (AH_nr) DN_HIP(hipMemcpy(AH_nr, f->AH, sizeof(float) * f->n * f->r, hipMemcpyDeviceToHost));
+  if (AH_nr) DN_HIP(copy_down(AH_nr, f->AH, sizeof(float) * f->n * f->r));
   if (HH_rr)
     DN_HIP(hipMemcpy(HH_rr, f->HH, sizeof(float) * f->r * f->r, hipMemcpyDeviceToHost));
   if (sq_norm_A) *sq_norm_A = f->sq_norm_A;

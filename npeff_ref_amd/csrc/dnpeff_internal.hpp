@@ -60,21 +60,22 @@ bool side_stream_pending();
 
 namespace dn {
 
+// pool.hip: device memory (freed blocks of up to 256 MB are kept for later requests), copies between
+// the device and pageable host memory, pinned words for results of a few bytes.
+int device_alloc(void** out, size_t bytes, bool* reused = nullptr);
+void device_release(void* p);
+size_t pool_cached_bytes();  // freed blocks that the pool holds
+void pool_trim();            // back to the device
+hipError_t copy_up(void* dst_dev, const void* src_host, size_t bytes);
+hipError_t copy_down(void* dst_host, const void* src_dev, size_t bytes);
+int host_words(unsigned long long** out);  // 64 pinned words of the calling thread
+
 template <class T>
 inline int dmalloc(T** p, int64_t count) {
-  *p = nullptr;
-  size_t bytes = sizeof(T) * (size_t)(count > 0 ? count : 1);
-  hipError_t e = hipMalloc((void**)p, bytes);
-  if (e != hipSuccess) {
-    set_error("hipMalloc of %zu bytes failed: %s", bytes, hipGetErrorString(e));
-    return 1;
-  }
-  return 0;
+  return device_alloc((void**)p, sizeof(T) * (size_t)(count > 0 ? count : 1));
 }
 
-inline void dfree(void* p) {
-  if (p) (void)hipFree(p);
-}
+inline void dfree(void* p) { device_release(p); }
 
 inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 

@@ -522,6 +522,15 @@ __global__ void __launch_bounds__(256)
   __shared__ double sh[256];
   double s = 0.0;
   int64_t stride = (int64_t)gridDim.x * 256;
+    int64_t at = base + before;
+#pragma unroll
+    for (int k = 0; k < 4; k++)
+      if (ok[k]) {
+        idx_out[at] = (int32_t)(i + k);
+        val_out[at] = v[k];
+        at++;
+      }
+    base += all;
   for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += stride) {
     double x = (double)v[i];
     s += x * x;
@@ -1028,16 +1037,19 @@ DN_API int dnpeff_device_memory(int64_t* free_bytes, int64_t* total_bytes) {
 DN_API int dnpeff_dev_malloc(int64_t bytes, void** out) {
   clear_error();
   DN_CHECK(out != nullptr && bytes >= 0, "bad arguments");
-  char* p = nullptr;
-  DN_TRY(dmalloc(&p, bytes));
+  void* p = nullptr;
+  bool reused = false;
+  DN_TRY(device_alloc(&p, (size_t)bytes, &reused));
+  // (the caller may use the block on any stream: what the library has queued on it must be done)
+  if (reused) DN_HIP(hipStreamSynchronize(stream()));
   *out = p;
   return 0;
 }
 
 DN_API int dnpeff_dev_free(void* p) {
   if (!p) return 0;
-  DN_HIP(hipStreamSynchronize(stream()));
-  DN_HIP(hipFree(p));
+  DN_HIP(hipDeviceSynchronize());  // (work of any stream may still use the block, as for hipFree)
+  device_release(p);
   return 0;
 }
 
@@ -1045,7 +1057,8 @@ DN_API int dnpeff_dev_upload(void* dst_dev, const void* src_host, int64_t bytes)
   clear_error();
   DN_CHECK(bytes >= 0 && (bytes == 0 || (dst_dev && src_host)), "bad arguments");
   DN_HIP(hipStreamSynchronize(stream()));
-  if (bytes) DN_HIP(hipMemcpy(dst_dev, src_host, (size_t)bytes, hipMemcpyHostToDevice));
+  DN_HIP(hipStreamSynchronize(nullptr));  // (and for what other blocking streams still do, as hipMemcpy does)
+  if (bytes) DN_HIP(copy_up(dst_dev, src_host, (size_t)bytes));
   return 0;
 }
 
@@ -1053,7 +1066,8 @@ DN_API int dnpeff_dev_download(void* dst_host, const void* src_dev, int64_t byte
   clear_error();
   DN_CHECK(bytes >= 0 && (bytes == 0 || (dst_host && src_dev)), "bad arguments");
   DN_HIP(hipStreamSynchronize(stream()));
-  if (bytes) DN_HIP(hipMemcpy(dst_host, src_dev, (size_t)bytes, hipMemcpyDeviceToHost));
+  DN_HIP(hipStreamSynchronize(nullptr));
+  if (bytes) DN_HIP(copy_down(dst_host, src_dev, (size_t)bytes));
   return 0;
 }
 
@@ -1097,6 +1111,8 @@ static int check_cols_in_range(const dnpeff_csr* A) {
   return 0;
 }
 
+  DN_HIP(hipStreamSynchronize(stream()));
+  pool_trim();
 DN_API int dnpeff_csr_from_host(int64_t n_rows, int64_t n_cols, int64_t nnz, const int64_t* rowptr,
                                 const int32_t* colind, const float* vals, dnpeff_csr** out) {
   clear_error();
@@ -1110,9 +1126,9 @@ DN_API int dnpeff_csr_from_host(int64_t n_rows, int64_t n_cols, int64_t nnz, con
   if (s) { dnpeff_csr_destroy(A); return 1; }
   hipError_t e = hipMemcpy(A->rowptr, rowptr, sizeof(int64_t) * (n_rows + 1), hipMemcpyHostToDevice);
   if (e == hipSuccess && nnz)
-    e = hipMemcpy(A->colind, colind, sizeof(int32_t) * nnz, hipMemcpyHostToDevice);
+    e = copy_up(A->colind, colind, sizeof(int32_t) * nnz);
   if (e == hipSuccess && nnz)
-    e = hipMemcpy(A->vals, vals, sizeof(float) * nnz, hipMemcpyHostToDevice);
+    e = copy_up(A->vals, vals, sizeof(float) * nnz);
   if (e != hipSuccess) {
     set_error("upload of the CSR arrays failed: %s", hipGetErrorString(e));
     dnpeff_csr_destroy(A);
@@ -1142,9 +1158,9 @@ DN_API int dnpeff_csr_from_pef(int64_t n_rows, int64_t k, int64_t dense_fisher_s
                      A->rowptr);
   hipError_t e = hipGetLastError();
   if (e == hipSuccess && nnz)
-    e = hipMemcpy(A->colind, indices, sizeof(int32_t) * nnz, hipMemcpyHostToDevice);
+    e = copy_up(A->colind, indices, sizeof(int32_t) * nnz);
   if (e == hipSuccess && nnz)
-    e = hipMemcpy(A->vals, values, sizeof(float) * nnz, hipMemcpyHostToDevice);
+    e = copy_up(A->vals, values, sizeof(float) * nnz);
   if (e == hipSuccess) e = hipStreamSynchronize(stream());
   if (e != hipSuccess) {
     set_error("upload of the PEF arrays failed: %s", hipGetErrorString(e));
@@ -1221,7 +1237,7 @@ DN_API int dnpeff_csr_retain_columns(dnpeff_csr* A, const int32_t* kept, int64_t
   int32_t *table = nullptr, *kept_dev = nullptr;
   DN_TRY(dmalloc(&table, A->n_cols));
   DN_TRY(dmalloc(&kept_dev, n_kept));
-  if (n_kept) DN_HIP(hipMemcpy(kept_dev, kept, sizeof(int32_t) * n_kept, hipMemcpyHostToDevice));
+  if (n_kept) DN_HIP(copy_up(kept_dev, kept, sizeof(int32_t) * n_kept));
   hipLaunchKernelGGL(k_fill_i32, dim3(grid_for(A->n_cols)), dim3(256), 0, st, table, A->n_cols, -1);
   hipLaunchKernelGGL(k_retain_table, dim3(grid_for(n_kept)), dim3(256), 0, st, kept_dev, n_kept,
                      table);
@@ -1254,11 +1270,11 @@ DN_API int dnpeff_csr_download(const dnpeff_csr* A, int64_t* rowptr, int32_t* co
   DN_CHECK(A && has_row_major(A), "matrix is NULL or its row-major arrays were released");
   DN_HIP(hipStreamSynchronize(stream()));
   if (rowptr)
-    DN_HIP(hipMemcpy(rowptr, A->rowptr, sizeof(int64_t) * (A->n_rows + 1), hipMemcpyDeviceToHost));
+    DN_HIP(copy_down(rowptr, A->rowptr, sizeof(int64_t) * (A->n_rows + 1)));
   if (colind && A->nnz)
-    DN_HIP(hipMemcpy(colind, A->colind, sizeof(int32_t) * A->nnz, hipMemcpyDeviceToHost));
+    DN_HIP(copy_down(colind, A->colind, sizeof(int32_t) * A->nnz));
   if (vals && A->nnz)
-    DN_HIP(hipMemcpy(vals, A->vals, sizeof(float) * A->nnz, hipMemcpyDeviceToHost));
+    DN_HIP(copy_down(vals, A->vals, sizeof(float) * A->nnz));
   return 0;
 }
 
@@ -1267,7 +1283,7 @@ DN_API int dnpeff_csr_kept_indices(const dnpeff_csr* A, int32_t* new_to_og) {
   DN_CHECK(A && new_to_og, "NULL argument");
   if (A->kept) {
     if (A->n_cols)
-      DN_HIP(hipMemcpy(new_to_og, A->kept, sizeof(int32_t) * A->n_cols, hipMemcpyDeviceToHost));
+      DN_HIP(copy_down(new_to_og, A->kept, sizeof(int32_t) * A->n_cols));
   } else {
     for (int64_t i = 0; i < A->n_cols; i++) new_to_og[i] = (int32_t)i;
   }
@@ -1593,11 +1609,11 @@ DN_API int dnpeff_csr_download_transpose(dnpeff_csr* A, int64_t* colptr, int32_t
   clear_error();
   DN_TRY(dnpeff_csr_build_transpose(A));
   if (colptr)
-    DN_HIP(hipMemcpy(colptr, A->colptr, sizeof(int64_t) * (A->n_cols + 1), hipMemcpyDeviceToHost));
+    DN_HIP(copy_down(colptr, A->colptr, sizeof(int64_t) * (A->n_cols + 1)));
   if (rowind && A->nnz)
-    DN_HIP(hipMemcpy(rowind, A->rowind, sizeof(int32_t) * A->nnz, hipMemcpyDeviceToHost));
+    DN_HIP(copy_down(rowind, A->rowind, sizeof(int32_t) * A->nnz));
   if (vals && A->nnz)
-    DN_HIP(hipMemcpy(vals, A->tvals, sizeof(float) * A->nnz, hipMemcpyDeviceToHost));
+    DN_HIP(copy_down(vals, A->tvals, sizeof(float) * A->nnz));
   return 0;
 }
 
