@@ -282,6 +282,12 @@ class DeviceArray:
         _check(lib.dnpeff_dev_download(_ptr(out), self.ptr, self.nbytes))
         return out
 
+    def first(self, count: int) -> np.ndarray:
+        """The first `count` elements, flat."""
+        out = np.empty(count, dtype=self.dtype)
+        _check(lib.dnpeff_dev_download(_ptr(out), self.ptr, count * self.dtype.itemsize))
+        return out
+
     def free(self):
         if self.ptr is not None:
             lib.dnpeff_dev_free(self.ptr)
@@ -372,7 +378,7 @@ def op_threshold_compact(x: "DeviceArray", divisor: float, threshold: float):
     kept = _i64(0)
     _check(lib.dnpeff_op_threshold_compact(n, x.ptr, float(divisor), float(threshold), idx.ptr, val.ptr,
                                            C.byref(kept)))
-    return idx.numpy()[:kept.value].copy(), val.numpy()[:kept.value].copy()
+    return idx.first(kept.value), val.first(kept.value)
 
 
 class Csr:

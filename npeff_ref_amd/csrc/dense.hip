@@ -2027,15 +2027,14 @@ DN_API int dnpeff_op_xg_mu(int64_t rows, int r, const float* X, const float* G_r
 DN_API int dnpeff_op_dot(int64_t count, const float* x, const float* y, double* out_host) {
   clear_error();
   DN_CHECK(out_host != nullptr, "out is NULL");
-  double* ws = nullptr;
-  DN_TRY(dmalloc(&ws, DOT_BLOCKS + 1));
-  int s = launch_dot(count, x, y, ws, ws + DOT_BLOCKS);
-  if (!s && hipMemcpy(out_host, ws + DOT_BLOCKS, sizeof(double), hipMemcpyDeviceToHost) != hipSuccess) {
-    set_error("dot: copy of the result failed");
-    s = 1;
-  }
-  dfree(ws);
-  return s;
+  dbuf<double> ws;
+  DN_TRY(ws.alloc(DOT_BLOCKS));
+  unsigned long long* word = nullptr;
+  DN_TRY(host_words(&word));
+  DN_TRY(launch_dot(count, x, y, ws, reinterpret_cast<double*>(word)));
+  DN_HIP(hipStreamSynchronize(stream()));
+  *out_host = *reinterpret_cast<double*>(word);
+  return 0;
 }
 
 DN_API int dnpeff_op_init_uniform(int matrix_id, int64_t logical_rows, int64_t logical_cols,
