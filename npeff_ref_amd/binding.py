@@ -741,15 +741,21 @@ class Learner:
         history = []
         sync()
         t0 = time.perf_counter()
-        for i in range(p.max_iters):
-            self.step(1)
-            if p.log_every_n_steps > 0 and (i + 1) % p.log_every_n_steps == 0:
+        every = p.log_every_n_steps
+        done = 0
+        while done < p.max_iters:  # the steps up to the next logged one in one call
+            run = p.max_iters - done
+            if every > 0:
+                run = min(run, every - done % every)
+            self.step(run)
+            done += run
+            if every > 0 and done % every == 0:
                 sync()
                 elapsed_ms = (time.perf_counter() - t0) * 1e3
                 ref_loss, true_loss = self.losses()
-                ms = elapsed_ms / p.log_every_n_steps
-                log(f"step {i + 1}: {ref_loss:g} [{ms:g} ms/step]")
-                history.append((i + 1, ref_loss, true_loss, ms))
+                ms = elapsed_ms / every
+                log(f"step {done}: {ref_loss:g} [{ms:g} ms/step]")
+                history.append((done, ref_loss, true_loss, ms))
                 t0 = time.perf_counter()
         sync()
         return history

@@ -718,6 +718,7 @@ struct dnpeff_fit {
   float* AH = nullptr;   // [n, r]
   float* HH = nullptr;   // [r, r]
   float* W = nullptr;    // [n, r]
+  bool in_place = false; // all steps of a call in one launch (fit.hip), without the two buffers below
   float* W2 = nullptr;   // [n, r]
   float* WHH = nullptr;  // [n, r] W (H H^T) of the W before the last step
   float* tmp = nullptr;  // [n, r]
@@ -748,9 +749,12 @@ DN_API int dnpeff_fit_create(dnpeff_csr* A, dnpeff_csr* H, float eps, int64_t se
   dnpeff_fit* f = new dnpeff_fit();
   f->n = A->n_rows; f->r = r; f->eps = eps; f->seed = (uint64_t)seed;
   const int64_t nr = f->n * r;
+  f->in_place = fit_steps_supported(f->n, r);
+  int64_t dots = DOT_BLOCKS + 2;
+  if (f->in_place && 3 * fit_loss_parts(f->n) > dots) dots = 3 * fit_loss_parts(f->n);
   int s = dmalloc(&f->AH, nr) || dmalloc(&f->HH, (int64_t)r * r) || dmalloc(&f->W, nr) ||
-          dmalloc(&f->W2, nr) || dmalloc(&f->WHH, nr) || dmalloc(&f->tmp, nr) ||
-          dmalloc(&f->dot_ws, DOT_BLOCKS + 2);
+          dmalloc(&f->WHH, nr) || dmalloc(&f->dot_ws, dots);
+  if (!s && !f->in_place) s = dmalloc(&f->W2, nr) || dmalloc(&f->tmp, nr);
   if (!s) s = dnpeff_op_spsp_dense(H, H, f->HH);
   if (!s) s = dnpeff_op_spsp_dense(A, H, f->AH);
   if (!s) s = dnpeff_csr_sq_norm(A, &f->sq_norm_A);
@@ -782,6 +786,11 @@ DN_API int dnpeff_fit_set_W(dnpeff_fit* f, const float* W_nr) {
 DN_API int dnpeff_fit_step(dnpeff_fit* f, int n_steps) {
   clear_error();
   DN_CHECK(f != nullptr, "handle is NULL");
+  if (n_steps <= 0) return 0;
+  if (f->in_place) {
+    f->whh_valid = true;
+    return launch_fit_steps(f->n, f->r, f->W, f->HH, f->AH, f->eps, n_steps, f->WHH);
+  }
   struct held_g {  // H H^T is the same in every step: one transposed copy for all of them
     ~held_g() { xg_mu_release_g(); }
   } hold;
@@ -798,6 +807,17 @@ DN_API int dnpeff_fit_loss(dnpeff_fit* f, double* reference_loss, double* true_l
   clear_error();
   DN_CHECK(f != nullptr, "handle is NULL");
   const int64_t nr = f->n * f->r;
+  if (f->in_place) {
+    unsigned long long* words = nullptr;
+    DN_TRY(host_words(&words));
+    double* sums = reinterpret_cast<double*>(words);
+    DN_TRY(launch_fit_loss(f->n, f->r, f->W, f->HH, f->AH, f->whh_valid ? f->WHH : nullptr, f->dot_ws, sums));
+    DN_HIP(hipStreamSynchronize(stream()));
+    const double pos_ref = f->whh_valid ? sums[2] : sums[1];
+    if (true_loss) *true_loss = std::sqrt(f->sq_norm_A + sums[1] - 2.0 * sums[0]);
+    if (reference_loss) *reference_loss = std::sqrt(f->sq_norm_A + pos_ref - 2.0 * sums[0]);
+    return 0;
+  }
   double res[2];
   // neg = <A H^T, W>
   DN_TRY(launch_dot(nr, f->AH, f->W, f->dot_ws, f->dot_ws + DOT_BLOCKS));

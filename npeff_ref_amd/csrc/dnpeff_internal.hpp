@@ -143,6 +143,15 @@ int launch_init_uniform(int matrix_id, int64_t logical_rows, int64_t logical_col
 // out[c * rows + i] = in[i * cols + c]   (in is [rows, cols] row-major)
 int launch_transpose(int64_t rows, int64_t cols, const float* in, float* out);
 
+// ---- fixed-H learner (fit.hip) ----
+bool fit_steps_supported(int64_t n, int r);
+int64_t fit_loss_parts(int64_t n);  // 3 doubles each in launch_fit_loss's partials
+int launch_fit_steps(int64_t n, int r, float* W, const float* G, const float* AH, float eps, int n_steps,
+                     float* WHH);
+// out3 (device or pinned) = <AH, W>, <W G, W>, <WHH, W> (WHH may be NULL: 0)
+int launch_fit_loss(int64_t n, int r, const float* W, const float* G, const float* AH, const float* WHH,
+                    double* partials, double* out3);
+
 // ---- sparse kernels (spmm.hip) ----
 constexpr int64_t SPMM_N_CHUNK = 2048;  // entries of one row handled by one workgroup
 constexpr int64_t SPMM_T_LONG = 256;    // columns longer than this get a whole workgroup

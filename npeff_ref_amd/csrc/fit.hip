@@ -1,0 +1,225 @@
+// The W-only updates of the fixed-H learner, all steps of a call in one launch.
+//
+// W <- W * (A H^T) / (W (H H^T) + eps) works row by row, so a workgroup that holds 16 rows of W and
+// of A H^T and the whole of G = H H^T can do every step of the call without touching memory in
+// between: at r = 256 its registers hold G (32 columns per wave, 128 registers a lane), the 16 rows of W
+// lie in LDS as the A operand of the next step (two buffers: one barrier per step) and, with A H^T, in
+// registers in the accumulator layout for the update itself.  fp32 matrix cores, as the rows are too
+// few for the split-operand kernels: 2,000 rows are 125 workgroups.  Bound by the matrix cores of the CUs
+// it fills (16 r^2 multiply-adds per workgroup and step at 256 flop per clock and CU: 3.4 us at
+// r = 256).  25 steps of 2,000 x 256: 1.22 ms as launches of a product kernel, a transposition and
+// a kernel for the last rows per step; figures now at launch_fit_steps.
+#include "dnpeff_internal.hpp"
+
+#include <type_traits>
+
+namespace dn {
+
+typedef float acc4 __attribute__((ext_vector_type(4)));
+
+constexpr int FIT_ROWS = 16;
+
+// G in registers and the product of a workgroup's 16 rows (in LDS) with it.  RP: the rank padded to a
+// multiple of 32; wave w owns columns 32 w .. 32 w + 31 as two blocks of 16.  Lane (i = l % 16,
+// kg = l / 16) reads X[row i][16 q + 4 kg .. + 3] with one 16-byte LDS read and step s of the
+// group contracts component 16 q + 4 kg + s against the same row of G.
+template <int RP>
+struct FitTile {
+  static constexpr int LD = RP + 4;  // floats per row of X in LDS
+  static constexpr int Q = RP / 16;
+  float g[Q][2][4];
+  int lane, wave, kg, l16;
+
+  __device__ inline void init(const float* __restrict__ G, int r) {
+    lane = threadIdx.x & 63;
+    wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    l16 = lane & 15;
+    kg = lane >> 4;
+#pragma unroll
+    for (int q = 0; q < Q; q++)
+#pragma unroll
+      for (int b = 0; b < 2; b++)
+#pragma unroll
+        for (int s = 0; s < 4; s++) {
+          const int k = 16 * q + 4 * kg + s, c = col(b);
+          const bool ok = k < r && c < r;
+          const float v = G[ok ? (int64_t)k * r + c : 0];
+          g[q][b][s] = ok ? v : 0.0f;
+        }
+  }
+  __device__ inline int col(int b) const { return 32 * wave + 16 * b + l16; }
+  __device__ inline int row(int v) const { return 4 * kg + v; }  // of accumulator register v
+
+  __device__ inline void product(const float* buf, acc4 (&d)[2]) const {
+    d[0] = d[1] = acc4{0.0f, 0.0f, 0.0f, 0.0f};
+    const float* pa = buf + l16 * LD + 4 * kg;
+#pragma unroll
+    for (int q = 0; q < Q; q++) {
+      const float4 a = *reinterpret_cast<const float4*>(pa + 16 * q);
+#pragma unroll
+      for (int s = 0; s < 4; s++) {
+        const float as = s == 0 ? a.x : s == 1 ? a.y : s == 2 ? a.z : a.w;
+#pragma unroll
+        for (int b = 0; b < 2; b++) d[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(as, g[q][b][s], d[b], 0, 0, 0);
+      }
+    }
+  }
+};
+
+// n_steps updates of W in place; WHH receives W G of the W before the last of them.
+template <int RP>
+__global__ void __launch_bounds__(2 * RP)
+    k_fit_steps(float* __restrict__ W, const float* __restrict__ G, const float* __restrict__ AH, float eps,
+                int64_t n, int r, int n_steps, float* __restrict__ WHH) {
+  using T = FitTile<RP>;
+  __shared__ __align__(16) float buf[2][FIT_ROWS * T::LD];
+  T t;
+  t.init(G, r);
+  const int64_t row0 = (int64_t)blockIdx.x * FIT_ROWS;
+  float x[2][4], ah[2][4];
+  bool ok[2][4];
+  int64_t at[2][4];
+#pragma unroll
+  for (int b = 0; b < 2; b++)
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+      ok[b][v] = row0 + t.row(v) < n && t.col(b) < r;
+      at[b][v] = ok[b][v] ? (row0 + t.row(v)) * r + t.col(b) : 0;
+      x[b][v] = W[at[b][v]];
+      ah[b][v] = AH[at[b][v]];
+    }
+#pragma unroll
+  for (int b = 0; b < 2; b++)
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+      if (!ok[b][v]) x[b][v] = 0.0f;  // (rows and columns of the padding stay zero)
+      buf[0][t.row(v) * T::LD + t.col(b)] = x[b][v];
+    }
+  __syncthreads();
+  acc4 d[2];
+  for (int s = 0; s < n_steps; s++) {
+    t.product(buf[s & 1], d);
+#pragma unroll
+    for (int b = 0; b < 2; b++)
+#pragma unroll
+      for (int v = 0; v < 4; v++) {
+        const float q = ah[b][v] / (d[b][v] + eps);
+        x[b][v] = ok[b][v] ? x[b][v] * q : 0.0f;
+        buf[(s + 1) & 1][t.row(v) * T::LD + t.col(b)] = x[b][v];
+      }
+    __syncthreads();  // (the buffer just read is written again one barrier from here)
+  }
+#pragma unroll
+  for (int b = 0; b < 2; b++)
+#pragma unroll
+    for (int v = 0; v < 4; v++)
+      if (ok[b][v]) {
+        W[at[b][v]] = x[b][v];
+        WHH[at[b][v]] = d[b][v];
+      }
+}
+
+// <A H^T, W>, <W G, W> and (where WHH is given) <WHH, W> of a workgroup's rows, in fp64.
+template <int RP>
+__global__ void __launch_bounds__(2 * RP)
+    k_fit_loss(const float* __restrict__ W, const float* __restrict__ G, const float* __restrict__ AH,
+               const float* __restrict__ WHH, int64_t n, int r, double* __restrict__ partials) {
+  using T = FitTile<RP>;
+  __shared__ __align__(16) float buf[FIT_ROWS * T::LD];
+  __shared__ double red[RP / 32][3];
+  T t;
+  t.init(G, r);
+  const int64_t row0 = (int64_t)blockIdx.x * FIT_ROWS;
+  float x[2][4], ah[2][4], wh[2][4];
+#pragma unroll
+  for (int b = 0; b < 2; b++)
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+      const bool ok = row0 + t.row(v) < n && t.col(b) < r;
+      const int64_t at = ok ? (row0 + t.row(v)) * r + t.col(b) : 0;
+      const float w = W[at], a = AH[at], h = WHH ? WHH[at] : 0.0f;
+      x[b][v] = ok ? w : 0.0f;
+      ah[b][v] = ok ? a : 0.0f;
+      wh[b][v] = ok ? h : 0.0f;
+      buf[t.row(v) * T::LD + t.col(b)] = x[b][v];
+    }
+  __syncthreads();
+  acc4 d[2];
+  t.product(buf, d);
+  double s[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+  for (int b = 0; b < 2; b++)
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+      s[0] += (double)ah[b][v] * (double)x[b][v];
+      s[1] += (double)d[b][v] * (double)x[b][v];
+      s[2] += (double)wh[b][v] * (double)x[b][v];
+    }
+#pragma unroll
+  for (int k = 0; k < 3; k++) {
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) s[k] += __shfl_xor(s[k], off);
+    if (t.lane == 0) red[t.wave][k] = s[k];
+  }
+  __syncthreads();
+  if (threadIdx.x < 3) {
+    double sum = 0.0;
+    for (int w = 0; w < RP / 32; w++) sum += red[w][threadIdx.x];
+    partials[(int64_t)blockIdx.x * 3 + threadIdx.x] = sum;
+  }
+}
+
+// out[k] = sum of the workgroups' k-th sums, in a fixed order
+__global__ void __launch_bounds__(192) k_fit_loss_sum(const double* __restrict__ partials, int64_t n_parts,
+                                                      double* __restrict__ out) {
+  const int k = threadIdx.x / 64, lane = threadIdx.x & 63;
+  double s = 0.0;
+  for (int64_t p = lane; p < n_parts; p += 64) s += partials[p * 3 + k];
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off);
+  if (lane == 0) out[k] = s;
+}
+
+bool fit_steps_supported(int64_t n, int r) { return r >= 1 && r <= 256 && n >= 1 && n < ((int64_t)1 << 31); }
+int64_t fit_loss_parts(int64_t n) { return ceil_div(n, FIT_ROWS); }
+
+// f(integral constant RP) with the padded rank that fits r
+template <class F>
+static void fit_dispatch(int r, F&& f) {
+  if (r <= 32) f(std::integral_constant<int, 32>{});
+  else if (r <= 64) f(std::integral_constant<int, 64>{});
+  else if (r <= 96) f(std::integral_constant<int, 96>{});
+  else if (r <= 128) f(std::integral_constant<int, 128>{});
+  else if (r <= 192) f(std::integral_constant<int, 192>{});
+  else f(std::integral_constant<int, 256>{});
+}
+
+int launch_fit_steps(int64_t n, int r, float* W, const float* G, const float* AH, float eps, int n_steps,
+                     float* WHH) {
+  // (a launch of many steps would keep the device from everything else for long: 256 steps are about a
+  // millisecond per 4,096 rows at r = 256)
+  for (int done = 0; done < n_steps; done += 256) {
+    const int now = n_steps - done < 256 ? n_steps - done : 256;
+    fit_dispatch(r, [&](auto rp) {
+      constexpr int RP = decltype(rp)::value;
+      hipLaunchKernelGGL(k_fit_steps<RP>, dim3((unsigned)ceil_div(n, FIT_ROWS)), dim3(2 * RP), 0, stream(), W, G,
+                         AH, eps, n, r, now, WHH);
+    });
+    DN_LAUNCH_CHECK();
+  }
+  return 0;
+}
+
+int launch_fit_loss(int64_t n, int r, const float* W, const float* G, const float* AH, const float* WHH,
+                    double* partials, double* out3) {
+  fit_dispatch(r, [&](auto rp) {
+    constexpr int RP = decltype(rp)::value;
+    hipLaunchKernelGGL(k_fit_loss<RP>, dim3((unsigned)ceil_div(n, FIT_ROWS)), dim3(2 * RP), 0, stream(), W, G, AH,
+                       WHH, n, r, partials);
+  });
+  hipLaunchKernelGGL(k_fit_loss_sum, dim3(1), dim3(192), 0, stream(), partials, fit_loss_parts(n), out3);
+  DN_LAUNCH_CHECK();
+  return 0;
+}
+
+}  // namespace dn
