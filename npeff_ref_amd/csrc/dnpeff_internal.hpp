@@ -276,12 +276,13 @@ struct dnpeff_csr {
   int64_t* colptr = nullptr;
   int32_t* rowind = nullptr;
   float* tvals = nullptr;
-  // as the sparse factor of dnpeff_op_spsp_dense: per column 32 bytes holding its first four
-  // (row, value) pairs and, in the upper half of the first row word, its length
+  // as the sparse factor of dnpeff_op_spsp_dense: per column 32 bytes holding its first six
+  // (row, value) pairs and its length (spmm.hip)
   uint4* slots = nullptr;
   // work decomposition of A H^T: chunk_base[i] = chunks of rows before i
   int64_t* chunk_base = nullptr;
   int64_t n_chunks = 0;
+  int64_t max_row_chunks = 0;  // most chunks of one row (known for up to 4096 rows, else 0)
   // columns longer than SPMM_T_LONG
   int32_t* long_cols = nullptr;
   int64_t n_long = 0;

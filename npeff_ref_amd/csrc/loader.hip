@@ -750,8 +750,15 @@ int csr_ensure_chunks(dnpeff_csr* A) {
   DN_CHECK(A->rowptr != nullptr, "row-major copy of the matrix was released");
   DN_TRY(dmalloc(&A->chunk_base, A->n_rows + 1));
   DN_TRY(scan_row_chunks(A->rowptr, SPMM_N_CHUNK, A->n_rows, A->chunk_base));
-  DN_HIP(hipMemcpy(&A->n_chunks, A->chunk_base + A->n_rows, sizeof(int64_t),
-                   hipMemcpyDeviceToHost));
+  A->max_row_chunks = 0;
+  if (A->n_rows > 0 && A->n_rows <= 4096) {
+    std::vector<int64_t> base((size_t)A->n_rows + 1);
+    DN_HIP(hipMemcpy(base.data(), A->chunk_base, sizeof(int64_t) * base.size(), hipMemcpyDeviceToHost));
+    for (int64_t i = 0; i < A->n_rows; i++) A->max_row_chunks = std::max(A->max_row_chunks, base[i + 1] - base[i]);
+    A->n_chunks = base[A->n_rows];
+  } else {
+    DN_HIP(hipMemcpy(&A->n_chunks, A->chunk_base + A->n_rows, sizeof(int64_t), hipMemcpyDeviceToHost));
+  }
   return 0;
 }
 

@@ -906,14 +906,22 @@ __global__ void __launch_bounds__(256)
 // ---------------------------------------------------------------------------
 // partials[chunk, :] = sum over the chunk's entries (j, a) of a * B[:, j] for a sparse B, a
 // lane per entry.  B's transposed copy (per column j: component ids and values) is condensed
-// into one 32-byte slot per column (its first four (component, value) pairs, the column's
-// length in the upper half of the first component word), so that an entry of A costs one
-// random sector instead of three dependent ones (column offsets, component ids, values); only
-// columns longer than four go on to the transposed arrays.  Each wave keeps its r running sums
-// in LDS and the lanes add into them with ds_add_f32: step k of a batch applies the k-th pair
-// of all 64 entries at once, and where two lanes meet in a component the LDS adds them one
-// after the other in lane order, the same way in every run.
+// into one 32-byte slot per column: its first six values and, in 64 bits, the column's length (7 =
+// more than six) and six component ids of ten bits.  An entry of A then costs one random sector
+// instead of three dependent ones (column offsets, component ids, values); only columns longer than six
+// go on to the transposed arrays (1.5 % of them at 2.6 entries per column, where four pairs
+// per slot left 11 %).  Each wave keeps its r running sums in LDS and the lanes add into them with
+// ds_add_f32: step k of a batch applies the k-th pair of all 64 entries at once, and where two lanes
+// meet in a component the LDS adds them one after the other in lane order, the same way in every run.
+// Bound by the random sectors that miss the L2s: A H^T of 65.5 M entries with 256 x 22M at 1 % takes
+// 0.88 ms (1.60 with four pairs per slot, whose second half was read only where it was needed, one
+// round trip later).  With `across` the workgroups run over the rows first and along them second: rows
+// that hold their columns in ascending order, as those of H, then look up the same part of the slots
+// at one time and find it in the memory-side cache; H H^T of that H 1.06 ms (2.36 row by row, every
+// row reading all 704 MB of slots from HBM).
 // ---------------------------------------------------------------------------
+constexpr int SPSP_PAIRS = 6;
+
 __global__ void __launch_bounds__(256)
     k_spsp_build_slots(int64_t n_cols, const int64_t* __restrict__ colptr, const int32_t* __restrict__ comp,
                        const float* __restrict__ vals, uint4* __restrict__ slots) {
@@ -921,15 +929,15 @@ __global__ void __launch_bounds__(256)
   if (j >= n_cols) return;
   const int64_t q0 = colptr[j];
   const int len = (int)(colptr[j + 1] - q0);
-  unsigned w[8];
+  unsigned w[SPSP_PAIRS];
+  uint64_t ids = (uint64_t)(len <= SPSP_PAIRS ? len : SPSP_PAIRS + 1);
 #pragma unroll
-  for (int k = 0; k < 4; k++) {
-    w[2 * k] = k < len ? (unsigned)comp[q0 + k] : 0u;
-    w[2 * k + 1] = k < len ? __float_as_uint(vals[q0 + k]) : 0u;
+  for (int k = 0; k < SPSP_PAIRS; k++) {
+    w[k] = k < len ? __float_as_uint(vals[q0 + k]) : 0u;
+    ids |= (uint64_t)(k < len ? comp[q0 + k] : 0) << (4 + 10 * k);
   }
-  w[0] |= (unsigned)len << 16;
-  slots[2 * j] = make_uint4(w[0], w[1], w[2], w[3]);
-  slots[2 * j + 1] = make_uint4(w[4], w[5], w[6], w[7]);
+  slots[2 * j] = make_uint4(w[0], w[1], (unsigned)(ids & 0xffffffffu), (unsigned)(ids >> 32));
+  slots[2 * j + 1] = make_uint4(w[2], w[3], w[4], w[5]);
 }
 
 template <int VPL>
@@ -938,11 +946,18 @@ __global__ void __launch_bounds__(256)
                  const float* __restrict__ vals, const int64_t* __restrict__ chunk_base, int64_t n_rows,
                  int r, const uint4* __restrict__ slots, const int64_t* __restrict__ b_colptr,
                  const int32_t* __restrict__ b_comp, const float* __restrict__ b_vals,
-                 float* __restrict__ partials) {
+                 float* __restrict__ partials, int across) {
   __shared__ float red[4][64 * VPL];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-  const int64_t chunk = blockIdx.x;
-  const int64_t row = chunk_to_row(chunk_base, n_rows, chunk);
+  int64_t chunk, row;
+  if (across) {
+    row = blockIdx.x % n_rows;
+    chunk = chunk_base[row] + blockIdx.x / n_rows;
+    if (chunk >= chunk_base[row + 1]) return;
+  } else {
+    chunk = blockIdx.x;
+    row = chunk_to_row(chunk_base, n_rows, chunk);
+  }
   const int64_t e0 = rowptr[row] + (chunk - chunk_base[row]) * SPMM_N_CHUNK;
   int64_t e1 = e0 + SPMM_N_CHUNK;
   if (e1 > rowptr[row + 1]) e1 = rowptr[row + 1];
@@ -955,23 +970,28 @@ __global__ void __launch_bounds__(256)
 #pragma unroll
   for (int t = 0; t < VPL; t++) acc[lane + 64 * t] = 0.0f;
 
+  // (column, value) pairs one batch ahead of the slots
+  int32_t nj = w0 + lane < w1 ? colind[w0 + lane] : 0;
+  float na = w0 + lane < w1 ? vals[w0 + lane] : 0.0f;
   for (int64_t e = w0; e < w1; e += 64) {
-    if (e + lane < w1) {
-      const int32_t j = colind[e + lane];
-      const float a = vals[e + lane];
-      const uint4 s0 = slots[2 * (int64_t)j];
-      const int len = (int)(s0.x >> 16);
-      if (len > 0) atomicAdd(&acc[s0.x & 0xffffu], a * __uint_as_float(s0.y));
-      if (len > 1) atomicAdd(&acc[s0.z], a * __uint_as_float(s0.w));
-      if (len > 2) {
-        const uint4 s1 = slots[2 * (int64_t)j + 1];
-        atomicAdd(&acc[s1.x], a * __uint_as_float(s1.y));
-        if (len > 3) atomicAdd(&acc[s1.z], a * __uint_as_float(s1.w));
-        if (len > 4) {
-          const int64_t q = b_colptr[j];
-          for (int k = 4; k < len; k++) atomicAdd(&acc[b_comp[q + k]], a * b_vals[q + k]);
-        }
-      }
+    const int64_t j = nj;
+    const float a = na;
+    const bool in = e + lane < w1;
+    const uint4 s0 = slots[2 * j], s1 = slots[2 * j + 1];  // (lanes past the end: column 0, not added)
+    const int64_t en = e + 64 + lane;
+    if (en < w1) {
+      nj = colind[en];
+      na = vals[en];
+    }
+    const uint64_t ids = ((uint64_t)s0.w << 32) | s0.z;
+    const int len = in ? (int)(ids & 15u) : 0;
+    const unsigned v[SPSP_PAIRS] = {s0.x, s0.y, s1.x, s1.y, s1.z, s1.w};
+#pragma unroll
+    for (int k = 0; k < SPSP_PAIRS; k++)
+      if (len > k) atomicAdd(&acc[(ids >> (4 + 10 * k)) & 1023u], a * __uint_as_float(v[k]));
+    if (len > SPSP_PAIRS) {
+      const int64_t q1 = b_colptr[j + 1];
+      for (int64_t q = b_colptr[j] + SPSP_PAIRS; q < q1; q++) atomicAdd(&acc[b_comp[q]], a * b_vals[q]);
     }
   }
   __syncthreads();
@@ -1387,9 +1407,14 @@ int launch_spsp(const dnpeff_csr* A, dnpeff_csr* B, float* partials) {
     DN_LAUNCH_CHECK();
   }
   dim3 grid((unsigned)A->n_chunks), block(256);
+  // H H^T: its rows are of about the same length (at most as many empty workgroups as real ones) and
+  // keep their columns in order
+  const int64_t spread = A->max_row_chunks * A->n_rows;
+  const int across = A == B && A->max_row_chunks > 0 && spread <= 2 * A->n_chunks && spread < (int64_t)INT32_MAX;
+  if (across) grid = dim3((unsigned)spread);
 #define DN_SPSP(V)                                                                               \
   hipLaunchKernelGGL((k_spsp_slots<V>), grid, block, 0, stream(), A->rowptr, A->colind, A->vals,   \
-                     A->chunk_base, A->n_rows, r, B->slots, B->colptr, B->rowind, B->tvals, partials)
+                     A->chunk_base, A->n_rows, r, B->slots, B->colptr, B->rowind, B->tvals, partials, across)
   switch (vpl_for(r)) {
     case 1: DN_SPSP(1); break;
     case 2: DN_SPSP(2); break;
