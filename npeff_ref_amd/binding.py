@@ -621,15 +621,20 @@ class MuNmf:
         history = []
         sync()
         t0 = time.perf_counter()
-        for step in range(p.max_iters):
-            self.step(1)
-            if p.log_every > 0 and (step + 1) % p.log_every == 0:
+        done = 0
+        while done < p.max_iters:  # the steps up to the next logged one in one call
+            run = p.max_iters - done
+            if p.log_every > 0:
+                run = min(run, p.log_every - done % p.log_every)
+            self.step(run)
+            done += run
+            if p.log_every > 0 and done % p.log_every == 0:
                 sync()
                 elapsed_ms = (time.perf_counter() - t0) * 1e3
                 loss = self.computeUncachedLoss()
                 ms = elapsed_ms / p.log_every
-                log(f"step {step + 1}: {loss:g} [{ms:g} ms/step]")
-                history.append((step + 1, loss, ms))
+                log(f"step {done}: {loss:g} [{ms:g} ms/step]")
+                history.append((done, loss, ms))
                 t0 = time.perf_counter()
         sync()
         return history

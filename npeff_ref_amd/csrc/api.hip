@@ -2,6 +2,7 @@
 // run_nmf_on_pefs and the W-only learner of fit_coeffs_to_sparse_H.
 #include <chrono>
 #include "dnpeff_internal.hpp"
+#include "fused.hpp"
 
 #include <algorithm>
 #include <cmath>
@@ -111,7 +112,16 @@ struct dnpeff_nmf {
   bool nw_valid = false;     // Nw holds A H^T of the current H (left there by the loss)
   double sq_norm_A = 0.0;
   Profiler prof;
+  // The step of small ranks (fused.hip).  While the switch is off, another context's dense head is on
+  // the matrix or the launches of each class are being timed, the separate kernels run instead.
+  bool has_fused = false;
+  fused_state fu;
+  bool fu_n_valid = false;   // fu.n_part (or Nw, with panels) holds A H^T of the current H
 };
+
+static bool fused_now(const dnpeff_nmf* h) {
+  return h->has_fused && tuning().fused_gram != 0.0 && !h->A->tail && !h->prof.enabled;
+}
 
 DN_API int dnpeff_nmf_destroy(dnpeff_nmf* nmf) {
   if (!nmf) return 0;
@@ -119,6 +129,7 @@ DN_API int dnpeff_nmf_destroy(dnpeff_nmf* nmf) {
   dfree(nmf->W); dfree(nmf->W2); dfree(nmf->Nw); dfree(nmf->Hbuf); dfree(nmf->S); dfree(nmf->S2);
   dfree(nmf->G); dfree(nmf->G2); dfree(nmf->gram_ws); dfree(nmf->dot_ws);
   dfree(nmf->GH); dfree(nmf->gpart);
+  nmf->fu.destroy();
   delete nmf;
   return 0;
 }
@@ -204,7 +215,9 @@ DN_API int dnpeff_plan_estimate(int64_t n_rows, int64_t n_cols, int64_t nnz_spar
 // the rows hold it (dense_fill switch; 0 = never split); the fraction is raised until the dense
 // blocks and both sparse copies of the rest fit the memory left beside the factors.  *tiled
 // receives whether the H update must run on column tiles for everything to fit.
-static int plan_matrix(dnpeff_csr* A, int rank, bool consume, bool* tiled) {
+// *fused: whether the step of small ranks can run (it reads the whole matrix from its own lists: no
+// dense head is split off then).
+static int plan_matrix(dnpeff_csr* A, int rank, bool consume, bool* tiled, bool* fused) {
   const tuning_t& tn = tuning();
   size_t free_b = 0, total_b = 0;
   DN_HIP(hipMemGetInfo(&free_b, &total_b));
@@ -224,7 +237,11 @@ static int plan_matrix(dnpeff_csr* A, int rank, bool consume, bool* tiled) {
   const plan_table t_tiled = plan_overheads(A->n_rows, A->n_cols, A->nnz, rank, true, sweeps, (double)total_b);
   const double budget_full = avail - t_full.total();
   const double budget_tiled = avail - t_tiled.total();
-  const bool can_split = rank % 4 == 0 && rank >= 64 && A->n_rows >= 1024;
+  // (multiples of 64 with rows enough for a dense head keep it: its kernels are made for those ranks)
+  *fused = tn.fused_gram != 0.0 && tn.tiled_h <= 0.0 && !(rank % 64 == 0 && A->n_rows >= 1024) &&
+           fused_supported(A->n_rows, A->n_cols, A->nnz, rank) &&
+           16.0 * (double)A->nnz + fused_bytes(A->n_rows, A->nnz, rank) < budget_full;
+  const bool can_split = rank % 4 == 0 && rank >= 64 && A->n_rows >= 1024 && !*fused;
   double fill = tn.dense_fill;
   if (fill > 1.0) fill = 0.0;
   *tiled = tn.tiled_h > 0.0;
@@ -290,8 +307,8 @@ static int nmf_create_impl(dnpeff_csr* A, int rank, float eps, int64_t seed, uns
   double sq_norm = 0.0;
   DN_TRY(dnpeff_csr_sq_norm(A, &sq_norm));
   mark("||A||^2");
-  bool tiled = false;
-  DN_TRY(plan_matrix(A, rank, consume, &tiled));
+  bool tiled = false, fused = false;
+  DN_TRY(plan_matrix(A, rank, consume, &tiled, &fused));
   mark("memory plan, dense head and sparse tail");
   if (consume && A->tail) {  // the tail and the head hold everything the products read
     DN_HIP(hipStreamSynchronize(stream()));
@@ -314,8 +331,9 @@ static int nmf_create_impl(dnpeff_csr* A, int rank, float eps, int64_t seed, uns
   int64_t ws = gram_workspace_floats(h->m, rank);
   int64_t ws_n = gram_workspace_floats(h->n, rank);
   if (ws_n > ws) ws = ws_n;
-  int s = dmalloc(&h->W, nr) || dmalloc(&h->W2, nr) || dmalloc(&h->Nw, nr) ||
-          dmalloc(&h->Hbuf, h_floats) || dmalloc(&h->S, s_floats) ||
+  // (four spare floats: the step of small ranks reads rows in 16-byte pieces)
+  int s = dmalloc(&h->W, nr + 4) || dmalloc(&h->W2, nr + 4) || dmalloc(&h->Nw, nr + 4) ||
+          dmalloc(&h->Hbuf, h_floats + 4) || dmalloc(&h->S, s_floats + 4) ||
           dmalloc(&h->G, (int64_t)rank * rank) || dmalloc(&h->G2, (int64_t)rank * rank) ||
           dmalloc(&h->gram_ws, ws) || dmalloc(&h->dot_ws, DOT_BLOCKS + 2);
   h->H = h->Hbuf;
@@ -323,6 +341,10 @@ static int nmf_create_impl(dnpeff_csr* A, int rank, float eps, int64_t seed, uns
     s = dmalloc(&h->GH, (int64_t)rank * rank) || dmalloc(&h->gpart, xg_mu_gram_workspace_floats(h->m));
   if (!s && h->tiled && tuning().h_overlap != 0.0) s = dmalloc(&h->S2, s_floats);
   if (!s && h->tiled) s = csr_tile_lists(A);
+  if (!s && fused && !h->tiled && !A->tail) {
+    h->has_fused = true;
+    s = fused_plan_build(A, rank) || h->fu.create(A, h->n, rank);
+  }
   if (s) { dnpeff_nmf_destroy(h); return s; }
   mark("factors and workspaces");
   if (tuning().verbose != 0.0) {
@@ -357,6 +379,8 @@ DN_API int dnpeff_nmf_init_factors(dnpeff_nmf* nmf) {
   DN_CHECK(nmf != nullptr, "handle is NULL");
   nmf->gh_valid = false;
   nmf->nw_valid = false;
+  nmf->fu_n_valid = false;
+  nmf->fu.gh_state = nmf->fu.gw_state = fused_state::NONE;
   DN_TRY(launch_init_uniform(0, nmf->n, nmf->r, nmf->seed, nmf->W));
   DN_TRY(launch_init_uniform(1, nmf->r, nmf->m, nmf->seed, nmf->H));
   return 0;
@@ -366,11 +390,14 @@ DN_API int dnpeff_nmf_set_factors(dnpeff_nmf* nmf, const float* W_nr, const floa
   clear_error();
   DN_CHECK(nmf != nullptr, "handle is NULL");
   DN_HIP(hipStreamSynchronize(stream()));
+  if (W_nr) nmf->fu.gw_state = fused_state::NONE;
   if (W_nr)
     DN_HIP(copy_up(nmf->W, W_nr, sizeof(float) * nmf->n * nmf->r));
   if (H_rm) {
     nmf->gh_valid = false;
     nmf->nw_valid = false;
+    nmf->fu_n_valid = false;
+    nmf->fu.gh_state = fused_state::NONE;
     // [r, m] row-major on the host -> [m, r] on the device, through S, a column tile at a time
     // when S holds no more
     const int64_t step = nmf->tiled ? nmf->tile_cols : nmf->m;
@@ -396,8 +423,49 @@ static int products_for(dnpeff_nmf* h) {
   return 0;
 }
 
+// A H^T by chunks (or, where the factor is large enough for column panels, as Nw), and H^T H.
+static int fused_products(dnpeff_nmf* h) {
+  DN_TRY(products_for(h));
+  DN_TRY(fused_plan_build(h->A, h->r));
+  if (h->fu.gh_state == fused_state::NONE) {
+    DN_TRY(launch_gram(h->m, h->r, h->H, h->G, h->gram_ws));
+    DN_TRY(h->fu.set_gram(h->G, true));
+  }
+  if (!h->fu_n_valid) {
+    if (h->A->n_panels > 0) {
+      DN_TRY(launch_spmm_n(h->A, h->r, h->H));
+      DN_TRY(launch_spmm_n_reduce(h->A, h->r, h->Nw));
+      h->nw_valid = true;
+    } else {
+      DN_TRY(h->fu.product_n(h->A, h->H));
+    }
+    h->fu_n_valid = true;
+  }
+  return h->fu.sum_h();
+}
+
+static const float* fused_nw(const dnpeff_nmf* h) { return h->A->n_panels > 0 ? h->Nw : nullptr; }
+
+static int fused_update_W(dnpeff_nmf* h) {
+  DN_TRY(fused_products(h));
+  return h->fu.update_w(h->A, h->n, fused_nw(h), h->W, h->eps);
+}
+
+static int fused_update_H(dnpeff_nmf* h) {
+  DN_TRY(products_for(h));
+  DN_TRY(fused_plan_build(h->A, h->r));
+  if (h->fu.gw_state == fused_state::NONE) {
+    DN_TRY(launch_gram(h->n, h->r, h->W, h->G, h->gram_ws));
+    DN_TRY(h->fu.set_gram(h->G, false));
+  }
+  h->nw_valid = h->gh_valid = h->fu_n_valid = false;
+  return h->fu.update_h(h->A, h->W, h->H, h->eps);
+}
+
 DN_API int dnpeff_nmf_update_W(dnpeff_nmf* h) {
   DN_CHECK(h != nullptr, "handle is NULL");
+  if (fused_now(h)) return fused_update_W(h);
+  h->fu.gw_state = fused_state::NONE;
   dnpeff_csr* A = h->A;
   bool gram_done = false;
   if (!h->nw_valid && !h->gh_valid && tuning().gram_beside != 0.0) {
@@ -544,6 +612,9 @@ static int update_H_tiled(dnpeff_nmf* h) {
 
 DN_API int dnpeff_nmf_update_H(dnpeff_nmf* h) {
   DN_CHECK(h != nullptr, "handle is NULL");
+  if (fused_now(h)) return fused_update_H(h);
+  h->fu.gh_state = fused_state::NONE;
+  h->fu_n_valid = false;
   dnpeff_csr* A = h->A;
   DN_TRY(products_for(h));
   DN_TRY(h->prof.begin(DNPEFF_K_GRAM_W));
@@ -582,6 +653,22 @@ DN_API int dnpeff_nmf_loss_terms(dnpeff_nmf* h, double* sq_norm_A, double* pos, 
   clear_error();
   DN_CHECK(h != nullptr, "handle is NULL");
   dnpeff_csr* A = h->A;
+  if (fused_now(h)) {
+    unsigned long long* words = nullptr;
+    DN_TRY(host_words(&words));
+    double* sums = reinterpret_cast<double*>(words);
+    DN_TRY(fused_products(h));
+    if (h->fu.gw_state == fused_state::NONE) {
+      DN_TRY(launch_gram(h->n, h->r, h->W, h->G, h->gram_ws));
+      DN_TRY(h->fu.set_gram(h->G, false));
+    }
+    DN_TRY(h->fu.loss_sums(A, h->n, fused_nw(h), h->W, sums));
+    DN_HIP(hipStreamSynchronize(stream()));
+    if (sq_norm_A) *sq_norm_A = h->sq_norm_A;
+    if (neg) *neg = sums[0];
+    if (pos) *pos = sums[1];
+    return 0;
+  }
   // neg = <W^T A, H> = <A H^T, W>
   if (!h->nw_valid) {
     DN_TRY(products_for(h));
@@ -652,6 +739,7 @@ DN_API int dnpeff_nmf_sparsify_W(dnpeff_nmf* nmf, float l1_norm, float l2_norm, 
   clear_error();
   DN_CHECK(nmf, "NULL argument");
   // (H^T H and A H^T kept between calls depend on H only)
+  nmf->fu.gw_state = fused_state::NONE;
   return sparsify_columns(nmf->n, nmf->r, nmf->W, l1_norm, l2_norm, rounds);
 }
 

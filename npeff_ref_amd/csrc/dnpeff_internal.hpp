@@ -256,6 +256,26 @@ struct col_blocks {
   std::vector<int64_t> h_first;  // first block of every aligned group of 64 columns
 };
 
+// Work lists of the step of small ranks (fused.hip): tiles of columns with their entries packed as
+// (row, column within its aligned group of 256; value), and chunks of the rows' entries.
+struct fu_tile {
+  int64_t e0;  // first entry
+  int32_t col0, cols;
+};
+struct fu_chunk {
+  int64_t e0;
+  int32_t len, row;
+};
+struct fused_plan {
+  fu_tile* tiles = nullptr;  // [n_tiles + 1]: the last one only ends the entries
+  int64_t n_tiles = 0;
+  int tile_cols = 0;
+  uint2* pairs = nullptr;    // [nnz + 1]
+  fu_chunk* chunks = nullptr;
+  int64_t n_chunks = 0;
+  int* n_base = nullptr;     // [n_rows + 1] first chunk of each row
+};
+
 }  // namespace dn
 
 struct dnpeff_csr {
@@ -315,6 +335,7 @@ struct dnpeff_csr {
   dn::col_blocks tb;
   dn::dense_head head;
   dnpeff_csr* tail = nullptr;
+  dn::fused_plan fused;
   // host copies of head.cols and long_cols (ascending), made when a product runs on column tiles
   std::vector<int32_t> h_head_cols, h_long_cols;
   bool h_lists_valid = false;
@@ -382,6 +403,7 @@ int nlists_get_row(const dnpeff_csr* S, int64_t row, std::vector<int32_t>& cols,
 bool tlists_supported(const dnpeff_csr* S, int r);
 int tblocks_build(dnpeff_csr* S);
 void tblocks_drop(dnpeff_csr* S);
+void fused_drop(dnpeff_csr* S);  // fused.hip
 int launch_spmm_t_lists(const dnpeff_csr* S, int r, const float* W_nr, float* T, int64_t col0, int64_t col1);
 // Whether the products of the sparse part S at rank r run from the slot lists / column blocks.
 bool use_nlists(const dnpeff_csr* S, int r);       // the whole sparse part on slot lists

@@ -1,0 +1,917 @@
+// The factorisation step at ranks up to FUSED_MAX_RANK: three or four launches per iteration.
+//
+//   k_fu_n     A H^T as sums over chunks of a row's entries; its first workgroups sum the partial
+//              Gram matrices of H that the last H update left
+//   k_fu_w     W update: chunk sums, W G_H, the multiplicative update, and W^T W of the new W
+//   k_fu_sum   sums the partial Gram matrices of W (only where there are more than a few)
+//   k_fu_h     H update: A^T W of 64 columns gathered into LDS, H G_W, the update, and H^T H of the
+//              new H; A^T W never goes through memory and H is read once and written once
+//
+// The separate kernels move five times the factor per H update (A^T W written and read, H read twice,
+// written once) and need some ten launches per iteration, which is what bounds small problems.
+//
+// Matrix products run on the fp32 matrix cores (v_mfma_f32_16x16x4f32) with the factor's row as column
+// operand: lane (j = l % 16, g = l / 16) holds components 16 b + 4 g + i of row j, which is both what
+// the instruction wants as operand (with the contraction index permuted alike on both sides) and how
+// it returns the product.  A rank that is not a multiple of 16 leaves rem components in the last
+// block: they are dealt R = ceil(rem / 4) to a lane, so that the block takes R instead of four
+// contraction steps.  Rows are read and written with 16-byte accesses whatever the rank (global memory
+// needs no more than 4-byte alignment); the arrays end with four spare floats.
+//
+// All sums run in an order that the matrix and the launch shape fix: runs repeat bit for bit.
+#include "fused.hpp"
+
+#include <algorithm>
+
+namespace dn {
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+
+constexpr int FU_ROWS_WG = 64;       // rows of a workgroup of the W update
+constexpr int FU_GROUP = 256;        // columns whose entries are packed with one base
+constexpr int FU_ROW_BITS = 24;      // a packed entry: row below, column within its 256 above
+constexpr int FU_U = 8;              // gathers in flight per lane group of A H^T
+constexpr int FU_U_H = 2;            // the same in the H update, where a lane takes two pieces of a row
+constexpr int FU_SUM_DIRECT = 4;     // partial Gram matrices that their reader sums by itself
+
+__host__ __device__ constexpr int fu_blocks(int Q, int R) { return Q + (R ? 1 : 0); }
+__host__ __device__ constexpr int fu_pairs(int nb) { return nb * (nb + 1) / 2; }
+// Lanes that cover a row of W with two 16-byte pieces each.
+__host__ __device__ constexpr int fu_lpr(int Q, int R) {
+  return 16 * Q + 4 * R <= 8 ? 1 : 16 * Q + 4 * R <= 16 ? 2 : 16 * Q + 4 * R <= 32 ? 4 : 8;
+}
+__device__ inline int fu_pair(int b1, int b2, int nb) { return b1 * nb - b1 * (b1 - 1) / 2 + (b2 - b1); }
+
+// G as the A operand of the products: [block b of output components][contraction block q][lane][i].
+// part: n_parts partial matrices of packed upper block pairs ([pair][16][16]).
+template <int Q, int R>
+__device__ inline void fu_load_g(const float* __restrict__ part, int n_parts, int r, float* __restrict__ ga) {
+  constexpr int NB = fu_blocks(Q, R), S = fu_pairs(NB) * 256;
+  for (int x = threadIdx.x; x < NB * NB * 256; x += 256) {
+    const int i = x & 3, lane = (x >> 2) & 63, q = (x >> 8) % NB, b = (x >> 8) / NB;
+    const int rho = lane & 15, g = lane >> 4;
+    int k, c;
+    bool ok = true;
+    if (R == 0 || q < Q) k = 16 * q + 4 * g + i;
+    else { k = 16 * Q + R * g + i; ok = i < R; }
+    if (R == 0 || b < Q) c = 16 * b + rho;
+    else { c = 16 * Q + R * (rho >> 2) + (rho & 3); ok = ok && (rho & 3) < R; }
+    ok = ok && k < r && c < r;
+    float v = 0.0f;
+    if (ok) {
+      const int bk = k >> 4, bc = c >> 4;
+      const int at = bk <= bc ? fu_pair(bk, bc, NB) * 256 + (k & 15) * 16 + (c & 15)
+                              : fu_pair(bc, bk, NB) * 256 + (c & 15) * 16 + (k & 15);
+      double s = 0.0;
+      for (int p = 0; p < n_parts; p++) s += (double)part[(int64_t)p * S + at];
+      v = (float)s;
+    }
+    ga[x] = v;
+  }
+}
+
+// The components of one factor row that a lane holds: x[b][i] = row[component(b, g, i)], zero past r.
+template <int Q, int R>
+__device__ inline void fu_load_row(const float* __restrict__ row, int g, int r, f32x4 (&x)[fu_blocks(Q, R)]) {
+  constexpr int NB = fu_blocks(Q, R);
+#pragma unroll
+  for (int b = 0; b < Q; b++) {
+    x[b] = *reinterpret_cast<const f32x4u*>(row + 16 * b + 4 * g);
+    if (R == 0 && b == Q - 1) {
+#pragma unroll
+      for (int i = 0; i < 4; i++) x[b][i] = 16 * b + 4 * g + i < r ? x[b][i] : 0.0f;
+    }
+  }
+  if constexpr (R > 0) {
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const int c = 16 * Q + R * g + i;
+      x[NB - 1][i] = i < R && c < r ? row[c] : 0.0f;
+    }
+  }
+}
+
+// X G, the update and the new row for the 16 rows of a wave.  t: the numerators of the lane's row, laid
+// out as x.  The new rows go to `dst` (global, if store) and into the wave's part of the LDS tile
+// ([row][component], stride TS), from where they enter the Gram products.
+template <int Q, int R>
+__device__ inline void fu_update(const float* __restrict__ ga, f32x4 (&x)[fu_blocks(Q, R)],
+                                 const f32x4 (&t)[fu_blocks(Q, R)], float eps, int r, bool store,
+                                 float* __restrict__ dst, float* __restrict__ tile_row) {
+  constexpr int NB = fu_blocks(Q, R);
+  const int lane = threadIdx.x & 63, g = lane >> 4;
+  f32x4 d[NB];
+#pragma unroll
+  for (int b = 0; b < NB; b++) d[b] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+  for (int q = 0; q < NB; q++) {
+#pragma unroll
+    for (int b = 0; b < NB; b++) {
+      const f32x4 a = *reinterpret_cast<const f32x4*>(ga + ((b * NB + q) * 64 + lane) * 4);
+#pragma unroll
+      for (int i = 0; i < (q < Q ? 4 : R); i++)
+        d[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], x[q][i], d[b], 0, 0, 0);
+    }
+  }
+#pragma unroll
+  for (int b = 0; b < NB; b++) {
+    f32x4 y;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const int c = b < Q ? 16 * b + 4 * g + i : 16 * Q + R * g + i;
+      // reciprocal and one correction step: within an ulp of the division
+      const float den = d[b][i] + eps, inv = __builtin_amdgcn_rcpf(den), q0 = t[b][i] * inv;
+      const float v = x[b][i] * fmaf(fmaf(-q0, den, t[b][i]), inv, q0);
+      const bool in = R > 0 ? b < Q || (i < R && c < r) : b < Q - 1 || c < r;
+      y[i] = store && in ? v : 0.0f;
+    }
+    if (b < Q) {
+      *reinterpret_cast<f32x4*>(tile_row + 16 * b + 4 * g) = y;
+      if (store) {
+        if (R > 0 || b < Q - 1 || 16 * b + 4 * g + 3 < r) *reinterpret_cast<f32x4u*>(dst + 16 * b + 4 * g) = y;
+        else {
+#pragma unroll
+          for (int i = 0; i < 4; i++)
+            if (16 * b + 4 * g + i < r) dst[16 * b + 4 * g + i] = y[i];
+        }
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < R; i++) {
+        const int c = 16 * Q + R * g + i;
+        tile_row[c] = y[i];
+        if (store && c < r) dst[c] = y[i];
+      }
+    }
+  }
+}
+
+// acc += the Gram blocks of the 16 rows of the wave's part of the tile.
+template <int NB>
+__device__ inline void fu_gram(const float* __restrict__ rows, int ts, f32x4 (&acc)[fu_pairs(NB)]) {
+  const int lane = threadIdx.x & 63, l16 = lane & 15, g = lane >> 4;
+#pragma unroll
+  for (int s = 0; s < 4; s++) {
+    float a[NB];
+#pragma unroll
+    for (int b = 0; b < NB; b++) a[b] = rows[(4 * s + g) * ts + 16 * b + l16];
+    int p = 0;
+#pragma unroll
+    for (int b1 = 0; b1 < NB; b1++)
+#pragma unroll
+      for (int b2 = b1; b2 < NB; b2++, p++)
+        acc[p] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[b1], a[b2], acc[p], 0, 0, 0);
+  }
+}
+
+// The four waves' Gram blocks, added in wave order, to out ([pair][16][16]); lds: NP * 256 floats.
+template <int NP>
+__device__ inline void fu_gram_out(const f32x4 (&acc)[NP], float* __restrict__ lds, float* __restrict__ out) {
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, l16 = lane & 15, g = lane >> 4;
+  for (int w = 0; w < 4; w++) {
+    __syncthreads();
+    if (wave == w) {
+#pragma unroll
+      for (int p = 0; p < NP; p++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          float* at = lds + p * 256 + (4 * g + i) * 16 + l16;
+          *at = w == 0 ? acc[p][i] : *at + acc[p][i];
+        }
+    }
+  }
+  __syncthreads();
+  for (int x = threadIdx.x; x < NP * 256; x += 256) out[x] = lds[x];
+}
+
+// ---------------------------------------------------------------------------
+// H update.  A tile is up to TC = 64 JB columns that share one aligned group of TC, with up to 16 TC
+// entries (or one longer column); every wave has 16 JB of the group's columns.  The tile's entries,
+// column by column, are cut into equal shares for the lane groups of LPR lanes (16 bytes of a row of W
+// per lane); a group adds the entries of a column up in registers and stores the sum to the tile when
+// the column ends.  Columns hold 1 to n entries with a few on average, so whole columns per group would
+// leave most groups waiting for the longest one (a group walked up to 256 entries by itself: 110 us
+// at 300 rows); a column cut by a share's end leaves its later parts in `carry`, one per group, and
+// whoever reads the column adds them in order.  U gathers per group are in flight, the pairs of the
+// next U are requested behind them, and a tile's first pairs and offsets while the products of the
+// tile before run: without that a tile is a chain of five dependent trips to memory.
+//
+// Bound by vector and matrix instructions (at r = 50 about 80 and 65 us of the SIMDs' time), not by
+// memory: hence 32 bytes per lane and gathered row (the index arithmetic and the test for the column's
+// end are shared by eight components; with 16 bytes the r = 50 step took 335 us, now 316), 24-bit
+// multiplies into 32-bit offsets and the corrected reciprocal in place of the division sequence
+// (390 -> 335 us with it).  777 x 862k, r = 50: 181 us for 2.0 GFLOP of gathers and 12.9 of products
+// (922 us for A^T W, update and Gram as separate kernels); 512 x 431k, r = 16: 31 us (139).
+// ---------------------------------------------------------------------------
+template <int Q, int R, int JB>
+__global__ void __launch_bounds__(256, fu_blocks(Q, R) <= 2 ? 4 : 3)
+    k_fu_h(const fu_tile* __restrict__ tiles, int n_tiles, const int64_t* __restrict__ colptr,
+           const uint2* __restrict__ pairs, int r, const float* __restrict__ W, float* __restrict__ H, float eps,
+           const float* __restrict__ gw, int n_gw, float* __restrict__ gpart) {
+  constexpr int NB = fu_blocks(Q, R), NP = fu_pairs(NB), TS = 16 * NB + 4, TC = 64 * JB;
+  constexpr int LPR = fu_lpr(Q, R), NG = 256 / LPR, U = FU_U_H;
+  constexpr int CARRY = TC * TS;  // carry[NG][8 LPR] behind the tile
+  constexpr int T_FLOATS = CARRY + 2048 > NP * 256 ? CARRY + 2048 : NP * 256;
+  constexpr bool WHOLE = 8 * LPR <= 16 * NB;  // both pieces of a lane lie within the padded row
+  __shared__ __align__(16) float ga[NB * NB * 256];
+  __shared__ __align__(16) float tile[T_FLOATS];
+  __shared__ int cps[2][TC + 1];
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int l16 = lane & 15, g = lane >> 4;
+  const int grp = tid / LPR, sub = tid % LPR;
+  f32x4 acc[NP];
+#pragma unroll
+  for (int p = 0; p < NP; p++) acc[p] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  // components 4 sub .. and 4 (sub + LPR) .. (pieces past the rank: any valid address)
+  const unsigned r4 = 4u * (unsigned)r, off0 = 4 * sub < r ? 16u * (unsigned)sub : 0u,
+                 off1 = 4 * (sub + LPR) < r ? 16u * (unsigned)(sub + LPR) : 0u;
+  const char* Wb = reinterpret_cast<const char*>(W);
+
+  struct tile_at {
+    int64_t e0;
+    int col0, nc, E, share;
+  };
+  auto describe = [&](int t) {
+    tile_at d;
+    if (t >= n_tiles) t = n_tiles - 1;
+    d.e0 = tiles[t].e0;
+    d.col0 = tiles[t].col0;
+    d.nc = tiles[t].cols;
+    d.E = (int)(tiles[t + 1].e0 - d.e0);
+    d.share = (d.E + NG - 1) / NG;
+    return d;
+  };
+  uint2 pr[U];
+  unsigned before;
+  int64_t cpv[JB];
+  auto request = [&](const tile_at& d) {
+    const uint2* pp = pairs + d.e0;
+    const int s0 = grp * d.share;
+    const unsigned last = d.E > 0 ? (unsigned)(d.E - 1) : 0u;  // (the array has a spare entry)
+    before = pp[s0 > 0 && (unsigned)s0 <= last ? (unsigned)(s0 - 1) : 0u].x;
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const unsigned e = (unsigned)(s0 + u), end = (unsigned)(s0 + d.share - 1) < last ? (unsigned)(s0 + d.share - 1) : last;
+      pr[u] = pp[e < end ? e : end];
+    }
+#pragma unroll
+    for (int k = 0; k < JB; k++) {
+      const int at = tid + 256 * k;
+      cpv[k] = colptr[d.col0 + (at < d.nc ? at : d.nc)];
+    }
+  };
+  tile_at td = describe(blockIdx.x);
+  request(td);
+  fu_load_g<Q, R>(gw, n_gw, r, ga);
+
+  int par = 0;
+  for (int tl = blockIdx.x; tl < n_tiles; tl += gridDim.x, par ^= 1) {
+    const int l0 = td.col0 & (TC - 1);
+    const int nc = td.nc, share = td.share, E = td.E;
+    int* cp = cps[par];
+#pragma unroll
+    for (int k = 0; k < JB; k++) {
+      const int at = tid + 256 * k;
+      if (at <= nc) cp[l0 + at] = (int)(cpv[k] - td.e0);
+    }
+    const tile_at nd = describe(tl + gridDim.x);
+    // the wave's rows of H
+    const int64_t base = td.col0 - l0;
+    float* Hb = H + base * r;
+    f32x4 h[JB][NB];
+    bool mine[JB];
+    unsigned hoff[JB];
+#pragma unroll
+    for (int jb = 0; jb < JB; jb++) {
+      const int jl = 16 * (JB * wave + jb) + l16;
+      mine[jb] = jl >= l0 && jl < l0 + nc;
+      hoff[jb] = (unsigned)(mine[jb] ? jl : l0) * (unsigned)r;
+      fu_load_row<Q, R>(Hb + hoff[jb], g, r, h[jb]);
+    }
+
+    // gather
+    const int s0 = grp * share, s1 = s0 + share < E ? s0 + share : E;
+    if (s0 < s1) {
+      const uint2* pp = pairs + td.e0;
+      unsigned cur = pr[0].x;
+      int dst = s0 > 0 && ((cur ^ before) >> FU_ROW_BITS) == 0 ? CARRY + grp * (8 * LPR)
+                                                               : (int)((cur >> FU_ROW_BITS) & (TC - 1)) * TS;
+      dst += 4 * sub;
+      f32x4 a0 = f32x4{0.0f, 0.0f, 0.0f, 0.0f}, a1 = a0;
+      auto put = [&]() {
+        *reinterpret_cast<f32x4*>(tile + dst) = a0;
+        if (WHOLE || 4 * (sub + LPR) < 16 * NB) *reinterpret_cast<f32x4*>(tile + dst + 4 * LPR) = a1;
+      };
+      for (int b = s0; b < s1; b += U) {
+        f32x4 w0[U], w1[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+          const unsigned at = __umul24(pr[u].x & ((1u << FU_ROW_BITS) - 1u), r4);
+          w0[u] = *reinterpret_cast<const f32x4u*>(Wb + (at + off0));
+          w1[u] = *reinterpret_cast<const f32x4u*>(Wb + (at + off1));
+        }
+        uint2 nx[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+          const unsigned e = (unsigned)(b + U + u), end = (unsigned)(s1 - 1);
+          nx[u] = pp[e < end ? e : end];
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+          const float v = b + u < s1 ? __uint_as_float(pr[u].y) : 0.0f;
+          if (((pr[u].x ^ cur) >> FU_ROW_BITS) != 0) {
+            put();
+            cur = pr[u].x;
+            dst = (int)((cur >> FU_ROW_BITS) & (TC - 1)) * TS + 4 * sub;
+            a0 = a1 = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+          }
+#pragma unroll
+          for (int i = 0; i < 4; i++) {
+            a0[i] = fmaf(v, w0[u][i], a0[i]);
+            a1[i] = fmaf(v, w1[u][i], a1[i]);
+          }
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) pr[u] = nx[u];
+      }
+      put();
+    }
+    request(nd);
+    __syncthreads();
+
+    const float inv = 1.0f / (float)(share > 0 ? share : 1);
+#pragma unroll
+    for (int jb = 0; jb < JB; jb++) {
+      const int first = 16 * (JB * wave + jb);
+      if (first + 15 < l0 || first >= l0 + nc) continue;
+      f32x4 t[NB];
+      float* trow = tile + (first + l16) * TS;
+      const int a0 = mine[jb] ? cp[first + l16] : 0, a1 = mine[jb] ? cp[first + l16 + 1] : 0;
+      const bool some = a1 > a0;
+#pragma unroll
+      for (int b = 0; b < Q; b++) t[b] = *reinterpret_cast<const f32x4*>(trow + 16 * b + 4 * g);
+      if constexpr (R > 0) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) t[NB - 1][i] = i < R ? trow[16 * Q + R * g + i] : 0.0f;
+      }
+#pragma unroll
+      for (int b = 0; b < NB; b++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) t[b][i] = some ? t[b][i] : 0.0f;
+      // shares that start inside the column: floor(a0 / share) + 1 ... floor((a1 - 1) / share)
+      // (exact: entries per tile stay below 2^22, or the quotient is corrected)
+      auto quot = [&](int x) {
+        int q = (int)((float)x * inv);
+        if (q * share > x) q--;
+        if ((q + 1) * share <= x) q++;
+        return q;
+      };
+      if (some) {
+        const int k1 = quot(a1 - 1);
+        for (int k = quot(a0) + 1; k <= k1; k++) {
+          const float* src = tile + CARRY + k * (8 * LPR);
+#pragma unroll
+          for (int b = 0; b < NB; b++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+              if (b < Q || i < R) t[b][i] += src[b < Q ? 16 * b + 4 * g + i : 16 * Q + R * g + i];
+            }
+        }
+      }
+      fu_update<Q, R>(ga, h[jb], t, eps, r, mine[jb], Hb + hoff[jb], trow);
+      __builtin_amdgcn_wave_barrier();
+      fu_gram<NB>(tile + first * TS, TS, acc);
+    }
+    td = nd;
+    __syncthreads();  // (the tile has been read)
+  }
+  fu_gram_out<NP>(acc, tile, gpart + (int64_t)blockIdx.x * (NP * 256));
+}
+
+// W update: 64 rows per workgroup.  n_base (or NULL: N holds A H^T itself): first chunk of every row.
+template <int Q, int R>
+__global__ void __launch_bounds__(256)
+    k_fu_w(int64_t n, int r, const int* __restrict__ n_base, const float* __restrict__ N, float* __restrict__ W,
+           float eps, const float* __restrict__ gh, int n_gh, float* __restrict__ gpart) {
+  constexpr int NB = fu_blocks(Q, R), NP = fu_pairs(NB), TS = 16 * NB + 4;
+  constexpr int T_FLOATS = FU_ROWS_WG * TS > NP * 256 ? FU_ROWS_WG * TS : NP * 256;
+  __shared__ __align__(16) float ga[NB * NB * 256];
+  __shared__ __align__(16) float tile[T_FLOATS];
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, l16 = lane & 15, g = lane >> 4;
+  const int64_t row0 = (int64_t)blockIdx.x * FU_ROWS_WG;
+  const int64_t i = row0 + 16 * wave + l16;
+  const bool mine = i < n;
+  f32x4 x[NB], t[NB];
+  float* wrow = W + (mine ? i : row0) * r;
+  fu_load_row<Q, R>(wrow, g, r, x);
+  fu_load_g<Q, R>(gh, n_gh, r, ga);
+#pragma unroll
+  for (int b = 0; b < NB; b++) t[b] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  {
+    const int64_t at = mine ? i : row0;
+    const int64_t k0 = n_base ? n_base[at] : at, k1 = n_base ? n_base[at + 1] : at + 1;
+#pragma unroll 4
+    for (int64_t k = k0; k < k1; k++) {
+      f32x4 p[NB];
+      fu_load_row<Q, R>(N + k * r, g, r, p);
+#pragma unroll
+      for (int b = 0; b < NB; b++) t[b] += p[b];
+    }
+  }
+  f32x4 acc[NP];
+#pragma unroll
+  for (int p = 0; p < NP; p++) acc[p] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  __syncthreads();
+  fu_update<Q, R>(ga, x, t, eps, r, mine, wrow, tile + (16 * wave + l16) * TS);
+  __builtin_amdgcn_wave_barrier();
+  fu_gram<NB>(tile + 16 * wave * TS, TS, acc);
+  fu_gram_out<NP>(acc, tile, gpart + (int64_t)blockIdx.x * (NP * 256));
+}
+
+// Element x of the sum of n_parts partial Gram matrices: 16 elements per workgroup, 16 threads each.
+__device__ inline void fu_sum_parts(const float* __restrict__ part, int n_parts, int S, int block,
+                                    float* __restrict__ out, double* __restrict__ red) {
+  const int x = block * 16 + (threadIdx.x & 15), k = threadIdx.x >> 4;
+  const float* p = part + x;
+  double s = 0.0;
+  int q = k;
+  for (; q + 7 * 16 < n_parts; q += 8 * 16) {
+    float v[8];
+#pragma unroll
+    for (int u = 0; u < 8; u++) v[u] = p[(int64_t)(q + 16 * u) * S];
+#pragma unroll
+    for (int u = 0; u < 8; u++) s += (double)v[u];
+  }
+  for (; q < n_parts; q += 16) s += (double)p[(int64_t)q * S];
+  red[threadIdx.x] = s;
+  __syncthreads();
+  if (threadIdx.x < 16) {
+    for (int u = 1; u < 16; u++) s += red[16 * u + threadIdx.x];
+    out[x] = (float)s;
+  }
+}
+
+__global__ void __launch_bounds__(256)
+    k_fu_sum(const float* __restrict__ part, int n_parts, int S, float* __restrict__ out) {
+  __shared__ double red[256];
+  fu_sum_parts(part, n_parts, S, blockIdx.x, out, red);
+}
+
+// A full Gram matrix [r, r] as one packed partial.
+__global__ void __launch_bounds__(256) k_fu_pack(const float* __restrict__ G, int r, int nb, float* __restrict__ out) {
+  int p = blockIdx.x, b1 = 0;
+  while (p >= nb - b1) p -= nb - b1, b1++;
+  const int b2 = b1 + p;
+  const int a = 16 * b1 + (threadIdx.x >> 4), b = 16 * b2 + (threadIdx.x & 15);
+  out[blockIdx.x * 256 + threadIdx.x] = a < r && b < r ? G[(int64_t)a * r + b] : 0.0f;
+}
+
+// A H^T: chunk blockIdx.x - sum_wgs of the entries, all of one row; the wave's lane groups take them
+// round-robin, FU_U gathers each in flight.  Workgroups 0 .. sum_wgs - 1 sum Gram parts instead.
+// 777 x 862k, r = 50: 119 us for 3.9 M gathered rows of 200 bytes, nearly all of which come from the
+// memory-side cache (6.5 TB/s); 141 us as one 4-byte load per lane.
+template <int LPR>
+__global__ void __launch_bounds__(256)
+    k_fu_n(const fu_chunk* __restrict__ chunks, const int32_t* __restrict__ colind, const float* __restrict__ vals,
+           int r, const float* __restrict__ H, float* __restrict__ N, int sum_wgs, const float* __restrict__ part,
+           int n_parts, int S, float* __restrict__ gsum) {
+  __shared__ __align__(16) double red_d[256];
+  if ((int)blockIdx.x < sum_wgs) {
+    fu_sum_parts(part, n_parts, S, blockIdx.x, gsum, red_d);
+    return;
+  }
+  constexpr int G = 64 / LPR;
+  float* red = reinterpret_cast<float*>(red_d);  // [4][4 LPR]
+  const int64_t chunk = blockIdx.x - sum_wgs;
+  const int64_t e0 = chunks[chunk].e0;
+  const int len = chunks[chunk].len;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, sub = lane % LPR, grp = lane / LPR;
+  const bool lane_ok = 4 * sub < r;
+  const float* Hl = H + 4 * sub;
+  const int per = (len + 3) / 4;
+  const int w0 = wave * per, w1 = w0 + per < len ? w0 + per : len;
+  const int32_t* ci = colind + e0;
+  const float* va = vals + e0;
+  f32x4 a = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  if (w0 < w1) {
+    int j[FU_U];
+    float v[FU_U];
+    auto request = [&](int b, int (&jj)[FU_U], float (&vv)[FU_U]) {
+#pragma unroll
+      for (int u = 0; u < FU_U; u++) {
+        const int e = b + u * G + grp, at = e < w1 ? e : w1 - 1;
+        jj[u] = ci[at];
+        vv[u] = va[at];
+      }
+    };
+    request(w0, j, v);
+    for (int b = w0; b < w1; b += FU_U * G) {
+      f32x4 x[FU_U];
+#pragma unroll
+      for (int u = 0; u < FU_U; u++)
+        x[u] = lane_ok ? (f32x4)*reinterpret_cast<const f32x4u*>(Hl + (int64_t)j[u] * r)
+                       : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+      int jn[FU_U];
+      float vn[FU_U];
+      request(b + FU_U * G, jn, vn);
+#pragma unroll
+      for (int u = 0; u < FU_U; u++) {
+        const float w = b + u * G + grp < w1 ? v[u] : 0.0f;
+#pragma unroll
+        for (int i = 0; i < 4; i++) a[i] = fmaf(w, x[u][i], a[i]);
+      }
+#pragma unroll
+      for (int u = 0; u < FU_U; u++) j[u] = jn[u], v[u] = vn[u];
+    }
+  }
+#pragma unroll
+  for (int off = 32; off >= LPR; off >>= 1)
+#pragma unroll
+    for (int i = 0; i < 4; i++) a[i] += __shfl_xor(a[i], off);
+  if (grp == 0) *reinterpret_cast<f32x4*>(red + wave * 4 * LPR + 4 * sub) = a;
+  __syncthreads();
+  if (tid < r) N[chunk * r + tid] = ((red[tid] + red[4 * LPR + tid]) + red[8 * LPR + tid]) + red[12 * LPR + tid];
+}
+
+// Loss: <A H^T, W> over the chunk sums (one partial per workgroup, 64 rows), then with <W^T W, H^T H>.
+__global__ void __launch_bounds__(256)
+    k_fu_dot(int64_t n, int r, const int* __restrict__ n_base, const float* __restrict__ N,
+             const float* __restrict__ W, double* __restrict__ out) {
+  __shared__ double red[256];
+  const int64_t row0 = (int64_t)blockIdx.x * 16, rows = n - row0 < 16 ? n - row0 : 16;
+  double s = 0.0;
+  for (int x = threadIdx.x; x < rows * r; x += 256) {
+    const int64_t i = row0 + x / r;
+    const int c = x % r;
+    const int64_t k0 = n_base ? n_base[i] : i, k1 = n_base ? n_base[i + 1] : i + 1;
+    float t = 0.0f;
+    for (int64_t k = k0; k < k1; k++) t += N[k * r + c];
+    s += (double)t * (double)W[i * r + c];
+  }
+  red[threadIdx.x] = s;
+  __syncthreads();
+  for (int o = 128; o > 0; o >>= 1) {
+    if ((int)threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) out[blockIdx.x] = red[0];
+}
+
+__global__ void __launch_bounds__(256)
+    k_fu_loss(const double* __restrict__ part, int n_parts, int r, const float* __restrict__ gw,
+              const float* __restrict__ gh, double* __restrict__ out2) {
+  __shared__ double red[2][256];
+  double neg = 0.0, pos = 0.0;
+  for (int k = threadIdx.x; k < n_parts; k += 256) neg += part[k];
+  int p = 0;
+  const int nb = (r + 15) / 16;
+  for (int b1 = 0; b1 < nb; b1++)
+    for (int b2 = b1; b2 < nb; b2++, p++) {
+      const int x = p * 256 + threadIdx.x;
+      const int a = 16 * b1 + (threadIdx.x >> 4), b = 16 * b2 + (threadIdx.x & 15);
+      if (a >= r || b >= r) continue;  // (not defined there)
+      const double v = (double)gw[x] * (double)gh[x];
+      pos += b1 == b2 ? v : 2.0 * v;
+    }
+  red[0][threadIdx.x] = neg;
+  red[1][threadIdx.x] = pos;
+  __syncthreads();
+  for (int o = 128; o > 0; o >>= 1) {
+    if ((int)threadIdx.x < o) {
+      red[0][threadIdx.x] += red[0][threadIdx.x + o];
+      red[1][threadIdx.x] += red[1][threadIdx.x + o];
+    }
+    __syncthreads();
+  }
+  if (threadIdx.x < 2) out2[threadIdx.x] = red[threadIdx.x][0];
+}
+
+// ---------------------------------------------------------------------------
+// Plan: tiles and packed entries of A^T W, chunks of A H^T
+// ---------------------------------------------------------------------------
+// Tiles of the aligned group of `tc` columns `grp`: f(first column, columns) for each, in order.
+template <class F>
+__device__ inline void fu_split_group(const int64_t* __restrict__ colptr, int64_t m, int tc, int64_t grp, F&& f) {
+  const int64_t j0 = grp * tc, j1 = j0 + tc < m ? j0 + tc : m, most = 16 * tc;
+  int64_t start = j0, e0 = colptr[j0], before = e0;
+  if (colptr[j1] - e0 <= most) {
+    f(j0, (int)(j1 - j0));
+    return;
+  }
+  for (int64_t j = j0; j < j1; j++) {
+    const int64_t e1 = colptr[j + 1];
+    if (e1 - e0 > most && j > start) {
+      f(start, (int)(j - start));
+      start = j;
+      e0 = before;
+    }
+    before = e1;
+  }
+  f(start, (int)(j1 - start));
+}
+
+__global__ void __launch_bounds__(256)
+    k_fu_count_tiles(const int64_t* __restrict__ colptr, int64_t m, int tc, int64_t groups, int* __restrict__ count) {
+  const int64_t grp = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (grp >= groups) return;
+  int k = 0;
+  fu_split_group(colptr, m, tc, grp, [&](int64_t, int) { k++; });
+  count[grp] = k;
+}
+
+__global__ void __launch_bounds__(256)
+    k_fu_make_tiles(const int64_t* __restrict__ colptr, int64_t m, int tc, int64_t groups,
+                    const int64_t* __restrict__ first, fu_tile* __restrict__ tiles) {
+  const int64_t grp = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (grp >= groups) return;
+  int64_t k = first[grp];
+  fu_split_group(colptr, m, tc, grp, [&](int64_t col, int cols) {
+    tiles[k].e0 = colptr[col];
+    tiles[k].col0 = (int32_t)col;
+    tiles[k].cols = cols;
+    k++;
+  });
+  if (grp == groups - 1) {
+    tiles[k].e0 = colptr[m];
+    tiles[k].col0 = (int32_t)m;
+    tiles[k].cols = 0;
+  }
+}
+
+// A workgroup per 256 columns: the column of an entry from the offsets of its group.
+__global__ void __launch_bounds__(256)
+    k_fu_pack_entries(const int64_t* __restrict__ colptr, const int32_t* __restrict__ rowind,
+                      const float* __restrict__ tvals, int64_t m, int64_t groups, uint2* __restrict__ pairs) {
+  __shared__ int64_t cp[FU_GROUP + 1];
+  for (int64_t grp = blockIdx.x; grp < groups; grp += gridDim.x) {
+    const int64_t j0 = grp * FU_GROUP;
+    __syncthreads();
+    cp[threadIdx.x] = colptr[j0 + threadIdx.x < m ? j0 + threadIdx.x : m];
+    if (threadIdx.x == 0) cp[FU_GROUP] = colptr[j0 + FU_GROUP < m ? j0 + FU_GROUP : m];
+    __syncthreads();
+    const int64_t e1 = cp[FU_GROUP];
+    for (int64_t e = cp[0] + threadIdx.x; e < e1; e += 256) {
+      int lo = 0, hi = FU_GROUP;  // last column that starts at or before e
+      while (hi - lo > 1) {
+        const int mid = (lo + hi) >> 1;
+        if (cp[mid] <= e) lo = mid; else hi = mid;
+      }
+      pairs[e] = make_uint2((unsigned)rowind[e] | ((unsigned)lo << FU_ROW_BITS), __float_as_uint(tvals[e]));
+    }
+  }
+}
+
+__global__ void __launch_bounds__(256)
+    k_fu_make_chunks(const int64_t* __restrict__ rowptr, int64_t n, int64_t chunk, const int64_t* __restrict__ base,
+                     fu_chunk* __restrict__ chunks, int* __restrict__ base32) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i > n) return;
+  base32[i] = (int)base[i];
+  if (i == n) return;
+  int64_t e = rowptr[i];
+  const int64_t e1 = rowptr[i + 1];
+  for (int64_t k = base[i]; k < base[i + 1]; k++, e += chunk) {
+    chunks[k].e0 = e;
+    chunks[k].len = (int32_t)(e1 - e < chunk ? e1 - e : chunk);
+    chunks[k].row = (int32_t)i;
+  }
+}
+
+void fused_drop(dnpeff_csr* S) {
+  fused_plan& f = S->fused;
+  dfree(f.tiles); dfree(f.pairs); dfree(f.chunks); dfree(f.n_base);
+  f = fused_plan();
+}
+
+// Columns per tile: 256, 128 or 64 by the rank (a tile of the factor of about 16 KB; fewer columns
+// would leave a workgroup with more trips to memory than work), 64 where larger tiles would leave
+// compute units without one.
+static int fu_tile_cols(int64_t m, int r) {
+  const int tc = r <= 16 ? 256 : r <= 32 ? 128 : 64;
+  return m >= (int64_t)tc * 2 * n_cus() ? tc : 64;
+}
+
+int fused_plan_build(dnpeff_csr* S, int r) {
+  fused_plan& f = S->fused;
+  hipStream_t st = stream();
+  const int tc = fu_tile_cols(S->n_cols, r);
+  if (!f.pairs) {
+    DN_CHECK(S->colptr && S->n_cols > 0, "matrix has no transposed copy");
+    const int64_t groups = ceil_div(S->n_cols, FU_GROUP);
+    DN_TRY(dmalloc(&f.pairs, S->nnz + 1));
+    hipLaunchKernelGGL(k_fu_pack_entries, dim3((unsigned)std::min<int64_t>(groups, 1 << 20)), dim3(256), 0, st,
+                       S->colptr, S->rowind, S->tvals, S->n_cols, groups, f.pairs);
+    DN_LAUNCH_CHECK();
+  }
+  if (!f.tiles || f.tile_cols != tc) {
+    const int64_t m = S->n_cols, groups = ceil_div(m, tc);
+    dbuf<int> count;
+    dbuf<int64_t> first;
+    DN_TRY(count.alloc(groups));
+    DN_TRY(first.alloc(groups + 1));
+    const dim3 grid((unsigned)ceil_div(groups, 256)), block(256);
+    hipLaunchKernelGGL(k_fu_count_tiles, grid, block, 0, st, S->colptr, m, tc, groups, count.p);
+    DN_LAUNCH_CHECK();
+    DN_TRY(scan_counts_i64(count, groups, first));
+    int64_t n_tiles = 0;
+    DN_HIP(hipMemcpyAsync(&n_tiles, first + groups, sizeof(int64_t), hipMemcpyDeviceToHost, st));
+    DN_HIP(hipStreamSynchronize(st));
+    dfree(f.tiles);
+    f.tiles = nullptr;
+    DN_TRY(dmalloc(&f.tiles, n_tiles + 1));
+    f.n_tiles = n_tiles;
+    f.tile_cols = tc;
+    hipLaunchKernelGGL(k_fu_make_tiles, grid, block, 0, st, S->colptr, m, tc, groups, first.p, f.tiles);
+    DN_LAUNCH_CHECK();
+  }
+  if (!f.chunks && S->n_panels == 0) {
+    DN_CHECK(has_row_major(S), "row-major copy of the matrix was released");
+    // entries per workgroup of A H^T: about FU_CHUNKS workgroups in all, at least 256 entries each
+    int64_t chunk = ceil_div(ceil_div(S->nnz, FU_CHUNKS), 256) * 256;
+    if (chunk < 256) chunk = 256;
+    dbuf<int64_t> base;
+    DN_TRY(base.alloc(S->n_rows + 1));
+    DN_TRY(scan_row_chunks(S->rowptr, chunk, S->n_rows, base));
+    DN_HIP(hipMemcpyAsync(&f.n_chunks, base + S->n_rows, sizeof(int64_t), hipMemcpyDeviceToHost, st));
+    DN_HIP(hipStreamSynchronize(st));
+    DN_TRY(dmalloc(&f.chunks, f.n_chunks));
+    DN_TRY(dmalloc(&f.n_base, S->n_rows + 1));
+    hipLaunchKernelGGL(k_fu_make_chunks, dim3((unsigned)ceil_div(S->n_rows + 1, 256)), dim3(256), 0, st, S->rowptr,
+                       S->n_rows, chunk, base.p, f.chunks, f.n_base);
+    DN_LAUNCH_CHECK();
+  }
+  return 0;
+}
+
+// ---------------------------------------------------------------------------
+// Launchers
+// ---------------------------------------------------------------------------
+template <int Q_, int R_>
+struct fu_tag {
+  static constexpr int Q = Q_, R = R_;
+};
+
+template <class F>
+static int fu_dispatch(int r, F&& f) {
+  int q = r / 16, rem = (r % 16 + 3) / 4;
+  if (rem == 4) q++, rem = 0;
+  switch (4 * q + rem) {
+#define DN_FU(Q, R) \
+  case 4 * Q + R: return f(fu_tag<Q, R>{});
+    DN_FU(0, 1) DN_FU(0, 2) DN_FU(0, 3)
+    DN_FU(1, 0) DN_FU(1, 1) DN_FU(1, 2) DN_FU(1, 3)
+    DN_FU(2, 0) DN_FU(2, 1) DN_FU(2, 2) DN_FU(2, 3)
+    DN_FU(3, 0) DN_FU(3, 1) DN_FU(3, 2) DN_FU(3, 3)
+    DN_FU(4, 0)
+#undef DN_FU
+  }
+  DN_CHECK(false, "rank %d has no fused step", r);
+}
+
+int fused_gram_floats(int r) { return fu_pairs((r + 15) / 16) * 256; }
+static int fu_blocks_of(int r) { return (r + 15) / 16; }
+
+using fu_h_kernel = void (*)(const fu_tile*, int, const int64_t*, const uint2*, int, const float*, float*, float,
+                             const float*, int, float*);
+
+template <int Q, int R>
+static fu_h_kernel fu_h_of(int tile_cols) {
+  constexpr int NB = fu_blocks(Q, R);
+  if constexpr (NB == 1) return tile_cols == 256 ? k_fu_h<Q, R, 4> : k_fu_h<Q, R, 1>;
+  else if constexpr (NB == 2) return tile_cols == 128 ? k_fu_h<Q, R, 2> : k_fu_h<Q, R, 1>;
+  else return k_fu_h<Q, R, 1>;
+}
+
+int fused_state::create(const dnpeff_csr* S, int64_t n, int rank) {
+  r = rank;
+  S_floats = fused_gram_floats(r);
+  const fused_plan& f = S->fused;
+  int per_cu = 0;
+  DN_TRY(fu_dispatch(r, [&](auto tag) {
+    DN_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(
+        &per_cu, fu_h_of<decltype(tag)::Q, decltype(tag)::R>(f.tile_cols), 256, 0));
+    return 0;
+  }));
+  const int64_t most = (int64_t)n_cus() * (per_cu > 0 ? per_cu : 1);
+  h_wgs = (int)(f.n_tiles < most ? f.n_tiles : most);
+  w_wgs = (int)ceil_div(n, FU_ROWS_WG);
+  DN_TRY(dmalloc(&gh_part, (int64_t)h_wgs * S_floats));
+  DN_TRY(dmalloc(&gw_part, (int64_t)w_wgs * S_floats));
+  DN_TRY(dmalloc(&gh_sum, S_floats));
+  DN_TRY(dmalloc(&gw_sum, S_floats));
+  DN_TRY(dmalloc(&dots, ceil_div(n, 16)));
+  return 0;
+}
+
+void fused_state::destroy() {
+  dfree(gh_part); dfree(gw_part); dfree(gh_sum); dfree(gw_sum); dfree(dots); dfree(n_part);
+  *this = fused_state();
+}
+
+static int fu_sum(const float* part, int n_parts, int S, float* out) {
+  hipLaunchKernelGGL(k_fu_sum, dim3((unsigned)(S / 16)), dim3(256), 0, stream(), part, n_parts, S, out);
+  DN_LAUNCH_CHECK();
+  return 0;
+}
+
+int fused_state::set_gram(const float* G, bool of_h) {
+  const int nb = fu_blocks_of(r);
+  hipLaunchKernelGGL(k_fu_pack, dim3((unsigned)fu_pairs(nb)), dim3(256), 0, stream(), G, r, nb, of_h ? gh_sum : gw_sum);
+  DN_LAUNCH_CHECK();
+  (of_h ? gh_state : gw_state) = SUMMED;
+  return 0;
+}
+
+int fused_state::product_n(const dnpeff_csr* S, const float* H) {
+  const fused_plan& f = S->fused;
+  DN_CHECK(has_row_major(S) && f.chunks, "row-major copy of the matrix was released");
+  if (n_part_floats < f.n_chunks * r + 4) {
+    dfree(n_part);
+    n_part = nullptr;
+    n_part_floats = f.n_chunks * r + 4;
+    DN_TRY(dmalloc(&n_part, n_part_floats));
+  }
+  const int sums = gh_state == PARTS ? S_floats / 16 : 0;
+  const dim3 grid((unsigned)(f.n_chunks + sums)), block(256);
+  if (grid.x > 0) {
+#define DN_FU_N(LPR)                                                                                                \
+  hipLaunchKernelGGL((k_fu_n<LPR>), grid, block, 0, stream(), f.chunks, S->colind, S->vals, r, H, n_part, sums, gh_part, \
+                     h_wgs, S_floats, gh_sum)
+    if (r <= 8) DN_FU_N(2);
+    else if (r <= 16) DN_FU_N(4);
+    else if (r <= 32) DN_FU_N(8);
+    else DN_FU_N(16);
+#undef DN_FU_N
+    DN_LAUNCH_CHECK();
+  }
+  if (sums) gh_state = SUMMED;
+  return 0;
+}
+
+int fused_state::sum_h() {
+  if (gh_state != PARTS) return 0;
+  DN_TRY(fu_sum(gh_part, h_wgs, S_floats, gh_sum));
+  gh_state = SUMMED;
+  return 0;
+}
+
+int fused_state::sum_w() {
+  if (gw_state != PARTS) return 0;
+  DN_TRY(fu_sum(gw_part, w_wgs, S_floats, gw_sum));
+  gw_state = SUMMED;
+  return 0;
+}
+
+int fused_state::update_w(const dnpeff_csr* S, int64_t n, const float* Nw, float* W, float eps) {
+  DN_CHECK(gh_state == SUMMED, "H^T H is not at hand");
+  const float* N = Nw ? Nw : n_part;
+  const int* base = Nw ? nullptr : S->fused.n_base;
+  DN_TRY(fu_dispatch(r, [&](auto tag) {
+    hipLaunchKernelGGL((k_fu_w<decltype(tag)::Q, decltype(tag)::R>), dim3((unsigned)w_wgs), dim3(256), 0, stream(), n, r,
+                       base, N, W, eps, gh_sum, 1, gw_part);
+    return 0;
+  }));
+  DN_LAUNCH_CHECK();
+  gw_state = PARTS;
+  return 0;
+}
+
+int fused_state::update_h(const dnpeff_csr* S, const float* W, float* H, float eps) {
+  if (gw_state == PARTS && w_wgs > FU_SUM_DIRECT) DN_TRY(sum_w());
+  const float* gw = gw_state == PARTS ? gw_part : gw_sum;
+  const int n_gw = gw_state == PARTS ? w_wgs : 1;
+  const fused_plan& f = S->fused;
+  DN_TRY(fu_dispatch(r, [&](auto tag) {
+    hipLaunchKernelGGL((fu_h_of<decltype(tag)::Q, decltype(tag)::R>(f.tile_cols)), dim3((unsigned)h_wgs), dim3(256), 0,
+                       stream(), f.tiles, (int)f.n_tiles, S->colptr, f.pairs, r, W, H, eps, gw, n_gw, gh_part);
+    return 0;
+  }));
+  DN_LAUNCH_CHECK();
+  gh_state = PARTS;
+  return 0;
+}
+
+int fused_state::loss_sums(const dnpeff_csr* S, int64_t n, const float* Nw, const float* W, double* out2) {
+  DN_TRY(sum_h());
+  DN_TRY(sum_w());
+  const int parts = (int)ceil_div(n, 16);
+  hipLaunchKernelGGL(k_fu_dot, dim3((unsigned)parts), dim3(256), 0, stream(), n, r, Nw ? nullptr : S->fused.n_base,
+                     Nw ? Nw : n_part, W, dots);
+  hipLaunchKernelGGL(k_fu_loss, dim3(1), dim3(256), 0, stream(), dots, parts, r, gw_sum, gh_sum, out2);
+  DN_LAUNCH_CHECK();
+  return 0;
+}
+
+double fused_bytes(int64_t n, int64_t nnz, int r) {
+  const double S = 4.0 * fused_gram_floats(r);
+  return 8.0 * (double)nnz + 16.0 * ((double)nnz / 512.0) + 4.0 * (double)(FU_CHUNKS + n) * (r + 4) +
+         S * ((double)n_cus() * 8.0 + (double)n / FU_ROWS_WG + 3.0);
+}
+
+bool fused_supported(int64_t n, int64_t m, int64_t nnz, int r) {
+  return r >= 1 && r <= FUSED_MAX_RANK && n >= 1 && m >= 1 && nnz >= 1 && n < ((int64_t)1 << FU_ROW_BITS) &&
+         n * (int64_t)r < ((int64_t)1 << 30);  // (byte offsets into W in 32 bits)
+}
+
+}  // namespace dn

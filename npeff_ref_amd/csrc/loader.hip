@@ -736,6 +736,7 @@ static void drop_derived(dnpeff_csr* A) {
   drop_panels(A);
   nlists_drop(A);
   tblocks_drop(A);
+  fused_drop(A);
   dfree(A->colptr); A->colptr = nullptr;
   dfree(A->rowind); A->rowind = nullptr;
   dfree(A->tvals); A->tvals = nullptr;

@@ -1,0 +1,73 @@
+"""The step of small ranks (csrc/fused.hip) against the fp64 oracle: remainders of the rank, tiles cut by
+their number of entries, columns longer than a tile, empty columns and rows, and the changes between it
+and the separate kernels."""
+
+import numpy as np
+import pytest
+
+import npeff_ref_amd as d
+from oracle import oracle as orc
+
+pytestmark = pytest.mark.gpu
+EPS = 1e-8
+
+
+def _matrix(n, m, seed, fill=0.02, full=3, empty_row=True):
+    """Random columns; `full` of them hold every row (but the empty one), every seventh holds none."""
+    rng = np.random.default_rng(seed)
+    mask = rng.random((n, m)) < fill
+    mask[:, :full] = True
+    mask[:, 6::7] = False
+    if empty_row and n > 3:
+        mask[n // 2] = False
+    rowptr = np.concatenate([[0], np.cumsum(mask.sum(axis=1))]).astype(np.int64)
+    colind = np.concatenate([rng.permutation(np.flatnonzero(row)) for row in mask]).astype(np.int32)
+    vals = rng.random(len(colind)).astype(np.float32)
+    return rowptr, colind, vals
+
+
+def _close(nmf, oracle_out):
+    W64, H64, losses = oracle_out
+    for got, want in ((nmf.loadWToHostSync(), W64), (nmf.loadHToHostSync(), H64)):
+        assert np.linalg.norm(got - want) <= 1e-5 * np.linalg.norm(want)
+    sq, pos, neg = nmf.loss_terms()  # (squared, against ||A||^2: a run may end on an exact product)
+    assert abs(sq + pos - 2 * neg - losses[-1] ** 2) <= 1e-5 * sq
+
+
+@pytest.mark.parametrize("n,m,r", [(1, 1, 1), (2, 63, 3), (5, 64, 4), (33, 65, 5), (70, 300, 8), (65, 257, 12),
+                                   (40, 515, 13), (64, 1000, 16), (90, 130, 17), (1500, 1600, 20), (50, 129, 31),
+                                   (130, 700, 33), (30, 64, 44), (77, 333, 50), (2100, 2200, 61), (63, 191, 64)])
+def test_step_matches_the_oracle(n, m, r):
+    rp, ci, va = _matrix(n, m, seed=n + r, fill=0.3 if n < 100 else 0.02)
+    A = d.Csr.from_host(rp, ci, va, m)
+    nmf = d.MuNmf(A, d.MuNmfParams(rank=r, max_iters=6, eps=EPS, seed=5, log_every=3))
+    nmf.initialize()
+    W0, H0 = nmf.loadWToHostSync(), nmf.loadHToHostSync()
+    nmf.run(log=lambda s: None)
+    _close(nmf, orc.nmf_f64(rp, ci, va, m, W0, H0, np.float32(EPS), 6, 3))
+    nmf.close()
+    A.close()
+
+
+@pytest.mark.parametrize("r", [7, 48])
+def test_step_and_separate_kernels_in_turn(r, tune):
+    """A run that changes from the fused step to the separate kernels and back, between and within
+    iterations, keeps no product of an older factor."""
+    n, m = 120, 900
+    rp, ci, va = _matrix(n, m, seed=r, fill=0.05)
+    A = d.Csr.from_host(rp, ci, va, m)
+    nmf = d.MuNmf(A, d.MuNmfParams(rank=r, max_iters=6, eps=EPS, seed=5, log_every=0))
+    nmf.initialize()
+    W0, H0 = nmf.loadWToHostSync(), nmf.loadHToHostSync()
+    want = orc.nmf_f64(rp, ci, va, m, W0, H0, np.float32(EPS), 6, 6)
+    for fused in ((1, 1), (0, 0), (1, 0), (0, 1), (1, 1)):
+        tune("fused_gram", fused[0])
+        nmf.update_W()
+        nmf.computeUncachedLoss()
+        tune("fused_gram", fused[1])
+        nmf.update_H()
+    nmf.set_factors(nmf.loadWToHostSync(), nmf.loadHToHostSync())
+    nmf.step(1)
+    _close(nmf, want)
+    nmf.close()
+    A.close()
