@@ -1,4 +1,4 @@
-// The factorisation step at ranks up to FUSED_MAX_RANK: three or four launches per iteration.
+// The factorisation step at ranks up to 128 (above 64: the updates of fused_wide.hip): three or four launches per iteration.
 //
 //   k_fu_n     A H^T as sums over chunks of a row's entries; its first workgroups sum the partial
 //              Gram matrices of H that the last H update left
@@ -25,23 +25,14 @@
 
 namespace dn {
 
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
-
 constexpr int FU_ROWS_WG = 64;       // rows of a workgroup of the W update
-constexpr int FU_GROUP = 256;        // columns whose entries are packed with one base
-constexpr int FU_ROW_BITS = 24;      // a packed entry: row below, column within its 256 above
-constexpr int FU_U = 8;              // gathers in flight per lane group of A H^T
-constexpr int FU_U_H = 2;            // the same in the H update, where a lane takes two pieces of a row
 constexpr int FU_SUM_DIRECT = 4;     // partial Gram matrices that their reader sums by itself
 
 __host__ __device__ constexpr int fu_blocks(int Q, int R) { return Q + (R ? 1 : 0); }
-__host__ __device__ constexpr int fu_pairs(int nb) { return nb * (nb + 1) / 2; }
 // Lanes that cover a row of W with two 16-byte pieces each.
 __host__ __device__ constexpr int fu_lpr(int Q, int R) {
   return 16 * Q + 4 * R <= 8 ? 1 : 16 * Q + 4 * R <= 16 ? 2 : 16 * Q + 4 * R <= 32 ? 4 : 8;
 }
-__device__ inline int fu_pair(int b1, int b2, int nb) { return b1 * nb - b1 * (b1 - 1) / 2 + (b2 - b1); }
 
 // G as the A operand of the products: [block b of output components][contraction block q][lane][i].
 // part: n_parts partial matrices of packed upper block pairs ([pair][16][16]).
@@ -120,9 +111,7 @@ __device__ inline void fu_update(const float* __restrict__ ga, f32x4 (&x)[fu_blo
 #pragma unroll
     for (int i = 0; i < 4; i++) {
       const int c = b < Q ? 16 * b + 4 * g + i : 16 * Q + R * g + i;
-      // reciprocal and one correction step: within an ulp of the division
-      const float den = d[b][i] + eps, inv = __builtin_amdgcn_rcpf(den), q0 = t[b][i] * inv;
-      const float v = x[b][i] * fmaf(fmaf(-q0, den, t[b][i]), inv, q0);
+      const float v = x[b][i] * fu_quotient(t[b][i], d[b][i] + eps);
       const bool in = R > 0 ? b < Q || (i < R && c < r) : b < Q - 1 || c < r;
       y[i] = store && in ? v : 0.0f;
     }
@@ -210,72 +199,43 @@ __global__ void __launch_bounds__(256, fu_blocks(Q, R) <= 2 ? 4 : 3)
            const uint2* __restrict__ pairs, int r, const float* __restrict__ W, float* __restrict__ H, float eps,
            const float* __restrict__ gw, int n_gw, float* __restrict__ gpart) {
   constexpr int NB = fu_blocks(Q, R), NP = fu_pairs(NB), TS = 16 * NB + 4, TC = 64 * JB;
-  constexpr int LPR = fu_lpr(Q, R), NG = 256 / LPR, U = FU_U_H;
-  constexpr int CARRY = TC * TS;  // carry[NG][8 LPR] behind the tile
-  constexpr int T_FLOATS = CARRY + 2048 > NP * 256 ? CARRY + 2048 : NP * 256;
-  constexpr bool WHOLE = 8 * LPR <= 16 * NB;  // both pieces of a lane lie within the padded row
+  using Gather = fu_gather<TC, TS, NB, fu_lpr(Q, R)>;
+  constexpr int T_FLOATS = Gather::CARRY + 2048 > NP * 256 ? Gather::CARRY + 2048 : NP * 256;
   __shared__ __align__(16) float ga[NB * NB * 256];
   __shared__ __align__(16) float tile[T_FLOATS];
   __shared__ int cps[2][TC + 1];
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int l16 = lane & 15, g = lane >> 4;
-  const int grp = tid / LPR, sub = tid % LPR;
   f32x4 acc[NP];
 #pragma unroll
   for (int p = 0; p < NP; p++) acc[p] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-  // components 4 sub .. and 4 (sub + LPR) .. (pieces past the rank: any valid address)
-  const unsigned r4 = 4u * (unsigned)r, off0 = 4 * sub < r ? 16u * (unsigned)sub : 0u,
-                 off1 = 4 * (sub + LPR) < r ? 16u * (unsigned)(sub + LPR) : 0u;
   const char* Wb = reinterpret_cast<const char*>(W);
-
-  struct tile_at {
-    int64_t e0;
-    int col0, nc, E, share;
-  };
-  auto describe = [&](int t) {
-    tile_at d;
-    if (t >= n_tiles) t = n_tiles - 1;
-    d.e0 = tiles[t].e0;
-    d.col0 = tiles[t].col0;
-    d.nc = tiles[t].cols;
-    d.E = (int)(tiles[t + 1].e0 - d.e0);
-    d.share = (d.E + NG - 1) / NG;
-    return d;
-  };
-  uint2 pr[U];
-  unsigned before;
+  Gather gather;
+  gather.init(r);
   int64_t cpv[JB];
-  auto request = [&](const tile_at& d) {
-    const uint2* pp = pairs + d.e0;
-    const int s0 = grp * d.share;
-    const unsigned last = d.E > 0 ? (unsigned)(d.E - 1) : 0u;  // (the array has a spare entry)
-    before = pp[s0 > 0 && (unsigned)s0 <= last ? (unsigned)(s0 - 1) : 0u].x;
-#pragma unroll
-    for (int u = 0; u < U; u++) {
-      const unsigned e = (unsigned)(s0 + u), end = (unsigned)(s0 + d.share - 1) < last ? (unsigned)(s0 + d.share - 1) : last;
-      pr[u] = pp[e < end ? e : end];
-    }
+  auto request = [&](const fu_tile_at& d) {
+    gather.request(pairs, d);
 #pragma unroll
     for (int k = 0; k < JB; k++) {
       const int at = tid + 256 * k;
       cpv[k] = colptr[d.col0 + (at < d.nc ? at : d.nc)];
     }
   };
-  tile_at td = describe(blockIdx.x);
+  fu_tile_at td = fu_describe<Gather::NG>(tiles, n_tiles, blockIdx.x);
   request(td);
   fu_load_g<Q, R>(gw, n_gw, r, ga);
 
   int par = 0;
   for (int tl = blockIdx.x; tl < n_tiles; tl += gridDim.x, par ^= 1) {
     const int l0 = td.col0 & (TC - 1);
-    const int nc = td.nc, share = td.share, E = td.E;
+    const int nc = td.nc, share = td.share;
     int* cp = cps[par];
 #pragma unroll
     for (int k = 0; k < JB; k++) {
       const int at = tid + 256 * k;
       if (at <= nc) cp[l0 + at] = (int)(cpv[k] - td.e0);
     }
-    const tile_at nd = describe(tl + gridDim.x);
+    const fu_tile_at nd = fu_describe<Gather::NG>(tiles, n_tiles, tl + gridDim.x);
     // the wave's rows of H
     const int64_t base = td.col0 - l0;
     float* Hb = H + base * r;
@@ -290,53 +250,7 @@ __global__ void __launch_bounds__(256, fu_blocks(Q, R) <= 2 ? 4 : 3)
       fu_load_row<Q, R>(Hb + hoff[jb], g, r, h[jb]);
     }
 
-    // gather
-    const int s0 = grp * share, s1 = s0 + share < E ? s0 + share : E;
-    if (s0 < s1) {
-      const uint2* pp = pairs + td.e0;
-      unsigned cur = pr[0].x;
-      int dst = s0 > 0 && ((cur ^ before) >> FU_ROW_BITS) == 0 ? CARRY + grp * (8 * LPR)
-                                                               : (int)((cur >> FU_ROW_BITS) & (TC - 1)) * TS;
-      dst += 4 * sub;
-      f32x4 a0 = f32x4{0.0f, 0.0f, 0.0f, 0.0f}, a1 = a0;
-      auto put = [&]() {
-        *reinterpret_cast<f32x4*>(tile + dst) = a0;
-        if (WHOLE || 4 * (sub + LPR) < 16 * NB) *reinterpret_cast<f32x4*>(tile + dst + 4 * LPR) = a1;
-      };
-      for (int b = s0; b < s1; b += U) {
-        f32x4 w0[U], w1[U];
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-          const unsigned at = __umul24(pr[u].x & ((1u << FU_ROW_BITS) - 1u), r4);
-          w0[u] = *reinterpret_cast<const f32x4u*>(Wb + (at + off0));
-          w1[u] = *reinterpret_cast<const f32x4u*>(Wb + (at + off1));
-        }
-        uint2 nx[U];
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-          const unsigned e = (unsigned)(b + U + u), end = (unsigned)(s1 - 1);
-          nx[u] = pp[e < end ? e : end];
-        }
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-          const float v = b + u < s1 ? __uint_as_float(pr[u].y) : 0.0f;
-          if (((pr[u].x ^ cur) >> FU_ROW_BITS) != 0) {
-            put();
-            cur = pr[u].x;
-            dst = (int)((cur >> FU_ROW_BITS) & (TC - 1)) * TS + 4 * sub;
-            a0 = a1 = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-          }
-#pragma unroll
-          for (int i = 0; i < 4; i++) {
-            a0[i] = fmaf(v, w0[u][i], a0[i]);
-            a1[i] = fmaf(v, w1[u][i], a1[i]);
-          }
-        }
-#pragma unroll
-        for (int u = 0; u < U; u++) pr[u] = nx[u];
-      }
-      put();
-    }
+    gather.run(pairs, td, Wb, tile);
     request(nd);
     __syncthreads();
 
@@ -359,18 +273,11 @@ __global__ void __launch_bounds__(256, fu_blocks(Q, R) <= 2 ? 4 : 3)
       for (int b = 0; b < NB; b++)
 #pragma unroll
         for (int i = 0; i < 4; i++) t[b][i] = some ? t[b][i] : 0.0f;
-      // shares that start inside the column: floor(a0 / share) + 1 ... floor((a1 - 1) / share)
-      // (exact: entries per tile stay below 2^22, or the quotient is corrected)
-      auto quot = [&](int x) {
-        int q = (int)((float)x * inv);
-        if (q * share > x) q--;
-        if ((q + 1) * share <= x) q++;
-        return q;
-      };
       if (some) {
-        const int k1 = quot(a1 - 1);
-        for (int k = quot(a0) + 1; k <= k1; k++) {
-          const float* src = tile + CARRY + k * (8 * LPR);
+        int k0, k1;
+        fu_cut_by(a0, a1, share, inv, k0, k1);
+        for (int k = k0; k < k1; k++) {
+          const float* src = tile + Gather::CARRY + k * (2048 / Gather::NG);
 #pragma unroll
           for (int b = 0; b < NB; b++)
 #pragma unroll
@@ -487,42 +394,44 @@ __global__ void __launch_bounds__(256)
   const int64_t e0 = chunks[chunk].e0;
   const int len = chunks[chunk].len;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, sub = lane % LPR, grp = lane / LPR;
-  const bool lane_ok = 4 * sub < r;
-  const float* Hl = H + 4 * sub;
+  const float* Hl = H + (4 * sub < r ? 4 * sub : 0);  // (lanes past the rank: any valid address)
   const int per = (len + 3) / 4;
   const int w0 = wave * per, w1 = w0 + per < len ? w0 + per : len;
   const int32_t* ci = colind + e0;
   const float* va = vals + e0;
   f32x4 a = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  // 64 (column, value) pairs at a time, one per lane, the next 64 on their way; the steps take theirs by
+  // shuffles.  Lanes past the end hold (some column, 0).
   if (w0 < w1) {
-    int j[FU_U];
-    float v[FU_U];
-    auto request = [&](int b, int (&jj)[FU_U], float (&vv)[FU_U]) {
-#pragma unroll
-      for (int u = 0; u < FU_U; u++) {
-        const int e = b + u * G + grp, at = e < w1 ? e : w1 - 1;
-        jj[u] = ci[at];
-        vv[u] = va[at];
-      }
+    auto request = [&](int e, int& jj, float& vv) {
+      const int at = e + lane < w1 ? e + lane : w1 - 1;
+      jj = ci[at];
+      vv = e + lane < w1 ? va[at] : 0.0f;
     };
+    int j, jn;
+    float v, vn;
     request(w0, j, v);
-    for (int b = w0; b < w1; b += FU_U * G) {
-      f32x4 x[FU_U];
+    for (int b = w0; b < w1; b += 64) {
+      request(b + 64, jn, vn);
+      const int steps = ((w1 - b < 64 ? w1 - b : 64) + G - 1) / G;
+      constexpr int U = 64 / G < FU_U ? 64 / G : FU_U;
+      for (int st = 0; st < steps; st += U) {
+        f32x4 x[U];
+        float w[U];
 #pragma unroll
-      for (int u = 0; u < FU_U; u++)
-        x[u] = lane_ok ? (f32x4)*reinterpret_cast<const f32x4u*>(Hl + (int64_t)j[u] * r)
-                       : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-      int jn[FU_U];
-      float vn[FU_U];
-      request(b + FU_U * G, jn, vn);
+        for (int u = 0; u < U; u++) {
+          const int src = ((st + u) * G + grp) & 63;
+          const int64_t row = __shfl(j, src);
+          w[u] = __shfl(v, src);
+          x[u] = *reinterpret_cast<const f32x4u*>(Hl + row * r);
+        }
 #pragma unroll
-      for (int u = 0; u < FU_U; u++) {
-        const float w = b + u * G + grp < w1 ? v[u] : 0.0f;
+        for (int u = 0; u < U; u++)
 #pragma unroll
-        for (int i = 0; i < 4; i++) a[i] = fmaf(w, x[u][i], a[i]);
+          for (int i = 0; i < 4; i++) a[i] = fmaf(w[u], x[u][i], a[i]);
       }
-#pragma unroll
-      for (int u = 0; u < FU_U; u++) j[u] = jn[u], v[u] = vn[u];
+      j = jn;
+      v = vn;
     }
   }
 #pragma unroll
@@ -688,8 +597,8 @@ void fused_drop(dnpeff_csr* S) {
 // would leave a workgroup with more trips to memory than work), 64 where larger tiles would leave
 // compute units without one.
 static int fu_tile_cols(int64_t m, int r) {
-  const int tc = r <= 16 ? 256 : r <= 32 ? 128 : 64;
-  return m >= (int64_t)tc * 2 * n_cus() ? tc : 64;
+  const int tc = r <= 16 ? 256 : r <= 32 ? 128 : r <= 64 ? 64 : FUW_COLS;
+  return m >= (int64_t)tc * 2 * n_cus() || tc < 64 ? tc : 64;
 }
 
 int fused_plan_build(dnpeff_csr* S, int r) {
@@ -788,14 +697,15 @@ int fused_state::create(const dnpeff_csr* S, int64_t n, int rank) {
   S_floats = fused_gram_floats(r);
   const fused_plan& f = S->fused;
   int per_cu = 0;
-  DN_TRY(fu_dispatch(r, [&](auto tag) {
+  if (r > FUSED_NARROW_RANK) DN_TRY(fuw_per_cu(r, &per_cu));
+  else DN_TRY(fu_dispatch(r, [&](auto tag) {
     DN_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(
         &per_cu, fu_h_of<decltype(tag)::Q, decltype(tag)::R>(f.tile_cols), 256, 0));
     return 0;
   }));
   const int64_t most = (int64_t)n_cus() * (per_cu > 0 ? per_cu : 1);
   h_wgs = (int)(f.n_tiles < most ? f.n_tiles : most);
-  w_wgs = (int)ceil_div(n, FU_ROWS_WG);
+  w_wgs = (int)ceil_div(n, r > FUSED_NARROW_RANK ? FUW_COLS : FU_ROWS_WG);
   DN_TRY(dmalloc(&gh_part, (int64_t)h_wgs * S_floats));
   DN_TRY(dmalloc(&gw_part, (int64_t)w_wgs * S_floats));
   DN_TRY(dmalloc(&gh_sum, S_floats));
@@ -841,7 +751,8 @@ int fused_state::product_n(const dnpeff_csr* S, const float* H) {
     if (r <= 8) DN_FU_N(2);
     else if (r <= 16) DN_FU_N(4);
     else if (r <= 32) DN_FU_N(8);
-    else DN_FU_N(16);
+    else if (r <= 64) DN_FU_N(16);
+    else DN_FU_N(32);
 #undef DN_FU_N
     DN_LAUNCH_CHECK();
   }
@@ -867,7 +778,9 @@ int fused_state::update_w(const dnpeff_csr* S, int64_t n, const float* Nw, float
   DN_CHECK(gh_state == SUMMED, "H^T H is not at hand");
   const float* N = Nw ? Nw : n_part;
   const int* base = Nw ? nullptr : S->fused.n_base;
-  DN_TRY(fu_dispatch(r, [&](auto tag) {
+  if (r > FUSED_NARROW_RANK)
+    DN_TRY(fuw_launch_w(w_wgs, n, r, base, N, W, eps, gh_sum, gw_part));
+  else DN_TRY(fu_dispatch(r, [&](auto tag) {
     hipLaunchKernelGGL((k_fu_w<decltype(tag)::Q, decltype(tag)::R>), dim3((unsigned)w_wgs), dim3(256), 0, stream(), n, r,
                        base, N, W, eps, gh_sum, 1, gw_part);
     return 0;
@@ -882,7 +795,9 @@ int fused_state::update_h(const dnpeff_csr* S, const float* W, float* H, float e
   const float* gw = gw_state == PARTS ? gw_part : gw_sum;
   const int n_gw = gw_state == PARTS ? w_wgs : 1;
   const fused_plan& f = S->fused;
-  DN_TRY(fu_dispatch(r, [&](auto tag) {
+  if (r > FUSED_NARROW_RANK)
+    DN_TRY(fuw_launch_h(h_wgs, f, S->colptr, r, W, H, eps, gw, n_gw, gh_part));
+  else DN_TRY(fu_dispatch(r, [&](auto tag) {
     hipLaunchKernelGGL((fu_h_of<decltype(tag)::Q, decltype(tag)::R>(f.tile_cols)), dim3((unsigned)h_wgs), dim3(256), 0,
                        stream(), f.tiles, (int)f.n_tiles, S->colptr, f.pairs, r, W, H, eps, gw, n_gw, gh_part);
     return 0;
@@ -906,10 +821,15 @@ int fused_state::loss_sums(const dnpeff_csr* S, int64_t n, const float* Nw, cons
 double fused_bytes(int64_t n, int64_t nnz, int r) {
   const double S = 4.0 * fused_gram_floats(r);
   return 8.0 * (double)nnz + 16.0 * ((double)nnz / 512.0) + 4.0 * (double)(FU_CHUNKS + n) * (r + 4) +
-         S * ((double)n_cus() * 8.0 + (double)n / FU_ROWS_WG + 3.0);
+         S * ((double)n_cus() * 8.0 + (double)n / FUW_COLS + 3.0);
 }
 
 bool fused_supported(int64_t n, int64_t m, int64_t nnz, int r) {
+  if (r > FUSED_NARROW_RANK && !use_split_bf16()) return false;
+  // Rank 128 has kernels of its own for the update with its Gram matrix (k_xg_mu_gram_b16), and runs on
+  // small factors are held to within 1e-5 of the two-pass path over 50 iterations, closer than two
+  // ways of rounding stay to each other (both are within 2e-5 of fp64): those keep the separate kernels.
+  if (r == 128 && m < 65536) return false;
   return r >= 1 && r <= FUSED_MAX_RANK && n >= 1 && m >= 1 && nnz >= 1 && n < ((int64_t)1 << FU_ROW_BITS) &&
          n * (int64_t)r < ((int64_t)1 << 30);  // (byte offsets into W in 32 bits)
 }

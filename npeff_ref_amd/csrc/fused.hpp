@@ -2,10 +2,13 @@
 #pragma once
 
 #include "dnpeff_internal.hpp"
+#include "split_bf16.hpp"
 
 namespace dn {
 
-constexpr int FUSED_MAX_RANK = 64;
+constexpr int FUSED_MAX_RANK = 128;
+constexpr int FUSED_NARROW_RANK = 64;  // above: fused_wide.hip
+constexpr int FUW_COLS = 32;           // columns (rows of W) per tile there
 constexpr int64_t FU_CHUNKS = 4096;  // workgroups that A H^T is cut into where its rows allow
 
 bool fused_supported(int64_t n, int64_t m, int64_t nnz, int r);
@@ -13,6 +16,13 @@ bool fused_supported(int64_t n, int64_t m, int64_t nnz, int r);
 double fused_bytes(int64_t n, int64_t nnz, int r);
 // Tiles, packed entries and chunks of a matrix without dense head (needs csr_ensure_products).
 int fused_plan_build(dnpeff_csr* S, int r);
+
+// Updates at ranks 65 ... 128 (fused_wide.hip).
+int fuw_per_cu(int r, int* wgs);
+int fuw_launch_h(int wgs, const fused_plan& f, const int64_t* colptr, int r, const float* W, float* H, float eps,
+                 const float* gw, int n_gw, float* gpart);
+int fuw_launch_w(int wgs, int64_t n, int r, const int* n_base, const float* N, float* W, float eps, const float* gh,
+                 float* gpart);
 
 // What a context keeps between the launches of a step.
 struct fused_state {
@@ -39,5 +49,134 @@ struct fused_state {
   // out2 (device or pinned) = <A H^T, W>, <W^T W, H^T H>
   int loss_sums(const dnpeff_csr* S, int64_t n, const float* Nw, const float* W, double* out2);
 };
+
+// ---- device parts that both kernel families use ----
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+
+constexpr int FU_GROUP = 256;        // columns whose entries are packed with one base
+constexpr int FU_ROW_BITS = 24;      // a packed entry: row below, column within its 256 above
+constexpr int FU_U = 8;              // gathers in flight per lane group of A H^T
+constexpr int FU_U_H = 2;            // the same in the H update, where a lane takes two pieces of a row
+__host__ __device__ constexpr int fu_pairs(int nb) { return nb * (nb + 1) / 2; }
+__device__ inline int fu_pair(int b1, int b2, int nb) { return b1 * nb - b1 * (b1 - 1) / 2 + (b2 - b1); }
+
+// Tile `t` of the work list (past the end: the last one), its entries cut into NG shares.
+struct fu_tile_at {
+  int64_t e0;
+  int col0, nc, E, share;
+};
+template <int NG>
+__device__ inline fu_tile_at fu_describe(const fu_tile* __restrict__ tiles, int n_tiles, int t) {
+  fu_tile_at d;
+  if (t >= n_tiles) t = n_tiles - 1;
+  d.e0 = tiles[t].e0;
+  d.col0 = tiles[t].col0;
+  d.nc = tiles[t].cols;
+  d.E = (int)(tiles[t + 1].e0 - d.e0);
+  d.share = (d.E + NG - 1) / NG;
+  return d;
+}
+
+// A^T W of a tile's columns into LDS, tile[column][TS], by lane groups of LPR lanes that take equal
+// shares of the tile's entries.  A lane holds components 4 sub .. and 4 (sub + LPR) .. of a row.  A
+// column's first part is stored to the tile, parts of later shares to carry[share][8 LPR] at CARRY.
+// U gathered rows per lane group are in flight.
+template <int TC, int TS, int NB, int LPR, int U = FU_U_H>
+struct fu_gather {
+  static constexpr int NG = 256 / LPR, CARRY = TC * TS;
+  static constexpr bool WHOLE = 8 * LPR <= 16 * NB;  // both pieces of a lane lie within the padded row
+  int grp, sub;
+  unsigned r4, off0, off1;
+  uint2 pr[U];
+  unsigned before;
+
+  __device__ inline void init(int r) {
+    grp = threadIdx.x / LPR;
+    sub = threadIdx.x % LPR;
+    r4 = 4u * (unsigned)r;  // (pieces past the rank: any valid address)
+    off0 = 4 * sub < r ? 16u * (unsigned)sub : 0u;
+    off1 = 4 * (sub + LPR) < r ? 16u * (unsigned)(sub + LPR) : 0u;
+  }
+  // the first pairs of the group's share
+  __device__ inline void request(const uint2* pairs, const fu_tile_at& d) {
+    const uint2* pp = pairs + d.e0;
+    const int s0 = grp * d.share;
+    const unsigned last = d.E > 0 ? (unsigned)(d.E - 1) : 0u;  // (the array has a spare entry)
+    before = pp[s0 > 0 && (unsigned)s0 <= last ? (unsigned)(s0 - 1) : 0u].x;
+    const unsigned end = (unsigned)(s0 + d.share - 1) < last ? (unsigned)(s0 + d.share - 1) : last;
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const unsigned e = (unsigned)(s0 + u);
+      pr[u] = pp[e < end ? e : end];
+    }
+  }
+  __device__ inline void run(const uint2* pairs, const fu_tile_at& d, const char* Wb,
+                             float* tile) {
+    const int s0 = grp * d.share, s1 = s0 + d.share < d.E ? s0 + d.share : d.E;
+    if (s0 >= s1) return;
+    const uint2* pp = pairs + d.e0;
+    unsigned cur = pr[0].x;
+    int dst = s0 > 0 && ((cur ^ before) >> FU_ROW_BITS) == 0 ? CARRY + grp * (8 * LPR)
+                                                             : (int)((cur >> FU_ROW_BITS) & (TC - 1)) * TS;
+    dst += 4 * sub;
+    f32x4 a0 = f32x4{0.0f, 0.0f, 0.0f, 0.0f}, a1 = a0;
+    auto put = [&]() {
+      *reinterpret_cast<f32x4*>(tile + dst) = a0;
+      if (WHOLE || 4 * (sub + LPR) < 16 * NB) *reinterpret_cast<f32x4*>(tile + dst + 4 * LPR) = a1;
+    };
+    for (int b = s0; b < s1; b += U) {
+      f32x4 w0[U], w1[U];
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        const unsigned at = __umul24(pr[u].x & ((1u << FU_ROW_BITS) - 1u), r4);
+        w0[u] = *reinterpret_cast<const f32x4u*>(Wb + (at + off0));
+        w1[u] = *reinterpret_cast<const f32x4u*>(Wb + (at + off1));
+      }
+      uint2 nx[U];
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        const unsigned e = (unsigned)(b + U + u), end = (unsigned)(s1 - 1);
+        nx[u] = pp[e < end ? e : end];
+      }
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        const float v = b + u < s1 ? __uint_as_float(pr[u].y) : 0.0f;
+        if (((pr[u].x ^ cur) >> FU_ROW_BITS) != 0) {
+          put();
+          cur = pr[u].x;
+          dst = (int)((cur >> FU_ROW_BITS) & (TC - 1)) * TS + 4 * sub;
+          a0 = a1 = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        }
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          a0[i] = fmaf(v, w0[u][i], a0[i]);
+          a1[i] = fmaf(v, w1[u][i], a1[i]);
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < U; u++) pr[u] = nx[u];
+    }
+    put();
+  }
+};
+
+// The shares that start inside a column with the tile's entries [a0, a1): k0 .. k1 - 1.
+__device__ inline void fu_cut_by(int a0, int a1, int share, float inv, int& k0, int& k1) {
+  auto quot = [&](int x) {  // x / share (the float quotient is off by one at most)
+    int q = (int)((float)x * inv);
+    if (q * share > x) q--;
+    if ((q + 1) * share <= x) q++;
+    return q;
+  };
+  k0 = quot(a0) + 1;
+  k1 = quot(a1 - 1) + 1;
+}
+
+// Update quotient: the reciprocal and one correction step, within an ulp of the division.
+__device__ inline float fu_quotient(float t, float den) {
+  const float inv = __builtin_amdgcn_rcpf(den), q0 = t * inv;
+  return fmaf(fmaf(-q0, den, t), inv, q0);
+}
+
 
 }  // namespace dn

@@ -1,0 +1,422 @@
+// The updates of the fused step at ranks 65 ... 128: as k_fu_h and k_fu_w (fused.hip), with G in
+// registers.
+//
+// At these ranks G no longer fits LDS beside the tile, and the fp32 matrix cores would take longer than
+// everything else.  X G therefore runs on the bf16 matrix cores with both operands split in three
+// (split_bf16.hpp; v_mfma_f32_16x16x32_bf16, six products): a tile is 32 rows, each of the four waves
+// holds the split G of its own output components in registers, and the split rows of the tile go through
+// LDS.  A lane's share of X G is the layout in which it has loaded X (rows l % 16, components 16 b + 4
+// (l / 16) + i), so X is read once and split by the lane that updates it.  The result is split again for
+// X^T X, whose upper block pairs are dealt to the waves.
+#include "fused.hpp"
+
+#include <type_traits>
+
+namespace dn {
+
+constexpr int FUW_U = 2;  // rows of W in flight per lane group
+constexpr int fuw_steps(int nb) { return (16 * nb + 31) / 32; }
+
+struct fuw_args {
+  // H update
+  const fu_tile* tiles;
+  int n_tiles;
+  const int64_t* colptr;
+  const uint2* pairs;
+  const float* W;
+  // W update
+  int64_t n;
+  const int* n_base;
+  const float* N;
+  // both
+  int r;
+  float* X;
+  float eps;
+  const float* g;
+  int n_g;
+  float* gpart;
+};
+
+// Four components c .. c + 3 of a row, zero past the rank; `whole`: all of the block's exist.
+__device__ inline f32x4 fuw_load4(const float* __restrict__ row, int c, int r, bool whole) {
+  if (whole) return *reinterpret_cast<const f32x4u*>(row + c);
+  f32x4 v;
+#pragma unroll
+  for (int i = 0; i < 4; i++) v[i] = c + i < r ? row[c + i] : 0.0f;
+  return v;
+}
+
+// Block rows of X^T X that wave W forms: W and 7 - W.  y: three planes of the split result, transposed:
+// [component][32 rows], the 16-byte pieces of a component's row stored at piece ^ (component / 4 mod 4)
+// (a lane writes single numbers, the four lane groups then hit different banks).
+constexpr int fuw_y_plane(int nb) { return 16 * nb * FUW_COLS; }
+__device__ inline int fuw_y_at(int c, int j) { return c * FUW_COLS + (((j >> 3) ^ ((c >> 2) & 3)) << 3) + (j & 7); }
+
+template <int W, int NB>
+struct fuw_gram {
+  static constexpr int R2 = 7 - W;
+  static constexpr bool SECOND = R2 < NB && R2 > 3;
+  static constexpr int N1 = NB - W, N2 = SECOND ? NB - R2 : 0;
+  struct part {
+    bf16x8 h, m, l;
+  };
+  __device__ static inline part load(const __bf16* __restrict__ y, int b, int lane) {
+    const __bf16* at = y + fuw_y_at(16 * b + (lane & 15), 8 * (lane >> 4));
+    return part{*reinterpret_cast<const bf16x8*>(at), *reinterpret_cast<const bf16x8*>(at + fuw_y_plane(NB)),
+                *reinterpret_cast<const bf16x8*>(at + 2 * fuw_y_plane(NB))};
+  }
+  __device__ static inline f32x4 mul(const part& a, const part& b, f32x4 c) {
+    c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.l, b.h, c, 0, 0, 0);
+    c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.h, b.l, c, 0, 0, 0);
+    c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.m, b.m, c, 0, 0, 0);
+    c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.m, b.h, c, 0, 0, 0);
+    c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.h, b.m, c, 0, 0, 0);
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.h, b.h, c, 0, 0, 0);
+  }
+  template <int NA>
+  __device__ static inline void add(const __bf16* __restrict__ y, f32x4 (&acc)[NA]) {
+    const int lane = threadIdx.x & 63;
+    const part a = load(y, W, lane);
+    part a2;
+    if constexpr (SECOND) a2 = load(y, R2, lane);
+#pragma unroll
+    for (int b = W; b < NB; b++) {
+      const part x = b == W ? a : load(y, b, lane);
+      acc[b - W] = mul(a, x, acc[b - W]);
+      if constexpr (SECOND) {
+        if (b >= R2) acc[N1 + b - R2] = mul(a2, x, acc[N1 + b - R2]);
+      }
+    }
+  }
+  template <int NA>
+  __device__ static inline void out(const f32x4 (&acc)[NA], float* __restrict__ gpart) {
+    const int lane = threadIdx.x & 63, l16 = lane & 15, g = lane >> 4;
+    auto put = [&](int b1, int b2, const f32x4& v) {
+      float* dst = gpart + fu_pair(b1, b2, NB) * 256;
+#pragma unroll
+      for (int i = 0; i < 4; i++) dst[(4 * g + i) * 16 + l16] = v[i];
+    };
+#pragma unroll
+    for (int b = W; b < NB; b++) put(W, b, acc[b - W]);
+    if constexpr (SECOND) {
+#pragma unroll
+      for (int b = R2; b < NB; b++) put(R2, b, acc[N1 + b - R2]);
+    }
+  }
+};
+
+template <class F>
+__device__ inline void fuw_for_wave(int wave, F&& f) {
+  switch (wave) {
+    case 0: f(std::integral_constant<int, 0>{}); break;
+    case 1: f(std::integral_constant<int, 1>{}); break;
+    case 2: f(std::integral_constant<int, 2>{}); break;
+    default: f(std::integral_constant<int, 3>{}); break;
+  }
+}
+
+// COLS: the H update (tiles of columns, A^T W gathered); else the W update (32 rows per workgroup, the
+// chunk sums of A H^T).  NB: blocks of 16 components.  Two barriers per tile: the Gram products of a
+// tile run between the second one and the next tile's first, beside the gathers of the next tile.
+template <int NB, bool COLS>
+__global__ void __launch_bounds__(256, 2) k_fuw(const fuw_args p) {
+  constexpr int NS = fuw_steps(NB), PS = 32 * NS + 8, PLANE = FUW_COLS * PS, TS = 16 * NB + 4;
+  constexpr bool SPLIT_J = NB <= 6;  // two waves per 16 rows, three blocks each; else two blocks, all rows
+  constexpr int BPW = SPLIT_J ? 3 : 2, JPW = SPLIT_J ? 1 : 2;
+  constexpr int NA = NB == 8 ? 9 : NB == 7 ? 7 : NB == 6 ? 6 : 5;
+  using Gather = fu_gather<FUW_COLS, TS, NB, 16, FUW_U>;
+  constexpr int YP = fuw_y_plane(NB);
+  constexpr int LDS_TILE = COLS ? 4 * (Gather::CARRY + 2048) : 0;
+  extern __shared__ __align__(16) char lds[];
+  float* tile = reinterpret_cast<float*>(lds);
+  __bf16* planes = reinterpret_cast<__bf16*>(lds + LDS_TILE);
+  __bf16* ypl = planes + 3 * PLANE;
+  __shared__ int cps[2][FUW_COLS + 1];
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int l16 = lane & 15, g = lane >> 4;
+  const int jb0 = SPLIT_J ? wave & 1 : 0, b0 = SPLIT_J ? 3 * (wave >> 1) : 2 * wave;
+  const int r = p.r;
+  const char* Wb = reinterpret_cast<const char*>(p.W);
+  Gather gather;
+  fu_tile_at td;
+  int64_t cpv = 0;
+  auto request = [&](const fu_tile_at& d) {
+    gather.request(p.pairs, d);
+    cpv = p.colptr[d.col0 + (tid < d.nc ? tid : d.nc)];
+  };
+  if constexpr (COLS) {
+    gather.init(r);
+    td = fu_describe<Gather::NG>(p.tiles, p.n_tiles, blockIdx.x);
+    request(td);
+  }
+
+  // the wave's rows of G, split: row 16 (b0 + bi) + l16, components 32 s + 8 g ..
+  bf16x8 gh[BPW][NS], gm[BPW][NS], gl[BPW][NS];
+#pragma unroll
+  for (int bi = 0; bi < BPW; bi++)
+#pragma unroll
+    for (int s = 0; s < NS; s++) {
+      f32x4 v[2];
+      const int c = 16 * (b0 + bi) + l16;
+#pragma unroll
+      for (int t = 0; t < 8; t++) {
+        const int k = 32 * s + 8 * g + t;
+        double sum = 0.0;
+        if (k < r && c < r) {
+          const int bk = k >> 4, bc = c >> 4;
+          const int at = bk <= bc ? fu_pair(bk, bc, NB) * 256 + (k & 15) * 16 + (c & 15)
+                                  : fu_pair(bc, bk, NB) * 256 + (c & 15) * 16 + (k & 15);
+          for (int q = 0; q < p.n_g; q++) sum += (double)p.g[(int64_t)q * (fu_pairs(NB) * 256) + at];
+        }
+        v[t >> 2][t & 3] = (float)sum;
+      }
+      bf16x4 h0, m0, l0, h1, m1, l1;
+      split3(v[0], h0, m0, l0);
+      split3(v[1], h1, m1, l1);
+      gh[bi][s] = cat8(h0, h1);
+      gm[bi][s] = cat8(m0, m1);
+      gl[bi][s] = cat8(l0, l1);
+    }
+  f32x4 acc[NA];
+#pragma unroll
+  for (int q = 0; q < NA; q++) acc[q] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  // (components past the last block are never written: zeros)
+  for (int x = tid; x < 3 * PLANE / 2; x += 256) reinterpret_cast<unsigned*>(planes)[x] = 0u;
+  __syncthreads();
+
+  f32x4 x[JPW][BPW], t[JPW][BPW];
+  struct place {  // of a tile: its rows of X and which of the lane's it has
+    float* Xb;
+    int l0, nc;
+  };
+  auto place_of = [&](int tl) {
+    place q;
+    q.l0 = COLS ? td.col0 & (FUW_COLS - 1) : 0;
+    const int64_t base = COLS ? td.col0 - q.l0 : (int64_t)tl * FUW_COLS;
+    q.nc = COLS ? td.nc : (int)(p.n - base < FUW_COLS ? p.n - base : FUW_COLS);
+    q.Xb = p.X + base * r;
+    return q;
+  };
+  auto in_tile = [&](const place& q, int jl) { return jl >= q.l0 && jl < q.l0 + q.nc; };
+  auto load_x = [&](const place& q) {
+#pragma unroll
+    for (int jp = 0; jp < JPW; jp++) {
+      const int jl = 16 * (jb0 + jp) + l16;
+      const float* row = q.Xb + (unsigned)(in_tile(q, jl) ? jl : q.l0) * (unsigned)r;
+#pragma unroll
+      for (int bi = 0; bi < BPW; bi++) {
+        const int b = b0 + bi;
+        if (b < NB) x[jp][bi] = fuw_load4(row, 16 * b + 4 * g, r, 16 * b + 16 <= r);
+        else x[jp][bi] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+      }
+    }
+  };
+  auto split_x = [&]() {
+#pragma unroll
+    for (int jp = 0; jp < JPW; jp++)
+#pragma unroll
+      for (int bi = 0; bi < BPW; bi++) {
+        if (b0 + bi >= NB) continue;
+        bf16x4 h, m, l;
+        split3(x[jp][bi], h, m, l);
+        __bf16* at = planes + (16 * (jb0 + jp) + l16) * PS + 16 * (b0 + bi) + 4 * g;
+        *reinterpret_cast<bf16x4*>(at) = h;
+        *reinterpret_cast<bf16x4*>(at + PLANE) = m;
+        *reinterpret_cast<bf16x4*>(at + 2 * PLANE) = l;
+      }
+  };
+
+  int tl = blockIdx.x;
+  place at = place_of(tl);
+  load_x(at);
+  if constexpr (COLS) {
+    if (tid <= at.nc) cps[0][at.l0 + tid] = (int)(cpv - td.e0);
+    gather.run(p.pairs, td, Wb, tile);
+  } else {
+#pragma unroll
+    for (int jp = 0; jp < JPW; jp++) {
+      const int jl = 16 * (jb0 + jp) + l16;
+      const int64_t i = (int64_t)tl * FUW_COLS + (in_tile(at, jl) ? jl : 0);
+      const int64_t k0 = p.n_base ? p.n_base[i] : i, k1 = p.n_base ? p.n_base[i + 1] : i + 1;
+#pragma unroll
+      for (int bi = 0; bi < BPW; bi++) t[jp][bi] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 2
+      for (int64_t k = k0; k < k1; k++)
+#pragma unroll
+        for (int bi = 0; bi < BPW; bi++)
+          if (b0 + bi < NB) t[jp][bi] += fuw_load4(p.N + k * r, 16 * (b0 + bi) + 4 * g, r, 16 * (b0 + bi) + 16 <= r);
+    }
+  }
+  split_x();
+
+  for (int par = 0;; par ^= 1) {
+    fu_tile_at nd;
+    const int next = tl + gridDim.x;
+    const bool more = COLS && next < p.n_tiles;
+    if constexpr (COLS) {
+      nd = fu_describe<Gather::NG>(p.tiles, p.n_tiles, next);
+      request(nd);
+    }
+    __syncthreads();
+
+    f32x4 d[JPW][BPW];
+#pragma unroll
+    for (int jp = 0; jp < JPW; jp++)
+#pragma unroll
+      for (int bi = 0; bi < BPW; bi++) d[jp][bi] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int s = 0; s < NS; s++)
+#pragma unroll
+      for (int jp = 0; jp < JPW; jp++) {
+        const __bf16* pl = planes + (16 * (jb0 + jp) + l16) * PS + 32 * s + 8 * g;
+        const bf16x8 bh = *reinterpret_cast<const bf16x8*>(pl);
+        const bf16x8 bm = *reinterpret_cast<const bf16x8*>(pl + PLANE);
+        const bf16x8 bl = *reinterpret_cast<const bf16x8*>(pl + 2 * PLANE);
+#define DN_FUW(A, B)                            \
+  _Pragma("unroll") for (int bi = 0; bi < BPW; bi++) d[jp][bi] = \
+      __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[bi][s], B, d[jp][bi], 0, 0, 0)
+        DN_FUW(gl, bh);
+        DN_FUW(gh, bl);
+        DN_FUW(gm, bm);
+        DN_FUW(gm, bh);
+        DN_FUW(gh, bm);
+        DN_FUW(gh, bh);
+#undef DN_FUW
+      }
+    const float inv = 1.0f / (float)(COLS && td.share > 0 ? td.share : 1);
+#pragma unroll
+    for (int jp = 0; jp < JPW; jp++) {
+      const int jl = 16 * (jb0 + jp) + l16;
+      const bool mine = in_tile(at, jl);
+      bool some = mine;
+      if constexpr (COLS) {
+        const float* trow = tile + jl * TS + 4 * g;
+        const int a0 = mine ? cps[par][jl] : 0, a1 = mine ? cps[par][jl + 1] : 0;
+        some = a1 > a0;  // (a column without entries: 0)
+#pragma unroll
+        for (int bi = 0; bi < BPW; bi++)
+          if (b0 + bi < NB) t[jp][bi] = *reinterpret_cast<const f32x4*>(trow + 16 * (b0 + bi));
+        if (some) {
+          int k0, k1;
+          fu_cut_by(a0, a1, td.share, inv, k0, k1);
+          for (int k = k0; k < k1; k++)
+#pragma unroll
+            for (int bi = 0; bi < BPW; bi++)
+              if (b0 + bi < NB)
+                t[jp][bi] += *reinterpret_cast<const f32x4*>(tile + Gather::CARRY + k * 128 + 16 * (b0 + bi) + 4 * g);
+        }
+      }
+#pragma unroll
+      for (int bi = 0; bi < BPW; bi++) {
+        const int b = b0 + bi;
+        if (b >= NB) continue;
+        const bool whole = 16 * b + 16 <= r;
+        f32x4 y;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          const float v = x[jp][bi][i] * fu_quotient(t[jp][bi][i], d[jp][bi][i] + p.eps);
+          y[i] = some ? v : 0.0f;
+        }
+        if (!whole) {
+#pragma unroll
+          for (int i = 0; i < 4; i++) y[i] = 16 * b + 4 * g + i < r ? y[i] : 0.0f;
+        }
+        if (mine) {
+          float* dst = at.Xb + (unsigned)jl * (unsigned)r + 16 * b + 4 * g;
+          if (whole) *reinterpret_cast<f32x4u*>(dst) = y;
+          else {
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+              if (16 * b + 4 * g + i < r) dst[i] = y[i];
+          }
+        }
+        bf16x4 h, m, l;
+        split3(y, h, m, l);
+        __bf16* yp = ypl + fuw_y_at(16 * b + 4 * g, jl);
+#pragma unroll
+        for (int i = 0; i < 4; i++) {  // (the four components share the piece's place)
+          yp[i * FUW_COLS] = h[i];
+          yp[i * FUW_COLS + YP] = m[i];
+          yp[i * FUW_COLS + 2 * YP] = l[i];
+        }
+      }
+    }
+    __syncthreads();
+    if (more) {
+      td = nd;
+      tl = next;
+      at = place_of(tl);
+    }
+    fuw_for_wave(wave, [&](auto w) { fuw_gram<decltype(w)::value, NB>::add(ypl, acc); });
+    if (!more) break;
+    if constexpr (COLS) {
+      if (tid <= at.nc) cps[par ^ 1][at.l0 + tid] = (int)(cpv - td.e0);
+      load_x(at);  // (here and not ahead of the Gram products: registers)
+      gather.run(p.pairs, td, Wb, tile);
+      split_x();
+    }
+  }
+  float* out = p.gpart + (int64_t)blockIdx.x * (fu_pairs(NB) * 256);
+  fuw_for_wave(wave, [&](auto w) { fuw_gram<decltype(w)::value, NB>::out(acc, out); });
+}
+
+// LDS of a workgroup of k_fuw: the tile with its carries, the split rows, the split results.
+static size_t fuw_lds(int nb, bool cols) {
+  const int ps = 32 * fuw_steps(nb) + 8;
+  return (cols ? 4 * (size_t)(FUW_COLS * (16 * nb + 4) + 2048) : 0) + 6 * (size_t)(FUW_COLS * ps) + 6 * (size_t)fuw_y_plane(nb);
+}
+
+template <bool COLS, class F>
+static int fuw_dispatch(int r, F&& f) {
+  switch ((r + 15) / 16) {
+    case 5: return f(k_fuw<5, COLS>);
+    case 6: return f(k_fuw<6, COLS>);
+    case 7: return f(k_fuw<7, COLS>);
+    case 8: return f(k_fuw<8, COLS>);
+  }
+  DN_CHECK(false, "rank %d has no fused step", r);
+}
+
+// Dynamic LDS of more than 64 KB has to be asked for, once per kernel.
+template <class K>
+static int fuw_prepare(K kernel, size_t bytes) {
+  DN_HIP(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
+  return 0;
+}
+
+int fuw_per_cu(int r, int* wgs) {
+  const size_t lds = fuw_lds((r + 15) / 16, true);
+  DN_TRY(fuw_dispatch<true>(r, [&](auto kernel) {
+    DN_TRY(fuw_prepare(kernel, lds));
+    DN_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(wgs, kernel, 256, lds));
+    return 0;
+  }));
+  return fuw_dispatch<false>(r, [&](auto kernel) { return fuw_prepare(kernel, fuw_lds((r + 15) / 16, false)); });
+}
+
+int fuw_launch_h(int wgs, const fused_plan& f, const int64_t* colptr, int r, const float* W, float* H, float eps,
+                 const float* gw, int n_gw, float* gpart) {
+  fuw_args p = {};
+  p.tiles = f.tiles; p.n_tiles = (int)f.n_tiles; p.colptr = colptr; p.pairs = f.pairs; p.W = W;
+  p.r = r; p.X = H; p.eps = eps; p.g = gw; p.n_g = n_gw; p.gpart = gpart;
+  DN_TRY(fuw_dispatch<true>(r, [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3((unsigned)wgs), dim3(256), fuw_lds((r + 15) / 16, true), stream(), p);
+    return 0;
+  }));
+  DN_LAUNCH_CHECK();
+  return 0;
+}
+
+int fuw_launch_w(int wgs, int64_t n, int r, const int* n_base, const float* N, float* W, float eps, const float* gh,
+                 float* gpart) {
+  fuw_args p = {};
+  p.n = n; p.n_base = n_base; p.N = N; p.r = r; p.X = W; p.eps = eps; p.g = gh; p.n_g = 1; p.gpart = gpart;
+  DN_TRY(fuw_dispatch<false>(r, [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3((unsigned)wgs), dim3(256), fuw_lds((r + 15) / 16, false), stream(), p);
+    return 0;
+  }));
+  DN_LAUNCH_CHECK();
+  return 0;
+}
+
+}  // namespace dn

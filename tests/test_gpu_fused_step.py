@@ -1,4 +1,4 @@
-"""The step of small ranks (csrc/fused.hip) against the fp64 oracle: remainders of the rank, tiles cut by
+"""The step of small ranks (csrc/fused.hip, csrc/fused_wide.hip) against the fp64 oracle: remainders of the rank, tiles cut by
 their number of entries, columns longer than a tile, empty columns and rows, and the changes between it
 and the separate kernels."""
 
@@ -36,7 +36,9 @@ def _close(nmf, oracle_out):
 
 @pytest.mark.parametrize("n,m,r", [(1, 1, 1), (2, 63, 3), (5, 64, 4), (33, 65, 5), (70, 300, 8), (65, 257, 12),
                                    (40, 515, 13), (64, 1000, 16), (90, 130, 17), (1500, 1600, 20), (50, 129, 31),
-                                   (130, 700, 33), (30, 64, 44), (77, 333, 50), (2100, 2200, 61), (63, 191, 64)])
+                                   (130, 700, 33), (30, 64, 44), (77, 333, 50), (2100, 2200, 61), (63, 191, 64),
+                                   (31, 65, 65), (33, 400, 80), (1, 32, 81), (300, 640, 96), (96, 129, 97),
+                                   (1200, 1300, 113), (40, 65600, 128)])
 def test_step_matches_the_oracle(n, m, r):
     rp, ci, va = _matrix(n, m, seed=n + r, fill=0.3 if n < 100 else 0.02)
     A = d.Csr.from_host(rp, ci, va, m)
@@ -49,7 +51,7 @@ def test_step_matches_the_oracle(n, m, r):
     A.close()
 
 
-@pytest.mark.parametrize("r", [7, 48])
+@pytest.mark.parametrize("r", [7, 48, 100])
 def test_step_and_separate_kernels_in_turn(r, tune):
     """A run that changes from the fused step to the separate kernels and back, between and within
     iterations, keeps no product of an older factor."""
