@@ -355,7 +355,7 @@ static void gram_b16_slices(int64_t rows, int r, int64_t* s_diag, int64_t* s_off
   *s_off = n_off > 0 ? (o < 1 ? 1 : o) : 0;
 }
 
-int64_t gram_tiles_workspace_floats(int64_t rows, int r) {
+static int64_t gram_tiles_sums_at(int64_t rows, int r) {
   int64_t d, o, dp, op;
   gram_b16_slices(rows, r, &d, &o);
   gram_b16_slices(rows, r, &dp, &op, true);
@@ -363,32 +363,81 @@ int64_t gram_tiles_workspace_floats(int64_t rows, int r) {
   return (s + 1) * (int64_t)r * r;
 }
 
-// Diagonal tiles hold s_diag slices, the others s_off, and slice number `extra` (if >= 0) holds
-// one more term of every tile (the last rows, from the fp32 kernel).
+int64_t gram_tiles_workspace_floats(int64_t rows, int r) {
+  return gram_tiles_sums_at(rows, r) + 2 * (int64_t)r * r;
+}
+
+// Slice sums: diagonal tiles hold s_diag slices, the others s_off, and slice number `extra` (if >= 0)
+// holds one more term of every tile (the last rows, from the fp32 kernel: k_gram_tiles_fold adds it).
+// folded = 1: diagonal tiles of 128 from k_gram_diag_b16; 2: diagonal squares of 256 from
+// k_gram_pair_b16, where the block four block columns to the right of the diagonal comes in
+// two halves, one of them stored transposed below the diagonal.
+//
+// A workgroup sums 32 elements of one row, eight threads each over every eighth slice (the 65 MB of 256
+// slices at r = 256 in 12 us; one thread per element, with the mirrored elements read column-wise, took
+// 150 us).  The sums stay fp64 until k_gram_tiles_fold has added mirrored parts.
+__device__ inline bool gram_own(int a, int b, int folded) {
+  return folded == 2 ? (a >> 8) == (b >> 8) : (a >> 7) == (b >> 7);
+}
+// element (a, b), a <= b, has a second part at (b, a)
+__device__ inline bool gram_mirrored(int a, int b, int folded) {
+  return folded && ((a >> 5) == (b >> 5) || (folded == 2 && gram_own(a, b, folded) && (b >> 5) - (a >> 5) == 4));
+}
+
 __global__ void __launch_bounds__(256)
-    k_gram_tiles_reduce(const float* __restrict__ ws, int64_t s_diag, int64_t s_off, int64_t extra, int r,
-                        int folded, float* __restrict__ G) {
-  const int e = blockIdx.x * 256 + threadIdx.x;
-  if (e >= r * r) return;
-  const int a = e / r, b = e % r;
-  if (a > b) return;  // upper triangle only
-  double s = 0.0;
+    k_gram_tiles_sum(const float* __restrict__ ws, int64_t s_diag, int64_t s_off, int r, int folded,
+                     double* __restrict__ sums) {
+  __shared__ double red[256];
+  const int a = blockIdx.y, b = blockIdx.x * 32 + (threadIdx.x & 31), k = threadIdx.x >> 5;
+  const int ab = a >> 5, bb = blockIdx.x;
+  if (bb < ab && !gram_mirrored(bb << 5, ab << 5, folded)) return;  // (nothing is stored there)
   const int64_t stride = (int64_t)r * r;
-  // folded = 1: diagonal tiles of 128 from k_gram_diag_b16; 2: diagonal squares of 256 from
-  // k_gram_pair_b16, where the block four block columns to the right of the diagonal comes in
-  // two halves, one of them stored transposed below the diagonal
-  const bool own = folded == 2 ? (a >> 8) == (b >> 8) : (a >> 7) == (b >> 7);
-  const int64_t slices = own ? s_diag : s_off;
-  if (folded && ((a >> 5) == (b >> 5) || (folded == 2 && own && (b >> 5) - (a >> 5) == 4))) {
-    // the stored block plus (the stored block at the mirrored place) transposed
-    const int et = b * r + a;
-    for (int64_t sl = 0; sl < slices; sl++)
-      s += (double)ws[sl * stride + e] + (double)ws[sl * stride + et];
-  } else
-  for (int64_t sl = 0; sl < slices; sl++) s += (double)ws[sl * stride + e];
-  if (extra >= 0) s += (double)ws[extra * stride + e];
-  G[(int64_t)a * r + b] = (float)s;
-  G[(int64_t)b * r + a] = (float)s;
+  const int64_t slices = gram_own(a, b, folded) ? s_diag : s_off;
+  const float* p = ws + (int64_t)a * r + b;
+  double s = 0.0;
+  int64_t q = k;
+  for (; q + 24 < slices; q += 32) {
+    const float x0 = p[q * stride], x1 = p[(q + 8) * stride], x2 = p[(q + 16) * stride], x3 = p[(q + 24) * stride];
+    s += ((double)x0 + (double)x1) + ((double)x2 + (double)x3);
+  }
+  for (; q < slices; q += 8) s += (double)p[q * stride];
+  red[threadIdx.x] = s;
+  __syncthreads();
+  if (k == 0) {
+    for (int u = 1; u < 8; u++) s += red[32 * u + (threadIdx.x & 31)];
+    sums[(int64_t)a * r + b] = s;
+  }
+}
+
+// Element (a, b) with a <= b and its mirror image; the mirrored parts of a block are read through LDS.
+// extra (or NULL): the last rows' term, upper triangle.
+__global__ void __launch_bounds__(256)
+    k_gram_tiles_fold(const double* __restrict__ sums, const float* __restrict__ extra, int r, int folded,
+                      float* __restrict__ G) {
+  __shared__ double tile[32][33];
+  const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+  const int a0 = 32 * blockIdx.y, b0 = 32 * blockIdx.x;
+  if (b0 < a0) return;
+  const bool mirrored = gram_mirrored(a0, b0, folded);
+  if (mirrored) {
+    for (int i = ty; i < 32; i += 8) tile[i][tx] = sums[(int64_t)(b0 + i) * r + a0 + tx];
+  }
+  __syncthreads();
+  double v[4];
+  for (int q = 0; q < 4; q++) {
+    const int i = ty + 8 * q;
+    v[q] = sums[(int64_t)(a0 + i) * r + b0 + tx];
+    if (mirrored) v[q] += tile[tx][i];
+    if (extra) v[q] += (double)extra[(int64_t)(a0 + i) * r + b0 + tx];  // (below the diagonal: not used)
+  }
+  __syncthreads();
+  for (int q = 0; q < 4; q++) tile[ty + 8 * q][tx] = v[q];
+  __syncthreads();
+  for (int i = ty; i < 32; i += 8) {
+    // (a diagonal block: its upper triangle twice)
+    if (a0 != b0 || i <= tx) G[(int64_t)(a0 + i) * r + b0 + tx] = (float)tile[i][tx];
+    if (a0 != b0 || i > tx) G[(int64_t)(b0 + i) * r + a0 + tx] = (float)tile[tx][i];
+  }
 }
 
 // The same on the bf16 matrix cores with split operands (abt_b16.hpp): both operand tiles are
@@ -571,8 +620,11 @@ int launch_gram_tiles(int64_t rows, int r, const float* X, float* G, float* work
     s_diag = s_off = gram_tiles_slices(rows, r);
     DN_TRY(launch_ptq(X, r, rows, X, r, r, r, s_diag, workspace, t));
   }
-  hipLaunchKernelGGL(k_gram_tiles_reduce, dim3((unsigned)ceil_div((int64_t)r * r, 256)), dim3(256), 0,
-                     stream(), workspace, s_diag, s_off, extra, r, folded, G);
+  double* sums = reinterpret_cast<double*>(workspace + gram_tiles_sums_at(rows, r));
+  const dim3 blocks((unsigned)(r / 32), (unsigned)r);
+  hipLaunchKernelGGL(k_gram_tiles_sum, blocks, dim3(256), 0, stream(), workspace, s_diag, s_off, r, folded, sums);
+  hipLaunchKernelGGL(k_gram_tiles_fold, dim3((unsigned)(r / 32), (unsigned)(r / 32)), dim3(256), 0, stream(), sums,
+                     extra >= 0 ? workspace + extra * (int64_t)r * r : nullptr, r, folded, G);
   DN_LAUNCH_CHECK();
   return 0;
 }
