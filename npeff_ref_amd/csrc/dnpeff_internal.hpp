@@ -128,8 +128,10 @@ int launch_gram_tiles(int64_t rows, int r, const float* X, float* G, float* work
 // must not change G in between).
 int xg_mu_hold_g(const float* G, int r);
 void xg_mu_release_g();
+// rows_there: rows that X, num and out have memory for (0: `rows`); up to the next multiple of 128 they
+// may be read and overwritten with anything.
 int launch_xg_mu(int64_t rows, int r, const float* X, const float* G, const float* num, float eps,
-                 float* out, float* D_out);
+                 float* out, float* D_out, int64_t rows_there = 0);
 // r = 128: the update and the Gram matrix of its output in one pass (dense.hip).
 int64_t xg_mu_gram_workspace_floats(int64_t rows);
 int launch_xg_mu_gram(int64_t rows, const float* X, const float* G, const float* num, float eps,
@@ -142,6 +144,10 @@ int launch_init_uniform(int matrix_id, int64_t logical_rows, int64_t logical_col
                         float* x);
 // out[c * rows + i] = in[i * cols + c]   (in is [rows, cols] row-major)
 int launch_transpose(int64_t rows, int64_t cols, const float* in, float* out);
+// out[c * ldo + i] = in[i * ldi + c]
+int launch_transpose_ld(int64_t rows, int64_t cols, const float* in, int64_t ldi, float* out, int64_t ldo);
+// out[i * ldo + c] = c < w ? in[i * ldi + c] : 0, c < ldo
+int launch_copy_rows(int64_t rows, int w, const float* in, int ldi, float* out, int ldo);
 
 // ---- fixed-H learner (fit.hip) ----
 bool fit_steps_supported(int64_t n, int r);
@@ -196,6 +202,7 @@ struct tuning_t {
                                    // multiple of 256, else as 1 = diagonal tiles of 128 with their symmetry; 0 = all sixteen blocks
   double nl_wgs = 64.0;            // workgroups of the slot-list kernel per XCD (two per CU)
   double nl_spin = 50000.0;        // polls (about 1 us each) before a workgroup of the slot-list kernel stops waiting
+  double pad_rank = 1.0;           // ranks above 128 stored as the next multiple of 128 (0 = as they are)
   double verbose = 0.0;
 };
 tuning_t& tuning();
@@ -270,6 +277,8 @@ struct fused_plan {
   fu_tile* tiles = nullptr;  // [n_tiles + 1]: the last one only ends the entries
   int64_t n_tiles = 0;
   int tile_cols = 0;
+  int64_t tile_most = 0;
+  std::vector<int64_t> h_first;  // first tile of every group of tile_cols columns, for products on column tiles
   uint2* pairs = nullptr;    // [nnz + 1]
   fu_chunk* chunks = nullptr;
   int64_t n_chunks = 0;
@@ -404,6 +413,9 @@ bool tlists_supported(const dnpeff_csr* S, int r);
 int tblocks_build(dnpeff_csr* S);
 void tblocks_drop(dnpeff_csr* S);
 void fused_drop(dnpeff_csr* S);  // fused.hip
+int fused_tiles_build(dnpeff_csr* S, int r);  // the tiles of fused_plan for rank r (32 columns each above 64)
+int fused_tiles_first(dnpeff_csr* S);         // h_first of the tiles that are there
+bool use_spmm_t_bal(const dnpeff_csr* S, int r);  // spmm.hip
 int launch_spmm_t_lists(const dnpeff_csr* S, int r, const float* W_nr, float* T, int64_t col0, int64_t col1);
 // Whether the products of the sparse part S at rank r run from the slot lists / column blocks.
 bool use_nlists(const dnpeff_csr* S, int r);       // the whole sparse part on slot lists

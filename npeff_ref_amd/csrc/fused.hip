@@ -501,8 +501,9 @@ __global__ void __launch_bounds__(256)
 // ---------------------------------------------------------------------------
 // Tiles of the aligned group of `tc` columns `grp`: f(first column, columns) for each, in order.
 template <class F>
-__device__ inline void fu_split_group(const int64_t* __restrict__ colptr, int64_t m, int tc, int64_t grp, F&& f) {
-  const int64_t j0 = grp * tc, j1 = j0 + tc < m ? j0 + tc : m, most = 16 * tc;
+__device__ inline void fu_split_group(const int64_t* __restrict__ colptr, int64_t m, int tc, int64_t most, int64_t grp,
+                                      F&& f) {
+  const int64_t j0 = grp * tc, j1 = j0 + tc < m ? j0 + tc : m;
   int64_t start = j0, e0 = colptr[j0], before = e0;
   if (colptr[j1] - e0 <= most) {
     f(j0, (int)(j1 - j0));
@@ -521,21 +522,22 @@ __device__ inline void fu_split_group(const int64_t* __restrict__ colptr, int64_
 }
 
 __global__ void __launch_bounds__(256)
-    k_fu_count_tiles(const int64_t* __restrict__ colptr, int64_t m, int tc, int64_t groups, int* __restrict__ count) {
+    k_fu_count_tiles(const int64_t* __restrict__ colptr, int64_t m, int tc, int64_t most, int64_t groups,
+                     int* __restrict__ count) {
   const int64_t grp = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (grp >= groups) return;
   int k = 0;
-  fu_split_group(colptr, m, tc, grp, [&](int64_t, int) { k++; });
+  fu_split_group(colptr, m, tc, most, grp, [&](int64_t, int) { k++; });
   count[grp] = k;
 }
 
 __global__ void __launch_bounds__(256)
-    k_fu_make_tiles(const int64_t* __restrict__ colptr, int64_t m, int tc, int64_t groups,
+    k_fu_make_tiles(const int64_t* __restrict__ colptr, int64_t m, int tc, int64_t most, int64_t groups,
                     const int64_t* __restrict__ first, fu_tile* __restrict__ tiles) {
   const int64_t grp = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (grp >= groups) return;
   int64_t k = first[grp];
-  fu_split_group(colptr, m, tc, grp, [&](int64_t col, int cols) {
+  fu_split_group(colptr, m, tc, most, grp, [&](int64_t col, int cols) {
     tiles[k].e0 = colptr[col];
     tiles[k].col0 = (int32_t)col;
     tiles[k].cols = cols;
@@ -601,10 +603,55 @@ static int fu_tile_cols(int64_t m, int r) {
   return m >= (int64_t)tc * 2 * n_cus() || tc < 64 ? tc : 64;
 }
 
+static int fused_tiles_make(dnpeff_csr* S, int tc, int64_t most, bool with_first) {
+  fused_plan& f = S->fused;
+  hipStream_t st = stream();
+  DN_CHECK(S->colptr && S->n_cols > 0, "matrix has no transposed copy");
+  if (!f.tiles || f.tile_cols != tc || f.tile_most != most || (with_first && f.h_first.empty())) {
+    const int64_t m = S->n_cols, groups = ceil_div(m, tc);
+    dbuf<int> count;
+    dbuf<int64_t> first;
+    DN_TRY(count.alloc(groups));
+    DN_TRY(first.alloc(groups + 1));
+    const dim3 grid((unsigned)ceil_div(groups, 256)), block(256);
+    hipLaunchKernelGGL(k_fu_count_tiles, grid, block, 0, st, S->colptr, m, tc, most, groups, count.p);
+    DN_LAUNCH_CHECK();
+    DN_TRY(scan_counts_i64(count, groups, first));
+    int64_t n_tiles = 0;
+    f.h_first.clear();
+    if (with_first) {
+      f.h_first.resize((size_t)groups + 1);
+      DN_HIP(hipMemcpyAsync(f.h_first.data(), first, sizeof(int64_t) * f.h_first.size(), hipMemcpyDeviceToHost, st));
+    }
+    DN_HIP(hipMemcpyAsync(&n_tiles, first + groups, sizeof(int64_t), hipMemcpyDeviceToHost, st));
+    DN_HIP(hipStreamSynchronize(st));
+    dfree(f.tiles);
+    f.tiles = nullptr;
+    DN_TRY(dmalloc(&f.tiles, n_tiles + 1));
+    f.n_tiles = n_tiles;
+    f.tile_cols = tc;
+    f.tile_most = most;
+    hipLaunchKernelGGL(k_fu_make_tiles, grid, block, 0, st, S->colptr, m, tc, most, groups, first.p, f.tiles);
+    DN_LAUNCH_CHECK();
+  }
+  return 0;
+}
+
+int fused_tiles_build(dnpeff_csr* S, int r) {
+  const int tc = fu_tile_cols(S->n_cols, r);
+  // Entries per tile: 16 per column.  The 32 columns of a tile at ranks above 64 are the smallest
+  // matrix operand: a denser matrix gets as many as leave every compute unit 16 tiles (2000 x 2M with 64 M
+  // entries, r = 90: 57 against 63 ms; at r = 20 smaller tiles are the better ones, 16.4 against 18.6).
+  int64_t most = 16 * tc;
+  if (r > FUSED_NARROW_RANK && r <= FUSED_MAX_RANK) most = std::max<int64_t>(most, S->nnz / (16 * (int64_t)n_cus()));
+  return fused_tiles_make(S, tc, most, false);
+}
+
+int fused_tiles_first(dnpeff_csr* S) { return fused_tiles_make(S, S->fused.tile_cols, S->fused.tile_most, true); }
+
 int fused_plan_build(dnpeff_csr* S, int r) {
   fused_plan& f = S->fused;
   hipStream_t st = stream();
-  const int tc = fu_tile_cols(S->n_cols, r);
   if (!f.pairs) {
     DN_CHECK(S->colptr && S->n_cols > 0, "matrix has no transposed copy");
     const int64_t groups = ceil_div(S->n_cols, FU_GROUP);
@@ -613,27 +660,7 @@ int fused_plan_build(dnpeff_csr* S, int r) {
                        S->colptr, S->rowind, S->tvals, S->n_cols, groups, f.pairs);
     DN_LAUNCH_CHECK();
   }
-  if (!f.tiles || f.tile_cols != tc) {
-    const int64_t m = S->n_cols, groups = ceil_div(m, tc);
-    dbuf<int> count;
-    dbuf<int64_t> first;
-    DN_TRY(count.alloc(groups));
-    DN_TRY(first.alloc(groups + 1));
-    const dim3 grid((unsigned)ceil_div(groups, 256)), block(256);
-    hipLaunchKernelGGL(k_fu_count_tiles, grid, block, 0, st, S->colptr, m, tc, groups, count.p);
-    DN_LAUNCH_CHECK();
-    DN_TRY(scan_counts_i64(count, groups, first));
-    int64_t n_tiles = 0;
-    DN_HIP(hipMemcpyAsync(&n_tiles, first + groups, sizeof(int64_t), hipMemcpyDeviceToHost, st));
-    DN_HIP(hipStreamSynchronize(st));
-    dfree(f.tiles);
-    f.tiles = nullptr;
-    DN_TRY(dmalloc(&f.tiles, n_tiles + 1));
-    f.n_tiles = n_tiles;
-    f.tile_cols = tc;
-    hipLaunchKernelGGL(k_fu_make_tiles, grid, block, 0, st, S->colptr, m, tc, groups, first.p, f.tiles);
-    DN_LAUNCH_CHECK();
-  }
+  DN_TRY(fused_tiles_build(S, r));
   if (!f.chunks && S->n_panels == 0) {
     DN_CHECK(has_row_major(S), "row-major copy of the matrix was released");
     // entries per workgroup of A H^T: about FU_CHUNKS workgroups in all, at least 256 entries each

@@ -55,7 +55,7 @@ typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
 
 constexpr int FU_GROUP = 256;        // columns whose entries are packed with one base
 constexpr int FU_ROW_BITS = 24;      // a packed entry: row below, column within its 256 above
-constexpr int FU_U = 8;              // gathers in flight per lane group of A H^T
+constexpr int FU_U = 4;              // gathers in flight per lane group of A H^T
 constexpr int FU_U_H = 2;            // the same in the H update, where a lane takes two pieces of a row
 __host__ __device__ constexpr int fu_pairs(int nb) { return nb * (nb + 1) / 2; }
 __device__ inline int fu_pair(int b1, int b2, int nb) { return b1 * nb - b1 * (b1 - 1) / 2 + (b2 - b1); }

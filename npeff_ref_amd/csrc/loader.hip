@@ -111,7 +111,7 @@ static const tuning_entry g_tuning_table[] = {
     {"nl_spin", &tuning_t::nl_spin},             {"nl_wgs", &tuning_t::nl_wgs},
     {"gram_beside", &tuning_t::gram_beside},
     {"gram_fold", &tuning_t::gram_fold},         {"xg_wgs", &tuning_t::xg_wgs},
-    {"h_overlap", &tuning_t::h_overlap},
+    {"h_overlap", &tuning_t::h_overlap},         {"pad_rank", &tuning_t::pad_rank},
 };
 
 static tuning_t tuning_from_env() {
@@ -993,6 +993,7 @@ int csr_ensure_products(dnpeff_csr* A, int r) {
     }
   }
   if (use_tlists(S, r)) DN_TRY(tblocks_build(S));
+  if (use_spmm_t_bal(S, r)) DN_TRY(fused_tiles_build(S, r));
   DN_TRY(csr_ensure_partials(S, r));
   return head_ensure_workspace(A, r);
 }
@@ -1015,8 +1016,9 @@ int csr_consume_for_products(dnpeff_csr* A) {
 }
 
 int csr_tile_lists(dnpeff_csr* A) {
+  dnpeff_csr* S = sparse_part(A);
+  if (S->fused.tiles && S->fused.tile_cols == 32) DN_TRY(fused_tiles_first(S));
   if (A->h_lists_valid) return 0;
-  const dnpeff_csr* S = sparse_part(A);
   A->h_head_cols.assign((size_t)A->head.n_d, 0);
   A->h_long_cols.assign((size_t)S->n_long, 0);
   DN_HIP(hipStreamSynchronize(stream()));

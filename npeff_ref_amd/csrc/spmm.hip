@@ -873,6 +873,140 @@ __global__ void __launch_bounds__(256)
   }
 }
 
+// Entry-balanced A^T W for ranks that fill a wave (r a multiple of 4, up to 256 V) and a W that fits an
+// L2.  A workgroup takes a tile of up to 32 consecutive columns (the tiles of fused.hip: up to 512
+// entries, or one longer column); its four waves take equal shares of the tile's entries, each entry
+// read by the whole wave (16 V bytes per lane).  Row and value are wave-uniform, so the walk over the
+// columns is scalar work beside U gathers in flight.  A column inside a share is stored directly; of
+// one that a share's end cuts, each wave leaves its part in LDS and the parts are added in order.
+// (k_spmm_t_grouped gives a wave 32 whole columns one after the other at these ranks: 180 us where the
+// first 32 columns of 100 rows hold every row, and a gather's latency per column everywhere: 500 x 823k with
+// 4 M entries 637 us at r = 256, 1087 at r = 512.)
+template <int V, bool FULL>
+__global__ void __launch_bounds__(256)
+    k_spmm_t_bal(const fu_tile* __restrict__ tiles, const int64_t* __restrict__ colptr,
+                 const int32_t* __restrict__ rowind, const float* __restrict__ tvals, int r,
+                 const float* __restrict__ W, float* __restrict__ T, int64_t col_base) {
+  extern __shared__ __align__(16) float parts[];  // [4][r] first parts of cut columns, [4][r] later parts
+  __shared__ int first_col[4], later_col[4];      // their columns (-1: none)
+  __shared__ int later_ends[4];
+  constexpr int U = V >= 4 ? 2 : 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int64_t e0 = tiles[blockIdx.x].e0;
+  const int col0 = tiles[blockIdx.x].col0, nc = tiles[blockIdx.x].cols;
+  const int E = (int)(tiles[blockIdx.x + 1].e0 - e0);
+  float* Tt = T + (int64_t)(col0 - col_base) * r;
+  // lane l: first entry of column l of the tile (past the last column: E)
+  const int cp = lane < nc ? (int)(colptr[col0 + lane] - e0) : E;
+  if (lane == 0) first_col[wave] = later_col[wave] = -1;
+  bool ok[V];
+#pragma unroll
+  for (int v = 0; v < V; v++) ok[v] = FULL || 4 * (lane + 64 * v) < r;
+  auto put = [&](float* dst, const float4 (&a)[V]) {
+#pragma unroll
+    for (int v = 0; v < V; v++)
+      if (ok[v]) *reinterpret_cast<float4*>(dst + 4 * (lane + 64 * v)) = a[v];
+  };
+  const float4 zero = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  const int share = (E + 3) / 4;
+  const int s0 = wave * share, s1 = s0 + share < E ? s0 + share : E;
+  if (s0 < s1) {
+    const int32_t* ri = rowind + e0;
+    const float* va = tvals + e0;
+    unsigned off[V];  // (lanes past the rank: any valid place)
+#pragma unroll
+    for (int v = 0; v < V; v++) off[v] = ok[v] ? 4u * (unsigned)(lane + 64 * v) : 0u;
+    // the column of entry s0: the last one that starts at or before it
+    int c = (int)__popcll(__ballot(lane < nc && cp <= s0)) - 1;
+    int next = bcast_i(cp, c + 1);
+    bool later = bcast_i(cp, c) < s0;
+    float4 acc[V];
+#pragma unroll
+    for (int v = 0; v < V; v++) acc[v] = zero;
+    int mi = ri[s0 + lane < s1 ? s0 + lane : s1 - 1];
+    float mv = va[s0 + lane < s1 ? s0 + lane : s1 - 1];
+    for (int b = s0; b < s1; b += 64) {
+      const int cnt = s1 - b < 64 ? s1 - b : 64;
+      const int ne = b + 64 + lane < s1 ? b + 64 + lane : s1 - 1;
+      const int ni = ri[ne];
+      const float nv = va[ne];
+      for (int u = 0; u < cnt; u += U) {
+        float4 h[U][V];
+#pragma unroll
+        for (int k = 0; k < U; k++) {
+          // (past the share's end: entries of weight 0)
+          const float* x = W + (int64_t)bcast_i(mi, (u + k) & 63) * r;
+#pragma unroll
+          for (int v = 0; v < V; v++) h[k][v] = *reinterpret_cast<const float4*>(x + off[v]);
+        }
+#pragma unroll
+        for (int k = 0; k < U; k++) {
+          const int e = b + u + k;
+          if (e < s1) {
+            if (e >= next) {  // column c is complete
+              put(later ? parts + (4 + wave) * r : Tt + (int64_t)c * r, acc);
+              if (later && lane == 0) later_col[wave] = c, later_ends[wave] = 1;
+              later = false;
+              do next = bcast_i(cp, ++c + 1);
+              while (e >= next);
+#pragma unroll
+              for (int v = 0; v < V; v++) acc[v] = zero;
+            }
+            const float a = bcast_f(mv, (u + k) & 63);
+#pragma unroll
+            for (int v = 0; v < V; v++) {
+              acc[v].x = fmaf(a, h[k][v].x, acc[v].x);
+              acc[v].y = fmaf(a, h[k][v].y, acc[v].y);
+              acc[v].z = fmaf(a, h[k][v].z, acc[v].z);
+              acc[v].w = fmaf(a, h[k][v].w, acc[v].w);
+            }
+          }
+        }
+      }
+      mi = ni;
+      mv = nv;
+    }
+    if (later) {
+      put(parts + (4 + wave) * r, acc);
+      if (lane == 0) later_col[wave] = c, later_ends[wave] = next <= s1;
+    } else if (next > s1) {
+      put(parts + wave * r, acc);
+      if (lane == 0) first_col[wave] = c;
+    } else {
+      put(Tt + (int64_t)c * r, acc);
+    }
+  }
+  // columns without entries
+  {
+    const int cn = __shfl(cp, (lane + 1) & 63);
+    unsigned long long empty = __ballot(lane < nc && cp == cn) & (0x1111111111111111ull << wave);
+    float4 z[V];
+#pragma unroll
+    for (int v = 0; v < V; v++) z[v] = zero;
+    while (empty) {
+      const int c = __ffsll(empty) - 1;
+      put(Tt + (int64_t)c * r, z);
+      empty &= empty - 1;
+    }
+  }
+  __syncthreads();
+  const int c = first_col[wave];
+  if (c >= 0) {
+    float4 acc[V];
+#pragma unroll
+    for (int v = 0; v < V; v++) acc[v] = ok[v] ? *reinterpret_cast<const float4*>(parts + wave * r + 4 * (lane + 64 * v)) : zero;
+    for (int w = wave + 1; w < 4 && later_col[w] == c; w++) {
+#pragma unroll
+      for (int v = 0; v < V; v++) {
+        const float4 x = ok[v] ? *reinterpret_cast<const float4*>(parts + (4 + w) * r + 4 * (lane + 64 * v)) : zero;
+        acc[v].x += x.x; acc[v].y += x.y; acc[v].z += x.z; acc[v].w += x.w;
+      }
+      if (later_ends[w]) break;
+    }
+    put(Tt + (int64_t)c * r, acc);
+  }
+}
+
 template <class GT>
 __global__ void __launch_bounds__(256)
     k_spmm_t_long(const int32_t* __restrict__ long_cols, const int64_t* __restrict__ colptr,
@@ -1301,6 +1435,13 @@ static int spmm_t_slices(int64_t n, int r) {
   return v;
 }
 
+// Ranks above 128 (below, a wave reads several rows of W at once) with a W that an L2 holds, unless the
+// switch asks for the older kernel by its slices.
+bool use_spmm_t_bal(const dnpeff_csr* S, int r) {
+  return r > 128 && r <= 1024 && r % 4 == 0 && tuning().spmm_t_slices == 0.0 && 4.0 * (double)S->n_rows * r <= 6.0e6 &&
+         S->nnz > 0 && S->n_cols > 0 && ceil_div(S->n_cols, 32) + S->nnz / 256 < ((int64_t)1 << 24);
+}
+
 // The sparse part of rows [col0, col1) of A^T W into T (row j - col0); long_cols[l0 .. l1) are the
 // long columns in that range.
 static int launch_spmm_t_sparse(const dnpeff_csr* A, int r, const float* W_nr, float* T, int64_t col0,
@@ -1312,6 +1453,33 @@ static int launch_spmm_t_sparse(const dnpeff_csr* A, int r, const float* W_nr, f
   const bool aligned = ((uintptr_t)T % 16) == 0 && ((uintptr_t)W_nr % 16) == 0;
   if (A->tb.cols && aligned && col0 % 64 == 0 && (col1 % 64 == 0 || col1 == A->n_cols) && use_tlists(A, r))
     return launch_spmm_t_lists(A, r, W_nr, T, col0, col1);
+  if (A->fused.tiles && A->fused.tile_cols == 32 && aligned && use_spmm_t_bal(A, r)) {
+    int64_t t0 = 0, t1 = A->fused.n_tiles;
+    if (col0 > 0 || col1 < A->n_cols) {
+      DN_CHECK(!A->fused.h_first.empty() && col0 % 32 == 0 && (col1 % 32 == 0 || col1 == A->n_cols),
+               "column tile [%lld, %lld) does not lie on the plan's groups", (long long)col0, (long long)col1);
+      t0 = A->fused.h_first[col0 / 32];
+      t1 = A->fused.h_first[ceil_div(col1, 32)];
+    }
+    DN_CHECK(t1 - t0 < ((int64_t)1 << 24), "too many tiles for one launch");
+    const dim3 gb((unsigned)(t1 - t0)), bb(256);
+    const size_t lds = sizeof(float) * 8 * (size_t)r;
+#define DN_BAL(V)                                                                                                   \
+  do {                                                                                                              \
+    if (r == 256 * V)                                                                                               \
+      hipLaunchKernelGGL((k_spmm_t_bal<V, true>), gb, bb, lds, stream(), A->fused.tiles + t0, A->colptr, A->rowind, \
+                         A->tvals, r, W_nr, T, col0);                                                               \
+    else                                                                                                            \
+      hipLaunchKernelGGL((k_spmm_t_bal<V, false>), gb, bb, lds, stream(), A->fused.tiles + t0, A->colptr,           \
+                         A->rowind, A->tvals, r, W_nr, T, col0);                                                    \
+  } while (0)
+    if (r <= 256) DN_BAL(1);
+    else if (r <= 512) DN_BAL(2);
+    else DN_BAL(4);
+#undef DN_BAL
+    DN_LAUNCH_CHECK();
+    return 0;
+  }
   const int n_slices = (aligned && r % 4 == 0) ? spmm_t_slices(A->n_rows, r) : 1;
   const int width = r / n_slices;
   // one wave per (column, slice); a launch holds at most 2^32 threads, so beyond 2^23 workgroups
