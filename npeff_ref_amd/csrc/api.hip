@@ -85,7 +85,14 @@ struct Profiler {
 // ---------------------------------------------------------------------------
 struct dnpeff_nmf {
   dnpeff_csr* A = nullptr;
-  int r = 0;
+  int r = 0;                 // components a row of the factors has in memory
+  // The rank.  Ranks above 128 that are not multiples of 128 are stored with zero components up to the
+  // next one (padded_rank): the updates keep those zero, and every kernel made for multiples of 128
+  // runs.  The factors that callers see are packed.
+  int rl = 0;
+  float* Wp = nullptr;       // packed copies handed out by dnpeff_nmf_device_factors, while r != rl
+  float* Hp = nullptr;
+  bool handed_out = false;   // ... since the factors last changed: a caller may have written to them
   float eps = 0.0f;
   uint64_t seed = 0;
   int64_t n = 0, m = 0;
@@ -128,7 +135,7 @@ DN_API int dnpeff_nmf_destroy(dnpeff_nmf* nmf) {
   (void)hipStreamSynchronize(stream());
   dfree(nmf->W); dfree(nmf->W2); dfree(nmf->Nw); dfree(nmf->Hbuf); dfree(nmf->S); dfree(nmf->S2);
   dfree(nmf->G); dfree(nmf->G2); dfree(nmf->gram_ws); dfree(nmf->dot_ws);
-  dfree(nmf->GH); dfree(nmf->gpart);
+  dfree(nmf->GH); dfree(nmf->gpart); dfree(nmf->Wp); dfree(nmf->Hp);
   nmf->fu.destroy();
   delete nmf;
   return 0;
@@ -139,6 +146,11 @@ DN_API int dnpeff_nmf_destroy(dnpeff_nmf* nmf) {
 static bool fused_update(const dnpeff_nmf* h) {
   if (tuning().fused_gram == 0.0 || h->tiled) return false;
   return h->r == 128 && h->m >= 4096;
+}
+
+// Rows that the arrays of a factor have memory for: whole tiles of the update kernel where the rank has one.
+static int64_t rows_there(int r, int64_t rows) {
+  return r > 128 && r % 128 == 0 ? ceil_div(rows, 128) * 128 : rows;
 }
 
 // Columns of a tile of the tiled H update: h_tile_mb MiB of the factor, a multiple of 128.
@@ -283,6 +295,25 @@ static int plan_matrix(dnpeff_csr* A, int rank, bool consume, bool* tiled, bool*
   return split_dense_head_at(A, c.thr, nullptr);
 }
 
+// The rank that the factors are stored with.  At 500 x 823k ten updates take 111 ms at r = 301 as it
+// is (fp32 matrix cores, 4-byte loads) and 41 ms with 384 components of which 83 are zero.  Not
+// where the longer rows do not fit (with the packed copy that callers may ask for), nor without an eps to
+// keep 0 * (0 / eps) zero.
+static int padded_rank(const dnpeff_csr* A, int rank, float eps, int* out) {
+  *out = rank;
+  const int p = (rank + 127) / 128 * 128;
+  if (rank <= 128 || p == rank || !(eps >= 1e-30f) || !use_split_bf16() || tuning().pad_rank == 0.0 ||
+      tuning().tiled_h > 0.0)
+    return 0;
+  size_t free_b = 0, total_b = 0;
+  DN_HIP(hipMemGetInfo(&free_b, &total_b));
+  const plan_table t = plan_overheads(A->n_rows, A->n_cols, A->nnz, p, false, sweeps_for_rank(p), (double)total_b);
+  if (t.total() + 4.0 * (double)rank * (double)(A->n_rows + A->n_cols) + 24.0 * (double)A->nnz <
+      (double)free_b + (double)pool_cached_bytes())
+    *out = p;
+  return 0;
+}
+
 static int nmf_create_impl(dnpeff_csr* A, int rank, float eps, int64_t seed, unsigned flags,
                            dnpeff_nmf** out) {
   clear_error();
@@ -307,8 +338,14 @@ static int nmf_create_impl(dnpeff_csr* A, int rank, float eps, int64_t seed, uns
   double sq_norm = 0.0;
   DN_TRY(dnpeff_csr_sq_norm(A, &sq_norm));
   mark("||A||^2");
+  const int rank_asked = rank;
+  DN_TRY(padded_rank(A, rank_asked, eps, &rank));
   bool tiled = false, fused = false;
   DN_TRY(plan_matrix(A, rank, consume, &tiled, &fused));
+  if (tiled && rank != rank_asked) {  // (only where the two estimates of the memory disagree)
+    rank = rank_asked;
+    DN_TRY(plan_matrix(A, rank, consume, &tiled, &fused));
+  }
   mark("memory plan, dense head and sparse tail");
   if (consume && A->tail) {  // the tail and the head hold everything the products read
     DN_HIP(hipStreamSynchronize(stream()));
@@ -320,13 +357,14 @@ static int nmf_create_impl(dnpeff_csr* A, int rank, float eps, int64_t seed, uns
   if (consume) DN_TRY(csr_consume_for_products(A));
   mark("release of what the products do not read");
   dnpeff_nmf* h = new dnpeff_nmf();
-  h->A = A; h->r = rank; h->eps = eps; h->seed = (uint64_t)seed;
+  h->A = A; h->r = rank; h->rl = rank_asked; h->eps = eps; h->seed = (uint64_t)seed;
   h->n = A->n_rows; h->m = A->n_cols;
   h->sq_norm_A = sq_norm;
   h->tiled = tiled && A->n_cols > 0;
   h->tile_cols = h->tiled ? tile_cols_for(h->m, rank) : 0;
-  const int64_t nr = h->n * rank, mr = h->m * rank;
-  const int64_t h_floats = h->tiled ? (h->m + h->tile_cols) * rank : mr;
+  const int64_t n_there = rows_there(rank, h->n), m_there = rows_there(rank, h->m);
+  const int64_t nr = n_there * rank, mr = m_there * rank;
+  const int64_t h_floats = h->tiled ? (m_there + h->tile_cols) * rank : mr;
   const int64_t s_floats = h->tiled ? h->tile_cols * rank : mr;
   int64_t ws = gram_workspace_floats(h->m, rank);
   int64_t ws_n = gram_workspace_floats(h->n, rank);
@@ -381,9 +419,24 @@ DN_API int dnpeff_nmf_init_factors(dnpeff_nmf* nmf) {
   nmf->nw_valid = false;
   nmf->fu_n_valid = false;
   nmf->fu.gh_state = nmf->fu.gw_state = fused_state::NONE;
+  nmf->handed_out = false;
+  if (nmf->r != nmf->rl) {
+    DN_TRY(launch_init_uniform(0, nmf->n, nmf->rl, nmf->seed, nmf->W2));
+    DN_TRY(launch_copy_rows(nmf->n, nmf->rl, nmf->W2, nmf->rl, nmf->W, nmf->r));
+    DN_TRY(launch_init_uniform(1, nmf->rl, nmf->m, nmf->seed, nmf->S));
+    return launch_copy_rows(nmf->m, nmf->rl, nmf->S, nmf->rl, nmf->H, nmf->r);
+  }
   DN_TRY(launch_init_uniform(0, nmf->n, nmf->r, nmf->seed, nmf->W));
   DN_TRY(launch_init_uniform(1, nmf->r, nmf->m, nmf->seed, nmf->H));
   return 0;
+}
+
+// Packed copies that were handed out become the factors again before anything reads them.
+static int take_back(dnpeff_nmf* h) {
+  if (!h->handed_out) return 0;
+  h->handed_out = false;
+  DN_TRY(launch_copy_rows(h->n, h->rl, h->Wp, h->rl, h->W, h->r));
+  return launch_copy_rows(h->m, h->rl, h->Hp, h->rl, h->H, h->r);
 }
 
 DN_API int dnpeff_nmf_set_factors(dnpeff_nmf* nmf, const float* W_nr, const float* H_rm) {
@@ -391,8 +444,13 @@ DN_API int dnpeff_nmf_set_factors(dnpeff_nmf* nmf, const float* W_nr, const floa
   DN_CHECK(nmf != nullptr, "handle is NULL");
   DN_HIP(hipStreamSynchronize(stream()));
   if (W_nr) nmf->fu.gw_state = fused_state::NONE;
-  if (W_nr)
+  DN_TRY(take_back(nmf));
+  if (W_nr && nmf->r != nmf->rl) {
+    DN_HIP(copy_up(nmf->W2, W_nr, sizeof(float) * nmf->n * nmf->rl));
+    DN_TRY(launch_copy_rows(nmf->n, nmf->rl, nmf->W2, nmf->rl, nmf->W, nmf->r));
+  } else if (W_nr) {
     DN_HIP(copy_up(nmf->W, W_nr, sizeof(float) * nmf->n * nmf->r));
+  }
   if (H_rm) {
     nmf->gh_valid = false;
     nmf->nw_valid = false;
@@ -401,14 +459,15 @@ DN_API int dnpeff_nmf_set_factors(dnpeff_nmf* nmf, const float* W_nr, const floa
     // [r, m] row-major on the host -> [m, r] on the device, through S, a column tile at a time
     // when S holds no more
     const int64_t step = nmf->tiled ? nmf->tile_cols : nmf->m;
+    if (nmf->r != nmf->rl) DN_HIP(hipMemsetAsync(nmf->H, 0, sizeof(float) * nmf->m * nmf->r, stream()));
     for (int64_t c0 = 0; c0 < nmf->m; c0 += step) {
       const int64_t len = nmf->m - c0 < step ? nmf->m - c0 : step;
       if (len == nmf->m)
-        DN_HIP(copy_up(nmf->S, H_rm, sizeof(float) * len * nmf->r));
+        DN_HIP(copy_up(nmf->S, H_rm, sizeof(float) * len * nmf->rl));
       else
         DN_HIP(hipMemcpy2D(nmf->S, sizeof(float) * len, H_rm + c0, sizeof(float) * nmf->m,
-                           sizeof(float) * len, (size_t)nmf->r, hipMemcpyHostToDevice));
-      DN_TRY(launch_transpose(nmf->r, len, nmf->S, nmf->H + c0 * nmf->r));
+                           sizeof(float) * len, (size_t)nmf->rl, hipMemcpyHostToDevice));
+      DN_TRY(launch_transpose_ld(nmf->rl, len, nmf->S, len, nmf->H + c0 * nmf->r, nmf->r));
       DN_HIP(hipStreamSynchronize(stream()));
     }
   }
@@ -464,6 +523,7 @@ static int fused_update_H(dnpeff_nmf* h) {
 
 DN_API int dnpeff_nmf_update_W(dnpeff_nmf* h) {
   DN_CHECK(h != nullptr, "handle is NULL");
+  DN_TRY(take_back(h));
   if (fused_now(h)) return fused_update_W(h);
   h->fu.gw_state = fused_state::NONE;
   dnpeff_csr* A = h->A;
@@ -516,7 +576,7 @@ DN_API int dnpeff_nmf_update_W(dnpeff_nmf* h) {
     Gh = h->G;
   }
   DN_TRY(h->prof.begin(DNPEFF_K_XG_MU_W));
-  DN_TRY(launch_xg_mu(h->n, h->r, h->W, Gh, h->Nw, h->eps, h->W2, nullptr));
+  DN_TRY(launch_xg_mu(h->n, h->r, h->W, Gh, h->Nw, h->eps, h->W2, nullptr, rows_there(h->r, h->n)));
   DN_TRY(h->prof.end());
   std::swap(h->W, h->W2);
   return 0;
@@ -569,7 +629,7 @@ static int update_H_tiled_overlapped(dnpeff_nmf* h) {
     DN_HIP(hipStreamWaitEvent(s1, ev_t[b], 0));
     side_stream_route(true);
     DN_TRY(h->prof.begin(DNPEFF_K_XG_MU_H));
-    DN_TRY(launch_xg_mu(c1 - c0, r, h->H + c0 * r, h->G, Sb, h->eps, Hnew + c0 * r, nullptr));
+    DN_TRY(launch_xg_mu(c1 - c0, r, h->H + c0 * r, h->G, Sb, h->eps, Hnew + c0 * r, nullptr, rows_there(r, c1 - c0)));
     DN_TRY(h->prof.end());
     side_stream_route(false);
     DN_HIP(hipEventRecord(ev_x[b], s1));
@@ -602,7 +662,7 @@ static int update_H_tiled(dnpeff_nmf* h) {
     DN_TRY(q == 0 ? h->prof.begin(DNPEFF_K_SPMM_T) : h->prof.next(DNPEFF_K_SPMM_T));
     DN_TRY(launch_spmm_t_tile(A, r, h->W, c0, c1, h->S));
     DN_TRY(h->prof.next(DNPEFF_K_XG_MU_H));
-    DN_TRY(launch_xg_mu(c1 - c0, r, h->H + c0 * r, h->G, h->S, h->eps, Hnew + c0 * r, nullptr));
+    DN_TRY(launch_xg_mu(c1 - c0, r, h->H + c0 * r, h->G, h->S, h->eps, Hnew + c0 * r, nullptr, rows_there(r, c1 - c0)));
   }
   DN_TRY(h->prof.end());
   h->H = Hnew;
@@ -612,6 +672,7 @@ static int update_H_tiled(dnpeff_nmf* h) {
 
 DN_API int dnpeff_nmf_update_H(dnpeff_nmf* h) {
   DN_CHECK(h != nullptr, "handle is NULL");
+  DN_TRY(take_back(h));
   if (fused_now(h)) return fused_update_H(h);
   h->fu.gh_state = fused_state::NONE;
   h->fu_n_valid = false;
@@ -630,7 +691,7 @@ DN_API int dnpeff_nmf_update_H(dnpeff_nmf* h) {
     DN_TRY(launch_xg_mu_gram(h->m, h->H, h->G, h->S, h->eps, h->S, h->GH, h->gpart, h->G2, h->gram_ws));
     h->gh_valid = true;
   } else {
-    DN_TRY(launch_xg_mu(h->m, h->r, h->H, h->G, h->S, h->eps, h->S, nullptr));
+    DN_TRY(launch_xg_mu(h->m, h->r, h->H, h->G, h->S, h->eps, h->S, nullptr, rows_there(h->r, h->m)));
     h->gh_valid = false;
   }
   DN_TRY(h->prof.end());
@@ -652,6 +713,7 @@ DN_API int dnpeff_nmf_step(dnpeff_nmf* nmf, int n_steps) {
 DN_API int dnpeff_nmf_loss_terms(dnpeff_nmf* h, double* sq_norm_A, double* pos, double* neg) {
   clear_error();
   DN_CHECK(h != nullptr, "handle is NULL");
+  DN_TRY(take_back(h));
   dnpeff_csr* A = h->A;
   if (fused_now(h)) {
     unsigned long long* words = nullptr;
@@ -698,6 +760,7 @@ DN_API int dnpeff_nmf_loss_terms(dnpeff_nmf* h, double* sq_norm_A, double* pos, 
 DN_API int dnpeff_nmf_check_products(dnpeff_nmf* h, double* via_rows, double* via_columns) {
   clear_error();
   DN_CHECK(h && via_rows && via_columns, "NULL argument");
+  DN_TRY(take_back(h));
   dnpeff_csr* A = h->A;
   DN_TRY(products_for(h));
   // <A H^T, W> through the row-ordered structures
@@ -740,40 +803,61 @@ DN_API int dnpeff_nmf_sparsify_W(dnpeff_nmf* nmf, float l1_norm, float l2_norm, 
   DN_CHECK(nmf, "NULL argument");
   // (H^T H and A H^T kept between calls depend on H only)
   nmf->fu.gw_state = fused_state::NONE;
+  DN_TRY(take_back(nmf));
+  if (nmf->r != nmf->rl) {
+    DN_TRY(launch_copy_rows(nmf->n, nmf->rl, nmf->W, nmf->r, nmf->W2, nmf->rl));
+    DN_TRY(sparsify_columns(nmf->n, nmf->rl, nmf->W2, l1_norm, l2_norm, rounds));
+    return launch_copy_rows(nmf->n, nmf->rl, nmf->W2, nmf->rl, nmf->W, nmf->r);
+  }
   return sparsify_columns(nmf->n, nmf->r, nmf->W, l1_norm, l2_norm, rounds);
 }
 
 DN_API int dnpeff_nmf_get_W(dnpeff_nmf* nmf, float* W_nr) {
   clear_error();
   DN_CHECK(nmf && W_nr, "NULL argument");
+  DN_TRY(take_back(nmf));
+  const float* W = nmf->W;
+  if (nmf->r != nmf->rl) {
+    DN_TRY(launch_copy_rows(nmf->n, nmf->rl, nmf->W, nmf->r, nmf->W2, nmf->rl));
+    W = nmf->W2;
+  }
   DN_HIP(hipStreamSynchronize(stream()));
-  DN_HIP(copy_down(W_nr, nmf->W, sizeof(float) * nmf->n * nmf->r));
+  DN_HIP(copy_down(W_nr, W, sizeof(float) * nmf->n * nmf->rl));
   return 0;
 }
 
 DN_API int dnpeff_nmf_get_H(dnpeff_nmf* nmf, float* H_rm) {
   clear_error();
   DN_CHECK(nmf && H_rm, "NULL argument");
+  DN_TRY(take_back(nmf));
   // [m, r] on the device -> [r, m] row-major on the host, through S: all at once, or a column
   // tile at a time when S holds no more (the tiled H update)
   const int64_t step = nmf->tiled ? nmf->tile_cols : nmf->m;
   for (int64_t c0 = 0; c0 < nmf->m; c0 += step) {
     const int64_t len = nmf->m - c0 < step ? nmf->m - c0 : step;
-    DN_TRY(launch_transpose(len, nmf->r, nmf->H + c0 * nmf->r, nmf->S));
+    DN_TRY(launch_transpose_ld(len, nmf->rl, nmf->H + c0 * nmf->r, nmf->r, nmf->S, len));
     DN_HIP(hipStreamSynchronize(stream()));
     if (len == nmf->m)
-      DN_HIP(copy_down(H_rm, nmf->S, sizeof(float) * len * nmf->r));
+      DN_HIP(copy_down(H_rm, nmf->S, sizeof(float) * len * nmf->rl));
     else
       DN_HIP(hipMemcpy2D(H_rm + c0, sizeof(float) * nmf->m, nmf->S, sizeof(float) * len,
-                         sizeof(float) * len, (size_t)nmf->r, hipMemcpyDeviceToHost));
+                         sizeof(float) * len, (size_t)nmf->rl, hipMemcpyDeviceToHost));
   }
   return 0;
 }
 
 DN_API int dnpeff_nmf_device_factors(dnpeff_nmf* nmf, void** W_dev, void** H_dev) {
   DN_CHECK(nmf != nullptr, "handle is NULL");
-  if (W_dev) *W_dev = nmf->W;
-  if (H_dev) *H_dev = nmf->H;
+  if (nmf->r != nmf->rl && !nmf->handed_out) {
+    if (!nmf->Wp) DN_TRY(dmalloc(&nmf->Wp, nmf->n * nmf->rl));
+    if (!nmf->Hp) DN_TRY(dmalloc(&nmf->Hp, nmf->m * nmf->rl));
+    DN_TRY(launch_copy_rows(nmf->n, nmf->rl, nmf->W, nmf->r, nmf->Wp, nmf->rl));
+    DN_TRY(launch_copy_rows(nmf->m, nmf->rl, nmf->H, nmf->r, nmf->Hp, nmf->rl));
+    nmf->handed_out = true;
+  }
+  const bool packed = nmf->r != nmf->rl;
+  if (W_dev) *W_dev = packed ? nmf->Wp : nmf->W;
+  if (H_dev) *H_dev = packed ? nmf->Hp : nmf->H;
   return 0;
 }
 

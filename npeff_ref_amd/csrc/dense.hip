@@ -6,6 +6,7 @@
 #include "abt_b16.hpp"
 #include "synth_rng.h"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace dn {
@@ -77,7 +78,7 @@ static int gram_pairs(int r) {
   return nb * (nb + 1) / 2;
 }
 
-static bool gram_uses_tiles(int64_t rows, int r) { return r > 128 && r % 128 == 0 && rows >= 1024; }
+static bool gram_uses_tiles(int64_t rows, int r) { return r > 128 && r % 128 == 0 && rows >= 128; }
 
 static int64_t gram_small_wgs(int64_t rows);
 
@@ -1154,7 +1155,7 @@ int xg_mu_hold_g(const float* G, int r) {
 void xg_mu_release_g() { g_gt_of = nullptr; }
 
 static int launch_xg_mu_tile_b16(int64_t rows, int r, const float* X, const float* G, const float* num,
-                                 float eps, float* out, float* D_out) {
+                                 float eps, float* out, float* D_out, int64_t rows_there) {
   static bool attr_set = false;
   if (!attr_set) {
     DN_HIP(hipFuncSetAttribute((const void*)k_xg_mu_tile_b16<false>,
@@ -1165,6 +1166,9 @@ static int launch_xg_mu_tile_b16(int64_t rows, int r, const float* X, const floa
   }
   if (!(g_gt_of == G && g_gt_rank == r)) DN_TRY(xg_mu_transpose_g(G, r));
   const int n_chunks = r / 128;
+  // (where the arrays go on to the end of the last tile, it is a whole one: the fp32 kernel on fewer than
+  // 128 rows takes 25 to 55 us, as long as 40 million elements of the whole tiles)
+  if (!D_out && rows_there >= ceil_div(rows, 128) * 128) rows = ceil_div(rows, 128) * 128;
   const int64_t tiles = rows / 128;
   // The last rows (fewer than 128, through the fp32 kernel: two workgroups that take a third of
   // the time of a few hundred row tiles) run on the second stream beside the whole tiles.
@@ -1789,7 +1793,7 @@ DN_API int dnpeff_op_xg_mu_gram(int64_t rows, const float* X, const float* G_rr,
 }
 
 int launch_xg_mu(int64_t rows, int r, const float* X, const float* G, const float* num, float eps,
-                 float* out, float* D_out) {
+                 float* out, float* D_out, int64_t rows_there) {
   DN_CHECK(r >= 1 && r <= 1024, "rank %d outside [1, 1024]", r);
   DN_CHECK(out != X, "xg_mu: out must not alias X");
   if (rows <= 0) return 0;
@@ -1812,10 +1816,11 @@ int launch_xg_mu(int64_t rows, int r, const float* X, const float* G, const floa
     return launch_xg_mu_nb<4>(rows - head, r, X + off, G, num + off, eps, out + off,
                               D_out ? D_out + off : nullptr);
   }
-  if (r > 128 && r % 128 == 0 && aligned && ((uintptr_t)G % 16) == 0 && rows >= 256 &&
+  if (r > 128 && r % 128 == 0 && aligned && ((uintptr_t)G % 16) == 0 &&
+      (rows >= 256 || (rows_there >= ceil_div(rows, 128) * 128 && use_split_bf16())) &&
       ceil_div(rows, 128) * (r / 128) < ((int64_t)1 << 24)) {
     if (use_split_bf16() && ((uintptr_t)num % 4) == 0)
-      return launch_xg_mu_tile_b16(rows, r, X, G, num, eps, out, D_out);
+      return launch_xg_mu_tile_b16(rows, r, X, G, num, eps, out, D_out, rows_there);
     return launch_xg_mu_tile(rows, r, X, G, num, eps, out, D_out);
   }
   // widest column chunk whose slice of G fits 128 KB of LDS
@@ -1898,10 +1903,11 @@ int launch_init_uniform(int matrix_id, int64_t logical_rows, int64_t logical_col
 }
 
 // ---------------------------------------------------------------------------
-// out[c * rows + i] = in[i * cols + c], 32 x 32 tiles through LDS.
+// out[c * ldo + i] = in[i * ldi + c], 32 x 32 tiles through LDS.
 // ---------------------------------------------------------------------------
 __global__ void __launch_bounds__(256)
-    k_transpose(const float* __restrict__ in, int64_t rows, int64_t cols, float* __restrict__ out) {
+    k_transpose(const float* __restrict__ in, int64_t rows, int64_t cols, int64_t ldi, float* __restrict__ out,
+                int64_t ldo) {
   __shared__ float tile[32][33];
   const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;  // 32 x 8
   const int64_t tiles_c = (cols + 31) / 32, tiles_r = (rows + 31) / 32;
@@ -1910,23 +1916,45 @@ __global__ void __launch_bounds__(256)
     const int64_t r0 = tile_r * 32, c0 = tile_c * 32;
     for (int i = ty; i < 32; i += 8) {
       int64_t rr = r0 + i, cc = c0 + tx;
-      tile[i][tx] = (rr < rows && cc < cols) ? in[rr * cols + cc] : 0.0f;
+      tile[i][tx] = (rr < rows && cc < cols) ? in[rr * ldi + cc] : 0.0f;
     }
     __syncthreads();
     for (int i = ty; i < 32; i += 8) {
       int64_t cc = c0 + i, rr = r0 + tx;
-      if (cc < cols && rr < rows) out[cc * rows + rr] = tile[tx][i];
+      if (cc < cols && rr < rows) out[cc * ldo + rr] = tile[tx][i];
     }
     __syncthreads();
   }
 }
 
-int launch_transpose(int64_t rows, int64_t cols, const float* in, float* out) {
+int launch_transpose_ld(int64_t rows, int64_t cols, const float* in, int64_t ldi, float* out, int64_t ldo) {
   if (rows <= 0 || cols <= 0) return 0;
   int64_t tiles = ceil_div(rows, 32) * ceil_div(cols, 32);
   if (tiles > ((int64_t)1 << 22)) tiles = (int64_t)1 << 22;  // the kernel loops over the rest
-  hipLaunchKernelGGL(k_transpose, dim3((unsigned)tiles), dim3(256), 0, stream(), in, rows, cols,
-                     out);
+  hipLaunchKernelGGL(k_transpose, dim3((unsigned)tiles), dim3(256), 0, stream(), in, rows, cols, ldi,
+                     out, ldo);
+  DN_LAUNCH_CHECK();
+  return 0;
+}
+
+int launch_transpose(int64_t rows, int64_t cols, const float* in, float* out) {
+  return launch_transpose_ld(rows, cols, in, cols, out, rows);
+}
+
+// Rows of w floats between leading dimensions: out[i * ldo + c] = in[i * ldi + c], zeros from w to ldo
+// when ldo is the longer one.
+__global__ void __launch_bounds__(256)
+    k_copy_rows(const float* __restrict__ in, int64_t rows, int w, int ldi, float* __restrict__ out, int ldo) {
+  // a wave per row at a time
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  for (int64_t i = (int64_t)blockIdx.x * 4 + wave; i < rows; i += (int64_t)gridDim.x * 4)
+    for (int c = lane; c < ldo; c += 64) out[i * ldo + c] = c < w ? in[i * ldi + c] : 0.0f;
+}
+
+int launch_copy_rows(int64_t rows, int w, const float* in, int ldi, float* out, int ldo) {
+  if (rows <= 0) return 0;
+  const int64_t wgs = std::min<int64_t>(ceil_div(rows, 4), 1 << 16);
+  hipLaunchKernelGGL(k_copy_rows, dim3((unsigned)wgs), dim3(256), 0, stream(), in, rows, w, ldi, out, ldo);
   DN_LAUNCH_CHECK();
   return 0;
 }

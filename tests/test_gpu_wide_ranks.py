@@ -1,0 +1,84 @@
+"""Ranks above 128: the entry-balanced A^T W, X^T X on few rows, and ranks stored with zero components up to
+the next multiple of 128."""
+
+import numpy as np
+import pytest
+
+import npeff_ref_amd as d
+from oracle import oracle as orc
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("r", [132, 256, 300, 512, 520, 1024])
+@pytest.mark.parametrize("n,m", [(1, 1), (3, 31), (600, 33), (257, 200)])
+def test_spmm_t_balanced(n, m, r):
+    """Columns inside a wave's share, cut by one, two and three of its ends, longer than a tile, empty."""
+    rng = np.random.default_rng(n + m + r)
+    fill = rng.choice([0.0, 0.003, 0.02, 0.3, 1.0], size=m)
+    mask = rng.random((n, m)) < fill
+    mask[0, 0] = True
+    rp = np.concatenate([[0], np.cumsum(mask.sum(axis=1))]).astype(np.int64)
+    ci = np.nonzero(mask)[1].astype(np.int32)
+    va = rng.random(len(ci)).astype(np.float32)
+    A = d.Csr.from_host(rp, ci, va, m)
+    W = rng.random((n, r)).astype(np.float32)
+    dW, dT = d.DeviceArray.from_numpy(W), d.DeviceArray.from_numpy(np.full((m, r), np.nan, dtype=np.float32))
+    d.op_spmm_t(A, r, dW, dT)
+    d.sync()
+    dense = np.zeros((n, m))
+    dense[mask] = va
+    want = dense.T @ W.astype(np.float64)
+    assert np.abs(dT.numpy() - want).max() <= 1e-5 * max(1.0, np.abs(want).max())
+    A.close()
+
+
+@pytest.mark.parametrize("rows", [128, 129, 160, 191, 1023])
+@pytest.mark.parametrize("r", [256, 384, 512, 768])
+def test_gram_on_few_rows(rows, r):
+    X = np.random.default_rng(rows + r).random((rows, r)).astype(np.float32)
+    dX, dG = d.DeviceArray.from_numpy(X), d.DeviceArray((r, r))
+    d.op_gram(dX, dG)
+    d.sync()
+    want = X.astype(np.float64).T @ X
+    assert (np.abs(dG.numpy() - want) / want).max() <= 2e-6
+
+
+@pytest.mark.parametrize("n,m_full,k,r", [(40, 4000, 200, 129), (300, 30000, 900, 200), (1100, 60000, 2000, 301)])
+def test_rank_between_the_tiles_of_128(n, m_full, k, r):
+    eps = 1e-8
+    A, norms = d.Csr.synth(n, m_full, k_fixed=k, seed=r)
+    A.normalize_rows(norms)
+    A.compact_columns(1)
+    rp, ci, va = A.download()
+    nmf = d.MuNmf(A, d.MuNmfParams(rank=r, max_iters=4, eps=eps, seed=7, log_every=2))
+    nmf.initialize()
+    W0, H0 = nmf.loadWToHostSync(), nmf.loadHToHostSync()
+    assert W0[1, r - 1] == np.float32(d.uniform_at(7, 0, 1, r - 1, r))
+    assert H0[r - 1, 3] == np.float32(d.uniform_at(7, 1, r - 1, 3, A.n_cols))
+    nmf.run(log=lambda s: None)
+    W64, H64, losses = orc.nmf_f64(rp, ci, va, A.n_cols, W0, H0, np.float32(eps), 4, 2)
+    W, H = nmf.loadWToHostSync(), nmf.loadHToHostSync()
+    assert np.linalg.norm(W - W64) <= 1e-5 * np.linalg.norm(W64)
+    assert np.linalg.norm(H - H64) <= 1e-5 * np.linalg.norm(H64)
+    assert abs(nmf.computeUncachedLoss() - losses[-1]) <= 1e-5 * losses[-1]
+    # the factors as callers see them are packed, and what they write to them counts
+    w_dev, h_dev = nmf.device_factors()
+    cols = np.array([0, A.n_cols - 1, 5], dtype=np.int32)
+    assert np.array_equal(d.gather_rows(h_dev, r, cols), H[:, cols].T)
+    assert np.array_equal(d.gather_rows(w_dev, r, np.arange(n)), W)
+    d.binding._check(d.lib.dnpeff_dev_upload(w_dev, d.binding._ptr(W0), W0.nbytes))
+    assert np.array_equal(nmf.loadWToHostSync(), W0)
+    # from the host, and a step on
+    nmf.set_factors(W0, H0)
+    assert np.array_equal(nmf.loadWToHostSync(), W0) and np.array_equal(nmf.loadHToHostSync(), H0)
+    nmf.step(4)
+    assert np.array_equal(nmf.loadWToHostSync(), W) and np.array_equal(nmf.loadHToHostSync(), H)
+    via_rows, via_cols = nmf.check_products()
+    assert abs(via_rows - via_cols) <= 1e-5 * abs(via_rows)
+    # the sparseness projection sees the rank's own components
+    dW = d.DeviceArray.from_numpy(W)
+    rounds = d.binding.op_sparsify_columns(dW, 3.0)
+    assert nmf.sparsify_W(3.0) == rounds and np.array_equal(nmf.loadWToHostSync(), dW.numpy())
+    nmf.close()
+    A.close()
