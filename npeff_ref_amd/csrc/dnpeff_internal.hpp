@@ -277,7 +277,7 @@ struct fused_plan {
   fu_tile* tiles = nullptr;  // [n_tiles + 1]: the last one only ends the entries
   int64_t n_tiles = 0;
   int tile_cols = 0;
-  int64_t tile_most = 0;
+  int64_t tile_most = 0, tile_alone = 0;
   std::vector<int64_t> h_first;  // first tile of every group of tile_cols columns, for products on column tiles
   uint2* pairs = nullptr;    // [nnz + 1]
   fu_chunk* chunks = nullptr;

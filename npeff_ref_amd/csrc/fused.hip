@@ -501,43 +501,47 @@ __global__ void __launch_bounds__(256)
 // ---------------------------------------------------------------------------
 // Tiles of the aligned group of `tc` columns `grp`: f(first column, columns) for each, in order.
 template <class F>
-__device__ inline void fu_split_group(const int64_t* __restrict__ colptr, int64_t m, int tc, int64_t most, int64_t grp,
-                                      F&& f) {
+__device__ inline void fu_split_group(const int64_t* __restrict__ colptr, int64_t m, int tc, int64_t most, int64_t alone,
+                                      int64_t grp, F&& f) {
   const int64_t j0 = grp * tc, j1 = j0 + tc < m ? j0 + tc : m;
   int64_t start = j0, e0 = colptr[j0], before = e0;
-  if (colptr[j1] - e0 <= most) {
+  bool after_lone = false;
+  if (colptr[j1] - e0 <= (most < alone ? most : alone)) {
     f(j0, (int)(j1 - j0));
     return;
   }
   for (int64_t j = j0; j < j1; j++) {
     const int64_t e1 = colptr[j + 1];
-    if (e1 - e0 > most && j > start) {
+    // (a column longer than `alone` shares its tile with no other)
+    const bool lone = e1 - before > alone;
+    if ((e1 - e0 > most || lone || after_lone) && j > start) {
       f(start, (int)(j - start));
       start = j;
       e0 = before;
     }
+    after_lone = lone;
     before = e1;
   }
   f(start, (int)(j1 - start));
 }
 
 __global__ void __launch_bounds__(256)
-    k_fu_count_tiles(const int64_t* __restrict__ colptr, int64_t m, int tc, int64_t most, int64_t groups,
+    k_fu_count_tiles(const int64_t* __restrict__ colptr, int64_t m, int tc, int64_t most, int64_t alone, int64_t groups,
                      int* __restrict__ count) {
   const int64_t grp = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (grp >= groups) return;
   int k = 0;
-  fu_split_group(colptr, m, tc, most, grp, [&](int64_t, int) { k++; });
+  fu_split_group(colptr, m, tc, most, alone, grp, [&](int64_t, int) { k++; });
   count[grp] = k;
 }
 
 __global__ void __launch_bounds__(256)
-    k_fu_make_tiles(const int64_t* __restrict__ colptr, int64_t m, int tc, int64_t most, int64_t groups,
+    k_fu_make_tiles(const int64_t* __restrict__ colptr, int64_t m, int tc, int64_t most, int64_t alone, int64_t groups,
                     const int64_t* __restrict__ first, fu_tile* __restrict__ tiles) {
   const int64_t grp = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (grp >= groups) return;
   int64_t k = first[grp];
-  fu_split_group(colptr, m, tc, most, grp, [&](int64_t col, int cols) {
+  fu_split_group(colptr, m, tc, most, alone, grp, [&](int64_t col, int cols) {
     tiles[k].e0 = colptr[col];
     tiles[k].col0 = (int32_t)col;
     tiles[k].cols = cols;
@@ -603,18 +607,18 @@ static int fu_tile_cols(int64_t m, int r) {
   return m >= (int64_t)tc * 2 * n_cus() || tc < 64 ? tc : 64;
 }
 
-static int fused_tiles_make(dnpeff_csr* S, int tc, int64_t most, bool with_first) {
+static int fused_tiles_make(dnpeff_csr* S, int tc, int64_t most, int64_t alone, bool with_first) {
   fused_plan& f = S->fused;
   hipStream_t st = stream();
   DN_CHECK(S->colptr && S->n_cols > 0, "matrix has no transposed copy");
-  if (!f.tiles || f.tile_cols != tc || f.tile_most != most || (with_first && f.h_first.empty())) {
+  if (!f.tiles || f.tile_cols != tc || f.tile_most != most || f.tile_alone != alone || (with_first && f.h_first.empty())) {
     const int64_t m = S->n_cols, groups = ceil_div(m, tc);
     dbuf<int> count;
     dbuf<int64_t> first;
     DN_TRY(count.alloc(groups));
     DN_TRY(first.alloc(groups + 1));
     const dim3 grid((unsigned)ceil_div(groups, 256)), block(256);
-    hipLaunchKernelGGL(k_fu_count_tiles, grid, block, 0, st, S->colptr, m, tc, most, groups, count.p);
+    hipLaunchKernelGGL(k_fu_count_tiles, grid, block, 0, st, S->colptr, m, tc, most, alone, groups, count.p);
     DN_LAUNCH_CHECK();
     DN_TRY(scan_counts_i64(count, groups, first));
     int64_t n_tiles = 0;
@@ -631,7 +635,8 @@ static int fused_tiles_make(dnpeff_csr* S, int tc, int64_t most, bool with_first
     f.n_tiles = n_tiles;
     f.tile_cols = tc;
     f.tile_most = most;
-    hipLaunchKernelGGL(k_fu_make_tiles, grid, block, 0, st, S->colptr, m, tc, most, groups, first.p, f.tiles);
+    f.tile_alone = alone;
+    hipLaunchKernelGGL(k_fu_make_tiles, grid, block, 0, st, S->colptr, m, tc, most, alone, groups, first.p, f.tiles);
     DN_LAUNCH_CHECK();
   }
   return 0;
@@ -644,10 +649,12 @@ int fused_tiles_build(dnpeff_csr* S, int r) {
   // entries, r = 90: 57 against 63 ms; at r = 20 smaller tiles are the better ones, 16.4 against 18.6).
   int64_t most = 16 * tc;
   if (r > FUSED_NARROW_RANK && r <= FUSED_MAX_RANK) most = std::max<int64_t>(most, S->nnz / (16 * (int64_t)n_cus()));
-  return fused_tiles_make(S, tc, most, false);
+  return fused_tiles_make(S, tc, most, r > FUSED_MAX_RANK ? SPMM_T_LONG : INT64_MAX, false);
 }
 
-int fused_tiles_first(dnpeff_csr* S) { return fused_tiles_make(S, S->fused.tile_cols, S->fused.tile_most, true); }
+int fused_tiles_first(dnpeff_csr* S) {
+  return fused_tiles_make(S, S->fused.tile_cols, S->fused.tile_most, S->fused.tile_alone, true);
+}
 
 int fused_plan_build(dnpeff_csr* S, int r) {
   fused_plan& f = S->fused;
@@ -857,6 +864,10 @@ bool fused_supported(int64_t n, int64_t m, int64_t nnz, int r) {
   // small factors are held to within 1e-5 of the two-pass path over 50 iterations, closer than two
   // ways of rounding stay to each other (both are within 2e-5 of fp64): those keep the separate kernels.
   if (r == 128 && m < 65536) return false;
+  // With as many components as rows the product can become A itself: the loss is then a difference of
+  // nearly equal sums whose digits depend on the order of every sum before it.  Such runs stay on the
+  // kernels they have always had.
+  if (r >= n) return false;
   return r >= 1 && r <= FUSED_MAX_RANK && n >= 1 && m >= 1 && nnz >= 1 && n < ((int64_t)1 << FU_ROW_BITS) &&
          n * (int64_t)r < ((int64_t)1 << 30);  // (byte offsets into W in 32 bits)
 }

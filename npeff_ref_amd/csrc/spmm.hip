@@ -874,55 +874,60 @@ __global__ void __launch_bounds__(256)
 }
 
 // Entry-balanced A^T W for ranks that fill a wave (r a multiple of 4, up to 256 V) and a W that fits an
-// L2.  A workgroup takes a tile of up to 32 consecutive columns (the tiles of fused.hip: up to 512
-// entries, or one longer column); its four waves take equal shares of the tile's entries, each entry
-// read by the whole wave (16 V bytes per lane).  Row and value are wave-uniform, so the walk over the
-// columns is scalar work beside U gathers in flight.  A column inside a share is stored directly; of
-// one that a share's end cuts, each wave leaves its part in LDS and the parts are added in order.
+// L2.  A workgroup takes a tile of up to 32 consecutive columns and 512 entries (the tiles of
+// fused.hip); the tile's entries are cut into four equal shares and a wave takes the columns that start
+// in its share, each entry read by the whole wave (16 V bytes per lane).  Row, value and the end of a
+// column are wave-uniform, so the walk over the columns is scalar work beside U gathers in flight, across
+// the ends of columns.  A column of more than SPMM_T_LONG entries is a tile of its own, a quarter for
+// each wave, added in wave order.  Every column is summed in the order k_spmm_t_grouped and k_spmm_t_long
+// sum it: the same bits.
 // (k_spmm_t_grouped gives a wave 32 whole columns one after the other at these ranks: 180 us where the
 // first 32 columns of 100 rows hold every row, and a gather's latency per column everywhere: 500 x 823k with
-// 4 M entries 637 us at r = 256, 1087 at r = 512.)
+// 4 M entries 637 us at r = 256, 1087 at r = 512; here 305 and 531.)
 template <int V, bool FULL>
 __global__ void __launch_bounds__(256)
     k_spmm_t_bal(const fu_tile* __restrict__ tiles, const int64_t* __restrict__ colptr,
                  const int32_t* __restrict__ rowind, const float* __restrict__ tvals, int r,
                  const float* __restrict__ W, float* __restrict__ T, int64_t col_base) {
-  extern __shared__ __align__(16) float parts[];  // [4][r] first parts of cut columns, [4][r] later parts
-  __shared__ int first_col[4], later_col[4];      // their columns (-1: none)
-  __shared__ int later_ends[4];
-  constexpr int U = V >= 4 ? 2 : 4;
+  extern __shared__ __align__(16) float parts[];  // [4][r] of a long column
+  constexpr int U = V == 1 ? 8 : V == 2 ? 4 : 2;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int64_t e0 = tiles[blockIdx.x].e0;
   const int col0 = tiles[blockIdx.x].col0, nc = tiles[blockIdx.x].cols;
   const int E = (int)(tiles[blockIdx.x + 1].e0 - e0);
+  const bool whole = nc > 1 || E <= SPMM_T_LONG;
   float* Tt = T + (int64_t)(col0 - col_base) * r;
   // lane l: first entry of column l of the tile (past the last column: E)
   const int cp = lane < nc ? (int)(colptr[col0 + lane] - e0) : E;
-  if (lane == 0) first_col[wave] = later_col[wave] = -1;
-  bool ok[V];
+  unsigned off[V];  // (lanes past the rank: any valid place)
 #pragma unroll
-  for (int v = 0; v < V; v++) ok[v] = FULL || 4 * (lane + 64 * v) < r;
+  for (int v = 0; v < V; v++) off[v] = FULL || 4 * (lane + 64 * v) < r ? 4u * (unsigned)(lane + 64 * v) : 0u;
   auto put = [&](float* dst, const float4 (&a)[V]) {
 #pragma unroll
     for (int v = 0; v < V; v++)
-      if (ok[v]) *reinterpret_cast<float4*>(dst + 4 * (lane + 64 * v)) = a[v];
+      if (FULL || 4 * (lane + 64 * v) < r) *reinterpret_cast<float4*>(dst + 4 * (lane + 64 * v)) = a[v];
   };
   const float4 zero = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-  const int share = (E + 3) / 4;
-  const int s0 = wave * share, s1 = s0 + share < E ? s0 + share : E;
+  float4 acc[V];
+#pragma unroll
+  for (int v = 0; v < V; v++) acc[v] = zero;
+  // the wave's columns [c, c1) and entries [s0, s1)
+  int c = 0, c1 = 1, s0, s1;
+  if (whole) {
+    const int share = (E + 3) / 4;
+    c = (int)__popcll(__ballot(lane < nc && cp < wave * share));
+    c1 = wave == 3 ? nc : (int)__popcll(__ballot(lane < nc && cp < (wave + 1) * share));
+    s0 = bcast_i(cp, c);
+    s1 = bcast_i(cp, c1);
+  } else {
+    const int per = ((E + 3) / 4 + 63) / 64 * 64;
+    s0 = wave * per < E ? wave * per : E;
+    s1 = s0 + per < E ? s0 + per : E;
+  }
+  int next = whole ? bcast_i(cp, c + 1) : E;
   if (s0 < s1) {
     const int32_t* ri = rowind + e0;
     const float* va = tvals + e0;
-    unsigned off[V];  // (lanes past the rank: any valid place)
-#pragma unroll
-    for (int v = 0; v < V; v++) off[v] = ok[v] ? 4u * (unsigned)(lane + 64 * v) : 0u;
-    // the column of entry s0: the last one that starts at or before it
-    int c = (int)__popcll(__ballot(lane < nc && cp <= s0)) - 1;
-    int next = bcast_i(cp, c + 1);
-    bool later = bcast_i(cp, c) < s0;
-    float4 acc[V];
-#pragma unroll
-    for (int v = 0; v < V; v++) acc[v] = zero;
     int mi = ri[s0 + lane < s1 ? s0 + lane : s1 - 1];
     float mv = va[s0 + lane < s1 ? s0 + lane : s1 - 1];
     for (int b = s0; b < s1; b += 64) {
@@ -934,7 +939,6 @@ __global__ void __launch_bounds__(256)
         float4 h[U][V];
 #pragma unroll
         for (int k = 0; k < U; k++) {
-          // (past the share's end: entries of weight 0)
           const float* x = W + (int64_t)bcast_i(mi, (u + k) & 63) * r;
 #pragma unroll
           for (int v = 0; v < V; v++) h[k][v] = *reinterpret_cast<const float4*>(x + off[v]);
@@ -943,12 +947,9 @@ __global__ void __launch_bounds__(256)
         for (int k = 0; k < U; k++) {
           const int e = b + u + k;
           if (e < s1) {
-            if (e >= next) {  // column c is complete
-              put(later ? parts + (4 + wave) * r : Tt + (int64_t)c * r, acc);
-              if (later && lane == 0) later_col[wave] = c, later_ends[wave] = 1;
-              later = false;
-              do next = bcast_i(cp, ++c + 1);
-              while (e >= next);
+            while (e >= next) {  // column c is complete
+              put(Tt + (int64_t)c * r, acc);
+              next = bcast_i(cp, ++c + 1);
 #pragma unroll
               for (int v = 0; v < V; v++) acc[v] = zero;
             }
@@ -966,44 +967,23 @@ __global__ void __launch_bounds__(256)
       mi = ni;
       mv = nv;
     }
-    if (later) {
-      put(parts + (4 + wave) * r, acc);
-      if (lane == 0) later_col[wave] = c, later_ends[wave] = next <= s1;
-    } else if (next > s1) {
-      put(parts + wave * r, acc);
-      if (lane == 0) first_col[wave] = c;
-    } else {
+  }
+  if (whole) {
+    for (; c < c1; c++) {  // the last column (and columns without entries)
       put(Tt + (int64_t)c * r, acc);
-    }
-  }
-  // columns without entries
-  {
-    const int cn = __shfl(cp, (lane + 1) & 63);
-    unsigned long long empty = __ballot(lane < nc && cp == cn) & (0x1111111111111111ull << wave);
-    float4 z[V];
 #pragma unroll
-    for (int v = 0; v < V; v++) z[v] = zero;
-    while (empty) {
-      const int c = __ffsll(empty) - 1;
-      put(Tt + (int64_t)c * r, z);
-      empty &= empty - 1;
+      for (int v = 0; v < V; v++) acc[v] = zero;
     }
+    return;
   }
+  put(parts + wave * r, acc);
   __syncthreads();
-  const int c = first_col[wave];
-  if (c >= 0) {
-    float4 acc[V];
-#pragma unroll
-    for (int v = 0; v < V; v++) acc[v] = ok[v] ? *reinterpret_cast<const float4*>(parts + wave * r + 4 * (lane + 64 * v)) : zero;
-    for (int w = wave + 1; w < 4 && later_col[w] == c; w++) {
-#pragma unroll
-      for (int v = 0; v < V; v++) {
-        const float4 x = ok[v] ? *reinterpret_cast<const float4*>(parts + (4 + w) * r + 4 * (lane + 64 * v)) : zero;
-        acc[v].x += x.x; acc[v].y += x.y; acc[v].z += x.z; acc[v].w += x.w;
-      }
-      if (later_ends[w]) break;
-    }
-    put(Tt + (int64_t)c * r, acc);
+  for (int i = threadIdx.x; i < r; i += 256) {
+    float s = parts[i];
+    s += parts[r + i];
+    s += parts[2 * r + i];
+    s += parts[3 * r + i];
+    Tt[i] = s;
   }
 }
 
@@ -1463,7 +1443,7 @@ static int launch_spmm_t_sparse(const dnpeff_csr* A, int r, const float* W_nr, f
     }
     DN_CHECK(t1 - t0 < ((int64_t)1 << 24), "too many tiles for one launch");
     const dim3 gb((unsigned)(t1 - t0)), bb(256);
-    const size_t lds = sizeof(float) * 8 * (size_t)r;
+    const size_t lds = sizeof(float) * 4 * (size_t)r;
 #define DN_BAL(V)                                                                                                   \
   do {                                                                                                              \
     if (r == 256 * V)                                                                                               \
