@@ -750,7 +750,7 @@ DN_API int dnpeff_nmf_loss_terms(dnpeff_nmf* h, double* sq_norm_A, double* pos, 
   DN_TRY(launch_dot((int64_t)h->r * h->r, Gh, h->G2, h->dot_ws, h->dot_ws + DOT_BLOCKS + 1));
   double res[2];
   DN_HIP(hipStreamSynchronize(stream()));
-  DN_HIP(hipMemcpy(res, h->dot_ws + DOT_BLOCKS, sizeof(double) * 2, hipMemcpyDeviceToHost));
+  DN_HIP(copy_down(res, h->dot_ws + DOT_BLOCKS, sizeof(double) * 2));
   if (sq_norm_A) *sq_norm_A = h->sq_norm_A;
   if (neg) *neg = res[0];
   if (pos) *pos = res[1];
@@ -769,7 +769,7 @@ DN_API int dnpeff_nmf_check_products(dnpeff_nmf* h, double* via_rows, double* vi
   h->nw_valid = true;
   DN_TRY(launch_dot(h->n * h->r, h->Nw, h->W, h->dot_ws, h->dot_ws + DOT_BLOCKS));
   DN_HIP(hipStreamSynchronize(stream()));
-  DN_HIP(hipMemcpy(via_rows, h->dot_ws + DOT_BLOCKS, sizeof(double), hipMemcpyDeviceToHost));
+  DN_HIP(copy_down(via_rows, h->dot_ws + DOT_BLOCKS, sizeof(double)));
   // <A^T W, H> through the column-ordered ones (S is free between two H updates)
   double sum = 0.0;
   const int64_t step = h->tiled ? h->tile_cols : h->m;
@@ -783,7 +783,7 @@ DN_API int dnpeff_nmf_check_products(dnpeff_nmf* h, double* via_rows, double* vi
     DN_TRY(launch_dot((c1 - c0) * h->r, h->S, h->H + c0 * h->r, h->dot_ws, h->dot_ws + DOT_BLOCKS + 1));
     double part = 0.0;
     DN_HIP(hipStreamSynchronize(stream()));
-    DN_HIP(hipMemcpy(&part, h->dot_ws + DOT_BLOCKS + 1, sizeof(double), hipMemcpyDeviceToHost));
+    DN_HIP(copy_down(&part, h->dot_ws + DOT_BLOCKS + 1, sizeof(double)));
     sum += part;
   }
   *via_columns = sum;
@@ -997,7 +997,7 @@ DN_API int dnpeff_fit_loss(dnpeff_fit* f, double* reference_loss, double* true_l
   DN_TRY(launch_xg_mu(f->n, f->r, f->W, f->HH, f->AH, f->eps, f->W2, f->tmp));
   DN_TRY(launch_dot(nr, f->tmp, f->W, f->dot_ws, f->dot_ws + DOT_BLOCKS + 1));
   DN_HIP(hipStreamSynchronize(stream()));
-  DN_HIP(hipMemcpy(res, f->dot_ws + DOT_BLOCKS, sizeof(double) * 2, hipMemcpyDeviceToHost));
+  DN_HIP(copy_down(res, f->dot_ws + DOT_BLOCKS, sizeof(double) * 2));
   const double neg = res[0], pos_true = res[1];
   if (true_loss) *true_loss = std::sqrt(f->sq_norm_A + pos_true - 2.0 * neg);
   if (reference_loss) {
@@ -1005,7 +1005,7 @@ DN_API int dnpeff_fit_loss(dnpeff_fit* f, double* reference_loss, double* true_l
     if (f->whh_valid) {
       DN_TRY(launch_dot(nr, f->WHH, f->W, f->dot_ws, f->dot_ws + DOT_BLOCKS));
       DN_HIP(hipStreamSynchronize(stream()));
-      DN_HIP(hipMemcpy(&pos_ref, f->dot_ws + DOT_BLOCKS, sizeof(double), hipMemcpyDeviceToHost));
+      DN_HIP(copy_down(&pos_ref, f->dot_ws + DOT_BLOCKS, sizeof(double)));
     }
     *reference_loss = std::sqrt(f->sq_norm_A + pos_ref - 2.0 * neg);
   }
@@ -1026,7 +1026,7 @@ DN_API int dnpeff_fit_get_products(dnpeff_fit* f, float* AH_nr, float* HH_rr, do
   DN_HIP(hipStreamSynchronize(stream()));
   if (AH_nr) DN_HIP(copy_down(AH_nr, f->AH, sizeof(float) * f->n * f->r));
   if (HH_rr)
-    DN_HIP(hipMemcpy(HH_rr, f->HH, sizeof(float) * f->r * f->r, hipMemcpyDeviceToHost));
+    DN_HIP(copy_down(HH_rr, f->HH, sizeof(float) * f->r * f->r));
   if (sq_norm_A) *sq_norm_A = f->sq_norm_A;
   return 0;
 }

@@ -625,9 +625,9 @@ static int fused_tiles_make(dnpeff_csr* S, int tc, int64_t most, int64_t alone, 
     f.h_first.clear();
     if (with_first) {
       f.h_first.resize((size_t)groups + 1);
-      DN_HIP(hipMemcpyAsync(f.h_first.data(), first, sizeof(int64_t) * f.h_first.size(), hipMemcpyDeviceToHost, st));
+      DN_HIP(copy_down(f.h_first.data(), first, sizeof(int64_t) * f.h_first.size()));
     }
-    DN_HIP(hipMemcpyAsync(&n_tiles, first + groups, sizeof(int64_t), hipMemcpyDeviceToHost, st));
+    DN_HIP(copy_down(&n_tiles, first + groups, sizeof(int64_t)));
     DN_HIP(hipStreamSynchronize(st));
     dfree(f.tiles);
     f.tiles = nullptr;
@@ -676,7 +676,7 @@ int fused_plan_build(dnpeff_csr* S, int r) {
     dbuf<int64_t> base;
     DN_TRY(base.alloc(S->n_rows + 1));
     DN_TRY(scan_row_chunks(S->rowptr, chunk, S->n_rows, base));
-    DN_HIP(hipMemcpyAsync(&f.n_chunks, base + S->n_rows, sizeof(int64_t), hipMemcpyDeviceToHost, st));
+    DN_HIP(copy_down(&f.n_chunks, base + S->n_rows, sizeof(int64_t)));
     DN_HIP(hipStreamSynchronize(st));
     DN_TRY(dmalloc(&f.chunks, f.n_chunks));
     DN_TRY(dmalloc(&f.n_base, S->n_rows + 1));

@@ -605,10 +605,10 @@ int nlists_build(dnpeff_csr* S, int r, int32_t floor_col, double max_extra_bytes
     DN_TRY(d_below.alloc(n));
     DN_TRY(csr_rows_count_below(S, floor_col, d_below.p));
     DN_HIP(hipStreamSynchronize(st));
-    DN_HIP(hipMemcpy(below.data(), d_below.p, sizeof(int) * n, hipMemcpyDeviceToHost));
+    DN_HIP(copy_down(below.data(), d_below.p, sizeof(int) * n));
   }
   DN_HIP(hipStreamSynchronize(st));
-  DN_HIP(hipMemcpy(rowptr.data(), S->rowptr, sizeof(int64_t) * (n + 1), hipMemcpyDeviceToHost));
+  DN_HIP(copy_down(rowptr.data(), S->rowptr, sizeof(int64_t) * (n + 1)));
   int64_t z = 0;
   for (int64_t i = 0; i < n; i++) {
     mine[(size_t)i] = rowptr[(size_t)i + 1] - rowptr[(size_t)i] - below[(size_t)i];
@@ -636,8 +636,8 @@ int nlists_build(dnpeff_csr* S, int r, int32_t floor_col, double max_extra_bytes
   DN_TRY(dmalloc(&L.progress, SWEEP_XCDS * NL_SYNC_STRIDE));
   DN_TRY(cnt.alloc(n * n_pieces));
   DN_TRY(nbat.alloc((int64_t)n_slots * n_pieces));
-  DN_HIP(hipMemcpy(L.row_slot, row_slot.data(), sizeof(int32_t) * n, hipMemcpyHostToDevice));
-  DN_HIP(hipMemcpy(L.slot_rows, slot_rows.data(), sizeof(int32_t) * slot_rows.size(), hipMemcpyHostToDevice));
+  DN_HIP(copy_up(L.row_slot, row_slot.data(), sizeof(int32_t) * n));
+  DN_HIP(copy_up(L.slot_rows, slot_rows.data(), sizeof(int32_t) * slot_rows.size()));
   const size_t lds = sizeof(int) * (size_t)n_pieces;
   hipLaunchKernelGGL(k_nl_row_count, dim3((unsigned)n), dim3(64), lds, st, S->rowptr, S->colind, floor_col,
                      n_pieces, piece_cols, cnt.p);
@@ -650,7 +650,7 @@ int nlists_build(dnpeff_csr* S, int r, int32_t floor_col, double max_extra_bytes
   DN_HIP(hipStreamSynchronize(st));
   if (tuning().verbose >= 2.0) {  // how far the lock step of an XCD's waves is from the mean work
     std::vector<uint32_t> hb((size_t)n_slots * n_pieces);
-    DN_HIP(hipMemcpy(hb.data(), nbat.p, hb.size() * 4, hipMemcpyDeviceToHost));
+    DN_HIP(copy_down(hb.data(), nbat.p, hb.size() * 4));
     double sum = 0, sum_max = 0, sum_wgmax = 0;
     for (int p = 0; p < n_pieces; p++) {
       uint32_t mx = 0;
@@ -679,8 +679,7 @@ int nlists_build(dnpeff_csr* S, int r, int32_t floor_col, double max_extra_bytes
   L.h_slot_base.assign((size_t)n_slots + 1, 0);
   for (int s = 0; s < n_slots; s++) L.h_slot_base[(size_t)s + 1] = L.h_slot_base[(size_t)s] + tot[(size_t)s];
   const int64_t n_batches = L.h_slot_base[(size_t)n_slots];
-  DN_HIP(hipMemcpy(L.slot_base, L.h_slot_base.data(), sizeof(int64_t) * ((size_t)n_slots + 1),
-                   hipMemcpyHostToDevice));
+  DN_HIP(copy_up(L.slot_base, L.h_slot_base.data(), sizeof(int64_t) * ((size_t)n_slots + 1)));
   if (max_extra_bytes >= 0.0 && (double)(n_batches + 8) * 512.0 - 8.0 * (double)z > max_extra_bytes) {
     if (tn.verbose != 0.0)
       fprintf(stderr, "dnpeff: slot lists of %lld entries would take %.2f GB: not built\n", (long long)z,
@@ -749,7 +748,7 @@ int launch_spmm_n_lists(const dnpeff_csr* S, int r, const float* H_mr, float* pa
     if (tn.verbose >= 2.0) {  // how the lock step went: counts past NL_GIVE_UP mean a wait ran out
       int h[SWEEP_XCDS * NL_SYNC_STRIDE];
       DN_HIP(hipStreamSynchronize(stream()));
-      DN_HIP(hipMemcpy(h, L.progress, sizeof(h), hipMemcpyDeviceToHost));
+      DN_HIP(copy_down(h, L.progress, sizeof(h)));
       fprintf(stderr, "dnpeff: slot-list launch at unit %d: progress counters", unit0);
       for (int x = 0; x < SWEEP_XCDS; x++) fprintf(stderr, " %d", h[x * NL_SYNC_STRIDE]);
       fprintf(stderr, " (%d pieces x %d workgroups)\n", L.n_pieces, L.wgs);
@@ -769,10 +768,9 @@ int nlists_get_row(const dnpeff_csr* S, int64_t row, std::vector<int32_t>& cols,
   std::vector<uint32_t> off((size_t)L.n_pieces + 1);
   std::vector<uint2> pairs((size_t)(b1 - b0) * 64);
   DN_HIP(hipStreamSynchronize(stream()));
-  DN_HIP(hipMemcpy(off.data(), L.off + (size_t)slot * (L.n_pieces + 1), sizeof(uint32_t) * off.size(),
-                   hipMemcpyDeviceToHost));
+  DN_HIP(copy_down(off.data(), L.off + (size_t)slot * (L.n_pieces + 1), sizeof(uint32_t) * off.size()));
   if (b1 > b0)
-    DN_HIP(hipMemcpy(pairs.data(), L.pairs + b0 * 64, sizeof(uint2) * pairs.size(), hipMemcpyDeviceToHost));
+    DN_HIP(copy_down(pairs.data(), L.pairs + b0 * 64, sizeof(uint2) * pairs.size()));
   cols.clear();
   vals.clear();
   const int g = lrow & 7;
@@ -856,7 +854,7 @@ int tblocks_build(dnpeff_csr* S) {
   DN_TRY(scan_counts_i64(count.p, n_groups, first.p));
   B.h_first.assign((size_t)n_groups + 1, 0);
   DN_HIP(hipStreamSynchronize(stream()));
-  DN_HIP(hipMemcpy(B.h_first.data(), first.p, sizeof(int64_t) * (n_groups + 1), hipMemcpyDeviceToHost));
+  DN_HIP(copy_down(B.h_first.data(), first.p, sizeof(int64_t) * (n_groups + 1)));
   B.n_blocks = B.h_first[(size_t)n_groups];
   DN_TRY(dmalloc(&B.cols, B.n_blocks + 1));
   hipLaunchKernelGGL(k_tb_fill, dim3((unsigned)ceil_div(n_groups + 1, 256)), dim3(256), 0, stream(), S->colptr,

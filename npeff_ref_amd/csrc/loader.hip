@@ -152,7 +152,7 @@ bool xcd_round_robin() {
   int h[N];
   hipLaunchKernelGGL(k_xcd_probe, dim3(N), dim3(64), 0, stream(), ids);
   if (hipGetLastError() == hipSuccess &&
-      hipMemcpy(h, ids, sizeof(int) * N, hipMemcpyDeviceToHost) == hipSuccess) {
+      copy_down(h, ids, sizeof(int) * N) == hipSuccess) {
     bool ok = true;
     unsigned seen = 0;
     for (int x = 0; x < SWEEP_XCDS; x++) {
@@ -676,7 +676,7 @@ static int apply_column_table(dnpeff_csr* A, const int32_t* table, int64_t new_n
   DN_TRY(newpos.alloc(A->nnz + 1));
   DN_TRY(scan_kept_entries(A->colind, table, A->nnz, newpos));
   int64_t new_nnz = 0;
-  DN_HIP(hipMemcpy(&new_nnz, newpos + A->nnz, sizeof(int64_t), hipMemcpyDeviceToHost));
+  DN_HIP(copy_down(&new_nnz, newpos + A->nnz, sizeof(int64_t)));
   if (new_nnz == A->nnz) {
     hipLaunchKernelGGL(k_remap_cols, dim3(grid_for(A->nnz)), dim3(256), 0, st, A->colind, A->nnz,
                        table);
@@ -754,11 +754,11 @@ int csr_ensure_chunks(dnpeff_csr* A) {
   A->max_row_chunks = 0;
   if (A->n_rows > 0 && A->n_rows <= 4096) {
     std::vector<int64_t> base((size_t)A->n_rows + 1);
-    DN_HIP(hipMemcpy(base.data(), A->chunk_base, sizeof(int64_t) * base.size(), hipMemcpyDeviceToHost));
+    DN_HIP(copy_down(base.data(), A->chunk_base, sizeof(int64_t) * base.size()));
     for (int64_t i = 0; i < A->n_rows; i++) A->max_row_chunks = std::max(A->max_row_chunks, base[i + 1] - base[i]);
     A->n_chunks = base[A->n_rows];
   } else {
-    DN_HIP(hipMemcpy(&A->n_chunks, A->chunk_base + A->n_rows, sizeof(int64_t), hipMemcpyDeviceToHost));
+    DN_HIP(copy_down(&A->n_chunks, A->chunk_base + A->n_rows, sizeof(int64_t)));
   }
   return 0;
 }
@@ -781,7 +781,7 @@ int csr_set_panels(dnpeff_csr* S, const panel_plan& plan) {
     hipError_t e = hipGetLastError();
     if (e == hipSuccess) e = hipStreamSynchronize(st);
     if (e == hipSuccess)
-      e = hipMemcpy(coarse.data(), d_coarse, sizeof(int32_t) * coarse.size(), hipMemcpyDeviceToHost);
+      e = copy_down(coarse.data(), d_coarse, sizeof(int32_t) * coarse.size());
     dfree(d_coarse);
     DN_CHECK(e == hipSuccess, "building the column panels failed: %s", hipGetErrorString(e));
   }
@@ -830,7 +830,7 @@ int csr_set_panels(dnpeff_csr* S, const panel_plan& plan) {
     int s0 = below.alloc(S->n_rows) || dmalloc(&S->prow, S->n_rows + 1) ||
              csr_rows_count_below(S, tail_floor, below.p) ||
              scan_counts_i64(below.p, S->n_rows, S->prow);
-    if (!s0 && hipMemcpy(&nnz_panels, S->prow + S->n_rows, sizeof(int64_t), hipMemcpyDeviceToHost) != hipSuccess) {
+    if (!s0 && copy_down(&nnz_panels, S->prow + S->n_rows, sizeof(int64_t)) != hipSuccess) {
       set_error("building the column panels failed (row prefixes)");
       s0 = 1;
     }
@@ -846,10 +846,9 @@ int csr_set_panels(dnpeff_csr* S, const panel_plan& plan) {
           dmalloc(&S->seg, S->n_rows * (P + 1)) || dmalloc(&S->pcol, nnz_panels + 64) ||
           dmalloc(&S->pval, nnz_panels + 64);  // (the sweep kernel reads 64 pairs at a time)
   if (!s) {
-    hipError_t e = hipMemcpy(S->panel_bounds, bounds.data(), sizeof(int32_t) * bounds.size(),
-                             hipMemcpyHostToDevice);
+    hipError_t e = copy_up(S->panel_bounds, bounds.data(), sizeof(int32_t) * bounds.size());
     if (e == hipSuccess)
-      e = hipMemcpy(S->panel_ids, ids.data(), sizeof(int32_t) * ids.size(), hipMemcpyHostToDevice);
+      e = copy_up(S->panel_ids, ids.data(), sizeof(int32_t) * ids.size());
     if (e == hipSuccess) {
       int64_t wgs = S->n_rows < 8192 ? S->n_rows : 8192;
       hipLaunchKernelGGL(k_panel_split, dim3((unsigned)(wgs < 1 ? 1 : wgs)), dim3(256), 0, st,
@@ -1023,11 +1022,9 @@ int csr_tile_lists(dnpeff_csr* A) {
   A->h_long_cols.assign((size_t)S->n_long, 0);
   DN_HIP(hipStreamSynchronize(stream()));
   if (A->head.n_d)
-    DN_HIP(hipMemcpy(A->h_head_cols.data(), A->head.cols, sizeof(int32_t) * A->head.n_d,
-                     hipMemcpyDeviceToHost));
+    DN_HIP(copy_down(A->h_head_cols.data(), A->head.cols, sizeof(int32_t) * A->head.n_d));
   if (S->n_long)
-    DN_HIP(hipMemcpy(A->h_long_cols.data(), S->long_cols, sizeof(int32_t) * S->n_long,
-                     hipMemcpyDeviceToHost));
+    DN_HIP(copy_down(A->h_long_cols.data(), S->long_cols, sizeof(int32_t) * S->n_long));
   A->h_lists_valid = true;
   return 0;
 }
@@ -1195,7 +1192,7 @@ static int check_cols_in_range(const dnpeff_csr* A) {
                      A->nnz, A->n_cols, bad);
   DN_LAUNCH_CHECK();
   int h = 0;
-  DN_HIP(hipMemcpy(&h, bad, sizeof(int), hipMemcpyDeviceToHost));
+  DN_HIP(copy_down(&h, bad, sizeof(int)));
   dfree(bad);
   DN_CHECK(h == 0, "%d column ids outside [0, n_cols)", h);
   return 0;
@@ -1212,7 +1209,7 @@ DN_API int dnpeff_csr_from_host(int64_t n_rows, int64_t n_cols, int64_t nnz, con
   A->n_rows = n_rows; A->n_cols = n_cols; A->nnz = nnz; A->full_dense_size = n_cols;
   int s = dmalloc(&A->rowptr, n_rows + 1) || dmalloc(&A->colind, nnz) || dmalloc(&A->vals, nnz);
   if (s) { dnpeff_csr_destroy(A); return 1; }
-  hipError_t e = hipMemcpy(A->rowptr, rowptr, sizeof(int64_t) * (n_rows + 1), hipMemcpyHostToDevice);
+  hipError_t e = copy_up(A->rowptr, rowptr, sizeof(int64_t) * (n_rows + 1));
   if (e == hipSuccess && nnz)
     e = copy_up(A->colind, colind, sizeof(int32_t) * nnz);
   if (e == hipSuccess && nnz)
@@ -1267,7 +1264,7 @@ DN_API int dnpeff_csr_normalize_rows(dnpeff_csr* A, const float* norms_host, flo
   if (A->n_rows == 0) return 0;
   float* norms = nullptr;
   DN_TRY(dmalloc(&norms, A->n_rows));
-  DN_HIP(hipMemcpy(norms, norms_host, sizeof(float) * A->n_rows, hipMemcpyHostToDevice));
+  DN_HIP(copy_up(norms, norms_host, sizeof(float) * A->n_rows));
   unsigned grid = (unsigned)(A->n_rows < 65536 ? A->n_rows : 65536);
   hipLaunchKernelGGL(k_normalize_rows, dim3(grid), dim3(256), 0, stream(), A->rowptr, A->vals,
                      norms, eps, A->n_rows);
@@ -1296,7 +1293,7 @@ DN_API int dnpeff_csr_compact_columns(dnpeff_csr* A, int min_count) {
   DN_TRY(pos.alloc(m_full + 1));
   DN_TRY(scan_keep_mask(count, min_count, m_full, pos));
   int32_t m_new = 0;
-  DN_HIP(hipMemcpy(&m_new, pos + m_full, sizeof(int32_t), hipMemcpyDeviceToHost));
+  DN_HIP(copy_down(&m_new, pos + m_full, sizeof(int32_t)));
   DN_TRY(og_to_new.alloc(m_full));
   DN_TRY(new_to_og.alloc((int64_t)m_new));
   hipLaunchKernelGGL(k_build_maps, dim3(grid_for(m_full)), dim3(256), 0, st, count.p, min_count,
@@ -1394,7 +1391,7 @@ DN_API int dnpeff_csr_sq_norm(const dnpeff_csr* A, double* out) {
   hipLaunchKernelGGL(k_sq_norm_partial, dim3(blocks), dim3(256), 0, stream(), v, A->nnz, partials);
   DN_LAUNCH_CHECK();
   std::vector<double> h(blocks);
-  DN_HIP(hipMemcpy(h.data(), partials, sizeof(double) * blocks, hipMemcpyDeviceToHost));
+  DN_HIP(copy_down(h.data(), partials, sizeof(double) * blocks));
   dfree(partials);
   double s = 0.0;
   for (int i = 0; i < blocks; i++) s += h[i];
@@ -1453,13 +1450,13 @@ int choose_dense_head(dnpeff_csr* A, double min_fill, double budget, int n_block
     int32_t n_d = 0;
     unsigned long long z_head = 0;
     DN_TRY(scan_keep_mask(count, (int)thr, m, pos));
-    DN_HIP(hipMemcpy(&n_d, pos + m, sizeof(int32_t), hipMemcpyDeviceToHost));
+    DN_HIP(copy_down(&n_d, pos + m, sizeof(int32_t)));
     if (n_d == 0) break;
     DN_HIP(hipMemsetAsync(zsum, 0, sizeof(unsigned long long), st));
     hipLaunchKernelGGL(k_sum_selected, dim3(grid_for(m, 4096)), dim3(256), 0, st, count.p, m, (int)thr,
                        zsum.p);
     DN_LAUNCH_CHECK();
-    DN_HIP(hipMemcpy(&z_head, zsum, sizeof(unsigned long long), hipMemcpyDeviceToHost));
+    DN_HIP(copy_down(&z_head, zsum, sizeof(unsigned long long)));
     const double blocks = n_blocks * 4.0 * (double)n_pad * (double)(ceil_div(n_d, 128) * 128);
     if (blocks > (double)total_b / 6.0) continue;
     head_choice c;
@@ -1498,7 +1495,7 @@ int split_dense_head_at(dnpeff_csr* A, int64_t thr, int64_t* n_dense) {
   DN_TRY(pos.alloc(m + 1));
   DN_TRY(scan_keep_mask(count, (int)thr, m, pos));
   int32_t n_d = 0;
-  DN_HIP(hipMemcpy(&n_d, pos + m, sizeof(int32_t), hipMemcpyDeviceToHost));
+  DN_HIP(copy_down(&n_d, pos + m, sizeof(int32_t)));
   if (n_d == 0) return 0;
   const int64_t n_pad = ceil_div(n, 128) * 128, n_d_pad = ceil_div(n_d, 128) * 128;
   DN_TRY(slot_of.alloc(m));
@@ -1522,7 +1519,7 @@ int split_dense_head_at(dnpeff_csr* A, int64_t thr, int64_t* n_dense) {
                        A->vals, n, slot_of.p, cm.p, n_pad, repeats.p);
     DN_LAUNCH_CHECK();
     int n_rep = 0;
-    DN_HIP(hipMemcpy(&n_rep, repeats.p, sizeof(int), hipMemcpyDeviceToHost));
+    DN_HIP(copy_down(&n_rep, repeats.p, sizeof(int)));
     DN_CHECK(n_rep == 0,
              "%d entries of the dense head's columns repeat a (row, column) pair: duplicate entries are "
              "not supported by the products",
@@ -1536,7 +1533,7 @@ int split_dense_head_at(dnpeff_csr* A, int64_t thr, int64_t* n_dense) {
   {
     dbuf<int64_t> newpos;
     status = newpos.alloc(A->nnz + 1) || scan_kept_entries(A->colind, table, A->nnz, newpos);
-    if (!status && hipMemcpy(&T->nnz, newpos + A->nnz, sizeof(int64_t), hipMemcpyDeviceToHost) != hipSuccess) {
+    if (!status && copy_down(&T->nnz, newpos + A->nnz, sizeof(int64_t)) != hipSuccess) {
       set_error("dense head: reading the size of the sparse part failed");
       status = 1;
     }
@@ -1657,8 +1654,7 @@ DN_API int dnpeff_csr_build_transpose(dnpeff_csr* A) {
   DN_TRY(tvals.alloc(A->nnz));
   DN_HIP(hipMemsetAsync(count, 0, sizeof(int) * (size_t)(m + 1), st));
   std::vector<int64_t> rowptr((size_t)A->n_rows + 1);
-  DN_HIP(hipMemcpy(rowptr.data(), A->rowptr, sizeof(int64_t) * (A->n_rows + 1),
-                   hipMemcpyDeviceToHost));
+  DN_HIP(copy_down(rowptr.data(), A->rowptr, sizeof(int64_t) * (A->n_rows + 1)));
   for (int64_t i = 0; i < A->n_rows; i++) {
     int64_t len = rowptr[i + 1] - rowptr[i];
     if (len <= 0) continue;
@@ -1674,7 +1670,7 @@ DN_API int dnpeff_csr_build_transpose(dnpeff_csr* A) {
                      count.p + m);
   DN_LAUNCH_CHECK();
   int repeats = 0;
-  DN_HIP(hipMemcpy(&repeats, count.p + m, sizeof(int), hipMemcpyDeviceToHost));
+  DN_HIP(copy_down(&repeats, count.p + m, sizeof(int)));
   DN_CHECK(repeats == 0,
            "%d column(s) hold the same row more than once: duplicate (row, column) entries are not "
            "supported by the products",
@@ -1684,7 +1680,7 @@ DN_API int dnpeff_csr_build_transpose(dnpeff_csr* A) {
   DN_TRY(pos.alloc(m + 1));
   DN_TRY(scan_long_cols(colptr, SPMM_T_LONG, m, pos));
   int32_t n_long = 0;
-  DN_HIP(hipMemcpy(&n_long, pos + m, sizeof(int32_t), hipMemcpyDeviceToHost));
+  DN_HIP(copy_down(&n_long, pos + m, sizeof(int32_t)));
   DN_TRY(long_cols.alloc((int64_t)n_long));
   if (n_long) {
     hipLaunchKernelGGL(k_collect_long, dim3(grid_for(m)), dim3(256), 0, st, colptr.p, SPMM_T_LONG, m,
@@ -1756,7 +1752,7 @@ DN_API int dnpeff_csr_get_row(dnpeff_csr* A, int64_t row, int64_t cap, int64_t* 
   const dnpeff_csr* S = sparse_part(A);
   DN_CHECK(S->rowptr != nullptr, "matrix has no row offsets");
   int64_t e[2];
-  DN_HIP(hipMemcpy(e, S->rowptr + row, sizeof(e), hipMemcpyDeviceToHost));
+  DN_HIP(copy_down(e, S->rowptr + row, sizeof(e)));
   const int32_t* src_c = S->colind ? S->colind : S->pcol;
   const float* src_v = S->vals ? S->vals : S->pval;
   std::vector<int32_t> list_cols;
@@ -1765,15 +1761,15 @@ DN_API int dnpeff_csr_get_row(dnpeff_csr* A, int64_t row, int64_t cap, int64_t* 
   if (!S->colind && S->pcol && S->tail_floor > 0 && S->nl.pairs) {
     // the panels hold the row's entries below tail_floor, the slot lists the others
     DN_TRY(nlists_get_row(S, row, list_cols, list_vals));
-    DN_HIP(hipMemcpy(e, S->prow + row, sizeof(e), hipMemcpyDeviceToHost));
+    DN_HIP(copy_down(e, S->prow + row, sizeof(e)));
     DN_CHECK((int64_t)list_cols.size() + (e[1] - e[0]) == row_entries,
              "panels and slot lists hold %lld entries of row %lld, not %lld",
              (long long)((int64_t)list_cols.size() + (e[1] - e[0])), (long long)row, (long long)row_entries);
     std::vector<int32_t> pc((size_t)(e[1] - e[0]));
     std::vector<float> pv((size_t)(e[1] - e[0]));
     if (e[1] > e[0]) {
-      DN_HIP(hipMemcpy(pc.data(), S->pcol + e[0], sizeof(int32_t) * pc.size(), hipMemcpyDeviceToHost));
-      DN_HIP(hipMemcpy(pv.data(), S->pval + e[0], sizeof(float) * pv.size(), hipMemcpyDeviceToHost));
+      DN_HIP(copy_down(pc.data(), S->pcol + e[0], sizeof(int32_t) * pc.size()));
+      DN_HIP(copy_down(pv.data(), S->pval + e[0], sizeof(float) * pv.size()));
     }
     list_cols.insert(list_cols.begin(), pc.begin(), pc.end());
     list_vals.insert(list_vals.begin(), pv.begin(), pv.end());
@@ -1796,9 +1792,8 @@ DN_API int dnpeff_csr_get_row(dnpeff_csr* A, int64_t row, int64_t cap, int64_t* 
                        A->head.n_pad, row, A->head.n_d, tmp.p);
     DN_LAUNCH_CHECK();
     DN_HIP(hipStreamSynchronize(stream()));
-    DN_HIP(hipMemcpy(head_row.data(), tmp.p, sizeof(float) * A->head.n_d, hipMemcpyDeviceToHost));
-    DN_HIP(hipMemcpy(head_cols.data(), A->head.cols, sizeof(int32_t) * A->head.n_d,
-                     hipMemcpyDeviceToHost));
+    DN_HIP(copy_down(head_row.data(), tmp.p, sizeof(float) * A->head.n_d));
+    DN_HIP(copy_down(head_cols.data(), A->head.cols, sizeof(int32_t) * A->head.n_d));
     for (float v : head_row) got += v != 0.0f;
   }
   *count = got;
@@ -1815,8 +1810,8 @@ DN_API int dnpeff_csr_get_row(dnpeff_csr* A, int64_t row, int64_t cap, int64_t* 
     memcpy(cols + w, list_cols.data(), sizeof(int32_t) * list_cols.size());
     memcpy(vals + w, list_vals.data(), sizeof(float) * list_vals.size());
   } else if (e[1] > e[0]) {
-    DN_HIP(hipMemcpy(cols + w, src_c + e[0], sizeof(int32_t) * (e[1] - e[0]), hipMemcpyDeviceToHost));
-    DN_HIP(hipMemcpy(vals + w, src_v + e[0], sizeof(float) * (e[1] - e[0]), hipMemcpyDeviceToHost));
+    DN_HIP(copy_down(cols + w, src_c + e[0], sizeof(int32_t) * (e[1] - e[0])));
+    DN_HIP(copy_down(vals + w, src_v + e[0], sizeof(float) * (e[1] - e[0])));
   }
   return 0;
 }
@@ -1836,8 +1831,7 @@ DN_API int dnpeff_csr_get_column(dnpeff_csr* A, int64_t col, int64_t cap, int64_
   if (it != hc.end() && *it == (int32_t)col) {  // a column of the dense head
     const int64_t k = it - hc.begin();
     std::vector<float> c((size_t)A->n_rows);
-    DN_HIP(hipMemcpy(c.data(), A->head.cm + k * A->head.n_pad, sizeof(float) * A->n_rows,
-                     hipMemcpyDeviceToHost));
+    DN_HIP(copy_down(c.data(), A->head.cm + k * A->head.n_pad, sizeof(float) * A->n_rows));
     int64_t got = 0;
     for (float v : c) got += v != 0.0f;
     *count = got;
@@ -1853,14 +1847,14 @@ DN_API int dnpeff_csr_get_column(dnpeff_csr* A, int64_t col, int64_t cap, int64_
     return 0;
   }
   int64_t p[2];
-  DN_HIP(hipMemcpy(p, S->colptr + col, sizeof(p), hipMemcpyDeviceToHost));
+  DN_HIP(copy_down(p, S->colptr + col, sizeof(p)));
   *count = p[1] - p[0];
   if (!rows || !vals) return 0;
   DN_CHECK(cap >= p[1] - p[0], "column %lld holds %lld entries, the buffers %lld", (long long)col,
            (long long)(p[1] - p[0]), (long long)cap);
   if (p[1] > p[0]) {
-    DN_HIP(hipMemcpy(rows, S->rowind + p[0], sizeof(int32_t) * (p[1] - p[0]), hipMemcpyDeviceToHost));
-    DN_HIP(hipMemcpy(vals, S->tvals + p[0], sizeof(float) * (p[1] - p[0]), hipMemcpyDeviceToHost));
+    DN_HIP(copy_down(rows, S->rowind + p[0], sizeof(int32_t) * (p[1] - p[0])));
+    DN_HIP(copy_down(vals, S->tvals + p[0], sizeof(float) * (p[1] - p[0])));
   }
   return 0;
 }

@@ -220,15 +220,135 @@ static hipError_t staged_copy(char* dst, const char* src, size_t bytes) {
   return (hipError_t)failed.load();
 }
 
+// Smaller copies go through one of a few pinned buffers, in two halves where they are longer than one.
+// (hipMemcpy of a few bytes from or to pageable memory takes 30 to 70 us here, and now and then
+// milliseconds for some MB; 15 us this way.)  Up to a page comes down through a kernel that writes to
+// the buffer: shorter still than a copy on the engines.
+constexpr size_t BOUNCE_HALF = (size_t)1 << 20;
+constexpr size_t BOUNCE_KERNEL = 16384;
+constexpr size_t BOUNCE_KEPT = 4;  // buffers that wait for the next call
+
+struct bounce_buf {
+  char* p = nullptr;
+  hipEvent_t done[2] = {};
+};
+struct bounce_state {
+  std::mutex lock;
+  std::vector<bounce_buf> idle;
+};
+static bounce_state& bounces() {
+  static bounce_state* b = new bounce_state();
+  return *b;
+}
+static void bounce_free(bounce_buf& b) {
+  if (b.p) (void)hipHostFree(b.p);
+  for (hipEvent_t e : b.done)
+    if (e) (void)hipEventDestroy(e);
+  b = bounce_buf();
+}
+static bool bounce_take(bounce_buf* b) {
+  {
+    bounce_state& B = bounces();
+    std::lock_guard<std::mutex> g(B.lock);
+    if (!B.idle.empty()) {
+      *b = B.idle.back();
+      B.idle.pop_back();
+      return true;
+    }
+  }
+  if (hipHostMalloc((void**)&b->p, 2 * BOUNCE_HALF, hipHostMallocDefault) == hipSuccess &&
+      hipEventCreateWithFlags(&b->done[0], hipEventDisableTiming) == hipSuccess &&
+      hipEventCreateWithFlags(&b->done[1], hipEventDisableTiming) == hipSuccess)
+    return true;
+  (void)hipGetLastError();
+  bounce_free(*b);
+  return false;
+}
+static void bounce_give(bounce_buf& b) {
+  bounce_state& B = bounces();
+  {
+    std::lock_guard<std::mutex> g(B.lock);
+    if (B.idle.size() < BOUNCE_KEPT) {
+      B.idle.push_back(b);
+      return;
+    }
+  }
+  bounce_free(b);
+}
+static void bounce_trim() {
+  bounce_state& B = bounces();
+  std::lock_guard<std::mutex> g(B.lock);
+  for (bounce_buf& b : B.idle) bounce_free(b);
+  B.idle.clear();
+}
+
+__global__ void __launch_bounds__(256) k_copy_words(const uint32_t* __restrict__ src, uint32_t* __restrict__ dst, int n) {
+  for (int i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) dst[i] = src[i];
+}
+
+template <bool UP>
+static hipError_t bounce_copy(char* dst, const char* src, size_t bytes) {
+  bounce_buf B;
+  if (!bounce_take(&B)) return hipMemcpy(dst, src, bytes, UP ? hipMemcpyHostToDevice : hipMemcpyDeviceToHost);
+  hipStream_t st = stream();
+  hipError_t e = hipSuccess;
+  if (!UP && bytes <= BOUNCE_KERNEL && bytes % 4 == 0 && (uintptr_t)src % 4 == 0) {
+    const int n = (int)(bytes / 4);
+    hipLaunchKernelGGL(k_copy_words, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, (const uint32_t*)src,
+                       (uint32_t*)B.p, n);
+    e = hipGetLastError();
+    if (e == hipSuccess) e = hipStreamSynchronize(st);
+    if (e == hipSuccess) memcpy(dst, B.p, bytes);
+  } else if (bytes <= 2 * BOUNCE_HALF && !UP) {
+    // down: both halves under way at once
+    const size_t n0 = bytes < BOUNCE_HALF ? bytes : bytes / 2;
+    e = hipMemcpyAsync(B.p, src, n0, hipMemcpyDeviceToHost, st);
+    if (e == hipSuccess) e = hipEventRecord(B.done[0], st);
+    if (e == hipSuccess && n0 < bytes) e = hipMemcpyAsync(B.p + n0, src + n0, bytes - n0, hipMemcpyDeviceToHost, st);
+    if (e == hipSuccess) e = hipEventSynchronize(B.done[0]);
+    if (e == hipSuccess) memcpy(dst, B.p, n0);
+    const hipError_t es = hipStreamSynchronize(st);
+    if (e == hipSuccess) e = es;
+    if (e == hipSuccess && n0 < bytes) memcpy(dst + n0, B.p + n0, bytes - n0);
+  } else {
+    size_t at[2] = {0, 0}, len[2] = {0, 0};
+    int k = 0;
+    for (size_t off = 0; off < bytes && e == hipSuccess; off += BOUNCE_HALF, k++) {
+      const int b = k & 1;
+      char* buf = B.p + b * BOUNCE_HALF;
+      const size_t n = bytes - off < BOUNCE_HALF ? bytes - off : BOUNCE_HALF;
+      if (k >= 2) e = hipEventSynchronize(B.done[b]);
+      if (e != hipSuccess) break;
+      if (UP) {
+        memcpy(buf, src + off, n);
+        e = hipMemcpyAsync(dst + off, buf, n, hipMemcpyHostToDevice, st);
+      } else {
+        if (len[b]) memcpy(dst + at[b], buf, len[b]);
+        e = hipMemcpyAsync(buf, src + off, n, hipMemcpyDeviceToHost, st);
+        at[b] = off;
+        len[b] = n;
+      }
+      if (e == hipSuccess) e = hipEventRecord(B.done[b], st);
+    }
+    const hipError_t es = hipStreamSynchronize(st);
+    if (e == hipSuccess) e = es;
+    if (!UP && e == hipSuccess)
+      for (int i = k >= 2 ? k - 2 : 0; i < k; i++) memcpy(dst + at[i & 1], B.p + (i & 1) * BOUNCE_HALF, len[i & 1]);
+  }
+  if (e != hipSuccess) (void)hipStreamSynchronize(st);  // (nothing may still be on its way to the buffer)
+  bounce_give(B);
+  return e;
+}
+
 hipError_t copy_up(void* dst_dev, const void* src_host, size_t bytes) {
   if (bytes == 0) return hipSuccess;
-  if (bytes < STAGED_MIN) return hipMemcpy(dst_dev, src_host, bytes, hipMemcpyHostToDevice);
+  if (bytes < STAGED_MIN) return bounce_copy<true>((char*)dst_dev, (const char*)src_host, bytes);
   return staged_copy<true>((char*)dst_dev, (const char*)src_host, bytes);
 }
 
 hipError_t copy_down(void* dst_host, const void* src_dev, size_t bytes) {
   if (bytes == 0) return hipSuccess;
-  if (bytes < STAGED_MIN) return hipMemcpy(dst_host, src_dev, bytes, hipMemcpyDeviceToHost);
+  if (bytes < STAGED_MIN) return bounce_copy<false>((char*)dst_host, (const char*)src_dev, bytes);
   return staged_copy<false>((char*)dst_host, (const char*)src_dev, bytes);
 }
 
@@ -252,5 +372,6 @@ DN_API int dnpeff_release_cached(void) {
   DN_HIP(hipStreamSynchronize(stream()));
   pool_trim();
   stage_trim();
+  bounce_trim();
   return 0;
 }

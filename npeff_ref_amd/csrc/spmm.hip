@@ -1232,7 +1232,7 @@ static int sweep_row_order(const dnpeff_csr* A, const sweep_shape& sh, std::vect
                      A->n_panels, counts.p);
   DN_LAUNCH_CHECK();
   std::vector<int64_t> h(n);
-  DN_HIP(hipMemcpy(h.data(), counts.p, sizeof(int64_t) * n, hipMemcpyDeviceToHost));
+  DN_HIP(copy_down(h.data(), counts.p, sizeof(int64_t) * n));
   std::vector<int32_t> order(n), perm(n);
   for (int64_t i = 0; i < n; i++) order[i] = (int32_t)i;
   std::stable_sort(order.begin(), order.end(), [&](int32_t a, int32_t b) { return h[a] > h[b]; });
@@ -1247,7 +1247,7 @@ static int sweep_row_order(const dnpeff_csr* A, const sweep_shape& sh, std::vect
     }
   }
   DN_TRY(dmalloc(&M->sweep_perm, n));
-  DN_HIP(hipMemcpy(M->sweep_perm, perm.data(), sizeof(int32_t) * n, hipMemcpyHostToDevice));
+  DN_HIP(copy_up(M->sweep_perm, perm.data(), sizeof(int32_t) * n));
   M->sweep_perm_key = key;
   return 0;
 }

@@ -194,7 +194,7 @@ DN_API int dnpeff_synth_pef(int64_t n_rows, int64_t n_cols, int64_t k_fixed, int
                        n_rows, k_fixed, k_min, k_max, seed, len);
   }
   if ((status = scan_counts_i64(len, n_rows, A->rowptr))) return fail(status);
-  if (hipMemcpy(&A->nnz, A->rowptr + n_rows, sizeof(int64_t), hipMemcpyDeviceToHost) != hipSuccess)
+  if (copy_down(&A->nnz, A->rowptr + n_rows, sizeof(int64_t)) != hipSuccess)
     return fail(1);
   if (dmalloc(&A->colind, A->nnz) || dmalloc(&A->vals, A->nnz)) return fail(1);
 
@@ -220,7 +220,7 @@ DN_API int dnpeff_synth_pef(int64_t n_rows, int64_t n_cols, int64_t k_fixed, int
   }
   if (hipGetLastError() != hipSuccess) { set_error("generator launch failed"); return fail(1); }
   int h_failed = 0;
-  if (hipMemcpy(&h_failed, failed, sizeof(int), hipMemcpyDeviceToHost) != hipSuccess) {
+  if (copy_down(&h_failed, failed, sizeof(int)) != hipSuccess) {
     set_error("generator kernel failed");
     return fail(1);
   }
@@ -232,7 +232,7 @@ DN_API int dnpeff_synth_pef(int64_t n_rows, int64_t n_cols, int64_t k_fixed, int
     if (dmalloc(&norms, n_rows)) return fail(1);
     hipLaunchKernelGGL(k_row_norms, dim3((unsigned)ceil_div(n_rows, 64)), dim3(64), 0, st, n_rows,
                        A->rowptr, A->vals, norms);
-    if (hipMemcpy(norms_out_host, norms, sizeof(float) * n_rows, hipMemcpyDeviceToHost) !=
+    if (copy_down(norms_out_host, norms, sizeof(float) * n_rows) !=
         hipSuccess) {
       set_error("norm kernel failed");
       return fail(1);

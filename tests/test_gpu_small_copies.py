@@ -1,0 +1,16 @@
+"""Host copies through the pinned bounce buffers (csrc/pool.hip): around one buffer, around the words
+kernel's limit, odd lengths, and on either side of the size from which copies are split over threads."""
+
+import numpy as np
+import pytest
+
+import npeff_ref_amd as d
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("nbytes", [1, 4, 16384, 16388, 16390, 1 << 20, (1 << 21) + 4, (3 << 20) + 1, (4 << 20) - 1])
+def test_small_copies(nbytes):
+    a = np.random.default_rng(nbytes).integers(0, 255, nbytes, dtype=np.uint8)
+    x = d.DeviceArray.from_numpy(a, dtype=np.uint8)
+    assert np.array_equal(x.numpy(), a)
