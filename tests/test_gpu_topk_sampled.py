@@ -1,0 +1,40 @@
+"""Top-k through the sampled threshold (csrc/topk.hip): rows long enough to be sampled, values that the
+sample misjudges, crowded buckets, and lengths around its chunks, against the full sort."""
+
+import numpy as np
+import pytest
+
+import npeff_ref_amd as d
+from oracle import oracle as orc
+
+pytestmark = pytest.mark.gpu
+
+
+def _values(kind, n, count, rng):
+    if kind == "lognormal":
+        return np.exp(rng.normal(-8, 2, (n, count))).astype(np.float32)
+    if kind == "uniform":
+        return rng.random((n, count), dtype=np.float32)
+    if kind == "normal":  # both signs
+        return rng.standard_normal((n, count), dtype=np.float32)
+    if kind == "equal":
+        return np.full((n, count), 0.25, dtype=np.float32)
+    if kind == "few":  # eight different values
+        return rng.integers(0, 8, (n, count)).astype(np.float32)
+    if kind == "hidden":  # everything large lies where no sample is taken
+        x = rng.random((n, count), dtype=np.float32)
+        x[:, 100:1100] += 100.0
+        return x
+    x = np.sort(rng.random((n, count), dtype=np.float32), axis=1)  # "sorted"
+    x[:, -1] = 1e30
+    return x
+
+
+@pytest.mark.parametrize("kind", ["lognormal", "uniform", "normal", "equal", "few", "hidden", "sorted"])
+@pytest.mark.parametrize("n,count,k", [(1, 600_000, 900), (3, 524_289, 4000), (2, 524_287, 64), (1, 65, 65), (5, 1, 1)])
+def test_topk_matches_the_full_sort(kind, n, count, k):
+    x = _values(kind, n, count, np.random.default_rng(count + k))
+    v, i, nrm = d.topk_rows(d.DeviceArray.from_numpy(x), k)
+    wv, wi, wn = orc.topk_rows(x, k)
+    assert np.array_equal(v, wv) and np.array_equal(i, wi)
+    assert np.allclose(nrm, wn, rtol=2e-7)
