@@ -124,6 +124,7 @@ struct fu_gather {
       *reinterpret_cast<f32x4*>(tile + dst) = a0;
       if (WHOLE || 4 * (sub + LPR) < 16 * NB) *reinterpret_cast<f32x4*>(tile + dst + 4 * LPR) = a1;
     };
+#pragma unroll 1
     for (int b = s0; b < s1; b += U) {
       f32x4 w0[U], w1[U];
 #pragma unroll

@@ -14,6 +14,15 @@
 
 namespace dn {
 
+// The lane, of which the compiler is not told that it stays the same: what is computed from it is computed
+// where it is used.  (Hoisted out of the loop over the tiles the addresses of a lane's LDS and global
+// accesses took 60 registers and, at rank 128, spilled.)
+__device__ inline int fuw_lane() {
+  int lane = threadIdx.x & 63;
+  asm volatile("" : "+v"(lane));
+  return lane;
+}
+
 constexpr int FUW_U = 2;  // rows of W in flight per lane group
 constexpr int fuw_steps(int nb) { return (16 * nb + 31) / 32; }
 
@@ -75,7 +84,7 @@ struct fuw_gram {
   }
   template <int NA>
   __device__ static inline void add(const __bf16* __restrict__ y, f32x4 (&acc)[NA]) {
-    const int lane = threadIdx.x & 63;
+    const int lane = fuw_lane();
     const part a = load(y, W, lane);
     part a2;
     if constexpr (SECOND) a2 = load(y, R2, lane);
@@ -117,7 +126,10 @@ __device__ inline void fuw_for_wave(int wave, F&& f) {
 
 // COLS: the H update (tiles of columns, A^T W gathered); else the W update (32 rows per workgroup, the
 // chunk sums of A H^T).  NB: blocks of 16 components.  Two barriers per tile: the Gram products of a
-// tile run between the second one and the next tile's first, beside the gathers of the next tile.
+// tile run between the second one and the next tile's first, beside the rows and the gathers of the next
+// tile.  1000 x 3.4 M, rank 128: 1.75 ms (matrix cores 24 % of it, other arithmetic 38 %, LDS 30 %, 7.8 TB/s
+// out of L2; 1.94 ms with the addresses kept over the loop, the descriptor asked for where it is needed
+// and the rows after the Gram products).  Eight waves of 128 registers, one block each: 1.84 ms.
 template <int NB, bool COLS>
 __global__ void __launch_bounds__(256, 2) k_fuw(const fuw_args p) {
   constexpr int NS = fuw_steps(NB), PS = 32 * NS + 8, PLANE = FUW_COLS * PS, TS = 16 * NB + 4;
@@ -132,13 +144,12 @@ __global__ void __launch_bounds__(256, 2) k_fuw(const fuw_args p) {
   __bf16* planes = reinterpret_cast<__bf16*>(lds + LDS_TILE);
   __bf16* ypl = planes + 3 * PLANE;
   __shared__ int cps[2][FUW_COLS + 1];
-  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
-  const int l16 = lane & 15, g = lane >> 4;
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int jb0 = SPLIT_J ? wave & 1 : 0, b0 = SPLIT_J ? 3 * (wave >> 1) : 2 * wave;
   const int r = p.r;
   const char* Wb = reinterpret_cast<const char*>(p.W);
   Gather gather;
-  fu_tile_at td;
+  fu_tile_at td, nd;  // this tile and the next (a descriptor is a load that nothing else hides)
   int64_t cpv = 0;
   auto request = [&](const fu_tile_at& d) {
     gather.request(p.pairs, d);
@@ -147,20 +158,22 @@ __global__ void __launch_bounds__(256, 2) k_fuw(const fuw_args p) {
   if constexpr (COLS) {
     gather.init(r);
     td = fu_describe<Gather::NG>(p.tiles, p.n_tiles, blockIdx.x);
+    nd = fu_describe<Gather::NG>(p.tiles, p.n_tiles, blockIdx.x + gridDim.x);
     request(td);
   }
 
-  // the wave's rows of G, split: row 16 (b0 + bi) + l16, components 32 s + 8 g ..
+  const int l16_0 = fuw_lane() & 15, g0 = fuw_lane() >> 4;
+  // the wave's rows of G, split: row 16 (b0 + bi) + l16_0, components 32 s + 8 g ..
   bf16x8 gh[BPW][NS], gm[BPW][NS], gl[BPW][NS];
 #pragma unroll
   for (int bi = 0; bi < BPW; bi++)
 #pragma unroll
     for (int s = 0; s < NS; s++) {
       f32x4 v[2];
-      const int c = 16 * (b0 + bi) + l16;
+      const int c = 16 * (b0 + bi) + l16_0;
 #pragma unroll
       for (int t = 0; t < 8; t++) {
-        const int k = 32 * s + 8 * g + t;
+        const int k = 32 * s + 8 * g0 + t;
         double sum = 0.0;
         if (k < r && c < r) {
           const int bk = k >> 4, bc = c >> 4;
@@ -199,6 +212,7 @@ __global__ void __launch_bounds__(256, 2) k_fuw(const fuw_args p) {
   };
   auto in_tile = [&](const place& q, int jl) { return jl >= q.l0 && jl < q.l0 + q.nc; };
   auto load_x = [&](const place& q) {
+    const int lane = fuw_lane(), l16 = lane & 15, g = lane >> 4;
 #pragma unroll
     for (int jp = 0; jp < JPW; jp++) {
       const int jl = 16 * (jb0 + jp) + l16;
@@ -212,6 +226,7 @@ __global__ void __launch_bounds__(256, 2) k_fuw(const fuw_args p) {
     }
   };
   auto split_x = [&]() {
+    const int lane = fuw_lane(), l16 = lane & 15, g = lane >> 4;
 #pragma unroll
     for (int jp = 0; jp < JPW; jp++)
 #pragma unroll
@@ -233,6 +248,7 @@ __global__ void __launch_bounds__(256, 2) k_fuw(const fuw_args p) {
     if (tid <= at.nc) cps[0][at.l0 + tid] = (int)(cpv - td.e0);
     gather.run(p.pairs, td, Wb, tile);
   } else {
+    const int lane = fuw_lane(), l16 = lane & 15, g = lane >> 4;
 #pragma unroll
     for (int jp = 0; jp < JPW; jp++) {
       const int jl = 16 * (jb0 + jp) + l16;
@@ -250,31 +266,29 @@ __global__ void __launch_bounds__(256, 2) k_fuw(const fuw_args p) {
   split_x();
 
   for (int par = 0;; par ^= 1) {
-    fu_tile_at nd;
     const int next = tl + gridDim.x;
     const bool more = COLS && next < p.n_tiles;
     if constexpr (COLS) {
-      nd = fu_describe<Gather::NG>(p.tiles, p.n_tiles, next);
       request(nd);
     }
     __syncthreads();
 
-    f32x4 d[JPW][BPW];
+    const int lane = fuw_lane(), l16 = lane & 15, g = lane >> 4;
+    const float inv = 1.0f / (float)(COLS && td.share > 0 ? td.share : 1);
 #pragma unroll
-    for (int jp = 0; jp < JPW; jp++)
+    for (int jp = 0; jp < JPW; jp++) {
+      f32x4 d[BPW];
 #pragma unroll
-      for (int bi = 0; bi < BPW; bi++) d[jp][bi] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+      for (int bi = 0; bi < BPW; bi++) d[bi] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-    for (int s = 0; s < NS; s++)
-#pragma unroll
-      for (int jp = 0; jp < JPW; jp++) {
+      for (int s = 0; s < NS; s++) {
         const __bf16* pl = planes + (16 * (jb0 + jp) + l16) * PS + 32 * s + 8 * g;
         const bf16x8 bh = *reinterpret_cast<const bf16x8*>(pl);
         const bf16x8 bm = *reinterpret_cast<const bf16x8*>(pl + PLANE);
         const bf16x8 bl = *reinterpret_cast<const bf16x8*>(pl + 2 * PLANE);
 #define DN_FUW(A, B)                            \
-  _Pragma("unroll") for (int bi = 0; bi < BPW; bi++) d[jp][bi] = \
-      __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[bi][s], B, d[jp][bi], 0, 0, 0)
+  _Pragma("unroll") for (int bi = 0; bi < BPW; bi++) d[bi] = \
+      __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[bi][s], B, d[bi], 0, 0, 0)
         DN_FUW(gl, bh);
         DN_FUW(gh, bl);
         DN_FUW(gm, bm);
@@ -283,9 +297,6 @@ __global__ void __launch_bounds__(256, 2) k_fuw(const fuw_args p) {
         DN_FUW(gh, bh);
 #undef DN_FUW
       }
-    const float inv = 1.0f / (float)(COLS && td.share > 0 ? td.share : 1);
-#pragma unroll
-    for (int jp = 0; jp < JPW; jp++) {
       const int jl = 16 * (jb0 + jp) + l16;
       const bool mine = in_tile(at, jl);
       bool some = mine;
@@ -314,7 +325,7 @@ __global__ void __launch_bounds__(256, 2) k_fuw(const fuw_args p) {
         f32x4 y;
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-          const float v = x[jp][bi][i] * fu_quotient(t[jp][bi][i], d[jp][bi][i] + p.eps);
+          const float v = x[jp][bi][i] * fu_quotient(t[jp][bi][i], d[bi][i] + p.eps);
           y[i] = some ? v : 0.0f;
         }
         if (!whole) {
@@ -344,14 +355,15 @@ __global__ void __launch_bounds__(256, 2) k_fuw(const fuw_args p) {
     __syncthreads();
     if (more) {
       td = nd;
+      if constexpr (COLS) nd = fu_describe<Gather::NG>(p.tiles, p.n_tiles, next + gridDim.x);
       tl = next;
       at = place_of(tl);
+      load_x(at);
     }
     fuw_for_wave(wave, [&](auto w) { fuw_gram<decltype(w)::value, NB>::add(ypl, acc); });
     if (!more) break;
     if constexpr (COLS) {
       if (tid <= at.nc) cps[par ^ 1][at.l0 + tid] = (int)(cpv - td.e0);
-      load_x(at);  // (here and not ahead of the Gram products: registers)
       gather.run(p.pairs, td, Wb, tile);
       split_x();
     }
