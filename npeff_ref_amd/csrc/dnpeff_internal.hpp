@@ -5,6 +5,7 @@
 
 #include <cstdint>
 #include <cstdio>
+#include <initializer_list>
 #include <vector>
 
 #include "../../include/dnpeff.h"
@@ -68,6 +69,14 @@ size_t pool_cached_bytes();  // freed blocks that the pool holds
 void pool_trim();            // back to the device
 hipError_t copy_up(void* dst_dev, const void* src_host, size_t bytes);
 hipError_t copy_down(void* dst_host, const void* src_dev, size_t bytes);
+// The same for several arrays at once.
+struct copy_part {
+  void* dst;
+  const void* src;
+  size_t bytes;
+};
+hipError_t copy_up_parts(std::initializer_list<copy_part> parts);
+hipError_t copy_down_parts(std::initializer_list<copy_part> parts);
 int host_words(unsigned long long** out);  // 64 pinned words of the calling thread
 
 template <class T>

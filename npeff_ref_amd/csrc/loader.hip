@@ -1209,11 +1209,9 @@ DN_API int dnpeff_csr_from_host(int64_t n_rows, int64_t n_cols, int64_t nnz, con
   A->n_rows = n_rows; A->n_cols = n_cols; A->nnz = nnz; A->full_dense_size = n_cols;
   int s = dmalloc(&A->rowptr, n_rows + 1) || dmalloc(&A->colind, nnz) || dmalloc(&A->vals, nnz);
   if (s) { dnpeff_csr_destroy(A); return 1; }
-  hipError_t e = copy_up(A->rowptr, rowptr, sizeof(int64_t) * (n_rows + 1));
-  if (e == hipSuccess && nnz)
-    e = copy_up(A->colind, colind, sizeof(int32_t) * nnz);
-  if (e == hipSuccess && nnz)
-    e = copy_up(A->vals, vals, sizeof(float) * nnz);
+  hipError_t e = copy_up_parts({{A->rowptr, rowptr, sizeof(int64_t) * (n_rows + 1)},
+                                {A->colind, colind, sizeof(int32_t) * nnz},
+                                {A->vals, vals, sizeof(float) * nnz}});
   if (e != hipSuccess) {
     set_error("upload of the CSR arrays failed: %s", hipGetErrorString(e));
     dnpeff_csr_destroy(A);
@@ -1243,9 +1241,7 @@ DN_API int dnpeff_csr_from_pef(int64_t n_rows, int64_t k, int64_t dense_fisher_s
                      A->rowptr);
   hipError_t e = hipGetLastError();
   if (e == hipSuccess && nnz)
-    e = copy_up(A->colind, indices, sizeof(int32_t) * nnz);
-  if (e == hipSuccess && nnz)
-    e = copy_up(A->vals, values, sizeof(float) * nnz);
+    e = copy_up_parts({{A->colind, indices, sizeof(int32_t) * nnz}, {A->vals, values, sizeof(float) * nnz}});
   if (e == hipSuccess) e = hipStreamSynchronize(stream());
   if (e != hipSuccess) {
     set_error("upload of the PEF arrays failed: %s", hipGetErrorString(e));
@@ -1353,13 +1349,9 @@ DN_API int dnpeff_csr_full_dense_size(const dnpeff_csr* A, int64_t* out) {
 DN_API int dnpeff_csr_download(const dnpeff_csr* A, int64_t* rowptr, int32_t* colind, float* vals) {
   clear_error();
   DN_CHECK(A && has_row_major(A), "matrix is NULL or its row-major arrays were released");
-  DN_HIP(hipStreamSynchronize(stream()));
-  if (rowptr)
-    DN_HIP(copy_down(rowptr, A->rowptr, sizeof(int64_t) * (A->n_rows + 1)));
-  if (colind && A->nnz)
-    DN_HIP(copy_down(colind, A->colind, sizeof(int32_t) * A->nnz));
-  if (vals && A->nnz)
-    DN_HIP(copy_down(vals, A->vals, sizeof(float) * A->nnz));
+  DN_HIP(copy_down_parts({{rowptr, A->rowptr, rowptr ? sizeof(int64_t) * (A->n_rows + 1) : 0},
+                          {colind, A->colind, colind ? sizeof(int32_t) * A->nnz : 0},
+                          {vals, A->vals, vals ? sizeof(float) * A->nnz : 0}}));
   return 0;
 }
 

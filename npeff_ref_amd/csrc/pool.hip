@@ -128,77 +128,137 @@ void device_release(void* p) {
 // GB/s down (less into memory that has not been touched yet) where the link carries 57 GB/s from
 // pinned memory.  From STAGED_MIN bytes on, COPY_THREADS threads each move every COPY_THREADS-th
 // piece through two pinned buffers of their own: the host copy (and the page faults of a fresh
-// destination) of one piece runs beside the DMA of the others.  The copies are queued on the library
-// stream (behind everything launched so far) and finished on return.
+// destination) of one piece runs beside the transfer of the others.  A transfer is a kernel that reads or
+// writes the pinned buffer (a piece on the copy engines waits 14 us for its turn), the threads alternate
+// between two streams, so that one piece's completion is not in the way of the next, and several arrays go
+// as one run of pieces.  The copies wait for everything launched on the library stream so far and are
+// finished on return.  131 MB in two arrays: 2.6 ms up and 2.9 ms
+// down, 3.7 and 3.4 ms piece by piece on the copy engines (64 workgroups the same, 128 slower).
 // ---------------------------------------------------------------------------
 constexpr size_t STAGED_MIN = (size_t)4 << 20;
 constexpr size_t STAGE_PIECE = (size_t)2 << 20;
-constexpr int COPY_THREADS = 6;
+constexpr int COPY_THREADS = 8;
+constexpr int COPY_STREAMS = 2;
+constexpr int COPY_WGS = 32;
 
 struct stage_state {
   std::mutex lock;  // one staged copy at a time
+  int dev = -1;
   char* buf[COPY_THREADS][2] = {};
   hipEvent_t done[COPY_THREADS][2] = {};
+  hipEvent_t before = nullptr;  // what the library stream had to do
+  hipStream_t st[COPY_STREAMS] = {};
 };
 static stage_state& stage() {
   static stage_state* s = new stage_state();
   return *s;
 }
 
-static bool stage_ready(stage_state& S) {
+static void stage_free(stage_state& S) {
   for (int t = 0; t < COPY_THREADS; t++)
     for (int b = 0; b < 2; b++) {
-      if (!S.buf[t][b] && hipHostMalloc((void**)&S.buf[t][b], STAGE_PIECE, hipHostMallocDefault) != hipSuccess) {
-        S.buf[t][b] = nullptr;
-        (void)hipGetLastError();
-        return false;
-      }
-      if (!S.done[t][b] && hipEventCreateWithFlags(&S.done[t][b], hipEventDisableTiming) != hipSuccess) {
-        S.done[t][b] = nullptr;
-        (void)hipGetLastError();
-        return false;
-      }
+      if (S.buf[t][b]) (void)hipHostFree(S.buf[t][b]);
+      if (S.done[t][b]) (void)hipEventDestroy(S.done[t][b]);
+      S.buf[t][b] = nullptr;
+      S.done[t][b] = nullptr;
     }
+  for (hipStream_t& st : S.st) {
+    if (st) (void)hipStreamDestroy(st);
+    st = nullptr;
+  }
+  if (S.before) (void)hipEventDestroy(S.before);
+  S.before = nullptr;
+  S.dev = -1;
+}
+
+static bool stage_ready(stage_state& S, int dev) {
+  if (S.dev == dev) return true;
+  stage_free(S);
+  bool ok = hipEventCreateWithFlags(&S.before, hipEventDisableTiming) == hipSuccess;
+  for (int t = 0; t < COPY_THREADS && ok; t++)
+    for (int b = 0; b < 2 && ok; b++)
+      ok = hipHostMalloc((void**)&S.buf[t][b], STAGE_PIECE, hipHostMallocDefault) == hipSuccess &&
+           hipEventCreateWithFlags(&S.done[t][b], hipEventDisableTiming) == hipSuccess;
+  for (int q = 0; q < COPY_STREAMS && ok; q++) ok = hipStreamCreateWithFlags(&S.st[q], hipStreamNonBlocking) == hipSuccess;
+  if (!ok) {
+    (void)hipGetLastError();
+    stage_free(S);
+    return false;
+  }
+  S.dev = dev;
   return true;
 }
 
 static void stage_trim() {
   stage_state& S = stage();
   std::lock_guard<std::mutex> g(S.lock);
-  for (int t = 0; t < COPY_THREADS; t++)
-    for (int b = 0; b < 2; b++) {
-      if (S.buf[t][b]) (void)hipHostFree(S.buf[t][b]);
-      S.buf[t][b] = nullptr;
-    }
+  stage_free(S);
+}
+
+__global__ void __launch_bounds__(256) k_copy_piece(const uint4* __restrict__ src, uint4* __restrict__ dst, int n) {
+  for (int at = blockIdx.x * 1024 + threadIdx.x; at < n; at += gridDim.x * 1024) {
+    uint4 v[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) v[u] = src[at + 256 * u < n ? at + 256 * u : n - 1];
+#pragma unroll
+    for (int u = 0; u < 4; u++)
+      if (at + 256 * u < n) dst[at + 256 * u] = v[u];
+  }
+}
+
+static hipError_t piece_copy(void* dst, const void* src, size_t n, hipMemcpyKind kind, hipStream_t st) {
+  if (n % 16 != 0 || (uintptr_t)dst % 16 != 0 || (uintptr_t)src % 16 != 0) return hipMemcpyAsync(dst, src, n, kind, st);
+  const int quads = (int)(n / 16), wgs = (quads + 1023) / 1024;
+  hipLaunchKernelGGL(k_copy_piece, dim3(wgs < COPY_WGS ? wgs : COPY_WGS), dim3(256), 0, st, (const uint4*)src,
+                     (uint4*)dst, quads);
+  return hipGetLastError();
 }
 
 template <bool UP>
-static hipError_t staged_copy(char* dst, const char* src, size_t bytes) {
+static hipError_t staged_copy(const copy_part* parts, int n_parts) {
   stage_state& S = stage();
   std::lock_guard<std::mutex> g(S.lock);
-  if (!stage_ready(S)) return hipMemcpy(dst, src, bytes, UP ? hipMemcpyHostToDevice : hipMemcpyDeviceToHost);
   int dev = 0;
   hipError_t e = hipGetDevice(&dev);
   if (e != hipSuccess) return e;
-  hipStream_t st = stream();
-  const size_t n_pieces = (bytes + STAGE_PIECE - 1) / STAGE_PIECE;
+  if (!stage_ready(S, dev)) {
+    for (int q = 0; q < n_parts && e == hipSuccess; q++)
+      e = hipMemcpy(parts[q].dst, parts[q].src, parts[q].bytes, UP ? hipMemcpyHostToDevice : hipMemcpyDeviceToHost);
+    return e;
+  }
+  e = hipEventRecord(S.before, stream());
+  for (int q = 0; q < COPY_STREAMS && e == hipSuccess; q++) e = hipStreamWaitEvent(S.st[q], S.before, 0);
+  if (e != hipSuccess) return e;
+  size_t n_pieces = 0;
+  for (int q = 0; q < n_parts; q++) n_pieces += (parts[q].bytes + STAGE_PIECE - 1) / STAGE_PIECE;
   std::atomic<int> failed{(int)hipSuccess};
   auto work = [&](int t) {
     hipError_t e = hipSetDevice(dev);
-    size_t at[2] = {0, 0}, len[2] = {0, 0};  // downwards: the piece a buffer is receiving
-    int k = 0;
+    hipStream_t st = S.st[t % COPY_STREAMS];
+    char* to[2] = {};  // downwards: where the piece goes that a buffer is receiving
+    size_t len[2] = {0, 0};
+    int k = 0, part = 0;
+    size_t first = 0;  // the part's first piece
     for (size_t p = (size_t)t; p < n_pieces && e == hipSuccess; p += COPY_THREADS, k++) {
+      for (;; part++) {
+        const size_t of_part = (parts[part].bytes + STAGE_PIECE - 1) / STAGE_PIECE;
+        if (p < first + of_part) break;
+        first += of_part;
+      }
+      const size_t off = (p - first) * STAGE_PIECE, left = parts[part].bytes - off;
+      const size_t n = left < STAGE_PIECE ? left : STAGE_PIECE;
+      const char* src = (const char*)parts[part].src + off;
+      char* dst = (char*)parts[part].dst + off;
       const int b = k & 1;
-      const size_t off = p * STAGE_PIECE, n = off + STAGE_PIECE < bytes ? STAGE_PIECE : bytes - off;
       if (k >= 2) e = hipEventSynchronize(S.done[t][b]);
       if (e != hipSuccess) break;
       if (UP) {
-        memcpy(S.buf[t][b], src + off, n);
-        e = hipMemcpyAsync(dst + off, S.buf[t][b], n, hipMemcpyHostToDevice, st);
+        memcpy(S.buf[t][b], src, n);
+        e = piece_copy(dst, S.buf[t][b], n, hipMemcpyHostToDevice, st);
       } else {
-        if (len[b]) memcpy(dst + at[b], S.buf[t][b], len[b]);
-        e = hipMemcpyAsync(S.buf[t][b], src + off, n, hipMemcpyDeviceToHost, st);
-        at[b] = off;
+        if (len[b]) memcpy(to[b], S.buf[t][b], len[b]);
+        e = piece_copy(S.buf[t][b], src, n, hipMemcpyDeviceToHost, st);
+        to[b] = dst;
         len[b] = n;
       }
       if (e == hipSuccess) e = hipEventRecord(S.done[t][b], st);
@@ -208,7 +268,7 @@ static hipError_t staged_copy(char* dst, const char* src, size_t bytes) {
       const int b = i & 1;
       const hipError_t es = hipEventSynchronize(S.done[t][b]);
       if (e == hipSuccess) e = es;
-      if (!UP && e == hipSuccess) memcpy(dst + at[b], S.buf[t][b], len[b]);
+      if (!UP && e == hipSuccess) memcpy(to[b], S.buf[t][b], len[b]);
     }
     if (e != hipSuccess) failed = (int)e;
   };
@@ -219,6 +279,7 @@ static hipError_t staged_copy(char* dst, const char* src, size_t bytes) {
   for (std::thread& h : helpers) h.join();
   return (hipError_t)failed.load();
 }
+
 
 // Smaller copies go through one of a few pinned buffers, in two halves where they are longer than one.
 // (hipMemcpy of a few bytes from or to pageable memory takes 30 to 70 us here, and now and then
@@ -340,16 +401,27 @@ static hipError_t bounce_copy(char* dst, const char* src, size_t bytes) {
   return e;
 }
 
-hipError_t copy_up(void* dst_dev, const void* src_host, size_t bytes) {
-  if (bytes == 0) return hipSuccess;
-  if (bytes < STAGED_MIN) return bounce_copy<true>((char*)dst_dev, (const char*)src_host, bytes);
-  return staged_copy<true>((char*)dst_dev, (const char*)src_host, bytes);
+// Short parts one after another through a bounce buffer, the rest in one run of pieces.
+template <bool UP>
+static hipError_t copy_parts(std::initializer_list<copy_part> parts) {
+  std::vector<copy_part> large;
+  for (const copy_part& q : parts) {
+    if (q.bytes >= STAGED_MIN) large.push_back(q);
+    else if (q.bytes) {
+      const hipError_t e = bounce_copy<UP>((char*)q.dst, (const char*)q.src, q.bytes);
+      if (e != hipSuccess) return e;
+    }
+  }
+  return large.empty() ? hipSuccess : staged_copy<UP>(large.data(), (int)large.size());
 }
 
+hipError_t copy_up_parts(std::initializer_list<copy_part> parts) { return copy_parts<true>(parts); }
+hipError_t copy_down_parts(std::initializer_list<copy_part> parts) { return copy_parts<false>(parts); }
+hipError_t copy_up(void* dst_dev, const void* src_host, size_t bytes) {
+  return copy_parts<true>({{dst_dev, src_host, bytes}});
+}
 hipError_t copy_down(void* dst_host, const void* src_dev, size_t bytes) {
-  if (bytes == 0) return hipSuccess;
-  if (bytes < STAGED_MIN) return bounce_copy<false>((char*)dst_host, (const char*)src_dev, bytes);
-  return staged_copy<false>((char*)dst_host, (const char*)src_dev, bytes);
+  return copy_parts<false>({{dst_host, src_dev, bytes}});
 }
 
 // A few pinned words that kernels write results into (one stream synchronisation then replaces a
