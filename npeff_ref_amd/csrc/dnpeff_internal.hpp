@@ -113,6 +113,13 @@ struct dbuf {
   operator T*() const { return p; }
 };
 
+// ---- kept columns, one bit each (columns.hip) ----
+int count_columns(const int32_t* colind, int64_t nnz, int64_t n_cols, int* count);  // (loader.hip)
+int column_mask_of_counts(const int32_t* colind, int64_t nnz, int64_t n_cols, int min_count, uint32_t* mask);
+int column_mask_of_list(const int32_t* kept_ascending, int64_t n_kept, int64_t n_cols, uint32_t* mask);
+// Drops the columns whose bit is clear and renumbers the others; new_to_og (or NULL): their old numbers.
+int keep_columns(dnpeff_csr* A, const uint32_t* mask, int32_t** new_to_og);
+
 // ---- scans (loader.hip) ----
 // out[i] = sum_{i' < i} (count[i'] >= min_count), i in [0, n]; out has n+1 entries.
 int scan_keep_mask(const int* count, int min_count, int64_t n, int32_t* out);

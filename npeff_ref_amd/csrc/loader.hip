@@ -670,6 +670,13 @@ __global__ void __launch_bounds__(256)
 }
 
 // Drops entries whose table[col] == -1 and renumbers the rest (in place on A).
+int count_columns(const int32_t* colind, int64_t nnz, int64_t n_cols, int* count) {
+  DN_HIP(hipMemsetAsync(count, 0, sizeof(int) * (size_t)(n_cols > 0 ? n_cols : 1), stream()));
+  hipLaunchKernelGGL(k_col_hist, dim3(grid_for(nnz, 65536)), dim3(256), 0, stream(), colind, nnz, count);
+  DN_LAUNCH_CHECK();
+  return 0;
+}
+
 static int apply_column_table(dnpeff_csr* A, const int32_t* table, int64_t new_n_cols) {
   hipStream_t st = stream();
   dbuf<int64_t> newpos;
@@ -1275,33 +1282,16 @@ DN_API int dnpeff_csr_normalize_rows(dnpeff_csr* A, const float* norms_host, flo
 DN_API int dnpeff_csr_compact_columns(dnpeff_csr* A, int min_count) {
   clear_error();
   DN_CHECK(A && has_row_major(A), "matrix is NULL or its row-major arrays were released");
-  hipStream_t st = stream();
   drop_derived(A);
   A->sq_norm_valid = false;
-  const int64_t m_full = A->n_cols;
-  dbuf<int> count;
-  dbuf<int32_t> pos, og_to_new, new_to_og;
-  DN_TRY(count.alloc(m_full));
-  DN_HIP(hipMemsetAsync(count, 0, sizeof(int) * (size_t)(m_full > 0 ? m_full : 1), st));
-  hipLaunchKernelGGL(k_col_hist, dim3(grid_for(A->nnz, 65536)), dim3(256), 0, st, A->colind, A->nnz,
-                     count.p);
-  DN_LAUNCH_CHECK();
-  DN_TRY(pos.alloc(m_full + 1));
-  DN_TRY(scan_keep_mask(count, min_count, m_full, pos));
-  int32_t m_new = 0;
-  DN_HIP(copy_down(&m_new, pos + m_full, sizeof(int32_t)));
-  DN_TRY(og_to_new.alloc(m_full));
-  DN_TRY(new_to_og.alloc((int64_t)m_new));
-  hipLaunchKernelGGL(k_build_maps, dim3(grid_for(m_full)), dim3(256), 0, st, count.p, min_count,
-                     pos.p, m_full, og_to_new.p, new_to_og.p);
-  DN_LAUNCH_CHECK();
-  DN_HIP(hipStreamSynchronize(st));
-  count.reset();
-  pos.reset();
-  A->full_dense_size = m_full;
-  DN_TRY(apply_column_table(A, og_to_new, (int64_t)m_new));
+  dbuf<uint32_t> mask;
+  DN_TRY(mask.alloc(ceil_div(A->n_cols, 32)));
+  DN_TRY(column_mask_of_counts(A->colind, A->nnz, A->n_cols, min_count, mask));
+  A->full_dense_size = A->n_cols;
+  int32_t* new_to_og = nullptr;
+  DN_TRY(keep_columns(A, mask, &new_to_og));
   dfree(A->kept);
-  A->kept = new_to_og.release();
+  A->kept = new_to_og;
   return 0;
 }
 
@@ -1309,26 +1299,45 @@ DN_API int dnpeff_csr_retain_columns(dnpeff_csr* A, const int32_t* kept, int64_t
   clear_error();
   DN_CHECK(A && has_row_major(A), "matrix is NULL or its row-major arrays were released");
   DN_CHECK(n_kept >= 0 && (kept || n_kept == 0), "kept is NULL");
-  for (int64_t i = 0; i < n_kept; i++)
+  // (without branches: they took longer than the list's way to the device)
+  const int32_t n_cols = (int32_t)A->n_cols;
+  int outside = 0, descents = 0;
+  if (n_kept) outside = (int)(kept[0] < 0) | (int)(kept[0] >= n_cols);
+  for (int64_t i = 1; i < n_kept; i++) {
+    outside |= (int)(kept[i] < 0) | (int)(kept[i] >= n_cols);
+    descents |= (int)(kept[i] <= kept[i - 1]);
+  }
+  for (int64_t i = 0; outside && i < n_kept; i++)
     DN_CHECK(kept[i] >= 0 && kept[i] < A->n_cols, "kept[%lld] = %d outside [0, %lld)",
              (long long)i, kept[i], (long long)A->n_cols);
   hipStream_t st = stream();
   drop_derived(A);
   A->sq_norm_valid = false;
-  int32_t *table = nullptr, *kept_dev = nullptr;
-  DN_TRY(dmalloc(&table, A->n_cols));
-  DN_TRY(dmalloc(&kept_dev, n_kept));
+  dbuf<int32_t> kept_dev;
+  DN_TRY(kept_dev.alloc(n_kept));
   if (n_kept) DN_HIP(copy_up(kept_dev, kept, sizeof(int32_t) * n_kept));
+  if (!descents) {  // (a new number is the rank among the kept columns)
+    dbuf<uint32_t> mask;
+    DN_TRY(mask.alloc(ceil_div(A->n_cols, 32)));
+    DN_TRY(column_mask_of_list(kept_dev, n_kept, A->n_cols, mask));
+    A->full_dense_size = A->n_cols;
+    DN_TRY(keep_columns(A, mask, nullptr));
+    dfree(A->kept);
+    A->kept = kept_dev.release();
+    return 0;
+  }
+  int32_t* table = nullptr;
+  DN_TRY(dmalloc(&table, A->n_cols));
   hipLaunchKernelGGL(k_fill_i32, dim3(grid_for(A->n_cols)), dim3(256), 0, st, table, A->n_cols, -1);
-  hipLaunchKernelGGL(k_retain_table, dim3(grid_for(n_kept)), dim3(256), 0, st, kept_dev, n_kept,
+  hipLaunchKernelGGL(k_retain_table, dim3(grid_for(n_kept)), dim3(256), 0, st, kept_dev.p, n_kept,
                      table);
   DN_LAUNCH_CHECK();
   A->full_dense_size = A->n_cols;
   int s = apply_column_table(A, table, n_kept);
   dfree(table);
-  if (s) { dfree(kept_dev); return s; }
+  if (s) return s;
   dfree(A->kept);
-  A->kept = kept_dev;
+  A->kept = kept_dev.release();
   return 0;
 }
 
@@ -1426,10 +1435,7 @@ int choose_dense_head(dnpeff_csr* A, double min_fill, double budget, int n_block
   DN_TRY(count.alloc(m));
   DN_TRY(pos.alloc(m + 1));
   DN_TRY(zsum.alloc(1));
-  DN_HIP(hipMemsetAsync(count, 0, sizeof(int) * (size_t)m, st));
-  hipLaunchKernelGGL(k_col_hist, dim3(grid_for(A->nnz, 65536)), dim3(256), 0, st, A->colind, A->nnz,
-                     count.p);
-  DN_LAUNCH_CHECK();
+  DN_TRY(count_columns(A->colind, A->nnz, m, count));
   size_t free_b = 0, total_b = 0;
   DN_HIP(hipMemGetInfo(&free_b, &total_b));
   const int64_t n_pad = ceil_div(n, 128) * 128;
@@ -1480,10 +1486,7 @@ int split_dense_head_at(dnpeff_csr* A, int64_t thr, int64_t* n_dense) {
   dbuf<int> count;
   dbuf<int32_t> pos, slot_of, cols, table;
   DN_TRY(count.alloc(m));
-  DN_HIP(hipMemsetAsync(count, 0, sizeof(int) * (size_t)m, st));
-  hipLaunchKernelGGL(k_col_hist, dim3(grid_for(A->nnz, 65536)), dim3(256), 0, st, A->colind, A->nnz,
-                     count.p);
-  DN_LAUNCH_CHECK();
+  DN_TRY(count_columns(A->colind, A->nnz, m, count));
   DN_TRY(pos.alloc(m + 1));
   DN_TRY(scan_keep_mask(count, (int)thr, m, pos));
   int32_t n_d = 0;
