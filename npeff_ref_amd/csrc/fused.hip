@@ -36,11 +36,16 @@ __host__ __device__ constexpr int fu_lpr(int Q, int R) {
 
 // G as the A operand of the products: [block b of output components][contraction block q][lane][i].
 // part: n_parts partial matrices of packed upper block pairs ([pair][16][16]).
+// (Every thread's numbers of one part are asked for together: one after the other, with the parts inside, the
+// prologue took half of an H update of 145 k columns.)
 template <int Q, int R>
 __device__ inline void fu_load_g(const float* __restrict__ part, int n_parts, int r, float* __restrict__ ga) {
-  constexpr int NB = fu_blocks(Q, R), S = fu_pairs(NB) * 256;
-  for (int x = threadIdx.x; x < NB * NB * 256; x += 256) {
-    const int i = x & 3, lane = (x >> 2) & 63, q = (x >> 8) % NB, b = (x >> 8) / NB;
+  constexpr int NB = fu_blocks(Q, R), S = fu_pairs(NB) * 256, N = NB * NB;
+  int at[N];
+  double sum[N];
+#pragma unroll
+  for (int u = 0; u < N; u++) {
+    const int i = threadIdx.x & 3, lane = (threadIdx.x >> 2) & 63, q = u % NB, b = u / NB;
     const int rho = lane & 15, g = lane >> 4;
     int k, c;
     bool ok = true;
@@ -49,17 +54,22 @@ __device__ inline void fu_load_g(const float* __restrict__ part, int n_parts, in
     if (R == 0 || b < Q) c = 16 * b + rho;
     else { c = 16 * Q + R * (rho >> 2) + (rho & 3); ok = ok && (rho & 3) < R; }
     ok = ok && k < r && c < r;
-    float v = 0.0f;
-    if (ok) {
-      const int bk = k >> 4, bc = c >> 4;
-      const int at = bk <= bc ? fu_pair(bk, bc, NB) * 256 + (k & 15) * 16 + (c & 15)
-                              : fu_pair(bc, bk, NB) * 256 + (c & 15) * 16 + (k & 15);
-      double s = 0.0;
-      for (int p = 0; p < n_parts; p++) s += (double)part[(int64_t)p * S + at];
-      v = (float)s;
-    }
-    ga[x] = v;
+    const int bk = k >> 4, bc = c >> 4;
+    const int x = bk <= bc ? fu_pair(bk, bc, NB) * 256 + (k & 15) * 16 + (c & 15)
+                           : fu_pair(bc, bk, NB) * 256 + (c & 15) * 16 + (k & 15);
+    at[u] = ok ? x : -1;
+    sum[u] = 0.0;
   }
+  for (int p = 0; p < n_parts; p++) {
+    const float* src = part + (int64_t)p * S;
+    float v[N];
+#pragma unroll
+    for (int u = 0; u < N; u++) v[u] = src[at[u] < 0 ? 0 : at[u]];
+#pragma unroll
+    for (int u = 0; u < N; u++) sum[u] += (double)v[u];
+  }
+#pragma unroll
+  for (int u = 0; u < N; u++) ga[threadIdx.x + 256 * u] = at[u] < 0 ? 0.0f : (float)sum[u];
 }
 
 // The components of one factor row that a lane holds: x[b][i] = row[component(b, g, i)], zero past r.

@@ -162,27 +162,34 @@ __global__ void __launch_bounds__(256, 2) k_fuw(const fuw_args p) {
     request(td);
   }
 
-  const int l16_0 = fuw_lane() & 15, g0 = fuw_lane() >> 4;
-  // the wave's rows of G, split: row 16 (b0 + bi) + l16_0, components 32 s + 8 g ..
+  // the wave's rows of G, split: row 16 (b0 + bi) + l16, components 32 s + 8 g ..
   bf16x8 gh[BPW][NS], gm[BPW][NS], gl[BPW][NS];
 #pragma unroll
   for (int bi = 0; bi < BPW; bi++)
 #pragma unroll
     for (int s = 0; s < NS; s++) {
-      f32x4 v[2];
-      const int c = 16 * (b0 + bi) + l16_0;
+      const int lane = fuw_lane(), c = 16 * (b0 + bi) + (lane & 15);
+      int at[8];
+      double sum[8];
 #pragma unroll
       for (int t = 0; t < 8; t++) {
-        const int k = 32 * s + 8 * g0 + t;
-        double sum = 0.0;
-        if (k < r && c < r) {
-          const int bk = k >> 4, bc = c >> 4;
-          const int at = bk <= bc ? fu_pair(bk, bc, NB) * 256 + (k & 15) * 16 + (c & 15)
-                                  : fu_pair(bc, bk, NB) * 256 + (c & 15) * 16 + (k & 15);
-          for (int q = 0; q < p.n_g; q++) sum += (double)p.g[(int64_t)q * (fu_pairs(NB) * 256) + at];
-        }
-        v[t >> 2][t & 3] = (float)sum;
+        const int k = 32 * s + 8 * (lane >> 4) + t, bk = k >> 4, bc = c >> 4;
+        const int x = bk <= bc ? fu_pair(bk, bc, NB) * 256 + (k & 15) * 16 + (c & 15)
+                               : fu_pair(bc, bk, NB) * 256 + (c & 15) * 16 + (k & 15);
+        at[t] = k < r && c < r ? x : -1;
+        sum[t] = 0.0;
       }
+      for (int q = 0; q < p.n_g; q++) {  // (eight numbers of a part at a time under way)
+        const float* src = p.g + (int64_t)q * (fu_pairs(NB) * 256);
+        float w[8];
+#pragma unroll
+        for (int t = 0; t < 8; t++) w[t] = src[at[t] < 0 ? 0 : at[t]];
+#pragma unroll
+        for (int t = 0; t < 8; t++) sum[t] += (double)w[t];
+      }
+      f32x4 v[2];
+#pragma unroll
+      for (int t = 0; t < 8; t++) v[t >> 2][t & 3] = at[t] < 0 ? 0.0f : (float)sum[t];
       bf16x4 h0, m0, l0, h1, m1, l1;
       split3(v[0], h0, m0, l0);
       split3(v[1], h1, m1, l1);
