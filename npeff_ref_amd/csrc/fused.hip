@@ -352,15 +352,13 @@ __device__ inline void fu_sum_parts(const float* __restrict__ part, int n_parts,
   const int x = block * 16 + (threadIdx.x & 15), k = threadIdx.x >> 4;
   const float* p = part + x;
   double s = 0.0;
-  int q = k;
-  for (; q + 7 * 16 < n_parts; q += 8 * 16) {
-    float v[8];
+  for (int q = k; q < n_parts; q += 16 * 16) {  // (sixteen parts at a time under way)
+    float v[16];
 #pragma unroll
-    for (int u = 0; u < 8; u++) v[u] = p[(int64_t)(q + 16 * u) * S];
+    for (int u = 0; u < 16; u++) v[u] = p[(int64_t)(q + 16 * u < n_parts ? q + 16 * u : q) * S];
 #pragma unroll
-    for (int u = 0; u < 8; u++) s += (double)v[u];
+    for (int u = 0; u < 16; u++) s += q + 16 * u < n_parts ? (double)v[u] : 0.0;
   }
-  for (; q < n_parts; q += 16) s += (double)p[(int64_t)q * S];
   red[threadIdx.x] = s;
   __syncthreads();
   if (threadIdx.x < 16) {
