@@ -338,7 +338,12 @@ int dnpeff_nmf_sparsify_W(dnpeff_nmf* nmf, float l1_norm, float l2_norm, int* ro
 int dnpeff_nmf_get_W(dnpeff_nmf* nmf, float* W_nr);
 int dnpeff_nmf_get_H(dnpeff_nmf* nmf, float* H_rm);
 
-/* Device pointers of W [n, r] and H [m, r] (device layout). */
+/* Device pointers of W [n, r] and H [m, r] (device layout); either argument may be NULL.  A pointer
+ * stands for its factor until that factor's next update (dnpeff_nmf_update_W / _update_H, both in
+ * dnpeff_nmf_step) or dnpeff_nmf_destroy; ask again after it.  Until then the caller may read and write
+ * through it between any two calls (with its own work finished when a call begins, and after
+ * dnpeff_sync() for what the calls do): no product that the context keeps from an earlier call is used for
+ * a factor whose pointer is out, so the first update after this call forms H^T H and A H^T again. */
 int dnpeff_nmf_device_factors(dnpeff_nmf* nmf, void** W_dev, void** H_dev);
 
 /* Per-kernel timing with HIP events on the library stream.  enable != 0 turns

@@ -124,7 +124,19 @@ struct dnpeff_nmf {
   bool has_fused = false;
   fused_state fu;
   bool fu_n_valid = false;   // fu.n_part (or Nw, with panels) holds A H^T of the current H
+  // The factor's device pointer was handed out since its last update: the caller may write through it
+  // between any two calls, so no product kept from an earlier call stands for the factor.
+  bool w_out = false, h_out = false;
 };
+
+// Forgets the products kept of factors that a caller may have written to.
+static void forget_handed_out(dnpeff_nmf* h) {
+  if (h->w_out) h->fu.gw_state = fused_state::NONE;
+  if (h->h_out) {
+    h->fu.gh_state = fused_state::NONE;
+    h->gh_valid = h->nw_valid = h->fu_n_valid = false;
+  }
+}
 
 static bool fused_now(const dnpeff_nmf* h) {
   return h->has_fused && tuning().fused_gram != 0.0 && !h->A->tail && !h->prof.enabled;
@@ -524,6 +536,8 @@ static int fused_update_H(dnpeff_nmf* h) {
 DN_API int dnpeff_nmf_update_W(dnpeff_nmf* h) {
   DN_CHECK(h != nullptr, "handle is NULL");
   DN_TRY(take_back(h));
+  forget_handed_out(h);
+  h->w_out = false;
   if (fused_now(h)) return fused_update_W(h);
   h->fu.gw_state = fused_state::NONE;
   dnpeff_csr* A = h->A;
@@ -673,6 +687,8 @@ static int update_H_tiled(dnpeff_nmf* h) {
 DN_API int dnpeff_nmf_update_H(dnpeff_nmf* h) {
   DN_CHECK(h != nullptr, "handle is NULL");
   DN_TRY(take_back(h));
+  forget_handed_out(h);
+  h->h_out = false;
   if (fused_now(h)) return fused_update_H(h);
   h->fu.gh_state = fused_state::NONE;
   h->fu_n_valid = false;
@@ -714,6 +730,7 @@ DN_API int dnpeff_nmf_loss_terms(dnpeff_nmf* h, double* sq_norm_A, double* pos, 
   clear_error();
   DN_CHECK(h != nullptr, "handle is NULL");
   DN_TRY(take_back(h));
+  forget_handed_out(h);
   dnpeff_csr* A = h->A;
   if (fused_now(h)) {
     unsigned long long* words = nullptr;
@@ -858,6 +875,8 @@ DN_API int dnpeff_nmf_device_factors(dnpeff_nmf* nmf, void** W_dev, void** H_dev
   const bool packed = nmf->r != nmf->rl;
   if (W_dev) *W_dev = packed ? nmf->Wp : nmf->W;
   if (H_dev) *H_dev = packed ? nmf->Hp : nmf->H;
+  nmf->w_out = nmf->w_out || W_dev;
+  nmf->h_out = nmf->h_out || H_dev;
   return 0;
 }
 
