@@ -90,9 +90,8 @@ struct dnpeff_nmf {
   // next one (padded_rank): the updates keep those zero, and every kernel made for multiples of 128
   // runs.  The factors that callers see are packed.
   int rl = 0;
-  float* Wp = nullptr;       // packed copies handed out by dnpeff_nmf_device_factors, while r != rl
-  float* Hp = nullptr;
-  bool handed_out = false;   // ... since the factors last changed: a caller may have written to them
+  float* Wp = nullptr;       // packed copies handed out by dnpeff_nmf_device_factors, while r != rl: they
+  float* Hp = nullptr;       // are the factors as long as their pointers are out (take_back, show)
   float eps = 0.0f;
   uint64_t seed = 0;
   int64_t n = 0, m = 0;
@@ -129,13 +128,28 @@ struct dnpeff_nmf {
   bool w_out = false, h_out = false;
 };
 
-// Forgets the products kept of factors that a caller may have written to.
-static void forget_handed_out(dnpeff_nmf* h) {
-  if (h->w_out) h->fu.gw_state = fused_state::NONE;
+// At the start of every call that uses the factors: those whose pointers are out are what the caller
+// has left there (packed copies are copied back), and what is kept of them is forgotten.
+static int take_back(dnpeff_nmf* h) {
+  const bool packed = h->r != h->rl;
+  if (h->w_out) {
+    if (packed) DN_TRY(launch_copy_rows(h->n, h->rl, h->Wp, h->rl, h->W, h->r));
+    h->fu.gw_state = fused_state::NONE;
+  }
   if (h->h_out) {
+    if (packed) DN_TRY(launch_copy_rows(h->m, h->rl, h->Hp, h->rl, h->H, h->r));
     h->fu.gh_state = fused_state::NONE;
     h->gh_valid = h->nw_valid = h->fu_n_valid = false;
   }
+  return 0;
+}
+
+// At the end of every call that changes a factor in place: packed copies whose pointers are out show it.
+static int show(dnpeff_nmf* h, bool w, bool hh) {
+  if (h->r == h->rl) return 0;
+  if (w && h->w_out) DN_TRY(launch_copy_rows(h->n, h->rl, h->W, h->r, h->Wp, h->rl));
+  if (hh && h->h_out) DN_TRY(launch_copy_rows(h->m, h->rl, h->H, h->r, h->Hp, h->rl));
+  return 0;
 }
 
 static bool fused_now(const dnpeff_nmf* h) {
@@ -431,24 +445,16 @@ DN_API int dnpeff_nmf_init_factors(dnpeff_nmf* nmf) {
   nmf->nw_valid = false;
   nmf->fu_n_valid = false;
   nmf->fu.gh_state = nmf->fu.gw_state = fused_state::NONE;
-  nmf->handed_out = false;
   if (nmf->r != nmf->rl) {
     DN_TRY(launch_init_uniform(0, nmf->n, nmf->rl, nmf->seed, nmf->W2));
     DN_TRY(launch_copy_rows(nmf->n, nmf->rl, nmf->W2, nmf->rl, nmf->W, nmf->r));
     DN_TRY(launch_init_uniform(1, nmf->rl, nmf->m, nmf->seed, nmf->S));
-    return launch_copy_rows(nmf->m, nmf->rl, nmf->S, nmf->rl, nmf->H, nmf->r);
+    DN_TRY(launch_copy_rows(nmf->m, nmf->rl, nmf->S, nmf->rl, nmf->H, nmf->r));
+    return show(nmf, true, true);
   }
   DN_TRY(launch_init_uniform(0, nmf->n, nmf->r, nmf->seed, nmf->W));
   DN_TRY(launch_init_uniform(1, nmf->r, nmf->m, nmf->seed, nmf->H));
   return 0;
-}
-
-// Packed copies that were handed out become the factors again before anything reads them.
-static int take_back(dnpeff_nmf* h) {
-  if (!h->handed_out) return 0;
-  h->handed_out = false;
-  DN_TRY(launch_copy_rows(h->n, h->rl, h->Wp, h->rl, h->W, h->r));
-  return launch_copy_rows(h->m, h->rl, h->Hp, h->rl, h->H, h->r);
 }
 
 DN_API int dnpeff_nmf_set_factors(dnpeff_nmf* nmf, const float* W_nr, const float* H_rm) {
@@ -483,7 +489,7 @@ DN_API int dnpeff_nmf_set_factors(dnpeff_nmf* nmf, const float* W_nr, const floa
       DN_HIP(hipStreamSynchronize(stream()));
     }
   }
-  return 0;
+  return show(nmf, W_nr != nullptr, H_rm != nullptr);
 }
 
 // The matrix may have been planned again for another rank since this handle was made (a second
@@ -536,7 +542,6 @@ static int fused_update_H(dnpeff_nmf* h) {
 DN_API int dnpeff_nmf_update_W(dnpeff_nmf* h) {
   DN_CHECK(h != nullptr, "handle is NULL");
   DN_TRY(take_back(h));
-  forget_handed_out(h);
   h->w_out = false;
   if (fused_now(h)) return fused_update_W(h);
   h->fu.gw_state = fused_state::NONE;
@@ -687,7 +692,6 @@ static int update_H_tiled(dnpeff_nmf* h) {
 DN_API int dnpeff_nmf_update_H(dnpeff_nmf* h) {
   DN_CHECK(h != nullptr, "handle is NULL");
   DN_TRY(take_back(h));
-  forget_handed_out(h);
   h->h_out = false;
   if (fused_now(h)) return fused_update_H(h);
   h->fu.gh_state = fused_state::NONE;
@@ -730,7 +734,6 @@ DN_API int dnpeff_nmf_loss_terms(dnpeff_nmf* h, double* sq_norm_A, double* pos, 
   clear_error();
   DN_CHECK(h != nullptr, "handle is NULL");
   DN_TRY(take_back(h));
-  forget_handed_out(h);
   dnpeff_csr* A = h->A;
   if (fused_now(h)) {
     unsigned long long* words = nullptr;
@@ -824,7 +827,8 @@ DN_API int dnpeff_nmf_sparsify_W(dnpeff_nmf* nmf, float l1_norm, float l2_norm, 
   if (nmf->r != nmf->rl) {
     DN_TRY(launch_copy_rows(nmf->n, nmf->rl, nmf->W, nmf->r, nmf->W2, nmf->rl));
     DN_TRY(sparsify_columns(nmf->n, nmf->rl, nmf->W2, l1_norm, l2_norm, rounds));
-    return launch_copy_rows(nmf->n, nmf->rl, nmf->W2, nmf->rl, nmf->W, nmf->r);
+    DN_TRY(launch_copy_rows(nmf->n, nmf->rl, nmf->W2, nmf->rl, nmf->W, nmf->r));
+    return show(nmf, true, false);
   }
   return sparsify_columns(nmf->n, nmf->r, nmf->W, l1_norm, l2_norm, rounds);
 }
@@ -865,14 +869,15 @@ DN_API int dnpeff_nmf_get_H(dnpeff_nmf* nmf, float* H_rm) {
 
 DN_API int dnpeff_nmf_device_factors(dnpeff_nmf* nmf, void** W_dev, void** H_dev) {
   DN_CHECK(nmf != nullptr, "handle is NULL");
-  if (nmf->r != nmf->rl && !nmf->handed_out) {
-    if (!nmf->Wp) DN_TRY(dmalloc(&nmf->Wp, nmf->n * nmf->rl));
-    if (!nmf->Hp) DN_TRY(dmalloc(&nmf->Hp, nmf->m * nmf->rl));
-    DN_TRY(launch_copy_rows(nmf->n, nmf->rl, nmf->W, nmf->r, nmf->Wp, nmf->rl));
-    DN_TRY(launch_copy_rows(nmf->m, nmf->rl, nmf->H, nmf->r, nmf->Hp, nmf->rl));
-    nmf->handed_out = true;
-  }
   const bool packed = nmf->r != nmf->rl;
+  if (packed && W_dev && !nmf->w_out) {
+    if (!nmf->Wp) DN_TRY(dmalloc(&nmf->Wp, nmf->n * nmf->rl));
+    DN_TRY(launch_copy_rows(nmf->n, nmf->rl, nmf->W, nmf->r, nmf->Wp, nmf->rl));
+  }
+  if (packed && H_dev && !nmf->h_out) {
+    if (!nmf->Hp) DN_TRY(dmalloc(&nmf->Hp, nmf->m * nmf->rl));
+    DN_TRY(launch_copy_rows(nmf->m, nmf->rl, nmf->H, nmf->r, nmf->Hp, nmf->rl));
+  }
   if (W_dev) *W_dev = packed ? nmf->Wp : nmf->W;
   if (H_dev) *H_dev = packed ? nmf->Hp : nmf->H;
   nmf->w_out = nmf->w_out || W_dev;

@@ -63,7 +63,7 @@ class Run:
             assert np.linalg.norm(got - want) <= 1e-5 * np.linalg.norm(want)
 
 
-RANKS = [5, 16, 50, 100, 128, 256]
+RANKS = [5, 16, 50, 100, 128, 129, 200, 256]
 
 
 @pytest.mark.parametrize("r", RANKS)
@@ -96,4 +96,43 @@ def test_written_between_calls(n, m, r):
         t.nmf.update_H()
         t.step_is_that_of(W, H, W_between=W1, H_between=H1)
         t.loss_is_that_of(*t.factors())
+    t.close()
+
+
+@pytest.mark.parametrize("r", [16, 100, 129, 200, 256])
+def test_pointers_follow_what_changes_the_factors_in_place(r):
+    n, m = 60, 400
+    t = Run(n, m, r)
+    w, h = t.nmf.device_factors()
+
+    def show(W, H):
+        assert np.array_equal(d.gather_rows(w, r, np.arange(n)), W)
+        assert np.array_equal(d.gather_rows(h, r, np.arange(m)), H.T)
+
+    W, H = t.new_W(), t.new_H()
+    t.nmf.set_factors(W, None)
+    t.nmf.set_factors(None, H)
+    show(W, H)
+    t.loss_is_that_of(W, H)
+    # one written through its pointer, the other set from the host
+    W, H = t.new_W(), t.new_H()
+    t.write(h, H.T)
+    t.nmf.set_factors(W, None)
+    show(W, H)
+    t.loss_is_that_of(W, H)
+    t.write(w, W)
+    t.nmf.sparsify_W(3.0)
+    W = t.nmf.loadWToHostSync()
+    show(W, H)
+    t.loss_is_that_of(W, H)
+    t.nmf.initialize()
+    show(*t.factors())
+    # W's pointer alone: H keeps what is at hand of it
+    t.nmf.step(1)
+    W, H = t.factors()
+    ptr = C.c_void_p()
+    d.binding._check(d.lib.dnpeff_nmf_device_factors(t.nmf._h, C.byref(ptr), None))
+    W = t.new_W()
+    t.write(ptr.value, W)
+    t.loss_is_that_of(W, H)
     t.close()
