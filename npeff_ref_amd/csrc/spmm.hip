@@ -1433,11 +1433,13 @@ static int launch_spmm_t_sparse(const dnpeff_csr* A, int r, const float* W_nr, f
   const bool aligned = ((uintptr_t)T % 16) == 0 && ((uintptr_t)W_nr % 16) == 0;
   if (A->tb.cols && aligned && col0 % 64 == 0 && (col1 % 64 == 0 || col1 == A->n_cols) && use_tlists(A, r))
     return launch_spmm_t_lists(A, r, W_nr, T, col0, col1);
-  if (A->fused.tiles && A->fused.tile_cols == 32 && aligned && use_spmm_t_bal(A, r)) {
+  // (a range of columns that does not begin and end between the work list's groups: the grouped kernel below)
+  const bool all = col0 == 0 && col1 == A->n_cols;
+  const bool on_groups = col0 % 32 == 0 && (col1 % 32 == 0 || col1 == A->n_cols);
+  if (A->fused.tiles && A->fused.tile_cols == 32 && aligned && use_spmm_t_bal(A, r) && (all || on_groups)) {
     int64_t t0 = 0, t1 = A->fused.n_tiles;
-    if (col0 > 0 || col1 < A->n_cols) {
-      DN_CHECK(!A->fused.h_first.empty() && col0 % 32 == 0 && (col1 % 32 == 0 || col1 == A->n_cols),
-               "column tile [%lld, %lld) does not lie on the plan's groups", (long long)col0, (long long)col1);
+    if (!all) {
+      DN_CHECK(!A->fused.h_first.empty(), "matrix has no host lists for column tiles");
       t0 = A->fused.h_first[col0 / 32];
       t1 = A->fused.h_first[ceil_div(col1, 32)];
     }

@@ -33,6 +33,29 @@ def test_spmm_t_balanced(n, m, r):
     A.close()
 
 
+@pytest.mark.parametrize("r", [132, 256, 600])
+def test_spmm_t_tile_at_any_column(r):
+    """Tiles on and off the groups of 32 columns: the rows of the whole product, bit for bit."""
+    n, m = 600, 203
+    rng = np.random.default_rng(r)
+    mask = rng.random((n, m)) < rng.choice([0.0, 0.02, 0.3, 1.0], size=m)
+    mask[0, 0] = True
+    rp = np.concatenate([[0], np.cumsum(mask.sum(axis=1))]).astype(np.int64)
+    ci = np.nonzero(mask)[1].astype(np.int32)
+    A = d.Csr.from_host(rp, ci, rng.random(len(ci)).astype(np.float32), m)
+    dW, dT = d.DeviceArray.from_numpy(rng.random((n, r)).astype(np.float32)), d.DeviceArray((m, r))
+    d.op_spmm_t(A, r, dW, dT)
+    d.sync()
+    whole = dT.numpy()
+    for c0, c1 in ((0, m), (32, 96), (64, m), (1, 32), (31, 33), (5, 200), (32, 50), (m - 1, m), (7, 7)):
+        dP = d.DeviceArray.from_numpy(np.full((m, r), np.nan, dtype=np.float32))
+        d.binding._check(d.lib.dnpeff_op_spmm_t_tile(A._h, r, dW.ptr, c0, c1, dP.ptr))
+        d.sync()
+        got = dP.numpy()
+        assert np.array_equal(got[:c1 - c0], whole[c0:c1]) and np.isnan(got[c1 - c0:]).all()
+    A.close()
+
+
 @pytest.mark.parametrize("rows", [128, 129, 160, 191, 1023])
 @pytest.mark.parametrize("r", [256, 384, 512, 768])
 def test_gram_on_few_rows(rows, r):
