@@ -4,6 +4,7 @@
 // accumulation, seeded initialisation and the [m, r] <-> [r, m] transposition.
 #include "dnpeff_internal.hpp"
 #include "abt_b16.hpp"
+#include "quotient.hpp"
 #include "synth_rng.h"
 
 #include <algorithm>
@@ -12,14 +13,6 @@
 namespace dn {
 
 typedef float acc16 __attribute__((ext_vector_type(16)));
-
-// n / den from the reciprocal (1 ulp) and one correction step: 5 vector instructions where the
-// IEEE division sequence takes 11.  For the epilogues of the split-operand updates, where
-// den = (X G) + eps is positive and normal; within 2 ulp of the quotient.
-__device__ __forceinline__ float mu_quotient(float n, float den) {
-  const float rc = __builtin_amdgcn_rcpf(den), q0 = n * rc;
-  return __builtin_fmaf(__builtin_fmaf(-den, q0, n), rc, q0);
-}
 
 // ---------------------------------------------------------------------------
 // F[i] *= num[i] / (den[i] + eps)      (divide first, then multiply)
@@ -1039,12 +1032,20 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
   auto finish = [&](int blk, const float (&n_)[16], const float (&x_)[16]) {
     const int i = blk >> 1, j = blk & 1;
 #pragma unroll
-    for (int v = 0; v < 16; v++) {
-      const int64_t off = (32 * i + 8 * (v >> 2) + (v & 3)) * (int64_t)r + 32 * j + l32;
-      const float d = acc[i][j][v];
-      const float q = mu_quotient(n_[v], d + eps);
-      tout[off] = x_[v] * q;
-      if (WITH_D) tD[off] = d;
+    for (int v4 = 0; v4 < 16; v4 += 4) {
+      f32x4 n4, d4;
+#pragma unroll
+      for (int u = 0; u < 4; u++) {
+        n4[u] = n_[v4 + u];
+        d4[u] = acc[i][j][v4 + u];
+      }
+      const f32x4 q = mu_quotients(n4, d4 + eps);
+#pragma unroll
+      for (int u = 0; u < 4; u++) {
+        const int64_t off = (32 * i + 2 * v4 + u) * (int64_t)r + 32 * j + l32;
+        tout[off] = x_[v4 + u] * q[u];
+        if (WITH_D) tD[off] = d4[u];
+      }
     }
   };
   request(0, pn[0], px[0]);
@@ -1104,12 +1105,20 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))
   auto finish = [&](int blk, const float (&n_)[16], const float (&x_)[16]) {
     const int i = blk >> 1, j = blk & 1;
 #pragma unroll
-    for (int v = 0; v < 16; v++) {
-      const int64_t off = (32 * i + 8 * (v >> 2) + (v & 3)) * (int64_t)r + 32 * j + l32;
-      const float d = acc[i][j][v];
-      const float q = mu_quotient(n_[v], d + eps);
-      tout[off] = x_[v] * q;
-      if (WITH_D) tD[off] = d;
+    for (int v4 = 0; v4 < 16; v4 += 4) {
+      f32x4 n4, d4;
+#pragma unroll
+      for (int u = 0; u < 4; u++) {
+        n4[u] = n_[v4 + u];
+        d4[u] = acc[i][j][v4 + u];
+      }
+      const f32x4 q = mu_quotients(n4, d4 + eps);
+#pragma unroll
+      for (int u = 0; u < 4; u++) {
+        const int64_t off = (32 * i + 2 * v4 + u) * (int64_t)r + 32 * j + l32;
+        tout[off] = x_[v4 + u] * q[u];
+        if (WITH_D) tD[off] = d4[u];
+      }
     }
   };
   request(0, pn[0], px[0]);
@@ -1629,10 +1638,20 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 #pragma unroll
       for (int v = 0; v < 16; v++) x[v] = xraw[(8 * (v >> 2) + 4 * half + (v & 3)) * XB_LDR + col];
 #pragma unroll
-      for (int v = 0; v < 16; v++) {
-        const float o = x[v] * mu_quotient(pn[v], a0[v] + eps);
-        pn[v] = o;
-        (tout + (8 * (v >> 2) + (v & 3)) * r)[off0] = o;
+      for (int v4 = 0; v4 < 16; v4 += 4) {
+        f32x4 n4, d4;
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+          n4[u] = pn[v4 + u];
+          d4[u] = a0[v4 + u];
+        }
+        const f32x4 q = mu_quotients(n4, d4 + eps);
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+          const float o = x[v4 + u] * q[u];
+          pn[v4 + u] = o;
+          (tout + (2 * v4 + u) * r)[off0] = o;
+        }
       }
     }
     // parts of the result: registers for the A side, LDS (transposed) for the other waves.

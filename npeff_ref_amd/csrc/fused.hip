@@ -118,10 +118,11 @@ __device__ inline void fu_update(const float* __restrict__ ga, f32x4 (&x)[fu_blo
 #pragma unroll
   for (int b = 0; b < NB; b++) {
     f32x4 y;
+    const f32x4 q = mu_quotients(t[b], d[b] + eps);
 #pragma unroll
     for (int i = 0; i < 4; i++) {
       const int c = b < Q ? 16 * b + 4 * g + i : 16 * Q + R * g + i;
-      const float v = x[b][i] * fu_quotient(t[b][i], d[b][i] + eps);
+      const float v = x[b][i] * q[i];
       const bool in = R > 0 ? b < Q || (i < R && c < r) : b < Q - 1 || c < r;
       y[i] = store && in ? v : 0.0f;
     }

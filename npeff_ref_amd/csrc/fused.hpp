@@ -2,6 +2,7 @@
 #pragma once
 
 #include "dnpeff_internal.hpp"
+#include "quotient.hpp"
 #include "split_bf16.hpp"
 
 namespace dn {
@@ -172,12 +173,5 @@ __device__ inline void fu_cut_by(int a0, int a1, int share, float inv, int& k0, 
   k0 = quot(a0) + 1;
   k1 = quot(a1 - 1) + 1;
 }
-
-// Update quotient: the reciprocal and one correction step, within an ulp of the division.
-__device__ inline float fu_quotient(float t, float den) {
-  const float inv = __builtin_amdgcn_rcpf(den), q0 = t * inv;
-  return fmaf(fmaf(-q0, den, t), inv, q0);
-}
-
 
 }  // namespace dn

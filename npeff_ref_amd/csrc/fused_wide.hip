@@ -330,9 +330,10 @@ __global__ void __launch_bounds__(256, 2) k_fuw(const fuw_args p) {
         if (b >= NB) continue;
         const bool whole = 16 * b + 16 <= r;
         f32x4 y;
+        const f32x4 quot = mu_quotients(t[jp][bi], d[bi] + p.eps);
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-          const float v = x[jp][bi][i] * fu_quotient(t[jp][bi][i], d[bi][i] + p.eps);
+          const float v = x[jp][bi][i] * quot[i];
           y[i] = some ? v : 0.0f;
         }
         if (!whole) {
