@@ -504,10 +504,7 @@ static int products_for(dnpeff_nmf* h) {
 static int fused_products(dnpeff_nmf* h) {
   DN_TRY(products_for(h));
   DN_TRY(fused_plan_build(h->A, h->r));
-  if (h->fu.gh_state == fused_state::NONE) {
-    DN_TRY(launch_gram(h->m, h->r, h->H, h->G, h->gram_ws));
-    DN_TRY(h->fu.set_gram(h->G, true));
-  }
+  if (h->fu.gh_state == fused_state::NONE) DN_TRY(h->fu.gram_of(h->H, h->m, true));
   if (!h->fu_n_valid) {
     if (h->A->n_panels > 0) {
       DN_TRY(launch_spmm_n(h->A, h->r, h->H));
@@ -531,10 +528,7 @@ static int fused_update_W(dnpeff_nmf* h) {
 static int fused_update_H(dnpeff_nmf* h) {
   DN_TRY(products_for(h));
   DN_TRY(fused_plan_build(h->A, h->r));
-  if (h->fu.gw_state == fused_state::NONE) {
-    DN_TRY(launch_gram(h->n, h->r, h->W, h->G, h->gram_ws));
-    DN_TRY(h->fu.set_gram(h->G, false));
-  }
+  if (h->fu.gw_state == fused_state::NONE) DN_TRY(h->fu.gram_of(h->W, h->n, false));
   h->nw_valid = h->gh_valid = h->fu_n_valid = false;
   return h->fu.update_h(h->A, h->W, h->H, h->eps);
 }
@@ -740,10 +734,7 @@ DN_API int dnpeff_nmf_loss_terms(dnpeff_nmf* h, double* sq_norm_A, double* pos, 
     DN_TRY(host_words(&words));
     double* sums = reinterpret_cast<double*>(words);
     DN_TRY(fused_products(h));
-    if (h->fu.gw_state == fused_state::NONE) {
-      DN_TRY(launch_gram(h->n, h->r, h->W, h->G, h->gram_ws));
-      DN_TRY(h->fu.set_gram(h->G, false));
-    }
+    if (h->fu.gw_state == fused_state::NONE) DN_TRY(h->fu.gram_of(h->W, h->n, false));
     DN_TRY(h->fu.loss_sums(A, h->n, fused_nw(h), h->W, sums));
     DN_HIP(hipStreamSynchronize(stream()));
     if (sq_norm_A) *sq_norm_A = h->sq_norm_A;

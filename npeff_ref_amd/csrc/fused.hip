@@ -374,13 +374,156 @@ __global__ void __launch_bounds__(256)
   fu_sum_parts(part, n_parts, S, blockIdx.x, out, red);
 }
 
-// A full Gram matrix [r, r] as one packed partial.
-__global__ void __launch_bounds__(256) k_fu_pack(const float* __restrict__ G, int r, int nb, float* __restrict__ out) {
-  int p = blockIdx.x, b1 = 0;
-  while (p >= nb - b1) p -= nb - b1, b1++;
-  const int b2 = b1 + p;
-  const int a = 16 * b1 + (threadIdx.x >> 4), b = 16 * b2 + (threadIdx.x & 15);
-  out[blockIdx.x * 256 + threadIdx.x] = a < r && b < r ? G[(int64_t)a * r + b] : 0.0f;
+// X^T X of a factor that no update of the step has left, `per` rows (a multiple of 64) per workgroup, as
+// partial matrices like the updates'.  The fp32 sums of 256 rows are added up in fp64.
+//
+// Up to 4 blocks of 16 components each wave takes every fourth 16 rows and all block pairs; the operands
+// need no LDS there: a lane's number of a row is one 4-byte load, 16 lanes a whole sector.  861,696 x 50 in
+// 80 us (708 with k_gram), 429,626 x 16 in 9 (36).
+template <int NB>
+__device__ inline void fu_gram_fold(double (&sum)[NB][4], f32x4 (&acc)[NB]) {
+#pragma unroll
+  for (int p = 0; p < NB; p++)
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      sum[p][i] += (double)acc[p][i];
+      acc[p][i] = 0.0f;
+    }
+}
+
+template <int NB>
+__global__ void __launch_bounds__(256)
+    k_fu_gram(const float* __restrict__ X, int64_t rows, int64_t per, int r, float* __restrict__ gpart) {
+  constexpr int NP = fu_pairs(NB);
+  __shared__ float lds[NP * 256];
+  const int64_t row0 = blockIdx.x * per, row1 = row0 + per < rows ? row0 + per : rows;
+  const int lane = threadIdx.x & 63, l16 = lane & 15, g = lane >> 4;
+  float a[4][NB], nx[4][NB];
+  auto load = [&](int64_t base, float (&v)[4][NB]) {
+#pragma unroll
+    for (int s = 0; s < 4; s++) {
+      const int64_t row = base + 4 * s + g;
+#pragma unroll
+      for (int b = 0; b < NB; b++)
+        v[s][b] = X[row < row1 && 16 * b + l16 < r ? row * r + 16 * b + l16 : 0];
+    }
+  };
+  double sum[NP][4] = {};
+  f32x4 acc[NP] = {};
+  int64_t base = row0 + 16 * (int)(threadIdx.x >> 6);
+  load(base, a);
+  for (int k = 1; base < row1; base += 64, k++) {
+    load(base + 64, nx);
+#pragma unroll
+    for (int s = 0; s < 4; s++) {
+#pragma unroll
+      for (int b = 0; b < NB; b++) a[s][b] = base + 4 * s + g < row1 && 16 * b + l16 < r ? a[s][b] : 0.0f;
+      int p = 0;
+#pragma unroll
+      for (int b1 = 0; b1 < NB; b1++)
+#pragma unroll
+        for (int b2 = b1; b2 < NB; b2++, p++)
+          acc[p] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[s][b1], a[s][b2], acc[p], 0, 0, 0);
+#pragma unroll
+      for (int b = 0; b < NB; b++) a[s][b] = nx[s][b];
+    }
+    if (k % 16 == 0) fu_gram_fold<NP>(sum, acc);
+  }
+  fu_gram_fold<NP>(sum, acc);
+#pragma unroll
+  for (int p = 0; p < NP; p++)
+#pragma unroll
+    for (int i = 0; i < 4; i++) acc[p][i] = (float)sum[p][i];
+  fu_gram_out<NP>(acc, lds, gpart + (int64_t)blockIdx.x * (NP * 256));
+}
+
+// 5 to 8 blocks: all waves take the same rows, 32 at a time through LDS (rows 16 banks apart: the four
+// rows of an operand do not meet), and their share of the pairs, block rows W and 7 - W.  Bound by the fp32
+// matrix cores (400 us of them at 3.4 M x 128): 597 us (1362 with k_gram; 964 with every wave's operands
+// straight from global memory, one trip of latency for 36 matrix instructions).
+constexpr int FU_GRAM_ROWS = 32;
+constexpr int fu_gram_stride(int nb) { return 16 * (nb | 1); }
+
+template <int NB>
+__global__ void __launch_bounds__(256, 2)
+    k_fu_gram_wide(const float* __restrict__ X, int64_t rows, int64_t per, int r, float* __restrict__ gpart) {
+  constexpr int NA = fuw_pairs(NB), LD = fu_gram_stride(NB);
+  __shared__ __align__(16) float lds[2 * FU_GRAM_ROWS * LD];
+  const int64_t row0 = blockIdx.x * per, row1 = row0 + per < rows ? row0 + per : rows;
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, l16 = lane & 15, g = lane >> 4;
+  const int c4 = 4 * (tid & 31), lr = tid >> 5;  // loader: four components of every eighth row
+  f32x4 st[4];
+  auto fetch = [&](int64_t base) {
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      const int64_t row = base + lr + 8 * q;
+      // (a row's last piece may end past it: the arrays have four spare floats)
+      st[q] = *reinterpret_cast<const f32x4u*>(X + (row < row1 && c4 < r ? row * r + c4 : 0));
+    }
+  };
+  auto commit = [&](int64_t base, float* to) {  // (zeros past the rows and the rank put in here: the loads stay on their way)
+    if (c4 < 16 * NB) {
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        f32x4 v;
+#pragma unroll
+        for (int i = 0; i < 4; i++) v[i] = base + lr + 8 * q < row1 && c4 + i < r ? st[q][i] : 0.0f;
+        *reinterpret_cast<f32x4*>(to + (lr + 8 * q) * LD + c4) = v;
+      }
+    }
+  };
+  double sum[NA][4] = {};
+  f32x4 acc[NA] = {};
+  fetch(row0);
+  commit(row0, lds);
+  fetch(row0 + FU_GRAM_ROWS);
+  __syncthreads();
+  int k = 0;
+  for (int64_t base = row0; base < row1; base += FU_GRAM_ROWS, k++) {
+    const float* at = lds + (k & 1) * FU_GRAM_ROWS * LD + g * LD + l16;
+    fuw_for_wave(wave, [&](auto w) {
+      constexpr int W = decltype(w)::value, W1 = 7 - W;
+      float a[2][NB];  // the next rows' operands are read ahead of the matrix instructions
+      auto read = [&](int s, float (&v)[NB]) {
+#pragma unroll
+        for (int b = W; b < NB; b++) v[b] = at[4 * s * LD + 16 * b];
+      };
+      read(0, a[0]);
+#pragma unroll
+      for (int s = 0; s < FU_GRAM_ROWS / 4; s++) {
+        const float (&v)[NB] = a[s & 1];
+        if (s + 1 < FU_GRAM_ROWS / 4) read(s + 1, a[(s + 1) & 1]);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int b = W; b < NB; b++) {
+          acc[b - W] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[W], v[b], acc[b - W], 0, 0, 0);
+          if constexpr (W1 < NB) {
+            if (b >= W1) acc[NB - W + b - W1] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[W1], v[b], acc[NB - W + b - W1], 0, 0, 0);
+          }
+        }
+      }
+    });
+    // (the other buffer was last read before the barrier that ended the step before)
+    commit(base + FU_GRAM_ROWS, lds + ((k + 1) & 1) * FU_GRAM_ROWS * LD);
+    fetch(base + 2 * FU_GRAM_ROWS);
+    if (k % 8 == 7) fu_gram_fold<NA>(sum, acc);
+    __syncthreads();
+  }
+  fu_gram_fold<NA>(sum, acc);
+  float* out = gpart + (int64_t)blockIdx.x * (fu_pairs(NB) * 256);
+  auto put = [&](int b1, int b2, const double (&v)[4]) {
+#pragma unroll
+    for (int i = 0; i < 4; i++) out[fu_pair(b1, b2, NB) * 256 + (4 * g + i) * 16 + l16] = (float)v[i];
+  };
+  fuw_for_wave(wave, [&](auto w) {
+    constexpr int W = decltype(w)::value, W1 = 7 - W;
+#pragma unroll
+    for (int b = W; b < NB; b++) put(W, b, sum[b - W]);
+    if constexpr (W1 < NB) {
+#pragma unroll
+      for (int b = W1; b < NB; b++) put(W1, b, sum[NB - W + b - W1]);
+    }
+  });
 }
 
 // A H^T: chunk blockIdx.x - sum_wgs of the entries, all of one row; the wave's lane groups take them
@@ -771,11 +914,21 @@ static int fu_sum(const float* part, int n_parts, int S, float* out) {
   return 0;
 }
 
-int fused_state::set_gram(const float* G, bool of_h) {
-  const int nb = fu_blocks_of(r);
-  hipLaunchKernelGGL(k_fu_pack, dim3((unsigned)fu_pairs(nb)), dim3(256), 0, stream(), G, r, nb, of_h ? gh_sum : gw_sum);
+int fused_state::gram_of(const float* X, int64_t rows, bool of_h) {
+  const int parts = of_h ? h_wgs : w_wgs;
+  float* out = of_h ? gh_part : gw_part;
+  const int64_t per = ceil_div(ceil_div(rows, parts), 64) * 64;
+  const dim3 grid((unsigned)parts), block(256);
+  switch (fu_blocks_of(r)) {  // (workgroups past the last row leave zeros)
+#define DN_FU_GRAM(NB, K) \
+  case NB: hipLaunchKernelGGL(K<NB>, grid, block, 0, stream(), X, rows, per, r, out); break;
+    DN_FU_GRAM(1, k_fu_gram) DN_FU_GRAM(2, k_fu_gram) DN_FU_GRAM(3, k_fu_gram) DN_FU_GRAM(4, k_fu_gram)
+    DN_FU_GRAM(5, k_fu_gram_wide) DN_FU_GRAM(6, k_fu_gram_wide) DN_FU_GRAM(7, k_fu_gram_wide) DN_FU_GRAM(8, k_fu_gram_wide)
+#undef DN_FU_GRAM
+    default: DN_CHECK(false, "rank %d has no fused step", r);
+  }
   DN_LAUNCH_CHECK();
-  (of_h ? gh_state : gw_state) = SUMMED;
+  (of_h ? gh_state : gw_state) = PARTS;
   return 0;
 }
 

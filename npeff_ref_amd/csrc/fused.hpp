@@ -5,6 +5,8 @@
 #include "quotient.hpp"
 #include "split_bf16.hpp"
 
+#include <type_traits>
+
 namespace dn {
 
 constexpr int FUSED_MAX_RANK = 128;
@@ -40,7 +42,8 @@ struct fused_state {
 
   int create(const dnpeff_csr* S, int64_t n, int rank);
   void destroy();
-  int set_gram(const float* G, bool of_h);
+  // X^T X of a factor as it is ([rows, r]): partial matrices of H or of W
+  int gram_of(const float* X, int64_t rows, bool of_h);
   int product_n(const dnpeff_csr* S, const float* H);
   int sum_h();
   int sum_w();
@@ -172,6 +175,19 @@ __device__ inline void fu_cut_by(int a0, int a1, int share, float inv, int& k0, 
   };
   k0 = quot(a0) + 1;
   k1 = quot(a1 - 1) + 1;
+}
+
+// Block pairs of X^T X at 5 to 8 blocks, dealt to four waves: block rows W and 7 - W (where there is one) of
+// the upper triangle.  The most a wave has.
+__host__ __device__ constexpr int fuw_pairs(int nb) { return nb == 8 ? 9 : nb == 7 ? 7 : nb == 6 ? 6 : 5; }
+template <class F>
+__device__ inline void fuw_for_wave(int wave, F&& f) {
+  switch (wave) {
+    case 0: f(std::integral_constant<int, 0>{}); break;
+    case 1: f(std::integral_constant<int, 1>{}); break;
+    case 2: f(std::integral_constant<int, 2>{}); break;
+    default: f(std::integral_constant<int, 3>{}); break;
+  }
 }
 
 }  // namespace dn

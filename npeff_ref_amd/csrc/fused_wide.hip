@@ -10,8 +10,6 @@
 // X^T X, whose upper block pairs are dealt to the waves.
 #include "fused.hpp"
 
-#include <type_traits>
-
 namespace dn {
 
 // The lane, of which the compiler is not told that it stays the same: what is computed from it is computed
@@ -114,16 +112,6 @@ struct fuw_gram {
   }
 };
 
-template <class F>
-__device__ inline void fuw_for_wave(int wave, F&& f) {
-  switch (wave) {
-    case 0: f(std::integral_constant<int, 0>{}); break;
-    case 1: f(std::integral_constant<int, 1>{}); break;
-    case 2: f(std::integral_constant<int, 2>{}); break;
-    default: f(std::integral_constant<int, 3>{}); break;
-  }
-}
-
 // COLS: the H update (tiles of columns, A^T W gathered); else the W update (32 rows per workgroup, the
 // chunk sums of A H^T).  NB: blocks of 16 components.  Two barriers per tile: the Gram products of a
 // tile run between the second one and the next tile's first, beside the rows and the gathers of the next
@@ -135,7 +123,7 @@ __global__ void __launch_bounds__(256, 2) k_fuw(const fuw_args p) {
   constexpr int NS = fuw_steps(NB), PS = 32 * NS + 8, PLANE = FUW_COLS * PS, TS = 16 * NB + 4;
   constexpr bool SPLIT_J = NB <= 6;  // two waves per 16 rows, three blocks each; else two blocks, all rows
   constexpr int BPW = SPLIT_J ? 3 : 2, JPW = SPLIT_J ? 1 : 2;
-  constexpr int NA = NB == 8 ? 9 : NB == 7 ? 7 : NB == 6 ? 6 : 5;
+  constexpr int NA = fuw_pairs(NB);
   using Gather = fu_gather<FUW_COLS, TS, NB, 16, FUW_U>;
   constexpr int YP = fuw_y_plane(NB);
   constexpr int LDS_TILE = COLS ? 4 * (Gather::CARRY + 2048) : 0;
