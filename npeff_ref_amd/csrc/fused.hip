@@ -165,6 +165,18 @@ __device__ inline void fu_gram(const float* __restrict__ rows, int ts, f32x4 (&a
   }
 }
 
+// sum += acc, acc = 0
+template <int NP>
+__device__ inline void fu_gram_fold(double (&sum)[NP][4], f32x4 (&acc)[NP]) {
+#pragma unroll
+  for (int p = 0; p < NP; p++)
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      sum[p][i] += (double)acc[p][i];
+      acc[p][i] = 0.0f;
+    }
+}
+
 // The four waves' Gram blocks, added in wave order, to out ([pair][16][16]); lds: NP * 256 floats.
 template <int NP>
 __device__ inline void fu_gram_out(const f32x4 (&acc)[NP], float* __restrict__ lds, float* __restrict__ out) {
@@ -217,6 +229,11 @@ __global__ void __launch_bounds__(256, fu_blocks(Q, R) <= 2 ? 4 : 3)
   __shared__ int cps[2][TC + 1];
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int l16 = lane & 15, g = lane >> 4;
+  // Up to 32 components the Gram sums of a tile are added up in fp64: fp32 sums over all tiles of a workgroup
+  // lose what follows a column with large entries (W update at 2000 x 6.4 M, r = 16: error 3.3e-6, now 1e-7, in
+  // the same time).  Above, the registers hold the fp32 sums only.
+  constexpr bool TOTALS = NB <= 2;
+  double sum[TOTALS ? NP : 1][4] = {};
   f32x4 acc[NP];
 #pragma unroll
   for (int p = 0; p < NP; p++) acc[p] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
@@ -301,8 +318,15 @@ __global__ void __launch_bounds__(256, fu_blocks(Q, R) <= 2 ? 4 : 3)
       __builtin_amdgcn_wave_barrier();
       fu_gram<NB>(tile + first * TS, TS, acc);
     }
+    if constexpr (TOTALS) fu_gram_fold<NP>(sum, acc);
     td = nd;
     __syncthreads();  // (the tile has been read)
+  }
+  if constexpr (TOTALS) {
+#pragma unroll
+    for (int p = 0; p < NP; p++)
+#pragma unroll
+      for (int i = 0; i < 4; i++) acc[p][i] = (float)sum[p][i];
   }
   fu_gram_out<NP>(acc, tile, gpart + (int64_t)blockIdx.x * (NP * 256));
 }
@@ -380,17 +404,6 @@ __global__ void __launch_bounds__(256)
 // Up to 4 blocks of 16 components each wave takes every fourth 16 rows and all block pairs; the operands
 // need no LDS there: a lane's number of a row is one 4-byte load, 16 lanes a whole sector.  861,696 x 50 in
 // 80 us (708 with k_gram), 429,626 x 16 in 9 (36).
-template <int NB>
-__device__ inline void fu_gram_fold(double (&sum)[NB][4], f32x4 (&acc)[NB]) {
-#pragma unroll
-  for (int p = 0; p < NB; p++)
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-      sum[p][i] += (double)acc[p][i];
-      acc[p][i] = 0.0f;
-    }
-}
-
 template <int NB>
 __global__ void __launch_bounds__(256)
     k_fu_gram(const float* __restrict__ X, int64_t rows, int64_t per, int r, float* __restrict__ gpart) {
@@ -894,6 +907,10 @@ int fused_state::create(const dnpeff_csr* S, int64_t n, int rank) {
   }));
   const int64_t most = (int64_t)n_cus() * (per_cu > 0 ? per_cu : 1);
   h_wgs = (int)(f.n_tiles < most ? f.n_tiles : most);
+  // (above 32 the sums stay fp32 in registers: as many rounds of workgroups as keep them short.  3.4 M columns
+  // at r = 128: in one round of 512 workgroups H^T H costs the W update an error of 8.5e-7, in four 2.0e-7; the
+  // update takes 1.78 ms either way, the sum of the parts 28 against 8 us)
+  if (fu_blocks_of(r) > 2) h_wgs *= (int)ceil_div(f.n_tiles * f.tile_cols, (int64_t)h_wgs * FU_MOST_COLS);
   w_wgs = (int)ceil_div(n, r > FUSED_NARROW_RANK ? FUW_COLS : FU_ROWS_WG);
   DN_TRY(dmalloc(&gh_part, (int64_t)h_wgs * S_floats));
   DN_TRY(dmalloc(&gw_part, (int64_t)w_wgs * S_floats));

@@ -12,6 +12,9 @@ namespace dn {
 constexpr int FUSED_MAX_RANK = 128;
 constexpr int FUSED_NARROW_RANK = 64;  // above: fused_wide.hip
 constexpr int FUW_COLS = 32;           // columns (rows of W) per tile there
+// Columns whose X^T X a workgroup of the H update adds up in fp32 before it leaves the sum as a partial matrix
+// (those are summed in fp64): a column with large entries takes bits from all that is added after it.
+constexpr int FU_MOST_COLS = 2048;
 constexpr int64_t FU_CHUNKS = 4096;  // workgroups that A H^T is cut into where its rows allow
 
 bool fused_supported(int64_t n, int64_t m, int64_t nnz, int r);

@@ -73,3 +73,31 @@ def test_step_and_separate_kernels_in_turn(r, tune):
     _close(nmf, want)
     nmf.close()
     A.close()
+
+
+@pytest.mark.parametrize("r", [8, 16, 32, 66, 100])
+def test_gram_of_many_columns(r):
+    """H^T H as the H update leaves it, where a workgroup meets a column with large entries and then thousands
+    with small ones (in one fp32 sum each of those would cost half a unit in the last place of the large
+    one's square).  Seen in the loss's <W^T W, H^T H>."""
+    n, m = 128, 4_000_000
+    rng = np.random.default_rng(r)
+    rows = np.sort(rng.integers(0, n, m))
+    rp = np.concatenate([[0], np.cumsum(np.bincount(rows, minlength=n))]).astype(np.int64)
+    cols = rng.permutation(m).astype(np.int32)
+    vals = rng.random(m, dtype=np.float32) + np.float32(0.5)
+    vals[(cols < 65536) & (cols % 64 == 0)] *= np.float32(1000)
+    A = d.Csr.from_host(rp, cols, vals, m)
+    nmf = d.MuNmf(A, d.MuNmfParams(rank=r, max_iters=1, eps=EPS, seed=5, log_every=0))
+    nmf.initialize()
+    nmf.step(1)
+    _, pos, _ = nmf.loss_terms()
+    W, H = nmf.loadWToHostSync().astype(np.float64), nmf.loadHToHostSync()
+    G = np.zeros((r, r))
+    for c0 in range(0, m, 500_000):
+        part = H[:, c0:c0 + 500_000].astype(np.float64)
+        G += part @ part.T
+    want = float(((W.T @ W) * G).sum())
+    assert abs(pos - want) <= 2.4e-7 * want  # (four roundings to fp32)
+    nmf.close()
+    A.close()
