@@ -278,7 +278,7 @@ __global__ void __launch_bounds__(256, fu_blocks(Q, R) <= 2 ? 4 : 3)
       fu_load_row<Q, R>(Hb + hoff[jb], g, r, h[jb]);
     }
 
-    gather.run(pairs, td, Wb, tile);
+    gather.template run<0>(pairs, td, Wb, tile);
     request(nd);
     __syncthreads();
 
@@ -304,14 +304,28 @@ __global__ void __launch_bounds__(256, fu_blocks(Q, R) <= 2 ? 4 : 3)
       if (some) {
         int k0, k1;
         fu_cut_by(a0, a1, share, inv, k0, k1);
-        for (int k = k0; k < k1; k++) {
+        auto add = [&](int k, f32x4 (&to)[NB]) {
           const float* src = tile + Gather::CARRY + k * (2048 / Gather::NG);
 #pragma unroll
           for (int b = 0; b < NB; b++)
 #pragma unroll
             for (int i = 0; i < 4; i++) {
-              if (b < Q || i < R) t[b][i] += src[b < Q ? 16 * b + 4 * g + i : 16 * Q + R * g + i];
+              if (b < Q || i < R) to[b][i] += src[b < Q ? 16 * b + 4 * g + i : 16 * Q + R * g + i];
             }
+        };
+        if (NB > 2 || !__any(k1 - k0 > 16)) {
+          for (int k = k0; k < k1; k++) add(k, t);
+        } else {
+          // The parts of a long column eight at a time: one by one the sum rounds as often as it has parts
+          // (62 for 2000 rows at r = 16, where the update was off by 1.3e-7, now 9.8e-8).
+          for (int k = k0; k < k1;) {
+            f32x4 part[NB];
+#pragma unroll
+            for (int b = 0; b < NB; b++) part[b] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            for (const int k8 = k + 8; k < k1 && k < k8; k++) add(k, part);
+#pragma unroll
+            for (int b = 0; b < NB; b++) t[b] += part[b];
+          }
         }
       }
       fu_update<Q, R>(ga, h[jb], t, eps, r, mine[jb], Hb + hoff[jb], trow);
@@ -554,6 +568,10 @@ __global__ void __launch_bounds__(256)
     return;
   }
   constexpr int G = 64 / LPR;
+  // A lane group adds up 64 entries at a time and their sums in LDS: one sum over its share of a chunk, 1000
+  // entries of 32 M at r = 90, left the W update at 2000 x 0.5 M with an error of 1.0e-6 (now 2.5e-7; 117.4
+  // against 115.6 us at the size above).
+  __shared__ __align__(16) float totals[256][4];
   float* red = reinterpret_cast<float*>(red_d);  // [4][4 LPR]
   const int64_t chunk = blockIdx.x - sum_wgs;
   const int64_t e0 = chunks[chunk].e0;
@@ -576,7 +594,16 @@ __global__ void __launch_bounds__(256)
     int j, jn;
     float v, vn;
     request(w0, j, v);
+    int run = G;
+    bool more = false;
     for (int b = w0; b < w1; b += 64) {
+      if (run-- == 0) {
+        f32x4* t = reinterpret_cast<f32x4*>(totals[tid]);
+        *t = more ? *t + a : a;
+        a = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        more = true;
+        run = G - 1;
+      }
       request(b + 64, jn, vn);
       const int steps = ((w1 - b < 64 ? w1 - b : 64) + G - 1) / G;
       constexpr int U = 64 / G < FU_U ? 64 / G : FU_U;
@@ -598,6 +625,7 @@ __global__ void __launch_bounds__(256)
       j = jn;
       v = vn;
     }
+    if (more) a += *reinterpret_cast<f32x4*>(totals[tid]);
   }
 #pragma unroll
   for (int off = 32; off >= LPR; off >>= 1)
@@ -910,7 +938,10 @@ int fused_state::create(const dnpeff_csr* S, int64_t n, int rank) {
   // (above 32 the sums stay fp32 in registers: as many rounds of workgroups as keep them short.  3.4 M columns
   // at r = 128: in one round of 512 workgroups H^T H costs the W update an error of 8.5e-7, in four 2.0e-7; the
   // update takes 1.78 ms either way, the sum of the parts 28 against 8 us)
-  if (fu_blocks_of(r) > 2) h_wgs *= (int)ceil_div(f.n_tiles * f.tile_cols, (int64_t)h_wgs * FU_MOST_COLS);
+  if (fu_blocks_of(r) > 2) {
+    const int64_t per_wg = ceil_div(f.n_tiles * f.tile_cols, h_wgs);
+    h_wgs *= (int)std::max<int64_t>(ceil_div(per_wg, FU_MOST_COLS), r > FUSED_NARROW_RANK && per_wg > FU_MOST_COLS / 2 ? 2 : 1);
+  }
   w_wgs = (int)ceil_div(n, r > FUSED_NARROW_RANK ? FUW_COLS : FU_ROWS_WG);
   DN_TRY(dmalloc(&gh_part, (int64_t)h_wgs * S_floats));
   DN_TRY(dmalloc(&gw_part, (int64_t)w_wgs * S_floats));

@@ -13,7 +13,8 @@ constexpr int FUSED_MAX_RANK = 128;
 constexpr int FUSED_NARROW_RANK = 64;  // above: fused_wide.hip
 constexpr int FUW_COLS = 32;           // columns (rows of W) per tile there
 // Columns whose X^T X a workgroup of the H update adds up in fp32 before it leaves the sum as a partial matrix
-// (those are summed in fp64): a column with large entries takes bits from all that is added after it.
+// (those are summed in fp64): a column with large entries takes bits from all that is added after it.  Above
+// 64 components half of them where that takes no more than two rounds of workgroups.
 constexpr int FU_MOST_COLS = 2048;
 constexpr int64_t FU_CHUNKS = 4096;  // workgroups that A H^T is cut into where its rows allow
 
@@ -117,8 +118,9 @@ struct fu_gather {
       pr[u] = pp[e < end ? e : end];
     }
   }
-  __device__ inline void run(const uint2* pairs, const fu_tile_at& d, const char* Wb,
-                             float* tile) {
+  // RUN > 0: no more than RUN entries are added up one after the other before their sum joins the column's.
+  template <int RUN>
+  __device__ inline void run(const uint2* pairs, const fu_tile_at& d, const char* Wb, float* tile) {
     const int s0 = grp * d.share, s1 = s0 + d.share < d.E ? s0 + d.share : d.E;
     if (s0 >= s1) return;
     const uint2* pp = pairs + d.e0;
@@ -127,12 +129,26 @@ struct fu_gather {
                                                              : (int)((cur >> FU_ROW_BITS) & (TC - 1)) * TS;
     dst += 4 * sub;
     f32x4 a0 = f32x4{0.0f, 0.0f, 0.0f, 0.0f}, a1 = a0;
+    bool more = false;  // (RUN > 0) dst holds a sum of the column's entries before these
     auto put = [&]() {
+      if constexpr (RUN > 0) {
+        if (more) {
+          a0 += *reinterpret_cast<f32x4*>(tile + dst);
+          if (WHOLE || 4 * (sub + LPR) < 16 * NB) a1 += *reinterpret_cast<f32x4*>(tile + dst + 4 * LPR);
+        }
+      }
       *reinterpret_cast<f32x4*>(tile + dst) = a0;
       if (WHOLE || 4 * (sub + LPR) < 16 * NB) *reinterpret_cast<f32x4*>(tile + dst + 4 * LPR) = a1;
     };
 #pragma unroll 1
     for (int b = s0; b < s1; b += U) {
+      if constexpr (RUN > 0) {
+        if (b > s0 && (b - s0) % RUN == 0) {
+          put();
+          more = true;
+          a0 = a1 = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        }
+      }
       f32x4 w0[U], w1[U];
 #pragma unroll
       for (int u = 0; u < U; u++) {
@@ -151,6 +167,7 @@ struct fu_gather {
         const float v = b + u < s1 ? __uint_as_float(pr[u].y) : 0.0f;
         if (((pr[u].x ^ cur) >> FU_ROW_BITS) != 0) {
           put();
+          more = false;
           cur = pr[u].x;
           dst = (int)((cur >> FU_ROW_BITS) & (TC - 1)) * TS + 4 * sub;
           a0 = a1 = f32x4{0.0f, 0.0f, 0.0f, 0.0f};

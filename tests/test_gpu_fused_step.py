@@ -101,3 +101,49 @@ def test_gram_of_many_columns(r):
     assert abs(pos - want) <= 2.4e-7 * want  # (four roundings to fp32)
     nmf.close()
     A.close()
+
+
+@pytest.mark.parametrize("r", [8, 16, 72])
+def test_long_columns(r):
+    """A^T W of columns that 40,000 rows hold: neither a lane group's entries nor the parts of its 15 to 127
+    neighbours are all added up one by one.  (Sums, quotient and product with H round some ten times, with
+    either sign: about three of 2^-24.)"""
+    n, m, full = 40_000, 66_000, 6
+    rng = np.random.default_rng(r)
+    rows = np.concatenate([np.repeat(np.arange(n), full), rng.integers(0, n, m - full)])
+    cols = np.concatenate([np.tile(np.arange(full), n), np.arange(full, m)]).astype(np.int32)
+    order = np.argsort(rows, kind="stable")
+    rows, cols = rows[order], cols[order]
+    vals = rng.random(len(rows), dtype=np.float32) + np.float32(0.5)
+    rp = np.concatenate([[0], np.cumsum(np.bincount(rows, minlength=n))]).astype(np.int64)
+    A = d.Csr.from_host(rp, cols, vals, m)
+    nmf = d.MuNmf(A, d.MuNmfParams(rank=r, max_iters=1, eps=EPS, seed=5, log_every=0))
+    nmf.initialize()
+    W, H = nmf.loadWToHostSync().astype(np.float64), nmf.loadHToHostSync()[:, :full].astype(np.float64)
+    T = np.stack([W.T @ np.bincount(rows[cols == j], weights=vals[cols == j], minlength=n) for j in range(full)], axis=1)
+    want = H * T / (W.T @ W @ H + EPS)
+    nmf.update_H()
+    err = np.linalg.norm(nmf.loadHToHostSync()[:, :full] - want) / np.linalg.norm(want)
+    assert err <= 1.7e-7
+    nmf.close()
+    A.close()
+
+
+def test_long_rows():
+    """A H^T of rows whose large entries come first: those that follow in the same chunk join them in sums.  (Up
+    to 24 roundings per chunk at the large entries' size, with either sign: about six of 2^-24.)"""
+    n, m, r = 80, 300_000, 72
+    rng = np.random.default_rng(r)
+    vals = rng.random((n, m), dtype=np.float32) + np.float32(0.5)
+    vals[:, :16] *= np.float32(700)
+    A = d.Csr.from_host(np.arange(n + 1, dtype=np.int64) * m, np.tile(np.arange(m, dtype=np.int32), n), vals.reshape(-1), m)
+    nmf = d.MuNmf(A, d.MuNmfParams(rank=r, max_iters=1, eps=EPS, seed=5, log_every=0))
+    nmf.initialize()
+    nmf.step(1)
+    W, H = nmf.loadWToHostSync().astype(np.float64), nmf.loadHToHostSync().astype(np.float64)
+    want = W * (vals.astype(np.float64) @ H.T) / (W @ (H @ H.T) + EPS)
+    nmf.update_W()
+    err = np.linalg.norm(nmf.loadWToHostSync() - want) / np.linalg.norm(want)
+    assert err <= 4e-7
+    nmf.close()
+    A.close()
