@@ -584,12 +584,12 @@ __global__ void __launch_bounds__(256)
   const float* va = vals + e0;
   f32x4 a = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
   // 64 (column, value) pairs at a time, one per lane, the next 64 on their way; the steps take theirs by
-  // shuffles.  Lanes past the end hold (some column, 0).
+  // shuffles.  Lanes past the end hold some column and are not counted in.
   if (w0 < w1) {
     auto request = [&](int e, int& jj, float& vv) {
       const int at = e + lane < w1 ? e + lane : w1 - 1;
       jj = ci[at];
-      vv = e + lane < w1 ? va[at] : 0.0f;
+      vv = va[at];
     };
     int j, jn;
     float v, vn;
@@ -605,7 +605,7 @@ __global__ void __launch_bounds__(256)
         run = G - 1;
       }
       request(b + 64, jn, vn);
-      const int steps = ((w1 - b < 64 ? w1 - b : 64) + G - 1) / G;
+      const int cnt = w1 - b < 64 ? w1 - b : 64, steps = (cnt + G - 1) / G;
       constexpr int U = 64 / G < FU_U ? 64 / G : FU_U;
       for (int st = 0; st < steps; st += U) {
         f32x4 x[U];
@@ -618,9 +618,11 @@ __global__ void __launch_bounds__(256)
           x[u] = *reinterpret_cast<const f32x4u*>(Hl + row * r);
         }
 #pragma unroll
-        for (int u = 0; u < U; u++)
+        for (int u = 0; u < U; u++) {
+          if ((st + u) * G + grp >= cnt) continue;  // (0 times an infinite entry is no 0)
 #pragma unroll
           for (int i = 0; i < 4; i++) a[i] = fmaf(w[u], x[u][i], a[i]);
+        }
       }
       j = jn;
       v = vn;

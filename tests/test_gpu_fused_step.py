@@ -147,3 +147,20 @@ def test_long_rows():
     assert err <= 4e-7
     nmf.close()
     A.close()
+
+
+@pytest.mark.parametrize("r", [7, 16, 30, 64, 100])
+def test_infinite_entry_stays_infinite(r):
+    """<A H^T, W> with an infinite entry of H at the end of a row: infinite, with any number of lanes idle."""
+    n, m = 130, 400
+    for length in (1, 2, 3, 5, 33, 63, 64, 65, 130, 257):
+        rp = np.arange(n + 1, dtype=np.int64) * length
+        cols = np.tile(np.concatenate([np.arange(length - 1), [m - 1]]), n).astype(np.int32)
+        A = d.Csr.from_host(rp, cols, np.ones(n * length, dtype=np.float32), m)
+        nmf = d.MuNmf(A, d.MuNmfParams(rank=r, max_iters=1, eps=EPS, seed=5, log_every=0))
+        W, H = np.ones((n, r), dtype=np.float32), np.ones((r, m), dtype=np.float32)
+        H[0, m - 1] = np.inf
+        nmf.set_factors(W, H)
+        assert nmf.loss_terms()[2] == np.inf
+        nmf.close()
+        A.close()
