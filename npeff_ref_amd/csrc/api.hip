@@ -128,6 +128,15 @@ struct dnpeff_nmf {
   bool w_out = false, h_out = false;
 };
 
+// Rows that one fp32 sum may take in at padded ranks, in X^T X and in the dense head's A^T W.  As they are, those
+// ranks sum over a 2048th part of the rows, or 500 of them: left to fill the chip alone, the tiles would sum over
+// many times that.  Errors against 64 bits of one update, as they are / padded / padded with these bounds: W at
+// 2000 x 3.9 M, r = 385 4.3e-6 / 1.0e-5 / 4.7e-7, H at 2000 x 0.4 M, r = 150 2.5e-7 / 4.5e-7 / 2.2e-7.  Ten
+// iterations take 247 against 239 ms there, 28.6 against 28.4, 66.6 against 64.3 at 700 x 1.0 M, r = 500.
+constexpr int64_t PADDED_GRAM_RUN = 1024, PADDED_HEAD_RUN = 512;
+static int64_t gram_run(const dnpeff_nmf* h) { return h->r != h->rl ? PADDED_GRAM_RUN : 0; }
+static int64_t head_run(int rank, int asked) { return rank != asked ? PADDED_HEAD_RUN : HEAD_RUN; }
+
 // At the start of every call that uses the factors: those whose pointers are out are what the caller
 // has left there (packed copies are copied back), and what is kept of them is forgotten.
 static int take_back(dnpeff_nmf* h) {
@@ -190,9 +199,9 @@ static int64_t tile_cols_for(int64_t m, int rank) {
 }
 
 // Bytes of device memory that the handle allocates besides the structures of the matrix.
-static double factor_bytes(int64_t n, int64_t m, int rank, bool tiled) {
+static double factor_bytes(int64_t n, int64_t m, int rank, bool tiled, int64_t run) {
   const double nr = 4.0 * (double)n * rank, mr = 4.0 * (double)m * rank;
-  double ws = (double)gram_workspace_floats(m, rank), ws_n = (double)gram_workspace_floats(n, rank);
+  double ws = (double)gram_workspace_floats(m, rank, run), ws_n = (double)gram_workspace_floats(n, rank, run);
   if (ws_n > ws) ws = ws_n;
   const double tile = 4.0 * (double)tile_cols_for(m, rank) * rank;
   return 3.0 * nr + (tiled ? mr + 2.0 * tile : 2.0 * mr) + 4.0 * ws + 3.0 * 4.0 * rank * rank +
@@ -211,10 +220,11 @@ struct plan_table {
   double total() const { return factors + partials + segments + offsets + reserve; }
 };
 
-static plan_table plan_overheads(int64_t n, int64_t m, int64_t nnz_sparse, int rank, bool tiled, bool sweeps,
+// rank: as stored, asked: the caller's.
+static plan_table plan_overheads(int64_t n, int64_t m, int64_t nnz_sparse, int rank, int asked, bool tiled, bool sweeps,
                                  double total_bytes) {
   plan_table t;
-  t.factors = factor_bytes(n, m, rank, tiled);
+  t.factors = factor_bytes(n, m, rank, tiled, rank != asked ? PADDED_GRAM_RUN : 0);
   const int64_t P = coarse_panels_for(n, m, rank, sweeps);
   const double by_chunks = 4.0 * rank * ((double)nnz_sparse / (double)SPMM_N_CHUNK + (double)n);
   const double by_panels = P > 0 ? 4.0 * rank * (double)n * (double)(P + SWEEP_XCDS) : 0.0;
@@ -237,13 +247,13 @@ DN_API int dnpeff_plan_estimate(int64_t n_rows, int64_t n_cols, int64_t nnz_spar
   DN_CHECK(n_rows >= 0 && n_cols >= 0 && nnz_sparse >= 0 && n_dense >= 0 && n_dense <= n_cols,
            "negative size");
   DN_CHECK(rank >= 1 && rank <= 1024, "rank %d outside [1, 1024]", rank);
-  const plan_table t = plan_overheads(n_rows, n_cols, nnz_sparse, rank, tiled != 0, sweeps != 0, (double)total_bytes);
+  const plan_table t = plan_overheads(n_rows, n_cols, nnz_sparse, rank, rank, tiled != 0, sweeps != 0, (double)total_bytes);
   out[0] = t.factors; out[1] = t.partials; out[2] = t.segments; out[3] = t.offsets; out[4] = t.reserve;
   out[5] = 16.0 * (double)nnz_sparse;
   out[6] = n_dense ? 4.0 * head_blocks_for_rank(rank) * (double)(ceil_div(n_rows, 128) * 128) *
                          (double)(ceil_div(n_dense, 128) * 128)
                    : 0.0;
-  out[7] = 4.0 * (double)head_workspace_floats(n_rows, n_dense, rank);
+  out[7] = 4.0 * (double)head_workspace_floats(n_rows, n_dense, rank, HEAD_RUN);
   return 0;
 }
 
@@ -255,7 +265,7 @@ DN_API int dnpeff_plan_estimate(int64_t n_rows, int64_t n_cols, int64_t nnz_spar
 // receives whether the H update must run on column tiles for everything to fit.
 // *fused: whether the step of small ranks can run (it reads the whole matrix from its own lists: no
 // dense head is split off then).
-static int plan_matrix(dnpeff_csr* A, int rank, bool consume, bool* tiled, bool* fused) {
+static int plan_matrix(dnpeff_csr* A, int rank, int asked, bool consume, bool* tiled, bool* fused) {
   const tuning_t& tn = tuning();
   size_t free_b = 0, total_b = 0;
   DN_HIP(hipMemGetInfo(&free_b, &total_b));
@@ -271,8 +281,8 @@ static int plan_matrix(dnpeff_csr* A, int rank, bool consume, bool* tiled, bool*
   if (S0->colptr) avail += 8.0 * (double)S0->nnz;
   if (S0->pcol || S0->nl.pairs) avail += 8.0 * (double)S0->nnz;
   const bool sweeps = sweeps_for_rank(rank);
-  const plan_table t_full = plan_overheads(A->n_rows, A->n_cols, A->nnz, rank, false, sweeps, (double)total_b);
-  const plan_table t_tiled = plan_overheads(A->n_rows, A->n_cols, A->nnz, rank, true, sweeps, (double)total_b);
+  const plan_table t_full = plan_overheads(A->n_rows, A->n_cols, A->nnz, rank, asked, false, sweeps, (double)total_b);
+  const plan_table t_tiled = plan_overheads(A->n_rows, A->n_cols, A->nnz, rank, asked, true, sweeps, (double)total_b);
   const double budget_full = avail - t_full.total();
   const double budget_tiled = avail - t_tiled.total();
   // (multiples of 64 with rows enough for a dense head keep it: its kernels are made for those ranks)
@@ -286,7 +296,7 @@ static int plan_matrix(dnpeff_csr* A, int rank, bool consume, bool* tiled, bool*
   if (A->tail) {
     if (rank % 4 == 0) {  // split by the caller (or an earlier handle): keep it
       const double foot = 4.0 * head_blocks_for_rank(rank) * (double)A->head.n_pad * (double)A->head.n_d_pad +
-                          16.0 * (double)S0->nnz + 4.0 * (double)head_workspace_floats(A->n_rows, A->head.n_d, rank);
+                          16.0 * (double)S0->nnz + 4.0 * (double)head_workspace_floats(A->n_rows, A->head.n_d, rank, head_run(rank, asked));
       if (tn.tiled_h < 0.0) *tiled = foot > budget_full;
       return 0;
     }
@@ -300,10 +310,10 @@ static int plan_matrix(dnpeff_csr* A, int rank, bool consume, bool* tiled, bool*
   }
   head_choice c;
   const int n_blocks = head_blocks_for_rank(rank);
-  DN_TRY(choose_dense_head(A, fill, *tiled ? budget_tiled : budget_full, n_blocks, rank, &c));
+  DN_TRY(choose_dense_head(A, fill, *tiled ? budget_tiled : budget_full, n_blocks, rank, head_run(rank, asked), &c));
   if (!c.fits && tn.tiled_h < 0.0 && !*tiled) {
     *tiled = true;
-    DN_TRY(choose_dense_head(A, fill, budget_tiled, n_blocks, rank, &c));
+    DN_TRY(choose_dense_head(A, fill, budget_tiled, n_blocks, rank, head_run(rank, asked), &c));
   }
   if (tn.verbose != 0.0) {
     const plan_table& t = *tiled ? t_tiled : t_full;
@@ -333,7 +343,7 @@ static int padded_rank(const dnpeff_csr* A, int rank, float eps, int* out) {
     return 0;
   size_t free_b = 0, total_b = 0;
   DN_HIP(hipMemGetInfo(&free_b, &total_b));
-  const plan_table t = plan_overheads(A->n_rows, A->n_cols, A->nnz, p, false, sweeps_for_rank(p), (double)total_b);
+  const plan_table t = plan_overheads(A->n_rows, A->n_cols, A->nnz, p, rank, false, sweeps_for_rank(p), (double)total_b);
   if (t.total() + 4.0 * (double)rank * (double)(A->n_rows + A->n_cols) + 24.0 * (double)A->nnz <
       (double)free_b + (double)pool_cached_bytes())
     *out = p;
@@ -367,10 +377,10 @@ static int nmf_create_impl(dnpeff_csr* A, int rank, float eps, int64_t seed, uns
   const int rank_asked = rank;
   DN_TRY(padded_rank(A, rank_asked, eps, &rank));
   bool tiled = false, fused = false;
-  DN_TRY(plan_matrix(A, rank, consume, &tiled, &fused));
+  DN_TRY(plan_matrix(A, rank, rank_asked, consume, &tiled, &fused));
   if (tiled && rank != rank_asked) {  // (only where the two estimates of the memory disagree)
     rank = rank_asked;
-    DN_TRY(plan_matrix(A, rank, consume, &tiled, &fused));
+    DN_TRY(plan_matrix(A, rank, rank_asked, consume, &tiled, &fused));
   }
   mark("memory plan, dense head and sparse tail");
   if (consume && A->tail) {  // the tail and the head hold everything the products read
@@ -378,6 +388,7 @@ static int nmf_create_impl(dnpeff_csr* A, int rank, float eps, int64_t seed, uns
     dfree(A->colind); A->colind = nullptr;
     dfree(A->vals); A->vals = nullptr;
   }
+  A->head.t_run = head_run(rank, rank_asked);
   DN_TRY(csr_ensure_products(A, rank));
   mark("transposed copy, panels, pieces, work lists");
   if (consume) DN_TRY(csr_consume_for_products(A));
@@ -392,8 +403,8 @@ static int nmf_create_impl(dnpeff_csr* A, int rank, float eps, int64_t seed, uns
   const int64_t nr = n_there * rank, mr = m_there * rank;
   const int64_t h_floats = h->tiled ? (m_there + h->tile_cols) * rank : mr;
   const int64_t s_floats = h->tiled ? h->tile_cols * rank : mr;
-  int64_t ws = gram_workspace_floats(h->m, rank);
-  int64_t ws_n = gram_workspace_floats(h->n, rank);
+  int64_t ws = gram_workspace_floats(h->m, rank, gram_run(h));
+  int64_t ws_n = gram_workspace_floats(h->n, rank, gram_run(h));
   if (ws_n > ws) ws = ws_n;
   // (four spare floats: the step of small ranks reads rows in 16-byte pieces)
   int s = dmalloc(&h->W, nr + 4) || dmalloc(&h->W2, nr + 4) || dmalloc(&h->Nw, nr + 4) ||
@@ -495,6 +506,7 @@ DN_API int dnpeff_nmf_set_factors(dnpeff_nmf* nmf, const float* W_nr, const floa
 // The matrix may have been planned again for another rank since this handle was made (a second
 // handle, a single-kernel call): make its work lists and workspaces fit this rank again.
 static int products_for(dnpeff_nmf* h) {
+  h->A->head.t_run = head_run(h->r, h->rl);
   DN_TRY(csr_ensure_products(h->A, h->r));
   if (h->tiled) DN_TRY(csr_tile_lists(h->A));
   return 0;
@@ -552,7 +564,7 @@ DN_API int dnpeff_nmf_update_W(dnpeff_nmf* h) {
     } g;
     DN_TRY(side_stream_begin());
     int st = h->prof.begin(DNPEFF_K_GRAM_H);
-    if (!st) st = launch_gram(h->m, h->r, h->H, h->G, h->gram_ws);
+    if (!st) st = launch_gram(h->m, h->r, h->H, h->G, h->gram_ws, gram_run(h));
     if (!st) st = h->prof.next(DNPEFF_K_SPMM_N);
     DN_TRY(side_stream_end());
     DN_TRY(st);
@@ -584,7 +596,7 @@ DN_API int dnpeff_nmf_update_W(dnpeff_nmf* h) {
     Gh = h->G;
   } else if (!h->gh_valid) {
     DN_TRY(h->prof.begin(DNPEFF_K_GRAM_H));
-    DN_TRY(launch_gram(h->m, h->r, h->H, h->G, h->gram_ws));
+    DN_TRY(launch_gram(h->m, h->r, h->H, h->G, h->gram_ws, gram_run(h)));
     DN_TRY(h->prof.end());
     Gh = h->G;
   }
@@ -693,7 +705,7 @@ DN_API int dnpeff_nmf_update_H(dnpeff_nmf* h) {
   dnpeff_csr* A = h->A;
   DN_TRY(products_for(h));
   DN_TRY(h->prof.begin(DNPEFF_K_GRAM_W));
-  DN_TRY(launch_gram(h->n, h->r, h->W, h->G, h->gram_ws));
+  DN_TRY(launch_gram(h->n, h->r, h->W, h->G, h->gram_ws, gram_run(h)));
   DN_TRY(h->prof.end());
   h->nw_valid = false;
   if (h->tiled) return update_H_tiled(h);
@@ -756,8 +768,8 @@ DN_API int dnpeff_nmf_loss_terms(dnpeff_nmf* h, double* sq_norm_A, double* pos, 
   if (h->GH && h->gh_valid)
     Gh = h->GH;
   else
-    DN_TRY(launch_gram(h->m, h->r, h->H, h->G, h->gram_ws));
-  DN_TRY(launch_gram(h->n, h->r, h->W, h->G2, h->gram_ws));
+    DN_TRY(launch_gram(h->m, h->r, h->H, h->G, h->gram_ws, gram_run(h)));
+  DN_TRY(launch_gram(h->n, h->r, h->W, h->G2, h->gram_ws, gram_run(h)));
   DN_TRY(launch_dot((int64_t)h->r * h->r, Gh, h->G2, h->dot_ws, h->dot_ws + DOT_BLOCKS + 1));
   double res[2];
   DN_HIP(hipStreamSynchronize(stream()));

@@ -75,9 +75,9 @@ static bool gram_uses_tiles(int64_t rows, int r) { return r > 128 && r % 128 == 
 
 static int64_t gram_small_wgs(int64_t rows);
 
-int64_t gram_workspace_floats(int64_t rows, int r) {
+int64_t gram_workspace_floats(int64_t rows, int r, int64_t run) {
   if (r <= 32) return gram_small_wgs(rows) * 1024;  // one 32 x 32 block per workgroup of k_gram_small
-  if (gram_uses_tiles(rows, r)) return gram_tiles_workspace_floats(rows, r);
+  if (gram_uses_tiles(rows, r)) return gram_tiles_workspace_floats(rows, r, run);
   return gram_slices(rows) * (int64_t)gram_pairs(r) * 1024;
 }
 
@@ -451,7 +451,7 @@ __global__ void __launch_bounds__(256)
   }
 }
 
-int launch_gram(int64_t rows, int r, const float* X, float* G, float* workspace) {
+int launch_gram(int64_t rows, int r, const float* X, float* G, float* workspace, int64_t run) {
   DN_CHECK(r >= 1 && r <= 1024, "rank %d outside [1, 1024]", r);
   if (r <= 32 && rows >= 1) {
     const int64_t wgs = gram_small_wgs(rows);
@@ -462,7 +462,7 @@ int launch_gram(int64_t rows, int r, const float* X, float* G, float* workspace)
     return 0;
   }
   if (gram_uses_tiles(rows, r) && ((uintptr_t)X % 16) == 0)
-    return launch_gram_tiles(rows, r, X, G, workspace);
+    return launch_gram_tiles(rows, r, X, G, workspace, run);
   const int n_pairs = gram_pairs(r);
   const int n_tiles = (r + 127) / 128;
   int64_t slices = gram_slices(rows);

@@ -134,12 +134,13 @@ int scan_long_cols(const int64_t* colptr, int64_t limit, int64_t n, int32_t* out
 
 // ---- dense kernels (dense.hip) ----
 int launch_mu(int64_t count, float* F, const float* num, const float* den, float eps);
-// Needs a workspace of gram_workspace_floats(rows, r) floats.
-int64_t gram_workspace_floats(int64_t rows, int r);
-int launch_gram(int64_t rows, int r, const float* X, float* G, float* workspace);
+// Needs a workspace of gram_workspace_floats(rows, r, run) floats.  run > 0: at ranks that go by tiles no fp32
+// sum runs over more than that many rows (and no more than 1/2048 of all; 0: as the launch fills the chip).
+int64_t gram_workspace_floats(int64_t rows, int r, int64_t run = 0);
+int launch_gram(int64_t rows, int r, const float* X, float* G, float* workspace, int64_t run = 0);
 // ranks 256, 384, ..., 1024 (head.hip)
-int64_t gram_tiles_workspace_floats(int64_t rows, int r);
-int launch_gram_tiles(int64_t rows, int r, const float* X, float* G, float* workspace);
+int64_t gram_tiles_workspace_floats(int64_t rows, int r, int64_t run);
+int launch_gram_tiles(int64_t rows, int r, const float* X, float* G, float* workspace, int64_t run);
 // Between the two, launch_xg_mu calls with this G reuse one transposed copy of it (the caller
 // must not change G in between).
 int xg_mu_hold_g(const float* G, int r);
@@ -227,8 +228,12 @@ tuning_t& tuning();
 // split in three (split_bf16.hpp) unless the split_bf16 switch selects the fp32 matrix cores.
 inline bool use_split_bf16() { return tuning().split_bf16 != 0.0; }
 
+// Products that one fp32 running sum of the head's products may hold (the slices are added in fp64).
+constexpr int64_t HEAD_RUN = 8192;
+
 // Columns present in many rows, held as a dense block in both orientations (head.hip).
 struct dense_head {
+  int64_t t_run = HEAD_RUN;  // the same for A^T W at the rank the products are planned for
   int64_t n_d = 0;      // columns in the head
   int64_t n_d_pad = 0;  // n_d rounded up to 128
   int64_t n_pad = 0;    // rows rounded up to 128
@@ -445,8 +450,8 @@ struct head_choice {
 };
 constexpr double NO_BUDGET = 1e300;
 // rank > 0: the footprint also counts the head's workspace at that rank
-int choose_dense_head(dnpeff_csr* A, double min_fill, double budget, int n_blocks, int rank, head_choice* out);
-int64_t head_workspace_floats(int64_t n_rows, int64_t n_d, int r);
+int choose_dense_head(dnpeff_csr* A, double min_fill, double budget, int n_blocks, int rank, int64_t t_run, head_choice* out);
+int64_t head_workspace_floats(int64_t n_rows, int64_t n_d, int r, int64_t t_run);
 // Sizes that the memory plan shares with the code that allocates (loader.hip).
 constexpr double PANEL_PARTIALS_BYTES = 3.0e9;  // the plain panels' partial sums stay within this
 int64_t coarse_panels_for(int64_t n_rows, int64_t n_cols, int r, bool sweeps);

@@ -343,28 +343,33 @@ static int64_t gram_tiles_slices(int64_t rows, int r) {
 // paired: the diagonal tiles go two and two as squares of 256 columns (one workgroup of eight
 // waves per CU), and the other launch takes the tile pairs that lie outside those squares.
 static bool gram_paired(int r) { return tuning().gram_fold >= 2 && r % 256 == 0; }
-static void gram_b16_slices(int64_t rows, int r, int64_t* s_diag, int64_t* s_off, bool paired = false) {
+static void gram_b16_slices(int64_t rows, int r, int64_t run, int64_t* s_diag, int64_t* s_off, bool paired = false) {
   const int64_t t = r / 128, slots = 2 * (int64_t)n_cus(), k_tiles = rows / 32;
   const int64_t n_off = t * (t - 1) / 2 - (paired ? t / 2 : 0);
   int64_t d = slots / t, o = n_off > 0 ? slots / n_off : 0;  // (paired: t / 2 squares, one slot per CU)
   if (d < 1) d = 1;
   if (n_off > 0 && o < 1) o = 1;
+  if (run > 0) {
+    const int64_t by_run = std::min<int64_t>(2048, ceil_div(rows, run));
+    d = std::max(d, by_run);
+    o = std::max(o, by_run);
+  }
   if (d > k_tiles) d = k_tiles;
   if (o > k_tiles) o = k_tiles;
   *s_diag = d < 1 ? 1 : d;
   *s_off = n_off > 0 ? (o < 1 ? 1 : o) : 0;
 }
 
-static int64_t gram_tiles_sums_at(int64_t rows, int r) {
+static int64_t gram_tiles_sums_at(int64_t rows, int r, int64_t run) {
   int64_t d, o, dp, op;
-  gram_b16_slices(rows, r, &d, &o);
-  gram_b16_slices(rows, r, &dp, &op, true);
+  gram_b16_slices(rows, r, run, &d, &o);
+  gram_b16_slices(rows, r, run, &dp, &op, true);
   const int64_t s = std::max(std::max(gram_tiles_slices(rows, r), std::max(d, o)), std::max(dp, op));
   return (s + 1) * (int64_t)r * r;
 }
 
-int64_t gram_tiles_workspace_floats(int64_t rows, int r) {
-  return gram_tiles_sums_at(rows, r) + 2 * (int64_t)r * r;
+int64_t gram_tiles_workspace_floats(int64_t rows, int r, int64_t run) {
+  return gram_tiles_sums_at(rows, r, run) + 2 * (int64_t)r * r;
 }
 
 // Slice sums: diagonal tiles hold s_diag slices, the others s_off, and slice number `extra` (if >= 0)
@@ -574,7 +579,7 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
   store(wave, (wave + 4) & 7, acc[5]);
 }
 
-int launch_gram_tiles(int64_t rows, int r, const float* X, float* G, float* workspace) {
+int launch_gram_tiles(int64_t rows, int r, const float* X, float* G, float* workspace, int64_t run) {
   const int t = r / 128;
   int64_t s_diag, s_off, extra = -1;
   int folded = 0;
@@ -595,7 +600,7 @@ int launch_gram_tiles(int64_t rows, int r, const float* X, float* G, float* work
     // more slice through the fp32 kernel
     const int64_t k_tiles = rows / ABT_KB, whole = k_tiles * ABT_KB;
     const bool paired = gram_paired(r);
-    gram_b16_slices(rows, r, &s_diag, &s_off, paired);
+    gram_b16_slices(rows, r, run, &s_diag, &s_off, paired);
     folded = paired ? 2 : tuning().gram_fold != 0 ? 1 : 0;
     const int n_off = t * (t - 1) / 2 - (paired ? t / 2 : 0);
     if (paired)
@@ -620,7 +625,7 @@ int launch_gram_tiles(int64_t rows, int r, const float* X, float* G, float* work
     s_diag = s_off = gram_tiles_slices(rows, r);
     DN_TRY(launch_ptq(X, r, rows, X, r, r, r, s_diag, workspace, t));
   }
-  double* sums = reinterpret_cast<double*>(workspace + gram_tiles_sums_at(rows, r));
+  double* sums = reinterpret_cast<double*>(workspace + gram_tiles_sums_at(rows, r, run));
   const dim3 blocks((unsigned)(r / 32), (unsigned)r);
   hipLaunchKernelGGL(k_gram_tiles_sum, blocks, dim3(256), 0, stream(), workspace, s_diag, s_off, r, folded, sums);
   hipLaunchKernelGGL(k_gram_tiles_fold, dim3((unsigned)(r / 32), (unsigned)(r / 32)), dim3(256), 0, stream(), sums,
@@ -707,27 +712,28 @@ static int64_t head_gather_floats(const dense_head& h, int r) {
 }
 
 // Slices of the contraction: enough workgroups to fill the chip, and no fp32 running sum longer
-// than 8192 products (the slices are added in fp64).
-static int64_t head_slices_for(int64_t tiles_mn, int64_t K) {
+// than `run` products (the slices are added in fp64).
+static int64_t head_slices_for(int64_t tiles_mn, int64_t K, int64_t run) {
   const int64_t k_tiles = ceil_div(K, PTQ_KB);
   int64_t s = ptq_slices(tiles_mn, k_tiles);
-  const int64_t by_length = ceil_div(K, 8192);
+  const int64_t by_length = ceil_div(K, run);
   if (s < by_length) s = by_length;
   return s < k_tiles ? s : (k_tiles > 0 ? k_tiles : 1);
 }
 static int64_t head_slices_n(const dense_head& h, int r) {
-  return head_slices_for((h.n_pad / 128) * ceil_div(r, 128), h.n_d);
+  return head_slices_for((h.n_pad / 128) * ceil_div(r, 128), h.n_d, HEAD_RUN);
 }
 static int64_t head_slices_t(const dense_head& h, int r, int64_t n) {
-  return head_slices_for((h.n_d_pad / 128) * ceil_div(r, 128), n);
+  return head_slices_for((h.n_d_pad / 128) * ceil_div(r, 128), n, h.t_run);
 }
 
 // Floats of the workspace that the products of a head of n_d columns over n_rows rows use at rank r:
 // the gathered rows of H of the head, or W transposed (the split-operand product wants the
 // contraction index fast), plus the slice partials of the larger of the two products.
-int64_t head_workspace_floats(int64_t n_rows, int64_t n_d, int r) {
+int64_t head_workspace_floats(int64_t n_rows, int64_t n_d, int r, int64_t t_run) {
   if (n_d <= 0) return 0;
   dense_head h;
+  h.t_run = t_run;
   h.n_d = n_d;
   h.n_d_pad = ceil_div(n_d, 128) * 128;
   h.n_pad = ceil_div(n_rows, 128) * 128;
@@ -741,7 +747,7 @@ int head_ensure_workspace(dnpeff_csr* A, int r) {
   dense_head& h = A->head;
   if (h.n_d == 0) return 0;
   DN_CHECK(r % 4 == 0, "a matrix with a dense head needs a rank that is a multiple of 4 (got %d)", r);
-  const int64_t need = head_workspace_floats(A->n_rows, h.n_d, r);
+  const int64_t need = head_workspace_floats(A->n_rows, h.n_d, r, h.t_run);
   if (!head_uses_split(r) && !h.rm) {  // the fp32 kernel of A^T W wants the block row by row
     if (dmalloc(&h.rm, h.n_pad * h.n_d_pad)) {
       // no room for the second copy: at ranks that the split-operand kernel handles the head's

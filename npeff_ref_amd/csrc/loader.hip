@@ -1463,7 +1463,7 @@ namespace dn {
 // the remaining entries (16 bytes each).  The choice is the first admissible candidate
 // whose footprint is within `budget` bytes (NO_BUDGET: the first admissible one), else the
 // admissible candidate with the smallest footprint (fits = false).
-int choose_dense_head(dnpeff_csr* A, double min_fill, double budget, int n_blocks, int rank, head_choice* out) {
+int choose_dense_head(dnpeff_csr* A, double min_fill, double budget, int n_blocks, int rank, int64_t t_run, head_choice* out) {
   *out = head_choice();
   out->footprint = 16.0 * (double)A->nnz;
   out->fits = out->footprint <= budget;
@@ -1503,7 +1503,7 @@ int choose_dense_head(dnpeff_csr* A, double min_fill, double budget, int n_block
     c.thr = thr;
     c.n_d = n_d;
     c.footprint = blocks + 16.0 * (double)(A->nnz - (int64_t)z_head) +
-                  (rank > 0 ? 4.0 * (double)head_workspace_floats(n, n_d, rank) : 0.0);
+                  (rank > 0 ? 4.0 * (double)head_workspace_floats(n, n_d, rank, t_run) : 0.0);
     c.fits = c.footprint <= budget;
     if (c.fits) {
       best = c;
@@ -1611,7 +1611,7 @@ DN_API int dnpeff_csr_split_dense_head(dnpeff_csr* A, double min_fill, int64_t* 
     return 0;
   }
   head_choice c;
-  DN_TRY(choose_dense_head(A, min_fill, NO_BUDGET, 2, 0, &c));
+  DN_TRY(choose_dense_head(A, min_fill, NO_BUDGET, 2, 0, HEAD_RUN, &c));
   return split_dense_head_at(A, c.thr, n_dense);
 }
 

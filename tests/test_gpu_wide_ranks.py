@@ -105,3 +105,53 @@ def test_rank_between_the_tiles_of_128(n, m_full, k, r):
     assert nmf.sparsify_W(3.0) == rounds and np.array_equal(nmf.loadWToHostSync(), dW.numpy())
     nmf.close()
     A.close()
+
+
+def test_padded_rank_sums_many_columns():
+    """H^T H at a rank stored as 512, with large columns before small ones in every slice of the tiles: seen in
+    the loss's <W^T W, H^T H>.  (W, and with it H, in eight of the components, one or two per tile.)"""
+    n, m, r = 400, 2_000_000, 385
+    rng = np.random.default_rng(r)
+    rows = np.sort(rng.integers(0, n, m))
+    rp = np.concatenate([[0], np.cumsum(np.bincount(rows, minlength=n))]).astype(np.int64)
+    cols = rng.permutation(m).astype(np.int32)
+    vals = rng.random(m, dtype=np.float32) + np.float32(0.5)
+    vals[cols < 20_000] *= np.float32(300)
+    A = d.Csr.from_host(rp, cols, vals, m)
+    nmf = d.MuNmf(A, d.MuNmfParams(rank=r, max_iters=1, eps=1e-8, seed=5, log_every=0))
+    nmf.initialize()
+    held = np.array([0, 50, 100, 130, 200, 256, 300, 384])
+    W = np.zeros((n, r), dtype=np.float32)
+    W[:, held] = rng.random((n, len(held)), dtype=np.float32) + np.float32(0.5)
+    nmf.set_factors(W, None)
+    nmf.update_H()
+    _, pos, _ = nmf.loss_terms()
+    H = nmf.loadHToHostSync()[held].astype(np.float64)
+    W = W[:, held].astype(np.float64)
+    want = float(((W.T @ W) * (H @ H.T)).sum())
+    assert abs(pos - want) <= 1.2e-7 * want  # (two roundings to fp32)
+    nmf.close()
+    A.close()
+
+
+def test_padded_rank_sums_many_rows():
+    """A^T W of the dense head's columns at a rank stored as 256, 2000 rows: one H update."""
+    n, m, full, r = 2000, 40_000, 20_000, 150
+    rng = np.random.default_rng(r)
+    dense = np.zeros((n, m), dtype=np.float32)
+    dense[:, :full] = rng.random((n, full), dtype=np.float32) + np.float32(0.5)
+    dense[np.arange(m - full) % n, np.arange(full, m)] = 1
+    dense[400:, 1:full:2] *= np.float32(1e-3)
+    mask = dense != 0
+    A = d.Csr.from_host(np.concatenate([[0], np.cumsum(mask.sum(axis=1))]).astype(np.int64),
+                        np.nonzero(mask)[1].astype(np.int32), dense[mask], m)
+    nmf = d.MuNmf(A, d.MuNmfParams(rank=r, max_iters=1, eps=1e-8, seed=5, log_every=0))
+    assert A.head_info()[0] == full
+    nmf.initialize()
+    W, H = nmf.loadWToHostSync().astype(np.float64), nmf.loadHToHostSync().astype(np.float64)[:, :full]
+    want = H * (W.T @ dense[:, :full]) / (W.T @ W @ H + 1e-8)
+    nmf.update_H()
+    err = np.linalg.norm(nmf.loadHToHostSync()[:, :full] - want) / np.linalg.norm(want)
+    assert err <= 2.4e-7  # (four roundings to fp32)
+    nmf.close()
+    A.close()
