@@ -73,9 +73,12 @@ int dnpeff_release_cached(void);
  * and whose dense head holds n_dense columns, at the given rank, with the tiled (1) or full-size
  * (0) H update, on a device of total_bytes; sweeps = 1 when A H^T has swept pieces (ranks 32, 64,
  * 128, 256 and multiples of 128 above, on a device whose workgroups go to the XCDs round-robin).
- * out[0..7] = factors and their workspaces, partial sums of A H^T, segment offsets, column/row
- * offsets, reserve left free, both sparse copies, dense blocks of the head, workspace of the
- * head's products; all in bytes, upper bounds from the rules that size the allocations.  The
+ * out[0..7] = factors with their workspaces, partial sums and (ranks above 128 that are stored as the
+ * next multiple of 128) packed copies, partial sums of A H^T, segment offsets, column/row
+ * offsets and work lists, reserve left free, the sparse copies (two; at ranks up to 128, without a dense
+ * head, the packed entries of their step as well), dense blocks of the head, workspace of the
+ * head's products; all in bytes, upper bounds from the rules that size the allocations.  A rank is
+ * priced as it would be stored on that device with nothing else on it.  The
  * reference sizes its buffers inside the constructor
  * (multi_mu_dense_factors_device_contexts1.h:128-200) and has no such call. */
 int dnpeff_plan_estimate(int64_t n_rows, int64_t n_cols, int64_t nnz_sparse, int64_t n_dense, int rank,

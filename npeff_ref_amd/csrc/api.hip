@@ -199,23 +199,26 @@ static int64_t tile_cols_for(int64_t m, int rank) {
 }
 
 // Bytes of device memory that the handle allocates besides the structures of the matrix.
-static double factor_bytes(int64_t n, int64_t m, int rank, bool tiled, int64_t run) {
+static double factor_bytes(int64_t n, int64_t m, int rank, int asked, bool tiled) {
+  const int64_t run = rank != asked ? PADDED_GRAM_RUN : 0;
   const double nr = 4.0 * (double)n * rank, mr = 4.0 * (double)m * rank;
+  const double spare = 5.0 * 4.0 * (double)(rank > 128 && rank % 128 == 0 ? 128 * rank : 4);  // (rows_there, 16-byte loads)
+  const double packed = rank != asked ? 4.0 * (double)asked * (double)(n + m) : 0.0;
   double ws = (double)gram_workspace_floats(m, rank, run), ws_n = (double)gram_workspace_floats(n, rank, run);
   if (ws_n > ws) ws = ws_n;
   const double tile = 4.0 * (double)tile_cols_for(m, rank) * rank;
   return 3.0 * nr + (tiled ? mr + 2.0 * tile : 2.0 * mr) + 4.0 * ws + 3.0 * 4.0 * rank * rank +
-         4.0 * (double)xg_mu_gram_workspace_floats(m);
+         4.0 * (double)xg_mu_gram_workspace_floats(m) + spare + packed;
 }
 
 // What the products' own buffers take besides the two sparse copies (16 bytes per entry of the
 // sparse part), the dense blocks and the head's workspace, which the choice of the head prices
 // per candidate: upper bounds from the same rules that size the allocations.
 struct plan_table {
-  double factors = 0.0;   // W, its double buffer, A H^T, H (+ tile), A^T W (or its tile), Grams, workspaces
+  double factors = 0.0;   // W, its double buffer, A H^T, H (+ tile), A^T W (or its tile), Grams, workspaces, packed copies
   double partials = 0.0;  // partial sums of A H^T: per 2048-entry chunk, or per (row, plain panel / XCD)
   double segments = 0.0;  // offsets of the (row, panel) segments
-  double offsets = 0.0;   // column offsets, long-column list, row offsets and chunk counts
+  double offsets = 0.0;   // column offsets, long-column list, row offsets and chunk counts, tiles of A^T W
   double reserve = 0.0;   // left free (1/64 of the device, at least 1 GiB): allocation granularity, code objects, the runtime's own
   double total() const { return factors + partials + segments + offsets + reserve; }
 };
@@ -224,7 +227,7 @@ struct plan_table {
 static plan_table plan_overheads(int64_t n, int64_t m, int64_t nnz_sparse, int rank, int asked, bool tiled, bool sweeps,
                                  double total_bytes) {
   plan_table t;
-  t.factors = factor_bytes(n, m, rank, tiled, rank != asked ? PADDED_GRAM_RUN : 0);
+  t.factors = factor_bytes(n, m, rank, asked, tiled);
   const int64_t P = coarse_panels_for(n, m, rank, sweeps);
   const double by_chunks = 4.0 * rank * ((double)nnz_sparse / (double)SPMM_N_CHUNK + (double)n);
   const double by_panels = P > 0 ? 4.0 * rank * (double)n * (double)(P + SWEEP_XCDS) : 0.0;
@@ -233,8 +236,27 @@ static plan_table plan_overheads(int64_t n, int64_t m, int64_t nnz_sparse, int r
   t.segments = P > 0 ? 8.0 * (double)n * (double)((sweeps ? max_panels() : P) + 1) : 0.0;
   const double n_long = std::min((double)m, (double)nnz_sparse / (double)(SPMM_T_LONG + 1));
   t.offsets = 8.0 * (double)(m + 1) + 4.0 * n_long + 2.0 * 8.0 * (double)(n + 1) + 2.0 * 8.0 * 64.0;
+  if (rank > 128) t.offsets += spmm_t_bal_fits(n, rank) ? fused_tiles_bytes(m, nnz_sparse) : 0.0;
   t.reserve = std::max(1073741824.0, total_bytes / 64.0);
   return t;
+}
+
+// Whether a rank is stored as the next multiple of 128.  At 500 x 823k ten updates take 111 ms at r = 301 as it
+// is (fp32 matrix cores, 4-byte loads) and 41 ms with 384 components of which 83 are zero.  Not where the longer
+// rows, with the packed copies that callers may ask for, do not fit into `there` bytes.
+static int stored_rank(int64_t n, int64_t m, int64_t nnz, int rank, bool sweeps, double there, double total_bytes) {
+  const int p = (rank + 127) / 128 * 128;
+  if (rank <= 128 || p == rank || !use_split_bf16() || tuning().pad_rank == 0.0 || tuning().tiled_h > 0.0) return rank;
+  const plan_table t = plan_overheads(n, m, nnz, p, rank, false, sweeps, total_bytes);
+  return t.total() + 24.0 * (double)nnz <= there ? p : rank;
+}
+
+// Whether the step of small ranks runs where memory allows.  (It reads the whole matrix from its own lists: no
+// dense head is split off then.  Multiples of 64 with rows enough for a dense head keep it: its kernels are made
+// for those ranks.)
+static bool fused_step_wanted(int64_t n, int64_t m, int64_t nnz, int rank) {
+  return tuning().fused_gram != 0.0 && tuning().tiled_h <= 0.0 && !(rank % 64 == 0 && n >= 1024) &&
+         fused_supported(n, m, nnz, rank);
 }
 
 // For tests and capacity planning without a GPU: the table above and, for a head of n_dense columns,
@@ -247,13 +269,20 @@ DN_API int dnpeff_plan_estimate(int64_t n_rows, int64_t n_cols, int64_t nnz_spar
   DN_CHECK(n_rows >= 0 && n_cols >= 0 && nnz_sparse >= 0 && n_dense >= 0 && n_dense <= n_cols,
            "negative size");
   DN_CHECK(rank >= 1 && rank <= 1024, "rank %d outside [1, 1024]", rank);
-  const plan_table t = plan_overheads(n_rows, n_cols, nnz_sparse, rank, rank, tiled != 0, sweeps != 0, (double)total_bytes);
-  out[0] = t.factors; out[1] = t.partials; out[2] = t.segments; out[3] = t.offsets; out[4] = t.reserve;
+  const double total = (double)total_bytes;
+  const int asked = rank;
+  if (!tiled) rank = stored_rank(n_rows, n_cols, nnz_sparse, asked, sweeps != 0, total, total);
+  plan_table t = plan_overheads(n_rows, n_cols, nnz_sparse, rank, asked, tiled != 0, sweeps != 0, total);
   out[5] = 16.0 * (double)nnz_sparse;
+  if (!tiled && n_dense == 0 && fused_step_wanted(n_rows, n_cols, nnz_sparse, rank)) {
+    out[5] += fused_list_bytes(n_rows, n_cols, nnz_sparse);
+    t.factors += fused_state_bytes(n_rows, n_cols, nnz_sparse, rank);
+  }
+  out[0] = t.factors; out[1] = t.partials; out[2] = t.segments; out[3] = t.offsets; out[4] = t.reserve;
   out[6] = n_dense ? 4.0 * head_blocks_for_rank(rank) * (double)(ceil_div(n_rows, 128) * 128) *
                          (double)(ceil_div(n_dense, 128) * 128)
                    : 0.0;
-  out[7] = 4.0 * (double)head_workspace_floats(n_rows, n_dense, rank, HEAD_RUN);
+  out[7] = 4.0 * (double)head_workspace_floats(n_rows, n_dense, rank, head_run(rank, asked));
   return 0;
 }
 
@@ -263,8 +292,7 @@ DN_API int dnpeff_plan_estimate(int64_t n_rows, int64_t n_cols, int64_t nnz_spar
 // the rows hold it (dense_fill switch; 0 = never split); the fraction is raised until the dense
 // blocks and both sparse copies of the rest fit the memory left beside the factors.  *tiled
 // receives whether the H update must run on column tiles for everything to fit.
-// *fused: whether the step of small ranks can run (it reads the whole matrix from its own lists: no
-// dense head is split off then).
+// *fused: whether the step of small ranks runs.
 static int plan_matrix(dnpeff_csr* A, int rank, int asked, bool consume, bool* tiled, bool* fused) {
   const tuning_t& tn = tuning();
   size_t free_b = 0, total_b = 0;
@@ -285,10 +313,9 @@ static int plan_matrix(dnpeff_csr* A, int rank, int asked, bool consume, bool* t
   const plan_table t_tiled = plan_overheads(A->n_rows, A->n_cols, A->nnz, rank, asked, true, sweeps, (double)total_b);
   const double budget_full = avail - t_full.total();
   const double budget_tiled = avail - t_tiled.total();
-  // (multiples of 64 with rows enough for a dense head keep it: its kernels are made for those ranks)
-  *fused = tn.fused_gram != 0.0 && tn.tiled_h <= 0.0 && !(rank % 64 == 0 && A->n_rows >= 1024) &&
-           fused_supported(A->n_rows, A->n_cols, A->nnz, rank) &&
-           16.0 * (double)A->nnz + fused_bytes(A->n_rows, A->nnz, rank) < budget_full;
+  *fused = fused_step_wanted(A->n_rows, A->n_cols, A->nnz, rank) &&
+           16.0 * (double)A->nnz + fused_list_bytes(A->n_rows, A->n_cols, A->nnz) +
+                   fused_state_bytes(A->n_rows, A->n_cols, A->nnz, rank) < budget_full;
   const bool can_split = rank % 4 == 0 && rank >= 64 && A->n_rows >= 1024 && !*fused;
   double fill = tn.dense_fill;
   if (fill > 1.0) fill = 0.0;
@@ -331,22 +358,13 @@ static int plan_matrix(dnpeff_csr* A, int rank, int asked, bool consume, bool* t
   return split_dense_head_at(A, c.thr, nullptr);
 }
 
-// The rank that the factors are stored with.  At 500 x 823k ten updates take 111 ms at r = 301 as it
-// is (fp32 matrix cores, 4-byte loads) and 41 ms with 384 components of which 83 are zero.  Not
-// where the longer rows do not fit (with the packed copy that callers may ask for), nor without an eps to
-// keep 0 * (0 / eps) zero.
+// The rank that the factors are stored with.  Padded ones need an eps that keeps 0 * (0 / eps) zero.
 static int padded_rank(const dnpeff_csr* A, int rank, float eps, int* out) {
   *out = rank;
-  const int p = (rank + 127) / 128 * 128;
-  if (rank <= 128 || p == rank || !(eps >= 1e-30f) || !use_split_bf16() || tuning().pad_rank == 0.0 ||
-      tuning().tiled_h > 0.0)
-    return 0;
+  if (rank <= 128 || !(eps >= 1e-30f)) return 0;
   size_t free_b = 0, total_b = 0;
   DN_HIP(hipMemGetInfo(&free_b, &total_b));
-  const plan_table t = plan_overheads(A->n_rows, A->n_cols, A->nnz, p, rank, false, sweeps_for_rank(p), (double)total_b);
-  if (t.total() + 4.0 * (double)rank * (double)(A->n_rows + A->n_cols) + 24.0 * (double)A->nnz <
-      (double)free_b + (double)pool_cached_bytes())
-    *out = p;
+  *out = stored_rank(A->n_rows, A->n_cols, A->nnz, rank, sweeps_for_rank((rank + 127) / 128 * 128), (double)free_b + (double)pool_cached_bytes(), (double)total_b);
   return 0;
 }
 

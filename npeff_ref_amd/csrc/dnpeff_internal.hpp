@@ -436,7 +436,8 @@ void tblocks_drop(dnpeff_csr* S);
 void fused_drop(dnpeff_csr* S);  // fused.hip
 int fused_tiles_build(dnpeff_csr* S, int r);  // the tiles of fused_plan for rank r (32 columns each above 64)
 int fused_tiles_first(dnpeff_csr* S);         // h_first of the tiles that are there
-bool use_spmm_t_bal(const dnpeff_csr* S, int r);  // spmm.hip
+bool spmm_t_bal_fits(int64_t n_rows, int r);      // spmm.hip
+bool use_spmm_t_bal(const dnpeff_csr* S, int r);
 int launch_spmm_t_lists(const dnpeff_csr* S, int r, const float* W_nr, float* T, int64_t col0, int64_t col1);
 // Whether the products of the sparse part S at rank r run from the slot lists / column blocks.
 bool use_nlists(const dnpeff_csr* S, int r);       // the whole sparse part on slot lists

@@ -1067,10 +1067,20 @@ int fused_state::loss_sums(const dnpeff_csr* S, int64_t n, const float* Nw, cons
   return 0;
 }
 
-double fused_bytes(int64_t n, int64_t nnz, int r) {
+double fused_tiles_bytes(int64_t m, int64_t nnz) {
+  // (a group of columns is cut where its tile would pass 512 entries or more: two tiles hold more than that)
+  return 16.0 * ((double)m / FUW_COLS + (double)nnz / 256.0 + 2.0);
+}
+
+double fused_list_bytes(int64_t n, int64_t m, int64_t nnz) {
+  return 8.0 * (double)(nnz + 1) + fused_tiles_bytes(m, nnz) + 16.0 * (double)(FU_CHUNKS + n) + 4.0 * (double)(n + 1);
+}
+
+double fused_state_bytes(int64_t n, int64_t m, int64_t nnz, int r) {
   const double S = 4.0 * fused_gram_floats(r);
-  return 8.0 * (double)nnz + 16.0 * ((double)nnz / 512.0) + 4.0 * (double)(FU_CHUNKS + n) * (r + 4) +
-         S * ((double)n_cus() * 8.0 + (double)n / FUW_COLS + 3.0);
+  // workgroups of the H update: one round of what the chip holds, or enough rounds of them
+  const double wgs = (r > FUSED_NARROW_RANK ? 4.0 : 8.0) * n_cus() + ((double)m + (double)nnz / 8.0) / FU_MOST_COLS;
+  return 4.0 * ((double)(FU_CHUNKS + n) * r + 4.0) + S * (wgs + (double)n / FUW_COLS + 3.0) + (double)n;
 }
 
 bool fused_supported(int64_t n, int64_t m, int64_t nnz, int r) {

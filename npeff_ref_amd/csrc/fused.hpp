@@ -19,8 +19,11 @@ constexpr int FU_MOST_COLS = 2048;
 constexpr int64_t FU_CHUNKS = 4096;  // workgroups that A H^T is cut into where its rows allow
 
 bool fused_supported(int64_t n, int64_t m, int64_t nnz, int r);
-// What the lists and a context's buffers take at most.
-double fused_bytes(int64_t n, int64_t nnz, int r);
+// What the lists of a matrix (alone: its tiles, which ranks above 128 use as well) and a context's buffers take at
+// most, in bytes.
+double fused_tiles_bytes(int64_t m, int64_t nnz);
+double fused_list_bytes(int64_t n, int64_t m, int64_t nnz);
+double fused_state_bytes(int64_t n, int64_t m, int64_t nnz, int r);
 // Tiles, packed entries and chunks of a matrix without dense head (needs csr_ensure_products).
 int fused_plan_build(dnpeff_csr* S, int r);
 

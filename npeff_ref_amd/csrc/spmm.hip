@@ -1417,8 +1417,11 @@ static int spmm_t_slices(int64_t n, int r) {
 
 // Ranks above 128 (below, a wave reads several rows of W at once) with a W that an L2 holds, unless the
 // switch asks for the older kernel by its slices.
+bool spmm_t_bal_fits(int64_t n_rows, int r) {
+  return r > 128 && r <= 1024 && r % 4 == 0 && tuning().spmm_t_slices == 0.0 && 4.0 * (double)n_rows * r <= 6.0e6;
+}
 bool use_spmm_t_bal(const dnpeff_csr* S, int r) {
-  return r > 128 && r <= 1024 && r % 4 == 0 && tuning().spmm_t_slices == 0.0 && 4.0 * (double)S->n_rows * r <= 6.0e6 &&
+  return spmm_t_bal_fits(S->n_rows, r) &&
          S->nnz > 0 && S->n_cols > 0 && ceil_div(S->n_cols, 32) + S->nnz / 256 < ((int64_t)1 << 24);
 }
 

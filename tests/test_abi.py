@@ -186,3 +186,19 @@ def test_memory_plan_arithmetic_for_the_benchmark_shapes():
     assert d.plan_estimate(512, 900_000, 2_097_152, 0, 16, False, total_bytes=8 * 2**30)["reserve"] == 2.0**30
     with pytest.raises(d.DnpeffError):
         d.plan_estimate(10, 5, 1, 6, 16, False)  # more head columns than columns
+
+
+def test_memory_plan_of_padded_ranks_and_small_ranks():
+    """Ranks stored as the next multiple of 128 are priced as stored, with the packed copies that callers may ask
+    for; the step of small ranks with its packed entries, chunk sums and partial Gram matrices."""
+    n, m, z = 1000, 800_000, 4_000_000
+    p200, p256 = (d.plan_estimate(n, m, z, 0, r, False) for r in (200, 256))
+    assert p200["factors"] >= p256["factors"] + 4.0 * 200 * (n + m) and p200["offsets"] >= p256["offsets"]
+    # (not where the padded factors would not fit)
+    small = 4 * 4 * 200 * m
+    assert d.plan_estimate(n, m, z, 0, 200, False, total_bytes=small)["factors"] < p200["factors"] * 0.75
+    for r in (8, 50, 100):
+        e = d.plan_estimate(n, m, z, 0, r, False)
+        assert e["sparse_copies"] >= 24.0 * z  # row-major, by columns, packed for the step
+        assert e["factors"] >= 4.0 * r * (2 * m + 3 * n) + 4.0 * r * n
+    assert d.plan_estimate(n, m, z, 5000, 100, False)["sparse_copies"] == 16.0 * z  # a dense head: the separate kernels
