@@ -12,12 +12,12 @@
 // get or give back memory directly (dnpeff_dev_malloc / dnpeff_dev_free) may use other streams:
 // those calls wait, as hipFree does.  One lock guards the lists.
 #include "dnpeff_internal.hpp"
+#include "host_parts.hpp"
 
 #include <atomic>
 #include <cstring>
 #include <map>
 #include <mutex>
-#include <thread>
 #include <unordered_map>
 #include <utility>
 #include <vector>
@@ -273,10 +273,7 @@ static hipError_t staged_copy(const copy_part* parts, int n_parts) {
     if (e != hipSuccess) failed = (int)e;
   };
   const int n_threads = n_pieces < (size_t)COPY_THREADS ? (int)n_pieces : COPY_THREADS;
-  std::vector<std::thread> helpers;
-  for (int t = 1; t < n_threads; t++) helpers.emplace_back(work, t);
-  work(0);
-  for (std::thread& h : helpers) h.join();
+  run_shares(n_threads, work, [](auto f) { return std::thread(f); });
   return (hipError_t)failed.load();
 }
 

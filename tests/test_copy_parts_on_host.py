@@ -1,0 +1,41 @@
+"""The parts of the host-device copies that need no GPU (csrc/host_parts.hpp), compiled as they are."""
+
+import os
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+
+def _run(tmp_path, body):
+    src, exe = tmp_path / "t.cc", tmp_path / "t"
+    src.write_text('#include "host_parts.hpp"\n#include <atomic>\n#include <cstdio>\n#include <set>\n#include <system_error>\n'
+                   '#define CHECK(x) do { if (!(x)) { std::printf("%d: %s\\n", __LINE__, #x); return 1; } } while (0)\n'
+                   + body)
+    subprocess.run(["g++", "-std=c++17", "-O1", "-pthread", "-I", os.path.join(ROOT, "npeff_ref_amd", "csrc"), str(src),
+                    "-o", str(exe)], check=True)
+    out = subprocess.run([str(exe)], capture_output=True, text=True, timeout=60)
+    assert out.returncode == 0, out.stdout + out.stderr
+
+
+@pytest.mark.parametrize("threads", [0, 1, 3, 7])
+def test_shares_run_without_threads(tmp_path, threads):
+    """As many threads as can be made, every share once."""
+    _run(tmp_path, """
+int main() {
+  for (int n = 1; n <= 8; n++) {
+    std::atomic<int> ran[8] = {};
+    int made = 0;
+    auto spawn = [&](auto f) {
+      if (made == %d) throw std::system_error(std::make_error_code(std::errc::resource_unavailable_try_again));
+      made++;
+      return std::thread(f);
+    };
+    dn::run_shares(n, [&](int t) { ran[t]++; }, spawn);
+    for (int t = 0; t < n; t++) CHECK(ran[t] == 1);
+    for (int t = n; t < 8; t++) CHECK(ran[t] == 0);
+  }
+}
+""" % threads)
+
