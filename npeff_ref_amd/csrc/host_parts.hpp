@@ -1,7 +1,11 @@
 // Parts of the copies between host and device that need no GPU.
 #pragma once
 
+#include <map>
+#include <mutex>
 #include <thread>
+#include <utility>
+#include <vector>
 
 namespace dn {
 
@@ -20,5 +24,42 @@ void run_shares(int n, Work&& work, Spawn&& spawn) {
   for (int t = made; t < n; t++) work(t);
   for (int t = 1; t < made; t++) helpers[t].join();
 }
+
+// Objects that wait for their next use on the device they belong to.
+template <class T>
+class idle_by_device {
+ public:
+  bool take(int dev, T* out) {
+    std::lock_guard<std::mutex> g(lock_);
+    auto it = idle_.find(dev);
+    if (it == idle_.end() || it->second.empty()) return false;
+    *out = it->second.back();
+    it->second.pop_back();
+    return true;
+  }
+  // false: `most` of the device wait already (or there is no memory to note one more)
+  bool give(int dev, const T& x, size_t most) {
+    std::lock_guard<std::mutex> g(lock_);
+    try {
+      std::vector<T>& of_dev = idle_[dev];
+      if (of_dev.size() >= most) return false;
+      of_dev.push_back(x);
+    } catch (...) {
+      return false;
+    }
+    return true;
+  }
+  template <class F>
+  void drain(F&& f) {
+    std::lock_guard<std::mutex> g(lock_);
+    for (auto& of_dev : idle_)
+      for (T& x : of_dev.second) f(x);
+    idle_.clear();
+  }
+
+ private:
+  std::mutex lock_;
+  std::map<int, std::vector<T>> idle_;
+};
 
 }  // namespace dn

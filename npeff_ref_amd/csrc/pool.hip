@@ -284,18 +284,14 @@ static hipError_t staged_copy(const copy_part* parts, int n_parts) {
 // the buffer: shorter still than a copy on the engines.
 constexpr size_t BOUNCE_HALF = (size_t)1 << 20;
 constexpr size_t BOUNCE_KERNEL = 16384;
-constexpr size_t BOUNCE_KEPT = 4;  // buffers that wait for the next call
+constexpr size_t BOUNCE_KEPT = 4;  // buffers of a device that wait for the next call
 
 struct bounce_buf {
   char* p = nullptr;
   hipEvent_t done[2] = {};
 };
-struct bounce_state {
-  std::mutex lock;
-  std::vector<bounce_buf> idle;
-};
-static bounce_state& bounces() {
-  static bounce_state* b = new bounce_state();
+static idle_by_device<bounce_buf>& bounces() {  // (the events belong to a device)
+  static auto* b = new idle_by_device<bounce_buf>();
   return *b;
 }
 static void bounce_free(bounce_buf& b) {
@@ -304,16 +300,8 @@ static void bounce_free(bounce_buf& b) {
     if (e) (void)hipEventDestroy(e);
   b = bounce_buf();
 }
-static bool bounce_take(bounce_buf* b) {
-  {
-    bounce_state& B = bounces();
-    std::lock_guard<std::mutex> g(B.lock);
-    if (!B.idle.empty()) {
-      *b = B.idle.back();
-      B.idle.pop_back();
-      return true;
-    }
-  }
+static bool bounce_take(int dev, bounce_buf* b) {
+  if (bounces().take(dev, b)) return true;
   if (hipHostMalloc((void**)&b->p, 2 * BOUNCE_HALF, hipHostMallocDefault) == hipSuccess &&
       hipEventCreateWithFlags(&b->done[0], hipEventDisableTiming) == hipSuccess &&
       hipEventCreateWithFlags(&b->done[1], hipEventDisableTiming) == hipSuccess)
@@ -322,23 +310,10 @@ static bool bounce_take(bounce_buf* b) {
   bounce_free(*b);
   return false;
 }
-static void bounce_give(bounce_buf& b) {
-  bounce_state& B = bounces();
-  {
-    std::lock_guard<std::mutex> g(B.lock);
-    if (B.idle.size() < BOUNCE_KEPT) {
-      B.idle.push_back(b);
-      return;
-    }
-  }
-  bounce_free(b);
+static void bounce_give(int dev, bounce_buf& b) {
+  if (!bounces().give(dev, b, BOUNCE_KEPT)) bounce_free(b);
 }
-static void bounce_trim() {
-  bounce_state& B = bounces();
-  std::lock_guard<std::mutex> g(B.lock);
-  for (bounce_buf& b : B.idle) bounce_free(b);
-  B.idle.clear();
-}
+static void bounce_trim() { bounces().drain(bounce_free); }
 
 __global__ void __launch_bounds__(256) k_copy_words(const uint32_t* __restrict__ src, uint32_t* __restrict__ dst, int n) {
   for (int i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) dst[i] = src[i];
@@ -347,7 +322,8 @@ __global__ void __launch_bounds__(256) k_copy_words(const uint32_t* __restrict__
 template <bool UP>
 static hipError_t bounce_copy(char* dst, const char* src, size_t bytes) {
   bounce_buf B;
-  if (!bounce_take(&B)) return hipMemcpy(dst, src, bytes, UP ? hipMemcpyHostToDevice : hipMemcpyDeviceToHost);
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || !bounce_take(dev, &B)) return hipMemcpy(dst, src, bytes, UP ? hipMemcpyHostToDevice : hipMemcpyDeviceToHost);
   hipStream_t st = stream();
   hipError_t e = hipSuccess;
   if (!UP && bytes <= BOUNCE_KERNEL && bytes % 4 == 0 && (uintptr_t)src % 4 == 0) {
@@ -394,7 +370,7 @@ static hipError_t bounce_copy(char* dst, const char* src, size_t bytes) {
       for (int i = k >= 2 ? k - 2 : 0; i < k; i++) memcpy(dst + at[i & 1], B.p + (i & 1) * BOUNCE_HALF, len[i & 1]);
   }
   if (e != hipSuccess) (void)hipStreamSynchronize(st);  // (nothing may still be on its way to the buffer)
-  bounce_give(B);
+  bounce_give(dev, B);
   return e;
 }
 

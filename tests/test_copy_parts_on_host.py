@@ -39,3 +39,22 @@ int main() {
 }
 """ % threads)
 
+
+def test_idle_objects_stay_with_their_device(tmp_path):
+    _run(tmp_path, """
+int main() {
+  dn::idle_by_device<int> idle;
+  int x = -1;
+  CHECK(!idle.take(0, &x));
+  for (int k = 0; k < 4; k++) CHECK(idle.give(0, 10 + k, 4));
+  CHECK(!idle.give(0, 14, 4));
+  CHECK(idle.give(1, 20, 4));
+  CHECK(idle.take(1, &x) && x == 20);
+  CHECK(!idle.take(1, &x));
+  CHECK(idle.take(0, &x) && x == 13);
+  std::set<int> left;
+  idle.drain([&](int& y) { left.insert(y); });
+  CHECK(left == (std::set<int>{10, 11, 12}));
+  CHECK(!idle.take(0, &x));
+}
+""")
