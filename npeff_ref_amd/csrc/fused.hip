@@ -177,9 +177,9 @@ __device__ inline void fu_gram_fold(double (&sum)[NP][4], f32x4 (&acc)[NP]) {
     }
 }
 
-// The four waves' Gram blocks, added in wave order, to out ([pair][16][16]); lds: NP * 256 floats.
-template <int NP>
-__device__ inline void fu_gram_out(const f32x4 (&acc)[NP], float* __restrict__ lds, float* __restrict__ out) {
+// The four waves' Gram blocks, added in fp64 in wave order, to out ([pair][16][16]); lds: NP * 256 doubles.
+template <int NP, class V>
+__device__ inline void fu_gram_out(const V& v, double* __restrict__ lds, float* __restrict__ out) {
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, l16 = lane & 15, g = lane >> 4;
   for (int w = 0; w < 4; w++) {
     __syncthreads();
@@ -188,13 +188,13 @@ __device__ inline void fu_gram_out(const f32x4 (&acc)[NP], float* __restrict__ l
       for (int p = 0; p < NP; p++)
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-          float* at = lds + p * 256 + (4 * g + i) * 16 + l16;
-          *at = w == 0 ? acc[p][i] : *at + acc[p][i];
+          double* at = lds + p * 256 + (4 * g + i) * 16 + l16;
+          *at = w == 0 ? (double)v[p][i] : *at + (double)v[p][i];
         }
     }
   }
   __syncthreads();
-  for (int x = threadIdx.x; x < NP * 256; x += 256) out[x] = lds[x];
+  for (int x = threadIdx.x; x < NP * 256; x += 256) out[x] = (float)lds[x];
 }
 
 // ---------------------------------------------------------------------------
@@ -216,23 +216,19 @@ __device__ inline void fu_gram_out(const f32x4 (&acc)[NP], float* __restrict__ l
 // (390 -> 335 us with it).  777 x 862k, r = 50: 181 us for 2.0 GFLOP of gathers and 12.9 of products
 // (922 us for A^T W, update and Gram as separate kernels); 512 x 431k, r = 16: 31 us (139).
 // ---------------------------------------------------------------------------
-template <int Q, int R, int JB>
+template <int Q, int R, int JB, bool TOTALS>
 __global__ void __launch_bounds__(256, fu_blocks(Q, R) <= 2 ? 4 : 3)
     k_fu_h(const fu_tile* __restrict__ tiles, int n_tiles, const int64_t* __restrict__ colptr,
            const uint2* __restrict__ pairs, int r, const float* __restrict__ W, float* __restrict__ H, float eps,
            const float* __restrict__ gw, int n_gw, float* __restrict__ gpart) {
   constexpr int NB = fu_blocks(Q, R), NP = fu_pairs(NB), TS = 16 * NB + 4, TC = 64 * JB;
   using Gather = fu_gather<TC, TS, NB, fu_lpr(Q, R)>;
-  constexpr int T_FLOATS = Gather::CARRY + 2048 > NP * 256 ? Gather::CARRY + 2048 : NP * 256;
+  constexpr int T_FLOATS = Gather::CARRY + 2048 > NP * 512 ? Gather::CARRY + 2048 : NP * 512;
   __shared__ __align__(16) float ga[NB * NB * 256];
   __shared__ __align__(16) float tile[T_FLOATS];
   __shared__ int cps[2][TC + 1];
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int l16 = lane & 15, g = lane >> 4;
-  // Up to 32 components the Gram sums of a tile are added up in fp64: fp32 sums over all tiles of a workgroup
-  // lose what follows a column with large entries (W update at 2000 x 6.4 M, r = 16: error 3.3e-6, now 1e-7, in
-  // the same time).  Above, the registers hold the fp32 sums only.
-  constexpr bool TOTALS = NB <= 2;
   double sum[TOTALS ? NP : 1][4] = {};
   f32x4 acc[NP];
 #pragma unroll
@@ -336,13 +332,10 @@ __global__ void __launch_bounds__(256, fu_blocks(Q, R) <= 2 ? 4 : 3)
     td = nd;
     __syncthreads();  // (the tile has been read)
   }
-  if constexpr (TOTALS) {
-#pragma unroll
-    for (int p = 0; p < NP; p++)
-#pragma unroll
-      for (int i = 0; i < 4; i++) acc[p][i] = (float)sum[p][i];
-  }
-  fu_gram_out<NP>(acc, tile, gpart + (int64_t)blockIdx.x * (NP * 256));
+  double* lds = reinterpret_cast<double*>(tile);
+  float* out = gpart + (int64_t)blockIdx.x * (NP * 256);
+  if constexpr (TOTALS) fu_gram_out<NP>(sum, lds, out);
+  else fu_gram_out<NP>(acc, lds, out);
 }
 
 // W update: 64 rows per workgroup.  n_base (or NULL: N holds A H^T itself): first chunk of every row.
@@ -351,7 +344,7 @@ __global__ void __launch_bounds__(256)
     k_fu_w(int64_t n, int r, const int* __restrict__ n_base, const float* __restrict__ N, float* __restrict__ W,
            float eps, const float* __restrict__ gh, int n_gh, float* __restrict__ gpart) {
   constexpr int NB = fu_blocks(Q, R), NP = fu_pairs(NB), TS = 16 * NB + 4;
-  constexpr int T_FLOATS = FU_ROWS_WG * TS > NP * 256 ? FU_ROWS_WG * TS : NP * 256;
+  constexpr int T_FLOATS = FU_ROWS_WG * TS > NP * 512 ? FU_ROWS_WG * TS : NP * 512;
   __shared__ __align__(16) float ga[NB * NB * 256];
   __shared__ __align__(16) float tile[T_FLOATS];
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, l16 = lane & 15, g = lane >> 4;
@@ -382,7 +375,7 @@ __global__ void __launch_bounds__(256)
   fu_update<Q, R>(ga, x, t, eps, r, mine, wrow, tile + (16 * wave + l16) * TS);
   __builtin_amdgcn_wave_barrier();
   fu_gram<NB>(tile + 16 * wave * TS, TS, acc);
-  fu_gram_out<NP>(acc, tile, gpart + (int64_t)blockIdx.x * (NP * 256));
+  fu_gram_out<NP>(acc, reinterpret_cast<double*>(tile), gpart + (int64_t)blockIdx.x * (NP * 256));
 }
 
 // Element x of the sum of n_parts partial Gram matrices: 16 elements per workgroup, 16 threads each.
@@ -422,7 +415,7 @@ template <int NB>
 __global__ void __launch_bounds__(256)
     k_fu_gram(const float* __restrict__ X, int64_t rows, int64_t per, int r, float* __restrict__ gpart) {
   constexpr int NP = fu_pairs(NB);
-  __shared__ float lds[NP * 256];
+  __shared__ double lds[NP * 256];
   const int64_t row0 = blockIdx.x * per, row1 = row0 + per < rows ? row0 + per : rows;
   const int lane = threadIdx.x & 63, l16 = lane & 15, g = lane >> 4;
   float a[4][NB], nx[4][NB];
@@ -457,11 +450,7 @@ __global__ void __launch_bounds__(256)
     if (k % 16 == 0) fu_gram_fold<NP>(sum, acc);
   }
   fu_gram_fold<NP>(sum, acc);
-#pragma unroll
-  for (int p = 0; p < NP; p++)
-#pragma unroll
-    for (int i = 0; i < 4; i++) acc[p][i] = (float)sum[p][i];
-  fu_gram_out<NP>(acc, lds, gpart + (int64_t)blockIdx.x * (NP * 256));
+  fu_gram_out<NP>(sum, lds, gpart + (int64_t)blockIdx.x * (NP * 256));
 }
 
 // 5 to 8 blocks: all waves take the same rows, 32 at a time through LDS (rows 16 banks apart: the four
@@ -916,26 +905,42 @@ static int fu_blocks_of(int r) { return (r + 15) / 16; }
 using fu_h_kernel = void (*)(const fu_tile*, int, const int64_t*, const uint2*, int, const float*, float*, float,
                              const float*, int, float*);
 
+// Whether the Gram sums of a tile are added up in fp64: fp32 sums over all tiles of a workgroup lose what follows
+// a column with large entries (W update at 2000 x 6.4 M, r = 16: error 3.3e-6, with fp64 totals 1e-7, in the same
+// time).  Up to 16 components always.  Up to 32 where a workgroup has more than one tile: the totals leave room
+// for four workgroups per CU instead of five, which one tile each would notice (300 x 146k, r = 20: 21.8 against
+// 19.6 us) and has no use for.  Above, the registers hold the fp32 sums only.
 template <int Q, int R>
-static fu_h_kernel fu_h_of(int tile_cols) {
+static fu_h_kernel fu_h_of(int tile_cols, bool totals) {
   constexpr int NB = fu_blocks(Q, R);
-  if constexpr (NB == 1) return tile_cols == 256 ? k_fu_h<Q, R, 4> : k_fu_h<Q, R, 1>;
-  else if constexpr (NB == 2) return tile_cols == 128 ? k_fu_h<Q, R, 2> : k_fu_h<Q, R, 1>;
-  else return k_fu_h<Q, R, 1>;
+  if constexpr (NB == 1) return tile_cols == 256 ? k_fu_h<Q, R, 4, true> : k_fu_h<Q, R, 1, true>;
+  else if constexpr (NB == 2)
+    return totals ? (tile_cols == 128 ? k_fu_h<Q, R, 2, true> : k_fu_h<Q, R, 1, true>)
+                  : (tile_cols == 128 ? k_fu_h<Q, R, 2, false> : k_fu_h<Q, R, 1, false>);
+  else return k_fu_h<Q, R, 1, false>;
 }
 
 int fused_state::create(const dnpeff_csr* S, int64_t n, int rank) {
   r = rank;
   S_floats = fused_gram_floats(r);
   const fused_plan& f = S->fused;
-  int per_cu = 0;
-  if (r > FUSED_NARROW_RANK) DN_TRY(fuw_per_cu(r, &per_cu));
-  else DN_TRY(fu_dispatch(r, [&](auto tag) {
-    DN_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(
-        &per_cu, fu_h_of<decltype(tag)::Q, decltype(tag)::R>(f.tile_cols), 256, 0));
+  int64_t most = 0;  // workgroups that the chip holds
+  auto count = [&]() {
+    int per_cu = 0;
+    if (r > FUSED_NARROW_RANK) DN_TRY(fuw_per_cu(r, &per_cu));
+    else DN_TRY(fu_dispatch(r, [&](auto tag) {
+      DN_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(
+          &per_cu, fu_h_of<decltype(tag)::Q, decltype(tag)::R>(f.tile_cols, h_totals), 256, 0));
+      return 0;
+    }));
+    most = (int64_t)n_cus() * (per_cu > 0 ? per_cu : 1);
     return 0;
-  }));
-  const int64_t most = (int64_t)n_cus() * (per_cu > 0 ? per_cu : 1);
+  };
+  DN_TRY(count());
+  if (f.n_tiles > most) {
+    h_totals = true;
+    DN_TRY(count());
+  }
   h_wgs = (int)(f.n_tiles < most ? f.n_tiles : most);
   // (above 32 the sums stay fp32 in registers: as many rounds of workgroups as keep them short.  3.4 M columns
   // at r = 128: in one round of 512 workgroups H^T H costs the W update an error of 8.5e-7, in four 2.0e-7; the
@@ -1047,7 +1052,7 @@ int fused_state::update_h(const dnpeff_csr* S, const float* W, float* H, float e
   if (r > FUSED_NARROW_RANK)
     DN_TRY(fuw_launch_h(h_wgs, f, S->colptr, r, W, H, eps, gw, n_gw, gh_part));
   else DN_TRY(fu_dispatch(r, [&](auto tag) {
-    hipLaunchKernelGGL((fu_h_of<decltype(tag)::Q, decltype(tag)::R>(f.tile_cols)), dim3((unsigned)h_wgs), dim3(256), 0,
+    hipLaunchKernelGGL((fu_h_of<decltype(tag)::Q, decltype(tag)::R>(f.tile_cols, h_totals)), dim3((unsigned)h_wgs), dim3(256), 0,
                        stream(), f.tiles, (int)f.n_tiles, S->colptr, f.pairs, r, W, H, eps, gw, n_gw, gh_part);
     return 0;
   }));

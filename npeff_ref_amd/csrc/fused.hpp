@@ -38,6 +38,7 @@ int fuw_launch_w(int wgs, int64_t n, int r, const int* n_base, const float* N, f
 struct fused_state {
   enum gram_state { NONE, PARTS, SUMMED };
   int r = 0, S_floats = 0, h_wgs = 0, w_wgs = 0;
+  bool h_totals = false;     // the H update adds its Gram sums up in fp64
   float* gh_part = nullptr;  // partial H^T H of the last H update, one per workgroup
   float* gw_part = nullptr;
   float* gh_sum = nullptr;
