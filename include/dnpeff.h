@@ -62,9 +62,11 @@ void* dnpeff_stream(void);
 int dnpeff_device_memory(int64_t* free_bytes, int64_t* total_bytes);
 
 /* Gives back what the library keeps between calls: freed device blocks (at most 1 GiB of them, none
- * larger than 256 MB, reused by later calls) and the pinned buffers that large copies to and from
- * pageable memory go through (24 MB).  The blocks also go back when an allocation fails and before
- * dnpeff_device_memory reports.  The reference allocates and frees per object and keeps nothing
+ * larger than 256 MB, reused by later calls; more than 64 MB only while a sixteenth of the device is
+ * free) and the pinned buffers that copies to and from pageable memory go through (32 MB for copies
+ * of 4 MB and more, up to 8 MB for smaller ones).  The blocks also go back when an allocation of the
+ * library fails and before dnpeff_device_memory reports; a process that needs the memory for another
+ * allocator calls this.  The reference allocates and frees per object and keeps nothing
  * (cc/cuda_d_npeff/src/cuda/cuda_context.h:58-69). */
 int dnpeff_release_cached(void);
 

@@ -5,7 +5,10 @@
 // ten such blocks per call: more than their kernels take.  Freed blocks of up to POOL_MAX_BLOCK
 // bytes therefore stay with the library, at most POOL_CAP bytes of them, and serve later requests of
 // the same size class (an eighth of a power of two).  They go back to the device when an allocation
-// fails, when the free memory is asked for and on dnpeff_release_cached().
+// fails, when the free memory is asked for and on dnpeff_release_cached().  Other allocators of the
+// process cannot ask for them: more than POOL_LOW bytes are kept only while a sixteenth of the device is
+// free, as last seen at most 0.1 s ago and since the last large block (hipMemGetInfo waits for kernels
+// under way: asked at every release it added 20 to 80 us to the calls of the fixed-H learner and the top-k).
 //
 // A block is reused in the order of the library stream: whatever the library still has queued on
 // it runs first.  (Blocks that the second stream touches live longer than any call.)  Callers who
@@ -15,6 +18,7 @@
 #include "host_parts.hpp"
 
 #include <atomic>
+#include <chrono>
 #include <cstring>
 #include <map>
 #include <mutex>
@@ -26,12 +30,15 @@ namespace dn {
 
 constexpr size_t POOL_MAX_BLOCK = (size_t)256 << 20;
 constexpr size_t POOL_CAP = (size_t)1 << 30;
+constexpr size_t POOL_LOW = (size_t)64 << 20;
 
 struct pool_state {
   std::mutex lock;
   std::map<std::pair<int, size_t>, std::vector<void*>> idle;        // (device, class) -> blocks
   std::unordered_map<void*, std::pair<int, size_t>> live;           // blocks handed out
   size_t cached = 0;
+  bool asked = false, is_short = false;  // whether the device was nearly full, and when that was looked up
+  std::chrono::steady_clock::time_point asked_at;
 };
 static pool_state& pool() {
   static pool_state* p = new pool_state();  // (never destroyed: handles may outlive static destructors)
@@ -50,6 +57,17 @@ static void trim_locked(pool_state& P) {
     for (void* p : e.second) (void)hipFree(p);
   P.idle.clear();
   P.cached = 0;
+}
+
+static bool memory_is_short(pool_state& P) {
+  const auto now = std::chrono::steady_clock::now();
+  if (!P.asked || now - P.asked_at > std::chrono::milliseconds(100)) {
+    size_t free_b = 0, total_b = 0;
+    P.is_short = hipMemGetInfo(&free_b, &total_b) != hipSuccess || free_b < total_b / 16;
+    P.asked = true;
+    P.asked_at = now;
+  }
+  return P.is_short;
 }
 
 size_t pool_cached_bytes() {
@@ -95,10 +113,9 @@ int device_alloc(void** out, size_t bytes, bool* reused) {
     set_error("hipMalloc of %zu bytes failed: %s", size, hipGetErrorString(e));
     return 1;
   }
-  if (pooled) {
-    std::lock_guard<std::mutex> g(P.lock);
-    P.live[*out] = {dev, size};
-  }
+  std::lock_guard<std::mutex> g(P.lock);
+  if (pooled) P.live[*out] = {dev, size};
+  else P.asked = false;
   return 0;
 }
 
@@ -111,10 +128,18 @@ void device_release(void* p) {
     if (it != P.live.end()) {
       const auto key = it->second;
       P.live.erase(it);
-      if (P.cached + key.second <= POOL_CAP) {
-        P.idle[key].push_back(p);
-        P.cached += key.second;
-        return;
+      bool keep = P.cached + key.second <= POOL_CAP;
+      if (keep && P.cached + key.second > POOL_LOW && memory_is_short(P)) {
+        trim_locked(P);
+        keep = false;
+      }
+      if (keep) {
+        try {
+          P.idle[key].push_back(p);
+          P.cached += key.second;
+          return;
+        } catch (...) {  // (no memory to note it: back to the device)
+        }
       }
     }
   }
