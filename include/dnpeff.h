@@ -88,7 +88,10 @@ int dnpeff_plan_estimate(int64_t n_rows, int64_t n_cols, int64_t nnz_sparse, int
 
 /* Switches for experiments and for tests that must reach a particular code path; no counterpart
  * in the reference.  Names: dense_fill, panels, sweep_bytes, sweep_min, sweep_waves, sweep_lag,
- * sweep_spin, spmm_t_slices, split_bf16, fused_gram, h_tile_mb, tiled_h, topk_fast_cap, verbose,
+ * sweep_spin, spmm_t_slices, split_bf16, h_tile_mb, tiled_h, topk_fast_cap, verbose,
+ * fused_gram (1: ranks up to 128 run their iterations in three or four launches, and the update of H
+ * at rank 128 also produces H^T H; 0: a kernel per product), pad_rank (1: ranks above 128 that are not
+ * multiples of 128 are stored as the next multiple where that fits; 0: as they are),
  * h_overlap (1: tiled H update with A^T W of the next tile on the library stream beside the
  * update of this tile on a second stream, through two tile buffers; off by default),
  * xg_wgs (3: the update kernel of ranks from 256 with three workgroups per CU on LDS planes
@@ -354,7 +357,9 @@ int dnpeff_nmf_device_factors(dnpeff_nmf* nmf, void** W_dev, void** H_dev);
 /* Per-kernel timing with HIP events on the library stream.  enable != 0 turns
  * it on for subsequent steps; dnpeff_nmf_timings waits for the stream and
  * returns, per kernel class, summed milliseconds and launch counts since the
- * last reset.  Classes (DNPEFF_K_*) below. */
+ * last reset.  Classes (DNPEFF_K_*) below.  While it is on, ranks up to 128 run a kernel per class
+ * instead of the few launches that do several classes' work at once: the times are those of the classes,
+ * their sum is more than an iteration takes otherwise. */
 enum {
   DNPEFF_K_SPMM_N = 0,   /* A H^T                     */
   DNPEFF_K_SPMM_N_REDUCE = 1,

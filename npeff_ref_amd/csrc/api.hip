@@ -253,7 +253,10 @@ static int stored_rank(int64_t n, int64_t m, int64_t nnz, int rank, bool sweeps,
 
 // Whether the step of small ranks runs where memory allows.  (It reads the whole matrix from its own lists: no
 // dense head is split off then.  Multiples of 64 with rows enough for a dense head keep it: its kernels are made
-// for those ranks.)
+// for those ranks.  Ten iterations with head / fused: r = 128 14.7 / 16.0 ms at 1500 x 1.4M, 24.2 / 31.2 at
+// 2000 x 1.9M, 79 / 84 at 2000 x 9.8M, but 8.5 / 7.2 at 1024 x 0.8M; at r = 64, where the head is a smaller
+// part, the fused step is ahead up to 2000 rows, 11.9 / 3.1 at 1024 x 0.8M, 27.2 / 18.7 at 2000 x 1.9M: the line
+// there follows the kernels, not the clock.)
 static bool fused_step_wanted(int64_t n, int64_t m, int64_t nnz, int rank) {
   return tuning().fused_gram != 0.0 && tuning().tiled_h <= 0.0 && !(rank % 64 == 0 && n >= 1024) &&
          fused_supported(n, m, nnz, rank);

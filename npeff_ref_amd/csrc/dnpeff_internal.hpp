@@ -202,7 +202,8 @@ struct tuning_t {
   double sweep_spin = 400.0;       // polls before a workgroup of the sweep stops waiting
   double spmm_t_slices = 0.0;      // component slices of A^T W (0 = by the size of W)
   double split_bf16 = 1.0;         // matrix products on the bf16 cores with split fp32 operands (0 = fp32 cores)
-  double fused_gram = 1.0;         // rank 128: the H update also produces H^T H
+  double fused_gram = 1.0;         // ranks up to 128: the step in three or four launches (fused.hip), and at rank 128 an H update that
+                                   // also produces H^T H (0 = separate kernels for every product)
   double h_tile_mb = 768.0;        // size of a column tile of the tiled H update, MiB of the factor
   double tiled_h = -1.0;           // tiled H update: 1 = always, 0 = never, -1 = when the full-size buffer does not fit
   double topk_fast_cap = -1.0;     // top-k: candidate list length that ends the histogram passes (-1 = default)
@@ -292,7 +293,7 @@ struct fu_tile {
 };
 struct fu_chunk {
   int64_t e0;
-  int32_t len, row;
+  int32_t len;
 };
 struct fused_plan {
   fu_tile* tiles = nullptr;  // [n_tiles + 1]: the last one only ends the entries

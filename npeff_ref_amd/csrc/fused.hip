@@ -209,11 +209,11 @@ __device__ inline void fu_gram_out(const V& v, double* __restrict__ lds, float* 
 // next U are requested behind them, and a tile's first pairs and offsets while the products of the
 // tile before run: without that a tile is a chain of five dependent trips to memory.
 //
-// Bound by vector and matrix instructions (at r = 50 about 80 and 65 us of the SIMDs' time), not by
+// Bound by vector and matrix instructions (at r = 50 they hold the SIMDs for 32 and 37 % of the time), not by
 // memory: hence 32 bytes per lane and gathered row (the index arithmetic and the test for the column's
 // end are shared by eight components; with 16 bytes the r = 50 step took 335 us, now 316), 24-bit
 // multiplies into 32-bit offsets and the corrected reciprocal in place of the division sequence
-// (390 -> 335 us with it).  777 x 862k, r = 50: 181 us for 2.0 GFLOP of gathers and 12.9 of products
+// (390 -> 335 us with it).  777 x 862k, r = 50: 188 us for 2.0 GFLOP of gathers and 12.9 of products
 // (922 us for A^T W, update and Gram as separate kernels); 512 x 431k, r = 16: 31 us (139).
 // ---------------------------------------------------------------------------
 template <int Q, int R, int JB, bool TOTALS>
@@ -544,8 +544,8 @@ __global__ void __launch_bounds__(256, 2)
 
 // A H^T: chunk blockIdx.x - sum_wgs of the entries, all of one row; the wave's lane groups take them
 // round-robin, FU_U gathers each in flight.  Workgroups 0 .. sum_wgs - 1 sum Gram parts instead.
-// 777 x 862k, r = 50: 119 us for 3.9 M gathered rows of 200 bytes, nearly all of which come from the
-// memory-side cache (6.5 TB/s); 141 us as one 4-byte load per lane.
+// 777 x 862k, r = 50: 117 us for 3.9 M gathered rows of 200 bytes (6.6 TB/s), half of which the L2s hold;
+// 141 us as one 4-byte load per lane.
 template <int LPR>
 __global__ void __launch_bounds__(256)
     k_fu_n(const fu_chunk* __restrict__ chunks, const int32_t* __restrict__ colind, const float* __restrict__ vals,
@@ -775,7 +775,6 @@ __global__ void __launch_bounds__(256)
   for (int64_t k = base[i]; k < base[i + 1]; k++, e += chunk) {
     chunks[k].e0 = e;
     chunks[k].len = (int32_t)(e1 - e < chunk ? e1 - e : chunk);
-    chunks[k].row = (int32_t)i;
   }
 }
 
@@ -1092,7 +1091,9 @@ bool fused_supported(int64_t n, int64_t m, int64_t nnz, int r) {
   if (r > FUSED_NARROW_RANK && !use_split_bf16()) return false;
   // Rank 128 has kernels of its own for the update with its Gram matrix (k_xg_mu_gram_b16), and runs on
   // small factors are held to within 1e-5 of the two-pass path over 50 iterations, closer than two
-  // ways of rounding stay to each other (both are within 2e-5 of fp64): those keep the separate kernels.
+  // ways of rounding stay to each other (both are within 2e-5 of fp64): those keep the separate kernels.  That
+  // is no line of speed: ten iterations at 300 x 44,008 take 4.1 ms so and 0.88 with the fused step (0.93 at
+  // r = 127), at 500 x 83,420, past the line, 1.65.
   if (r == 128 && m < 65536) return false;
   // With as many components as rows the product can become A itself: the loss is then a difference of
   // nearly equal sums whose digits depend on the order of every sum before it.  Such runs stay on the

@@ -116,9 +116,11 @@ struct fuw_gram {
 // COLS: the H update (tiles of columns, A^T W gathered); else the W update (32 rows per workgroup, the
 // chunk sums of A H^T).  NB: blocks of 16 components.  Two barriers per tile: the Gram products of a
 // tile run between the second one and the next tile's first, beside the rows and the gathers of the next
-// tile.  1000 x 3.4 M, rank 128: 1.75 ms (matrix cores 24 % of it, other arithmetic 38 %, LDS 30 %, 7.8 TB/s
-// out of L2; 1.94 ms with the addresses kept over the loop, the descriptor asked for where it is needed
-// and the rows after the Gram products).  Eight waves of 128 registers, one block each: 1.84 ms.
+// tile.  1000 x 3.4 M, rank 128: 1.79 ms (matrix cores 25 % of it, vector instructions with theirs 42 %, LDS 31 %;
+// 1.94 ms with the addresses kept over the loop, the descriptor asked for where it is needed
+// and the rows after the Gram products).  Eight waves of 128 registers, one block each: 1.84 ms.  Infinite
+// entries of X or G leave NaN (their parts are infinity and NaN), and entries below 1e-33 lose the parts that
+// bf16 cannot hold.
 template <int NB, bool COLS>
 __global__ void __launch_bounds__(256, 2) k_fuw(const fuw_args p) {
   constexpr int NS = fuw_steps(NB), PS = 32 * NS + 8, PLANE = FUW_COLS * PS, TS = 16 * NB + 4;

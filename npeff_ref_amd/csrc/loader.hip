@@ -711,7 +711,6 @@ __global__ void __launch_bounds__(256)
   }
 }
 
-// Drops entries whose table[col] == -1 and renumbers the rest (in place on A).
 int count_columns(const int32_t* colind, int64_t nnz, int64_t n_cols, int* count) {
   DN_HIP(hipMemsetAsync(count, 0, sizeof(int) * (size_t)(n_cols > 0 ? n_cols : 1), stream()));
   hipLaunchKernelGGL(k_col_hist, dim3(grid_for(nnz, 65536)), dim3(256), 0, stream(), colind, nnz, count);
@@ -719,6 +718,7 @@ int count_columns(const int32_t* colind, int64_t nnz, int64_t n_cols, int* count
   return 0;
 }
 
+// Drops entries whose table[col] == -1 and renumbers the rest (in place on A).
 static int apply_column_table(dnpeff_csr* A, const int32_t* table, int64_t new_n_cols) {
   hipStream_t st = stream();
   dbuf<int64_t> newpos;
@@ -947,7 +947,7 @@ int64_t coarse_panels_for(int64_t n_rows, int64_t n_cols, int r, bool sweeps) {
   const double bytes = 4.0 * (double)n_cols * r;
   if (bytes >= 512e6 && n_rows >= 64) {
     // with swept pieces for the panels in between, half as many coarse panels do as well for the
-    // gathers and halve the sum over the panels (configs[1]: 19.8 -> 19.4 ms for both)
+    // gathers and halve the sum over the panels (10,000 x 65.9M, r = 128: 19.8 -> 19.4 ms for both)
     P = (int64_t)ceil(bytes / (sweeps ? 96e6 : 48e6));
     if (P < 8) P = 8;
     if (P > (sweeps ? 256 : 512)) P = sweeps ? 256 : 512;

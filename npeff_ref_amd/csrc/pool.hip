@@ -305,7 +305,7 @@ static hipError_t staged_copy(const copy_part* parts, int n_parts) {
 
 // Smaller copies go through one of a few pinned buffers, in two halves where they are longer than one.
 // (hipMemcpy of a few bytes from or to pageable memory takes 30 to 70 us here, and now and then
-// milliseconds for some MB; 15 us this way.)  Up to a page comes down through a kernel that writes to
+// milliseconds for some MB; 15 us this way.)  Up to 16 KB come down through a kernel that writes to
 // the buffer: shorter still than a copy on the engines.
 constexpr size_t BOUNCE_HALF = (size_t)1 << 20;
 constexpr size_t BOUNCE_KERNEL = 16384;

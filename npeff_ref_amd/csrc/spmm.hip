@@ -1416,7 +1416,10 @@ static int spmm_t_slices(int64_t n, int r) {
 }
 
 // Ranks above 128 (below, a wave reads several rows of W at once) with a W that an L2 holds, unless the
-// switch asks for the older kernel by its slices.
+// switch asks for the older kernel by its slices.  A^T W with / without: 24 / 184 us at 100 x 38k, r = 256, 322 /
+// 702 at 500 x 772k, 619 / 936 at 1000 x 1.4M, 568 / 1222 at 500 x 772k, r = 512, 2677 / 2860 at 1400 x 1.7M,
+// r = 1024; beside a dense head that has taken the long columns it is the other way round by 2 to 5 %: 2947 /
+// 2876 at 2000 x 6.4M, r = 256, 2546 / 2428 at 1500 x 3.4M, r = 512.
 bool spmm_t_bal_fits(int64_t n_rows, int r) {
   return r > 128 && r <= 1024 && r % 4 == 0 && tuning().spmm_t_slices == 0.0 && 4.0 * (double)n_rows * r <= 6.0e6;
 }

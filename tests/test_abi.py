@@ -129,7 +129,7 @@ def test_host_generator_row_range_matches_the_whole_matrix():
 
 def test_bench_work_model_and_sample_sizes():
     """bench.py's algorithmic bytes follow the formulas of the measurement plan, and the CPU
-    sample is the whole matrix for configs[1] and a few hundred rows for configs[3]."""
+    sample is the whole matrix for 10,000 x 110M and a few hundred rows for 20,000 x 350M."""
     import bench
 
     n, m, z, r = 20_000, 211_311_151, 5_242_880_000, 256
@@ -153,7 +153,7 @@ def test_bench_work_model_and_sample_sizes():
 
 def test_memory_plan_arithmetic_for_the_benchmark_shapes():
     """dnpeff_plan_estimate needs no GPU: the byte table of the memory plan for the shapes of
-    BASELINE configs[1], [3] and [4] as generated (kept columns, entries of the sparse part and head
+    10,000 x 110M, 20,000 x 350M and 40,000 ragged rows as generated (kept columns, entries of the sparse part and head
     columns as the full-size runs report them) follows the sizing rules, fits the 309.2 GB the
     device reports, and prices a larger head higher."""
     total = 309_220_868_096

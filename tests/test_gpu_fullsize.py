@@ -1,5 +1,5 @@
-"""The configurations that bench.py times, at their full size: BASELINE configs[1] (10,000 x
-110M, 65,536 entries per row, r = 128) and configs[3] (20,000 x 350M, 262,144 entries per row,
+"""The configurations that bench.py times, at their full size: (10,000 x
+110M, 65,536 entries per row, r = 128), (20,000 x 350M, 262,144 entries per row,
 Zipf 1.3, r = 256: 5.24e9 entries, past 2^31).  No CPU run of the whole matrix is possible at
 these sizes; instead
   * sampled rows are made again on the host by the generator's host twin, pushed through the
@@ -133,23 +133,23 @@ def test_configs1_at_full_size():
 def test_configs3_at_full_size():
     free, total = d.device_memory()
     if total < 280e9:
-        pytest.skip("configs[3] needs the 288 GB of an MI355X")
+        pytest.skip("20,000 x 350M needs the 288 GB of an MI355X")
     _full_size_checks(20_000, 350_000_000, 262_144, 1.3, 256, 43190432042, n_rows_sampled=8,
                       tiled_expected=True, tail_lists_expected=True)
 
 
 @pytest.mark.timeout(600)
 def test_configs4_ragged_rows_at_full_size():
-    """configs[4]: 40,000 rows of 1,024 ... 524,288 entries (3.34e9 in all) x 110M, r = 512."""
+    """40,000 rows of 1,024 ... 524,288 entries (3.34e9 in all) x 110M, r = 512."""
     free, total = d.device_memory()
     if total < 280e9:
-        pytest.skip("configs[4] needs the 288 GB of an MI355X")
+        pytest.skip("40,000 ragged rows at r = 512 need the 288 GB of an MI355X")
     _full_size_checks(40_000, 110_000_000, 0, 1.1, 512, 43190432042, n_rows_sampled=6, tiled_expected=True,
                       k_min=1_024, k_max=524_288, tail_lists_expected=True)
 
 
 def test_configs2_fit_path_at_full_size():
-    """configs[2]: 50,000 new examples x 65,536 entries (3.28e9, past 2^31) against a fixed sparse
+    """50,000 new examples x 65,536 entries (3.28e9, past 2^31) against a fixed sparse
     H of rank 256 over 110M features at 1 % density.  First stage: sampled rows of A H^T and the
     whole of H H^T against fp64 sums on the host; second stage: the W update works row by row, so
     the sampled rows are followed on the host in fp64 from the same seeded start, and the logged

@@ -42,7 +42,7 @@ def _run_case(n, m_full, k, r, eps, iters, seed, zipf_s=1.1, log_every=10):
 
 
 def test_config0_50_iterations_within_1e4():
-    """512 x 1,048,576, 4096 nnz/row, Zipf 1.1, r = 16, eps 1e-12, 50 its."""
+    """The smallest benchmark shape: 512 x 1,048,576, 4096 nnz/row, Zipf 1.1, r = 16, eps 1e-12, 50 its."""
     nmf, A, (W0, H0), (W, H), (W64, H64), hist, losses64 = _run_case(
         512, 1 << 20, 4096, 16, 1e-12, 50, seed=20240607)
     assert W0.min() >= 0 and W0.max() < 1 and H0.min() >= 0 and H0.max() < 1

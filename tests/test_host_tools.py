@@ -237,7 +237,7 @@ def test_sparsify_d_npeff_feeds_the_fit(tmp_path):
 
 @pytest.mark.gpu
 def test_run_nmf_on_pefs_at_a_realistic_size(tmp_path):
-    """configs[1] downscaled (1,000 examples x 16,384 values of 11M parameters, a 130 MB file made by
+    """A downscaled job (1,000 examples x 16,384 values of 11M parameters, a 130 MB file made by
     the device generator, rank 128, dense head and column panels in use): the executable's W, H and
     reduce_kept_indices equal, bit for bit, those of the same fit driven through the C ABI."""
     n, m_full, k, r, iters = 1000, 11_000_000, 16_384, 128, 10
