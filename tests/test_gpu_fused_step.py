@@ -164,3 +164,39 @@ def test_infinite_entry_stays_infinite(r):
         assert nmf.loss_terms()[2] == np.inf
         nmf.close()
         A.close()
+
+
+def test_contexts_of_several_ranks_in_turn():
+    """Contexts on one matrix whose ranks cut its columns into different tiles (64 to 256 columns each, 32, 32 with
+    the long ones alone) and one without: each goes on where it was, bit for bit as by itself."""
+    n, m, ranks = 150, 40_000, (8, 20, 50, 100, 129, 140)
+    rp, ci, va = _matrix(n, m, seed=3, fill=0.01, full=40)
+
+    def fresh(r):
+        A = d.Csr.from_host(rp, ci, va, m)
+        return A, d.MuNmf(A, d.MuNmfParams(rank=r, max_iters=1, eps=EPS, seed=5, log_every=0))
+
+    want = {}
+    for r in ranks:
+        A, nmf = fresh(r)
+        nmf.initialize()
+        nmf.step(3)
+        want[r] = (nmf.loadWToHostSync(), nmf.loadHToHostSync(), nmf.computeUncachedLoss())
+        nmf.close()
+        A.close()
+    A, first = fresh(ranks[0])
+    contexts = {ranks[0]: first}
+    for r in ranks[1:]:
+        contexts[r] = d.MuNmf(A, d.MuNmfParams(rank=r, max_iters=1, eps=EPS, seed=5, log_every=0))
+    for nmf in contexts.values():
+        nmf.initialize()
+    for _ in range(3):
+        for nmf in contexts.values():
+            nmf.update_W()
+        for nmf in reversed(contexts.values()):
+            nmf.update_H()
+    for r, nmf in contexts.items():
+        assert np.array_equal(nmf.loadWToHostSync(), want[r][0]) and np.array_equal(nmf.loadHToHostSync(), want[r][1])
+        assert nmf.computeUncachedLoss() == want[r][2]
+        nmf.close()
+    A.close()
