@@ -183,7 +183,7 @@ constexpr int64_t SPMM_T_LONG = 256;    // columns longer than this get a whole 
 int launch_spmm_n(const dnpeff_csr* A, int r, const float* H_mr, int part = 0);
 int launch_spmm_n_reduce(const dnpeff_csr* A, int r, float* N_nr);
 int launch_spmm_t(const dnpeff_csr* A, int r, const float* W_nr, float* T_mr);
-int launch_spsp(const dnpeff_csr* A, dnpeff_csr* B, float* partials);
+int launch_spsp(dnpeff_csr* A, dnpeff_csr* B, float* out_nr);
 // sparsity.hip: the sparseness projection of the columns of a row-major [n, r] factor, in place
 int sparsify_columns(int64_t n, int r, float* W, float l1, float l2, int* rounds_out);
 int launch_chunk_reduce(const dnpeff_csr* A, int r, const float* partials, float* N_nr);
@@ -330,6 +330,11 @@ struct dnpeff_csr {
   // as the sparse factor of dnpeff_op_spsp_dense: per column 32 bytes holding its first six
   // (row, value) pairs and its length (spmm.hip)
   uint4* slots = nullptr;
+  // and for its product with itself: rows in ascending column order cut at the same columns,
+  // spsp_at[row (spsp_cuts + 1) + p] = first entry of the row in cut p (spsp_cut: looked for; 0 cuts: none)
+  int64_t* spsp_at = nullptr;
+  int64_t spsp_cuts = 0;
+  bool spsp_cut = false;
   // work decomposition of A H^T: chunk_base[i] = chunks of rows before i
   int64_t* chunk_base = nullptr;
   int64_t n_chunks = 0;

@@ -778,6 +778,13 @@ static void drop_panels(dnpeff_csr* A) {
   A->plan = panel_plan();
 }
 
+static void drop_slots(dnpeff_csr* A) {
+  dfree(A->slots); A->slots = nullptr;
+  dfree(A->spsp_at); A->spsp_at = nullptr;
+  A->spsp_cuts = 0;
+  A->spsp_cut = false;
+}
+
 static void drop_derived(dnpeff_csr* A) {
   A->h_lists_valid = false;
   A->tail_declined = false;
@@ -789,7 +796,7 @@ static void drop_derived(dnpeff_csr* A) {
   dfree(A->colptr); A->colptr = nullptr;
   dfree(A->rowind); A->rowind = nullptr;
   dfree(A->tvals); A->tvals = nullptr;
-  dfree(A->slots); A->slots = nullptr;
+  drop_slots(A);
   dfree(A->chunk_base); A->chunk_base = nullptr; A->n_chunks = 0;
   dfree(A->long_cols); A->long_cols = nullptr; A->n_long = 0;
   dfree(A->partials); A->partials = nullptr; A->partials_floats = 0;
@@ -1952,7 +1959,7 @@ DN_API int dnpeff_csr_release(dnpeff_csr* A, int which) {
     dfree(A->colptr); A->colptr = nullptr;
     dfree(A->rowind); A->rowind = nullptr;
     dfree(A->tvals); A->tvals = nullptr;
-    dfree(A->slots); A->slots = nullptr;
+    drop_slots(A);
     dfree(A->long_cols); A->long_cols = nullptr; A->n_long = 0;
   } else {
     DN_CHECK(false, "which must be 1 (row-major copy) or 2 (transposed copy)");

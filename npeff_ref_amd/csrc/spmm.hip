@@ -692,6 +692,7 @@ __global__ void __launch_bounds__(256)
   const int64_t c0 = chunk_base[row], c1 = chunk_base[row + 1];
   for (int c = threadIdx.x; c < r; c += 256) {
     float s = 0.0f;
+#pragma unroll 8
     for (int64_t k = c0; k < c1; k++) s += partials[k * r + c];
     N[row * r + c] = s;
   }
@@ -1024,17 +1025,26 @@ __global__ void __launch_bounds__(256)
 // more than six) and six component ids of ten bits.  An entry of A then costs one random sector
 // instead of three dependent ones (column offsets, component ids, values); only columns longer than six
 // go on to the transposed arrays (1.5 % of them at 2.6 entries per column, where four pairs
-// per slot left 11 %).  Each wave keeps its r running sums in LDS and the lanes add into them with
-// ds_add_f32: step k of a batch applies the k-th pair of all 64 entries at once, and where two lanes
-// meet in a component the LDS adds them one after the other in lane order, the same way in every run.
+// per slot left 11 %).  Each wave keeps its r running sums in LDS and the lanes add into them: step k of
+// a batch applies the k-th pair of all 64 entries at once, and where two lanes meet in a component the LDS
+// adds them one after the other in lane order, the same way in every run.  The sums are fp64 because
+// ds_add_f64 takes 9 / 13 / 23 cycles of a CU for 16 / 32 / 64 lanes at random components where ds_add_f32
+// takes 2.7 per lane (43 / 85 / 170): with fp32 sums the LDS was taken 98 % of the time.
 // Bound by the random sectors that miss the L2s: A H^T of 65.5 M entries with 256 x 22M at 1 % takes
-// 0.88 ms (1.60 with four pairs per slot, whose second half was read only where it was needed, one
-// round trip later).  With `across` the workgroups run over the rows first and along them second: rows
-// that hold their columns in ascending order, as those of H, then look up the same part of the slots
-// at one time and find it in the memory-side cache; H H^T of that H 1.06 ms (2.36 row by row, every
-// row reading all 704 MB of slots from HBM).
+// 0.88 ms, 50 M sectors of 64 bytes at 3.5 TB/s (1.60 with four pairs per slot, whose second half was read
+// only where it was needed, one round trip later).
+//
+// H H^T (CUTS) has an order to use: rows that hold their columns in ascending order are cut at the same
+// columns, some 65,536 (2 MB of slots) apart, a wave takes one row's part of a cut, and all rows of a cut
+// run on one XCD (workgroups are dealt to the XCDs round-robin) side by side, so that the slots they share stay
+// in its L2.  Only components from the row's own up are added, its own in a register (every lane meets
+// there).  256 rows of 220 k entries, 22M columns: 0.63 ms with 14 M misses (1.07 with 61 M when the rows ran
+// side by side in chunks of equal length on all XCDs, which is what `across` still does for rows in
+// another order or of uneven parts); what is left is the L2s' line rate and the rest of long columns.
 // ---------------------------------------------------------------------------
 constexpr int SPSP_PAIRS = 6;
+constexpr int SPSP_XCDS = 8;
+constexpr int64_t SPSP_CUT_COLS = 65536;
 
 __global__ void __launch_bounds__(256)
     k_spsp_build_slots(int64_t n_cols, const int64_t* __restrict__ colptr, const int32_t* __restrict__ comp,
@@ -1054,67 +1064,138 @@ __global__ void __launch_bounds__(256)
   slots[2 * j + 1] = make_uint4(w[2], w[3], w[4], w[5]);
 }
 
-template <int VPL>
+__device__ inline void spsp_add(double* at, float v) { unsafeAtomicAdd(at, (double)v); }
+
+// *uneven |= 1 unless the columns of every row ascend
+__global__ void __launch_bounds__(256)
+    k_spsp_check_order(const int64_t* __restrict__ rowptr, const int32_t* __restrict__ colind, int* __restrict__ uneven) {
+  const int64_t e0 = rowptr[blockIdx.x], e1 = rowptr[blockIdx.x + 1];
+  bool bad = false;
+  for (int64_t e = e0 + 1 + 256 * (int64_t)blockIdx.y + threadIdx.x; e < e1; e += 256 * (int64_t)gridDim.y)
+    bad = bad || colind[e - 1] >= colind[e];
+  if (bad) atomicOr(uneven, 1);
+}
+
+// at[row (cuts + 1) + p] = first entry of the row in cut p, which starts at the column that has p / cuts of all
+// entries before it; *uneven |= 1 where a row has more than `most` entries in a cut.
+__global__ void __launch_bounds__(256)
+    k_spsp_cuts(const int64_t* __restrict__ rowptr, const int32_t* __restrict__ colind, const int64_t* __restrict__ colptr,
+                int64_t n_rows, int64_t n_cols, int64_t cuts, int64_t most, int64_t* __restrict__ at,
+                int* __restrict__ uneven) {
+  const int64_t x = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (x >= n_rows * (cuts + 1)) return;
+  const int64_t row = x / (cuts + 1), p = x % (cuts + 1), r0 = rowptr[row], r1 = rowptr[row + 1], nnz = colptr[n_cols];
+  auto first = [&](int64_t cut) {
+    if (cut >= cuts) return r1;
+    const int64_t before = nnz / cuts * cut;
+    int64_t lo = 0, hi = n_cols;
+    while (lo < hi) {
+      const int64_t mid = (lo + hi) >> 1;
+      if (colptr[mid] >= before) hi = mid; else lo = mid + 1;
+    }
+    const int64_t col = lo;
+    lo = r0;
+    hi = r1;
+    while (lo < hi) {
+      const int64_t mid = (lo + hi) >> 1;
+      if (colind[mid] >= col) hi = mid; else lo = mid + 1;
+    }
+    return lo;
+  };
+  const int64_t e = first(p);
+  at[x] = e;
+  if (p < cuts && first(p + 1) - e > most) atomicOr(uneven, 1);
+}
+
+template <int VPL, bool CUTS>
 __global__ void __launch_bounds__(256)
     k_spsp_slots(const int64_t* __restrict__ rowptr, const int32_t* __restrict__ colind,
                  const float* __restrict__ vals, const int64_t* __restrict__ chunk_base, int64_t n_rows,
                  int r, const uint4* __restrict__ slots, const int64_t* __restrict__ b_colptr,
                  const int32_t* __restrict__ b_comp, const float* __restrict__ b_vals,
-                 float* __restrict__ partials, int across) {
-  __shared__ float red[4][64 * VPL];
+                 float* __restrict__ partials, const int64_t* __restrict__ at, int64_t cuts) {
+  __shared__ double red[4][64 * VPL];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-  int64_t chunk, row;
-  if (across) {
-    row = blockIdx.x % n_rows;
-    chunk = chunk_base[row] + blockIdx.x / n_rows;
-    if (chunk >= chunk_base[row + 1]) return;
+  int64_t chunk, row, w0, e1;
+  int step;
+  if (CUTS) {  // a wave per row and cut
+    const int64_t b = blockIdx.x / SPSP_XCDS, quads = (n_rows + 3) / 4;
+    const int64_t cut = b / quads * SPSP_XCDS + blockIdx.x % SPSP_XCDS;
+    row = 4 * (b % quads) + wave;
+    if (cut >= cuts || row >= n_rows) return;
+    chunk = row * cuts + cut;
+    w0 = at[row * (cuts + 1) + cut];
+    e1 = at[row * (cuts + 1) + cut + 1];
+    step = 64;
   } else {
-    chunk = blockIdx.x;
-    row = chunk_to_row(chunk_base, n_rows, chunk);
-  }
-  const int64_t e0 = rowptr[row] + (chunk - chunk_base[row]) * SPMM_N_CHUNK;
-  int64_t e1 = e0 + SPMM_N_CHUNK;
-  if (e1 > rowptr[row + 1]) e1 = rowptr[row + 1];
-  int64_t w0 = e0 + wave * (SPMM_N_CHUNK / 4);
-  int64_t w1 = w0 + SPMM_N_CHUNK / 4;
-  if (w0 > e1) w0 = e1;
-  if (w1 > e1) w1 = e1;
-
-  float* acc = red[wave];
-#pragma unroll
-  for (int t = 0; t < VPL; t++) acc[lane + 64 * t] = 0.0f;
-
-  // (column, value) pairs one batch ahead of the slots
-  int32_t nj = w0 + lane < w1 ? colind[w0 + lane] : 0;
-  float na = w0 + lane < w1 ? vals[w0 + lane] : 0.0f;
-  for (int64_t e = w0; e < w1; e += 64) {
-    const int64_t j = nj;
-    const float a = na;
-    const bool in = e + lane < w1;
-    const uint4 s0 = slots[2 * j], s1 = slots[2 * j + 1];  // (lanes past the end: column 0, not added)
-    const int64_t en = e + 64 + lane;
-    if (en < w1) {
-      nj = colind[en];
-      na = vals[en];
+    if (cuts) {  // across
+      row = blockIdx.x % n_rows;
+      chunk = chunk_base[row] + blockIdx.x / n_rows;
+      if (chunk >= chunk_base[row + 1]) return;
+    } else {
+      chunk = blockIdx.x;
+      row = chunk_to_row(chunk_base, n_rows, chunk);
     }
+    const int64_t e0 = rowptr[row] + (chunk - chunk_base[row]) * SPMM_N_CHUNK;
+    e1 = e0 + SPMM_N_CHUNK;
+    if (e1 > rowptr[row + 1]) e1 = rowptr[row + 1];
+    w0 = e0 + 64 * wave;
+    step = 256;
+  }
+
+  double* acc = red[wave];
+#pragma unroll
+  for (int t = 0; t < VPL; t++) acc[lane + 64 * t] = 0.0;
+
+  // the slots of the next batch are on their way while a batch is added up, and the pairs of the one after
+  const int64_t last = e1 - 1;
+  auto pair = [&](int64_t e, int32_t& j, float& a) {
+    const int64_t at = e + lane < e1 ? e + lane : last;
+    j = colind[at];
+    a = vals[at];
+  };
+  int32_t j0 = 0, j1 = 0, j2 = 0;
+  float a0 = 0.0f, a1 = 0.0f, a2 = 0.0f;
+  uint4 s0 = {}, s1 = {}, t0, t1;
+  if (w0 < e1) {
+    pair(w0, j0, a0);
+    pair(w0 + step, j1, a1);
+    s0 = slots[2 * (int64_t)j0];
+    s1 = slots[2 * (int64_t)j0 + 1];
+  }
+  double own = 0.0;  // (CUTS) the row with itself
+  auto add = [&](int c, float v) {
+    if (!CUTS || c > (int)row) spsp_add(&acc[c], v);
+    else if (c == (int)row) own += (double)v;
+  };
+  for (int64_t e = w0; e < e1; e += step) {
+    t0 = slots[2 * (int64_t)j1];
+    t1 = slots[2 * (int64_t)j1 + 1];
+    pair(e + 2 * step, j2, a2);
     const uint64_t ids = ((uint64_t)s0.w << 32) | s0.z;
-    const int len = in ? (int)(ids & 15u) : 0;
+    const int len = e + lane < e1 ? (int)(ids & 15u) : 0;
     const unsigned v[SPSP_PAIRS] = {s0.x, s0.y, s1.x, s1.y, s1.z, s1.w};
 #pragma unroll
     for (int k = 0; k < SPSP_PAIRS; k++)
-      if (len > k) atomicAdd(&acc[(ids >> (4 + 10 * k)) & 1023u], a * __uint_as_float(v[k]));
+      if (len > k) add((int)((ids >> (4 + 10 * k)) & 1023u), a0 * __uint_as_float(v[k]));
     if (len > SPSP_PAIRS) {
-      const int64_t q1 = b_colptr[j + 1];
-      for (int64_t q = b_colptr[j] + SPSP_PAIRS; q < q1; q++) atomicAdd(&acc[b_comp[q]], a * b_vals[q]);
+      const int64_t q1 = b_colptr[(int64_t)j0 + 1];
+      for (int64_t q = b_colptr[j0] + SPSP_PAIRS; q < q1; q++) add(b_comp[q], a0 * b_vals[q]);
     }
+    j0 = j1; a0 = a1; s0 = t0; s1 = t1;
+    j1 = j2; a1 = a2;
+  }
+  if (CUTS) {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) own += __shfl_xor(own, off);
+    for (int c = lane; c < r; c += 64)
+      if (c >= (int)row) partials[chunk * r + c] = (float)(c == (int)row ? own : acc[c]);
+    return;
   }
   __syncthreads();
   for (int c = threadIdx.x; c < r; c += 256) {
-    float s = red[0][c];
-    s += red[1][c];
-    s += red[2][c];
-    s += red[3][c];
-    partials[chunk * r + c] = s;
+    partials[chunk * r + c] = (float)(((red[0][c] + red[1][c]) + red[2][c]) + red[3][c]);
   }
 }
 
@@ -1548,29 +1629,95 @@ int launch_spmm_t_tile(const dnpeff_csr* A_full, int r, const float* W_nr, int64
   return launch_head_t_scatter(A_full, r, k0, k1, col0, T_tile);
 }
 
-int launch_spsp(const dnpeff_csr* A, dnpeff_csr* B, float* partials) {
+// out = the cuts' sums of B B^T, of which they hold the upper triangle: 16 components of a row, 16 threads each.
+__global__ void __launch_bounds__(256)
+    k_spsp_sum_cuts(int r, int64_t cuts, const float* __restrict__ partials, float* __restrict__ out) {
+  __shared__ double red[256];
+  const int row = blockIdx.y, c = 16 * blockIdx.x + (threadIdx.x & 15), k = threadIdx.x >> 4;
+  if (16 * (int)blockIdx.x + 15 < row) return;
+  const bool in = c >= row && c < r;
+  const float* p = partials + (int64_t)row * cuts * r + (in ? c : row);
+  double s = 0.0;
+#pragma unroll 8
+  for (int64_t q = k; q < cuts; q += 16) s += (double)p[q * r];
+  red[threadIdx.x] = s;
+  __syncthreads();
+  if (k == 0 && in) {
+    for (int u = 1; u < 16; u++) s += red[16 * u + threadIdx.x];
+    out[(int64_t)row * r + c] = (float)s;
+    out[(int64_t)c * r + row] = (float)s;
+  }
+}
+
+// Cuts for B B^T, or none: with fewer than 16 cuts (1 M columns, 32 MB of slots) an XCD would not have two,
+// below 256 entries a wave's sums cost more than its entries, and from 4 times a cut's share on (rows of
+// uneven length, blocks of columns of their own) its longest wave would be waited for.
+static int spsp_make_cuts(dnpeff_csr* B) {
+  const int64_t n = B->n_rows, m = B->n_cols;
+  B->spsp_cut = true;
+  if (n < 1 || n > 1024 || !xcd_round_robin()) return 0;
+  const int64_t per_row = B->nnz / n;
+  const int64_t cuts = std::min(std::max(m / SPSP_CUT_COLS, per_row / 2048), per_row / 256);
+  if (cuts < 2 * SPSP_XCDS) return 0;
+  dbuf<int64_t> at;
+  dbuf<int> uneven;
+  DN_TRY(at.alloc(n * (cuts + 1)));
+  DN_TRY(uneven.alloc(1));
+  DN_HIP(hipMemsetAsync(uneven.p, 0, sizeof(int), stream()));
+  hipLaunchKernelGGL(k_spsp_check_order, dim3((unsigned)n, 16), dim3(256), 0, stream(), B->rowptr, B->colind, uneven.p);
+  hipLaunchKernelGGL(k_spsp_cuts, dim3((unsigned)ceil_div(n * (cuts + 1), 256)), dim3(256), 0, stream(), B->rowptr,
+                     B->colind, B->colptr, n, m, cuts, 4 * ceil_div(per_row, cuts), at.p, uneven.p);
+  DN_LAUNCH_CHECK();
+  int bad = 0;
+  DN_HIP(copy_down(&bad, uneven.p, sizeof(int)));
+  if (bad) return 0;
+  B->spsp_at = at.release();
+  B->spsp_cuts = cuts;
+  return 0;
+}
+
+int launch_spsp(dnpeff_csr* A, dnpeff_csr* B, float* out_nr) {
   const int r = (int)B->n_rows;
   DN_CHECK(r >= 1 && r <= MAX_RANK, "rank %d outside [1, %d]", r, MAX_RANK);
   DN_CHECK(A->rowptr && A->chunk_base, "matrix has no row-major copy / work list");
   DN_CHECK(B->colptr != nullptr, "sparse factor has no transposed copy");
   DN_CHECK(A->n_cols == B->n_cols, "column counts differ (%lld vs %lld)", (long long)A->n_cols,
            (long long)B->n_cols);
-  if (A->n_chunks == 0) return 0;
   if (!B->slots && B->n_cols > 0) {
     DN_TRY(dmalloc(&B->slots, 2 * B->n_cols));
     hipLaunchKernelGGL(k_spsp_build_slots, dim3((unsigned)ceil_div(B->n_cols, 256)), dim3(256), 0, stream(),
                        B->n_cols, B->colptr, B->rowind, B->tvals, B->slots);
     DN_LAUNCH_CHECK();
   }
+  if (A == B && !B->spsp_cut) DN_TRY(spsp_make_cuts(B));
+  bool by_cuts = A == B && B->spsp_cuts > 0;
+  const int64_t need = B->spsp_cuts * B->n_rows * r;
+  if (by_cuts && A->partials_floats < need) {
+    float* more = nullptr;
+    if (dmalloc(&more, need) == 0) {
+      dfree(A->partials);
+      A->partials = more;
+      A->partials_floats = need;
+    } else {
+      clear_error();
+      by_cuts = false;
+    }
+  }
+  float* partials = A->partials;
   dim3 grid((unsigned)A->n_chunks), block(256);
-  // H H^T: its rows are of about the same length (at most as many empty workgroups as real ones) and
-  // keep their columns in order
+  // otherwise its rows are of about the same length (at most as many empty workgroups as real ones), or the
+  // chunks go row by row
   const int64_t spread = A->max_row_chunks * A->n_rows;
-  const int across = A == B && A->max_row_chunks > 0 && spread <= 2 * A->n_chunks && spread < (int64_t)INT32_MAX;
-  if (across) grid = dim3((unsigned)spread);
-#define DN_SPSP(V)                                                                               \
-  hipLaunchKernelGGL((k_spsp_slots<V>), grid, block, 0, stream(), A->rowptr, A->colind, A->vals,   \
-                     A->chunk_base, A->n_rows, r, B->slots, B->colptr, B->rowind, B->tvals, partials, across)
+  const bool across = A == B && A->max_row_chunks > 0 && spread <= 2 * A->n_chunks && spread < (int64_t)INT32_MAX;
+  if (by_cuts) grid = dim3((unsigned)(ceil_div(B->spsp_cuts, SPSP_XCDS) * SPSP_XCDS * ceil_div(B->n_rows, 4)));
+  else if (across) grid = dim3((unsigned)spread);
+  if (grid.x == 0) return launch_chunk_reduce(A, r, partials, out_nr);
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, block, 0, stream(), A->rowptr, A->colind, A->vals, A->chunk_base, A->n_rows, r,
+                       B->slots, B->colptr, B->rowind, B->tvals, partials, B->spsp_at,
+                       by_cuts ? B->spsp_cuts : (int64_t)across);
+  };
+#define DN_SPSP(V) by_cuts ? go(k_spsp_slots<V, true>) : go(k_spsp_slots<V, false>)
   switch (vpl_for(r)) {
     case 1: DN_SPSP(1); break;
     case 2: DN_SPSP(2); break;
@@ -1579,6 +1726,10 @@ int launch_spsp(const dnpeff_csr* A, dnpeff_csr* B, float* partials) {
     default: DN_SPSP(16); break;
   }
 #undef DN_SPSP
+  DN_LAUNCH_CHECK();
+  if (!by_cuts) return launch_chunk_reduce(A, r, partials, out_nr);
+  hipLaunchKernelGGL(k_spsp_sum_cuts, dim3((unsigned)ceil_div(r, 16), (unsigned)r), block, 0, stream(), r, B->spsp_cuts,
+                     partials, out_nr);
   DN_LAUNCH_CHECK();
   return 0;
 }
@@ -1684,6 +1835,5 @@ DN_API int dnpeff_op_spsp_dense(dnpeff_csr* A, dnpeff_csr* B, float* out_nr) {
   DN_TRY(dnpeff_csr_build_transpose(B));
   const int r = (int)B->n_rows;
   DN_TRY(csr_ensure_partials(A, r));
-  DN_TRY(launch_spsp(A, B, A->partials));
-  return launch_chunk_reduce(A, r, A->partials, out_nr);
+  return launch_spsp(A, B, out_nr);
 }

@@ -58,3 +58,30 @@ def test_products_with_short_and_long_columns(r, per_col):
     assert _rel(AH.numpy(), orc.spsp_dense_f64(A, m, B, r)) < 2e-6
     assert _rel(HH.numpy(), orc.spsp_dense_f64(B, m, B, r)) < 2e-6
     assert np.array_equal(HH.numpy(), HH2.numpy())
+
+
+@pytest.mark.parametrize("r,order", [(2, "up"), (37, "up"), (70, "up"), (37, "mixed"), (37, "blocks")])
+def test_h_ht_in_cuts_of_columns(r, order):
+    """H H^T where the rows are cut at the same columns (17 cuts, in which only the components from the
+    row's own up are added), and rows that are not in order or each in a block of columns of its own, which
+    are not cut.  Some columns hold more than the six entries of a slot.  The products and sums of positive numbers are
+    rounded a few times each: 2e-6.  Symmetric, and two runs give the same bits."""
+    rng = np.random.default_rng(r)
+    m, k = 17 * 65536 + 5, 17 * 256 + 9
+    few = np.arange(0, m, m // 300)  # columns that every row has
+    rows = []
+    for i in range(r):
+        lo, hi = (m * i // r, m * (i + 1) // r) if order == "blocks" else (0, m)
+        c = np.unique(np.concatenate([few, rng.choice(hi - lo, min(k, hi - lo), replace=False) + lo]))
+        rows.append(rng.permutation(c) if order == "mixed" else c)
+    rowptr = np.concatenate(([0], np.cumsum([len(c) for c in rows]))).astype(np.int64)
+    B = (rowptr, np.concatenate(rows).astype(np.int32), rng.lognormal(0, 1, rowptr[-1]).astype(np.float32))
+    cH = d.Csr.from_host(*B, m)
+    HH, HH2 = d.DeviceArray((r, r)), d.DeviceArray((r, r))
+    d.op_spsp_dense(cH, cH, HH)
+    d.op_spsp_dense(cH, cH, HH2)
+    got = HH.numpy()
+    np.testing.assert_allclose(got, orc.spsp_dense_f64(B, m, B, r), rtol=2e-6)
+    assert np.array_equal(got, HH2.numpy())
+    if order == "up":
+        assert np.array_equal(got, got.T)
