@@ -26,7 +26,9 @@
 namespace dn {
 
 constexpr int FU_ROWS_WG = 64;       // rows of a workgroup of the W update
-constexpr int FU_SUM_DIRECT = 4;     // partial Gram matrices that their reader sums by itself
+// Partial Gram matrices of W that the H update sums by itself (5 of them at 300 x 146k, r = 20: half a us where k_fu_sum
+// takes 3.3; above two blocks every workgroup would read 80 KB).
+constexpr int fu_sum_direct(int nb) { return nb > 2 ? 4 : 8; }
 
 __host__ __device__ constexpr int fu_blocks(int Q, int R) { return Q + (R ? 1 : 0); }
 // Lanes that cover a row of W with two 16-byte pieces each.
@@ -35,14 +37,44 @@ __host__ __device__ constexpr int fu_lpr(int Q, int R) {
 }
 
 // G as the A operand of the products: [block b of output components][contraction block q][lane][i].
-// part: n_parts partial matrices of packed upper block pairs ([pair][16][16]).
-// (Every thread's numbers of one part are asked for together: one after the other, with the parts inside, the
-// prologue took half of an H update of 145 k columns.)
+// part: n_parts partial matrices of packed upper block pairs ([pair][16][16]), summed in fp64 in order.
+// They are read in 16-byte pieces, up to eight parts at a time, and come to their places through `stage` (as
+// much LDS as a packed matrix, free again when this returns): with every thread picking its numbers from memory
+// the vector-memory unit was busy for 16 lines per load (5 parts, 300 x 146k, r = 20: H update 23.6 us, now 20.0).
 template <int Q, int R>
-__device__ inline void fu_load_g(const float* __restrict__ part, int n_parts, int r, float* __restrict__ ga) {
-  constexpr int NB = fu_blocks(Q, R), S = fu_pairs(NB) * 256, N = NB * NB;
-  int at[N];
-  double sum[N];
+__device__ inline void fu_load_g(const float* __restrict__ part, int n_parts, int r, float* __restrict__ ga,
+                                 float* __restrict__ stage) {
+  constexpr int NB = fu_blocks(Q, R), S = fu_pairs(NB) * 256, N = NB * NB, P = NB > 2 ? 4 : 8;
+  if constexpr (NB == 1) {  // (one number per thread: no detour)
+    const int i = threadIdx.x & 3, rho = (threadIdx.x >> 2) & 15, g = threadIdx.x >> 6;
+    const int k = R == 0 ? 4 * g + i : R * g + i, c = R == 0 ? rho : R * (rho >> 2) + (rho & 3);
+    const bool ok = k < r && c < r && (R == 0 || (i < R && (rho & 3) < R));
+    double sum = 0.0;
+    for (int p = 0; p < n_parts; p += P) {
+      float v[P];
+#pragma unroll
+      for (int u = 0; u < P; u++) v[u] = part[(int64_t)(p + u < n_parts ? p + u : p) * S + (ok ? k * 16 + c : 0)];
+#pragma unroll
+      for (int u = 0; u < P; u++) sum += p + u < n_parts ? (double)v[u] : 0.0;
+    }
+    ga[threadIdx.x] = ok ? (float)sum : 0.0f;
+    return;
+  }
+#pragma unroll
+  for (int x = 4 * (int)threadIdx.x; x < S; x += 1024) {
+    double sum[4] = {};
+    for (int p = 0; p < n_parts; p += P) {
+      f32x4 v[P];
+#pragma unroll
+      for (int k = 0; k < P; k++) v[k] = *reinterpret_cast<const f32x4*>(part + (int64_t)(p + k < n_parts ? p + k : p) * S + x);
+#pragma unroll
+      for (int k = 0; k < P; k++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) sum[i] += p + k < n_parts ? (double)v[k][i] : 0.0;
+    }
+    *reinterpret_cast<f32x4*>(stage + x) = f32x4{(float)sum[0], (float)sum[1], (float)sum[2], (float)sum[3]};
+  }
+  __syncthreads();
 #pragma unroll
   for (int u = 0; u < N; u++) {
     const int i = threadIdx.x & 3, lane = (threadIdx.x >> 2) & 63, q = u % NB, b = u / NB;
@@ -57,19 +89,9 @@ __device__ inline void fu_load_g(const float* __restrict__ part, int n_parts, in
     const int bk = k >> 4, bc = c >> 4;
     const int x = bk <= bc ? fu_pair(bk, bc, NB) * 256 + (k & 15) * 16 + (c & 15)
                            : fu_pair(bc, bk, NB) * 256 + (c & 15) * 16 + (k & 15);
-    at[u] = ok ? x : -1;
-    sum[u] = 0.0;
+    ga[threadIdx.x + 256 * u] = ok ? stage[x] : 0.0f;
   }
-  for (int p = 0; p < n_parts; p++) {
-    const float* src = part + (int64_t)p * S;
-    float v[N];
-#pragma unroll
-    for (int u = 0; u < N; u++) v[u] = src[at[u] < 0 ? 0 : at[u]];
-#pragma unroll
-    for (int u = 0; u < N; u++) sum[u] += (double)v[u];
-  }
-#pragma unroll
-  for (int u = 0; u < N; u++) ga[threadIdx.x + 256 * u] = at[u] < 0 ? 0.0f : (float)sum[u];
+  __syncthreads();
 }
 
 // The components of one factor row that a lane holds: x[b][i] = row[component(b, g, i)], zero past r.
@@ -93,10 +115,25 @@ __device__ inline void fu_load_row(const float* __restrict__ row, int g, int r, 
   }
 }
 
+// past: the new rows go past the L2s, which write back what is left in them when the launch ends.  H update with /
+// without: 18.4 / 19.9 us at 300 x 146k, r = 20, 30.7 / 31.4 at 512 x 431k, r = 16; a factor that the memory-side
+// cache would hold in part is better left to it (777 x 862k, r = 50, 172 MB: ten iterations 3.35 / 3.32 ms).
+constexpr int64_t FU_PAST_BYTES = 64 << 20;
+template <bool PAST>
+__device__ inline void fu_store(float* dst, float v) {
+  if constexpr (PAST) __builtin_nontemporal_store(v, dst);
+  else *dst = v;
+}
+template <bool PAST>
+__device__ inline void fu_store4(float* dst, const f32x4& v) {
+  if constexpr (PAST) __builtin_nontemporal_store(f32x4u(v), reinterpret_cast<f32x4u*>(dst));
+  else *reinterpret_cast<f32x4u*>(dst) = v;
+}
+
 // X G, the update and the new row for the 16 rows of a wave.  t: the numerators of the lane's row, laid
 // out as x.  The new rows go to `dst` (global, if store) and into the wave's part of the LDS tile
 // ([row][component], stride TS), from where they enter the Gram products.
-template <int Q, int R>
+template <int Q, int R, bool PAST = false>
 __device__ inline void fu_update(const float* __restrict__ ga, f32x4 (&x)[fu_blocks(Q, R)],
                                  const f32x4 (&t)[fu_blocks(Q, R)], float eps, int r, bool store,
                                  float* __restrict__ dst, float* __restrict__ tile_row) {
@@ -129,11 +166,11 @@ __device__ inline void fu_update(const float* __restrict__ ga, f32x4 (&x)[fu_blo
     if (b < Q) {
       *reinterpret_cast<f32x4*>(tile_row + 16 * b + 4 * g) = y;
       if (store) {
-        if (R > 0 || b < Q - 1 || 16 * b + 4 * g + 3 < r) *reinterpret_cast<f32x4u*>(dst + 16 * b + 4 * g) = y;
+        if (R > 0 || b < Q - 1 || 16 * b + 4 * g + 3 < r) fu_store4<PAST>(dst + 16 * b + 4 * g, y);
         else {
 #pragma unroll
           for (int i = 0; i < 4; i++)
-            if (16 * b + 4 * g + i < r) dst[16 * b + 4 * g + i] = y[i];
+            if (16 * b + 4 * g + i < r) fu_store<PAST>(dst + 16 * b + 4 * g + i, y[i]);
         }
       }
     } else {
@@ -141,7 +178,7 @@ __device__ inline void fu_update(const float* __restrict__ ga, f32x4 (&x)[fu_blo
       for (int i = 0; i < R; i++) {
         const int c = 16 * Q + R * g + i;
         tile_row[c] = y[i];
-        if (store && c < r) dst[c] = y[i];
+        if (store && c < r) fu_store<PAST>(dst + c, y[i]);
       }
     }
   }
@@ -177,10 +214,32 @@ __device__ inline void fu_gram_fold(double (&sum)[NP][4], f32x4 (&acc)[NP]) {
     }
 }
 
-// The four waves' Gram blocks, added in fp64 in wave order, to out ([pair][16][16]); lds: NP * 256 doubles.
-template <int NP, class V>
-__device__ inline void fu_gram_out(const V& v, double* __restrict__ lds, float* __restrict__ out) {
+// The four waves' Gram blocks, added in fp64 in wave order, to out ([pair][16][16]).  All waves' blocks through
+// LDS at once where the tile's share of it holds them (fu_out_floats); else one wave after the other.
+template <int NP, class T>
+constexpr int fu_out_floats(int room) {
+  return NP * 1024 * (int)(sizeof(T) / sizeof(float)) <= room ? NP * 1024 * (int)(sizeof(T) / sizeof(float)) : NP * 512;
+}
+template <int NP, int ROOM, class T, class V>
+__device__ inline void fu_gram_out(const V& v, float* __restrict__ lds, float* __restrict__ out) {
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, l16 = lane & 15, g = lane >> 4;
+  if constexpr (fu_out_floats<NP, T>(ROOM) > NP * 512) {
+    T* all = reinterpret_cast<T*>(lds);
+    __syncthreads();
+#pragma unroll
+    for (int p = 0; p < NP; p++)
+#pragma unroll
+      for (int i = 0; i < 4; i++) all[(wave * NP + p) * 256 + (4 * g + i) * 16 + l16] = v[p][i];
+    __syncthreads();
+    for (int x = threadIdx.x; x < NP * 256; x += 256) {
+      double s = (double)all[x];
+#pragma unroll
+      for (int w = 1; w < 4; w++) s += (double)all[w * NP * 256 + x];
+      out[x] = (float)s;
+    }
+    return;
+  }
+  double* sum = reinterpret_cast<double*>(lds);
   for (int w = 0; w < 4; w++) {
     __syncthreads();
     if (wave == w) {
@@ -188,13 +247,13 @@ __device__ inline void fu_gram_out(const V& v, double* __restrict__ lds, float* 
       for (int p = 0; p < NP; p++)
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-          double* at = lds + p * 256 + (4 * g + i) * 16 + l16;
+          double* at = sum + p * 256 + (4 * g + i) * 16 + l16;
           *at = w == 0 ? (double)v[p][i] : *at + (double)v[p][i];
         }
     }
   }
   __syncthreads();
-  for (int x = threadIdx.x; x < NP * 256; x += 256) out[x] = (float)lds[x];
+  for (int x = threadIdx.x; x < NP * 256; x += 256) out[x] = (float)sum[x];
 }
 
 // ---------------------------------------------------------------------------
@@ -214,16 +273,18 @@ __device__ inline void fu_gram_out(const V& v, double* __restrict__ lds, float* 
 // end are shared by eight components; with 16 bytes the r = 50 step took 335 us, now 316), 24-bit
 // multiplies into 32-bit offsets and the corrected reciprocal in place of the division sequence
 // (390 -> 335 us with it).  777 x 862k, r = 50: 188 us for 2.0 GFLOP of gathers and 12.9 of products
-// (922 us for A^T W, update and Gram as separate kernels); 512 x 431k, r = 16: 31 us (139).
+// (922 us for A^T W, update and Gram as separate kernels); 512 x 431k, r = 16: 31 us (139); 300 x 146k,
+// r = 20: 18.4, of which a workgroup has 12 us (prologue 2.8, rows and gathers 4 to 8, products and stores 3.5).
 // ---------------------------------------------------------------------------
-template <int Q, int R, int JB, bool TOTALS>
+template <int Q, int R, int JB, bool TOTALS, bool PAST>
 __global__ void __launch_bounds__(256, fu_blocks(Q, R) <= 2 ? 4 : 3)
     k_fu_h(const fu_tile* __restrict__ tiles, int n_tiles, const int64_t* __restrict__ colptr,
            const uint2* __restrict__ pairs, int r, const float* __restrict__ W, float* __restrict__ H, float eps,
            const float* __restrict__ gw, int n_gw, float* __restrict__ gpart) {
   constexpr int NB = fu_blocks(Q, R), NP = fu_pairs(NB), TS = 16 * NB + 4, TC = 64 * JB;
   using Gather = fu_gather<TC, TS, NB, fu_lpr(Q, R)>;
-  constexpr int T_FLOATS = Gather::CARRY + 2048 > NP * 512 ? Gather::CARRY + 2048 : NP * 512;
+  using Out = std::conditional_t<TOTALS, double, float>;
+  constexpr int ROOM = Gather::CARRY + 2048, T_OUT = fu_out_floats<NP, Out>(ROOM), T_FLOATS = ROOM > T_OUT ? ROOM : T_OUT;
   __shared__ __align__(16) float ga[NB * NB * 256];
   __shared__ __align__(16) float tile[T_FLOATS];
   __shared__ int cps[2][TC + 1];
@@ -245,12 +306,15 @@ __global__ void __launch_bounds__(256, fu_blocks(Q, R) <= 2 ? 4 : 3)
       cpv[k] = colptr[d.col0 + (at < d.nc ? at : d.nc)];
     }
   };
+  // (round by round in turn: where the long columns are the first or the last, who had a full tile gets an
+  // empty one or none)
+  auto tile_of = [&](int k) { return k * (int)gridDim.x + (k & 1 ? (int)(gridDim.x - 1 - blockIdx.x) : (int)blockIdx.x); };
   fu_tile_at td = fu_describe<Gather::NG>(tiles, n_tiles, blockIdx.x);
   request(td);
-  fu_load_g<Q, R>(gw, n_gw, r, ga);
+  fu_load_g<Q, R>(gw, n_gw, r, ga, tile);
 
   int par = 0;
-  for (int tl = blockIdx.x; tl < n_tiles; tl += gridDim.x, par ^= 1) {
+  for (int k = 0; tile_of(k) < n_tiles; k++, par ^= 1) {
     const int l0 = td.col0 & (TC - 1);
     const int nc = td.nc, share = td.share;
     int* cp = cps[par];
@@ -259,7 +323,7 @@ __global__ void __launch_bounds__(256, fu_blocks(Q, R) <= 2 ? 4 : 3)
       const int at = tid + 256 * k;
       if (at <= nc) cp[l0 + at] = (int)(cpv[k] - td.e0);
     }
-    const fu_tile_at nd = fu_describe<Gather::NG>(tiles, n_tiles, tl + gridDim.x);
+    const fu_tile_at nd = fu_describe<Gather::NG>(tiles, n_tiles, tile_of(k + 1));
     // the wave's rows of H
     const int64_t base = td.col0 - l0;
     float* Hb = H + base * r;
@@ -324,7 +388,7 @@ __global__ void __launch_bounds__(256, fu_blocks(Q, R) <= 2 ? 4 : 3)
           }
         }
       }
-      fu_update<Q, R>(ga, h[jb], t, eps, r, mine[jb], Hb + hoff[jb], trow);
+      fu_update<Q, R, PAST>(ga, h[jb], t, eps, r, mine[jb], Hb + hoff[jb], trow);
       __builtin_amdgcn_wave_barrier();
       fu_gram<NB>(tile + first * TS, TS, acc);
     }
@@ -332,10 +396,9 @@ __global__ void __launch_bounds__(256, fu_blocks(Q, R) <= 2 ? 4 : 3)
     td = nd;
     __syncthreads();  // (the tile has been read)
   }
-  double* lds = reinterpret_cast<double*>(tile);
   float* out = gpart + (int64_t)blockIdx.x * (NP * 256);
-  if constexpr (TOTALS) fu_gram_out<NP>(sum, lds, out);
-  else fu_gram_out<NP>(acc, lds, out);
+  if constexpr (TOTALS) fu_gram_out<NP, ROOM, double>(sum, tile, out);
+  else fu_gram_out<NP, ROOM, float>(acc, tile, out);
 }
 
 // W update: 64 rows per workgroup.  n_base (or NULL: N holds A H^T itself): first chunk of every row.
@@ -344,29 +407,32 @@ __global__ void __launch_bounds__(256)
     k_fu_w(int64_t n, int r, const int* __restrict__ n_base, const float* __restrict__ N, float* __restrict__ W,
            float eps, const float* __restrict__ gh, int n_gh, float* __restrict__ gpart) {
   constexpr int NB = fu_blocks(Q, R), NP = fu_pairs(NB), TS = 16 * NB + 4;
-  constexpr int T_FLOATS = FU_ROWS_WG * TS > NP * 512 ? FU_ROWS_WG * TS : NP * 512;
+  constexpr int T_OUT = NP * 1024, T_FLOATS = FU_ROWS_WG * TS > T_OUT ? FU_ROWS_WG * TS : T_OUT;
   __shared__ __align__(16) float ga[NB * NB * 256];
   __shared__ __align__(16) float tile[T_FLOATS];
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, l16 = lane & 15, g = lane >> 4;
   const int64_t row0 = (int64_t)blockIdx.x * FU_ROWS_WG;
   const int64_t i = row0 + 16 * wave + l16;
   const bool mine = i < n;
+  const int64_t at = mine ? i : row0;
+  const int k0 = n_base ? n_base[at] : (int)at, k1 = n_base ? n_base[at + 1] : (int)at + 1;
   f32x4 x[NB], t[NB];
-  float* wrow = W + (mine ? i : row0) * r;
+  float* wrow = W + at * r;
   fu_load_row<Q, R>(wrow, g, r, x);
-  fu_load_g<Q, R>(gh, n_gh, r, ga);
+  fu_load_g<Q, R>(gh, n_gh, r, ga, tile);
 #pragma unroll
   for (int b = 0; b < NB; b++) t[b] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-  {
-    const int64_t at = mine ? i : row0;
-    const int64_t k0 = n_base ? n_base[at] : at, k1 = n_base ? n_base[at + 1] : at + 1;
-#pragma unroll 4
-    for (int64_t k = k0; k < k1; k++) {
-      f32x4 p[NB];
-      fu_load_row<Q, R>(N + k * r, g, r, p);
+  constexpr int U = 4;  // chunk sums asked for at a time (one by one they are a chain of trips to memory)
+  for (int k = k0; k < k1; k += U) {
+    f32x4 p[U][NB];
 #pragma unroll
-      for (int b = 0; b < NB; b++) t[b] += p[b];
-    }
+    for (int u = 0; u < U; u++) fu_load_row<Q, R>(N + (int64_t)(k + u < k1 ? k + u : k) * r, g, r, p[u]);
+#pragma unroll
+    for (int u = 0; u < U; u++)
+#pragma unroll
+      for (int b = 0; b < NB; b++)
+#pragma unroll
+        for (int c = 0; c < 4; c++) t[b][c] += k + u < k1 ? p[u][b][c] : 0.0f;
   }
   f32x4 acc[NP];
 #pragma unroll
@@ -375,7 +441,7 @@ __global__ void __launch_bounds__(256)
   fu_update<Q, R>(ga, x, t, eps, r, mine, wrow, tile + (16 * wave + l16) * TS);
   __builtin_amdgcn_wave_barrier();
   fu_gram<NB>(tile + 16 * wave * TS, TS, acc);
-  fu_gram_out<NP>(acc, reinterpret_cast<double*>(tile), gpart + (int64_t)blockIdx.x * (NP * 256));
+  fu_gram_out<NP, T_OUT, float>(acc, tile, gpart + (int64_t)blockIdx.x * (NP * 256));
 }
 
 // Element x of the sum of n_parts partial Gram matrices: 16 elements per workgroup, 16 threads each.
@@ -415,7 +481,7 @@ template <int NB>
 __global__ void __launch_bounds__(256)
     k_fu_gram(const float* __restrict__ X, int64_t rows, int64_t per, int r, float* __restrict__ gpart) {
   constexpr int NP = fu_pairs(NB);
-  __shared__ double lds[NP * 256];
+  __shared__ __align__(16) float lds[NP * 512];
   const int64_t row0 = blockIdx.x * per, row1 = row0 + per < rows ? row0 + per : rows;
   const int lane = threadIdx.x & 63, l16 = lane & 15, g = lane >> 4;
   float a[4][NB], nx[4][NB];
@@ -450,7 +516,7 @@ __global__ void __launch_bounds__(256)
     if (k % 16 == 0) fu_gram_fold<NP>(sum, acc);
   }
   fu_gram_fold<NP>(sum, acc);
-  fu_gram_out<NP>(sum, lds, gpart + (int64_t)blockIdx.x * (NP * 256));
+  fu_gram_out<NP, 0, double>(sum, lds, gpart + (int64_t)blockIdx.x * (NP * 256));
 }
 
 // 5 to 8 blocks: all waves take the same rows, 32 at a time through LDS (rows 16 banks apart: the four
@@ -909,14 +975,18 @@ using fu_h_kernel = void (*)(const fu_tile*, int, const int64_t*, const uint2*, 
 // time).  Up to 16 components always.  Up to 32 where a workgroup has more than one tile: the totals leave room
 // for four workgroups per CU instead of five, which one tile each would notice (300 x 146k, r = 20: 21.8 against
 // 19.6 us) and has no use for.  Above, the registers hold the fp32 sums only.
-template <int Q, int R>
+template <int Q, int R, bool PAST>
 static fu_h_kernel fu_h_of(int tile_cols, bool totals) {
   constexpr int NB = fu_blocks(Q, R);
-  if constexpr (NB == 1) return tile_cols == 256 ? k_fu_h<Q, R, 4, true> : k_fu_h<Q, R, 1, true>;
+  if constexpr (NB == 1) return tile_cols == 256 ? k_fu_h<Q, R, 4, true, PAST> : k_fu_h<Q, R, 1, true, PAST>;
   else if constexpr (NB == 2)
-    return totals ? (tile_cols == 128 ? k_fu_h<Q, R, 2, true> : k_fu_h<Q, R, 1, true>)
-                  : (tile_cols == 128 ? k_fu_h<Q, R, 2, false> : k_fu_h<Q, R, 1, false>);
-  else return k_fu_h<Q, R, 1, false>;
+    return totals ? (tile_cols == 128 ? k_fu_h<Q, R, 2, true, PAST> : k_fu_h<Q, R, 1, true, PAST>)
+                  : (tile_cols == 128 ? k_fu_h<Q, R, 2, false, PAST> : k_fu_h<Q, R, 1, false, PAST>);
+  else return k_fu_h<Q, R, 1, false, PAST>;
+}
+template <int Q, int R>
+static fu_h_kernel fu_h_of(int64_t m, int tile_cols, bool totals) {
+  return 64 * m * fu_blocks(Q, R) <= FU_PAST_BYTES ? fu_h_of<Q, R, true>(tile_cols, totals) : fu_h_of<Q, R, false>(tile_cols, totals);
 }
 
 int fused_state::create(const dnpeff_csr* S, int64_t n, int rank) {
@@ -929,7 +999,7 @@ int fused_state::create(const dnpeff_csr* S, int64_t n, int rank) {
     if (r > FUSED_NARROW_RANK) DN_TRY(fuw_per_cu(r, &per_cu));
     else DN_TRY(fu_dispatch(r, [&](auto tag) {
       DN_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(
-          &per_cu, fu_h_of<decltype(tag)::Q, decltype(tag)::R>(f.tile_cols, h_totals), 256, 0));
+          &per_cu, fu_h_of<decltype(tag)::Q, decltype(tag)::R>(S->n_cols, f.tile_cols, h_totals), 256, 0));
       return 0;
     }));
     most = (int64_t)n_cus() * (per_cu > 0 ? per_cu : 1);
@@ -1044,14 +1114,14 @@ int fused_state::update_w(const dnpeff_csr* S, int64_t n, const float* Nw, float
 }
 
 int fused_state::update_h(const dnpeff_csr* S, const float* W, float* H, float eps) {
-  if (gw_state == PARTS && w_wgs > FU_SUM_DIRECT) DN_TRY(sum_w());
+  if (gw_state == PARTS && w_wgs > fu_sum_direct(fu_blocks_of(r))) DN_TRY(sum_w());
   const float* gw = gw_state == PARTS ? gw_part : gw_sum;
   const int n_gw = gw_state == PARTS ? w_wgs : 1;
   const fused_plan& f = S->fused;
   if (r > FUSED_NARROW_RANK)
     DN_TRY(fuw_launch_h(h_wgs, f, S->colptr, r, W, H, eps, gw, n_gw, gh_part));
   else DN_TRY(fu_dispatch(r, [&](auto tag) {
-    hipLaunchKernelGGL((fu_h_of<decltype(tag)::Q, decltype(tag)::R>(f.tile_cols, h_totals)), dim3((unsigned)h_wgs), dim3(256), 0,
+    hipLaunchKernelGGL((fu_h_of<decltype(tag)::Q, decltype(tag)::R>(S->n_cols, f.tile_cols, h_totals)), dim3((unsigned)h_wgs), dim3(256), 0,
                        stream(), f.tiles, (int)f.n_tiles, S->colptr, f.pairs, r, W, H, eps, gw, n_gw, gh_part);
     return 0;
   }));

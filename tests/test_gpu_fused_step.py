@@ -200,3 +200,19 @@ def test_contexts_of_several_ranks_in_turn():
         assert nmf.computeUncachedLoss() == want[r][2]
         nmf.close()
     A.close()
+
+
+@pytest.mark.parametrize("n,m,r,fill", [(512, 3000, 9, 0.45), (512, 3000, 20, 0.45), (513, 3000, 20, 0.45),
+                                        (257, 2500, 40, 0.3), (24, 1_100_000, 5, 1e-4)])
+def test_partial_sums_on_either_side_of_their_limits(n, m, r, fill):
+    """Eight and nine partial Gram matrices of W (summed by the H update, or before it), rows of five and six
+    chunk sums (four are read at a time), and a factor too large to be written past the caches."""
+    rp, ci, va = _matrix(n, m, seed=n + r, fill=fill)
+    A = d.Csr.from_host(rp, ci, va, m)
+    nmf = d.MuNmf(A, d.MuNmfParams(rank=r, max_iters=3, eps=EPS, seed=5, log_every=3))
+    nmf.initialize()
+    W0, H0 = nmf.loadWToHostSync(), nmf.loadHToHostSync()
+    nmf.run(log=lambda s: None)
+    _close(nmf, orc.nmf_f64(rp, ci, va, m, W0, H0, np.float32(EPS), 3, 3))
+    nmf.close()
+    A.close()
