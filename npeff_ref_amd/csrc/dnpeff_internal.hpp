@@ -305,6 +305,12 @@ struct fused_plan {
   fu_chunk* chunks = nullptr;
   int64_t n_chunks = 0;
   int* n_base = nullptr;     // [n_rows + 1] first chunk of each row
+  // or, for A H^T by XCD: every row's entries grouped by the XCD that their columns belong to,
+  // x_seg[8 row + x] = first entry of XCD x (and the end), in x_parts chunks each
+  int32_t* x_col = nullptr;
+  float* x_val = nullptr;
+  int64_t* x_seg = nullptr;
+  int x_parts = 0;
 };
 
 }  // namespace dn

@@ -612,14 +612,15 @@ __global__ void __launch_bounds__(256, 2)
 // round-robin, FU_U gathers each in flight.  Workgroups 0 .. sum_wgs - 1 sum Gram parts instead.
 // 777 x 862k, r = 50: 117 us for 3.9 M gathered rows of 200 bytes (6.6 TB/s), half of which the L2s hold;
 // 141 us as one 4-byte load per lane.
-template <int LPR>
+template <int LPR, bool XCD>
 __global__ void __launch_bounds__(256)
-    k_fu_n(const fu_chunk* __restrict__ chunks, const int32_t* __restrict__ colind, const float* __restrict__ vals,
-           int r, const float* __restrict__ H, float* __restrict__ N, int sum_wgs, const float* __restrict__ part,
-           int n_parts, int S, float* __restrict__ gsum) {
+    k_fu_n(const fu_chunk* __restrict__ chunks, const int64_t* __restrict__ x_seg, int x_parts,
+           const int32_t* __restrict__ colind, const float* __restrict__ vals, int r, const float* __restrict__ H,
+           float* __restrict__ N, int sum_wgs, const float* __restrict__ part, int n_parts, int S,
+           float* __restrict__ gsum) {
   __shared__ __align__(16) double red_d[256];
   if ((int)blockIdx.x < sum_wgs) {
-    fu_sum_parts(part, n_parts, S, blockIdx.x, gsum, red_d);
+    if ((int)blockIdx.x < S / 16) fu_sum_parts(part, n_parts, S, blockIdx.x, gsum, red_d);
     return;
   }
   constexpr int G = 64 / LPR;
@@ -628,9 +629,18 @@ __global__ void __launch_bounds__(256)
   // against 115.6 us at the size above).
   __shared__ __align__(16) float totals[256][4];
   float* red = reinterpret_cast<float*>(red_d);  // [4][4 LPR]
-  const int64_t chunk = blockIdx.x - sum_wgs;
-  const int64_t e0 = chunks[chunk].e0;
-  const int len = chunks[chunk].len;
+  int64_t chunk = blockIdx.x - sum_wgs, e0;
+  int len;
+  if constexpr (XCD) {  // (sum_wgs is a multiple of 8)
+    const unsigned u = (unsigned)chunk >> 3, x = (unsigned)chunk & 7, row = u / (unsigned)x_parts, k = u % (unsigned)x_parts;
+    const int64_t s0 = x_seg[8 * row + x], s1 = x_seg[8 * row + x + 1], each = (unsigned)(s1 - s0 + x_parts - 1) / (unsigned)x_parts;
+    e0 = s0 + k * each;
+    len = (int)(e0 >= s1 ? 0 : e0 + each < s1 ? each : s1 - e0);
+    chunk = (8 * row + x) * (unsigned)x_parts + k;
+  } else {
+    e0 = chunks[chunk].e0;
+    len = chunks[chunk].len;
+  }
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, sub = lane % LPR, grp = lane / LPR;
   const float* Hl = H + (4 * sub < r ? 4 * sub : 0);  // (lanes past the rank: any valid address)
   const int per = (len + 3) / 4;
@@ -847,6 +857,7 @@ __global__ void __launch_bounds__(256)
 void fused_drop(dnpeff_csr* S) {
   fused_plan& f = S->fused;
   dfree(f.tiles); dfree(f.pairs); dfree(f.chunks); dfree(f.n_base);
+  dfree(f.x_col); dfree(f.x_val); dfree(f.x_seg);
   f = fused_plan();
 }
 
@@ -907,6 +918,95 @@ int fused_tiles_first(dnpeff_csr* S) {
   return fused_tiles_make(S, S->fused.tile_cols, S->fused.tile_most, S->fused.tile_alone, true);
 }
 
+// Entries per workgroup of A H^T: about FU_CHUNKS workgroups in all, at least 256 entries each.
+static int64_t fu_chunk_entries(int64_t nnz) { return std::max<int64_t>(256, ceil_div(ceil_div(nnz, FU_CHUNKS), 256) * 256); }
+
+// A row's entries by the XCD that their columns belong to (16 columns each in turn), in their order, a workgroup per
+// row: every wave takes a quarter, counts, and places its entries behind those of the waves before.
+__device__ inline int fu_xcd_of(int col) { return (col >> 4) & 7; }
+__global__ void __launch_bounds__(256)
+    k_fu_xcd_split(const int64_t* __restrict__ rowptr, const int32_t* __restrict__ colind, const float* __restrict__ vals,
+                   int64_t n, int parts, int32_t* __restrict__ x_col, float* __restrict__ x_val, int64_t* __restrict__ x_seg,
+                   int* __restrict__ n_base) {
+  __shared__ int count[4][8];
+  const int64_t row = blockIdx.x, r0 = rowptr[row], r1 = rowptr[row + 1];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int64_t per = (r1 - r0 + 3) / 4, e0 = r0 + wave * per < r1 ? r0 + wave * per : r1, e1 = e0 + per < r1 ? e0 + per : r1;
+  int mine = 0;  // (lane x < 8: entries of XCD x)
+  auto walk = [&](auto&& f) {
+    for (int64_t e = e0; e < e1; e += 64) {
+      const bool in = e + lane < e1;
+      const int col = colind[in ? e + lane : e1 - 1], x = fu_xcd_of(col);
+      const uint64_t here = __ballot(in), b0 = __ballot(x & 1), b1 = __ballot(x & 2), b2 = __ballot(x & 4);
+      auto of = [&](int y) { return here & (y & 1 ? b0 : ~b0) & (y & 2 ? b1 : ~b1) & (y & 4 ? b2 : ~b2); };
+      f(e, in, col, x, of);
+    }
+  };
+  walk([&](int64_t, bool, int, int, auto of) { mine += __popcll(of(lane & 7)); });
+  if (lane < 8) count[wave][lane] = mine;
+  __syncthreads();
+  int64_t at = r0;  // (lane x < 8: where the wave's next entry of XCD x goes)
+  for (int y = 0; y < 8; y++)
+    for (int w = 0; w < 4; w++) at += y < (lane & 7) || (y == (lane & 7) && w < wave) ? count[w][y] : 0;
+  if (wave == 0 && lane < 8) {
+    x_seg[8 * row + lane] = at;
+    if (lane == 0) n_base[row] = (int)(8 * parts * row);
+    if (row == n - 1 && lane == 0) {
+      x_seg[8 * n] = r1;
+      n_base[n] = (int)(8 * parts * n);
+    }
+  }
+  walk([&](int64_t e, bool in, int col, int x, auto of) {
+    const int64_t base = __shfl(at, x);
+    if (in) {
+      const int64_t to = base + __popcll(of(x) & ((1ull << lane) - 1ull));
+      x_col[to] = col;
+      x_val[to] = vals[e + lane];
+    }
+    at += __popcll(of(lane & 7));
+  });
+}
+
+// A H^T by XCD: workgroups are dealt to the XCDs round-robin, and where each XCD has its own eighth of the
+// columns its L2 fetches a row of H once for all that gather it (and from a part of H an eighth as large), where
+// with chunks of whole rows every XCD fetches most of H.  The columns are dealt in sixteens: an eighth
+// in one piece has all the rare columns on the last XCD, whose misses are then waited for (777 x 862k, r = 50: 126
+// us; with columns dealt one by one two XCDs share every line of short rows).  k_fu_n at 777 x 862k, r = 50 / 512 x 431k, r = 16
+// / 300 x 146k, r = 20: 74.7 / 17.2 / 10.2 us, in chunks of whole rows 117 / 21.5 / 11.0.
+// Rows of FU_XCD_ROW entries or more on average, of which none is twice as long (a workgroup per row and XCD).  Ten iterations
+// in chunks of whole rows / by XCD: 191 / 215 us at 200 rows of 200 entries, r = 8, 252 / 281 at 500 of 512, r = 16, 488 / 546 at
+// 1000 of 1024, r = 32 (a workgroup has 128 entries then), 782 / 788 at 2000 of 2048, r = 8, 796 / 754 at 300 of 2048, r = 64,
+// 5880 / 5476 at 1000 of 4096, r = 96, 9751 / 8205 at 2000 of 8192, r = 60.
+static int fused_xcd_build(dnpeff_csr* S) {
+  fused_plan& f = S->fused;
+  const int64_t n = S->n_rows, mean = S->nnz / n;
+  if (mean < FU_XCD_ROW || !xcd_round_robin()) return 0;
+  std::vector<int64_t> rowptr((size_t)n + 1);
+  DN_HIP(copy_down(rowptr.data(), S->rowptr, sizeof(int64_t) * rowptr.size()));
+  int64_t most = 0;
+  for (int64_t i = 0; i < n; i++) most = std::max(most, rowptr[i + 1] - rowptr[i]);
+  const int64_t parts = std::max<int64_t>(1, S->nnz / (8 * n) / fu_chunk_entries(S->nnz));
+  if (most > 2 * mean || 8 * n * parts >= ((int64_t)1 << 24)) return 0;
+  dbuf<int32_t> col;
+  dbuf<int64_t> seg;
+  dbuf<float> val;
+  dbuf<int> base;
+  if (col.alloc(S->nnz) || val.alloc(S->nnz) || seg.alloc(8 * n + 1) || base.alloc(n + 1)) {  // (no room: chunks of whole rows)
+    clear_error();
+    return 0;
+  }
+  hipLaunchKernelGGL(k_fu_xcd_split, dim3((unsigned)n), dim3(256), 0, stream(), S->rowptr, S->colind, S->vals, n, (int)parts, col.p,
+                     val.p, seg.p, base.p);
+  DN_LAUNCH_CHECK();
+  f.x_seg = seg.release();
+  f.x_col = col.release();
+  f.x_val = val.release();
+  f.n_base = base.release();
+  f.x_parts = (int)parts;
+  f.n_chunks = 8 * n * parts;
+  return 0;
+}
+
 int fused_plan_build(dnpeff_csr* S, int r) {
   fused_plan& f = S->fused;
   hipStream_t st = stream();
@@ -920,11 +1020,11 @@ int fused_plan_build(dnpeff_csr* S, int r) {
     DN_LAUNCH_CHECK();
   }
   DN_TRY(fused_tiles_build(S, r));
-  if (!f.chunks && S->n_panels == 0) {
+  if (!f.chunks && !f.x_seg && S->n_panels == 0) {
     DN_CHECK(has_row_major(S), "row-major copy of the matrix was released");
-    // entries per workgroup of A H^T: about FU_CHUNKS workgroups in all, at least 256 entries each
-    int64_t chunk = ceil_div(ceil_div(S->nnz, FU_CHUNKS), 256) * 256;
-    if (chunk < 256) chunk = 256;
+    DN_TRY(fused_xcd_build(S));
+    if (f.x_seg) return 0;
+    const int64_t chunk = fu_chunk_entries(S->nnz);
     dbuf<int64_t> base;
     DN_TRY(base.alloc(S->n_rows + 1));
     DN_TRY(scan_row_chunks(S->rowptr, chunk, S->n_rows, base));
@@ -1058,19 +1158,22 @@ int fused_state::gram_of(const float* X, int64_t rows, bool of_h) {
 
 int fused_state::product_n(const dnpeff_csr* S, const float* H) {
   const fused_plan& f = S->fused;
-  DN_CHECK(has_row_major(S) && f.chunks, "row-major copy of the matrix was released");
+  DN_CHECK((has_row_major(S) && f.chunks) || f.x_seg, "row-major copy of the matrix was released");
   if (n_part_floats < f.n_chunks * r + 4) {
     dfree(n_part);
     n_part = nullptr;
     n_part_floats = f.n_chunks * r + 4;
     DN_TRY(dmalloc(&n_part, n_part_floats));
   }
-  const int sums = gh_state == PARTS ? S_floats / 16 : 0;
+  const int sums = gh_state == PARTS ? (int)ceil_div(S_floats / 16, 8) * 8 : 0;
   const dim3 grid((unsigned)(f.n_chunks + sums)), block(256);
   if (grid.x > 0) {
-#define DN_FU_N(LPR)                                                                                                \
-  hipLaunchKernelGGL((k_fu_n<LPR>), grid, block, 0, stream(), f.chunks, S->colind, S->vals, r, H, n_part, sums, gh_part, \
-                     h_wgs, S_floats, gh_sum)
+    const bool xcd = f.x_seg != nullptr;
+    auto go = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, grid, block, 0, stream(), f.chunks, f.x_seg, f.x_parts, xcd ? f.x_col : S->colind,
+                         xcd ? f.x_val : S->vals, r, H, n_part, sums, gh_part, h_wgs, S_floats, gh_sum);
+    };
+#define DN_FU_N(LPR) xcd ? go(k_fu_n<LPR, true>) : go(k_fu_n<LPR, false>)
     if (r <= 8) DN_FU_N(2);
     else if (r <= 16) DN_FU_N(4);
     else if (r <= 32) DN_FU_N(8);
@@ -1147,14 +1250,14 @@ double fused_tiles_bytes(int64_t m, int64_t nnz) {
 }
 
 double fused_list_bytes(int64_t n, int64_t m, int64_t nnz) {
-  return 8.0 * (double)(nnz + 1) + fused_tiles_bytes(m, nnz) + 16.0 * (double)(FU_CHUNKS + n) + 4.0 * (double)(n + 1);
+  return 16.0 * (double)(nnz + 1) + fused_tiles_bytes(m, nnz) + 16.0 * (double)(FU_CHUNKS + n) + 68.0 * (double)(n + 1);
 }
 
 double fused_state_bytes(int64_t n, int64_t m, int64_t nnz, int r) {
   const double S = 4.0 * fused_gram_floats(r);
   // workgroups of the H update: one round of what the chip holds, or enough rounds of them
   const double wgs = (r > FUSED_NARROW_RANK ? 4.0 : 8.0) * n_cus() + ((double)m + (double)nnz / 8.0) / FU_MOST_COLS;
-  return 4.0 * ((double)(FU_CHUNKS + n) * r + 4.0) + S * (wgs + (double)n / FUW_COLS + 3.0) + (double)n;
+  return 4.0 * ((double)(FU_CHUNKS + 8 * n) * r + 4.0) + S * (wgs + (double)n / FUW_COLS + 3.0) + (double)n;
 }
 
 bool fused_supported(int64_t n, int64_t m, int64_t nnz, int r) {

@@ -216,3 +216,19 @@ def test_partial_sums_on_either_side_of_their_limits(n, m, r, fill):
     _close(nmf, orc.nmf_f64(rp, ci, va, m, W0, H0, np.float32(EPS), 3, 3))
     nmf.close()
     A.close()
+
+
+@pytest.mark.parametrize("n,m,r,fill", [(5, 24_003, 3, 0.9), (40, 9000, 17, 0.25), (61, 8191, 40, 0.22),
+                                        (120, 6000, 100, 0.35), (9, 6000, 8, 0.32)])
+def test_rows_grouped_by_xcd(n, m, r, fill):
+    """Rows around the length from which their entries are grouped by XCD, an empty one, several chunks per
+    row and XCD, sizes that no group of columns divides."""
+    rp, ci, va = _matrix(n, m, seed=n + r, fill=fill)
+    A = d.Csr.from_host(rp, ci, va, m)
+    nmf = d.MuNmf(A, d.MuNmfParams(rank=r, max_iters=4, eps=EPS, seed=5, log_every=2))
+    nmf.initialize()
+    W0, H0 = nmf.loadWToHostSync(), nmf.loadHToHostSync()
+    nmf.run(log=lambda s: None)
+    _close(nmf, orc.nmf_f64(rp, ci, va, m, W0, H0, np.float32(EPS), 4, 2))
+    nmf.close()
+    A.close()
