@@ -165,6 +165,11 @@ static bool fused_now(const dnpeff_nmf* h) {
   return h->has_fused && tuning().fused_gram != 0.0 && !h->A->tail && !h->prof.enabled;
 }
 
+static bool small_now(const dnpeff_nmf* h) {
+  return fused_now(h) && h->A->n_panels == 0 && has_row_major(h->A) && h->A->colptr &&
+         fused_small_fits(h->n, h->m, h->A->nnz, h->r);
+}
+
 DN_API int dnpeff_nmf_destroy(dnpeff_nmf* nmf) {
   if (!nmf) return 0;
   (void)hipStreamSynchronize(stream());
@@ -750,6 +755,13 @@ DN_API int dnpeff_nmf_update_H(dnpeff_nmf* h) {
 DN_API int dnpeff_nmf_step(dnpeff_nmf* nmf, int n_steps) {
   clear_error();
   DN_CHECK(nmf != nullptr, "handle is NULL");
+  if (n_steps > 0 && small_now(nmf)) {
+    DN_TRY(take_back(nmf));
+    nmf->w_out = nmf->h_out = false;
+    nmf->fu.gh_state = nmf->fu.gw_state = fused_state::NONE;
+    nmf->gh_valid = nmf->nw_valid = nmf->fu_n_valid = false;
+    return fused_small_launch(nmf->A, nmf->r, nmf->W, nmf->H, nmf->eps, n_steps, nullptr);
+  }
   for (int s = 0; s < n_steps; s++) {
     DN_TRY(dnpeff_nmf_update_W(nmf));
     DN_TRY(dnpeff_nmf_update_H(nmf));
@@ -766,9 +778,13 @@ DN_API int dnpeff_nmf_loss_terms(dnpeff_nmf* h, double* sq_norm_A, double* pos, 
     unsigned long long* words = nullptr;
     DN_TRY(host_words(&words));
     double* sums = reinterpret_cast<double*>(words);
-    DN_TRY(fused_products(h));
-    if (h->fu.gw_state == fused_state::NONE) DN_TRY(h->fu.gram_of(h->W, h->n, false));
-    DN_TRY(h->fu.loss_sums(A, h->n, fused_nw(h), h->W, sums));
+    if (small_now(h)) {
+      DN_TRY(fused_small_launch(A, h->r, h->W, h->H, h->eps, 0, sums));
+    } else {
+      DN_TRY(fused_products(h));
+      if (h->fu.gw_state == fused_state::NONE) DN_TRY(h->fu.gram_of(h->W, h->n, false));
+      DN_TRY(h->fu.loss_sums(A, h->n, fused_nw(h), h->W, sums));
+    }
     DN_HIP(hipStreamSynchronize(stream()));
     if (sq_norm_A) *sq_norm_A = h->sq_norm_A;
     if (neg) *neg = sums[0];

@@ -35,6 +35,10 @@ int fuw_launch_h(int wgs, const fused_plan& f, const int64_t* colptr, int r, con
 int fuw_launch_w(int wgs, int64_t n, int r, const int* n_base, const float* N, float* W, float eps, const float* gh,
                  float* gpart);
 
+// Whole runs in one workgroup's LDS (fused_small.hip): steps, or the two sums of the loss.
+bool fused_small_fits(int64_t n, int64_t m, int64_t nnz, int r);
+int fused_small_launch(const dnpeff_csr* S, int r, float* W, float* H, float eps, int steps, double* loss);
+
 // What a context keeps between the launches of a step.
 struct fused_state {
   enum gram_state { NONE, PARTS, SUMMED };

@@ -232,3 +232,35 @@ def test_rows_grouped_by_xcd(n, m, r, fill):
     _close(nmf, orc.nmf_f64(rp, ci, va, m, W0, H0, np.float32(EPS), 4, 2))
     nmf.close()
     A.close()
+
+
+@pytest.mark.parametrize("n,m,r,fill", [(2, 3, 1, 0.9), (16, 33, 4, 0.5), (17, 2100, 5, 0.05), (128, 640, 16, 0.04),
+                                        (127, 300, 9, 0.1), (129, 300, 9, 0.1), (48, 907, 8, 0.07), (60, 500, 15, 0.08)])
+def test_runs_in_one_workgroup(n, m, r, fill):
+    """Runs that one workgroup's LDS holds (128 rows and 16 components at most): several steps in one launch give
+    the bits of as many launches of one step, and what the two updates of the launched step give (fp32 sums in another
+    order, a few 1e-7 per step)."""
+    rp, ci, va = _matrix(n, m, seed=n + m, fill=fill)
+    A = d.Csr.from_host(rp, ci, va, m)
+
+    def run(steps):
+        nmf = d.MuNmf(A, d.MuNmfParams(rank=r, max_iters=4, eps=EPS, seed=5, log_every=4))
+        nmf.initialize()
+        W0, H0 = nmf.loadWToHostSync(), nmf.loadHToHostSync()
+        steps(nmf)
+        out = nmf.loadWToHostSync(), nmf.loadHToHostSync(), nmf.loss_terms()
+        nmf.close()
+        return W0, H0, out
+
+    W0, H0, one = run(lambda nmf: nmf.step(4))
+    for got, want in zip(run(lambda nmf: [nmf.step(1) for _ in range(4)])[2], one):
+        assert np.array_equal(got, want)
+    two = run(lambda nmf: [(nmf.update_W(), nmf.update_H()) for _ in range(4)])[2]
+    for got, want in zip(one[:2], two[:2]):
+        assert np.linalg.norm(got - want) <= 5e-6 * np.linalg.norm(want)
+    W64, H64, losses = orc.nmf_f64(rp, ci, va, m, W0, H0, np.float32(EPS), 4, 4)
+    for got, want in zip(one[:2], (W64, H64)):
+        assert np.linalg.norm(got - want) <= 5e-6 * np.linalg.norm(want)
+    sq, pos, neg = one[2]
+    assert abs(sq + pos - 2 * neg - losses[-1] ** 2) <= 1e-5 * sq
+    A.close()
