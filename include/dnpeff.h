@@ -121,6 +121,12 @@ int dnpeff_dev_malloc(int64_t bytes, void** out);
 int dnpeff_dev_free(void* p);
 int dnpeff_dev_upload(void* dst_dev, const void* src_host, int64_t bytes);
 int dnpeff_dev_download(void* dst_host, const void* src_dev, int64_t bytes);
+/* Buffers for results that only the library's own calls write: handed out and taken back in the
+ * order of the library stream, without a wait.  Their download waits for that stream alone; several at
+ * once wait together. */
+int dnpeff_scratch_malloc(int64_t bytes, void** out);
+int dnpeff_scratch_free(void* p);
+int dnpeff_scratch_download(int n, void* const* dst_host, const void* const* src_dev, const int64_t* bytes);
 
 /* ------------------------------------------------------------------------- */
 /* Loader: CSR on the device, row normalisation, column compaction            */

@@ -55,6 +55,9 @@ SIGNATURES = {
     "dnpeff_dev_free": (C.c_int, [_p]),
     "dnpeff_dev_upload": (C.c_int, [_p, _p, _i64]),
     "dnpeff_dev_download": (C.c_int, [_p, _p, _i64]),
+    "dnpeff_scratch_malloc": (C.c_int, [_i64, C.POINTER(_p)]),
+    "dnpeff_scratch_free": (C.c_int, [_p]),
+    "dnpeff_scratch_download": (C.c_int, [C.c_int, C.POINTER(_p), C.POINTER(_p), C.POINTER(_i64)]),
     "dnpeff_csr_from_host": (C.c_int, [_i64, _i64, _i64, _p, _p, _p, _pp]),
     "dnpeff_csr_from_pef": (C.c_int, [_i64, _i64, _i64, _p, _p, _pp]),
     "dnpeff_csr_normalize_rows": (C.c_int, [_p, _p, _f32]),
@@ -300,6 +303,31 @@ class DeviceArray:
             pass
 
 
+class _Scratch:
+    """A device buffer for results of one call that only the library writes (no waits)."""
+
+    def __init__(self, nbytes: int):
+        self.ptr = C.c_void_p()
+        _check(lib.dnpeff_scratch_malloc(nbytes, C.byref(self.ptr)))
+
+    def __del__(self):
+        if self.ptr:
+            lib.dnpeff_scratch_free(self.ptr)
+
+
+def _scratch_numpy(*parts):
+    """The first elements of several scratch buffers, [(buffer, shape, dtype)], in one download."""
+    out = [np.empty(shape, dtype=dtype) for _, shape, dtype in parts]
+    n = len(parts)
+    _check(
+        lib.dnpeff_scratch_download(
+            n, (C.c_void_p * n)(*(a.ctypes.data for a in out)), (C.c_void_p * n)(*(b.ptr.value for b, _, _ in parts)),
+            (C.c_int64 * n)(*(a.nbytes for a in out)),
+        )
+    )
+    return out
+
+
 def op_mu(F: DeviceArray, num: DeviceArray, den: DeviceArray, eps: float):
     _check(lib.dnpeff_op_mu(int(np.prod(F.shape)), F.ptr, num.ptr, den.ptr, eps))
 
@@ -362,23 +390,19 @@ def op_init_uniform(matrix_id: int, logical_rows: int, logical_cols: int, seed: 
 def topk_rows(x: "DeviceArray", k: int):
     """(values [n, k], indices [n, k], norms [n]) of the k largest entries of each row of x."""
     n, count = x.shape
-    vals = DeviceArray((n, k), dtype=np.float32)
-    idx = DeviceArray((n, k), dtype=np.int32)
-    norms = DeviceArray((n,), dtype=np.float32)
+    vals, idx, norms = _Scratch(4 * n * k), _Scratch(4 * n * k), _Scratch(4 * n)
     _check(lib.dnpeff_topk_rows(n, count, k, x.ptr, vals.ptr, idx.ptr, norms.ptr))
-    sync()
-    return vals.numpy(), idx.numpy(), norms.numpy()
+    return tuple(_scratch_numpy((vals, (n, k), np.float32), (idx, (n, k), np.int32), (norms, (n,), np.float32)))
 
 
 def op_threshold_compact(x: "DeviceArray", divisor: float, threshold: float):
     """(positions, values) of the elements with x / divisor >= threshold, as numpy arrays."""
     n = int(np.prod(x.shape))
-    idx = DeviceArray((max(n, 1),), dtype=np.int32)
-    val = DeviceArray((max(n, 1),), dtype=np.float32)
+    idx, val = _Scratch(4 * max(n, 1)), _Scratch(4 * max(n, 1))
     kept = _i64(0)
     _check(lib.dnpeff_op_threshold_compact(n, x.ptr, float(divisor), float(threshold), idx.ptr, val.ptr,
                                            C.byref(kept)))
-    return idx.first(kept.value), val.first(kept.value)
+    return tuple(_scratch_numpy((idx, (kept.value,), np.int32), (val, (kept.value,), np.float32)))
 
 
 class Csr:

@@ -1214,6 +1214,29 @@ DN_API int dnpeff_dev_download(void* dst_host, const void* src_dev, int64_t byte
   return 0;
 }
 
+DN_API int dnpeff_scratch_malloc(int64_t bytes, void** out) {
+  clear_error();
+  DN_CHECK(out != nullptr && bytes >= 0, "bad arguments");
+  return device_alloc(out, (size_t)bytes);
+}
+
+DN_API int dnpeff_scratch_free(void* p) {
+  device_release(p);
+  return 0;
+}
+
+DN_API int dnpeff_scratch_download(int n, void* const* dst_host, const void* const* src_dev, const int64_t* bytes) {
+  clear_error();
+  DN_CHECK(n >= 0 && (n == 0 || (dst_host && src_dev && bytes)), "bad arguments");
+  std::vector<copy_part> parts;
+  for (int q = 0; q < n; q++) {
+    DN_CHECK(bytes[q] >= 0 && (bytes[q] == 0 || (dst_host[q] && src_dev[q])), "bad arguments");
+    if (bytes[q]) parts.push_back({dst_host[q], src_dev[q], (size_t)bytes[q]});
+  }
+  DN_HIP(copy_down_parts(parts.data(), (int)parts.size()));
+  return 0;
+}
+
 DN_API int64_t dnpeff_size_of_split(int64_t total, int64_t n_splits, int64_t split_index) {
   if (n_splits <= 0 || split_index < 0 || split_index >= n_splits) return -1;
   int64_t base = total / n_splits;
