@@ -6,12 +6,15 @@
 // A row has ~1e8 entries and k ~ 6.5e4, so sorting the row is out of the question.  Usual case, one read
 // of the row and a thirty-second of it before:
 //   1. two histograms (11 bits of an order-preserving integer key each) of a sample, 64 entries out
-//      of every 2048, give a threshold that a little more than k entries reach (all entries of a
-//      short row: exactly the k-th entry's 22 bits);
-//   2. every entry from the threshold up goes to a candidate list ((key, index) pairs, any order), and
-//      the sum of squares is taken on the way;
-//   3. the candidates are counted and scattered into buckets of equal key width; an entry's place is
-//      its bucket's start plus the number of larger pairs in the bucket.
+//      of every 2048 (of every 4096 where k leaves 512 of them above the threshold: 14 us instead of 23 for
+//      the first at 2 rows of 110 M), give a threshold that a little more than k entries reach (all entries
+//      of a short row: exactly the k-th entry's 22 bits);
+//   2. every entry from the threshold up goes to a candidate list ((key, index) pairs, any order) and is
+//      counted into its bucket, one of equal key width between the threshold and the largest sampled, and the
+//      sum of squares is taken on the way;
+//   3. the candidates are placed into their buckets by the count that they met (an atomic of their own on a
+//      cursor each took 18 us at 2 x 72,000 candidates, now 5; counting them after the collection 14 more); an
+//      entry's place is its bucket's start plus the number of larger pairs in the bucket.
 // When the threshold was too high (fewer than k candidates), when far more entries reach it than
 // expected, or when a bucket is crowded (many equal entries), the row goes through histograms of all
 // entries instead: 11 bits find the bin of the k-th entry, that bin and all above it are sorted
@@ -130,6 +133,17 @@ __global__ void __launch_bounds__(64)
   for (int i = threadIdx.x; i < TOPK_BINS; i += 64) h[i] = 0;
 }
 
+// Bucket of a key from the threshold up: 0 holds the largest, which may lie above kmax (the largest of a sample).
+// All other buckets span 2^shift keys.
+__device__ inline int topk_shift(uint32_t thr, uint32_t kmax, int log_nb) {
+  const uint32_t range = kmax - thr;
+  const int bits = range ? 32 - __clz(range) : 0;
+  return bits > log_nb ? bits - log_nb : 0;
+}
+__device__ inline int topk_bucket(uint32_t key, uint32_t thr, uint32_t kmax, int shift) {
+  return (int)(((kmax - thr) >> shift) - (((key < kmax ? key : kmax) - thr) >> shift));
+}
+
 // A wave's finds on their way to a row's candidate list.  They wait in LDS and room in the list is reserved
 // once per 256+ of them: the finds are sparse (k of ~1e8), and one global atomic each on a single counter
 // would serialise them.  Every wave keeps its own buffer and count, so the loop that reads the row has no
@@ -140,6 +154,10 @@ struct topk_finds {
   uint64_t* out;
   int64_t cap;
   unsigned long long* cursor;
+  int* buckets;  // (or NULL) entries per bucket, counted as they are written: `place` receives the count before
+  unsigned* place;
+  uint32_t thr, kmax;
+  int shift;
 
   // All lanes call these together.
   __device__ void put(bool take, uint32_t key, int64_t i) {
@@ -151,7 +169,10 @@ struct topk_finds {
   __device__ void write(unsigned long long base) {
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     for (unsigned i = threadIdx.x & 63; i < n; i += 64)
-      if (base + i < (unsigned long long)cap) out[base + i] = buf[i];
+      if (base + i < (unsigned long long)cap) {
+        out[base + i] = buf[i];
+        if (buckets) place[base + i] = (unsigned)atomicAdd(&buckets[topk_bucket((uint32_t)(buf[i] >> 32), thr, kmax, shift)], 1);
+      }
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     n = 0;
   }
@@ -222,7 +243,7 @@ __global__ void __launch_bounds__(256)
   const uint32_t prefix = st[row].prefix, mask = st[row].mask;
   const int64_t n_cand = k - st[row].need + st[row].in_bin;
   uint64_t* out = cand + (int64_t)row * kp;
-  topk_finds f{buf[threadIdx.x >> 6], 0u, out, kp, reinterpret_cast<unsigned long long*>(&st[row].cursor)};
+  topk_finds f{buf[threadIdx.x >> 6], 0u, out, kp, reinterpret_cast<unsigned long long*>(&st[row].cursor), nullptr, nullptr, 0u, 0u, 0};
   topk_sweep<VEC4>(x + (int64_t)row * count, count, [&](const float* v, int64_t first, bool) {
 #pragma unroll
     for (int e = 0; e < 4; e++) {
@@ -342,7 +363,7 @@ __global__ void __launch_bounds__(256)
 // The usual case
 // ---------------------------------------------------------------------------
 constexpr int TOPK_CHUNK = 64;            // sampled entries in a row
-constexpr int TOPK_STRIDE = 2048;         // one chunk of every so many entries
+constexpr int TOPK_STRIDE = 2048;         // one chunk of every so many entries, or of twice as many
 constexpr int64_t TOPK_SAMPLED = 1 << 19; // rows from this length on are sampled
 constexpr int TOPK_MAX_BUCKETS = 16384;
 constexpr int TOPK_CROWDED = 2048;        // entries of a bucket that are still ranked one against the other
@@ -353,9 +374,11 @@ struct TopkRow {
   unsigned long long cursor;   // candidates
 };
 
-__global__ void __launch_bounds__(256) k_topk_row_init(TopkRow* rows, unsigned target, unsigned* __restrict__ hist) {
-  if (threadIdx.x == 0) rows[blockIdx.x] = TopkRow{0u, 0u, 0u, target, 0ull};
-  for (int i = threadIdx.x; i < TOPK_BINS; i += 256) hist[(int64_t)blockIdx.x * TOPK_BINS + i] = 0;
+__global__ void __launch_bounds__(1024)
+    k_topk_row_init(TopkRow* rows, unsigned target, unsigned* __restrict__ hist, int log_nb, int* __restrict__ buckets) {
+  if (threadIdx.x == 0) rows[blockIdx.x] = TopkRow{0u, 0u, 0xffffffffu, target, 0ull};
+  for (int i = threadIdx.x; i < TOPK_BINS; i += 1024) hist[(int64_t)blockIdx.x * TOPK_BINS + i] = 0;
+  for (int i = threadIdx.x; i < 1 << log_nb; i += 1024) buckets[((int64_t)blockIdx.x << log_nb) + i] = 0;
 }
 
 // LEVEL 0: top 11 bits of the key; 1: the next 11 of the entries in the bin that level 0 found.
@@ -411,6 +434,11 @@ __global__ void __launch_bounds__(256) k_topk_threshold(unsigned* __restrict__ h
   const unsigned need = rows[blockIdx.x].need, total = part[255];
   unsigned above = part[t] - sum;
   __syncthreads();
+  if (LEVEL == 0 && above == 0 && sum > 0) {  // the end of the sample's largest bin
+    int b = 0;
+    while (c[b] == 0) b++;
+    rows[blockIdx.x].kmax = ((uint32_t)(top - b) << 21) | 0x1fffffu;
+  }
   if (above < need && above + sum >= need) {
     int b = 0;
     while (above + c[b] < need) above += c[b++];
@@ -436,17 +464,17 @@ __global__ void __launch_bounds__(256) k_topk_threshold(unsigned* __restrict__ h
 template <bool VEC4>
 __global__ void __launch_bounds__(256)
     k_topk_collect(const float* __restrict__ x, int64_t count, TopkRow* __restrict__ rows, uint64_t* __restrict__ cand,
-                   int64_t cap, double* __restrict__ sq_partials) {
+                   int64_t cap, int log_nb, int* __restrict__ buckets, unsigned* __restrict__ place,
+                   double* __restrict__ sq_partials) {
   __shared__ uint64_t buf[4][512];
   __shared__ unsigned counts[4];
   __shared__ unsigned long long list_base;
-  __shared__ unsigned most;
   __shared__ double red[256];
   const int row = blockIdx.y;
-  const uint32_t thr = rows[row].thr;
-  topk_finds f{buf[threadIdx.x >> 6], 0u, cand + (int64_t)row * cap, cap, &rows[row].cursor};
+  const uint32_t thr = rows[row].thr, kmax = rows[row].kmax;
+  topk_finds f{buf[threadIdx.x >> 6], 0u, cand + (int64_t)row * cap, cap, &rows[row].cursor,
+               buckets + ((int64_t)row << log_nb), place + (int64_t)row * cap, thr, kmax, topk_shift(thr, kmax, log_nb)};
   double sq = 0.0;
-  uint32_t mine = 0;
   // (from the key of +0 up, keys are in the order of the bits as signed integers)
   const bool plain = thr >= 0x80000000u;
   const int thr_bits = (int)(thr & 0x7fffffffu);
@@ -470,60 +498,32 @@ __global__ void __launch_bounds__(256)
         const int64_t i = topk_entry<VEC4>(first, e);
         const bool take = i < count && key >= thr;
         f.put(take, key, i);
-        if (take && key > mine) mine = key;
       }
       f.flush();
     }
   });
   f.finish(counts, &list_base);
-  if (threadIdx.x == 0) most = 0;
   red[threadIdx.x] = sq;
   __syncthreads();
-  if (mine) atomicMax(&most, mine);
   for (int off = 128; off > 0; off >>= 1) {
     if ((int)threadIdx.x < off) red[threadIdx.x] += red[threadIdx.x + off];
     __syncthreads();
   }
-  if (threadIdx.x == 0) {
-    sq_partials[(int64_t)row * gridDim.x + blockIdx.x] = red[0];
-    if (most) atomicMax(&rows[row].kmax, most);
-  }
+  if (threadIdx.x == 0) sq_partials[(int64_t)row * gridDim.x + blockIdx.x] = red[0];
 }
 
-// Bucket of a key: 0 holds the largest.  All buckets span 2^shift keys.
-__device__ inline int topk_shift(uint32_t thr, uint32_t kmax, int log_nb) {
-  const uint32_t range = kmax - thr;
-  const int bits = range ? 32 - __clz(range) : 0;
-  return bits > log_nb ? bits - log_nb : 0;
-}
-__device__ inline int topk_bucket(uint32_t key, uint32_t thr, uint32_t kmax, int shift) {
-  return (int)(((kmax - thr) >> shift) - ((key - thr) >> shift));
-}
-
-__global__ void __launch_bounds__(256)
-    k_topk_bucket_count(const TopkRow* __restrict__ rows, const uint64_t* __restrict__ cand, int64_t cap, int log_nb,
-                        int* __restrict__ buckets) {
-  const TopkRow r = rows[blockIdx.y];
-  const int64_t n = (int64_t)r.cursor < cap ? (int64_t)r.cursor : cap;
-  const int shift = topk_shift(r.thr, r.kmax, log_nb);
-  int* b = buckets + ((int64_t)blockIdx.y << log_nb);
-  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256)
-    atomicAdd(&b[topk_bucket((uint32_t)(cand[(int64_t)blockIdx.y * cap + i] >> 32), r.thr, r.kmax, shift)], 1);
-}
-
-// Counts to starts (in place and once more as cursors), the row's norm, and whether the list serves.
-// (A row has one workgroup here, so a thread has at most 16 counts and loads them four at a time: 16,384
-// counts, 2 rows, 43 -> 9.5 us against 64 counts one at a time.)
+// Counts to starts (in place), the row's norm, and whether the list serves.
+// (A row has one workgroup here, so a thread has at most 16 counts and loads them four at a time, and sums go
+// by shuffles: 16,384 counts, 2 rows, 6.3 us; 9.5 with ten barriers, 43 with 64 counts one at a time.)
 constexpr int TOPK_SCAN = 1024;
 __global__ void __launch_bounds__(TOPK_SCAN)
     k_topk_bucket_scan(const TopkRow* __restrict__ rows, int64_t cap, int64_t k, int log_nb, int* __restrict__ buckets,
-                       int* __restrict__ cursors, const double* __restrict__ sq_partials, int n_sq,
+                       const double* __restrict__ sq_partials, int n_sq,
                        float* __restrict__ norms, unsigned long long* __restrict__ failed) {
-  __shared__ int part[TOPK_SCAN];
-  __shared__ double red[TOPK_SCAN];
+  __shared__ int part[TOPK_SCAN / 64];
+  __shared__ double red[TOPK_SCAN / 64];
   const int row = blockIdx.x, t = threadIdx.x, quads = ((1 << log_nb) / 4 + TOPK_SCAN - 1) / TOPK_SCAN;
   int4* b = reinterpret_cast<int4*>(buckets + ((int64_t)row << log_nb));
-  int4* c = reinterpret_cast<int4*>(cursors + ((int64_t)row << log_nb));
   const bool in = t * quads * 4 < 1 << log_nb;
   int4 v[TOPK_MAX_BUCKETS / 4 / TOPK_SCAN];
   int sum = 0, most = 0;
@@ -533,54 +533,54 @@ __global__ void __launch_bounds__(TOPK_SCAN)
     sum += v[i].x + v[i].y + v[i].z + v[i].w;
     most = max(max(max(v[i].x, v[i].y), max(v[i].z, v[i].w)), most);
   }
-  part[t] = sum;
   double s = 0.0;
   for (int i = t; i < n_sq; i += TOPK_SCAN) s += sq_partials[(int64_t)row * n_sq + i];
-  red[t] = s;
-  __syncthreads();
-  for (int off = 1; off < TOPK_SCAN; off <<= 1) {
-    const int add = t >= off ? part[t - off] : 0;
-    __syncthreads();
-    part[t] += add;
-    __syncthreads();
+  const int wave = t >> 6, lane = t & 63;
+  int incl = sum;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const int up = __shfl_up(incl, off);
+    if (lane >= off) incl += up;
   }
-  int run = part[t] - sum;
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off);
+  if (lane == 63) part[wave] = incl;
+  if (lane == 0) red[wave] = s;
+  __syncthreads();
+  int run = incl - sum;
+  for (int w = 0; w < wave; w++) run += part[w];
 #pragma unroll
   for (int i = 0; i < TOPK_MAX_BUCKETS / 4 / TOPK_SCAN; i++) {
     if (!in || i >= quads) break;
     const int4 w{run, run + v[i].x, run + v[i].x + v[i].y, run + v[i].x + v[i].y + v[i].z};
     b[t * quads + i] = w;
-    c[t * quads + i] = w;
     run = w.w + v[i].w;
   }
-  for (int off = TOPK_SCAN / 2; off > 0; off >>= 1) {
-    __syncthreads();
-    if (t < off) red[t] += red[t + off];
-  }
   if (t == 0) {
-    if (norms) norms[row] = (float)sqrt(red[0]);
+    for (int w = 1; w < TOPK_SCAN / 64; w++) s += red[w];
+    if (norms) norms[row] = (float)sqrt(s);
     if ((int64_t)rows[row].cursor < k || (int64_t)rows[row].cursor > cap) *failed = 1;
   }
   if (most > TOPK_CROWDED) *failed = 1;
 }
 
 __global__ void __launch_bounds__(256)
-    k_topk_scatter(const TopkRow* __restrict__ rows, const uint64_t* __restrict__ cand, int64_t cap, int log_nb,
-                   int* __restrict__ cursors, uint64_t* __restrict__ out) {
+    k_topk_scatter(const TopkRow* __restrict__ rows, const uint64_t* __restrict__ cand, const unsigned* __restrict__ place,
+                   int64_t cap, int log_nb, const int* __restrict__ starts, uint64_t* __restrict__ out) {
   const TopkRow r = rows[blockIdx.y];
   const int64_t n = (int64_t)r.cursor < cap ? (int64_t)r.cursor : cap;
   const int shift = topk_shift(r.thr, r.kmax, log_nb);
-  int* c = cursors + ((int64_t)blockIdx.y << log_nb);
+  const int* s = starts + ((int64_t)blockIdx.y << log_nb);
   for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
     const uint64_t p = cand[(int64_t)blockIdx.y * cap + i];
-    out[(int64_t)blockIdx.y * cap + atomicAdd(&c[topk_bucket((uint32_t)(p >> 32), r.thr, r.kmax, shift)], 1)] = p;
+    out[(int64_t)blockIdx.y * cap + s[topk_bucket((uint32_t)(p >> 32), r.thr, r.kmax, shift)] + place[(int64_t)blockIdx.y * cap + i]] = p;
   }
 }
 
 // The k first places: a pair's is its bucket's start plus the larger pairs of the bucket.
 __global__ void __launch_bounds__(256)
     k_topk_rank(const TopkRow* __restrict__ rows, const uint64_t* __restrict__ sorted, int64_t cap, int64_t k, int log_nb,
-                const int* __restrict__ starts, const int* __restrict__ ends, float* __restrict__ vals,
+                const int* __restrict__ starts, float* __restrict__ vals,
                 int32_t* __restrict__ idx) {
   const TopkRow r = rows[blockIdx.y];
   const int64_t n = (int64_t)r.cursor < cap ? (int64_t)r.cursor : cap;
@@ -589,7 +589,8 @@ __global__ void __launch_bounds__(256)
   for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
     const uint64_t own = p[i];
     const int b = topk_bucket((uint32_t)(own >> 32), r.thr, r.kmax, shift);
-    const int s = starts[((int64_t)blockIdx.y << log_nb) + b], e = ends[((int64_t)blockIdx.y << log_nb) + b];
+    const int s = starts[((int64_t)blockIdx.y << log_nb) + b];
+    const int e = b + 1 < 1 << log_nb ? starts[((int64_t)blockIdx.y << log_nb) + b + 1] : (int)n;
     if (s >= k || e - s > TOPK_CROWDED) continue;
     int rank = s;
     for (int j = s; j < e; j++) rank += p[j] > own;
@@ -631,7 +632,7 @@ static int topk_by_sample(int64_t n_rows, int64_t count, int64_t k, const float*
                           float* norms, bool* done) {
   *done = false;
   const bool sampled = count >= TOPK_SAMPLED;
-  const int64_t stride = sampled ? TOPK_STRIDE : TOPK_CHUNK, chunks = ceil_div(count, stride);
+  const int64_t stride = !sampled ? TOPK_CHUNK : k >= 8 * TOPK_STRIDE * 2 ? 2 * TOPK_STRIDE : TOPK_STRIDE, chunks = ceil_div(count, stride);
   // entries of the sample to find above the threshold: their share of k and five times its deviation
   const double share = (double)k * TOPK_CHUNK / (double)stride;
   const unsigned target = sampled ? (unsigned)(share + 5.0 * sqrt(share) + 8.0) : (unsigned)k;
@@ -652,7 +653,8 @@ static int topk_by_sample(int64_t n_rows, int64_t count, int64_t k, const float*
   dbuf<TopkRow> rows;
   dbuf<unsigned> hist;
   dbuf<uint64_t> cand, sorted;
-  dbuf<int> starts, cursors;
+  dbuf<int> starts;
+  dbuf<unsigned> place;
   dbuf<double> sq;
   const dim3 gc = blocks(count, 4096);
   DN_TRY(rows.alloc(n_rows));
@@ -660,27 +662,25 @@ static int topk_by_sample(int64_t n_rows, int64_t count, int64_t k, const float*
   DN_TRY(cand.alloc(n_rows * cap));
   DN_TRY(sorted.alloc(n_rows * cap));
   DN_TRY(starts.alloc(n_rows << log_nb));
-  DN_TRY(cursors.alloc(n_rows << log_nb));
+  DN_TRY(place.alloc(n_rows * cap));
   DN_TRY(sq.alloc(n_rows * gc.x));
   unsigned long long* failed = nullptr;
   DN_TRY(host_words(&failed));
   *failed = 0;
-  DN_HIP(hipMemsetAsync(starts, 0, sizeof(int) * (size_t)(n_rows << log_nb), st));
-  hipLaunchKernelGGL(k_topk_row_init, dim3((unsigned)n_rows), block, 0, st, rows.p, target, hist.p);
-  const dim3 gs = blocks(chunks, 64), gr((unsigned)n_rows), gp = blocks(cap, 512);
+  hipLaunchKernelGGL(k_topk_row_init, dim3((unsigned)n_rows), dim3(1024), 0, st, rows.p, target, hist.p, log_nb, starts.p);
+  const dim3 gs = blocks(chunks, 64), gr((unsigned)n_rows), gp = blocks(cap, 256);
   hipLaunchKernelGGL(k_topk_sample<0>, gs, block, 0, st, x, count, stride, chunks, rows.p, hist.p);
   hipLaunchKernelGGL(k_topk_threshold<0>, gr, block, 0, st, hist.p, rows.p);
   hipLaunchKernelGGL(k_topk_sample<1>, gs, block, 0, st, x, count, stride, chunks, rows.p, hist.p);
   hipLaunchKernelGGL(k_topk_threshold<1>, gr, block, 0, st, hist.p, rows.p);
   if (count % 4 == 0 && ((uintptr_t)x % 16) == 0)
-    hipLaunchKernelGGL(k_topk_collect<true>, gc, block, 0, st, x, count, rows.p, cand.p, cap, sq.p);
+    hipLaunchKernelGGL(k_topk_collect<true>, gc, block, 0, st, x, count, rows.p, cand.p, cap, log_nb, starts.p, place.p, sq.p);
   else
-    hipLaunchKernelGGL(k_topk_collect<false>, gc, block, 0, st, x, count, rows.p, cand.p, cap, sq.p);
-  hipLaunchKernelGGL(k_topk_bucket_count, gp, block, 0, st, rows.p, cand.p, cap, log_nb, starts.p);
-  hipLaunchKernelGGL(k_topk_bucket_scan, gr, dim3(TOPK_SCAN), 0, st, rows.p, cap, k, log_nb, starts.p, cursors.p, sq.p, (int)gc.x,
+    hipLaunchKernelGGL(k_topk_collect<false>, gc, block, 0, st, x, count, rows.p, cand.p, cap, log_nb, starts.p, place.p, sq.p);
+  hipLaunchKernelGGL(k_topk_bucket_scan, gr, dim3(TOPK_SCAN), 0, st, rows.p, cap, k, log_nb, starts.p, sq.p, (int)gc.x,
                      norms, failed);
-  hipLaunchKernelGGL(k_topk_scatter, gp, block, 0, st, rows.p, cand.p, cap, log_nb, cursors.p, sorted.p);
-  hipLaunchKernelGGL(k_topk_rank, gp, block, 0, st, rows.p, sorted.p, cap, k, log_nb, starts.p, cursors.p, vals, idx);
+  hipLaunchKernelGGL(k_topk_scatter, gp, block, 0, st, rows.p, cand.p, place.p, cap, log_nb, starts.p, sorted.p);
+  hipLaunchKernelGGL(k_topk_rank, gp, block, 0, st, rows.p, sorted.p, cap, k, log_nb, starts.p, vals, idx);
   DN_LAUNCH_CHECK();
   DN_HIP(hipStreamSynchronize(st));
   *done = *failed == 0;

@@ -38,3 +38,18 @@ def test_topk_matches_the_full_sort(kind, n, count, k):
     wv, wi, wn = orc.topk_rows(x, k)
     assert np.array_equal(v, wv) and np.array_equal(i, wi)
     assert np.allclose(nrm, wn, rtol=2e-7)
+
+
+@pytest.mark.parametrize("count,k,outliers", [(600_001, 500, 60), (700_000, 40_000, 300), (1_200_000, 33_000, 5000),
+                                              (1_200_000, 32_767, 0)])
+def test_entries_above_all_of_the_sample(count, k, outliers):
+    """Values far above the largest one sampled, where no chunk of either stride looks (64 of 2048 or of 4096
+    entries): they share the first bucket, or are too many for it."""
+    rng = np.random.default_rng(count + k)
+    x = rng.lognormal(-8, 2, count).astype(np.float32)
+    where = np.flatnonzero(np.arange(count) % 2048 >= 64)
+    x[rng.choice(where, outliers, replace=False)] = rng.lognormal(20, 1, outliers).astype(np.float32)
+    vals, idx, norms = d.topk_rows(d.DeviceArray.from_numpy(x[None, :]), k)
+    order = np.lexsort((np.arange(count), -x))[:k]
+    assert np.array_equal(idx[0], order) and np.array_equal(vals[0], x[order])
+    np.testing.assert_allclose(norms[0], np.sqrt((x.astype(np.float64) ** 2).sum()), rtol=1e-7)
