@@ -2071,16 +2071,52 @@ DN_API int dnpeff_op_xg_mu(int64_t rows, int r, const float* X, const float* G_r
   return launch_xg_mu(rows, r, X, G_rr, num, eps, out, D_out);
 }
 
+// <x, y> for the host: sixteen numbers per thread under way, a workgroup's sum straight to pinned memory, where the
+// host adds them up in order (6 M numbers: 5.5 us where k_dot_partial and k_dot_final take 7.2 and 3.5 and a launch).
+__global__ void __launch_bounds__(256)
+    k_dot_host(int64_t count, const float* __restrict__ x, const float* __restrict__ y, double* __restrict__ out) {
+  __shared__ double sh[4];
+  typedef float f4 __attribute__((ext_vector_type(4), aligned(4)));
+  double s[4] = {};
+  const int64_t quads = count / 4, stride = (int64_t)gridDim.x * 256;
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < quads; i += 4 * stride) {
+    f4 a[4], b[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) a[u] = reinterpret_cast<const f4*>(x)[i + u * stride < quads ? i + u * stride : i];
+#pragma unroll
+    for (int u = 0; u < 4; u++) b[u] = x == y ? a[u] : reinterpret_cast<const f4*>(y)[i + u * stride < quads ? i + u * stride : i];
+#pragma unroll
+    for (int u = 0; u < 4; u++)
+      if (i + u * stride < quads) {
+#pragma unroll
+        for (int c = 0; c < 4; c++) s[u] = fma((double)a[u][c], (double)b[u][c], s[u]);
+      }
+  }
+  if (blockIdx.x == 0 && threadIdx.x < (count & 3)) {
+    const int64_t i = 4 * quads + threadIdx.x;
+    s[0] = fma((double)x[i], (double)y[i], s[0]);
+  }
+  double t = (s[0] + s[1]) + (s[2] + s[3]);
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) t += __shfl_xor(t, off);
+  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = t;
+  __syncthreads();
+  if (threadIdx.x == 0) out[blockIdx.x] = ((sh[0] + sh[1]) + sh[2]) + sh[3];
+}
+
 DN_API int dnpeff_op_dot(int64_t count, const float* x, const float* y, double* out_host) {
   clear_error();
   DN_CHECK(out_host != nullptr, "out is NULL");
-  dbuf<double> ws;
-  DN_TRY(ws.alloc(DOT_BLOCKS));
-  unsigned long long* word = nullptr;
-  DN_TRY(host_words(&word));
-  DN_TRY(launch_dot(count, x, y, ws, reinterpret_cast<double*>(word)));
+  unsigned long long* words = nullptr;
+  DN_TRY(host_words(&words));
+  double* part = reinterpret_cast<double*>(words);
+  const int wgs = (int)std::max<int64_t>(1, std::min<int64_t>(HOST_WORDS, ceil_div(count, 4096)));
+  hipLaunchKernelGGL(k_dot_host, dim3((unsigned)wgs), dim3(256), 0, stream(), count, x, y, part);
+  DN_LAUNCH_CHECK();
   DN_HIP(hipStreamSynchronize(stream()));
-  *out_host = *reinterpret_cast<double*>(word);
+  double sum = 0.0;
+  for (int i = 0; i < wgs; i++) sum += part[i];
+  *out_host = sum;
   return 0;
 }
 

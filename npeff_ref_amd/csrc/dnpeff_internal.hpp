@@ -78,7 +78,8 @@ struct copy_part {
 hipError_t copy_up_parts(std::initializer_list<copy_part> parts);
 hipError_t copy_down_parts(const copy_part* parts, int n_parts);
 inline hipError_t copy_down_parts(std::initializer_list<copy_part> parts) { return copy_down_parts(parts.begin(), (int)parts.size()); }
-int host_words(unsigned long long** out);  // 64 pinned words of the calling thread
+constexpr int HOST_WORDS = 512;
+int host_words(unsigned long long** out);  // HOST_WORDS pinned words of the calling thread
 
 template <class T>
 inline int dmalloc(T** p, int64_t count) {

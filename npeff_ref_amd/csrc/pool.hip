@@ -399,7 +399,28 @@ static hipError_t bounce_copy(char* dst, const char* src, size_t bytes) {
   return e;
 }
 
-// Several short arrays down as one: kernels write them to a bounce buffer side by side, one wait for all.
+constexpr int GATHER_PARTS = 4;
+struct gather_parts {
+  const uint32_t* src[GATHER_PARTS];
+  int words[GATHER_PARTS], at[GATHER_PARTS];  // `at`: a multiple of four words
+};
+// Part blockIdx.y to dst, in 16-byte pieces where it is aligned (the rest of a part: single words).
+__global__ void __launch_bounds__(256) k_gather_parts(gather_parts p, uint32_t* __restrict__ dst) {
+  const uint32_t* src = p.src[blockIdx.y];
+  uint32_t* to = dst + p.at[blockIdx.y];
+  const int n = p.words[blockIdx.y], quads = ((uintptr_t)src & 15) == 0 ? n / 4 : 0;
+  for (int i = blockIdx.x * 1024 + threadIdx.x; i < quads; i += gridDim.x * 1024) {
+    uint4 v[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) v[u] = reinterpret_cast<const uint4*>(src)[i + 256 * u < quads ? i + 256 * u : i];
+#pragma unroll
+    for (int u = 0; u < 4; u++)
+      if (i + 256 * u < quads) reinterpret_cast<uint4*>(to)[i + 256 * u] = v[u];
+  }
+  for (int i = 4 * quads + blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) to[i] = src[i];
+}
+
+// Several short arrays down as one: a kernel writes them to a bounce buffer side by side, one wait for all.
 // (Two arrays of 240 KB: one wait and 10 us of writes where the engine's copies took two waits and 14 us each before
 // they began.)
 static hipError_t gather_down(const copy_part* parts, int n_parts) {
@@ -413,15 +434,20 @@ static hipError_t gather_down(const copy_part* parts, int n_parts) {
   }
   hipStream_t st = stream();
   size_t at = 0;
-  for (int q = 0; q < n_parts && e == hipSuccess; q++, at += (parts[q - 1].bytes + 15) / 16 * 16) {
-    const int n = (int)(parts[q].bytes / 4);
-    if (parts[q].bytes % 16 == 0 && (uintptr_t)parts[q].src % 16 == 0) {
-      e = piece_copy(B.p + at, parts[q].src, parts[q].bytes, hipMemcpyDeviceToHost, st);
-    } else {
-      hipLaunchKernelGGL(k_copy_words, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, (const uint32_t*)parts[q].src,
-                         (uint32_t*)(B.p + at), n);
-      e = hipGetLastError();
+  for (int q = 0; q < n_parts && e == hipSuccess; q += GATHER_PARTS) {
+    gather_parts g = {};
+    size_t most = 0;
+    for (int i = 0; i < GATHER_PARTS && q + i < n_parts; i++) {
+      const copy_part& p = parts[q + i];
+      g.src[i] = (const uint32_t*)p.src;
+      g.words[i] = (int)(p.bytes / 4);
+      g.at[i] = (int)(at / 4);
+      at += (p.bytes + 15) / 16 * 16;
+      most = most > p.bytes ? most : p.bytes;
     }
+    const int wgs = (int)((most + 16383) / 16384);
+    hipLaunchKernelGGL(k_gather_parts, dim3(wgs < COPY_WGS ? wgs : COPY_WGS, GATHER_PARTS), dim3(256), 0, st, g, (uint32_t*)B.p);
+    e = hipGetLastError();
   }
   const hipError_t es = hipStreamSynchronize(st);
   if (e == hipSuccess) e = es;
@@ -480,7 +506,7 @@ hipError_t copy_down(void* dst_host, const void* src_dev, size_t bytes) {
 int host_words(unsigned long long** out) {
   static thread_local unsigned long long* words = nullptr;
   if (!words) {
-    DN_HIP(hipHostMalloc((void**)&words, 64 * sizeof(unsigned long long), hipHostMallocDefault));
+    DN_HIP(hipHostMalloc((void**)&words, HOST_WORDS * sizeof(unsigned long long), hipHostMallocDefault));
   }
   *out = words;
   return 0;

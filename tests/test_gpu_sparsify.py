@@ -93,3 +93,17 @@ def test_context_method_projects_W_and_the_loop_goes_on():
     other.close()
     nmf.close()
     A.close()
+
+
+@pytest.mark.parametrize("count", [0, 1, 3, 4, 4095, 4097, 16_387, 2_100_003])
+@pytest.mark.parametrize("same", [True, False])
+def test_dot_of_any_length(count, same):
+    """Remainders of four, one workgroup and all of them, x with itself and with another: fp64 sums of exact
+    products, 1e-12."""
+    rng = np.random.default_rng(count)
+    a = rng.standard_normal(max(count, 1)).astype(np.float32)[:count]
+    b = a if same else rng.standard_normal(max(count, 1)).astype(np.float32)[:count]
+    x = d.DeviceArray.from_numpy(a)
+    y = x if same else d.DeviceArray.from_numpy(b)
+    want = float((a.astype(np.float64) * b.astype(np.float64)).sum())
+    assert abs(d.op_dot(x, y) - want) <= 1e-12 * max(1.0, float(np.abs(a.astype(np.float64) * b).sum()))
