@@ -312,7 +312,8 @@ struct fused_plan {
   int32_t* x_col = nullptr;
   float* x_val = nullptr;
   int64_t* x_seg = nullptr;
-  int x_parts = 0;
+  int* x_base = nullptr;     // as n_base
+  int x_parts = 0;           // (-1: looked at, the rows do not suit it)
 };
 
 }  // namespace dn

@@ -857,7 +857,7 @@ __global__ void __launch_bounds__(256)
 void fused_drop(dnpeff_csr* S) {
   fused_plan& f = S->fused;
   dfree(f.tiles); dfree(f.pairs); dfree(f.chunks); dfree(f.n_base);
-  dfree(f.x_col); dfree(f.x_val); dfree(f.x_seg);
+  dfree(f.x_col); dfree(f.x_val); dfree(f.x_seg); dfree(f.x_base);
   f = fused_plan();
 }
 
@@ -973,13 +973,19 @@ __global__ void __launch_bounds__(256)
 // in one piece has all the rare columns on the last XCD, whose misses are then waited for (777 x 862k, r = 50: 126
 // us; with columns dealt one by one two XCDs share every line of short rows).  k_fu_n at 777 x 862k, r = 50 / 512 x 431k, r = 16
 // / 300 x 146k, r = 20: 74.7 / 17.2 / 10.2 us, in chunks of whole rows 117 / 21.5 / 11.0.
+// Up to 96 components: above, runs amplify the rounding of every sum (20 iterations at 772 x 467k, r = 128, end 1.7e-5
+// apart in the one order and the other, at r <= 64 5e-6 at most), and keep the order they have always had.
 // Rows of FU_XCD_ROW entries or more on average, of which none is twice as long (a workgroup per row and XCD).  Ten iterations
 // in chunks of whole rows / by XCD: 191 / 215 us at 200 rows of 200 entries, r = 8, 252 / 281 at 500 of 512, r = 16, 488 / 546 at
 // 1000 of 1024, r = 32 (a workgroup has 128 entries then), 782 / 788 at 2000 of 2048, r = 8, 796 / 754 at 300 of 2048, r = 64,
 // 5880 / 5476 at 1000 of 4096, r = 96, 9751 / 8205 at 2000 of 8192, r = 60.
+static bool by_xcd(const fused_plan& f, int r) { return f.x_seg && r <= FU_XCD_RANK; }
+static const int* first_chunks(const fused_plan& f, int r) { return by_xcd(f, r) ? f.x_base : f.n_base; }
+
 static int fused_xcd_build(dnpeff_csr* S) {
   fused_plan& f = S->fused;
   const int64_t n = S->n_rows, mean = S->nnz / n;
+  f.x_parts = -1;
   if (mean < FU_XCD_ROW || !xcd_round_robin()) return 0;
   std::vector<int64_t> rowptr((size_t)n + 1);
   DN_HIP(copy_down(rowptr.data(), S->rowptr, sizeof(int64_t) * rowptr.size()));
@@ -1001,9 +1007,8 @@ static int fused_xcd_build(dnpeff_csr* S) {
   f.x_seg = seg.release();
   f.x_col = col.release();
   f.x_val = val.release();
-  f.n_base = base.release();
+  f.x_base = base.release();
   f.x_parts = (int)parts;
-  f.n_chunks = 8 * n * parts;
   return 0;
 }
 
@@ -1020,10 +1025,12 @@ int fused_plan_build(dnpeff_csr* S, int r) {
     DN_LAUNCH_CHECK();
   }
   DN_TRY(fused_tiles_build(S, r));
-  if (!f.chunks && !f.x_seg && S->n_panels == 0) {
+  if (r <= FU_XCD_RANK && f.x_parts == 0 && S->n_panels == 0) {
     DN_CHECK(has_row_major(S), "row-major copy of the matrix was released");
     DN_TRY(fused_xcd_build(S));
-    if (f.x_seg) return 0;
+  }
+  if (!f.chunks && !by_xcd(f, r) && S->n_panels == 0) {
+    DN_CHECK(has_row_major(S), "row-major copy of the matrix was released");
     const int64_t chunk = fu_chunk_entries(S->nnz);
     dbuf<int64_t> base;
     DN_TRY(base.alloc(S->n_rows + 1));
@@ -1158,17 +1165,18 @@ int fused_state::gram_of(const float* X, int64_t rows, bool of_h) {
 
 int fused_state::product_n(const dnpeff_csr* S, const float* H) {
   const fused_plan& f = S->fused;
-  DN_CHECK((has_row_major(S) && f.chunks) || f.x_seg, "row-major copy of the matrix was released");
-  if (n_part_floats < f.n_chunks * r + 4) {
+  const bool xcd = by_xcd(f, r);
+  DN_CHECK(xcd || (has_row_major(S) && f.chunks), "row-major copy of the matrix was released");
+  const int64_t chunks = xcd ? 8 * S->n_rows * f.x_parts : f.n_chunks;
+  if (n_part_floats < chunks * r + 4) {
     dfree(n_part);
     n_part = nullptr;
-    n_part_floats = f.n_chunks * r + 4;
+    n_part_floats = chunks * r + 4;
     DN_TRY(dmalloc(&n_part, n_part_floats));
   }
   const int sums = gh_state == PARTS ? (int)ceil_div(S_floats / 16, 8) * 8 : 0;
-  const dim3 grid((unsigned)(f.n_chunks + sums)), block(256);
+  const dim3 grid((unsigned)(chunks + sums)), block(256);
   if (grid.x > 0) {
-    const bool xcd = f.x_seg != nullptr;
     auto go = [&](auto kernel) {
       hipLaunchKernelGGL(kernel, grid, block, 0, stream(), f.chunks, f.x_seg, f.x_parts, xcd ? f.x_col : S->colind,
                          xcd ? f.x_val : S->vals, r, H, n_part, sums, gh_part, h_wgs, S_floats, gh_sum);
@@ -1203,7 +1211,7 @@ int fused_state::sum_w() {
 int fused_state::update_w(const dnpeff_csr* S, int64_t n, const float* Nw, float* W, float eps) {
   DN_CHECK(gh_state == SUMMED, "H^T H is not at hand");
   const float* N = Nw ? Nw : n_part;
-  const int* base = Nw ? nullptr : S->fused.n_base;
+  const int* base = Nw ? nullptr : first_chunks(S->fused, r);
   if (r > FUSED_NARROW_RANK)
     DN_TRY(fuw_launch_w(w_wgs, n, r, base, N, W, eps, gh_sum, gw_part));
   else DN_TRY(fu_dispatch(r, [&](auto tag) {
@@ -1237,7 +1245,7 @@ int fused_state::loss_sums(const dnpeff_csr* S, int64_t n, const float* Nw, cons
   DN_TRY(sum_h());
   DN_TRY(sum_w());
   const int parts = (int)ceil_div(n, 16);
-  hipLaunchKernelGGL(k_fu_dot, dim3((unsigned)parts), dim3(256), 0, stream(), n, r, Nw ? nullptr : S->fused.n_base,
+  hipLaunchKernelGGL(k_fu_dot, dim3((unsigned)parts), dim3(256), 0, stream(), n, r, Nw ? nullptr : first_chunks(S->fused, r),
                      Nw ? Nw : n_part, W, dots);
   hipLaunchKernelGGL(k_fu_loss, dim3(1), dim3(256), 0, stream(), dots, parts, r, gw_sum, gh_sum, out2);
   DN_LAUNCH_CHECK();

@@ -16,7 +16,8 @@ constexpr int FUW_COLS = 32;           // columns (rows of W) per tile there
 // (those are summed in fp64): a column with large entries takes bits from all that is added after it.  Above
 // 64 components half of them where that takes no more than two rounds of workgroups.
 constexpr int FU_MOST_COLS = 2048;
-constexpr int64_t FU_XCD_ROW = 1792;  // entries of a row from which they are grouped by XCD
+constexpr int FU_XCD_RANK = 96;        // ranks up to which, and entries of a row from which, A H^T goes by XCD
+constexpr int64_t FU_XCD_ROW = 1792;
 constexpr int64_t FU_CHUNKS = 4096;  // workgroups that A H^T is cut into where its rows allow
 
 bool fused_supported(int64_t n, int64_t m, int64_t nnz, int r);

@@ -264,3 +264,29 @@ def test_runs_in_one_workgroup(n, m, r, fill):
     sq, pos, neg = one[2]
     assert abs(sq + pos - 2 * neg - losses[-1] ** 2) <= 1e-5 * sq
     A.close()
+
+
+def test_ranks_on_either_side_of_the_grouping():
+    """Contexts of 40 and of 100 components on one matrix, whose rows the first groups by XCD: each gives the bits
+    that it gives on a matrix of its own, whichever comes first."""
+    n, m = 120, 6000
+    rp, ci, va = _matrix(n, m, seed=3, fill=0.35)
+
+    def run(A, r):
+        nmf = d.MuNmf(A, d.MuNmfParams(rank=r, max_iters=3, eps=EPS, seed=5, log_every=3))
+        nmf.run(log=lambda s: None)
+        out = nmf.loadWToHostSync(), nmf.loadHToHostSync()
+        nmf.close()
+        return out
+
+    alone = {}
+    for r in (40, 100):
+        A = d.Csr.from_host(rp, ci, va, m)
+        alone[r] = run(A, r)
+        A.close()
+    for order in ((40, 100, 40), (100, 40, 100)):
+        A = d.Csr.from_host(rp, ci, va, m)
+        for r in order:
+            for got, want in zip(run(A, r), alone[r]):
+                assert np.array_equal(got, want)
+        A.close()
