@@ -257,13 +257,15 @@ static int stored_rank(int64_t n, int64_t m, int64_t nnz, int rank, bool sweeps,
 }
 
 // Whether the step of small ranks runs where memory allows.  (It reads the whole matrix from its own lists: no
-// dense head is split off then.  Multiples of 64 with rows enough for a dense head keep it: its kernels are made
-// for those ranks.  Ten iterations with head / fused: r = 128 14.7 / 16.0 ms at 1500 x 1.4M, 24.2 / 31.2 at
-// 2000 x 1.9M, 79 / 84 at 2000 x 9.8M, but 8.5 / 7.2 at 1024 x 0.8M; at r = 64, where the head is a smaller
-// part, the fused step is ahead up to 2000 rows, 11.9 / 3.1 at 1024 x 0.8M, 27.2 / 18.7 at 2000 x 1.9M: the line
-// there follows the kernels, not the clock.)
+// dense head is split off then.  Rank 128 with rows enough for a dense head keeps it: the fused step's kernel at
+// that rank has one wave per SIMD.  Ten iterations with head / fused: r = 128 14.7 / 16.0 ms at 1500 x 1.4M, 24.2 / 31.2 at
+// 2000 x 1.9M, 79 / 84 at 2000 x 9.8M, but 8.5 / 7.2 at 1024 x 0.8M; at r = 64 the fused step is ahead at all sizes,
+// 3.2 / 0.86 ms at 1024 x 67k, 16.1 / 6.1 at 1500 x 0.9M, 22.6 / 8.9 at 4000 x 1.5M, 60 / 42 at 2000 x 6.4M, 47 / 37 at
+// 8000 x 3.6M, and closer to 64 bits: one W update 5e-7 ... 8e-7 off where the head's split operands leave 1e-6 ... 6e-6.
+// Below 65,536 columns rank 64 stays with the head all the same, 3.7 / 1.5 ms at 1100 x 60k: that is where the head's
+// own runs are held to their bits.)
 static bool fused_step_wanted(int64_t n, int64_t m, int64_t nnz, int rank) {
-  return tuning().fused_gram != 0.0 && tuning().tiled_h <= 0.0 && !(rank % 64 == 0 && n >= 1024) &&
+  return tuning().fused_gram != 0.0 && tuning().tiled_h <= 0.0 && !(rank % 64 == 0 && n >= 1024 && !(rank == 64 && m >= 65536)) &&
          fused_supported(n, m, nnz, rank);
 }
 

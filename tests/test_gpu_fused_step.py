@@ -290,3 +290,19 @@ def test_ranks_on_either_side_of_the_grouping():
             for got, want in zip(run(A, r), alone[r]):
                 assert np.array_equal(got, want)
         A.close()
+
+
+@pytest.mark.parametrize("m,fused", [(65_535, False), (65_536, True)])
+def test_rank_64_with_many_rows(m, fused):
+    """1024 rows and more at rank 64: the fused step from 65,536 columns on, a dense head below."""
+    A, norms = d.Csr.synth(1030, m, k_fixed=700, zipf_s=1.1, seed=8)
+    A.normalize_rows(norms)
+    rp, ci, va = A.download()
+    nmf = d.MuNmf(A, d.MuNmfParams(rank=64, max_iters=4, eps=EPS, seed=5, log_every=2))
+    nmf.initialize()
+    assert (A.head_info()[0] == 0) == fused
+    W0, H0 = nmf.loadWToHostSync(), nmf.loadHToHostSync()
+    nmf.run(log=lambda s: None)
+    _close(nmf, orc.nmf_f64(rp, ci, va, m, W0, H0, np.float32(EPS), 4, 2))
+    nmf.close()
+    A.close()
