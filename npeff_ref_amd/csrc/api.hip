@@ -993,8 +993,7 @@ DN_API int dnpeff_fit_create(dnpeff_csr* A, dnpeff_csr* H, float eps, int64_t se
   int s = dmalloc(&f->AH, nr) || dmalloc(&f->HH, (int64_t)r * r) || dmalloc(&f->W, nr) ||
           dmalloc(&f->WHH, nr) || dmalloc(&f->dot_ws, dots);
   if (!s && !f->in_place) s = dmalloc(&f->W2, nr) || dmalloc(&f->tmp, nr);
-  if (!s) s = dnpeff_op_spsp_dense(H, H, f->HH);
-  if (!s) s = dnpeff_op_spsp_dense(A, H, f->AH);
+  if (!s) s = spsp_first_stage(A, H, f->HH, f->AH);
   if (!s) s = dnpeff_csr_sq_norm(A, &f->sq_norm_A);
   if (!s && hipStreamSynchronize(stream()) != hipSuccess) {
     set_error("first stage kernels failed");
@@ -1048,9 +1047,14 @@ DN_API int dnpeff_fit_loss(dnpeff_fit* f, double* reference_loss, double* true_l
   if (f->in_place) {
     unsigned long long* words = nullptr;
     DN_TRY(host_words(&words));
-    double* sums = reinterpret_cast<double*>(words);
-    DN_TRY(launch_fit_loss(f->n, f->r, f->W, f->HH, f->AH, f->whh_valid ? f->WHH : nullptr, f->dot_ws, sums));
+    double* out = reinterpret_cast<double*>(words);
+    const int64_t parts = fit_loss_parts(f->n);
+    const bool here = 3 * parts <= HOST_WORDS;  // (the workgroups' sums, added up here in order)
+    DN_TRY(launch_fit_loss(f->n, f->r, f->W, f->HH, f->AH, f->whh_valid ? f->WHH : nullptr, here ? out : f->dot_ws,
+                           here ? nullptr : out));
     DN_HIP(hipStreamSynchronize(stream()));
+    double sums[3] = {out[0], out[1], out[2]};
+    for (int64_t q = 3; here && q < 3 * parts; q++) sums[q % 3] += out[q];
     const double pos_ref = f->whh_valid ? sums[2] : sums[1];
     if (true_loss) *true_loss = std::sqrt(f->sq_norm_A + sums[1] - 2.0 * sums[0]);
     if (reference_loss) *reference_loss = std::sqrt(f->sq_norm_A + pos_ref - 2.0 * sums[0]);

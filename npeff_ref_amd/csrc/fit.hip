@@ -217,7 +217,7 @@ int launch_fit_loss(int64_t n, int r, const float* W, const float* G, const floa
     hipLaunchKernelGGL(k_fit_loss<RP>, dim3((unsigned)ceil_div(n, FIT_ROWS)), dim3(2 * RP), 0, stream(), W, G, AH,
                        WHH, n, r, partials);
   });
-  hipLaunchKernelGGL(k_fit_loss_sum, dim3(1), dim3(192), 0, stream(), partials, fit_loss_parts(n), out3);
+  if (out3) hipLaunchKernelGGL(k_fit_loss_sum, dim3(1), dim3(192), 0, stream(), partials, fit_loss_parts(n), out3);
   DN_LAUNCH_CHECK();
   return 0;
 }
