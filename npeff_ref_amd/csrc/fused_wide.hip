@@ -159,7 +159,33 @@ __global__ void __launch_bounds__(256, 2) k_fuw(const fuw_args p) {
     request(td);
   }
 
-  // the wave's rows of G, split: row 16 (b0 + bi) + l16, components 32 s + 8 g ..
+  // the wave's rows of G, split: row 16 (b0 + bi) + l16, components 32 s + 8 g ..  The partial matrices come through
+  // LDS in 16-byte pieces, all of a matrix under way at once; every lane picking its numbers from memory, eight at a
+  // time, is a chain of trips (W update at 467 x 67 23.1 us, now 15.8, at 300 x 100 26.2 and 19.1; H update at
+  // 467 x 84k, 67 components 66.8 and 64.2).  The H update of eight blocks stays with that: its loop has no register to
+  // spare and spills more behind the other prologue (3.4 M columns: 1.80 ms, 1.87 with it).
+  constexpr bool STAGED = !(COLS && NB == 8);
+  float* stage = reinterpret_cast<float*>(lds);
+  if constexpr (STAGED) {
+    constexpr int S = fu_pairs(NB) * 256, Q = (S + 1023) / 1024;
+    double sum[Q][4] = {};
+    for (int q = 0; q < p.n_g; q++) {
+      const float* src = p.g + (int64_t)q * S;
+      f32x4 v[Q];
+#pragma unroll
+      for (int u = 0; u < Q; u++) v[u] = *reinterpret_cast<const f32x4*>(src + (1024 * u + 4 * tid < S ? 1024 * u + 4 * tid : 0));
+#pragma unroll
+      for (int u = 0; u < Q; u++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) sum[u][i] += (double)v[u][i];
+    }
+#pragma unroll
+    for (int u = 0; u < Q; u++)
+      if (1024 * u + 4 * tid < S)
+        *reinterpret_cast<f32x4*>(stage + 1024 * u + 4 * tid) =
+            f32x4{(float)sum[u][0], (float)sum[u][1], (float)sum[u][2], (float)sum[u][3]};
+    __syncthreads();
+  }
   bf16x8 gh[BPW][NS], gm[BPW][NS], gl[BPW][NS];
 #pragma unroll
   for (int bi = 0; bi < BPW; bi++)
@@ -167,26 +193,33 @@ __global__ void __launch_bounds__(256, 2) k_fuw(const fuw_args p) {
     for (int s = 0; s < NS; s++) {
       const int lane = fuw_lane(), c = 16 * (b0 + bi) + (lane & 15);
       int at[8];
-      double sum[8];
 #pragma unroll
       for (int t = 0; t < 8; t++) {
         const int k = 32 * s + 8 * (lane >> 4) + t, bk = k >> 4, bc = c >> 4;
         const int x = bk <= bc ? fu_pair(bk, bc, NB) * 256 + (k & 15) * 16 + (c & 15)
                                : fu_pair(bc, bk, NB) * 256 + (c & 15) * 16 + (k & 15);
         at[t] = k < r && c < r ? x : -1;
-        sum[t] = 0.0;
-      }
-      for (int q = 0; q < p.n_g; q++) {  // (eight numbers of a part at a time under way)
-        const float* src = p.g + (int64_t)q * (fu_pairs(NB) * 256);
-        float w[8];
-#pragma unroll
-        for (int t = 0; t < 8; t++) w[t] = src[at[t] < 0 ? 0 : at[t]];
-#pragma unroll
-        for (int t = 0; t < 8; t++) sum[t] += (double)w[t];
       }
       f32x4 v[2];
+      if constexpr (STAGED) {
 #pragma unroll
-      for (int t = 0; t < 8; t++) v[t >> 2][t & 3] = at[t] < 0 ? 0.0f : (float)sum[t];
+        for (int t = 0; t < 8; t++) {
+          const float w = stage[at[t] < 0 ? 0 : at[t]];
+          v[t >> 2][t & 3] = at[t] < 0 ? 0.0f : w;
+        }
+      } else {
+        double sum[8] = {};
+        for (int q = 0; q < p.n_g; q++) {
+          const float* src = p.g + (int64_t)q * (fu_pairs(NB) * 256);
+          float w[8];
+#pragma unroll
+          for (int t = 0; t < 8; t++) w[t] = src[at[t] < 0 ? 0 : at[t]];
+#pragma unroll
+          for (int t = 0; t < 8; t++) sum[t] += (double)w[t];
+        }
+#pragma unroll
+        for (int t = 0; t < 8; t++) v[t >> 2][t & 3] = at[t] < 0 ? 0.0f : (float)sum[t];
+      }
       bf16x4 h0, m0, l0, h1, m1, l1;
       split3(v[0], h0, m0, l0);
       split3(v[1], h1, m1, l1);
@@ -194,6 +227,7 @@ __global__ void __launch_bounds__(256, 2) k_fuw(const fuw_args p) {
       gm[bi][s] = cat8(m0, m1);
       gl[bi][s] = cat8(l0, l1);
     }
+  if constexpr (STAGED) __syncthreads();
   f32x4 acc[NA];
 #pragma unroll
   for (int q = 0; q < NA; q++) acc[q] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
@@ -257,14 +291,24 @@ __global__ void __launch_bounds__(256, 2) k_fuw(const fuw_args p) {
     for (int jp = 0; jp < JPW; jp++) {
       const int jl = 16 * (jb0 + jp) + l16;
       const int64_t i = (int64_t)tl * FUW_COLS + (in_tile(at, jl) ? jl : 0);
-      const int64_t k0 = p.n_base ? p.n_base[i] : i, k1 = p.n_base ? p.n_base[i + 1] : i + 1;
+      const int k0 = p.n_base ? p.n_base[i] : (int)i, k1 = p.n_base ? p.n_base[i + 1] : (int)i + 1;
 #pragma unroll
       for (int bi = 0; bi < BPW; bi++) t[jp][bi] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll 2
-      for (int64_t k = k0; k < k1; k++)
+      for (int k = k0; k < k1; k += 4) {  // (four chunk sums under way)
+        f32x4 v[4][BPW];
 #pragma unroll
-        for (int bi = 0; bi < BPW; bi++)
-          if (b0 + bi < NB) t[jp][bi] += fuw_load4(p.N + k * r, 16 * (b0 + bi) + 4 * g, r, 16 * (b0 + bi) + 16 <= r);
+        for (int u = 0; u < 4; u++)
+#pragma unroll
+          for (int bi = 0; bi < BPW; bi++)
+            v[u][bi] = b0 + bi < NB ? fuw_load4(p.N + (int64_t)(k + u < k1 ? k + u : k) * r, 16 * (b0 + bi) + 4 * g, r, 16 * (b0 + bi) + 16 <= r)
+                                    : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+          if (k + u < k1) {
+#pragma unroll
+            for (int bi = 0; bi < BPW; bi++) t[jp][bi] += v[u][bi];
+          }
+      }
     }
   }
   split_x();
