@@ -666,7 +666,7 @@ static int update_H_tiled_overlapped(dnpeff_nmf* h) {
   DN_TRY(h->prof.begin(DNPEFF_K_SPMM_T));
   DN_TRY(launch_head_t_product(A, r, h->W));
   DN_TRY(h->prof.end());
-  DN_TRY(xg_mu_hold_g(h->G, r));
+  DN_TRY(xg_mu_hold_g(h->G, r, tile));
   DN_HIP(hipEventRecord(fork, s0));
   DN_HIP(hipStreamWaitEvent(s1, fork, 0));
   for (int64_t q = 0; q < n_tiles; q++) {
@@ -704,10 +704,10 @@ static int update_H_tiled(dnpeff_nmf* h) {
   DN_TRY(h->prof.begin(DNPEFF_K_SPMM_T));
   DN_TRY(launch_head_t_product(A, r, h->W));
   DN_TRY(h->prof.end());
-  struct held_g {  // G transposed once for all tiles
+  struct held_g {  // one copy of G for all tiles
     ~held_g() { xg_mu_release_g(); }
   } hold;
-  DN_TRY(xg_mu_hold_g(h->G, r));
+  DN_TRY(xg_mu_hold_g(h->G, r, tile));
   for (int64_t q = 0; q < n_tiles; q++) {
     const int64_t t = up ? n_tiles - 1 - q : q;
     const int64_t c0 = t * tile, c1 = c0 + tile < h->m ? c0 + tile : h->m;
@@ -1028,10 +1028,10 @@ DN_API int dnpeff_fit_step(dnpeff_fit* f, int n_steps) {
     f->whh_valid = true;
     return launch_fit_steps(f->n, f->r, f->W, f->HH, f->AH, f->eps, n_steps, f->WHH);
   }
-  struct held_g {  // H H^T is the same in every step: one transposed copy for all of them
+  struct held_g {  // H H^T is the same in every step: one copy for all of them
     ~held_g() { xg_mu_release_g(); }
   } hold;
-  DN_TRY(xg_mu_hold_g(f->HH, f->r));
+  DN_TRY(xg_mu_hold_g(f->HH, f->r, f->n));
   for (int s = 0; s < n_steps; s++) {
     DN_TRY(launch_xg_mu(f->n, f->r, f->W, f->HH, f->AH, f->eps, f->W2, f->WHH));
     std::swap(f->W, f->W2);

@@ -1131,37 +1131,258 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))
   finish(3, pn[1], px[1]);
 }
 
-// G transposed for the split-operand update: a buffer that grows to the largest rank seen and
-// lives until the process ends (one host thread drives the library).
-static float* g_gt = nullptr;
-static int64_t g_gt_floats = 0;
-// The G (and rank) whose transpose g_gt holds for a run of calls, between xg_mu_hold_g and
-// xg_mu_release_g: the column tiles of one H update all multiply by the same G.
-static const float* g_gt_of = nullptr;
-static int g_gt_rank = 0;
+// The same update for ranks that are multiples of 256, on tiles of 128 x 256: same products in the same
+// order, same bits.
+//
+// What bounds the tile kernels above is vector work beside the matrix instructions and, behind it, power
+// (MFMA busy 46 %, vector 45 % of the SIMD cycles at 1.72 GHz; 2 M rows, r = 256): every workgroup splits
+// its rows of X and all of G again.  Here G comes split (k_xg_mu_planes: the LDS image of every step, copied
+// with six 16-byte loads and stores per thread), a wave owns 64 x 128 elements, so X is split once per 256
+// columns, and a contraction step of 16 lets both LDS buffers of two workgroups fit a CU (72 KB each), one
+// barrier a step.  A row's 16 elements of a part lie in 32 bytes, the tile's one after the other: a 16-byte
+// read of a wave covers 1 KB without gaps (pieces exchanged by row as in abt_mainloop64: 2 % slower).  The
+// epilogue takes half a block of 32 x 32 at a time, through uniform row pointers and one offset per lane
+// (64-bit addresses per lane and whole blocks: 116 bytes of spills, 8 % slower), and past the caches: its
+// operands are used once here, and the X tiles still to be read stay in L2 (2 %).
+// 1.79 against 1.87 ms on 2 M rows at r = 256, 2.90 against 2.96 on 1 M rows at r = 512 (vector work 23 %
+// of the cycles, MFMA 43 / 57 % at 1.96 / 1.83 GHz, both before the stores past the caches); at a sustained
+// load 1.89 against 1.99 and 2.90 against 3.10.  Tried: tiles of 128 x 128 with three workgroups per CU
+// (1.77 / 2.96 alone, no gain at a sustained load), a raised wave priority around the matrix part (3 %
+// slower).
+constexpr int XGW_KB = 16;                       // contraction elements of a step
+constexpr int XGW_APLANE = 128 * XGW_KB * 2;     // bytes of one part of the X tile
+constexpr int XGW_BPLANE = 256 * XGW_KB * 2;
+constexpr int XGW_IMAGE = 3 * XGW_BPLANE;        // G's parts for a step and a column chunk
+constexpr int XGW_BUF = 3 * XGW_APLANE + XGW_IMAGE;
+constexpr int XGW_LDS = 2 * XGW_BUF;
+
+// G's parts as the steps of k_xg_mu_wide_b16 hold them in LDS: [chunk of 256 columns][step of 16
+// rows of G][part][column][16 elements].  A thread takes a column of a step.
+__global__ void __launch_bounds__(64) k_xg_mu_planes(const float* __restrict__ G, int r, unsigned char* __restrict__ image) {
+  const int step = blockIdx.x, col = 64 * blockIdx.y + threadIdx.x;
+  float g[XGW_KB];
+#pragma unroll
+  for (int k = 0; k < XGW_KB; k++) g[k] = G[(int64_t)(XGW_KB * step + k) * r + col];
+  unsigned char* dst = image + ((int64_t)(col >> 8) * (r / XGW_KB) + step) * XGW_IMAGE + (col & 255) * (2 * XGW_KB);
+#pragma unroll
+  for (int q = 0; q < XGW_KB; q += 8) {
+    bf16x4 h[2], m[2], l[2];
+#pragma unroll
+    for (int u = 0; u < 2; u++) split3(f32x4{g[q + 4 * u], g[q + 4 * u + 1], g[q + 4 * u + 2], g[q + 4 * u + 3]}, h[u], m[u], l[u]);
+    *reinterpret_cast<bf16x8*>(dst + 2 * q) = cat8(h[0], h[1]);
+    *reinterpret_cast<bf16x8*>(dst + XGW_BPLANE + 2 * q) = cat8(m[0], m[1]);
+    *reinterpret_cast<bf16x8*>(dst + 2 * XGW_BPLANE + 2 * q) = cat8(l[0], l[1]);
+  }
+}
+
+template <bool WITH_D>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
+    k_xg_mu_wide_b16(const float* __restrict__ X, const unsigned char* __restrict__ image, const float* num,
+                     float eps, int64_t n_row_tiles, int r, int n_chunks, float* out,
+                     float* __restrict__ D_out) {
+  extern __shared__ __align__(16) unsigned char ab[];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int l32 = lane & 31, half = lane >> 5;
+  const int wm = wave >> 1, wn = wave & 1;
+  const int64_t grp = blockIdx.x / (8 * n_chunks);
+  const int rem = (int)(blockIdx.x % (8 * n_chunks));
+  const int64_t tile = grp * 8 + rem % 8;
+  if (tile >= n_row_tiles) return;
+  const int chunk = rem / 8;
+  const int64_t row0 = tile * 128;
+  const int steps = r / XGW_KB;
+
+  abt_acc16 acc[2][4];
+#pragma unroll
+  for (int i = 0; i < 2; i++)
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+#pragma unroll
+      for (int v = 0; v < 16; v++) acc[i][j][v] = 0.0f;
+
+  // X: four threads a row, two rows a thread; G's parts: six pieces of 16 bytes a thread, as they lie
+  const float* xsrc = X + (row0 + (threadIdx.x >> 2)) * (int64_t)r + 4 * (threadIdx.x & 3);
+  const unsigned char* gsrc = image + (int64_t)chunk * steps * XGW_IMAGE + 16 * threadIdx.x;
+  f32x4 xs[2][2];
+  f32x4 gs[6];
+  auto fetch_x = [&](int s, int t) {
+    const float* p = xsrc + XGW_KB * (t < steps ? t : steps - 1);
+#pragma unroll
+    for (int q = 0; q < 2; q++) xs[s][q] = *reinterpret_cast<const f32x4*>(p + (int64_t)(64 * q) * r);
+  };
+  auto fetch_g = [&](int t) {
+    const unsigned char* p = gsrc + (int64_t)(t < steps ? t : steps - 1) * XGW_IMAGE;
+#pragma unroll
+    for (int q = 0; q < 6; q++) gs[q] = *reinterpret_cast<const f32x4*>(p + 4096 * q);
+  };
+  auto commit = [&](int s, unsigned char* buf) {
+#pragma unroll
+    for (int q = 0; q < 6; q++) *reinterpret_cast<f32x4*>(buf + 3 * XGW_APLANE + 4096 * q + 16 * threadIdx.x) = gs[q];
+#pragma unroll
+    for (int q = 0; q < 2; q++) {
+      bf16x4 h, m, l;
+      split3(xs[s][q], h, m, l);
+      unsigned char* dst = buf + 2048 * q + 8 * threadIdx.x;
+      *reinterpret_cast<bf16x4*>(dst) = h;
+      *reinterpret_cast<bf16x4*>(dst + XGW_APLANE) = m;
+      *reinterpret_cast<bf16x4*>(dst + 2 * XGW_APLANE) = l;
+    }
+  };
+  const int a_at = (64 * wm + l32) * (2 * XGW_KB) + 16 * half;
+  const int b_at = 3 * XGW_APLANE + (128 * wn + l32) * (2 * XGW_KB) + 16 * half;
+  auto mfma_step = [&](const unsigned char* buf) {
+    bf16x8 ah[2], am[2], al[2];
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+      const unsigned char* pa = buf + a_at + 32 * i * (2 * XGW_KB);
+      ah[i] = *reinterpret_cast<const bf16x8*>(pa);
+      am[i] = *reinterpret_cast<const bf16x8*>(pa + XGW_APLANE);
+      al[i] = *reinterpret_cast<const bf16x8*>(pa + 2 * XGW_APLANE);
+    }
+#pragma unroll
+    for (int jp = 0; jp < 4; jp += 2) {
+      bf16x8 bh[2], bm[2], bl[2];
+#pragma unroll
+      for (int j = 0; j < 2; j++) {
+        const unsigned char* pb = buf + b_at + 32 * (jp + j) * (2 * XGW_KB);
+        bh[j] = *reinterpret_cast<const bf16x8*>(pb);
+        bm[j] = *reinterpret_cast<const bf16x8*>(pb + XGW_BPLANE);
+        bl[j] = *reinterpret_cast<const bf16x8*>(pb + 2 * XGW_BPLANE);
+      }
+#define XGW_TERM(P, Q)                                                                          \
+  _Pragma("unroll") for (int i = 0; i < 2; i++) _Pragma("unroll") for (int j = 0; j < 2; j++)    \
+      acc[i][jp + j] = DN_MFMA_B16(P[i], Q[j], acc[i][jp + j]);
+      XGW_TERM(ah, bh)
+      XGW_TERM(ah, bm)
+      XGW_TERM(am, bh)
+      XGW_TERM(ah, bl)
+      XGW_TERM(al, bh)
+      XGW_TERM(am, bm)
+#undef XGW_TERM
+    }
+  };
+  fetch_x(0, 0);
+  fetch_g(0);
+  fetch_x(1, 1);
+  commit(0, ab);
+  fetch_g(1);
+  fetch_x(0, 2);
+  __syncthreads();
+  for (int t = 0; t < steps; t += 2) {
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+      mfma_step(ab + u * XGW_BUF);
+      commit(u ^ 1, ab + (u ^ 1) * XGW_BUF);
+      fetch_g(t + u + 2);
+      fetch_x(u ^ 1, t + u + 3);
+      __syncthreads();
+    }
+  }
+
+  // Element (i, j, v): row 64 wm + 32 i + 8 (v / 4) + 4 half + v % 4, column 128 wn + 32 j + l32 of the
+  // chunk: a uniform pointer per row and block, one offset in bytes per lane.
+  const int64_t t0 = (row0 + 64 * wm) * (int64_t)r + 256 * chunk + 128 * wn;
+  const unsigned lane_at = 4u * (unsigned)(4 * half * r + l32);
+  auto at = [&](int i, int j, int v) { return t0 + (int64_t)(32 * i + 8 * (v >> 2) + (v & 3)) * r + 32 * j; };
+  auto load = [&](const float* p) {
+    return __builtin_nontemporal_load(reinterpret_cast<const float*>(reinterpret_cast<const char*>(p) + lane_at));
+  };
+  auto store = [&](float* p, float x) {
+    __builtin_nontemporal_store(x, reinterpret_cast<float*>(reinterpret_cast<char*>(p) + lane_at));
+  };
+  // half a block (eight elements) at a time, the next one's operands on their way
+  float pn[2][8], px[2][8];
+  auto request = [&](int hb, float (&n_)[8], float (&x_)[8]) {
+#pragma unroll
+    for (int v = 0; v < 8; v++) {
+      const int64_t e = at(hb >> 3, (hb >> 1) & 3, 8 * (hb & 1) + v);
+      n_[v] = load(num + e);
+      x_[v] = load(X + e);
+    }
+  };
+  auto finish = [&](int hb, const float (&n_)[8], const float (&x_)[8]) {
+    const int i = hb >> 3, j = (hb >> 1) & 3;
+#pragma unroll
+    for (int v4 = 0; v4 < 8; v4 += 4) {
+      f32x4 n4, d4;
+#pragma unroll
+      for (int u = 0; u < 4; u++) {
+        n4[u] = n_[v4 + u];
+        d4[u] = acc[i][j][8 * (hb & 1) + v4 + u];
+      }
+      const f32x4 q = mu_quotients(n4, d4 + eps);
+#pragma unroll
+      for (int u = 0; u < 4; u++) {
+        const int64_t e = at(i, j, 8 * (hb & 1) + v4 + u);
+        store(out + e, x_[v4 + u] * q[u]);
+        if (WITH_D) store(D_out + e, d4[u]);
+      }
+    }
+  };
+  request(0, pn[0], px[0]);
+#pragma unroll
+  for (int hb = 0; hb < 16; hb++) {
+    if (hb < 15) request(hb + 1, pn[(hb + 1) & 1], px[(hb + 1) & 1]);
+    finish(hb, pn[hb & 1], px[hb & 1]);
+  }
+}
+
+// Copies of G for the split-operand updates, transposed or as LDS images of its parts: a buffer each
+// that grows to the largest rank seen and lives until the process ends (one host thread drives the
+// library).  `of` (and rank): the G whose copy a buffer holds for a run of calls, between
+// xg_mu_hold_g and xg_mu_release_g: the column tiles of one H update all multiply by the same G.
+struct g_copy {
+  float* buf = nullptr;
+  int64_t floats = 0;
+  const float* of = nullptr;
+  int rank = 0;
+  bool holds(const float* G, int r) const { return of == G && rank == r; }
+  int room(int64_t need) {
+    if (floats >= need) return 0;
+    DN_HIP(hipStreamSynchronize(stream()));
+    dfree(buf);
+    buf = nullptr;
+    floats = 0;
+    of = nullptr;
+    DN_TRY(dmalloc(&buf, need));
+    floats = need;
+    return 0;
+  }
+};
+static g_copy g_gt, g_image;
 
 static int xg_mu_transpose_g(const float* G, int r) {
-  if (g_gt_floats < (int64_t)r * r) {
-    DN_HIP(hipStreamSynchronize(stream()));
-    dfree(g_gt);
-    g_gt = nullptr;
-    g_gt_floats = 0;
-    g_gt_of = nullptr;
-    DN_TRY(dmalloc(&g_gt, (int64_t)r * r));
-    g_gt_floats = (int64_t)r * r;
-  }
-  return launch_transpose(r, r, G, g_gt);
+  DN_TRY(g_gt.room((int64_t)r * r));
+  return launch_transpose(r, r, G, g_gt.buf);
 }
-
-int xg_mu_hold_g(const float* G, int r) {
-  g_gt_of = nullptr;
-  if (!(use_split_bf16() && r > 128 && r % 128 == 0 && ((uintptr_t)G % 16) == 0)) return 0;  // (no transposed G on that path)
-  DN_TRY(xg_mu_transpose_g(G, r));
-  g_gt_of = G;
-  g_gt_rank = r;
+static int xg_mu_image_g(const float* G, int r) {
+  DN_TRY(g_image.room((int64_t)r * r * 3 / 2));
+  hipLaunchKernelGGL(k_xg_mu_planes, dim3((unsigned)(r / XGW_KB), (unsigned)(r / 64)), dim3(64), 0, stream(), G, r,
+                     reinterpret_cast<unsigned char*>(g_image.buf));
+  DN_LAUNCH_CHECK();
   return 0;
 }
-void xg_mu_release_g() { g_gt_of = nullptr; }
+
+// Tiles of 128 x 256 need two rounds of two workgroups per CU: 141 against 148 us at 132 000 x 256, 218
+// against 222 at 66 000 x 512, 240 against 248 at 20 000 x 1024; with fewer the last, partly filled round
+// weighs more than with tiles of half the size (115 against 115 at 100 000 x 256, 93 against 79 at 66 000).
+static bool xg_mu_wide(int64_t rows, int r) {
+  if (r % 256 != 0) return false;
+  const double w = tuning().xg_wgs;
+  return w >= 5.0 || (w == 3.0 && rows / 128 * (r / 256) >= 4 * (int64_t)n_cus());
+}
+
+int xg_mu_hold_g(const float* G, int r, int64_t rows) {
+  xg_mu_release_g();
+  if (!(use_split_bf16() && r > 128 && r % 128 == 0 && ((uintptr_t)G % 16) == 0)) return 0;  // (no copy of G on that path)
+  const bool wide = xg_mu_wide(rows, r);
+  DN_TRY(wide ? xg_mu_image_g(G, r) : xg_mu_transpose_g(G, r));
+  g_copy& c = wide ? g_image : g_gt;
+  c.of = G;
+  c.rank = r;
+  return 0;
+}
+void xg_mu_release_g() { g_gt.of = g_image.of = nullptr; }
 
 static int launch_xg_mu_tile_b16(int64_t rows, int r, const float* X, const float* G, const float* num,
                                  float eps, float* out, float* D_out, int64_t rows_there) {
@@ -1171,14 +1392,20 @@ static int launch_xg_mu_tile_b16(int64_t rows, int r, const float* X, const floa
                                hipFuncAttributeMaxDynamicSharedMemorySize, ABT_LDS));
     DN_HIP(hipFuncSetAttribute((const void*)k_xg_mu_tile_b16<true>,
                                hipFuncAttributeMaxDynamicSharedMemorySize, ABT_LDS));
+    DN_HIP(hipFuncSetAttribute((const void*)k_xg_mu_wide_b16<false>,
+                               hipFuncAttributeMaxDynamicSharedMemorySize, XGW_LDS));
+    DN_HIP(hipFuncSetAttribute((const void*)k_xg_mu_wide_b16<true>,
+                               hipFuncAttributeMaxDynamicSharedMemorySize, XGW_LDS));
     attr_set = true;
   }
-  if (!(g_gt_of == G && g_gt_rank == r)) DN_TRY(xg_mu_transpose_g(G, r));
-  const int n_chunks = r / 128;
   // (where the arrays go on to the end of the last tile, it is a whole one: the fp32 kernel on fewer than
   // 128 rows takes 25 to 55 us, as long as 40 million elements of the whole tiles)
   if (!D_out && rows_there >= ceil_div(rows, 128) * 128) rows = ceil_div(rows, 128) * 128;
   const int64_t tiles = rows / 128;
+  const bool wide = !g_gt.holds(G, r) && (g_image.holds(G, r) || xg_mu_wide(rows, r));
+  if (wide && !g_image.holds(G, r)) DN_TRY(xg_mu_image_g(G, r));
+  if (!wide && !g_gt.holds(G, r)) DN_TRY(xg_mu_transpose_g(G, r));
+  const int n_chunks = r / (wide ? 256 : 128);
   // The last rows (fewer than 128, through the fp32 kernel: two workgroups that take a third of
   // the time of a few hundred row tiles) run on the second stream beside the whole tiles.
   const int64_t head = tiles * 128;
@@ -1195,21 +1422,28 @@ static int launch_xg_mu_tile_b16(int64_t rows, int r, const float* X, const floa
     const int64_t wgs = ceil_div(tiles, 8) * 8 * n_chunks;
     DN_CHECK(wgs < ((int64_t)1 << 24), "xg_mu: too many tiles for one launch");
     const dim3 grid((unsigned)wgs), block(256);
-    // three workgroups per CU on planes without padding, where the launch fills them several
+    // Tiles of 128 columns: three workgroups per CU on planes without padding, where the launch fills them several
     // times over (a workgroup of three takes longer than one of two: few row tiles, as in the
     // fixed-H learner's W update, are done sooner two per CU)
     const bool three = tuning().xg_wgs >= 4.0 || (tuning().xg_wgs >= 3.0 && wgs >= 8 * 3 * (int64_t)n_cus());
-    if (three && D_out)
-      hipLaunchKernelGGL((k_xg_mu_tile_b16_w3<true>), grid, block, ABT_LDS64, stream(), X, g_gt, num, eps,
+    const unsigned char* image = reinterpret_cast<const unsigned char*>(g_image.buf);
+    if (wide && D_out)
+      hipLaunchKernelGGL((k_xg_mu_wide_b16<true>), grid, block, XGW_LDS, stream(), X, image, num, eps, tiles, r,
+                         n_chunks, out, D_out);
+    else if (wide)
+      hipLaunchKernelGGL((k_xg_mu_wide_b16<false>), grid, block, XGW_LDS, stream(), X, image, num, eps, tiles, r,
+                         n_chunks, out, D_out);
+    else if (three && D_out)
+      hipLaunchKernelGGL((k_xg_mu_tile_b16_w3<true>), grid, block, ABT_LDS64, stream(), X, g_gt.buf, num, eps,
                          tiles, r, n_chunks, out, D_out);
     else if (three)
-      hipLaunchKernelGGL((k_xg_mu_tile_b16_w3<false>), grid, block, ABT_LDS64, stream(), X, g_gt, num, eps,
+      hipLaunchKernelGGL((k_xg_mu_tile_b16_w3<false>), grid, block, ABT_LDS64, stream(), X, g_gt.buf, num, eps,
                          tiles, r, n_chunks, out, D_out);
     else if (D_out)
-      hipLaunchKernelGGL((k_xg_mu_tile_b16<true>), grid, block, ABT_LDS, stream(), X, g_gt, num, eps,
+      hipLaunchKernelGGL((k_xg_mu_tile_b16<true>), grid, block, ABT_LDS, stream(), X, g_gt.buf, num, eps,
                          tiles, r, n_chunks, out, D_out);
     else
-      hipLaunchKernelGGL((k_xg_mu_tile_b16<false>), grid, block, ABT_LDS, stream(), X, g_gt, num, eps,
+      hipLaunchKernelGGL((k_xg_mu_tile_b16<false>), grid, block, ABT_LDS, stream(), X, g_gt.buf, num, eps,
                          tiles, r, n_chunks, out, D_out);
     DN_LAUNCH_CHECK();
   }

@@ -143,9 +143,9 @@ int launch_gram(int64_t rows, int r, const float* X, float* G, float* workspace,
 // ranks 256, 384, ..., 1024 (head.hip)
 int64_t gram_tiles_workspace_floats(int64_t rows, int r, int64_t run);
 int launch_gram_tiles(int64_t rows, int r, const float* X, float* G, float* workspace, int64_t run);
-// Between the two, launch_xg_mu calls with this G reuse one transposed copy of it (the caller
-// must not change G in between).
-int xg_mu_hold_g(const float* G, int r);
+// Between the two, launch_xg_mu calls with this G and up to `rows` rows reuse one copy of it, transposed
+// or split as their kernel takes it (the caller must not change G in between).
+int xg_mu_hold_g(const float* G, int r, int64_t rows);
 void xg_mu_release_g();
 // rows_there: rows that X, num and out have memory for (0: `rows`); up to the next multiple of 128 they
 // may be read and overwritten with anything.
@@ -218,7 +218,7 @@ struct tuning_t {
   double nl_lag = 0.0;             // pieces the workgroups of an XCD may be apart
   double gram_beside = 1.0;        // H^T H of the W update on a second stream beside the dense head and the plain panels of A H^T (0 = after A H^T)
   double h_overlap = 0.0;          // tiled H update: A^T W of the next tile beside the update of this one (two streams, two tile buffers)
-  double xg_wgs = 3.0;             // workgroups per CU of the r >= 256 update kernel: 3 where the launch fills the CUs eight times, 4 = three always, 2 = two (padded planes, two operand stages)
+  double xg_wgs = 3.0;             // the r >= 256 update: 3 = by rule (tiles of 256 columns, else three or two workgroups per CU), 5 = tiles of 256 columns where r allows, 4 = three per CU, 2 = two (padded planes, two operand stages)
   double gram_fold = 2.0;          // X^T X on tiles: 2 = diagonal squares of 256 columns in one workgroup where the rank is a
                                    // multiple of 256, else as 1 = diagonal tiles of 128 with their symmetry; 0 = all sixteen blocks
   double nl_wgs = 64.0;            // workgroups of the slot-list kernel per XCD (two per CU)

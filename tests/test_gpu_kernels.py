@@ -158,6 +158,32 @@ def test_xg_mu_tiles_with_two_and_three_workgroups_per_cu(rows, r, tune):
     assert np.array_equal(dout.numpy(), outs[0][0])
 
 
+@pytest.mark.parametrize("rows,r", [(256, 256), (1153, 256), (131200, 256), (383, 512), (2300, 512), (300, 768),
+                                    (513, 1024)])
+def test_xg_mu_tiles_of_256_columns(rows, r, tune):
+    """Tiles of 128 x 256 on a G split beforehand: the products of the tiles of 128 x 128 in the same
+    order, so the same bits; 131 200 rows are past the line from which they run by themselves."""
+    rng = np.random.default_rng(rows + r)
+    X = (rng.random((rows, r)) * 10.0 ** rng.uniform(-3, 3, size=(1, r))).astype(np.float32)
+    G = (rng.random((r, r)) * 10.0 ** rng.uniform(-2, 2, size=(r, 1))).astype(np.float32)  # (not symmetric)
+    num = rng.random((rows, r)).astype(np.float32)
+    eps = np.float32(1e-8)
+    dX, dG, dnum = d.DeviceArray.from_numpy(X), d.DeviceArray.from_numpy(G), d.DeviceArray.from_numpy(num)
+    outs = []
+    for wgs in (2, 5, 3):
+        tune("xg_wgs", wgs)
+        dout, dD, dout2 = d.DeviceArray((rows, r)), d.DeviceArray((rows, r)), d.DeviceArray((rows, r))
+        d.op_xg_mu(dX, dG, dnum, eps, dout, dD)
+        d.op_xg_mu(dX, dG, dnum, eps, dout2, None)
+        outs.append((dout.numpy(), dD.numpy()))
+        assert np.array_equal(dout2.numpy(), outs[-1][0])
+    for o in outs[1:]:
+        assert np.array_equal(o[0], outs[0][0]) and np.array_equal(o[1], outs[0][1])
+    some = slice(0, rows, max(1, rows // 2000))
+    want, wantD = orc.xg_mu_f64(X[some], G, num[some], eps)
+    assert _rel(outs[1][1][some], wantD) < TOL and _rel(outs[1][0][some], want) < TOL
+
+
 @pytest.mark.parametrize("split", ["1", "0"])
 @pytest.mark.parametrize("rows", [64, 95, 4100, 70001, 300033])
 def test_xg_mu_gram_fused(rows, split, tune):
