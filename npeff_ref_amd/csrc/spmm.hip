@@ -9,6 +9,7 @@
 // summation orders are fixed by the matrix structure, so results are
 // reproducible run to run.
 #include "dnpeff_internal.hpp"
+#include "split_bf16.hpp"
 
 #include <algorithm>
 #include <cstdlib>
@@ -885,7 +886,8 @@ __global__ void __launch_bounds__(256)
 // (k_spmm_t_grouped gives a wave 32 whole columns one after the other at these ranks: 180 us where the
 // first 32 columns of 100 rows hold every row, and a gather's latency per column everywhere: 500 x 823k with
 // 4 M entries 637 us at r = 256, 1087 at r = 512; here 305 and 531.)
-template <int V, bool FULL>
+// PAST: the rows of T go past the L2s, which a large W then keeps (spmm_t_past).
+template <int V, bool FULL, bool PAST>
 __global__ void __launch_bounds__(256)
     k_spmm_t_bal(const fu_tile* __restrict__ tiles, const int64_t* __restrict__ colptr,
                  const int32_t* __restrict__ rowind, const float* __restrict__ tvals, int r,
@@ -907,6 +909,14 @@ __global__ void __launch_bounds__(256)
 #pragma unroll
     for (int v = 0; v < V; v++)
       if (FULL || 4 * (lane + 64 * v) < r) *reinterpret_cast<float4*>(dst + 4 * (lane + 64 * v)) = a[v];
+  };
+  auto put_t = [&](int col, const float4 (&a)[V]) {
+    float* dst = Tt + (int64_t)col * r;
+    if constexpr (!PAST) return put(dst, a);
+#pragma unroll
+    for (int v = 0; v < V; v++)
+      if (FULL || 4 * (lane + 64 * v) < r)
+        __builtin_nontemporal_store(f32x4{a[v].x, a[v].y, a[v].z, a[v].w}, reinterpret_cast<f32x4*>(dst + 4 * (lane + 64 * v)));
   };
   const float4 zero = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
   float4 acc[V];
@@ -949,7 +959,7 @@ __global__ void __launch_bounds__(256)
           const int e = b + u + k;
           if (e < s1) {
             while (e >= next) {  // column c is complete
-              put(Tt + (int64_t)c * r, acc);
+              put_t(c, acc);
               next = bcast_i(cp, ++c + 1);
 #pragma unroll
               for (int v = 0; v < V; v++) acc[v] = zero;
@@ -971,7 +981,7 @@ __global__ void __launch_bounds__(256)
   }
   if (whole) {
     for (; c < c1; c++) {  // the last column (and columns without entries)
-      put(Tt + (int64_t)c * r, acc);
+      put_t(c, acc);
 #pragma unroll
       for (int v = 0; v < V; v++) acc[v] = zero;
     }
@@ -1536,6 +1546,13 @@ bool use_spmm_t_bal(const dnpeff_csr* S, int r) {
          S->nnz > 0 && S->n_cols > 0 && ceil_div(S->n_cols, 32) + S->nnz / 256 < ((int64_t)1 << 24);
 }
 
+// Rows of T past the L2s where W takes two fifths of one (4 MB): the stores else push rows of W out.
+// k_spmm_t_bal with plain stores / past the L2s, us: 3094 / 2936 at 2000 rows of 256 floats (2.0 MB) and 12 M
+// columns, 1976 / 1863 at 2000 x 384, 1488 / 1424 at 1500 x 384, 786 / 779 at 1200 x 512, 1560 / 1521 at 800 x
+// 512 (1.6 MB), 1246 / 1247 at 1600 x 256 (1.6 MB); below the line T does better in the caches: 479 / 494 at
+// 1000 x 384 (1.5 MB), 170 / 176 at 600 x 256.
+static bool spmm_t_past(int64_t n, int r) { return n * r * (int64_t)sizeof(float) >= 1600000; }
+
 // The sparse part of rows [col0, col1) of A^T W into T (row j - col0); long_cols[l0 .. l1) are the
 // long columns in that range.
 static int launch_spmm_t_sparse(const dnpeff_csr* A, int r, const float* W_nr, float* T, int64_t col0,
@@ -1560,19 +1577,22 @@ static int launch_spmm_t_sparse(const dnpeff_csr* A, int r, const float* W_nr, f
     DN_CHECK(t1 - t0 < ((int64_t)1 << 24), "too many tiles for one launch");
     const dim3 gb((unsigned)(t1 - t0)), bb(256);
     const size_t lds = sizeof(float) * 4 * (size_t)r;
+    const bool past = spmm_t_past(A->n_rows, r);
+#define DN_BAL_KERNEL(V, FULL, PAST)                                                                                \
+  hipLaunchKernelGGL((k_spmm_t_bal<V, FULL, PAST>), gb, bb, lds, stream(), A->fused.tiles + t0, A->colptr,          \
+                     A->rowind, A->tvals, r, W_nr, T, col0)
 #define DN_BAL(V)                                                                                                   \
   do {                                                                                                              \
-    if (r == 256 * V)                                                                                               \
-      hipLaunchKernelGGL((k_spmm_t_bal<V, true>), gb, bb, lds, stream(), A->fused.tiles + t0, A->colptr, A->rowind, \
-                         A->tvals, r, W_nr, T, col0);                                                               \
-    else                                                                                                            \
-      hipLaunchKernelGGL((k_spmm_t_bal<V, false>), gb, bb, lds, stream(), A->fused.tiles + t0, A->colptr,           \
-                         A->rowind, A->tvals, r, W_nr, T, col0);                                                    \
+    if (r == 256 * V && past) DN_BAL_KERNEL(V, true, true);                                                         \
+    else if (r == 256 * V) DN_BAL_KERNEL(V, true, false);                                                           \
+    else if (past) DN_BAL_KERNEL(V, false, true);                                                                   \
+    else DN_BAL_KERNEL(V, false, false);                                                                            \
   } while (0)
     if (r <= 256) DN_BAL(1);
     else if (r <= 512) DN_BAL(2);
     else DN_BAL(4);
 #undef DN_BAL
+#undef DN_BAL_KERNEL
     DN_LAUNCH_CHECK();
     return 0;
   }

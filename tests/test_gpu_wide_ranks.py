@@ -33,6 +33,31 @@ def test_spmm_t_balanced(n, m, r):
     A.close()
 
 
+@pytest.mark.parametrize("n,r", [(1562, 256), (1563, 256), (1600, 252), (782, 512), (820, 492), (500, 1000)])
+def test_spmm_t_balanced_on_a_large_factor(n, r):
+    """On both sides of 1.6 MB of W, from which on the result goes past the caches."""
+    m = 150
+    rng = np.random.default_rng(n + r)
+    mask = rng.random((n, m)) < rng.choice([0.0, 0.003, 0.3, 1.0], size=m)
+    mask[0, 0] = True
+    rp = np.concatenate([[0], np.cumsum(mask.sum(axis=1))]).astype(np.int64)
+    ci = np.nonzero(mask)[1].astype(np.int32)
+    va = rng.random(len(ci)).astype(np.float32)
+    A = d.Csr.from_host(rp, ci, va, m)
+    W = rng.random((n, r)).astype(np.float32)
+    dW, dT = d.DeviceArray.from_numpy(W), d.DeviceArray.from_numpy(np.full((m + 1, r), np.nan, dtype=np.float32))
+    d.op_spmm_t(A, r, dW, dT)
+    d.sync()
+    dense = np.zeros((n, m))
+    dense[mask] = va
+    want = dense.T @ W.astype(np.float64)
+    got = dT.numpy()
+    # (sums of up to n products of numbers below 1: n roundings of at most 2^-24 of the largest sum each)
+    assert np.abs(got[:m] - want).max() <= n * 2.0 ** -24 * max(1.0, np.abs(want).max())
+    assert np.isnan(got[m]).all()
+    A.close()
+
+
 @pytest.mark.parametrize("r", [132, 256, 600])
 def test_spmm_t_tile_at_any_column(r):
     """Tiles on and off the groups of 32 columns: the rows of the whole product, bit for bit."""
