@@ -887,18 +887,46 @@ __global__ void __launch_bounds__(256)
 // first 32 columns of 100 rows hold every row, and a gather's latency per column everywhere: 500 x 823k with
 // 4 M entries 637 us at r = 256, 1087 at r = 512; here 305 and 531.)
 // PAST: the rows of T go past the L2s, which a large W then keeps (spmm_t_past).
+// Tiles of full columns are bound by their gathers, tiles of nearly empty ones by their stores (6.4 of the 33 GB
+// that 2000 x 5.8 M moves at rank 256; without the stores 1.25 ms, with them but every gather in L1 2.0), and
+// columns are often sorted by their entries: the workgroups, by eights (one per XCD), take tiles from `places`
+// places of the list in turn, so that both kinds run side by side.  (Powers of two below the number of
+// workgroups a CU holds put all full tiles on the same CUs: 3564 us with 4 places.)  With a light tile's
+// entries asked for beside the columns' ends: 2318 -> 2140 us there, 2127 -> 1940 at rank 512.  Tried: several tiles per
+// workgroup with the next one's entries on their way (rank 512 1980, rank 256 2350), 16 gathers in flight
+// (2366), a way without bounds checks for whole groups (2380).
 template <int V, bool FULL, bool PAST>
 __global__ void __launch_bounds__(256)
-    k_spmm_t_bal(const fu_tile* __restrict__ tiles, const int64_t* __restrict__ colptr,
+    k_spmm_t_bal(const fu_tile* __restrict__ tiles, int places, const int64_t* __restrict__ colptr,
                  const int32_t* __restrict__ rowind, const float* __restrict__ tvals, int r,
                  const float* __restrict__ W, float* __restrict__ T, int64_t col_base) {
   extern __shared__ __align__(16) float parts[];  // [4][r] of a long column
   constexpr int U = V == 1 ? 8 : V == 2 ? 4 : 2;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-  const int64_t e0 = tiles[blockIdx.x].e0;
-  const int col0 = tiles[blockIdx.x].col0, nc = tiles[blockIdx.x].cols;
-  const int E = (int)(tiles[blockIdx.x + 1].e0 - e0);
+  int at = blockIdx.x;
+  {
+    const int each = (int)gridDim.x / 8 / places, eight = at / 8;
+    if (eight < each * places) at = (eight % places * each + eight / places) * 8 + at % 8;
+  }
+  const int64_t e0 = tiles[at].e0;
+  const int col0 = tiles[at].col0, nc = tiles[at].cols;
+  const int E = (int)(tiles[at + 1].e0 - e0);
   const bool whole = nc > 1 || E <= SPMM_T_LONG;
+  // The wave's share of the entries begins at b0.  Of a tile of few entries its first 64 are asked for beside
+  // the columns' ends.
+  const int share = (E + 3) / 4, per = (share + 63) / 64 * 64;
+  const int b0 = wave * (whole ? share : per);
+  auto entry = [&](int e) {  // (of a tile without entries: the one before it, or the first)
+    const int64_t i = e0 + (e < E ? e : E - 1);
+    return i > 0 ? i : 0;
+  };
+  int mi = 0;
+  float mv = 0.0f;
+  const bool few = E <= 256;
+  if (few) {
+    mi = rowind[entry(b0 + lane)];
+    mv = tvals[entry(b0 + lane)];
+  }
   float* Tt = T + (int64_t)(col0 - col_base) * r;
   // lane l: first entry of column l of the tile (past the last column: E)
   const int cp = lane < nc ? (int)(colptr[col0 + lane] - e0) : E;
@@ -925,28 +953,28 @@ __global__ void __launch_bounds__(256)
   // the wave's columns [c, c1) and entries [s0, s1)
   int c = 0, c1 = 1, s0, s1;
   if (whole) {
-    const int share = (E + 3) / 4;
     c = (int)__popcll(__ballot(lane < nc && cp < wave * share));
     c1 = wave == 3 ? nc : (int)__popcll(__ballot(lane < nc && cp < (wave + 1) * share));
     s0 = bcast_i(cp, c);
     s1 = bcast_i(cp, c1);
   } else {
-    const int per = ((E + 3) / 4 + 63) / 64 * 64;
-    s0 = wave * per < E ? wave * per : E;
+    s0 = b0 < E ? b0 : E;
     s1 = s0 + per < E ? s0 + per : E;
   }
-  int next = whole ? bcast_i(cp, c + 1) : E;
+  int next = (whole ? bcast_i(cp, c + 1) : E) - s0;  // where column c ends in the share
   if (s0 < s1) {
-    const int32_t* ri = rowind + e0;
-    const float* va = tvals + e0;
-    int mi = ri[s0 + lane < s1 ? s0 + lane : s1 - 1];
-    float mv = va[s0 + lane < s1 ? s0 + lane : s1 - 1];
-    for (int b = s0; b < s1; b += 64) {
+    // (a share may begin with the rest of the column before it: those entries are passed over)
+    int b = b0;
+    if (!few || s0 - b0 >= 64) {
+      b = s0;
+      mi = rowind[entry(b + lane)];
+      mv = tvals[entry(b + lane)];
+    }
+    for (int u = (s0 - b) / U * U; b < s1; b += 64, u = 0) {
       const int cnt = s1 - b < 64 ? s1 - b : 64;
-      const int ne = b + 64 + lane < s1 ? b + 64 + lane : s1 - 1;
-      const int ni = ri[ne];
-      const float nv = va[ne];
-      for (int u = 0; u < cnt; u += U) {
+      const int ni = rowind[entry(b + 64 + lane)];
+      const float nv = tvals[entry(b + 64 + lane)];
+      for (; u < cnt; u += U) {
         float4 h[U][V];
 #pragma unroll
         for (int k = 0; k < U; k++) {
@@ -956,11 +984,11 @@ __global__ void __launch_bounds__(256)
         }
 #pragma unroll
         for (int k = 0; k < U; k++) {
-          const int e = b + u + k;
-          if (e < s1) {
+          const int e = b + u + k - s0;  // (entry of the share; below 0: passed over)
+          if ((unsigned)e < (unsigned)(s1 - s0)) {
             while (e >= next) {  // column c is complete
               put_t(c, acc);
-              next = bcast_i(cp, ++c + 1);
+              next = bcast_i(cp, ++c + 1) - s0;
 #pragma unroll
               for (int v = 0; v < V; v++) acc[v] = zero;
             }
@@ -1575,12 +1603,16 @@ static int launch_spmm_t_sparse(const dnpeff_csr* A, int r, const float* W_nr, f
       t1 = A->fused.h_first[ceil_div(col1, 32)];
     }
     DN_CHECK(t1 - t0 < ((int64_t)1 << 24), "too many tiles for one launch");
+    // (as many places as 8 workgroups per CU make eights, twice over: 2290 / 2145 / 2135 us with 1 / 256 / 512 of
+    // them at 2000 x 5.8 M, rank 256, 1388 / 1322 / 1327 at 1500 x 1.6 M, rank 384, 1956 / 2062 / 1950 at 1500 x
+    // 2.9 M, rank 512)
+    const int places = 2 * n_cus();
     const dim3 gb((unsigned)(t1 - t0)), bb(256);
     const size_t lds = sizeof(float) * 4 * (size_t)r;
     const bool past = spmm_t_past(A->n_rows, r);
 #define DN_BAL_KERNEL(V, FULL, PAST)                                                                                \
-  hipLaunchKernelGGL((k_spmm_t_bal<V, FULL, PAST>), gb, bb, lds, stream(), A->fused.tiles + t0, A->colptr,          \
-                     A->rowind, A->tvals, r, W_nr, T, col0)
+  hipLaunchKernelGGL((k_spmm_t_bal<V, FULL, PAST>), gb, bb, lds, stream(), A->fused.tiles + t0, places, \
+                     A->colptr, A->rowind, A->tvals, r, W_nr, T, col0)
 #define DN_BAL(V)                                                                                                   \
   do {                                                                                                              \
     if (r == 256 * V && past) DN_BAL_KERNEL(V, true, true);                                                         \

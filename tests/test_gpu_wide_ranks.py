@@ -58,6 +58,25 @@ def test_spmm_t_balanced_on_a_large_factor(n, r):
     A.close()
 
 
+@pytest.mark.parametrize("m", [32 * 4095, 32 * 4096, 32 * 4109 + 5])
+def test_spmm_t_balanced_dealt_tiles(m):
+    """Fewer, as many and more tiles than there are places to deal them from, with a rest."""
+    n, r = 5, 132
+    rng = np.random.default_rng(m)
+    mask = rng.random((n, m)) < 0.3
+    rp = np.concatenate([[0], np.cumsum(mask.sum(axis=1))]).astype(np.int64)
+    va = rng.random(int(rp[-1])).astype(np.float32)
+    A = d.Csr.from_host(rp, np.nonzero(mask)[1].astype(np.int32), va, m)
+    W = rng.random((n, r)).astype(np.float32)
+    dW, dT = d.DeviceArray.from_numpy(W), d.DeviceArray.from_numpy(np.full((m, r), np.nan, dtype=np.float32))
+    d.op_spmm_t(A, r, dW, dT)
+    d.sync()
+    dense = np.zeros((n, m))
+    dense[mask] = va
+    assert np.abs(dT.numpy() - dense.T @ W).max() <= n * 2.0 ** -24 * n
+    A.close()
+
+
 @pytest.mark.parametrize("r", [132, 256, 600])
 def test_spmm_t_tile_at_any_column(r):
     """Tiles on and off the groups of 32 columns: the rows of the whole product, bit for bit."""
