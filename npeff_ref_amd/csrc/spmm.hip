@@ -228,6 +228,99 @@ __global__ void __launch_bounds__(256)
   }
 }
 
+// The same sums for ranks above 128 on slices of 4 LPR components: LPR lanes gather a slice of a row of H,
+// and the 64 / LPR lane groups of a wave take a quarter of a chunk each, U gathers in flight.  Workgroup b has
+// slice b % slices of 64 / LPR consecutive chunks.
+//
+// k_spmm_n gives a quarter of a chunk to a wave with four (two above rank 256) gathers in flight: 512 entries
+// of one row after the other are 128 to 256 trips.  Here they are 32, and with 8 slices (rank 512) an XCD only ever
+// holds its eighth of the rows in its L2: 56 -> 37 us at 300 rows of 1000 entries, rank 256, 360 -> 341 at 800 x
+// 4000 (3.3 GB of rows, mostly from the fabric), 110 -> 73 at 1000 x 500 and 177 -> 126 at 250 x 3000, rank 512, 192 ->
+// 171 at 400 x 3000, rank 384; 37.6 -> 39.0 at 1800 x 300, rank 256, where the L2s bound either.  LPR 8 / 16 / 32 /
+// 64 at 300 x 1000, rank 256: 46 / 41 / 37 / 39; at rank 512, 250 x 3000: 161 / 126 / 133 / 170.  Every sum is added up
+// in the order of k_spmm_n: the same bits.
+template <int LPR>
+__global__ void __launch_bounds__(256)
+    k_spmm_n_slices(const int64_t* __restrict__ rowptr, const int32_t* __restrict__ colind,
+                    const float* __restrict__ vals, const int64_t* __restrict__ chunk_base, int64_t n_rows,
+                    int64_t n_chunks, int slices, int r, const float* __restrict__ H, float* __restrict__ partials) {
+  constexpr int G = 64 / LPR, WIDTH = 4 * LPR, U = 16;
+  __shared__ __align__(16) float red[4 * G * WIDTH];  // [chunk][quarter][component]
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int grp = lane / LPR, sub = lane % LPR;
+  const int slice = blockIdx.x % slices;
+  const int64_t first = (int64_t)(blockIdx.x / slices) * G;
+  const int64_t chunk = first + grp;  // (a wave has one quarter: those that short rows lack are whole waves)
+  int64_t row = chunk_to_row(chunk_base, n_rows, first);
+  while (row + 1 < n_rows && chunk_base[row + 1] <= chunk) row++;
+  // the group's entries [e0, e0 + len)
+  int64_t e0 = 0;
+  int len = 0;
+  if (chunk < n_chunks) {
+    const int64_t at = rowptr[row] + (chunk - chunk_base[row]) * SPMM_N_CHUNK + wave * (SPMM_N_CHUNK / 4);
+    const int64_t left = rowptr[row + 1] - at;
+    len = left <= 0 ? 0 : left < SPMM_N_CHUNK / 4 ? (int)left : (int)(SPMM_N_CHUNK / 4);
+    if (len > 0) e0 = at;
+  }
+  int most = 0, least = SPMM_N_CHUNK;
+#pragma unroll
+  for (int g = 0; g < G; g++) {
+    const int l = __builtin_amdgcn_readlane(len, g * LPR);
+    most = l > most ? l : most;
+    least = l < least ? l : least;
+  }
+  // (past a group's entries: its last one again, or the matrix's first, gathered and not added)
+  auto entry = [&](int e) { return e0 + (e < len ? e : len > 0 ? len - 1 : 0); };
+  const float* Hs = H + slice * WIDTH + 4 * sub;
+  float4 acc = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  int mi = colind[entry(sub)];
+  float mv = vals[entry(sub)];
+  for (int p = 0; p < most; p += LPR) {
+    const int ni = colind[entry(p + LPR + sub)];
+    const float nv = vals[entry(p + LPR + sub)];
+#pragma unroll 1
+    for (int u = 0; u < LPR && p + u < most; u += U) {
+      float4 h[U];
+      float a[U];
+#pragma unroll
+      for (int k = 0; k < U; k++) {
+        const int from = grp * LPR + u + k;
+        const int j = __shfl(mi, from);
+        a[k] = __shfl(mv, from);
+        h[k] = *reinterpret_cast<const float4*>(Hs + (int64_t)j * r);
+      }
+      auto add = [&](int k) {
+        acc.x = fmaf(a[k], h[k].x, acc.x);
+        acc.y = fmaf(a[k], h[k].y, acc.y);
+        acc.z = fmaf(a[k], h[k].z, acc.z);
+        acc.w = fmaf(a[k], h[k].w, acc.w);
+      };
+      if (p + u + U <= least) {
+#pragma unroll
+        for (int k = 0; k < U; k++) add(k);
+      } else {
+#pragma unroll
+        for (int k = 0; k < U; k++)
+          if (p + u + k < len) add(k);
+      }
+    }
+    mi = ni;
+    mv = nv;
+  }
+  *reinterpret_cast<float4*>(red + (grp * 4 + wave) * WIDTH + 4 * sub) = acc;
+  __syncthreads();
+  for (int i = threadIdx.x; i < G * WIDTH; i += 256) {
+    const int k = i / WIDTH, c = i % WIDTH;
+    if (first + k >= n_chunks) break;
+    const float* q = red + 4 * k * WIDTH + c;
+    float s = q[0];
+    s += q[WIDTH];
+    s += q[2 * WIDTH];
+    s += q[3 * WIDTH];
+    partials[(first + k) * r + slice * WIDTH + c] = s;
+  }
+}
+
 // One wave per row, the whole row: the plain row-per-wavefront decomposition, kept for the
 // comparison of work decompositions on ragged rows (a long row then holds its wave for as long
 // as its length says, while the waves of short rows have long finished).
@@ -1508,6 +1601,18 @@ int launch_spmm_n(const dnpeff_csr* A_full, int r, const float* H_mr, int part) 
   if (A->n_chunks == 0) return 0;
   DN_CHECK(A->n_chunks < (int64_t)INT32_MAX, "too many work chunks");
   dim3 grid((unsigned)A->n_chunks), block(256);
+  // (slices of 128 components at rank 256, of 64 above)
+  const int slices = r / (r == 256 ? 128 : 64);
+  if (r >= 256 && r % 128 == 0 && ((uintptr_t)H_mr % 16) == 0 && A->n_chunks * slices < ((int64_t)1 << 24)) {
+    if (r == 256)
+      hipLaunchKernelGGL((k_spmm_n_slices<32>), dim3((unsigned)(ceil_div(A->n_chunks, 2) * slices)), block, 0, stream(),
+                         A->rowptr, A->colind, A->vals, A->chunk_base, A->n_rows, A->n_chunks, slices, r, H_mr, partials);
+    else
+      hipLaunchKernelGGL((k_spmm_n_slices<16>), dim3((unsigned)(ceil_div(A->n_chunks, 4) * slices)), block, 0, stream(),
+                         A->rowptr, A->colind, A->vals, A->chunk_base, A->n_rows, A->n_chunks, slices, r, H_mr, partials);
+    DN_LAUNCH_CHECK();
+    return 0;
+  }
   const size_t lds = sizeof(float) * 4 * (size_t)r;
   dispatch_gather(r, ((uintptr_t)H_mr % 16) == 0, [&](auto tag) {
     using GT = typename decltype(tag)::type;

@@ -100,6 +100,35 @@ def test_spmm_t_tile_at_any_column(r):
     A.close()
 
 
+@pytest.mark.parametrize("r", [256, 384, 512, 640, 1024])
+@pytest.mark.parametrize("n", [1, 2, 7, 40])
+def test_spmm_n_slices(n, r):
+    """Rows without entries, of one entry, of parts of a chunk, of several chunks: the bits of the row chunks."""
+    m = 9000
+    rng = np.random.default_rng(n + r)
+    lens = np.array([4097, 0, 1, 512, 513, 2048, 2049] + list(rng.integers(0, m, size=33)))[:n]
+    ci = np.concatenate([np.sort(rng.choice(m, k, replace=False)) for k in lens]).astype(np.int32)
+    rp = np.concatenate([[0], np.cumsum(lens)]).astype(np.int64)
+    va = rng.random(len(ci)).astype(np.float32)
+    A = d.Csr.from_host(rp, ci, va, m)
+    H = rng.random((m, r)).astype(np.float32)
+    if ci[0] != 0 and not np.any(ci == 0):
+        H[0] = np.nan  # (gathered for groups without entries, and not added)
+    dH = d.DeviceArray.from_numpy(H)
+    outs = []
+    for variant in (0, 2):
+        dN = d.DeviceArray.from_numpy(np.full((n, r), np.nan, dtype=np.float32))
+        d.binding._check(d.lib.dnpeff_op_spmm_n_variant(A._h, r, dH.ptr, dN.ptr, variant))
+        d.sync()
+        outs.append(dN.numpy())
+    want = orc.spmm_n_f64(rp, ci, va, H)
+    # (quarters of 512 entries added up one by one, then the parts: 600 roundings of 2^-24 of the sum at most)
+    assert (np.abs(outs[0] - want) <= 600 * 2.0 ** -24 * np.abs(want)).all()
+    if not np.isnan(H[0]).any():
+        assert np.array_equal(outs[0], outs[1])
+    A.close()
+
+
 @pytest.mark.parametrize("rows", [128, 129, 160, 191, 1023])
 @pytest.mark.parametrize("r", [256, 384, 512, 768])
 def test_gram_on_few_rows(rows, r):
