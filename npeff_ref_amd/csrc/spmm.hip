@@ -100,7 +100,10 @@ struct GatherDword {
 template <int LPR, int T, bool FULL = false>
 struct GatherVec4 {
   static constexpr int G = 64 / LPR;
-  static constexpr int UNR = T >= 4 ? 1 : T == 2 ? 2 : 4;
+  // Steps with their loads in flight: eight loads a lane (half as many / twice: panels of 1000 x 11 M, rank 128, 524
+  // -> 493 us / 505; 2000 x 20 M, rank 256, 1639 -> 1603 / 1617; 700 x 4 M, rank 512, 976 -> 815 / 865).
+  static constexpr int UNR = T >= 4 ? 2 : T == 2 ? 4 : LPR >= 8 ? 8 : 4;
+  static_assert(G * UNR <= 64, "a batch is 64 entries");
   float4 acc[T];
   bool ok[T];
   int lane, sub, grp;
