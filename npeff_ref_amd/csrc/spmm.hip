@@ -836,7 +836,8 @@ constexpr int SPMM_T_COLS = 32;
 // FULL: r = 4 LPR T, every lane holds components (no predicates); SMALL: W has fewer than 2^24
 // rows and 4 GB, a row is addressed as the (uniform) base of W plus a 32-bit offset made by one
 // 24-bit multiply-add.
-template <int LPR, int T, bool FULL, bool SMALL>
+// PAST: the rows of T go past the L2s (launch_spmm_t_sparse).
+template <int LPR, int T, bool FULL, bool SMALL, bool PAST>
 __global__ void __launch_bounds__(256)
     k_spmm_t_grouped(const int64_t* __restrict__ colptr, const int32_t* __restrict__ rowind,
                      const float* __restrict__ tvals, int64_t m, int r, int n_slices,
@@ -966,7 +967,11 @@ __global__ void __launch_bounds__(256)
     if (active) {
 #pragma unroll
       for (int t = 0; t < T; t++)
-        if (FULL || ok[t]) *reinterpret_cast<float4*>(Tout + j * r + 4 * (sub + LPR * t)) = acc[t];
+        if (FULL || ok[t]) {
+          float* dst = Tout + j * r + 4 * (sub + LPR * t);
+          if constexpr (PAST) __builtin_nontemporal_store(f32x4{acc[t].x, acc[t].y, acc[t].z, acc[t].w}, reinterpret_cast<f32x4*>(dst));
+          else *reinterpret_cast<float4*>(dst) = acc[t];
+        }
     }
   }
 }
@@ -1751,9 +1756,17 @@ static int launch_spmm_t_sparse(const dnpeff_csr* A, int r, const float* W_nr, f
   if (grouped) {
     dim3 gg((unsigned)(ceil_div(m, 4 * SPMM_T_COLS) * n_slices));
     const int w4 = width / 4;
-#define DN_GROUPED2(LPR, T_, FULL, SMALL)                                                     \
-  hipLaunchKernelGGL((k_spmm_t_grouped<LPR, T_, FULL, SMALL>), gg, block, 0, stream(), colptr, \
+    // Slices of a large W stay in the L2s, and a T that the memory-side cache does not hold goes past both: an
+    // iteration at 20 000 x 211 M, rank 256, tiles of 768 MiB, 667.5 -> 662.8 ms.
+    const bool past = n_slices > 1 && m * r * (int64_t)sizeof(float) > ((int64_t)256 << 20);
+#define DN_GROUPED3(LPR, T_, FULL, SMALL, PAST)                                                      \
+  hipLaunchKernelGGL((k_spmm_t_grouped<LPR, T_, FULL, SMALL, PAST>), gg, block, 0, stream(), colptr, \
                      A->rowind, A->tvals, m, r, n_slices, W_nr, T)
+#define DN_GROUPED2(LPR, T_, FULL, SMALL)              \
+  do {                                                 \
+    if (past) DN_GROUPED3(LPR, T_, FULL, SMALL, true); \
+    else DN_GROUPED3(LPR, T_, FULL, SMALL, false);     \
+  } while (0)
 #define DN_GROUPED(LPR, T_)                                     \
   do {                                                          \
     const bool full = width == 4 * LPR * T_;                    \
@@ -1770,6 +1783,7 @@ static int launch_spmm_t_sparse(const dnpeff_csr* A, int r, const float* W_nr, f
     else if (w4 <= 64) DN_GROUPED(64, 1);
     else if (w4 <= 128) DN_GROUPED(64, 2);
     else DN_GROUPED(64, 4);
+#undef DN_GROUPED3
 #undef DN_GROUPED2
 #undef DN_GROUPED
   }

@@ -5,6 +5,7 @@ partial sums; against fp64 the bound used is 2e-5 relative to the largest magnit
 output (norm-wise), far inside the 1e-4 the full 50-iteration run has to meet."""
 
 import numpy as np
+import scipy.sparse as sp
 import pytest
 
 import npeff_ref_amd as d
@@ -566,6 +567,28 @@ def test_row_and_column_inspection_and_gathered_rows():
     assert np.array_equal(rp2, rowptr[7:17] - rowptr[7])
     assert np.array_equal(ci2, colind[rowptr[7]:rowptr[16]]) and np.array_equal(va2, vals[rowptr[7]:rowptr[16]])
     assert np.array_equal(nr2, norms[7:16])
+
+
+@pytest.mark.parametrize("m", [524_000, 524_400])
+def test_spmm_t_slices_of_a_large_result(m):
+    """W in slices (6.4 MB), the result on both sides of 256 MiB, from which on it goes past the caches."""
+    n, r = 12_500, 128
+    rng = np.random.default_rng(m)
+    colptr = np.concatenate([[0], np.cumsum(rng.integers(0, 5, size=m))]).astype(np.int64)
+    rows = rng.integers(0, n, size=int(colptr[-1]))
+    rows[colptr[:-1][np.diff(colptr) > 0]] %= 97
+    T = sp.csc_matrix((rng.random(len(rows)).astype(np.float32), rows, colptr), shape=(n, m))
+    T.sum_duplicates()
+    C = T.tocsr()
+    C.sort_indices()
+    A = d.Csr.from_host(C.indptr.astype(np.int64), C.indices.astype(np.int32), C.data, m)
+    W = rng.random((n, r)).astype(np.float32)
+    dW, dT = d.DeviceArray.from_numpy(W), d.DeviceArray((m, r))
+    d.op_spmm_t(A, r, dW, dT)
+    d.sync()
+    want = C.T.astype(np.float64) @ W.astype(np.float64)
+    assert np.abs(dT.numpy() - want).max() <= 4 * 2.0 ** -24 * 5
+    A.close()
 
 
 @pytest.mark.parametrize("r", [64, 100, 512])
