@@ -199,8 +199,10 @@ DN_API int dnpeff_synth_pef(int64_t n_rows, int64_t n_cols, int64_t k_fixed, int
   if (dmalloc(&A->colind, A->nnz) || dmalloc(&A->vals, A->nnz)) return fail(1);
 
   const int64_t kmax_eff = k_min > 0 ? k_max : k_fixed;
+  // A row's last batch of draws meets fewer than k ids and may hold 256 SYNTH_D more: a full table has no end
+  // to a probe (k = 95 of 2.5 M columns: 1045 distinct ids in the first batch, 1024 slots).
   uint64_t cap = 1024;
-  while (cap < 2 * (uint64_t)(kmax_eff + 256)) cap <<= 1;
+  while (cap < 2 * (uint64_t)(kmax_eff + 256 * SYNTH_D)) cap <<= 1;
   // the draws are long chains of fp64 arithmetic: as many workgroups as the tables leave room for
   // (one table each, at most 24 GB together), up to 8 per CU
   int64_t wgs = 8 * (int64_t)n_cus();

@@ -569,6 +569,17 @@ def test_row_and_column_inspection_and_gathered_rows():
     assert np.array_equal(nr2, norms[7:16])
 
 
+def test_synth_rows_shorter_than_a_batch_of_draws():
+    """A batch of 2048 draws holds up to 1045 distinct columns here, eleven times a row's entries: the table of ids
+    has room for all of them."""
+    n, m, k = 41, 2_501_149, 95
+    A, norms = d.Csr.synth(n, m, k_fixed=k, zipf_s=1.1, seed=20230)
+    rowptr, cols, vals = A.download()
+    A.close()
+    want = d.synth_pef_host(n, m, k_fixed=k, zipf_s=1.1, seed=20230)
+    assert np.array_equal(rowptr, want[0]) and np.array_equal(cols, want[1])
+
+
 @pytest.mark.parametrize("m", [524_000, 524_400])
 def test_spmm_t_slices_of_a_large_result(m):
     """W in slices (6.4 MB), the result on both sides of 256 MiB, from which on it goes past the caches."""
