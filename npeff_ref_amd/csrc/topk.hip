@@ -10,8 +10,7 @@
 //      the first at 2 rows of 110 M), give a threshold that a little more than k entries reach (all entries
 //      of a short row: exactly the k-th entry's 22 bits);
 //   2. every entry from the threshold up goes to a candidate list ((key, index) pairs, any order) and is
-//      counted into its bucket, one of equal key width between the threshold and the largest sampled, and the
-//      sum of squares is taken on the way;
+//      counted into its bucket (topk_buckets.hpp), and the sum of squares is taken on the way;
 //   3. the candidates are placed into their buckets by the count that they met (an atomic of their own on a
 //      cursor each took 18 us at 2 x 72,000 candidates, now 5; counting them after the collection 14 more); an
 //      entry's place is its bucket's start plus the number of larger pairs in the bucket.
@@ -25,6 +24,7 @@
 // scheduling.
 #include "dnpeff_internal.hpp"
 #include "scan.hpp"
+#include "topk_buckets.hpp"
 
 #include <algorithm>
 #include <cmath>
@@ -133,17 +133,6 @@ __global__ void __launch_bounds__(64)
   for (int i = threadIdx.x; i < TOPK_BINS; i += 64) h[i] = 0;
 }
 
-// Bucket of a key from the threshold up: 0 holds the largest, which may lie above kmax (the largest of a sample).
-// All other buckets span 2^shift keys.
-__device__ inline int topk_shift(uint32_t thr, uint32_t kmax, int log_nb) {
-  const uint32_t range = kmax - thr;
-  const int bits = range ? 32 - __clz(range) : 0;
-  return bits > log_nb ? bits - log_nb : 0;
-}
-__device__ inline int topk_bucket(uint32_t key, uint32_t thr, uint32_t kmax, int shift) {
-  return (int)(((kmax - thr) >> shift) - (((key < kmax ? key : kmax) - thr) >> shift));
-}
-
 // A wave's finds on their way to a row's candidate list.  They wait in LDS and room in the list is reserved
 // once per 256+ of them: the finds are sparse (k of ~1e8), and one global atomic each on a single counter
 // would serialise them.  Every wave keeps its own buffer and count, so the loop that reads the row has no
@@ -156,8 +145,8 @@ struct topk_finds {
   unsigned long long* cursor;
   int* buckets;  // (or NULL) entries per bucket, counted as they are written: `place` receives the count before
   unsigned* place;
-  uint32_t thr, kmax;
-  int shift;
+  uint32_t thr, top;
+  int shift, above;
 
   // All lanes call these together.
   __device__ void put(bool take, uint32_t key, int64_t i) {
@@ -171,7 +160,7 @@ struct topk_finds {
     for (unsigned i = threadIdx.x & 63; i < n; i += 64)
       if (base + i < (unsigned long long)cap) {
         out[base + i] = buf[i];
-        if (buckets) place[base + i] = (unsigned)atomicAdd(&buckets[topk_bucket((uint32_t)(buf[i] >> 32), thr, kmax, shift)], 1);
+        if (buckets) place[base + i] = (unsigned)atomicAdd(&buckets[topk_bucket((uint32_t)(buf[i] >> 32), thr, top, shift, above)], 1);
       }
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     n = 0;
@@ -243,7 +232,7 @@ __global__ void __launch_bounds__(256)
   const uint32_t prefix = st[row].prefix, mask = st[row].mask;
   const int64_t n_cand = k - st[row].need + st[row].in_bin;
   uint64_t* out = cand + (int64_t)row * kp;
-  topk_finds f{buf[threadIdx.x >> 6], 0u, out, kp, reinterpret_cast<unsigned long long*>(&st[row].cursor), nullptr, nullptr, 0u, 0u, 0};
+  topk_finds f{buf[threadIdx.x >> 6], 0u, out, kp, reinterpret_cast<unsigned long long*>(&st[row].cursor), nullptr, nullptr, 0u, 0u, 0, 0};
   topk_sweep<VEC4>(x + (int64_t)row * count, count, [&](const float* v, int64_t first, bool) {
 #pragma unroll
     for (int e = 0; e < 4; e++) {
@@ -362,34 +351,30 @@ __global__ void __launch_bounds__(256)
 // ---------------------------------------------------------------------------
 // The usual case
 // ---------------------------------------------------------------------------
-constexpr int TOPK_CHUNK = 64;            // sampled entries in a row
-constexpr int TOPK_STRIDE = 2048;         // one chunk of every so many entries, or of twice as many
-constexpr int64_t TOPK_SAMPLED = 1 << 19; // rows from this length on are sampled
-constexpr int TOPK_MAX_BUCKETS = 16384;
-constexpr int TOPK_CROWDED = 2048;        // entries of a bucket that are still ranked one against the other
-
 struct TopkRow {
-  uint32_t bin, thr, kmax;
+  uint32_t bin, thr, top;      // top: the largest key of the sample
   unsigned need;               // of the sample, still to find
   unsigned long long cursor;   // candidates
 };
 
 __global__ void __launch_bounds__(1024)
-    k_topk_row_init(TopkRow* rows, unsigned target, unsigned* __restrict__ hist, int log_nb, int* __restrict__ buckets) {
-  if (threadIdx.x == 0) rows[blockIdx.x] = TopkRow{0u, 0u, 0xffffffffu, target, 0ull};
+    k_topk_row_init(TopkRow* rows, unsigned target, unsigned* __restrict__ hist, int nb, int* __restrict__ buckets) {
+  if (threadIdx.x == 0) rows[blockIdx.x] = TopkRow{0u, 0u, 0u, target, 0ull};
   for (int i = threadIdx.x; i < TOPK_BINS; i += 1024) hist[(int64_t)blockIdx.x * TOPK_BINS + i] = 0;
-  for (int i = threadIdx.x; i < 1 << log_nb; i += 1024) buckets[((int64_t)blockIdx.x << log_nb) + i] = 0;
+  for (int i = threadIdx.x; i < nb; i += 1024) buckets[(int64_t)blockIdx.x * nb + i] = 0;
 }
 
-// LEVEL 0: top 11 bits of the key; 1: the next 11 of the entries in the bin that level 0 found.
+// LEVEL 0: top 11 bits of the key, and the largest key; 1: the next 11 of the entries in the bin that level 0 found.
 template <int LEVEL>
 __global__ void __launch_bounds__(256)
     k_topk_sample(const float* __restrict__ x, int64_t count, int64_t stride, int64_t chunks,
-                  const TopkRow* __restrict__ rows, unsigned* __restrict__ hist) {
+                  TopkRow* __restrict__ rows, unsigned* __restrict__ hist) {
   __shared__ unsigned h[TOPK_BINS];
+  __shared__ uint32_t most[4];
   const int row = blockIdx.y, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   for (int i = threadIdx.x; i < TOPK_BINS; i += 256) h[i] = 0;
   const uint32_t bin = LEVEL ? rows[row].bin : 0u;
+  uint32_t top = 0;
   __syncthreads();
   const float* xr = x + (int64_t)row * count;
   const int64_t step = (int64_t)gridDim.x * 4;
@@ -406,12 +391,19 @@ __global__ void __launch_bounds__(256)
     for (int u = 0; u < 4; u++) {
       const uint32_t key = sort_key(v[u]);
       if (LEVEL) ok[u] = ok[u] && (key >> 21) == bin;
+      else top = ok[u] ? max(top, key) : top;
       if (ok[u]) atomicAdd(&h[LEVEL ? (key >> 10) & (TOPK_BINS - 1) : key >> 21], 1u);
     }
+  }
+  if (!LEVEL) {
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) top = max(top, (uint32_t)__shfl_xor((int)top, off));
+    if (lane == 0) most[wave] = top;
   }
   __syncthreads();
   for (int i = threadIdx.x; i < TOPK_BINS; i += 256)
     if (h[i]) atomicAdd(&hist[(int64_t)row * TOPK_BINS + i], h[i]);
+  if (!LEVEL && threadIdx.x == 0) atomicMax(&rows[row].top, max(max(most[0], most[1]), max(most[2], most[3])));
 }
 
 // The bin from the top where the sample's entries reach the target.
@@ -434,11 +426,6 @@ __global__ void __launch_bounds__(256) k_topk_threshold(unsigned* __restrict__ h
   const unsigned need = rows[blockIdx.x].need, total = part[255];
   unsigned above = part[t] - sum;
   __syncthreads();
-  if (LEVEL == 0 && above == 0 && sum > 0) {  // the end of the sample's largest bin
-    int b = 0;
-    while (c[b] == 0) b++;
-    rows[blockIdx.x].kmax = ((uint32_t)(top - b) << 21) | 0x1fffffu;
-  }
   if (above < need && above + sum >= need) {
     int b = 0;
     while (above + c[b] < need) above += c[b++];
@@ -464,16 +451,16 @@ __global__ void __launch_bounds__(256) k_topk_threshold(unsigned* __restrict__ h
 template <bool VEC4>
 __global__ void __launch_bounds__(256)
     k_topk_collect(const float* __restrict__ x, int64_t count, TopkRow* __restrict__ rows, uint64_t* __restrict__ cand,
-                   int64_t cap, int log_nb, int* __restrict__ buckets, unsigned* __restrict__ place,
+                   int64_t cap, int log_nb, int above, int* __restrict__ buckets, unsigned* __restrict__ place,
                    double* __restrict__ sq_partials) {
   __shared__ uint64_t buf[4][512];
   __shared__ unsigned counts[4];
   __shared__ unsigned long long list_base;
   __shared__ double red[256];
   const int row = blockIdx.y;
-  const uint32_t thr = rows[row].thr, kmax = rows[row].kmax;
+  const uint32_t thr = rows[row].thr, top = rows[row].top;
   topk_finds f{buf[threadIdx.x >> 6], 0u, cand + (int64_t)row * cap, cap, &rows[row].cursor,
-               buckets + ((int64_t)row << log_nb), place + (int64_t)row * cap, thr, kmax, topk_shift(thr, kmax, log_nb)};
+               buckets + (int64_t)row * ((1 << log_nb) + above), place + (int64_t)row * cap, thr, top, topk_shift(thr, top, log_nb), above};
   double sq = 0.0;
   // (from the key of +0 up, keys are in the order of the bits as signed integers)
   const bool plain = thr >= 0x80000000u;
@@ -513,23 +500,24 @@ __global__ void __launch_bounds__(256)
 }
 
 // Counts to starts (in place), the row's norm, and whether the list serves.
-// (A row has one workgroup here, so a thread has at most 16 counts and loads them four at a time, and sums go
+// (A row has one workgroup here, so a thread has at most 20 counts and loads them four at a time, and sums go
 // by shuffles: 16,384 counts, 2 rows, 6.3 us; 9.5 with ten barriers, 43 with 64 counts one at a time.)
 constexpr int TOPK_SCAN = 1024;
 __global__ void __launch_bounds__(TOPK_SCAN)
-    k_topk_bucket_scan(const TopkRow* __restrict__ rows, int64_t cap, int64_t k, int log_nb, int* __restrict__ buckets,
+    k_topk_bucket_scan(const TopkRow* __restrict__ rows, int64_t cap, int64_t k, int nb, int* __restrict__ buckets,
                        const double* __restrict__ sq_partials, int n_sq,
                        float* __restrict__ norms, unsigned long long* __restrict__ failed) {
   __shared__ int part[TOPK_SCAN / 64];
   __shared__ double red[TOPK_SCAN / 64];
-  const int row = blockIdx.x, t = threadIdx.x, quads = ((1 << log_nb) / 4 + TOPK_SCAN - 1) / TOPK_SCAN;
-  int4* b = reinterpret_cast<int4*>(buckets + ((int64_t)row << log_nb));
-  const bool in = t * quads * 4 < 1 << log_nb;
-  int4 v[TOPK_MAX_BUCKETS / 4 / TOPK_SCAN];
+  const int row = blockIdx.x, t = threadIdx.x, quads = (nb / 4 + TOPK_SCAN - 1) / TOPK_SCAN;
+  int4* b = reinterpret_cast<int4*>(buckets + (int64_t)row * nb);
+  constexpr int MOST = TOPK_MAX_BUCKETS / 4 / TOPK_SCAN;
+  const int mine = min(quads, max(0, nb / 4 - t * quads));
+  int4 v[MOST];
   int sum = 0, most = 0;
 #pragma unroll
-  for (int i = 0; i < TOPK_MAX_BUCKETS / 4 / TOPK_SCAN; i++) {
-    v[i] = in && i < quads ? b[t * quads + i] : int4{0, 0, 0, 0};
+  for (int i = 0; i < MOST; i++) {
+    v[i] = i < mine ? b[t * quads + i] : int4{0, 0, 0, 0};
     sum += v[i].x + v[i].y + v[i].z + v[i].w;
     most = max(max(max(v[i].x, v[i].y), max(v[i].z, v[i].w)), most);
   }
@@ -550,8 +538,8 @@ __global__ void __launch_bounds__(TOPK_SCAN)
   int run = incl - sum;
   for (int w = 0; w < wave; w++) run += part[w];
 #pragma unroll
-  for (int i = 0; i < TOPK_MAX_BUCKETS / 4 / TOPK_SCAN; i++) {
-    if (!in || i >= quads) break;
+  for (int i = 0; i < MOST; i++) {
+    if (i >= mine) break;
     const int4 w{run, run + v[i].x, run + v[i].x + v[i].y, run + v[i].x + v[i].y + v[i].z};
     b[t * quads + i] = w;
     run = w.w + v[i].w;
@@ -566,31 +554,32 @@ __global__ void __launch_bounds__(TOPK_SCAN)
 
 __global__ void __launch_bounds__(256)
     k_topk_scatter(const TopkRow* __restrict__ rows, const uint64_t* __restrict__ cand, const unsigned* __restrict__ place,
-                   int64_t cap, int log_nb, const int* __restrict__ starts, uint64_t* __restrict__ out) {
+                   int64_t cap, int log_nb, int above, const int* __restrict__ starts, uint64_t* __restrict__ out) {
   const TopkRow r = rows[blockIdx.y];
   const int64_t n = (int64_t)r.cursor < cap ? (int64_t)r.cursor : cap;
-  const int shift = topk_shift(r.thr, r.kmax, log_nb);
-  const int* s = starts + ((int64_t)blockIdx.y << log_nb);
+  const int shift = topk_shift(r.thr, r.top, log_nb);
+  const int* s = starts + (int64_t)blockIdx.y * ((1 << log_nb) + above);
   for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
     const uint64_t p = cand[(int64_t)blockIdx.y * cap + i];
-    out[(int64_t)blockIdx.y * cap + s[topk_bucket((uint32_t)(p >> 32), r.thr, r.kmax, shift)] + place[(int64_t)blockIdx.y * cap + i]] = p;
+    out[(int64_t)blockIdx.y * cap + s[topk_bucket((uint32_t)(p >> 32), r.thr, r.top, shift, above)] + place[(int64_t)blockIdx.y * cap + i]] = p;
   }
 }
 
 // The k first places: a pair's is its bucket's start plus the larger pairs of the bucket.
 __global__ void __launch_bounds__(256)
     k_topk_rank(const TopkRow* __restrict__ rows, const uint64_t* __restrict__ sorted, int64_t cap, int64_t k, int log_nb,
-                const int* __restrict__ starts, float* __restrict__ vals,
+                int above, const int* __restrict__ starts, float* __restrict__ vals,
                 int32_t* __restrict__ idx) {
   const TopkRow r = rows[blockIdx.y];
   const int64_t n = (int64_t)r.cursor < cap ? (int64_t)r.cursor : cap;
-  const int shift = topk_shift(r.thr, r.kmax, log_nb);
+  const int shift = topk_shift(r.thr, r.top, log_nb);
   const uint64_t* p = sorted + (int64_t)blockIdx.y * cap;
+  const int nb = (1 << log_nb) + above;
+  const int* row_starts = starts + (int64_t)blockIdx.y * nb;
   for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
     const uint64_t own = p[i];
-    const int b = topk_bucket((uint32_t)(own >> 32), r.thr, r.kmax, shift);
-    const int s = starts[((int64_t)blockIdx.y << log_nb) + b];
-    const int e = b + 1 < 1 << log_nb ? starts[((int64_t)blockIdx.y << log_nb) + b + 1] : (int)n;
+    const int b = topk_bucket((uint32_t)(own >> 32), r.thr, r.top, shift, above);
+    const int s = row_starts[b], e = b + 1 < nb ? row_starts[b + 1] : (int)n;
     if (s >= k || e - s > TOPK_CROWDED) continue;
     int rank = s;
     for (int j = s; j < e; j++) rank += p[j] > own;
@@ -631,17 +620,10 @@ static int bitonic_sort_rows(uint64_t* cand, int64_t kp, int64_t n_rows) {
 static int topk_by_sample(int64_t n_rows, int64_t count, int64_t k, const float* x, float* vals, int32_t* idx,
                           float* norms, bool* done) {
   *done = false;
-  const bool sampled = count >= TOPK_SAMPLED;
-  const int64_t stride = !sampled ? TOPK_CHUNK : k >= 8 * TOPK_STRIDE * 2 ? 2 * TOPK_STRIDE : TOPK_STRIDE, chunks = ceil_div(count, stride);
-  // entries of the sample to find above the threshold: their share of k and five times its deviation
-  const double share = (double)k * TOPK_CHUNK / (double)stride;
-  const unsigned target = sampled ? (unsigned)(share + 5.0 * sqrt(share) + 8.0) : (unsigned)k;
-  const double expected = sampled ? (double)target * stride / TOPK_CHUNK : (double)k;
-  int64_t cap = (int64_t)(1.5 * expected) + 4096;
-  if (cap > count) cap = count;
+  const topk_plan plan = topk_plan_of(count, k);
+  const int64_t stride = plan.stride, chunks = ceil_div(count, stride), cap = plan.cap;
+  const int log_nb = plan.log_nb, above = plan.above;
   if ((double)n_rows * (double)cap * 16.0 > 4.0e9) return 0;
-  int log_nb = 8;
-  while (log_nb < 14 && ((int64_t)4 << log_nb) < cap) log_nb++;
   hipStream_t st = stream();
   const dim3 block(256);
   // (one launch fills the chip several times over, however many rows there are)
@@ -661,26 +643,26 @@ static int topk_by_sample(int64_t n_rows, int64_t count, int64_t k, const float*
   DN_TRY(hist.alloc(n_rows * TOPK_BINS));
   DN_TRY(cand.alloc(n_rows * cap));
   DN_TRY(sorted.alloc(n_rows * cap));
-  DN_TRY(starts.alloc(n_rows << log_nb));
+  DN_TRY(starts.alloc(n_rows * plan.buckets()));
   DN_TRY(place.alloc(n_rows * cap));
   DN_TRY(sq.alloc(n_rows * gc.x));
   unsigned long long* failed = nullptr;
   DN_TRY(host_words(&failed));
   *failed = 0;
-  hipLaunchKernelGGL(k_topk_row_init, dim3((unsigned)n_rows), dim3(1024), 0, st, rows.p, target, hist.p, log_nb, starts.p);
+  hipLaunchKernelGGL(k_topk_row_init, dim3((unsigned)n_rows), dim3(1024), 0, st, rows.p, plan.target, hist.p, plan.buckets(), starts.p);
   const dim3 gs = blocks(chunks, 64), gr((unsigned)n_rows), gp = blocks(cap, 256);
   hipLaunchKernelGGL(k_topk_sample<0>, gs, block, 0, st, x, count, stride, chunks, rows.p, hist.p);
   hipLaunchKernelGGL(k_topk_threshold<0>, gr, block, 0, st, hist.p, rows.p);
   hipLaunchKernelGGL(k_topk_sample<1>, gs, block, 0, st, x, count, stride, chunks, rows.p, hist.p);
   hipLaunchKernelGGL(k_topk_threshold<1>, gr, block, 0, st, hist.p, rows.p);
   if (count % 4 == 0 && ((uintptr_t)x % 16) == 0)
-    hipLaunchKernelGGL(k_topk_collect<true>, gc, block, 0, st, x, count, rows.p, cand.p, cap, log_nb, starts.p, place.p, sq.p);
+    hipLaunchKernelGGL(k_topk_collect<true>, gc, block, 0, st, x, count, rows.p, cand.p, cap, log_nb, above, starts.p, place.p, sq.p);
   else
-    hipLaunchKernelGGL(k_topk_collect<false>, gc, block, 0, st, x, count, rows.p, cand.p, cap, log_nb, starts.p, place.p, sq.p);
-  hipLaunchKernelGGL(k_topk_bucket_scan, gr, dim3(TOPK_SCAN), 0, st, rows.p, cap, k, log_nb, starts.p, sq.p, (int)gc.x,
+    hipLaunchKernelGGL(k_topk_collect<false>, gc, block, 0, st, x, count, rows.p, cand.p, cap, log_nb, above, starts.p, place.p, sq.p);
+  hipLaunchKernelGGL(k_topk_bucket_scan, gr, dim3(TOPK_SCAN), 0, st, rows.p, cap, k, plan.buckets(), starts.p, sq.p, (int)gc.x,
                      norms, failed);
-  hipLaunchKernelGGL(k_topk_scatter, gp, block, 0, st, rows.p, cand.p, place.p, cap, log_nb, starts.p, sorted.p);
-  hipLaunchKernelGGL(k_topk_rank, gp, block, 0, st, rows.p, sorted.p, cap, k, log_nb, starts.p, vals, idx);
+  hipLaunchKernelGGL(k_topk_scatter, gp, block, 0, st, rows.p, cand.p, place.p, cap, log_nb, above, starts.p, sorted.p);
+  hipLaunchKernelGGL(k_topk_rank, gp, block, 0, st, rows.p, sorted.p, cap, k, log_nb, above, starts.p, vals, idx);
   DN_LAUNCH_CHECK();
   DN_HIP(hipStreamSynchronize(st));
   *done = *failed == 0;

@@ -53,3 +53,20 @@ def test_entries_above_all_of_the_sample(count, k, outliers):
     order = np.lexsort((np.arange(count), -x))[:k]
     assert np.array_equal(idx[0], order) and np.array_equal(vals[0], x[order])
     np.testing.assert_allclose(norms[0], np.sqrt((x.astype(np.float64) ** 2).sum()), rtol=1e-7)
+
+
+@pytest.mark.parametrize("count,k,kind", [(2_000_000, 40_000, "close"), (2_000_001, 700, "close"), (1_500_000, 33_000, "edge"),
+                                          (1_500_000, 33_000, "gap"), (700_001, 900, "gap")])
+def test_threshold_and_largest_entry_close_together(count, k, kind):
+    """Candidates within one bin of the sample's histogram, on either side of a bin's end, or (gap) a run of larger
+    entries between two chunks of the sample, twice its length with the larger stride."""
+    rng = np.random.default_rng(count + k)
+    x = (1.0 if kind == "close" else 0.9965) + 1e-3 * rng.standard_normal(count)
+    if kind == "gap":
+        stride = 4096 if k >= 32_768 else 2048
+        x[3 * stride + 64:4 * stride] += 0.01 + 1e-3 * rng.random(stride - 64)
+    x = x.astype(np.float32)
+    vals, idx, norms = d.topk_rows(d.DeviceArray.from_numpy(x[None, :]), k)
+    order = np.lexsort((np.arange(count), -x))[:k]
+    assert np.array_equal(idx[0], order) and np.array_equal(vals[0], x[order])
+    np.testing.assert_allclose(norms[0], np.sqrt((x.astype(np.float64) ** 2).sum()), rtol=1e-7)
