@@ -256,17 +256,24 @@ static int stored_rank(int64_t n, int64_t m, int64_t nnz, int rank, bool sweeps,
   return t.total() + 24.0 * (double)nnz <= there ? p : rank;
 }
 
-// Whether the step of small ranks runs where memory allows.  (It reads the whole matrix from its own lists: no
-// dense head is split off then.  Rank 128 with rows enough for a dense head keeps it: the fused step's kernel at
-// that rank has one wave per SIMD.  Ten iterations with head / fused: r = 128 14.7 / 16.0 ms at 1500 x 1.4M, 24.2 / 31.2 at
-// 2000 x 1.9M, 79 / 84 at 2000 x 9.8M, but 8.5 / 7.2 at 1024 x 0.8M; at r = 64 the fused step is ahead at all sizes,
-// 3.2 / 0.86 ms at 1024 x 67k, 16.1 / 6.1 at 1500 x 0.9M, 22.6 / 8.9 at 4000 x 1.5M, 60 / 42 at 2000 x 6.4M, 47 / 37 at
-// 8000 x 3.6M, and closer to 64 bits: one W update 5e-7 ... 8e-7 off where the head's split operands leave 1e-6 ... 6e-6.
-// Below 65,536 columns rank 64 stays with the head all the same, 3.7 / 1.5 ms at 1100 x 60k: that is where the head's
-// own runs are held to their bits.)
+// Whether the step of small ranks runs where memory allows.  It reads the whole matrix from its own lists: no
+// dense head is split off then.
+// Rank 128 with rows enough for a dense head keeps it: the fused step's kernel at that rank has one wave per SIMD.
+// Ten iterations with head / fused: 14.7 / 16.0 ms at 1500 x 1.4M, 24.2 / 31.2 at 2000 x 1.9M, 79 / 84 at 2000 x
+// 9.8M, but 8.5 / 7.2 at 1024 x 0.8M.
+// Rank 64 keeps it where the matrix is dense: a gathered entry takes as long as eight cells of the head, and the head's
+// launches as long as 6 M entries (1.7 ms in ten iterations).  Ten iterations with head / fused, by the share of the
+// cells that hold an entry: 23.3 / 40.7 ms at 2000 x 200k, 120 M entries (0.30), 3.17 / 4.49 at 1500 x 20k, 15 M (0.50),
+// 3.17 / 3.50 with 12 M (0.40) but 3.17 / 2.51 with 8.3 M (0.28), 34.1 / 43.2 at 4000 x 200k (0.16), 18.7 / 20.6 at 8000 x
+// 60k (0.14), 10.4 / 10.7 at 4000 x 60k (0.14) but 5.6 / 3.4 at 3000 x 20k, 12 M (0.20), 23.0 / 21.7 at 4000 x 200k
+// (0.08), 57 / 53 at 20000 x 200k (0.04).  Below, the fused step is ahead by 1.1 to 5 from 1024 x 1100 to 100000 x
+// 4.0M (1.73 / 0.32, 3.4 / 1.3 at 1100 x 60k, 52 / 36 at 8000 x 5.7M, 145 / 107), except where few columns hold most of
+// very many entries: 113 / 128 at 40000 x 3.9M, 328 M entries by a Zipf law of 1.3, 48 / 54 at 2000 x 1M, 131 M.  It is
+// also closer to 64 bits: one W update 5e-7 ... 8e-7 off where the head's split operands leave 1e-6 ... 6e-6.
 static bool fused_step_wanted(int64_t n, int64_t m, int64_t nnz, int rank) {
-  return tuning().fused_gram != 0.0 && tuning().tiled_h <= 0.0 && !(rank % 64 == 0 && n >= 1024 && !(rank == 64 && m >= 65536)) &&
-         fused_supported(n, m, nnz, rank);
+  if (tuning().fused_gram == 0.0 || tuning().tiled_h > 0.0 || !fused_supported(n, m, nnz, rank)) return false;
+  if (n < 1024 || rank % 64 != 0) return true;
+  return rank == 64 && 9.0 * ((double)nnz - 6e6) <= (double)n * (double)m;
 }
 
 // For tests and capacity planning without a GPU: the table above and, for a head of n_dense columns,

@@ -292,17 +292,25 @@ def test_ranks_on_either_side_of_the_grouping():
         A.close()
 
 
-@pytest.mark.parametrize("m,fused", [(65_535, False), (65_536, True)])
-def test_rank_64_with_many_rows(m, fused):
-    """1024 rows and more at rank 64: the fused step from 65,536 columns on, a dense head below."""
-    A, norms = d.Csr.synth(1030, m, k_fixed=700, zipf_s=1.1, seed=8)
-    A.normalize_rows(norms)
+@pytest.mark.parametrize("m,k,fused", [(2000, 120, True), (65_535, 700, True), (65_536, 700, True), (9000, 6800, True),
+                                       (9000, 6850, False)])
+def test_rank_64_with_many_rows(m, k, fused):
+    """1024 rows and more at rank 64: a dense head where nine times the entries past 6 M are more than the cells (1030 x
+    9000: 6826 entries per row), else the fused step."""
+    n = 1030
+    if 2 * k <= m:
+        A, norms = d.Csr.synth(n, m, k_fixed=k, zipf_s=1.1, seed=8)
+        A.normalize_rows(norms)
+    else:
+        rng = np.random.default_rng(m + k)
+        cols = np.argsort(rng.random((n, m), dtype=np.float32), axis=1)[:, :k].astype(np.int32)
+        A = d.Csr.from_host(np.arange(n + 1, dtype=np.int64) * k, cols.ravel(), rng.random(n * k, dtype=np.float32), m)
     rp, ci, va = A.download()
-    nmf = d.MuNmf(A, d.MuNmfParams(rank=64, max_iters=4, eps=EPS, seed=5, log_every=2))
+    nmf = d.MuNmf(A, d.MuNmfParams(rank=64, max_iters=2, eps=EPS, seed=5, log_every=2))
     nmf.initialize()
     assert (A.head_info()[0] == 0) == fused
     W0, H0 = nmf.loadWToHostSync(), nmf.loadHToHostSync()
     nmf.run(log=lambda s: None)
-    _close(nmf, orc.nmf_f64(rp, ci, va, m, W0, H0, np.float32(EPS), 4, 2))
+    _close(nmf, orc.nmf_f64(rp, ci, va, m, W0, H0, np.float32(EPS), 2, 2))
     nmf.close()
     A.close()

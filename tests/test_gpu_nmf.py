@@ -264,6 +264,7 @@ def test_dense_head_run_matches_oracle_and_unsplit_run(tune):
     """n >= 1024 rows and r >= 64: dnpeff_nmf_create moves the columns most rows hold into the
     dense block by itself; the run stays within the bar of the fp64 oracle and close to the run
     with the split switched off."""
+    tune("fused_gram", 0)  # (the separate kernels: the fused step is the faster one here)
     n, m_full, k, r, eps, iters, seed = 1100, 60000, 3000, 64, 1e-8, 50, 77
     nmf, A, (W0, H0), (W, H), (W64, H64), hist, losses64 = _run_case(n, m_full, k, r, eps, iters, seed)
     nd, z_sparse = A.head_info()
@@ -349,9 +350,10 @@ def test_heavier_skew_rank_256_with_dense_head():
     A.close()
 
 
-def test_fit_after_nmf_on_the_same_matrix():
+def test_fit_after_nmf_on_the_same_matrix(tune):
     """A matrix that an NMF has split (dense head, tail) is handed to the fit path afterwards:
     the sparse-sparse product undoes the split and gives the same A H^T as on a fresh matrix."""
+    tune("fused_gram", 0)
     n, m_full, k, r = 1100, 60000, 3000, 64
     A, norms = d.Csr.synth(n, m_full, k_fixed=k, zipf_s=1.1, seed=77)
     A.normalize_rows(norms)
