@@ -121,7 +121,7 @@ struct dnpeff_nmf {
   // The step of small ranks (fused.hip).  While the switch is off, another context's dense head is on
   // the matrix or the launches of each class are being timed, the separate kernels run instead.
   bool has_fused = false;
-  fused_state fu;
+  fused_state fu;            // (fu.xcd: the memory plan had room for the lists by XCD)
   bool fu_n_valid = false;   // fu.n_part (or Nw, with panels) holds A H^T of the current H
   // The factor's device pointer was handed out since its last update: the caller may write through it
   // between any two calls, so no product kept from an earlier call stands for the factor.
@@ -276,6 +276,23 @@ static bool fused_step_wanted(int64_t n, int64_t m, int64_t nnz, int rank) {
   return rank == 64 && 9.0 * ((double)nnz - 6e6) <= (double)n * (double)m;
 }
 
+// Whether it does within `budget` bytes beside the factors, and whether with lists by XCD.
+struct fused_choice {
+  bool on = false, xcd = false;
+  double lists = 0.0, state = 0.0;  // bytes
+};
+static fused_choice choose_fused(int64_t n, int64_t m, int64_t nnz, int rank, double budget) {
+  fused_choice c;
+  if (!fused_step_wanted(n, m, nnz, rank)) return c;
+  c.lists = fused_list_bytes(n, m, nnz);
+  c.state = fused_state_bytes(n, m, nnz, rank);
+  const double need = 16.0 * (double)nnz + c.lists + c.state, more = fused_xcd_bytes(n, nnz, rank);
+  c.on = need < budget;
+  c.xcd = more > 0.0 && need + more < budget;
+  if (c.xcd) c.lists += more;
+  return c;
+}
+
 // For tests and capacity planning without a GPU: the table above and, for a head of n_dense columns,
 // its blocks and workspace.  out[0..7] = factors, partials, segments, offsets, reserve, sparse
 // copies, head blocks, head workspace (bytes).
@@ -291,9 +308,10 @@ DN_API int dnpeff_plan_estimate(int64_t n_rows, int64_t n_cols, int64_t nnz_spar
   if (!tiled) rank = stored_rank(n_rows, n_cols, nnz_sparse, asked, sweeps != 0, total, total);
   plan_table t = plan_overheads(n_rows, n_cols, nnz_sparse, rank, asked, tiled != 0, sweeps != 0, total);
   out[5] = 16.0 * (double)nnz_sparse;
-  if (!tiled && n_dense == 0 && fused_step_wanted(n_rows, n_cols, nnz_sparse, rank)) {
-    out[5] += fused_list_bytes(n_rows, n_cols, nnz_sparse);
-    t.factors += fused_state_bytes(n_rows, n_cols, nnz_sparse, rank);
+  const fused_choice fused = choose_fused(n_rows, n_cols, nnz_sparse, rank, total - t.total());
+  if (!tiled && n_dense == 0 && fused.on) {
+    out[5] += fused.lists;
+    t.factors += fused.state;
   }
   out[0] = t.factors; out[1] = t.partials; out[2] = t.segments; out[3] = t.offsets; out[4] = t.reserve;
   out[6] = n_dense ? 4.0 * head_blocks_for_rank(rank) * (double)(ceil_div(n_rows, 128) * 128) *
@@ -310,7 +328,7 @@ DN_API int dnpeff_plan_estimate(int64_t n_rows, int64_t n_cols, int64_t nnz_spar
 // blocks and both sparse copies of the rest fit the memory left beside the factors.  *tiled
 // receives whether the H update must run on column tiles for everything to fit.
 // *fused: whether the step of small ranks runs.
-static int plan_matrix(dnpeff_csr* A, int rank, int asked, bool consume, bool* tiled, bool* fused) {
+static int plan_matrix(dnpeff_csr* A, int rank, int asked, bool consume, bool* tiled, fused_choice* fused) {
   const tuning_t& tn = tuning();
   size_t free_b = 0, total_b = 0;
   DN_HIP(hipMemGetInfo(&free_b, &total_b));
@@ -330,10 +348,8 @@ static int plan_matrix(dnpeff_csr* A, int rank, int asked, bool consume, bool* t
   const plan_table t_tiled = plan_overheads(A->n_rows, A->n_cols, A->nnz, rank, asked, true, sweeps, (double)total_b);
   const double budget_full = avail - t_full.total();
   const double budget_tiled = avail - t_tiled.total();
-  *fused = fused_step_wanted(A->n_rows, A->n_cols, A->nnz, rank) &&
-           16.0 * (double)A->nnz + fused_list_bytes(A->n_rows, A->n_cols, A->nnz) +
-                   fused_state_bytes(A->n_rows, A->n_cols, A->nnz, rank) < budget_full;
-  const bool can_split = rank % 4 == 0 && rank >= 64 && A->n_rows >= 1024 && !*fused;
+  *fused = choose_fused(A->n_rows, A->n_cols, A->nnz, rank, budget_full);
+  const bool can_split = rank % 4 == 0 && rank >= 64 && A->n_rows >= 1024 && !fused->on;
   double fill = tn.dense_fill;
   if (fill > 1.0) fill = 0.0;
   *tiled = tn.tiled_h > 0.0;
@@ -411,7 +427,8 @@ static int nmf_create_impl(dnpeff_csr* A, int rank, float eps, int64_t seed, uns
   mark("||A||^2");
   const int rank_asked = rank;
   DN_TRY(padded_rank(A, rank_asked, eps, &rank));
-  bool tiled = false, fused = false;
+  bool tiled = false;
+  fused_choice fused;
   DN_TRY(plan_matrix(A, rank, rank_asked, consume, &tiled, &fused));
   if (tiled && rank != rank_asked) {  // (only where the two estimates of the memory disagree)
     rank = rank_asked;
@@ -451,9 +468,9 @@ static int nmf_create_impl(dnpeff_csr* A, int rank, float eps, int64_t seed, uns
     s = dmalloc(&h->GH, (int64_t)rank * rank) || dmalloc(&h->gpart, xg_mu_gram_workspace_floats(h->m));
   if (!s && h->tiled && tuning().h_overlap != 0.0) s = dmalloc(&h->S2, s_floats);
   if (!s && h->tiled) s = csr_tile_lists(A);
-  if (!s && fused && !h->tiled && !A->tail) {
+  if (!s && fused.on && !h->tiled && !A->tail) {
     h->has_fused = true;
-    s = fused_plan_build(A, rank) || h->fu.create(A, h->n, rank);
+    s = fused_plan_build(A, rank, fused.xcd) || h->fu.create(A, h->n, rank, fused.xcd);
   }
   if (s) { dnpeff_nmf_destroy(h); return s; }
   mark("factors and workspaces");
@@ -550,7 +567,8 @@ static int products_for(dnpeff_nmf* h) {
 // A H^T by chunks (or, where the factor is large enough for column panels, as Nw), and H^T H.
 static int fused_products(dnpeff_nmf* h) {
   DN_TRY(products_for(h));
-  DN_TRY(fused_plan_build(h->A, h->r));
+  DN_TRY(fused_plan_build(h->A, h->r, h->fu.xcd));
+  if (h->A->n_panels == 0 && !h->fu.n_part_fits(h->A)) h->fu_n_valid = false;  // (the lists were built again, others)
   if (h->fu.gh_state == fused_state::NONE) DN_TRY(h->fu.gram_of(h->H, h->m, true));
   if (!h->fu_n_valid) {
     if (h->A->n_panels > 0) {
@@ -574,7 +592,7 @@ static int fused_update_W(dnpeff_nmf* h) {
 
 static int fused_update_H(dnpeff_nmf* h) {
   DN_TRY(products_for(h));
-  DN_TRY(fused_plan_build(h->A, h->r));
+  DN_TRY(fused_plan_build(h->A, h->r, h->fu.xcd));
   if (h->fu.gw_state == fused_state::NONE) DN_TRY(h->fu.gram_of(h->W, h->n, false));
   h->nw_valid = h->gh_valid = h->fu_n_valid = false;
   return h->fu.update_h(h->A, h->W, h->H, h->eps);

@@ -980,7 +980,6 @@ __global__ void __launch_bounds__(256)
 // 1000 of 1024, r = 32 (a workgroup has 128 entries then), 782 / 788 at 2000 of 2048, r = 8, 796 / 754 at 300 of 2048, r = 64,
 // 5880 / 5476 at 1000 of 4096, r = 96, 9751 / 8205 at 2000 of 8192, r = 60.
 static bool by_xcd(const fused_plan& f, int r) { return f.x_seg && r <= FU_XCD_RANK; }
-static const int* first_chunks(const fused_plan& f, int r) { return by_xcd(f, r) ? f.x_base : f.n_base; }
 
 static int fused_xcd_build(dnpeff_csr* S) {
   fused_plan& f = S->fused;
@@ -1012,7 +1011,7 @@ static int fused_xcd_build(dnpeff_csr* S) {
   return 0;
 }
 
-int fused_plan_build(dnpeff_csr* S, int r) {
+int fused_plan_build(dnpeff_csr* S, int r, bool xcd) {
   fused_plan& f = S->fused;
   hipStream_t st = stream();
   if (!f.pairs) {
@@ -1025,11 +1024,11 @@ int fused_plan_build(dnpeff_csr* S, int r) {
     DN_LAUNCH_CHECK();
   }
   DN_TRY(fused_tiles_build(S, r));
-  if (r <= FU_XCD_RANK && f.x_parts == 0 && S->n_panels == 0) {
+  if (xcd && r <= FU_XCD_RANK && f.x_parts == 0 && S->n_panels == 0) {
     DN_CHECK(has_row_major(S), "row-major copy of the matrix was released");
     DN_TRY(fused_xcd_build(S));
   }
-  if (!f.chunks && !by_xcd(f, r) && S->n_panels == 0) {
+  if (!f.chunks && !(xcd && by_xcd(f, r)) && S->n_panels == 0) {
     DN_CHECK(has_row_major(S), "row-major copy of the matrix was released");
     const int64_t chunk = fu_chunk_entries(S->nnz);
     dbuf<int64_t> base;
@@ -1096,8 +1095,9 @@ static fu_h_kernel fu_h_of(int64_t m, int tile_cols, bool totals) {
   return 64 * m * fu_blocks(Q, R) <= FU_PAST_BYTES ? fu_h_of<Q, R, true>(tile_cols, totals) : fu_h_of<Q, R, false>(tile_cols, totals);
 }
 
-int fused_state::create(const dnpeff_csr* S, int64_t n, int rank) {
+int fused_state::create(const dnpeff_csr* S, int64_t n, int rank, bool xcd_lists) {
   r = rank;
+  xcd = xcd_lists;
   S_floats = fused_gram_floats(r);
   const fused_plan& f = S->fused;
   int64_t most = 0;  // workgroups that the chip holds
@@ -1165,9 +1165,9 @@ int fused_state::gram_of(const float* X, int64_t rows, bool of_h) {
 
 int fused_state::product_n(const dnpeff_csr* S, const float* H) {
   const fused_plan& f = S->fused;
-  const bool xcd = by_xcd(f, r);
-  DN_CHECK(xcd || (has_row_major(S) && f.chunks), "row-major copy of the matrix was released");
-  const int64_t chunks = xcd ? 8 * S->n_rows * f.x_parts : f.n_chunks;
+  n_by_xcd = xcd && by_xcd(f, r);
+  DN_CHECK(n_by_xcd || (has_row_major(S) && f.chunks), "row-major copy of the matrix was released");
+  const int64_t chunks = n_by_xcd ? 8 * S->n_rows * f.x_parts : f.n_chunks;
   if (n_part_floats < chunks * r + 4) {
     dfree(n_part);
     n_part = nullptr;
@@ -1178,10 +1178,10 @@ int fused_state::product_n(const dnpeff_csr* S, const float* H) {
   const dim3 grid((unsigned)(chunks + sums)), block(256);
   if (grid.x > 0) {
     auto go = [&](auto kernel) {
-      hipLaunchKernelGGL(kernel, grid, block, 0, stream(), f.chunks, f.x_seg, f.x_parts, xcd ? f.x_col : S->colind,
-                         xcd ? f.x_val : S->vals, r, H, n_part, sums, gh_part, h_wgs, S_floats, gh_sum);
+      hipLaunchKernelGGL(kernel, grid, block, 0, stream(), f.chunks, f.x_seg, f.x_parts, n_by_xcd ? f.x_col : S->colind,
+                         n_by_xcd ? f.x_val : S->vals, r, H, n_part, sums, gh_part, h_wgs, S_floats, gh_sum);
     };
-#define DN_FU_N(LPR) xcd ? go(k_fu_n<LPR, true>) : go(k_fu_n<LPR, false>)
+#define DN_FU_N(LPR) n_by_xcd ? go(k_fu_n<LPR, true>) : go(k_fu_n<LPR, false>)
     if (r <= 8) DN_FU_N(2);
     else if (r <= 16) DN_FU_N(4);
     else if (r <= 32) DN_FU_N(8);
@@ -1193,6 +1193,8 @@ int fused_state::product_n(const dnpeff_csr* S, const float* H) {
   if (sums) gh_state = SUMMED;
   return 0;
 }
+
+bool fused_state::n_part_fits(const dnpeff_csr* S) const { return n_by_xcd == (xcd && by_xcd(S->fused, r)); }
 
 int fused_state::sum_h() {
   if (gh_state != PARTS) return 0;
@@ -1211,7 +1213,7 @@ int fused_state::sum_w() {
 int fused_state::update_w(const dnpeff_csr* S, int64_t n, const float* Nw, float* W, float eps) {
   DN_CHECK(gh_state == SUMMED, "H^T H is not at hand");
   const float* N = Nw ? Nw : n_part;
-  const int* base = Nw ? nullptr : first_chunks(S->fused, r);
+  const int* base = Nw ? nullptr : n_by_xcd ? S->fused.x_base : S->fused.n_base;
   if (r > FUSED_NARROW_RANK)
     DN_TRY(fuw_launch_w(w_wgs, n, r, base, N, W, eps, gh_sum, gw_part));
   else DN_TRY(fu_dispatch(r, [&](auto tag) {
@@ -1245,7 +1247,7 @@ int fused_state::loss_sums(const dnpeff_csr* S, int64_t n, const float* Nw, cons
   DN_TRY(sum_h());
   DN_TRY(sum_w());
   const int parts = (int)ceil_div(n, 16);
-  hipLaunchKernelGGL(k_fu_dot, dim3((unsigned)parts), dim3(256), 0, stream(), n, r, Nw ? nullptr : first_chunks(S->fused, r),
+  hipLaunchKernelGGL(k_fu_dot, dim3((unsigned)parts), dim3(256), 0, stream(), n, r, Nw ? nullptr : n_by_xcd ? S->fused.x_base : S->fused.n_base,
                      Nw ? Nw : n_part, W, dots);
   hipLaunchKernelGGL(k_fu_loss, dim3(1), dim3(256), 0, stream(), dots, parts, r, gw_sum, gh_sum, out2);
   DN_LAUNCH_CHECK();
@@ -1258,14 +1260,19 @@ double fused_tiles_bytes(int64_t m, int64_t nnz) {
 }
 
 double fused_list_bytes(int64_t n, int64_t m, int64_t nnz) {
-  return 16.0 * (double)(nnz + 1) + fused_tiles_bytes(m, nnz) + 16.0 * (double)(FU_CHUNKS + n) + 68.0 * (double)(n + 1);
+  return 8.0 * (double)(nnz + 1) + fused_tiles_bytes(m, nnz) + 16.0 * (double)(FU_CHUNKS + n) + 4.0 * (double)(n + 1);
+}
+
+double fused_xcd_bytes(int64_t n, int64_t nnz, int r) {
+  if (r > FU_XCD_RANK || nnz / n < FU_XCD_ROW) return 0.0;
+  return 8.0 * (double)nnz + 68.0 * (double)(n + 1) + 4.0 * 7.0 * (double)n * r;  // (eight chunks to a row)
 }
 
 double fused_state_bytes(int64_t n, int64_t m, int64_t nnz, int r) {
   const double S = 4.0 * fused_gram_floats(r);
   // workgroups of the H update: one round of what the chip holds, or enough rounds of them
   const double wgs = (r > FUSED_NARROW_RANK ? 4.0 : 8.0) * n_cus() + ((double)m + (double)nnz / 8.0) / FU_MOST_COLS;
-  return 4.0 * ((double)(FU_CHUNKS + 8 * n) * r + 4.0) + S * (wgs + (double)n / FUW_COLS + 3.0) + (double)n;
+  return 4.0 * ((double)(FU_CHUNKS + n) * r + 4.0) + S * (wgs + (double)n / FUW_COLS + 3.0) + (double)n;
 }
 
 bool fused_supported(int64_t n, int64_t m, int64_t nnz, int r) {

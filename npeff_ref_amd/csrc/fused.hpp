@@ -22,12 +22,14 @@ constexpr int64_t FU_CHUNKS = 4096;  // workgroups that A H^T is cut into where 
 
 bool fused_supported(int64_t n, int64_t m, int64_t nnz, int r);
 // What the lists of a matrix (alone: its tiles, which ranks above 128 use as well) and a context's buffers take at
-// most, in bytes.
+// most, in bytes; fused_xcd_bytes: what they take on top where A H^T goes by XCD, which the step can do without.
 double fused_tiles_bytes(int64_t m, int64_t nnz);
 double fused_list_bytes(int64_t n, int64_t m, int64_t nnz);
+double fused_xcd_bytes(int64_t n, int64_t nnz, int r);
 double fused_state_bytes(int64_t n, int64_t m, int64_t nnz, int r);
-// Tiles, packed entries and chunks of a matrix without dense head (needs csr_ensure_products).
-int fused_plan_build(dnpeff_csr* S, int r);
+// Tiles, packed entries and chunks of a matrix without dense head (needs csr_ensure_products).  xcd: the lists by XCD
+// as well where its rows suit them (there is room for fused_xcd_bytes).
+int fused_plan_build(dnpeff_csr* S, int r, bool xcd);
 
 // Updates at ranks 65 ... 128 (fused_wide.hip).
 int fuw_per_cu(int r, int* wgs);
@@ -45,6 +47,8 @@ struct fused_state {
   enum gram_state { NONE, PARTS, SUMMED };
   int r = 0, S_floats = 0, h_wgs = 0, w_wgs = 0;
   bool h_totals = false;     // the H update adds its Gram sums up in fp64
+  bool xcd = false;          // A H^T goes by XCD where the matrix has the lists for it
+  bool n_by_xcd = false;     // n_part is by XCD
   float* gh_part = nullptr;  // partial H^T H of the last H update, one per workgroup
   float* gw_part = nullptr;
   float* gh_sum = nullptr;
@@ -54,11 +58,13 @@ struct fused_state {
   double* dots = nullptr;
   gram_state gh_state = NONE, gw_state = NONE;
 
-  int create(const dnpeff_csr* S, int64_t n, int rank);
+  int create(const dnpeff_csr* S, int64_t n, int rank, bool xcd_lists);
   void destroy();
   // X^T X of a factor as it is ([rows, r]): partial matrices of H or of W
   int gram_of(const float* X, int64_t rows, bool of_h);
   int product_n(const dnpeff_csr* S, const float* H);
+  // whether n_part is laid out as the lists that the matrix has now say
+  bool n_part_fits(const dnpeff_csr* S) const;
   int sum_h();
   int sum_w();
   // Nw: A H^T [n, r], or NULL for the chunk sums of product_n

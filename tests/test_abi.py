@@ -202,3 +202,21 @@ def test_memory_plan_of_padded_ranks_and_small_ranks():
         assert e["sparse_copies"] >= 24.0 * z  # row-major, by columns, packed for the step
         assert e["factors"] >= 4.0 * r * (2 * m + 3 * n) + 4.0 * r * n
     assert d.plan_estimate(n, m, z, 5000, 100, False)["sparse_copies"] == 16.0 * z  # a dense head: the separate kernels
+
+
+def test_memory_plan_of_the_lists_by_xcd():
+    """The lists that A H^T uses by XCD (8 bytes per entry) are priced where they are built, up to 96 components on long
+    rows, and the step of small ranks does not need them: on a device too small for them it runs without."""
+    n, m, z = 1000, 800_000, 4_000_000
+
+    def per_entry(rank, nnz=z, **on):
+        return d.plan_estimate(n, m, nnz, 0, rank, False, **on)["sparse_copies"] / nnz
+
+    assert 32.0 <= per_entry(96) < 33.0 and 32.0 <= per_entry(8) < 33.0
+    assert 24.0 <= per_entry(97) < 25.0 and 24.0 <= per_entry(128) < 25.0
+    assert 24.0 <= per_entry(50, nnz=1_000_000) < 26.0  # 1000 entries to a row
+    whole = sum(d.plan_estimate(n, m, z, 0, 50, False, total_bytes=16 * 2**30).values())
+    assert 32.0 <= per_entry(50, total_bytes=int(whole + 1)) < 33.0
+    assert 24.0 <= per_entry(50, total_bytes=int(whole - 1)) < 25.0
+    assert 24.0 <= per_entry(50, total_bytes=int(whole - 7 * z)) < 25.0
+    assert per_entry(50, total_bytes=int(whole - 10 * z)) == 16.0
