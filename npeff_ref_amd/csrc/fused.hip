@@ -22,6 +22,7 @@
 #include "fused.hpp"
 
 #include <algorithm>
+#include <cstdio>
 
 namespace dn {
 
@@ -981,6 +982,57 @@ __global__ void __launch_bounds__(256)
 // 5880 / 5476 at 1000 of 4096, r = 96, 9751 / 8205 at 2000 of 8192, r = 60.
 static bool by_xcd(const fused_plan& f, int r) { return f.x_seg && r <= FU_XCD_RANK; }
 
+// How evenly the lists deal the entries out.  out[10 workgroup + x]: entries of XCD x, + 8: the sum of the rows' largest
+// shares, + 9: the largest share of all.
+constexpr int FU_BALANCE = 10;
+__global__ void __launch_bounds__(256) k_fu_xcd_balance(const int64_t* __restrict__ x_seg, int64_t n, unsigned long long* __restrict__ out) {
+  __shared__ unsigned long long sums[FU_BALANCE];
+  if (threadIdx.x < FU_BALANCE) sums[threadIdx.x] = 0;
+  __syncthreads();
+  unsigned long long mine[FU_BALANCE] = {};
+  for (int64_t row = (int64_t)blockIdx.x * 256 + threadIdx.x; row < n; row += (int64_t)gridDim.x * 256) {
+    unsigned long long most = 0;
+#pragma unroll
+    for (int x = 0; x < 8; x++) {
+      const unsigned long long len = (unsigned long long)(x_seg[8 * row + x + 1] - x_seg[8 * row + x]);
+      mine[x] += len;
+      most = len > most ? len : most;
+    }
+    mine[8] += most;
+    mine[9] = most > mine[9] ? most : mine[9];
+  }
+#pragma unroll
+  for (int i = 0; i < 9; i++) atomicAdd(&sums[i], mine[i]);
+  atomicMax(&sums[9], mine[9]);
+  __syncthreads();
+  if (threadIdx.x < FU_BALANCE) out[FU_BALANCE * blockIdx.x + threadIdx.x] = sums[threadIdx.x];
+}
+
+// Column ids that repeat with a period of 128, or rows of blocks of columns, leave an XCD or a workgroup with more than
+// its share, and the rest of the chip waits for it.  Ten iterations in chunks of whole rows / by XCD at 500 rows of 4096, r = 8,
+// 2000 of 2048, r = 32, and 300 of 16,384, r = 32, where one XCD has 1.2 times its share: 418 / 440, 1226 / 1031, 1483 / 1058
+// us, 1.4 times: 420 / 456, 1217 / 1046, 1471 / 1117, twice: 421 / 508, 1208 / 1150, 1464 / 1258, all: 391 / 976, 902 /
+// 2401, 999 / 2860; where every row gives another XCD 1.6 times its share: 420 / 453, 1222 / 1039, 1490 / 1073, twice: 419 /
+// 462, 1220 / 1062, 1462 / 1154, all: 421 / 684, 935 / 1646, 1034 / 2438.
+static int fused_xcd_balanced(const int64_t* x_seg, int64_t n, int64_t nnz, bool* even) {
+  unsigned long long* words = nullptr;
+  DN_TRY(host_words(&words));
+  const int wgs = (int)std::min<int64_t>(HOST_WORDS / FU_BALANCE, ceil_div(n, 256));
+  hipLaunchKernelGGL(k_fu_xcd_balance, dim3((unsigned)wgs), dim3(256), 0, stream(), x_seg, n, words);
+  DN_LAUNCH_CHECK();
+  DN_HIP(hipStreamSynchronize(stream()));
+  double xcd[8] = {}, rows = 0.0, share = 0.0, most = 0.0;
+  for (int w = 0; w < wgs; w++) {
+    for (int x = 0; x < 8; x++) xcd[x] += (double)words[FU_BALANCE * w + x];
+    rows += (double)words[FU_BALANCE * w + 8];
+    share = std::max(share, (double)words[FU_BALANCE * w + 9]);
+  }
+  for (double x : xcd) most = std::max(most, x);
+  const double eighth = (double)nnz / 8.0;
+  *even = most <= 1.25 * eighth && rows <= 1.6 * eighth && share <= 4.0 * eighth / (double)n;
+  return 0;
+}
+
 static int fused_xcd_build(dnpeff_csr* S) {
   fused_plan& f = S->fused;
   const int64_t n = S->n_rows, mean = S->nnz / n;
@@ -1003,6 +1055,11 @@ static int fused_xcd_build(dnpeff_csr* S) {
   hipLaunchKernelGGL(k_fu_xcd_split, dim3((unsigned)n), dim3(256), 0, stream(), S->rowptr, S->colind, S->vals, n, (int)parts, col.p,
                      val.p, seg.p, base.p);
   DN_LAUNCH_CHECK();
+  bool even = false;
+  DN_TRY(fused_xcd_balanced(seg.p, n, S->nnz, &even));
+  if (tuning().verbose != 0.0)
+    fprintf(stderr, "dnpeff: A H^T %s\n", even ? "by XCD" : "in chunks of whole rows: the columns load the XCDs unevenly");
+  if (!even) return 0;
   f.x_seg = seg.release();
   f.x_col = col.release();
   f.x_val = val.release();

@@ -234,6 +234,34 @@ def test_rows_grouped_by_xcd(n, m, r, fill):
     A.close()
 
 
+@pytest.mark.parametrize("kind,by_xcd", [("any", True), ("one eighth", False), ("an eighth per row", False),
+                                         ("one long share", False)])
+def test_columns_that_load_the_xcds_unevenly(kind, by_xcd, tune, capfd):
+    """Entries grouped by XCD (16 columns each in turn) where that gives every XCD and every workgroup about the same, not
+    where the column ids repeat with a period of 128: all rows the same sixteen of it, every row its own, or one row alone."""
+    n, m, k, r = 24, 24_000, 2000, 20
+    rng = np.random.default_rng(7)
+    of = (np.arange(m) >> 4) & 7
+    rows = []
+    for i in range(n):
+        narrow = kind in ("one eighth", "an eighth per row") or (kind == "one long share" and i == 5)
+        among = np.flatnonzero(of == (i % 8 if kind == "an eighth per row" else 3)) if narrow else np.arange(m)
+        rows.append(rng.permutation(among)[:k])
+    rp, ci = np.arange(n + 1, dtype=np.int64) * k, np.concatenate(rows).astype(np.int32)
+    va = rng.random(n * k, dtype=np.float32)
+    A = d.Csr.from_host(rp, ci, va, m)
+    tune("verbose", 1)
+    nmf = d.MuNmf(A, d.MuNmfParams(rank=r, max_iters=4, eps=EPS, seed=5, log_every=2))
+    assert ("A H^T by XCD" in capfd.readouterr().err) == by_xcd
+    tune("verbose", 0)
+    nmf.initialize()
+    W0, H0 = nmf.loadWToHostSync(), nmf.loadHToHostSync()
+    nmf.run(log=lambda s: None)
+    _close(nmf, orc.nmf_f64(rp, ci, va, m, W0, H0, np.float32(EPS), 4, 2))
+    nmf.close()
+    A.close()
+
+
 @pytest.mark.parametrize("n,m,r,fill", [(2, 3, 1, 0.9), (16, 33, 4, 0.5), (17, 2100, 5, 0.05), (128, 640, 16, 0.04),
                                         (127, 300, 9, 0.1), (129, 300, 9, 0.1), (48, 907, 8, 0.07), (60, 500, 15, 0.08)])
 def test_runs_in_one_workgroup(n, m, r, fill):
