@@ -116,10 +116,13 @@ __device__ inline void fu_load_row(const float* __restrict__ row, int g, int r, 
   }
 }
 
-// past: the new rows go past the L2s, which write back what is left in them when the launch ends.  H update with /
-// without: 18.4 / 19.9 us at 300 x 146k, r = 20, 30.7 / 31.4 at 512 x 431k, r = 16; a factor that the memory-side
-// cache would hold in part is better left to it (777 x 862k, r = 50, 172 MB: ten iterations 3.35 / 3.32 ms).
-constexpr int64_t FU_PAST_BYTES = 64 << 20;
+// PAST: the new rows go past the L2s, which write back what is left in them when the launch ends.  That pays while they
+// hold the whole factor (32 MB together); of a larger one most is written back by then.  Ten iterations without / with: 342 /
+// 330 us at 500 x 234k, r = 16 (14 MB), 391 / 377 at 300 x 175k, r = 20 (21 MB), 418 / 403 at 500 x 328k, r = 8 (20 MB), 435 /
+// 428 at 300 x 399k, r = 8 (24 MB), 442 / 436 at 500 x 47k, r = 50 (11 MB); 497 / 505 at 300 x 402k, r = 16 (25 MB),
+// 686 / 705 at 300 x 643k, r = 16 (39 MB), 968 / 997 at 500 x 1.0M, r = 16 (61 MB),
+// 1721 / 1874 at 1500 x 1.1M, r = 32 (135 MB).
+constexpr int64_t FU_PAST_BYTES = 24 << 20;
 template <bool PAST>
 __device__ inline void fu_store(float* dst, float v) {
   if constexpr (PAST) __builtin_nontemporal_store(v, dst);
