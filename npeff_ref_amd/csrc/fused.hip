@@ -981,9 +981,20 @@ __global__ void __launch_bounds__(256)
 // apart in the one order and the other, at r <= 64 5e-6 at most), and keep the order they have always had.
 // Rows of FU_XCD_ROW entries or more on average, of which none is twice as long (a workgroup per row and XCD).  Ten iterations
 // in chunks of whole rows / by XCD: 191 / 215 us at 200 rows of 200 entries, r = 8, 252 / 281 at 500 of 512, r = 16, 488 / 546 at
-// 1000 of 1024, r = 32 (a workgroup has 128 entries then), 782 / 788 at 2000 of 2048, r = 8, 796 / 754 at 300 of 2048, r = 64,
-// 5880 / 5476 at 1000 of 4096, r = 96, 9751 / 8205 at 2000 of 8192, r = 60.
-static bool by_xcd(const fused_plan& f, int r) { return f.x_seg && r <= FU_XCD_RANK; }
+// 1000 of 1024, r = 32 (a workgroup has 128 entries then), 317 / 286 at 500 of 1800, r = 8, 896 / 811 at 2000 of 1800, r = 24,
+// 1550 / 1357, r = 64, 796 / 754 at 300 of 2048, r = 64, 5880 / 5476 at 1000 of 4096, r = 96, 9751 / 8205 at 2000 of 8192, r = 60.
+// Up to 8 components a workgroup of some 256 entries is little more than its start and end, and eight of them to a row of
+// fewer than FU_XCD_ROW_FEW lose where a row makes three even chunks or fewer: 1061 / 1141 at 4000 of 2000, r = 4 (one
+// chunk), 696 / 732 at 2000 of 2048, r = 8 (two), 427 / 435 at 1000 of 2200, r = 4 (three); but 1361 / 1078 at 4000 of 1800,
+// r = 8 (the second chunk has 8 entries), 774 / 741 at 2000 of 2100, 511 / 475 at 1000 of 2400, 1899 / 1367 at 4000 of 2600.
+static bool xcd_rows_suit(int64_t n, int64_t nnz, int r) {
+  const int64_t mean = nnz / n;
+  if (r > FU_XCD_RANK || mean < FU_XCD_ROW) return false;
+  if (r > 8 || mean >= FU_XCD_ROW_FEW) return true;
+  const int64_t chunk = fu_chunk_entries(nnz), cut = ceil_div(mean, chunk);
+  return cut > 3 || 10 * mean < 9 * cut * chunk;
+}
+static bool by_xcd(const dnpeff_csr* S, int r) { return S->fused.x_seg && xcd_rows_suit(S->n_rows, S->nnz, r); }
 
 // How evenly the lists deal the entries out.  out[10 workgroup + x]: entries of XCD x, + 8: the sum of the rows' largest
 // shares, + 9: the largest share of all.
@@ -1040,7 +1051,7 @@ static int fused_xcd_build(dnpeff_csr* S) {
   fused_plan& f = S->fused;
   const int64_t n = S->n_rows, mean = S->nnz / n;
   f.x_parts = -1;
-  if (mean < FU_XCD_ROW || !xcd_round_robin()) return 0;
+  if (!xcd_round_robin()) return 0;
   std::vector<int64_t> rowptr((size_t)n + 1);
   DN_HIP(copy_down(rowptr.data(), S->rowptr, sizeof(int64_t) * rowptr.size()));
   int64_t most = 0;
@@ -1084,11 +1095,11 @@ int fused_plan_build(dnpeff_csr* S, int r, bool xcd) {
     DN_LAUNCH_CHECK();
   }
   DN_TRY(fused_tiles_build(S, r));
-  if (xcd && r <= FU_XCD_RANK && f.x_parts == 0 && S->n_panels == 0) {
+  if (xcd && f.x_parts == 0 && S->n_panels == 0 && xcd_rows_suit(S->n_rows, S->nnz, r)) {
     DN_CHECK(has_row_major(S), "row-major copy of the matrix was released");
     DN_TRY(fused_xcd_build(S));
   }
-  if (!f.chunks && !(xcd && by_xcd(f, r)) && S->n_panels == 0) {
+  if (!f.chunks && !(xcd && by_xcd(S, r)) && S->n_panels == 0) {
     DN_CHECK(has_row_major(S), "row-major copy of the matrix was released");
     const int64_t chunk = fu_chunk_entries(S->nnz);
     dbuf<int64_t> base;
@@ -1225,7 +1236,7 @@ int fused_state::gram_of(const float* X, int64_t rows, bool of_h) {
 
 int fused_state::product_n(const dnpeff_csr* S, const float* H) {
   const fused_plan& f = S->fused;
-  n_by_xcd = xcd && by_xcd(f, r);
+  n_by_xcd = xcd && by_xcd(S, r);
   DN_CHECK(n_by_xcd || (has_row_major(S) && f.chunks), "row-major copy of the matrix was released");
   const int64_t chunks = n_by_xcd ? 8 * S->n_rows * f.x_parts : f.n_chunks;
   if (n_part_floats < chunks * r + 4) {
@@ -1254,7 +1265,7 @@ int fused_state::product_n(const dnpeff_csr* S, const float* H) {
   return 0;
 }
 
-bool fused_state::n_part_fits(const dnpeff_csr* S) const { return n_by_xcd == (xcd && by_xcd(S->fused, r)); }
+bool fused_state::n_part_fits(const dnpeff_csr* S) const { return n_by_xcd == (xcd && by_xcd(S, r)); }
 
 int fused_state::sum_h() {
   if (gh_state != PARTS) return 0;
@@ -1324,7 +1335,7 @@ double fused_list_bytes(int64_t n, int64_t m, int64_t nnz) {
 }
 
 double fused_xcd_bytes(int64_t n, int64_t nnz, int r) {
-  if (r > FU_XCD_RANK || nnz / n < FU_XCD_ROW) return 0.0;
+  if (!xcd_rows_suit(n, nnz, r)) return 0.0;
   return 8.0 * (double)nnz + 68.0 * (double)(n + 1) + 4.0 * 7.0 * (double)n * r;  // (eight chunks to a row)
 }
 

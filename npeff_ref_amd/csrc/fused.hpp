@@ -18,6 +18,7 @@ constexpr int FUW_COLS = 32;           // columns (rows of W) per tile there
 constexpr int FU_MOST_COLS = 2048;
 constexpr int FU_XCD_RANK = 96;        // ranks up to which, and entries of a row from which, A H^T goes by XCD
 constexpr int64_t FU_XCD_ROW = 1792;
+constexpr int64_t FU_XCD_ROW_FEW = 2560;  // (up to 8 components)
 constexpr int64_t FU_CHUNKS = 4096;  // workgroups that A H^T is cut into where its rows allow
 
 bool fused_supported(int64_t n, int64_t m, int64_t nnz, int r);

@@ -215,6 +215,9 @@ def test_memory_plan_of_the_lists_by_xcd():
     assert 32.0 <= per_entry(96) < 33.0 and 32.0 <= per_entry(8) < 33.0
     assert 24.0 <= per_entry(97) < 25.0 and 24.0 <= per_entry(128) < 25.0
     assert 24.0 <= per_entry(50, nnz=1_000_000) < 26.0  # 1000 entries to a row
+    # up to 8 components rows below 2560 entries only where they make uneven chunks (768 entries at these sizes)
+    assert 24.0 <= per_entry(8, nnz=2_300_000) < 25.0 and 32.0 <= per_entry(9, nnz=2_300_000) < 34.0
+    assert 32.0 <= per_entry(8, nnz=2_400_000) < 34.0 and 32.0 <= per_entry(8, nnz=2_560_000) < 34.0
     whole = sum(d.plan_estimate(n, m, z, 0, 50, False, total_bytes=16 * 2**30).values())
     assert 32.0 <= per_entry(50, total_bytes=int(whole + 1)) < 33.0
     assert 24.0 <= per_entry(50, total_bytes=int(whole - 1)) < 25.0

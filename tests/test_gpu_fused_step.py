@@ -294,11 +294,12 @@ def test_runs_in_one_workgroup(n, m, r, fill):
     A.close()
 
 
-def test_ranks_on_either_side_of_the_grouping():
-    """Contexts of 40 and of 100 components on one matrix, whose rows the first groups by XCD: each gives the bits
-    that it gives on a matrix of its own, whichever comes first."""
-    n, m = 120, 6000
-    rp, ci, va = _matrix(n, m, seed=3, fill=0.35)
+@pytest.mark.parametrize("n,fill,ranks", [(120, 0.35, (40, 100)), (1010, 0.42, (9, 8))])
+def test_ranks_on_either_side_of_the_grouping(n, fill, ranks):
+    """Contexts of two ranks on one matrix, whose rows only the first groups by XCD (40 and 100 components; 9 and 8
+    where a row makes three even chunks): each gives the bits that it gives on a matrix of its own, whichever comes first."""
+    m = 6000
+    rp, ci, va = _matrix(n, m, seed=3, fill=fill)
 
     def run(A, r):
         nmf = d.MuNmf(A, d.MuNmfParams(rank=r, max_iters=3, eps=EPS, seed=5, log_every=3))
@@ -308,11 +309,12 @@ def test_ranks_on_either_side_of_the_grouping():
         return out
 
     alone = {}
-    for r in (40, 100):
+    first, second = ranks
+    for r in ranks:
         A = d.Csr.from_host(rp, ci, va, m)
         alone[r] = run(A, r)
         A.close()
-    for order in ((40, 100, 40), (100, 40, 100)):
+    for order in ((first, second, first), (second, first, second)):
         A = d.Csr.from_host(rp, ci, va, m)
         for r in order:
             for got, want in zip(run(A, r), alone[r]):
