@@ -24,9 +24,13 @@ static int64_t fs_bytes(int64_t n, int64_t m, int64_t nnz, int r) {
   return FS_FIXED + 16 * (int64_t)((r + 3) / 4) * (m + 2 * n + 45) + 64 + 16 * nnz + 4 * (n + m + 2);
 }
 
-// (a column is one chain of multiply-adds: no more than 128 rows)
+// (A column is one chain of multiply-adds: no more than 128 rows.)  Where one compute unit is slower than the launches
+// the sizes are left to them: they take 145 to 160 us for ten iterations and the loss up to 128 rows, one workgroup some 47 + 0.050
+// m + 0.37 n + 0.0073 nnz (500 matrices of even and of Zipf columns, 6 us off on average).  One workgroup / launches: 63 / 149
+// at 8 x 40, 131 / 168 at 48 x 368 with 3,072 entries, 125 / 150 at 64 x 1000 with 1,280, 147 / 149 with 3,200; past the line
+// 193 / 153 at 128 x 1000 with 6,400, 233 / 150 at 87 x 2966 with 435, 314 / 149 at 128 x 4000 with 2,560.
 bool fused_small_fits(int64_t n, int64_t m, int64_t nnz, int r) {
-  return r <= 16 && n <= 128 && m < 65536 && nnz < 65536 && fs_bytes(n, m, nnz, r) <= FS_LDS;
+  return r <= 16 && n <= 128 && m < 65536 && nnz < 65536 && 20 * m + 150 * n + 3 * nnz <= 40000 && fs_bytes(n, m, nnz, r) <= FS_LDS;
 }
 
 struct fs_args {

@@ -263,7 +263,8 @@ def test_columns_that_load_the_xcds_unevenly(kind, by_xcd, tune, capfd):
 
 
 @pytest.mark.parametrize("n,m,r,fill", [(2, 3, 1, 0.9), (16, 33, 4, 0.5), (17, 2100, 5, 0.05), (128, 640, 16, 0.04),
-                                        (127, 300, 9, 0.1), (129, 300, 9, 0.1), (48, 907, 8, 0.07), (60, 500, 15, 0.08)])
+                                        (127, 300, 9, 0.1), (129, 300, 9, 0.1), (48, 907, 8, 0.07), (60, 500, 15, 0.08),
+                                        (128, 500, 16, 0.04), (17, 1600, 5, 0.05), (8, 1900, 3, 0.05)])
 def test_runs_in_one_workgroup(n, m, r, fill):
     """Runs that one workgroup's LDS holds (128 rows and 16 components at most): several steps in one launch give
     the bits of as many launches of one step, and what the two updates of the launched step give (fp32 sums in another
