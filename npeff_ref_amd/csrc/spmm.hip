@@ -239,9 +239,8 @@ __global__ void __launch_bounds__(256)
 // of one row after the other are 128 to 256 trips.  Here they are 32, and with 8 slices (rank 512) an XCD only ever
 // holds its eighth of the rows in its L2: 56 -> 37 us at 300 rows of 1000 entries, rank 256, 360 -> 341 at 800 x
 // 4000 (3.3 GB of rows, mostly from the fabric), 110 -> 73 at 1000 x 500 and 177 -> 126 at 250 x 3000, rank 512, 192 ->
-// 171 at 400 x 3000, rank 384; 37.6 -> 39.0 at 1800 x 300, rank 256, where the L2s bound either.  LPR 8 / 16 / 32 /
-// 64 at 300 x 1000, rank 256: 46 / 41 / 37 / 39; at rank 512, 250 x 3000: 161 / 126 / 133 / 170.  Every sum is added up
-// in the order of k_spmm_n: the same bits.
+// 171 at 400 x 3000, rank 384 (spmm_slices_from: where not).  LPR 8 / 16 / 32 / 64 at 300 x 1000, rank 256: 46 / 41 / 37 / 39;
+// at rank 512, 250 x 3000: 161 / 126 / 133 / 170.  Every sum is added up in the order of k_spmm_n: the same bits.
 template <int LPR>
 __global__ void __launch_bounds__(256)
     k_spmm_n_slices(const int64_t* __restrict__ rowptr, const int32_t* __restrict__ colind,
@@ -1558,6 +1557,28 @@ static int launch_spmm_n_sweep(const dnpeff_csr* A, int r, const float* H_mr, bo
   return 0;
 }
 
+// Entries of a chunk on average from which its sums go by slices.  Short rows are bound by what a workgroup does beside its
+// entries, and every slice does that again; with few chunks the slices are what fills the chip.  Time of k_spmm_n over that of
+// k_spmm_n_slices, by entries per row (two figures: H of few / of many rows):
+//              20     60    120          250          400          700          1000         2048
+//   10,000 rows
+//   r = 256    0.62   0.64  0.64         0.70         0.73 / 0.78  0.88 / 1.06  1.05 / 1.18  1.23 / 1.20 (4000 rows)
+//   r = 384    0.56   0.76  0.88         1.02         1.12         1.18         1.29 / 1.16  1.45 / 1.12
+//   r = 512    0.43   0.59  0.71         0.89 / 0.96  1.05 / 1.18  1.48         1.68         2.13 / 1.70
+//   r = 768    0.43   0.64  0.79         1.01 / 1.07  1.19 / 1.26  1.45         1.63 / 1.37  1.84 / 1.26
+//   r = 1024   0.36   0.58  0.80         1.11 / 1.18  1.37 / 1.43  1.81         2.01 / 1.78  2.34 / 1.51
+//   300 rows
+//   r = 256    0.81   0.84  0.87         0.92 / 1.12  0.95 / 1.07  0.94 / 1.09  0.95 / 1.05  1.10 / 1.04
+//   r = 384    0.87   1.26  1.66         2.2          2.5          2.6          2.5          1.90 / 1.22
+//   r = 512    0.79   0.94  1.10 / 1.28  1.32 / 1.92  1.44 / 1.93  1.82         1.93 / 1.52  1.76 / 1.59
+//   r = 768    1.04   1.61  2.15 / 2.70  3.2          3.9          4.0 / 3.1    3.1 / 2.2    1.79 / 1.26
+//   r = 1024   0.74   1.0   1.09 / 1.50  1.42 / 1.65  1.85         2.11 / 1.77  1.89 / 1.61  2.8 / 1.6
+static int64_t spmm_slices_from(int r, int64_t n_chunks) {
+  if (r == 256) return 1000;
+  if (n_chunks <= 512) return r % 512 == 0 ? 120 : 60;
+  return r == 512 ? 600 : r == 1024 ? 350 : 250;
+}
+
 // part: 0 = the whole product; 1 = what may run beside another kernel: the dense head, and the
 // plain panels where they are the far tail (no slot lists: a long kernel that waits for the
 // fabric); 2 = the rest (swept pieces and slot lists, whose workgroups walk in lock step and
@@ -1611,7 +1632,8 @@ int launch_spmm_n(const dnpeff_csr* A_full, int r, const float* H_mr, int part) 
   dim3 grid((unsigned)A->n_chunks), block(256);
   // (slices of 128 components at rank 256, of 64 above)
   const int slices = r / (r == 256 ? 128 : 64);
-  if (r >= 256 && r % 128 == 0 && ((uintptr_t)H_mr % 16) == 0 && A->n_chunks * slices < ((int64_t)1 << 24)) {
+  if (r >= 256 && r % 128 == 0 && A->nnz >= spmm_slices_from(r, A->n_chunks) * A->n_chunks && ((uintptr_t)H_mr % 16) == 0 &&
+      A->n_chunks * slices < ((int64_t)1 << 24)) {
     if (r == 256)
       hipLaunchKernelGGL((k_spmm_n_slices<32>), dim3((unsigned)(ceil_div(A->n_chunks, 2) * slices)), block, 0, stream(),
                          A->rowptr, A->colind, A->vals, A->chunk_base, A->n_rows, A->n_chunks, slices, r, H_mr, partials);

@@ -129,6 +129,30 @@ def test_spmm_n_slices(n, r):
     A.close()
 
 
+@pytest.mark.parametrize("n,r,per", [(37, 256, 999), (37, 256, 1001), (37, 384, 59), (37, 384, 61), (37, 512, 119),
+                                     (37, 1024, 121), (520, 512, 599), (520, 1024, 351), (520, 640, 249), (520, 896, 251)])
+def test_spmm_n_on_either_side_of_the_slices(n, r, per):
+    """Short rows stay with the row chunks, and slices give the bits of those: ranks and rows around the line."""
+    m = 4000
+    rng = np.random.default_rng(n + r + per)
+    ci = np.concatenate([rng.permutation(m)[:per] for _ in range(n)]).astype(np.int32)
+    rp = np.arange(n + 1, dtype=np.int64) * per
+    va = rng.random(n * per, dtype=np.float32)
+    A = d.Csr.from_host(rp, ci, va, m)
+    H = rng.random((m, r), dtype=np.float32)
+    dH = d.DeviceArray.from_numpy(H)
+    outs = []
+    for variant in (0, 2):
+        dN = d.DeviceArray.from_numpy(np.full((n, r), np.nan, dtype=np.float32))
+        d.binding._check(d.lib.dnpeff_op_spmm_n_variant(A._h, r, dH.ptr, dN.ptr, variant))
+        d.sync()
+        outs.append(dN.numpy())
+    want = orc.spmm_n_f64(rp, ci, va, H)
+    assert (np.abs(outs[0] - want) <= 600 * 2.0 ** -24 * np.abs(want)).all()
+    assert np.array_equal(outs[0], outs[1])
+    A.close()
+
+
 @pytest.mark.parametrize("rows", [128, 129, 160, 191, 1023])
 @pytest.mark.parametrize("r", [256, 384, 512, 768])
 def test_gram_on_few_rows(rows, r):
