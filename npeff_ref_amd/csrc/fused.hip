@@ -42,6 +42,8 @@ __host__ __device__ constexpr int fu_lpr(int Q, int R) {
 // They are read in 16-byte pieces, up to eight parts at a time, and come to their places through `stage` (as
 // much LDS as a packed matrix, free again when this returns): with every thread picking its numbers from memory
 // the vector-memory unit was busy for 16 lines per load (5 parts, 300 x 146k, r = 20: H update 23.6 us, now 20.0).
+// All pieces of a thread are asked for together, and a single matrix once: piece after piece, four parts each, ten iterations at
+// 500 x 2000, r = 64, took 355 us, now 337.
 template <int Q, int R>
 __device__ inline void fu_load_g(const float* __restrict__ part, int n_parts, int r, float* __restrict__ ga,
                                  float* __restrict__ stage) {
@@ -50,31 +52,48 @@ __device__ inline void fu_load_g(const float* __restrict__ part, int n_parts, in
     const int i = threadIdx.x & 3, rho = (threadIdx.x >> 2) & 15, g = threadIdx.x >> 6;
     const int k = R == 0 ? 4 * g + i : R * g + i, c = R == 0 ? rho : R * (rho >> 2) + (rho & 3);
     const bool ok = k < r && c < r && (R == 0 || (i < R && (rho & 3) < R));
+    const float* src = part + (ok ? k * 16 + c : 0);
     double sum = 0.0;
-    for (int p = 0; p < n_parts; p += P) {
-      float v[P];
+    if (n_parts == 1) sum = (double)*src;
+    else
+      for (int p = 0; p < n_parts; p += P) {
+        float v[P];
 #pragma unroll
-      for (int u = 0; u < P; u++) v[u] = part[(int64_t)(p + u < n_parts ? p + u : p) * S + (ok ? k * 16 + c : 0)];
+        for (int u = 0; u < P; u++) v[u] = src[(int64_t)(p + u < n_parts ? p + u : p) * S];
 #pragma unroll
-      for (int u = 0; u < P; u++) sum += p + u < n_parts ? (double)v[u] : 0.0;
-    }
+        for (int u = 0; u < P; u++) sum += p + u < n_parts ? (double)v[u] : 0.0;
+      }
     ga[threadIdx.x] = ok ? (float)sum : 0.0f;
     return;
   }
+  constexpr int PIECES = (S + 1023) / 1024;
+  const int first = 4 * (int)threadIdx.x;
+  auto at = [&](int j) { return first + 1024 * j < S ? first + 1024 * j : 0; };
+  f32x4 g[PIECES];
+  if (n_parts == 1) {
 #pragma unroll
-  for (int x = 4 * (int)threadIdx.x; x < S; x += 1024) {
-    double sum[4] = {};
+    for (int j = 0; j < PIECES; j++) g[j] = *reinterpret_cast<const f32x4*>(part + at(j));
+  } else {
+    double sum[PIECES][4] = {};
     for (int p = 0; p < n_parts; p += P) {
-      f32x4 v[P];
-#pragma unroll
-      for (int k = 0; k < P; k++) v[k] = *reinterpret_cast<const f32x4*>(part + (int64_t)(p + k < n_parts ? p + k : p) * S + x);
+      f32x4 v[P][PIECES];
 #pragma unroll
       for (int k = 0; k < P; k++)
 #pragma unroll
-        for (int i = 0; i < 4; i++) sum[i] += p + k < n_parts ? (double)v[k][i] : 0.0;
+        for (int j = 0; j < PIECES; j++) v[k][j] = *reinterpret_cast<const f32x4*>(part + (int64_t)(p + k < n_parts ? p + k : p) * S + at(j));
+#pragma unroll
+      for (int k = 0; k < P; k++)
+#pragma unroll
+        for (int j = 0; j < PIECES; j++)
+#pragma unroll
+          for (int i = 0; i < 4; i++) sum[j][i] += p + k < n_parts ? (double)v[k][j][i] : 0.0;
     }
-    *reinterpret_cast<f32x4*>(stage + x) = f32x4{(float)sum[0], (float)sum[1], (float)sum[2], (float)sum[3]};
+#pragma unroll
+    for (int j = 0; j < PIECES; j++) g[j] = f32x4{(float)sum[j][0], (float)sum[j][1], (float)sum[j][2], (float)sum[j][3]};
   }
+#pragma unroll
+  for (int j = 0; j < PIECES; j++)
+    if (first + 1024 * j < S) *reinterpret_cast<f32x4*>(stage + first + 1024 * j) = g[j];
   __syncthreads();
 #pragma unroll
   for (int u = 0; u < N; u++) {
