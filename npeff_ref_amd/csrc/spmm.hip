@@ -30,7 +30,7 @@ __device__ inline float bcast_f(float v, int src_lane) {
 // Any rank: lane l holds components l + 64 t; every entry is applied by the whole wave.
 template <int VPL>
 struct GatherDword {
-  static constexpr int UNR = VPL <= 2 ? 8 : VPL <= 4 ? 4 : 2;
+  static constexpr int UNR = VPL <= 2 ? 8 : VPL <= 4 ? 4 : 2, FEW = UNR;
   float acc[VPL];
   bool ok[VPL];
   int lane;
@@ -46,6 +46,7 @@ struct GatherDword {
     }
   }
 
+  template <int U = UNR>
   __device__ inline void run(const int32_t* __restrict__ idx, const float* __restrict__ val,
                              int64_t p0, int64_t p1, const float* __restrict__ X, int r) {
     for (int64_t p = p0; p < p1; p += 64) {
@@ -57,18 +58,18 @@ struct GatherDword {
         my_v = val[p + lane];
       }
       int u = 0;
-      for (; u + UNR <= cnt; u += UNR) {
-        float h[UNR][VPL];
-        float a[UNR];
+      for (; u + U <= cnt; u += U) {
+        float h[U][VPL];
+        float a[U];
 #pragma unroll
-        for (int q = 0; q < UNR; q++) {
+        for (int q = 0; q < U; q++) {
           const float* x = X + (int64_t)bcast_i(my_i, u + q) * r + lane;
           a[q] = bcast_f(my_v, u + q);
 #pragma unroll
           for (int t = 0; t < VPL; t++) h[q][t] = ok[t] ? x[64 * t] : 0.0f;
         }
 #pragma unroll
-        for (int q = 0; q < UNR; q++)
+        for (int q = 0; q < U; q++)
 #pragma unroll
           for (int t = 0; t < VPL; t++) acc[t] = fmaf(a[q], h[q][t], acc[t]);
       }
@@ -103,6 +104,10 @@ struct GatherVec4 {
   // Steps with their loads in flight: eight loads a lane (half as many / twice: panels of 1000 x 11 M, rank 128, 524
   // -> 493 us / 505; 2000 x 20 M, rank 256, 1639 -> 1603 / 1617; 700 x 4 M, rank 512, 976 -> 815 / 865).
   static constexpr int UNR = T >= 4 ? 2 : T == 2 ? 4 : LPR >= 8 ? 8 : 4;
+  // For runs of a few entries half of that: most of a larger step is padding (A^T W of 20,000 rows, rank 384: 663 -> 583 us for
+  // 193k columns of 8 entries, 1025 -> 920 for 304k of 5, 1385 -> 1308 for 298k of 30; 6000 rows and fewer than 40k columns, where
+  // the chip is not full, are 3 to 7 % faster with the larger one).
+  static constexpr int FEW = T >= 4 ? 1 : T == 2 ? 2 : 4;
   static_assert(G * UNR <= 64, "a batch is 64 entries");
   float4 acc[T];
   bool ok[T];
@@ -121,6 +126,7 @@ struct GatherVec4 {
     }
   }
 
+  template <int U = UNR>
   __device__ inline void run(const int32_t* __restrict__ idx, const float* __restrict__ val,
                              int64_t p0, int64_t p1, const float* __restrict__ X, int r) {
     for (int64_t p = p0; p < p1; p += 64) {
@@ -135,11 +141,11 @@ struct GatherVec4 {
       // so the steps need no predicates.  Row offsets are 32-bit when X is smaller than 4 GB
       // (one multiply-add per gathered row).
       const int nsteps = (cnt + G - 1) / G;
-      for (int q = 0; q < nsteps; q += UNR) {
-        float4 h[UNR][T];
-        float a[UNR];
+      for (int q = 0; q < nsteps; q += U) {
+        float4 h[U][T];
+        float a[U];
 #pragma unroll
-        for (int uu = 0; uu < UNR; uu++) {
+        for (int uu = 0; uu < U; uu++) {
           const int u = ((q + uu) * G + grp) & 63;
           const int j = __shfl(my_i, u);
           a[uu] = __shfl(my_v, u);
@@ -151,7 +157,7 @@ struct GatherVec4 {
                                      : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         }
 #pragma unroll
-        for (int uu = 0; uu < UNR; uu++)
+        for (int uu = 0; uu < U; uu++)
 #pragma unroll
           for (int t = 0; t < T; t++) {
             acc[t].x = fmaf(a[uu], h[uu][t].x, acc[t].x);
@@ -819,7 +825,7 @@ __global__ void __launch_bounds__(256)
     GT g;
     g.init(lane, width);
     g.small = w_small;
-    g.run(rowind, tvals, p0, p1, W + slice * width, r);
+    g.template run<GT::FEW>(rowind, tvals, p0, p1, W + slice * width, r);
     g.store(T + j * r + slice * width);
   }
 }
