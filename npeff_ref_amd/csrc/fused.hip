@@ -329,15 +329,12 @@ __global__ void __launch_bounds__(256, fu_blocks(Q, R) <= 2 ? 4 : 3)
       cpv[k] = colptr[d.col0 + (at < d.nc ? at : d.nc)];
     }
   };
-  // (round by round in turn: where the long columns are the first or the last, who had a full tile gets an
-  // empty one or none)
-  auto tile_of = [&](int k) { return k * (int)gridDim.x + (k & 1 ? (int)(gridDim.x - 1 - blockIdx.x) : (int)blockIdx.x); };
   fu_tile_at td = fu_describe<Gather::NG>(tiles, n_tiles, blockIdx.x);
   request(td);
   fu_load_g<Q, R>(gw, n_gw, r, ga, tile);
 
   int par = 0;
-  for (int k = 0; tile_of(k) < n_tiles; k++, par ^= 1) {
+  for (int tl = blockIdx.x; tl < n_tiles; tl += gridDim.x, par ^= 1) {
     const int l0 = td.col0 & (TC - 1);
     const int nc = td.nc, share = td.share;
     int* cp = cps[par];
@@ -346,7 +343,7 @@ __global__ void __launch_bounds__(256, fu_blocks(Q, R) <= 2 ? 4 : 3)
       const int at = tid + 256 * k;
       if (at <= nc) cp[l0 + at] = (int)(cpv[k] - td.e0);
     }
-    const fu_tile_at nd = fu_describe<Gather::NG>(tiles, n_tiles, tile_of(k + 1));
+    const fu_tile_at nd = fu_describe<Gather::NG>(tiles, n_tiles, tl + gridDim.x);
     // the wave's rows of H
     const int64_t base = td.col0 - l0;
     float* Hb = H + base * r;
