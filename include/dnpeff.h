@@ -94,9 +94,11 @@ int dnpeff_plan_estimate(int64_t n_rows, int64_t n_cols, int64_t nnz_sparse, int
  * multiples of 128 are stored as the next multiple where that fits; 0: as they are),
  * h_overlap (1: tiled H update with A^T W of the next tile on the library stream beside the
  * update of this tile on a second stream, through two tile buffers; off by default),
- * xg_wgs (3: the update kernel of ranks from 256 with three workgroups per CU on LDS planes
- * without padding where the launch fills the CUs eight times over; 4: always; 2: two, on padded
- * planes with two operand stages),
+ * xg_wgs (the update kernel of the multiples of 128 from rank 256 on.  3: by size: tiles of 128 x 256 where
+ * the rank is a multiple of 256 and they are two rounds of two workgroups per CU (131,072 rows at rank
+ * 256), else tiles of 128 x 128, three workgroups per CU on LDS planes without padding where the launch
+ * fills the CUs eight times over, two on padded planes below.  5: tiles of 128 x 256 wherever the rank
+ * allows, else as 4; 4: tiles of 128 x 128 with three workgroups; 2: with two),
  * gram_beside (1: H^T H of the W update on a second stream with the dense head of A H^T behind
  * it; 0: after A H^T on the library stream), gram_fold (2: X^T X with
  * its diagonal squares of 256 columns each in one workgroup where the rank is a multiple of 256;
@@ -314,7 +316,10 @@ int dnpeff_nmf_set_factors(dnpeff_nmf* nmf, const float* W_nr, const float* H_rm
 
 /* n_steps iterations of: W-update, then H-update with the new W
  * (MuNmf::run loop body, multi_mu_dense_factors_nmf1.h:175-182).  Returns
- * without waiting for the device. */
+ * without waiting for the device.  Runs of at most 16 components and 128 rows that are small enough
+ * run whole in one workgroup, with their sums in another order than dnpeff_nmf_update_W and
+ * dnpeff_nmf_update_H take them: there n steps give the bits of n calls of one step, and those of the two
+ * updates only up to the rounding of fp32 sums (a few 1e-7 per step). */
 int dnpeff_nmf_step(dnpeff_nmf* nmf, int n_steps);
 
 /* W <- W * (A H^T) / (W (H H^T) + eps)   (updateW, nmf1.h:293-305). */

@@ -296,7 +296,7 @@ __device__ inline void fu_gram_out(const V& v, float* __restrict__ lds, float* _
 // end are shared by eight components; with 16 bytes the r = 50 step took 335 us, now 316), 24-bit
 // multiplies into 32-bit offsets and the corrected reciprocal in place of the division sequence
 // (390 -> 335 us with it).  777 x 862k, r = 50: 188 us for 2.0 GFLOP of gathers and 12.9 of products
-// (922 us for A^T W, update and Gram as separate kernels); 512 x 431k, r = 16: 31 us (139); 300 x 146k,
+// (922 us for A^T W, update and Gram as separate kernels); 512 x 431k, r = 16: 32 us (139); 300 x 146k,
 // r = 20: 18.4, of which a workgroup has 12 us (prologue 2.8, rows and gathers 4 to 8, products and stores 3.5).
 // ---------------------------------------------------------------------------
 template <int Q, int R, int JB, bool TOTALS, bool PAST>
@@ -628,10 +628,10 @@ __global__ void __launch_bounds__(256, 2)
   });
 }
 
-// A H^T: chunk blockIdx.x - sum_wgs of the entries, all of one row; the wave's lane groups take them
-// round-robin, FU_U gathers each in flight.  Workgroups 0 .. sum_wgs - 1 sum Gram parts instead.
-// 777 x 862k, r = 50: 117 us for 3.9 M gathered rows of 200 bytes (6.6 TB/s), half of which the L2s hold;
-// 141 us as one 4-byte load per lane.
+// A H^T: chunk blockIdx.x - sum_wgs of the entries, all of one row (XCD: a part of a row's share of an XCD's
+// columns); the wave's lane groups take them round-robin, FU_U gathers each in flight.  Workgroups 0 .. sum_wgs - 1 sum
+// Gram parts instead.  777 x 862k, r = 50, in chunks of whole rows: 117 us for 3.9 M gathered rows of 200 bytes (6.6 TB/s),
+// half of which the L2s hold; 141 us as one 4-byte load per lane; by XCD 75.
 template <int LPR, bool XCD>
 __global__ void __launch_bounds__(256)
     k_fu_n(const fu_chunk* __restrict__ chunks, const int64_t* __restrict__ x_seg, int x_parts,
