@@ -267,13 +267,24 @@ static int stored_rank(int64_t n, int64_t m, int64_t nnz, int rank, bool sweeps,
 // 3.17 / 3.50 with 12 M (0.40) but 3.17 / 2.51 with 8.3 M (0.28), 34.1 / 43.2 at 4000 x 200k (0.16), 18.7 / 20.6 at 8000 x
 // 60k (0.14), 10.4 / 10.7 at 4000 x 60k (0.14) but 5.6 / 3.4 at 3000 x 20k, 12 M (0.20), 23.0 / 21.7 at 4000 x 200k
 // (0.08), 57 / 53 at 20000 x 200k (0.04).  Below, the fused step is ahead by 1.1 to 5 from 1024 x 1100 to 100000 x
-// 4.0M (1.73 / 0.32, 3.4 / 1.3 at 1100 x 60k, 52 / 36 at 8000 x 5.7M, 145 / 107), except where few columns hold most of
-// very many entries: 113 / 128 at 40000 x 3.9M, 328 M entries by a Zipf law of 1.3, 48 / 54 at 2000 x 1M, 131 M.  It is
-// also closer to 64 bits: one W update 5e-7 ... 8e-7 off where the head's split operands leave 1e-6 ... 6e-6.
+// 4.0M (1.73 / 0.32, 3.4 / 1.3 at 1100 x 60k, 52 / 36 at 8000 x 5.7M, 145 / 107), unless few columns hold most of very many
+// entries (head_beats_fused).  It is also closer to 64 bits: one W update 5e-7 ... 8e-7 off where the head's split operands
+// leave 1e-6 ... 6e-6.
 static bool fused_step_wanted(int64_t n, int64_t m, int64_t nnz, int rank) {
   if (tuning().fused_gram == 0.0 || tuning().tiled_h > 0.0 || !fused_supported(n, m, nnz, rank)) return false;
   if (n < 1024 || rank % 64 != 0) return true;
   return rank == 64 && 9.0 * ((double)nnz - 6e6) <= (double)n * (double)m;
+}
+
+// Rank 64, a head of z_head entries on the columns that a sixteenth of the rows hold: it pays for its launches and the passes
+// over H that the fused step does without (27 M entries and 7 to a column), and for the rest of the matrix, which its kernels
+// take at half the speed.  Of 313 matrices of 16 to 330 M entries (1030 to 70,000 rows, Zipf laws of 1.05 to 1.6) the choice
+// is 0.7 % from the faster way on average and 1.22 at most; by the rule for dense matrices alone 4.8 % and 1.61.  Five
+// iterations with head / fused: 36.3 / 45.0 ms at 40,000 x 1.8M with 262 M entries, exponent 1.6, 39.3 / 50.7 at 2000 x 3.9M with
+// 262 M, 1.3, 8.0 / 11.5 at 40,000 x 50k with 66 M, 1.6, 8.8 / 10.4 at 12,000 x 165k; past the line 13.4 / 11.4 at 12,000 x 1.1M with
+// 66 M, 1.6, 10.5 / 10.5 at 12,000 x 165k, 1.3, 24.5 / 23.5 at 40,000 x 1.0M with 131 M, 1.3, 27.2 / 24.2 at 5000 x 786k, 1.05.
+static bool head_beats_fused(int64_t m, int64_t nnz, int64_t z_head) {
+  return (double)z_head > 27e6 + (double)(nnz - z_head) + 7.0 * (double)m;
 }
 
 // Whether it does within `budget` bytes beside the factors, and whether with lists by XCD.
@@ -349,6 +360,14 @@ static int plan_matrix(dnpeff_csr* A, int rank, int asked, bool consume, bool* t
   const double budget_full = avail - t_full.total();
   const double budget_tiled = avail - t_tiled.total();
   *fused = choose_fused(A->n_rows, A->n_cols, A->nnz, rank, budget_full);
+  head_choice c;
+  bool chosen = false;
+  if (fused->on && rank == 64 && A->n_rows >= 1024 && !A->tail && has_row_major(A) && tn.dense_fill <= 1.0 &&
+      head_beats_fused(A->n_cols, A->nnz, A->nnz)) {
+    DN_TRY(choose_dense_head(A, tn.dense_fill, budget_full, head_blocks_for_rank(rank), rank, head_run(rank, asked), &c));
+    chosen = c.thr > 0 && c.fits && head_beats_fused(A->n_cols, A->nnz, c.z_head);
+    if (chosen) *fused = fused_choice();
+  }
   const bool can_split = rank % 4 == 0 && rank >= 64 && A->n_rows >= 1024 && !fused->on;
   double fill = tn.dense_fill;
   if (fill > 1.0) fill = 0.0;
@@ -368,9 +387,8 @@ static int plan_matrix(dnpeff_csr* A, int rank, int asked, bool consume, bool* t
     if (tn.tiled_h < 0.0) *tiled = 16.0 * (double)A->nnz > budget_full;
     return 0;
   }
-  head_choice c;
   const int n_blocks = head_blocks_for_rank(rank);
-  DN_TRY(choose_dense_head(A, fill, *tiled ? budget_tiled : budget_full, n_blocks, rank, head_run(rank, asked), &c));
+  if (!chosen) DN_TRY(choose_dense_head(A, fill, *tiled ? budget_tiled : budget_full, n_blocks, rank, head_run(rank, asked), &c));
   if (!c.fits && tn.tiled_h < 0.0 && !*tiled) {
     *tiled = true;
     DN_TRY(choose_dense_head(A, fill, budget_tiled, n_blocks, rank, head_run(rank, asked), &c));

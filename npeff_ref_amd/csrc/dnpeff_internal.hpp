@@ -462,6 +462,7 @@ bool use_tlists(const dnpeff_csr* S, int r);
 struct head_choice {
   int64_t thr = 0;   // columns with at least thr entries form the head (0 = no head)
   int64_t n_d = 0;
+  int64_t z_head = 0;      // their entries
   double footprint = 0.0;  // bytes of the dense blocks + both sparse copies of the rest
   bool fits = true;        // footprint within the budget given
 };

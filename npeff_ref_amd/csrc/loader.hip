@@ -1532,6 +1532,7 @@ int choose_dense_head(dnpeff_csr* A, double min_fill, double budget, int n_block
     head_choice c;
     c.thr = thr;
     c.n_d = n_d;
+    c.z_head = (int64_t)z_head;
     c.footprint = blocks + 16.0 * (double)(A->nnz - (int64_t)z_head) +
                   (rank > 0 ? 4.0 * (double)head_workspace_floats(n, n_d, rank, t_run) : 0.0);
     c.fits = c.footprint <= budget;

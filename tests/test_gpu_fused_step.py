@@ -347,3 +347,31 @@ def test_rank_64_with_many_rows(m, k, fused):
     _close(nmf, orc.nmf_f64(rp, ci, va, m, W0, H0, np.float32(EPS), 2, 2))
     nmf.close()
     A.close()
+
+
+@pytest.mark.parametrize("zipf,head", [(1.6, True), (1.05, False)])
+def test_rank_64_with_a_head_of_very_many_entries(zipf, head, tune):
+    """66 M entries on 49,500 columns: a dense head where its columns hold 27 M more than the others and 7 to every column
+    (52 M of them by a steep law), else the fused step (40 M).  Either way one step is the same to rounding."""
+    n, k = 40_000, 1650
+    A, norms = d.Csr.synth(n, 30 * k, k_fixed=k, zipf_s=zipf, seed=1)
+    A.normalize_rows(norms)
+    A.compact_columns(1)
+
+    def run():
+        nmf = d.MuNmf(A, d.MuNmfParams(rank=64, max_iters=1, eps=EPS, seed=3, log_every=1))
+        nmf.initialize()
+        nd = A.head_info()[0]
+        nmf.step(1)
+        W = nmf.loadWToHostSync()
+        nmf.close()
+        return nd, W
+
+    nd, W = run()
+    assert (nd > 0) == head
+    A.split_dense_head(0.0)
+    tune("dense_fill", 0)
+    nd, W0 = run()
+    assert nd == 0
+    assert np.linalg.norm(W - W0) <= 1e-5 * np.linalg.norm(W0)
+    A.close()
