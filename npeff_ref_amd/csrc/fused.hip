@@ -298,6 +298,11 @@ __device__ inline void fu_gram_out(const V& v, float* __restrict__ lds, float* _
 // (390 -> 335 us with it).  777 x 862k, r = 50: 188 us for 2.0 GFLOP of gathers and 12.9 of products
 // (922 us for A^T W, update and Gram as separate kernels); 512 x 431k, r = 16: 32 us (139); 300 x 146k,
 // r = 20: 18.4, of which a workgroup has 12 us (prologue 2.8, rows and gathers 4 to 8, products and stores 3.5).
+//
+// Which shares left a carry for a column (fu_cut_by) one thread per column finds before the entries are gathered, not every
+// lane that updates a part of it: two quotients a lane were up to a tenth of the vector instructions (ten iterations at
+// 512 x 431k, r = 16: 567 -> 558 us, 777 x 862k, r = 50: 2805 -> 2786, a job at 300 x 146k, r = 20: 4.33 -> 4.21 ms.  At
+// ranks above 64 the kernel has no two registers for it: 27.4 -> 27.6 ms at 1000 x 3.4M, r = 128).
 // ---------------------------------------------------------------------------
 template <int Q, int R, int JB, bool TOTALS, bool PAST>
 __global__ void __launch_bounds__(256, fu_blocks(Q, R) <= 2 ? 4 : 3)
@@ -310,7 +315,8 @@ __global__ void __launch_bounds__(256, fu_blocks(Q, R) <= 2 ? 4 : 3)
   constexpr int ROOM = Gather::CARRY + 2048, T_OUT = fu_out_floats<NP, Out>(ROOM), T_FLOATS = ROOM > T_OUT ? ROOM : T_OUT;
   __shared__ __align__(16) float ga[NB * NB * 256];
   __shared__ __align__(16) float tile[T_FLOATS];
-  __shared__ int cps[2][TC + 1];
+  // Of the tile's columns: the first share that left a carry and, above 16 bits, the one past the last; -1 without entries.
+  __shared__ int cut[2][TC];
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int l16 = lane & 15, g = lane >> 4;
   double sum[TOTALS ? NP : 1][4] = {};
@@ -320,14 +326,13 @@ __global__ void __launch_bounds__(256, fu_blocks(Q, R) <= 2 ? 4 : 3)
   const char* Wb = reinterpret_cast<const char*>(W);
   Gather gather;
   gather.init(r);
-  int64_t cpv[JB];
+  static_assert(TC <= 256, "a thread per column");
+  int64_t cp0, cp1;  // entries of column tid of the tile
   auto request = [&](const fu_tile_at& d) {
     gather.request(pairs, d);
-#pragma unroll
-    for (int k = 0; k < JB; k++) {
-      const int at = tid + 256 * k;
-      cpv[k] = colptr[d.col0 + (at < d.nc ? at : d.nc)];
-    }
+    const int64_t* at = colptr + d.col0 + (tid < d.nc ? tid : 0);
+    cp0 = at[0];
+    cp1 = at[1];
   };
   fu_tile_at td = fu_describe<Gather::NG>(tiles, n_tiles, blockIdx.x);
   request(td);
@@ -336,12 +341,12 @@ __global__ void __launch_bounds__(256, fu_blocks(Q, R) <= 2 ? 4 : 3)
   int par = 0;
   for (int tl = blockIdx.x; tl < n_tiles; tl += gridDim.x, par ^= 1) {
     const int l0 = td.col0 & (TC - 1);
-    const int nc = td.nc, share = td.share;
-    int* cp = cps[par];
-#pragma unroll
-    for (int k = 0; k < JB; k++) {
-      const int at = tid + 256 * k;
-      if (at <= nc) cp[l0 + at] = (int)(cpv[k] - td.e0);
+    const int nc = td.nc;
+    if (tid < nc) {
+      const int a0 = (int)(cp0 - td.e0), a1 = (int)(cp1 - td.e0);
+      int k0 = 0, k1 = -1;
+      if (a1 > a0) fu_cut_by(a0, a1, td.share, 1.0f / (float)td.share, k0, k1);
+      cut[par][l0 + tid] = k0 | (int)((unsigned)k1 << 16);
     }
     const fu_tile_at nd = fu_describe<Gather::NG>(tiles, n_tiles, tl + gridDim.x);
     // the wave's rows of H
@@ -362,15 +367,14 @@ __global__ void __launch_bounds__(256, fu_blocks(Q, R) <= 2 ? 4 : 3)
     request(nd);
     __syncthreads();
 
-    const float inv = 1.0f / (float)(share > 0 ? share : 1);
 #pragma unroll
     for (int jb = 0; jb < JB; jb++) {
       const int first = 16 * (JB * wave + jb);
       if (first + 15 < l0 || first >= l0 + nc) continue;
       f32x4 t[NB];
       float* trow = tile + (first + l16) * TS;
-      const int a0 = mine[jb] ? cp[first + l16] : 0, a1 = mine[jb] ? cp[first + l16 + 1] : 0;
-      const bool some = a1 > a0;
+      const int parts = mine[jb] ? cut[par][first + l16] : -1;
+      const bool some = parts >= 0;
 #pragma unroll
       for (int b = 0; b < Q; b++) t[b] = *reinterpret_cast<const f32x4*>(trow + 16 * b + 4 * g);
       if constexpr (R > 0) {
@@ -382,8 +386,7 @@ __global__ void __launch_bounds__(256, fu_blocks(Q, R) <= 2 ? 4 : 3)
 #pragma unroll
         for (int i = 0; i < 4; i++) t[b][i] = some ? t[b][i] : 0.0f;
       if (some) {
-        int k0, k1;
-        fu_cut_by(a0, a1, share, inv, k0, k1);
+        const int k0 = parts & 0xffff, k1 = parts >> 16;
         auto add = [&](int k, f32x4 (&to)[NB]) {
           const float* src = tile + Gather::CARRY + k * (2048 / Gather::NG);
 #pragma unroll
