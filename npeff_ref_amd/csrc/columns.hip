@@ -264,7 +264,6 @@ static int mark_columns(const int32_t* colind, int64_t nnz, int64_t n_cols, int6
   hipLaunchKernelGGL(k_merge_marks<TWO>, dim3((unsigned)ceil_div(n_words, 256)), dim3(256), 0, st, marks.p, (int)parts,
                      (int)words, n_words, mask);
   DN_LAUNCH_CHECK();
-  DN_HIP(hipStreamSynchronize(st));
   return 0;
 }
 
@@ -289,7 +288,6 @@ int column_mask_of_counts(const int32_t* colind, int64_t nnz, int64_t n_cols, in
   hipLaunchKernelGGL(k_mask_of_counts, dim3((unsigned)ceil_div(n_words, 256)), dim3(256), 0, stream(), count.p, min_count,
                      n_cols, n_words, mask);
   DN_LAUNCH_CHECK();
-  DN_HIP(hipStreamSynchronize(stream()));
   return 0;
 }
 
@@ -309,17 +307,18 @@ int keep_columns(dnpeff_csr* A, const uint32_t* mask, int32_t** new_to_og) {
   dbuf<int> kept;
   dbuf<int64_t> base;
   DN_TRY(rank.alloc(n_words + 1));
-  DN_TRY(exclusive_scan(MaskBitsF{mask}, n_words, rank.p));
+  unsigned long long* host = nullptr;
+  DN_TRY(host_words(&host));
+  int64_t* totals = reinterpret_cast<int64_t*>(host);
+  DN_TRY(exclusive_scan(MaskBitsF{mask}, n_words, rank.p, totals));
   DN_TRY(kept.alloc(tiles));
   DN_TRY(base.alloc(tiles + 1));
   if (tiles)
     hipLaunchKernelGGL(k_kept_count, dim3((unsigned)tiles), dim3(256), 0, st, A->colind, nnz, mask, kept.p);
   DN_LAUNCH_CHECK();
-  DN_TRY(exclusive_scan(TileCountF{kept}, tiles, base.p));
-  int32_t n_cols = 0;
-  int64_t n_kept = 0;
-  DN_HIP(copy_down(&n_cols, rank + n_words, sizeof(int32_t)));
-  DN_HIP(copy_down(&n_kept, base + tiles, sizeof(int64_t)));
+  DN_TRY(exclusive_scan(TileCountF{kept}, tiles, base.p, totals + 1));
+  DN_HIP(hipStreamSynchronize(st));
+  const int64_t n_cols = totals[0], n_kept = totals[1];
   if (new_to_og) {
     DN_TRY(list.alloc(n_cols));
     if (n_words)
@@ -333,7 +332,6 @@ int keep_columns(dnpeff_csr* A, const uint32_t* mask, int32_t** new_to_og) {
       hipLaunchKernelGGL(k_kept_renumber, dim3((unsigned)g), dim3(256), 0, st, A->colind, nnz, mask, rank.p);
       DN_LAUNCH_CHECK();
     }
-    DN_HIP(hipStreamSynchronize(st));
   } else {
     dbuf<int32_t> out_col;
     dbuf<float> out_val;
@@ -344,7 +342,6 @@ int keep_columns(dnpeff_csr* A, const uint32_t* mask, int32_t** new_to_og) {
     hipLaunchKernelGGL(k_kept_move, dim3((unsigned)tiles), dim3(256), 0, st, A->colind, A->vals, nnz, mask, rank.p, base.p,
                        A->rowptr, A->n_rows, out_col.p, out_val.p, out_rowptr.p);
     DN_LAUNCH_CHECK();
-    DN_HIP(hipStreamSynchronize(st));
     dfree(A->colind);
     dfree(A->vals);
     dfree(A->rowptr);

@@ -123,16 +123,17 @@ int column_mask_of_list(const int32_t* kept_ascending, int64_t n_kept, int64_t n
 int keep_columns(dnpeff_csr* A, const uint32_t* mask, int32_t** new_to_og);
 
 // ---- scans (loader.hip) ----
+// (none waits for the stream; total, or NULL: a pinned word (host_words) for the last element of `out`)
 // out[i] = sum_{i' < i} (count[i'] >= min_count), i in [0, n]; out has n+1 entries.
 int scan_keep_mask(const int* count, int min_count, int64_t n, int32_t* out);
 // out[i] = sum_{i' < i} count[i'], i in [0, n].
-int scan_counts_i64(const int* count, int64_t n, int64_t* out);
+int scan_counts_i64(const int* count, int64_t n, int64_t* out, int64_t* total = nullptr);
 // out[e] = number of kept entries before e (table[colind[e]] != -1), e in [0, nnz].
 int scan_kept_entries(const int32_t* colind, const int32_t* table, int64_t nnz, int64_t* out);
 // out[i] = sum_{i' < i} ceil(len_i' / chunk), i in [0, n].
-int scan_row_chunks(const int64_t* rowptr, int64_t chunk, int64_t n, int64_t* out);
+int scan_row_chunks(const int64_t* rowptr, int64_t chunk, int64_t n, int64_t* out, int64_t* total = nullptr);
 // out[j] = number of columns j' < j longer than `limit`, j in [0, n].
-int scan_long_cols(const int64_t* colptr, int64_t limit, int64_t n, int32_t* out);
+int scan_long_cols(const int64_t* colptr, int64_t limit, int64_t n, int32_t* out, int64_t* total = nullptr);
 
 // ---- dense kernels (dense.hip) ----
 int launch_mu(int64_t count, float* F, const float* num, const float* den, float eps);

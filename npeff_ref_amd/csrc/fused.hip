@@ -905,15 +905,17 @@ static int fused_tiles_make(dnpeff_csr* S, int tc, int64_t most, int64_t alone, 
     const dim3 grid((unsigned)ceil_div(groups, 256)), block(256);
     hipLaunchKernelGGL(k_fu_count_tiles, grid, block, 0, st, S->colptr, m, tc, most, alone, groups, count.p);
     DN_LAUNCH_CHECK();
-    DN_TRY(scan_counts_i64(count, groups, first));
-    int64_t n_tiles = 0;
+    unsigned long long* host = nullptr;
+    DN_TRY(host_words(&host));
+    int64_t* total = reinterpret_cast<int64_t*>(host);
+    DN_TRY(scan_counts_i64(count, groups, first, total));
     f.h_first.clear();
     if (with_first) {
       f.h_first.resize((size_t)groups + 1);
       DN_HIP(copy_down(f.h_first.data(), first, sizeof(int64_t) * f.h_first.size()));
     }
-    DN_HIP(copy_down(&n_tiles, first + groups, sizeof(int64_t)));
     DN_HIP(hipStreamSynchronize(st));
+    const int64_t n_tiles = *total;
     dfree(f.tiles);
     f.tiles = nullptr;
     DN_TRY(dmalloc(&f.tiles, n_tiles + 1));
@@ -1136,9 +1138,12 @@ int fused_plan_build(dnpeff_csr* S, int r, bool xcd) {
     const int64_t chunk = fu_chunk_entries(S->nnz);
     dbuf<int64_t> base;
     DN_TRY(base.alloc(S->n_rows + 1));
-    DN_TRY(scan_row_chunks(S->rowptr, chunk, S->n_rows, base));
-    DN_HIP(copy_down(&f.n_chunks, base + S->n_rows, sizeof(int64_t)));
+    unsigned long long* host = nullptr;
+    DN_TRY(host_words(&host));
+    int64_t* total = reinterpret_cast<int64_t*>(host);
+    DN_TRY(scan_row_chunks(S->rowptr, chunk, S->n_rows, base, total));
     DN_HIP(hipStreamSynchronize(st));
+    f.n_chunks = *total;
     DN_TRY(dmalloc(&f.chunks, f.n_chunks));
     DN_TRY(dmalloc(&f.n_base, S->n_rows + 1));
     hipLaunchKernelGGL(k_fu_make_chunks, dim3((unsigned)ceil_div(S->n_rows + 1, 256)), dim3(256), 0, st, S->rowptr,

@@ -203,17 +203,17 @@ struct LongColF {
 int scan_keep_mask(const int* count, int min_count, int64_t n, int32_t* out) {
   return exclusive_scan(KeepMaskF{count, min_count}, n, out);
 }
-int scan_counts_i64(const int* count, int64_t n, int64_t* out) {
-  return exclusive_scan(CountsF{count}, n, out);
+int scan_counts_i64(const int* count, int64_t n, int64_t* out, int64_t* total) {
+  return exclusive_scan(CountsF{count}, n, out, total);
 }
 int scan_kept_entries(const int32_t* colind, const int32_t* table, int64_t nnz, int64_t* out) {
   return exclusive_scan(KeptEntryF{colind, table}, nnz, out);
 }
-int scan_row_chunks(const int64_t* rowptr, int64_t chunk, int64_t n, int64_t* out) {
-  return exclusive_scan(RowChunksF{rowptr, chunk}, n, out);
+int scan_row_chunks(const int64_t* rowptr, int64_t chunk, int64_t n, int64_t* out, int64_t* total) {
+  return exclusive_scan(RowChunksF{rowptr, chunk}, n, out, total);
 }
-int scan_long_cols(const int64_t* colptr, int64_t limit, int64_t n, int32_t* out) {
-  return exclusive_scan(LongColF{colptr, limit}, n, out);
+int scan_long_cols(const int64_t* colptr, int64_t limit, int64_t n, int32_t* out, int64_t* total) {
+  return exclusive_scan(LongColF{colptr, limit}, n, out, total);
 }
 
 // ---------------------------------------------------------------------------
@@ -601,12 +601,12 @@ __global__ void __launch_bounds__(256)
 // [column][words].
 __global__ void __launch_bounds__(256)
     k_bits_set(const int64_t* __restrict__ rowptr, const int32_t* __restrict__ colind, int64_t n_rows, int words,
-               uint32_t* __restrict__ bits, int* __restrict__ repeats) {
+               uint32_t* __restrict__ bits) {
   for (int64_t row = blockIdx.y; row < n_rows; row += gridDim.y) {
     const int64_t e1 = rowptr[row + 1];
     const uint32_t bit = 1u << (row & 31);
     for (int64_t e = rowptr[row] + (int64_t)blockIdx.x * 256 + threadIdx.x; e < e1; e += (int64_t)gridDim.x * 256)
-      if (atomicOr(&bits[(int64_t)colind[e] * words + (row >> 5)], bit) & bit) *repeats = 1;
+      atomicOr(&bits[(int64_t)colind[e] * words + (row >> 5)], bit);
   }
 }
 
@@ -835,7 +835,6 @@ int csr_set_panels(dnpeff_csr* S, const panel_plan& plan) {
     hipLaunchKernelGGL(k_panel_bounds, dim3((unsigned)ceil_div(P0 + 1, 256)), dim3(256), 0, st,
                        S->colptr, S->n_cols, S->nnz, P0, d_coarse);
     hipError_t e = hipGetLastError();
-    if (e == hipSuccess) e = hipStreamSynchronize(st);
     if (e == hipSuccess)
       e = copy_down(coarse.data(), d_coarse, sizeof(int32_t) * coarse.size());
     dfree(d_coarse);
@@ -911,7 +910,6 @@ int csr_set_panels(dnpeff_csr* S, const panel_plan& plan) {
                          S->rowptr, S->colind, S->vals, S->n_rows, P, bits, S->panel_bounds, S->seg,
                          S->pcol, S->pval, (const int64_t*)S->prow);
       e = hipGetLastError();
-      if (e == hipSuccess) e = hipStreamSynchronize(st);
     }
     if (e != hipSuccess) {
       set_error("building the column panels failed: %s", hipGetErrorString(e));
@@ -1321,7 +1319,6 @@ DN_API int dnpeff_csr_from_pef(int64_t n_rows, int64_t k, int64_t dense_fisher_s
   hipError_t e = hipGetLastError();
   if (e == hipSuccess && nnz)
     e = copy_up_parts({{A->colind, indices, sizeof(int32_t) * nnz}, {A->vals, values, sizeof(float) * nnz}});
-  if (e == hipSuccess) e = hipStreamSynchronize(stream());
   if (e != hipSuccess) {
     set_error("upload of the PEF arrays failed: %s", hipGetErrorString(e));
     dnpeff_csr_destroy(A);
@@ -1344,7 +1341,6 @@ DN_API int dnpeff_csr_normalize_rows(dnpeff_csr* A, const float* norms_host, flo
   hipLaunchKernelGGL(k_normalize_rows, dim3(grid), dim3(256), 0, stream(), A->rowptr, A->vals,
                      norms, eps, A->n_rows);
   DN_LAUNCH_CHECK();
-  DN_HIP(hipStreamSynchronize(stream()));
   dfree(norms);
   drop_derived(A);
   A->sq_norm_valid = false;
@@ -1718,21 +1714,20 @@ static int transpose_by_bits(const dnpeff_csr* A, int* count, int64_t* colptr, i
   DN_TRY(bits.alloc(m * words));
   unsigned long long* host = nullptr;
   DN_TRY(host_words(&host));
-  int* repeats = reinterpret_cast<int*>(host);
-  *repeats = 0;
+  int64_t* total = reinterpret_cast<int64_t*>(host);
   DN_HIP(hipMemsetAsync(bits, 0, sizeof(uint32_t) * (size_t)(m * words), st));
   const int64_t per_row = std::min<int64_t>(64, std::max<int64_t>(1, ceil_div(ceil_div(A->nnz, n), 1024)));
   const dim3 grid((unsigned)per_row, (unsigned)n), block(256);
-  hipLaunchKernelGGL(k_bits_set, grid, block, 0, st, A->rowptr, A->colind, n, words, bits.p, repeats);
+  hipLaunchKernelGGL(k_bits_set, grid, block, 0, st, A->rowptr, A->colind, n, words, bits.p);
   hipLaunchKernelGGL(k_bits_count, dim3(grid_for(m)), block, 0, st, bits.p, words, m, count);
   DN_LAUNCH_CHECK();
-  DN_TRY(scan_counts_i64(count, m, colptr));  // (ends with the stream idle)
-  *done = *repeats == 0;
+  DN_TRY(scan_counts_i64(count, m, colptr, total));
+  DN_HIP(hipStreamSynchronize(st));
+  *done = *total == A->nnz;  // (an entry that repeats sets no bit of its own)
   if (!*done) return 0;
   hipLaunchKernelGGL(k_bits_place, grid, block, 0, st, A->rowptr, A->colind, A->vals, n, bits.p, words, colptr, rowind,
                      tvals);
   DN_LAUNCH_CHECK();
-  DN_HIP(hipStreamSynchronize(st));
   return 0;
 }
 
@@ -1788,16 +1783,18 @@ DN_API int dnpeff_csr_build_transpose(dnpeff_csr* A) {
   count.reset();
   // list of long columns for A^T W
   DN_TRY(pos.alloc(m + 1));
-  DN_TRY(scan_long_cols(colptr, SPMM_T_LONG, m, pos));
-  int32_t n_long = 0;
-  DN_HIP(copy_down(&n_long, pos + m, sizeof(int32_t)));
-  DN_TRY(long_cols.alloc((int64_t)n_long));
+  unsigned long long* host = nullptr;
+  DN_TRY(host_words(&host));
+  int64_t* total = reinterpret_cast<int64_t*>(host);
+  DN_TRY(scan_long_cols(colptr, SPMM_T_LONG, m, pos, total));
+  DN_HIP(hipStreamSynchronize(st));
+  const int64_t n_long = *total;
+  DN_TRY(long_cols.alloc(n_long));
   if (n_long) {
     hipLaunchKernelGGL(k_collect_long, dim3(grid_for(m)), dim3(256), 0, st, colptr.p, SPMM_T_LONG, m,
                        pos.p, long_cols.p);
     DN_LAUNCH_CHECK();
   }
-  DN_HIP(hipStreamSynchronize(st));
   A->colptr = colptr.release();
   A->rowind = rowind.release();
   A->tvals = tvals.release();
