@@ -166,6 +166,38 @@ def test_infinite_entry_stays_infinite(r):
         A.close()
 
 
+@pytest.mark.parametrize("r,m", [(8, 140_000), (20, 70_000), (40, 40_000), (90, 20_000)])
+def test_tiles_cut_where_lanes_and_groups_meet(r, m):
+    """Columns that fill a tile by themselves, nearly or exactly, right before and after the columns at which a wave's lanes
+    and the groups of columns end; empty ones beside them.  (Sums of up to n + r non-negative terms, a quotient and a product:
+    as many roundings of 2^-24 and four.)"""
+    n = 500
+    rng = np.random.default_rng(r)
+    length = np.ones(m, dtype=np.int64)
+    for edge in (64, 128, 192, 256, 320, 512, 1024, m):
+        at = np.arange(edge - 4, min(edge + 4, m))
+        length[at] = rng.choice([0, 1, 16, 255, 256, n], size=len(at))
+    length[700:900] = 33  # (many cuts in one group)
+    cols = np.repeat(np.arange(m), length)
+    rows = np.concatenate([rng.choice(n, size=k, replace=False) if k > 1 else [j % n] * k for j, k in enumerate(length)]).astype(np.int64)
+    order = np.argsort(rows, kind="stable")
+    rows, cols = rows[order], cols[order].astype(np.int32)
+    vals = rng.random(len(rows), dtype=np.float32) + np.float32(0.5)
+    rp = np.concatenate([[0], np.cumsum(np.bincount(rows, minlength=n))]).astype(np.int64)
+    A = d.Csr.from_host(rp, cols, vals, m)
+    nmf = d.MuNmf(A, d.MuNmfParams(rank=r, max_iters=1, eps=EPS, seed=5, log_every=0))
+    nmf.initialize()
+    W, H = nmf.loadWToHostSync().astype(np.float64), nmf.loadHToHostSync().astype(np.float64)
+    T = np.stack([np.bincount(cols, weights=vals * W[rows, c], minlength=m) for c in range(r)])
+    want = H * T / (W.T @ W @ H + EPS)
+    nmf.update_H()
+    got = nmf.loadHToHostSync()
+    assert np.abs(got - want).max(axis=0)[length == 0].max(initial=0.0) == 0.0
+    assert (np.abs(got - want) <= (n + r + 4) * 2.0 ** -24 * want).all()
+    nmf.close()
+    A.close()
+
+
 def test_contexts_of_several_ranks_in_turn():
     """Contexts on one matrix whose ranks cut its columns into different tiles (64 to 256 columns each, 32, 32 with
     the long ones alone) and one without: each goes on where it was, bit for bit as by itself."""
