@@ -1182,7 +1182,7 @@ __global__ void __launch_bounds__(256)
 // columns, some 65,536 (2 MB of slots) apart, a wave takes one row's part of a cut, and all rows of a cut
 // run on one XCD (workgroups are dealt to the XCDs round-robin) side by side, so that the slots they share stay
 // in its L2.  Only components from the row's own up are added, its own in a register (every lane meets
-// there).  256 rows of 220 k entries, 22M columns: 0.63 ms with 14 M misses (1.07 with 61 M when the rows ran
+// there).  256 rows of 220 k entries, 22M columns: 0.56 ms with 14 M misses (1.07 with 61 M when the rows ran
 // side by side in chunks of equal length on all XCDs, which is what `across` still does for rows in
 // another order or of uneven parts); what is left is the L2s' line rate and the rest of long columns.
 // ---------------------------------------------------------------------------
@@ -1325,14 +1325,29 @@ __global__ void __launch_bounds__(256)
     j = colind[at];
     a = vals[at];
   };
+  // CUTS, where the L2s hold the slots and their line rate is the bound: two lanes ask for a slot together, half each,
+  // first the even one's and then the odd one's, and change halves when they are there.  (Half the lines per instruction:
+  // H H^T 618 -> 559 us; A H^T, whose slots are not in the L2s, 882 -> 922.)
+  const bool odd = lane & 1;
+  auto ask = [&](int32_t j, uint4& p, uint4& q) {
+    const int32_t je = CUTS ? __builtin_amdgcn_mov_dpp(j, 0xa0, 0xf, 0xf, true) : j;
+    const int32_t jo = CUTS ? __builtin_amdgcn_mov_dpp(j, 0xf5, 0xf, 0xf, true) : j;
+    p = slots[2 * (int64_t)je + (CUTS && odd)];
+    q = slots[2 * (int64_t)jo + (!CUTS || odd)];
+  };
+  auto change = [&](const uint4& p, const uint4& q, uint4& lo, uint4& hi) {
+    auto other = [](unsigned x) { return (unsigned)__builtin_amdgcn_mov_dpp((int)x, 0xb1, 0xf, 0xf, true); };
+    const uint4 op = {other(p.x), other(p.y), other(p.z), other(p.w)}, oq = {other(q.x), other(q.y), other(q.z), other(q.w)};
+    lo = odd ? oq : p;
+    hi = odd ? q : op;
+  };
   int32_t j0 = 0, j1 = 0, j2 = 0;
   float a0 = 0.0f, a1 = 0.0f, a2 = 0.0f;
-  uint4 s0 = {}, s1 = {}, t0, t1;
+  uint4 p0 = {}, p1 = {}, t0, t1;
   if (w0 < e1) {
     pair(w0, j0, a0);
     pair(w0 + step, j1, a1);
-    s0 = slots[2 * (int64_t)j0];
-    s1 = slots[2 * (int64_t)j0 + 1];
+    ask(j0, p0, p1);
   }
   double own = 0.0;  // (CUTS) the row with itself
   auto add = [&](int c, float v) {
@@ -1340,9 +1355,10 @@ __global__ void __launch_bounds__(256)
     else if (c == (int)row) own += (double)v;
   };
   for (int64_t e = w0; e < e1; e += step) {
-    t0 = slots[2 * (int64_t)j1];
-    t1 = slots[2 * (int64_t)j1 + 1];
+    ask(j1, t0, t1);
     pair(e + 2 * step, j2, a2);
+    uint4 s0 = p0, s1 = p1;
+    if constexpr (CUTS) change(p0, p1, s0, s1);
     const uint64_t ids = ((uint64_t)s0.w << 32) | s0.z;
     const int len = e + lane < e1 ? (int)(ids & 15u) : 0;
     const unsigned v[SPSP_PAIRS] = {s0.x, s0.y, s1.x, s1.y, s1.z, s1.w};
@@ -1353,7 +1369,7 @@ __global__ void __launch_bounds__(256)
       const int64_t q1 = b_colptr[(int64_t)j0 + 1];
       for (int64_t q = b_colptr[j0] + SPSP_PAIRS; q < q1; q++) add(b_comp[q], a0 * b_vals[q]);
     }
-    j0 = j1; a0 = a1; s0 = t0; s1 = t1;
+    j0 = j1; a0 = a1; p0 = t0; p1 = t1;
     j1 = j2; a1 = a2;
   }
   if (CUTS) {
