@@ -1037,11 +1037,7 @@ DN_API int dnpeff_fit_create(dnpeff_csr* A, dnpeff_csr* H, float eps, int64_t se
           dmalloc(&f->WHH, nr) || dmalloc(&f->dot_ws, dots);
   if (!s && !f->in_place) s = dmalloc(&f->W2, nr) || dmalloc(&f->tmp, nr);
   if (!s) s = spsp_first_stage(A, H, f->HH, f->AH);
-  if (!s) s = dnpeff_csr_sq_norm(A, &f->sq_norm_A);
-  if (!s && hipStreamSynchronize(stream()) != hipSuccess) {
-    set_error("first stage kernels failed");
-    s = 1;
-  }
+  if (!s) s = dnpeff_csr_sq_norm(A, &f->sq_norm_A);  // (the first stage is not waited for: the steps follow it on the stream)
   if (s) { dnpeff_fit_destroy(f); return s; }
   *out = f;
   return 0;
