@@ -1217,7 +1217,7 @@ __global__ void __launch_bounds__(256)
   bool bad = false;
   for (int64_t e = e0 + 1 + 256 * (int64_t)blockIdx.y + threadIdx.x; e < e1; e += 256 * (int64_t)gridDim.y)
     bad = bad || colind[e - 1] >= colind[e];
-  if (bad) atomicOr(uneven, 1);
+  if (__any(bad) && (threadIdx.x & 63) == 0) *uneven = 1;  // (an atomic of every lane: 1.5 ms at 65 M entries)
 }
 
 // at[row (cuts + 1) + p] = first entry of the row in cut p, which starts at the column that has p / cuts of all
