@@ -471,6 +471,13 @@ int dnpeff_op_spmm_t_tile(dnpeff_csr* A, int r, const float* W_nr, int64_t col0,
 int dnpeff_op_threshold_compact(int64_t count, const float* x, float divisor, float threshold,
                                 int32_t* idx_out, float* val_out, int64_t* n_kept);
 
+/* The same for results that go to the host: dnpeff_threshold_find tells their number,
+ * dnpeff_threshold_take copies them to two host arrays of that many elements and frees what *found
+ * holds (both arrays NULL: they are not wanted).  Every successful find needs one take. */
+int dnpeff_threshold_find(int64_t count, const float* x, float divisor, float threshold,
+                          int64_t* n_kept, void** found);
+int dnpeff_threshold_take(void* found, int32_t* idx_host, float* val_host);
+
 /* Per-example top-k of dense rows x[n_rows, count] (device): vals_out / idx_out [n_rows, k] get
  * the k largest entries of each row in descending order, equal values in ascending index
  * order, norms_out [n_rows] (may be NULL) the L2 norm of the whole row (sum of squares in

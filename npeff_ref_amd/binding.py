@@ -71,6 +71,8 @@ SIGNATURES = {
     "dnpeff_csr_build_transpose": (C.c_int, [_p]),
     "dnpeff_topk_rows": (C.c_int, [C.c_int64, C.c_int64, C.c_int64, _p, _p, _p, _p]),
     "dnpeff_op_threshold_compact": (C.c_int, [C.c_int64, _p, C.c_float, C.c_float, _p, _p, C.POINTER(C.c_int64)]),
+    "dnpeff_threshold_find": (C.c_int, [C.c_int64, _p, C.c_float, C.c_float, C.POINTER(C.c_int64), _pp]),
+    "dnpeff_threshold_take": (C.c_int, [_p, _p, _p]),
     "dnpeff_csr_split_dense_head": (C.c_int, [_p, C.c_double, C.POINTER(C.c_int64)]),
     "dnpeff_csr_head_info": (C.c_int, [_p, C.POINTER(C.c_int64), C.POINTER(C.c_int64)]),
     "dnpeff_csr_products_info": (C.c_int, [_p, _p]),
@@ -397,12 +399,16 @@ def topk_rows(x: "DeviceArray", k: int):
 
 def op_threshold_compact(x: "DeviceArray", divisor: float, threshold: float):
     """(positions, values) of the elements with x / divisor >= threshold, as numpy arrays."""
-    n = int(np.prod(x.shape))
-    idx, val = _Scratch(4 * max(n, 1)), _Scratch(4 * max(n, 1))
-    kept = _i64(0)
-    _check(lib.dnpeff_op_threshold_compact(n, x.ptr, float(divisor), float(threshold), idx.ptr, val.ptr,
-                                           C.byref(kept)))
-    return tuple(_scratch_numpy((idx, (kept.value,), np.int32), (val, (kept.value,), np.float32)))
+    kept, found = _i64(0), C.c_void_p()
+    _check(lib.dnpeff_threshold_find(int(np.prod(x.shape)), x.ptr, float(divisor), float(threshold), C.byref(kept),
+                                     C.byref(found)))
+    try:
+        idx, val = np.empty(kept.value, np.int32), np.empty(kept.value, np.float32)
+    except MemoryError:
+        lib.dnpeff_threshold_take(found, None, None)
+        raise
+    _check(lib.dnpeff_threshold_take(found, idx.ctypes.data, val.ctypes.data))
+    return idx, val
 
 
 class Csr:

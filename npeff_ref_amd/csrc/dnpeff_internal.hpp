@@ -81,6 +81,25 @@ inline hipError_t copy_down_parts(std::initializer_list<copy_part> parts) { retu
 constexpr int HOST_WORDS = 512;
 int host_words(unsigned long long** out);  // HOST_WORDS pinned words of the calling thread
 
+// One of the pinned buffers that short copies go through, for a kernel that writes a call's results there.  p() is NULL
+// where none could be had.  Whoever gives it back has waited for what writes to it.
+class pinned_buf {
+ public:
+  static constexpr size_t BYTES = (size_t)2 << 20;
+  pinned_buf() = default;
+  pinned_buf(const pinned_buf&) = delete;
+  pinned_buf& operator=(const pinned_buf&) = delete;
+  ~pinned_buf() { give(); }
+  void take();
+  void give();
+  char* p() const { return p_; }
+
+ private:
+  char* p_ = nullptr;
+  hipEvent_t done_[2] = {};
+  int dev_ = 0;
+};
+
 template <class T>
 inline int dmalloc(T** p, int64_t count) {
   return device_alloc((void**)p, sizeof(T) * (size_t)(count > 0 ? count : 1));

@@ -59,11 +59,9 @@ int main(int argc, char** argv) {
   int n_dev = 0;
   ok(dnpeff_device_count(&n_dev));
   if (n_dev < 1) fatal("Error: no GPU visible.");
-  void *x = nullptr, *idx = nullptr, *val = nullptr;
+  void* x = nullptr;
   const size_t m = (size_t)out.m;
   ok(dnpeff_dev_malloc(m * 4 + 4, &x));
-  ok(dnpeff_dev_malloc(m * 4 + 4, &idx));
-  ok(dnpeff_dev_malloc(m * 4 + 4, &val));
   std::vector<float> row(m);
   out.H_row_offsets.assign(1, 0);
   for (long k = 0; k < out.r; k++) {
@@ -74,22 +72,17 @@ int main(int argc, char** argv) {
     const float norm = (float)std::sqrt(sq);
     const float divisor = norm > 0.0f ? norm : 1.0f;
     int64_t kept = 0;
-    ok(dnpeff_op_threshold_compact(out.m, (const float*)x, divisor, threshold, (int32_t*)idx,
-                                   (float*)val, &kept));
+    void* found = nullptr;
+    ok(dnpeff_threshold_find(out.m, (const float*)x, divisor, threshold, &kept, &found));
     const size_t at = out.H_values.size();
     out.H_values.resize(at + (size_t)kept);
     out.H_col_indices.resize(at + (size_t)kept);
-    if (kept) {
-      ok(dnpeff_dev_download(out.H_values.data() + at, val, (size_t)kept * 4));
-      ok(dnpeff_dev_download(out.H_col_indices.data() + at, idx, (size_t)kept * 4));
-    }
+    ok(dnpeff_threshold_take(found, out.H_col_indices.data() + at, out.H_values.data() + at));
     out.H_row_offsets.push_back((int64_t)out.H_values.size());
     for (long i = 0; i < out.n; i++) out.W[(size_t)i * out.r + k] *= divisor;
   }
   H5Fclose(file);
   dnpeff_dev_free(x);
-  dnpeff_dev_free(idx);
-  dnpeff_dev_free(val);
   std::printf("Sparse NNZ: %zu\n", out.H_values.size());
   h5io::write_sparse_decomposition(out_path, out);
   return 0;

@@ -338,6 +338,23 @@ static bool bounce_take(int dev, bounce_buf* b) {
 static void bounce_give(int dev, bounce_buf& b) {
   if (!bounces().give(dev, b, BOUNCE_KEPT)) bounce_free(b);
 }
+static_assert(pinned_buf::BYTES == 2 * BOUNCE_HALF, "one kind of buffer");
+void pinned_buf::take() {
+  bounce_buf b;
+  if (p_ || hipGetDevice(&dev_) != hipSuccess || !bounce_take(dev_, &b)) return;
+  p_ = b.p;
+  done_[0] = b.done[0];
+  done_[1] = b.done[1];
+}
+void pinned_buf::give() {
+  if (!p_) return;
+  bounce_buf b;
+  b.p = p_;
+  b.done[0] = done_[0];
+  b.done[1] = done_[1];
+  bounce_give(dev_, b);
+  p_ = nullptr;
+}
 static void bounce_trim() { bounces().drain(bounce_free); }
 
 __global__ void __launch_bounds__(256) k_copy_words(const uint32_t* __restrict__ src, uint32_t* __restrict__ dst, int n) {

@@ -4,6 +4,8 @@ Tolerances: the kernels compute in fp32 with fp32 (MFMA / FMA) accumulation over
 partial sums; against fp64 the bound used is 2e-5 relative to the largest magnitude of the
 output (norm-wise), far inside the 1e-4 the full 50-iteration run has to meet."""
 
+import ctypes as C
+
 import numpy as np
 import scipy.sparse as sp
 import pytest
@@ -512,6 +514,60 @@ def test_threshold_compact_bit_exact(n, div, thr):
     keep = q >= np.float32(thr)
     assert np.array_equal(idx, np.nonzero(keep)[0].astype(np.int32))
     assert np.array_equal(val, q[keep])
+
+
+@pytest.mark.parametrize("n,share,offset", [
+    (1, 1.0, 0), (3, 0.0, 0), (4095, 0.5, 1), (4 * 1024 * 1024 + 1029, 0.02, 0), (4 * 1024 * 1024 + 1029, 0.02, 3),
+    (262144, 1.0, 0),       # the last that the pinned buffer holds: 256 runs, 1024 finds each
+    (262145, 1.0, 0),       # one more
+    (9_000_000, 0.001, 0),  # runs of nine tiles: two steps of four and one tile over
+    (9_000_000, -1.0, 0),   # all finds in few runs: more than a run's notes, less than the buffer
+    (2_500_000, 0.3, 0),    # more than the buffer, staged down
+])
+def test_threshold_find_equals_compact(n, share, offset):
+    """Finds for a host caller equal the device compaction, bit for bit, wherever they are held."""
+    rng = np.random.default_rng(n)
+    x = rng.random(n + offset).astype(np.float32)
+    if share < 1:
+        x[offset:][::97] = np.nan
+    if share < 0:
+        x[:] = 0.0
+        x[70_000:75_000] = 9.0
+    thr = np.float32(0.5) if share < 0 else np.float32(2.0 * (1.0 - share))
+    buf = d.DeviceArray.from_numpy(x)
+    ptr = C.c_void_p(buf.ptr.value + 4 * offset)
+    outs, kept, found = [d.DeviceArray((n,), np.int32), d.DeviceArray((n,), np.float32)], C.c_int64(), C.c_void_p()
+    d.binding._check(d.binding.lib.dnpeff_op_threshold_compact(n, ptr, 0.5, thr, outs[0].ptr, outs[1].ptr, C.byref(kept)))
+    wi, wv = (o.numpy()[:kept.value] for o in outs)
+    with np.errstate(invalid="ignore"):
+        q = x[offset:] / np.float32(0.5)
+        assert np.array_equal(wi, np.nonzero(q >= thr)[0]) and np.array_equal(wv, q[wi])
+    d.binding._check(d.binding.lib.dnpeff_threshold_find(n, ptr, 0.5, thr, C.byref(kept), C.byref(found)))
+    assert kept.value == len(wi)
+    idx, val = np.empty(kept.value, np.int32), np.empty(kept.value, np.float32)
+    d.binding._check(d.binding.lib.dnpeff_threshold_take(found, idx.ctypes.data, val.ctypes.data))
+    assert np.array_equal(idx, wi) and np.array_equal(val, wv)
+
+
+@pytest.mark.parametrize("div", [3.7, 1e-38, 2e38, 1e-45, np.inf, -0.3, np.nan])
+@pytest.mark.parametrize("thr", [0.1, 0.0, -2.5, 1e-45, 3e38, np.inf, -np.inf, np.nan])
+def test_threshold_cut_is_exact(div, thr):
+    """The kept set is that of the rounded fp32 quotients, next to the cut and at the ends of the type."""
+    div, thr = np.float32(div), np.float32(thr)
+    with np.errstate(all="ignore"):
+        near = [np.float32(thr * div)]
+        for way in (np.float32(np.inf), np.float32(-np.inf)):
+            y = near[0]
+            for _ in range(8):
+                y = np.nextafter(y, way)
+                near.append(y)
+        rng = np.random.default_rng(5)
+        any_bits = rng.integers(0, 2**32, 3000, dtype=np.uint32).view(np.float32)
+        x = np.concatenate([near, [0.0, -0.0, np.inf, -np.inf, 1e-45, -1e-45, 3.4e38], any_bits]).astype(np.float32)
+        q = x / div
+        keep = q >= thr
+    idx, val = d.op_threshold_compact(d.DeviceArray.from_numpy(x), float(div), float(thr))
+    assert np.array_equal(idx, np.nonzero(keep)[0]) and np.array_equal(val, q[keep])
 
 
 @pytest.mark.parametrize("n,count,k", [(3, 100000, 4096), (2, 5000, 1), (1, 70001, 70001), (4, 30000, 5000),
