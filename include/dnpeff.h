@@ -487,6 +487,10 @@ int dnpeff_threshold_take(void* found, int32_t* idx_host, float* val_host);
 int dnpeff_topk_rows(int64_t n_rows, int64_t count, int64_t k, const float* x, float* vals_out,
                      int32_t* idx_out, float* norms_out);
 
+/* The same with the results in host arrays; its device memory for them is its own. */
+int dnpeff_topk_rows_host(int64_t n_rows, int64_t count, int64_t k, const float* x, float* vals_host,
+                          int32_t* idx_host, float* norms_host);
+
 /* G[r, r] = X^T X for X [rows, r].  cublasSgemm at device_contexts1.h:303,322. */
 int dnpeff_op_gram(int64_t rows, int r, const float* X, float* G_rr);
 

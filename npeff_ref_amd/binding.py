@@ -70,6 +70,7 @@ SIGNATURES = {
     "dnpeff_csr_sq_norm": (C.c_int, [_p, C.POINTER(_f64)]),
     "dnpeff_csr_build_transpose": (C.c_int, [_p]),
     "dnpeff_topk_rows": (C.c_int, [C.c_int64, C.c_int64, C.c_int64, _p, _p, _p, _p]),
+    "dnpeff_topk_rows_host": (C.c_int, [C.c_int64, C.c_int64, C.c_int64, _p, _p, _p, _p]),
     "dnpeff_op_threshold_compact": (C.c_int, [C.c_int64, _p, C.c_float, C.c_float, _p, _p, C.POINTER(C.c_int64)]),
     "dnpeff_threshold_find": (C.c_int, [C.c_int64, _p, C.c_float, C.c_float, C.POINTER(C.c_int64), _pp]),
     "dnpeff_threshold_take": (C.c_int, [_p, _p, _p]),
@@ -392,9 +393,10 @@ def op_init_uniform(matrix_id: int, logical_rows: int, logical_cols: int, seed: 
 def topk_rows(x: "DeviceArray", k: int):
     """(values [n, k], indices [n, k], norms [n]) of the k largest entries of each row of x."""
     n, count = x.shape
-    vals, idx, norms = _Scratch(4 * n * k), _Scratch(4 * n * k), _Scratch(4 * n)
-    _check(lib.dnpeff_topk_rows(n, count, k, x.ptr, vals.ptr, idx.ptr, norms.ptr))
-    return tuple(_scratch_numpy((vals, (n, k), np.float32), (idx, (n, k), np.int32), (norms, (n,), np.float32)))
+    kept = min(max(k, 0), count)  # (a k out of range is refused below)
+    out = np.empty((n, kept), np.float32), np.empty((n, kept), np.int32), np.empty((n,), np.float32)
+    _check(lib.dnpeff_topk_rows_host(n, count, k, x.ptr, *(a.ctypes.data for a in out)))
+    return out
 
 
 def op_threshold_compact(x: "DeviceArray", divisor: float, threshold: float):

@@ -99,6 +99,11 @@ class pinned_buf {
   hipEvent_t done_[2] = {};
   int dev_ = 0;
 };
+// Short arrays down through such a buffer: a kernel writes them side by side, each (whole words) in gather_room bytes, and
+// after a wait for the library stream they are taken from there.
+inline size_t gather_room(size_t bytes) { return (bytes + 15) / 16 * 16; }
+hipError_t gather_queue(const copy_part* parts, int n_parts, char* buf);
+void gather_take(const copy_part* parts, int n_parts, const char* buf);
 
 template <class T>
 inline int dmalloc(T** p, int64_t count) {

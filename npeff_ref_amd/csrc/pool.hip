@@ -437,20 +437,9 @@ __global__ void __launch_bounds__(256) k_gather_parts(gather_parts p, uint32_t* 
   for (int i = 4 * quads + blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) to[i] = src[i];
 }
 
-// Several short arrays down as one: a kernel writes them to a bounce buffer side by side, one wait for all.
-// (Two arrays of 240 KB: one wait and 10 us of writes where the engine's copies took two waits and 14 us each before
-// they began.)
-static hipError_t gather_down(const copy_part* parts, int n_parts) {
-  bounce_buf B;
-  int dev = 0;
-  hipError_t e = hipGetDevice(&dev);
-  if (e != hipSuccess) return e;
-  if (!bounce_take(dev, &B)) {
-    for (int q = 0; q < n_parts && e == hipSuccess; q++) e = hipMemcpy(parts[q].dst, parts[q].src, parts[q].bytes, hipMemcpyDeviceToHost);
-    return e;
-  }
-  hipStream_t st = stream();
+hipError_t gather_queue(const copy_part* parts, int n_parts, char* buf) {
   size_t at = 0;
+  hipError_t e = hipSuccess;
   for (int q = 0; q < n_parts && e == hipSuccess; q += GATHER_PARTS) {
     gather_parts g = {};
     size_t most = 0;
@@ -459,21 +448,34 @@ static hipError_t gather_down(const copy_part* parts, int n_parts) {
       g.src[i] = (const uint32_t*)p.src;
       g.words[i] = (int)(p.bytes / 4);
       g.at[i] = (int)(at / 4);
-      at += (p.bytes + 15) / 16 * 16;
+      at += gather_room(p.bytes);
       most = most > p.bytes ? most : p.bytes;
     }
     const int wgs = (int)((most + 16383) / 16384);
-    hipLaunchKernelGGL(k_gather_parts, dim3(wgs < COPY_WGS ? wgs : COPY_WGS, GATHER_PARTS), dim3(256), 0, st, g, (uint32_t*)B.p);
+    hipLaunchKernelGGL(k_gather_parts, dim3(wgs < COPY_WGS ? wgs : COPY_WGS, GATHER_PARTS), dim3(256), 0, stream(), g, (uint32_t*)buf);
     e = hipGetLastError();
   }
-  const hipError_t es = hipStreamSynchronize(st);
-  if (e == hipSuccess) e = es;
-  at = 0;
-  for (int q = 0; q < n_parts && e == hipSuccess; q++) {
-    memcpy(parts[q].dst, B.p + at, parts[q].bytes);
-    at += (parts[q].bytes + 15) / 16 * 16;
+  return e;
+}
+void gather_take(const copy_part* parts, int n_parts, const char* buf) {
+  for (int q = 0; q < n_parts; buf += gather_room(parts[q].bytes), q++) memcpy(parts[q].dst, buf, parts[q].bytes);
+}
+
+// Several short arrays down as one: a kernel writes them to a bounce buffer side by side, one wait for all.
+// (Two arrays of 240 KB: one wait and 10 us of writes where the engine's copies took two waits and 14 us each before
+// they began.)
+static hipError_t gather_down(const copy_part* parts, int n_parts) {
+  pinned_buf B;
+  B.take();
+  hipError_t e = hipSuccess;
+  if (!B.p()) {
+    for (int q = 0; q < n_parts && e == hipSuccess; q++) e = hipMemcpy(parts[q].dst, parts[q].src, parts[q].bytes, hipMemcpyDeviceToHost);
+    return e;
   }
-  bounce_give(dev, B);
+  e = gather_queue(parts, n_parts, B.p());
+  const hipError_t es = hipStreamSynchronize(stream());
+  if (e == hipSuccess) e = es;
+  if (e == hipSuccess) gather_take(parts, n_parts, B.p());
   return e;
 }
 

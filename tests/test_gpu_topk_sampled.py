@@ -70,3 +70,21 @@ def test_threshold_and_largest_entry_close_together(count, k, kind):
     order = np.lexsort((np.arange(count), -x))[:k]
     assert np.array_equal(idx[0], order) and np.array_equal(vals[0], x[order])
     np.testing.assert_allclose(norms[0], np.sqrt((x.astype(np.float64) ** 2).sum()), rtol=1e-7)
+
+
+@pytest.mark.parametrize("kind,n,count,k", [("lognormal", 2, 600_000, 65_536), ("lognormal", 1, 700_000, 262_100),
+                                            ("lognormal", 3, 600_001, 300_000), ("few", 2, 524_288, 5000),
+                                            ("hidden", 1, 600_000, 900), ("uniform", 1, 9, 1)])
+def test_results_for_the_host_equal_those_on_the_device(kind, n, count, k):
+    """One pinned buffer holds them (the second case just), or not, or the sample's threshold does not serve."""
+    x = d.DeviceArray.from_numpy(_values(kind, n, count, np.random.default_rng(k)))
+    on_dev = [d.DeviceArray((n, k)), d.DeviceArray((n, k), np.int32), d.DeviceArray((n,))]
+    d.binding._check(d.lib.dnpeff_topk_rows(n, count, k, x.ptr, *(a.ptr for a in on_dev)))
+    for got, want in zip(d.topk_rows(x, k), on_dev):
+        assert np.array_equal(got, want.numpy())
+    vals, idx = np.empty((n, k), np.float32), np.empty((n, k), np.int32)
+    d.binding._check(d.lib.dnpeff_topk_rows_host(n, count, k, x.ptr, vals.ctypes.data, idx.ctypes.data, None))
+    assert np.array_equal(vals, on_dev[0].numpy()) and np.array_equal(idx, on_dev[1].numpy())
+    for bad in (0, -1, count + 1):
+        with pytest.raises(d.DnpeffError):
+            d.topk_rows(x, bad)
