@@ -6,8 +6,7 @@
 // A row has ~1e8 entries and k ~ 6.5e4, so sorting the row is out of the question.  Usual case, one read
 // of the row and a thirty-second of it before:
 //   1. two histograms (11 bits of an order-preserving integer key each) of a sample, 64 entries out
-//      of every 2048 (of every 4096 where k leaves 512 of them above the threshold: 14 us instead of 23 for
-//      the first at 2 rows of 110 M), give a threshold that a little more than k entries reach (all entries
+//      of every 2048 (of every 4096, half the lines, where k leaves 512 of them above the threshold), give a threshold that a little more than k entries reach (all entries
 //      of a short row: exactly the k-th entry's 22 bits);
 //   2. every entry from the threshold up goes to a candidate list ((key, index) pairs, any order) and is
 //      counted into its bucket (topk_buckets.hpp), and the sum of squares is taken on the way;
@@ -364,21 +363,26 @@ __global__ void __launch_bounds__(1024)
   for (int i = threadIdx.x; i < nb; i += 1024) buckets[(int64_t)blockIdx.x * nb + i] = 0;
 }
 
+// A workgroup of 16 waves and two rounds of loads per wave (128 chunks): every workgroup adds its histogram to the row's few
+// busy lines, and it is those additions that wait for each other.  2 rows of 110 M, LEVEL 0: 8.7 us; 16.3 with workgroups
+// of four waves and 64 chunks, 10.9 with 512 chunks for 16 waves.
+constexpr int TOPK_SAMPLE_WAVES = 16;
+constexpr int TOPK_SAMPLE_EACH = 128;
 // LEVEL 0: top 11 bits of the key, and the largest key; 1: the next 11 of the entries in the bin that level 0 found.
 template <int LEVEL>
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(TOPK_SAMPLE_WAVES * 64)
     k_topk_sample(const float* __restrict__ x, int64_t count, int64_t stride, int64_t chunks,
                   TopkRow* __restrict__ rows, unsigned* __restrict__ hist) {
   __shared__ unsigned h[TOPK_BINS];
-  __shared__ uint32_t most[4];
+  __shared__ uint32_t most[TOPK_SAMPLE_WAVES];
   const int row = blockIdx.y, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  for (int i = threadIdx.x; i < TOPK_BINS; i += 256) h[i] = 0;
+  for (int i = threadIdx.x; i < TOPK_BINS; i += TOPK_SAMPLE_WAVES * 64) h[i] = 0;
   const uint32_t bin = LEVEL ? rows[row].bin : 0u;
   uint32_t top = 0;
   __syncthreads();
   const float* xr = x + (int64_t)row * count;
-  const int64_t step = (int64_t)gridDim.x * 4;
-  for (int64_t c = (int64_t)blockIdx.x * 4 + wave; c < chunks; c += 4 * step) {
+  const int64_t step = (int64_t)gridDim.x * TOPK_SAMPLE_WAVES;
+  for (int64_t c = (int64_t)blockIdx.x * TOPK_SAMPLE_WAVES + wave; c < chunks; c += 4 * step) {
     float v[4];
     bool ok[4];
 #pragma unroll
@@ -401,9 +405,12 @@ __global__ void __launch_bounds__(256)
     if (lane == 0) most[wave] = top;
   }
   __syncthreads();
-  for (int i = threadIdx.x; i < TOPK_BINS; i += 256)
+  for (int i = threadIdx.x; i < TOPK_BINS; i += TOPK_SAMPLE_WAVES * 64)
     if (h[i]) atomicAdd(&hist[(int64_t)row * TOPK_BINS + i], h[i]);
-  if (!LEVEL && threadIdx.x == 0) atomicMax(&rows[row].top, max(max(most[0], most[1]), max(most[2], most[3])));
+  if (!LEVEL && threadIdx.x == 0) {
+    for (int w = 1; w < TOPK_SAMPLE_WAVES; w++) top = max(top, most[w]);
+    atomicMax(&rows[row].top, top);
+  }
 }
 
 // The bin from the top where the sample's entries reach the target.
@@ -678,10 +685,10 @@ static int topk_by_sample(int64_t n_rows, int64_t count, int64_t k, const float*
   DN_TRY(host_words(&failed));
   *failed = 0;
   hipLaunchKernelGGL(k_topk_row_init, dim3((unsigned)n_rows), dim3(1024), 0, st, rows.p, plan.target, hist.p, plan.buckets(), starts.p);
-  const dim3 gs = blocks(chunks, 64), gr((unsigned)n_rows), gp = blocks(cap, 256);
-  hipLaunchKernelGGL(k_topk_sample<0>, gs, block, 0, st, x, count, stride, chunks, rows.p, hist.p);
+  const dim3 gs = blocks(chunks, TOPK_SAMPLE_EACH), gr((unsigned)n_rows), gp = blocks(cap, 256);
+  hipLaunchKernelGGL(k_topk_sample<0>, gs, dim3(TOPK_SAMPLE_WAVES * 64), 0, st, x, count, stride, chunks, rows.p, hist.p);
   hipLaunchKernelGGL(k_topk_threshold<0>, gr, block, 0, st, hist.p, rows.p);
-  hipLaunchKernelGGL(k_topk_sample<1>, gs, block, 0, st, x, count, stride, chunks, rows.p, hist.p);
+  hipLaunchKernelGGL(k_topk_sample<1>, gs, dim3(TOPK_SAMPLE_WAVES * 64), 0, st, x, count, stride, chunks, rows.p, hist.p);
   hipLaunchKernelGGL(k_topk_threshold<1>, gr, block, 0, st, hist.p, rows.p);
   if (count % 4 == 0 && ((uintptr_t)x % 16) == 0)
     hipLaunchKernelGGL(k_topk_collect<true>, gc, block, 0, st, x, count, rows.p, cand.p, cap, log_nb, above, starts.p, place.p, sq.p);
