@@ -982,24 +982,6 @@ __global__ void __launch_bounds__(256)
     if (colptr[j + 1] - colptr[j] > limit) long_cols[pos[j]] = (int32_t)j;
 }
 
-__global__ void __launch_bounds__(256)
-    k_sq_norm_partial(const float* __restrict__ v, int64_t n, double* __restrict__ partials) {
-  __shared__ double sh[256];
-  double s = 0.0;
-  int64_t stride = (int64_t)gridDim.x * 256;
-  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += stride) {
-    double x = (double)v[i];
-    s += x * x;
-  }
-  sh[threadIdx.x] = s;
-  __syncthreads();
-  for (int off = 128; off > 0; off >>= 1) {
-    if (threadIdx.x < off) sh[threadIdx.x] += sh[threadIdx.x + off];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) partials[blockIdx.x] = sh[0];
-}
-
 // Grid of a grid-stride kernel over n items (every kernel launched with it loops); a launch is
 // limited to 2^32 threads in total, so grids are capped well below that.
 static unsigned grid_for(int64_t n, int64_t cap = 1 << 20) {
@@ -1790,16 +1772,8 @@ DN_API int dnpeff_csr_sq_norm(const dnpeff_csr* A, double* out) {
   // (with a dense head the whole matrix's values only exist in the row-major copy)
   const float* v = A->vals ? A->vals : (A->tail ? nullptr : A->tvals);
   DN_CHECK(v != nullptr || A->nnz == 0, "the row-major copy of the matrix was released before its norm was taken");
-  const int blocks = 1024;
-  double* partials = nullptr;
-  DN_TRY(dmalloc(&partials, blocks));
-  hipLaunchKernelGGL(k_sq_norm_partial, dim3(blocks), dim3(256), 0, stream(), v, A->nnz, partials);
-  DN_LAUNCH_CHECK();
-  std::vector<double> h(blocks);
-  DN_HIP(copy_down(h.data(), partials, sizeof(double) * blocks));
-  dfree(partials);
   double s = 0.0;
-  for (int i = 0; i < blocks; i++) s += h[i];
+  DN_TRY(dnpeff_op_dot(A->nnz, v, v, &s));
   *out = s;
   dnpeff_csr* M = const_cast<dnpeff_csr*>(A);
   M->sq_norm = s;
@@ -2273,14 +2247,19 @@ DN_API int dnpeff_csr_build_transpose(dnpeff_csr* A) {
   if (!done && transpose_ranges_pay(A)) DN_TRY(transpose_by_ranges(A, colptr, rowind, tvals, &done));
   if (!done) DN_TRY(transpose_by_rows(A, count, colptr, rowind, tvals));
   count.reset();
-  // list of long columns for A^T W
-  DN_TRY(pos.alloc(m + 1));
-  unsigned long long* host = nullptr;
-  DN_TRY(host_words(&host));
-  int64_t* total = reinterpret_cast<int64_t*>(host);
-  DN_TRY(scan_long_cols(colptr, SPMM_T_LONG, m, pos, total));
-  DN_HIP(hipStreamSynchronize(st));
-  const int64_t n_long = *total;
+  // list of long columns for A^T W; a column has no row twice, so that few rows have none (22 M columns: 0.22 ms)
+  int64_t n_long = 0;
+  if (A->n_rows > SPMM_T_LONG) {
+    DN_TRY(pos.alloc(m + 1));
+    unsigned long long* host = nullptr;
+    DN_TRY(host_words(&host));
+    int64_t* total = reinterpret_cast<int64_t*>(host);
+    DN_TRY(scan_long_cols(colptr, SPMM_T_LONG, m, pos, total));
+    DN_HIP(hipStreamSynchronize(st));
+    n_long = *total;
+  } else {
+    DN_HIP(hipStreamSynchronize(st));
+  }
   DN_TRY(long_cols.alloc(n_long));
   if (n_long) {
     hipLaunchKernelGGL(k_collect_long, dim3(grid_for(m)), dim3(256), 0, st, colptr.p, SPMM_T_LONG, m,
