@@ -331,6 +331,10 @@ int dnpeff_nmf_update_H(dnpeff_nmf* nmf);
  * reductions: the quantity of computeUncachedLoss (nmf1.h:242-274,
  * device_contexts1.h:337-354) through the same trace identity. */
 int dnpeff_nmf_loss(dnpeff_nmf* nmf, double* out);
+/* dnpeff_nmf_step and dnpeff_nmf_loss of what it leaves, in one call, and in *steps_ms the time of the
+ * steps alone (the figure that nmf1.h:186-200 logs): their time on the device where steps and
+ * loss are one launch, the host's clock around them otherwise. */
+int dnpeff_nmf_step_loss(dnpeff_nmf* nmf, int n_steps, double* loss, double* steps_ms);
 
 /* The three terms of the loss: ||A||^2, <H,(W^T W)H>, <W^T A,H>. */
 int dnpeff_nmf_loss_terms(dnpeff_nmf* nmf, double* sq_norm_A, double* pos, double* neg);
@@ -412,6 +416,8 @@ int dnpeff_fit_step(dnpeff_fit* fit, int n_steps);
  * the reference logs (nmf_sparse_H.h:319-331).  true_loss uses W (H H^T) of
  * the current W.  Either pointer may be NULL. */
 int dnpeff_fit_loss(dnpeff_fit* fit, double* reference_loss, double* true_loss);
+/* dnpeff_fit_step and dnpeff_fit_loss in one call; *steps_ms as in dnpeff_nmf_step_loss. */
+int dnpeff_fit_step_loss(dnpeff_fit* fit, int n_steps, double* reference_loss, double* true_loss, double* steps_ms);
 
 int dnpeff_fit_get_W(dnpeff_fit* fit, float* W_nr);
 /* Stage-1 products: AH [n, r] row-major, HH [r, r]. */

@@ -5,7 +5,6 @@ from __future__ import annotations
 import ctypes as C
 import math
 import os
-import time
 from dataclasses import dataclass
 from typing import Callable, Optional
 
@@ -115,6 +114,8 @@ SIGNATURES = {
     "dnpeff_fit_create": (C.c_int, [_p, _p, _f32, _i64, _pp]),
     "dnpeff_fit_init_W": (C.c_int, [_p]),
     "dnpeff_fit_set_W": (C.c_int, [_p, _p]),
+    "dnpeff_nmf_step_loss": (C.c_int, [_p, C.c_int, C.POINTER(_f64), C.POINTER(_f64)]),
+    "dnpeff_fit_step_loss": (C.c_int, [_p, C.c_int, C.POINTER(_f64), C.POINTER(_f64), C.POINTER(_f64)]),
     "dnpeff_fit_step": (C.c_int, [_p, C.c_int]),
     "dnpeff_fit_loss": (C.c_int, [_p, C.POINTER(_f64), C.POINTER(_f64)]),
     "dnpeff_fit_get_W": (C.c_int, [_p, _p]),
@@ -651,23 +652,20 @@ class MuNmf:
             self.initialize()
         p = self.params
         history = []
-        sync()
-        t0 = time.perf_counter()
         done = 0
         while done < p.max_iters:  # the steps up to the next logged one in one call
             run = p.max_iters - done
             if p.log_every > 0:
                 run = min(run, p.log_every - done % p.log_every)
-            self.step(run)
             done += run
             if p.log_every > 0 and done % p.log_every == 0:
-                sync()
-                elapsed_ms = (time.perf_counter() - t0) * 1e3
-                loss = self.computeUncachedLoss()
-                ms = elapsed_ms / p.log_every
-                log(f"step {done}: {loss:g} [{ms:g} ms/step]")
-                history.append((done, loss, ms))
-                t0 = time.perf_counter()
+                loss, steps_ms = _f64(0), _f64(0)
+                _check(lib.dnpeff_nmf_step_loss(self._h, run, C.byref(loss), C.byref(steps_ms)))
+                ms = steps_ms.value / p.log_every
+                log(f"step {done}: {loss.value:g} [{ms:g} ms/step]")
+                history.append((done, loss.value, ms))
+            else:
+                self.step(run)
         sync()
         return history
 
@@ -776,24 +774,21 @@ class Learner:
             self.initialize()
         p = self.params
         history = []
-        sync()
-        t0 = time.perf_counter()
         every = p.log_every_n_steps
         done = 0
         while done < p.max_iters:  # the steps up to the next logged one in one call
             run = p.max_iters - done
             if every > 0:
                 run = min(run, every - done % every)
-            self.step(run)
             done += run
             if every > 0 and done % every == 0:
-                sync()
-                elapsed_ms = (time.perf_counter() - t0) * 1e3
-                ref_loss, true_loss = self.losses()
-                ms = elapsed_ms / every
-                log(f"step {done}: {ref_loss:g} [{ms:g} ms/step]")
-                history.append((done, ref_loss, true_loss, ms))
-                t0 = time.perf_counter()
+                ref_loss, true_loss, steps_ms = _f64(0), _f64(0), _f64(0)
+                _check(lib.dnpeff_fit_step_loss(self._h, run, C.byref(ref_loss), C.byref(true_loss), C.byref(steps_ms)))
+                ms = steps_ms.value / every
+                log(f"step {done}: {ref_loss.value:g} [{ms:g} ms/step]")
+                history.append((done, ref_loss.value, true_loss.value, ms))
+            else:
+                self.step(run)
         sync()
         return history
 

@@ -797,16 +797,18 @@ DN_API int dnpeff_nmf_update_H(dnpeff_nmf* h) {
   return 0;
 }
 
+static int small_steps(dnpeff_nmf* nmf, int n_steps, double* sums) {
+  DN_TRY(take_back(nmf));
+  nmf->w_out = nmf->h_out = false;
+  nmf->fu.gh_state = nmf->fu.gw_state = fused_state::NONE;
+  nmf->gh_valid = nmf->nw_valid = nmf->fu_n_valid = false;
+  return fused_small_launch(nmf->A, nmf->r, nmf->W, nmf->H, nmf->eps, n_steps, sums);
+}
+
 DN_API int dnpeff_nmf_step(dnpeff_nmf* nmf, int n_steps) {
   clear_error();
   DN_CHECK(nmf != nullptr, "handle is NULL");
-  if (n_steps > 0 && small_now(nmf)) {
-    DN_TRY(take_back(nmf));
-    nmf->w_out = nmf->h_out = false;
-    nmf->fu.gh_state = nmf->fu.gw_state = fused_state::NONE;
-    nmf->gh_valid = nmf->nw_valid = nmf->fu_n_valid = false;
-    return fused_small_launch(nmf->A, nmf->r, nmf->W, nmf->H, nmf->eps, n_steps, nullptr);
-  }
+  if (n_steps > 0 && small_now(nmf)) return small_steps(nmf, n_steps, nullptr);
   for (int s = 0; s < n_steps; s++) {
     DN_TRY(dnpeff_nmf_update_W(nmf));
     DN_TRY(dnpeff_nmf_update_H(nmf));
@@ -893,6 +895,40 @@ DN_API int dnpeff_nmf_check_products(dnpeff_nmf* h, double* via_rows, double* vi
   }
   *via_columns = sum;
   return 0;
+}
+
+// Ticks of wall_clock64() to milliseconds.
+static int ticks_to_ms(double ticks, double* ms) {
+  int dev = 0, khz = 0;
+  DN_HIP(hipGetDevice(&dev));
+  DN_HIP(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, dev));
+  *ms = khz > 0 ? ticks / (double)khz : 0.0;
+  return 0;
+}
+
+// steps(), the host's clock on it (nothing else in hand before and after), then loss()
+template <class Steps, class Loss>
+static int steps_then_loss(Steps steps, Loss loss, double* ms) {
+  DN_TRY(dnpeff_sync());
+  const auto t0 = std::chrono::steady_clock::now();
+  DN_TRY(steps());
+  DN_TRY(dnpeff_sync());
+  *ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
+  return loss();
+}
+
+DN_API int dnpeff_nmf_step_loss(dnpeff_nmf* h, int n_steps, double* loss, double* steps_ms) {
+  clear_error();
+  DN_CHECK(h && loss && steps_ms, "NULL argument");
+  if (n_steps < 1 || n_steps > FUSED_SMALL_STEPS || !small_now(h))
+    return steps_then_loss([&] { return dnpeff_nmf_step(h, n_steps); }, [&] { return dnpeff_nmf_loss(h, loss); }, steps_ms);
+  unsigned long long* words = nullptr;
+  DN_TRY(host_words(&words));
+  double* sums = reinterpret_cast<double*>(words);
+  DN_TRY(small_steps(h, n_steps, sums));
+  DN_HIP(hipStreamSynchronize(stream()));
+  *loss = std::sqrt(h->sq_norm_A + sums[1] - 2.0 * sums[0]);
+  return ticks_to_ms(sums[2], steps_ms);
 }
 
 DN_API int dnpeff_nmf_loss(dnpeff_nmf* nmf, double* out) {
@@ -1065,7 +1101,7 @@ DN_API int dnpeff_fit_step(dnpeff_fit* f, int n_steps) {
   if (n_steps <= 0) return 0;
   if (f->in_place) {
     f->whh_valid = true;
-    return launch_fit_steps(f->n, f->r, f->W, f->HH, f->AH, f->eps, n_steps, f->WHH);
+    return launch_fit_steps(f->n, f->r, f->W, f->HH, f->AH, f->eps, n_steps, f->WHH, nullptr);
   }
   struct held_g {  // H H^T is the same in every step: one copy for all of them
     ~held_g() { xg_mu_release_g(); }
@@ -1119,6 +1155,28 @@ DN_API int dnpeff_fit_loss(dnpeff_fit* f, double* reference_loss, double* true_l
     *reference_loss = std::sqrt(f->sq_norm_A + pos_ref - 2.0 * neg);
   }
   return 0;
+}
+
+DN_API int dnpeff_fit_step_loss(dnpeff_fit* f, int n_steps, double* reference_loss, double* true_loss, double* steps_ms) {
+  clear_error();
+  DN_CHECK(f && steps_ms, "NULL argument");
+  if (!f->in_place || !fit_loss_with_steps(f->n, n_steps))
+    return steps_then_loss([&] { return dnpeff_fit_step(f, n_steps); },
+                           [&] { return dnpeff_fit_loss(f, reference_loss, true_loss); }, steps_ms);
+  unsigned long long* words = nullptr;
+  DN_TRY(host_words(&words));
+  const double* out = reinterpret_cast<double*>(words);
+  f->whh_valid = true;
+  DN_TRY(launch_fit_steps(f->n, f->r, f->W, f->HH, f->AH, f->eps, n_steps, f->WHH, reinterpret_cast<double*>(words)));
+  DN_HIP(hipStreamSynchronize(stream()));
+  double sums[3] = {out[0], out[1], out[2]}, ticks = out[3];
+  for (int64_t q = 1; q < fit_loss_parts(f->n); q++) {
+    for (int k = 0; k < 3; k++) sums[k] += out[4 * q + k];
+    ticks = std::max(ticks, out[4 * q + 3]);
+  }
+  if (true_loss) *true_loss = std::sqrt(f->sq_norm_A + sums[1] - 2.0 * sums[0]);
+  if (reference_loss) *reference_loss = std::sqrt(f->sq_norm_A + sums[2] - 2.0 * sums[0]);
+  return ticks_to_ms(ticks, steps_ms);
 }
 
 DN_API int dnpeff_fit_get_W(dnpeff_fit* f, float* W_nr) {

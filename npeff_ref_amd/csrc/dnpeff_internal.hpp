@@ -196,8 +196,11 @@ int launch_copy_rows(int64_t rows, int w, const float* in, int ldi, float* out, 
 // ---- fixed-H learner (fit.hip) ----
 bool fit_steps_supported(int64_t n, int r);
 int64_t fit_loss_parts(int64_t n);  // 3 doubles each in launch_fit_loss's partials
+// sums (pinned, or NULL): 4 doubles per workgroup (fit_loss_parts), the three of launch_fit_loss after the steps and the
+// ticks of wall_clock64() that these took; only where fit_loss_with_steps.
+bool fit_loss_with_steps(int64_t n, int n_steps);
 int launch_fit_steps(int64_t n, int r, float* W, const float* G, const float* AH, float eps, int n_steps,
-                     float* WHH);
+                     float* WHH, double* sums);
 // out3 (device or pinned) = <AH, W>, <W G, W>, <WHH, W> (WHH may be NULL: 0)
 int launch_fit_loss(int64_t n, int r, const float* W, const float* G, const float* AH, const float* WHH,
                     double* partials, double* out3);

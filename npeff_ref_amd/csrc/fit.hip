@@ -66,13 +66,44 @@ struct FitTile {
   }
 };
 
-// n_steps updates of W in place; WHH receives W G of the W before the last of them.
+// <A H^T, W>, <W G, W> and <WHH, W> of a lane's entries, in fp64: to the workgroup's three sums.
 template <int RP>
+__device__ inline void fit_sums(const FitTile<RP>& t, const float (&x)[2][4], const float (&ah)[2][4], const acc4 (&d)[2],
+                                const acc4 (&wh)[2], double (&red)[RP / 32][3], double* __restrict__ out) {
+  double s[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+  for (int b = 0; b < 2; b++)
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+      s[0] += (double)ah[b][v] * (double)x[b][v];
+      s[1] += (double)d[b][v] * (double)x[b][v];
+      s[2] += (double)wh[b][v] * (double)x[b][v];
+    }
+#pragma unroll
+  for (int k = 0; k < 3; k++) {
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) s[k] += __shfl_xor(s[k], off);
+    if (t.lane == 0) red[t.wave][k] = s[k];
+  }
+  __syncthreads();
+  if (threadIdx.x < 3) {
+    double sum = 0.0;
+    for (int w = 0; w < RP / 32; w++) sum += red[w][threadIdx.x];
+    out[threadIdx.x] = sum;
+  }
+}
+
+// n_steps updates of W in place; WHH receives W G of the W before the last of them.  LOSS: the sums of k_fit_loss
+// after them, bit for bit, and the ticks that the steps took, four numbers per workgroup straight to pinned memory:
+// what the loss reads is at hand here, and a launch and a wait between the two are saved (a fit of 100 x 20 in 25 steps: 64 us,
+// 86 before).
+template <int RP, bool LOSS>
 __global__ void __launch_bounds__(2 * RP)
     k_fit_steps(float* __restrict__ W, const float* __restrict__ G, const float* __restrict__ AH, float eps,
-                int64_t n, int r, int n_steps, float* __restrict__ WHH) {
+                int64_t n, int r, int n_steps, float* __restrict__ WHH, double* __restrict__ sums) {
   using T = FitTile<RP>;
   __shared__ __align__(16) float buf[2][FIT_ROWS * T::LD];
+  const long long start = LOSS ? wall_clock64() : 0;
   T t;
   t.init(G, r);
   const int64_t row0 = (int64_t)blockIdx.x * FIT_ROWS;
@@ -117,6 +148,20 @@ __global__ void __launch_bounds__(2 * RP)
         W[at[b][v]] = x[b][v];
         WHH[at[b][v]] = d[b][v];
       }
+  if constexpr (LOSS) {
+    __shared__ double red[RP / 32][3];
+    const long long ticks = wall_clock64() - start;
+    double* out = sums + (int64_t)blockIdx.x * 4;
+    acc4 now[2];
+    t.product(buf[n_steps & 1], now);
+#pragma unroll
+    for (int b = 0; b < 2; b++)
+#pragma unroll
+      for (int v = 0; v < 4; v++)
+        if (!ok[b][v]) ah[b][v] = d[b][v] = 0.0f;
+    fit_sums<RP>(t, x, ah, now, d, red, out);
+    if (threadIdx.x == 0) out[3] = (double)ticks;
+  }
 }
 
 // <A H^T, W>, <W G, W> and (where WHH is given) <WHH, W> of a workgroup's rows, in fp64.
@@ -130,7 +175,8 @@ __global__ void __launch_bounds__(2 * RP)
   T t;
   t.init(G, r);
   const int64_t row0 = (int64_t)blockIdx.x * FIT_ROWS;
-  float x[2][4], ah[2][4], wh[2][4];
+  float x[2][4], ah[2][4];
+  acc4 wh[2];
 #pragma unroll
   for (int b = 0; b < 2; b++)
 #pragma unroll
@@ -146,27 +192,7 @@ __global__ void __launch_bounds__(2 * RP)
   __syncthreads();
   acc4 d[2];
   t.product(buf, d);
-  double s[3] = {0.0, 0.0, 0.0};
-#pragma unroll
-  for (int b = 0; b < 2; b++)
-#pragma unroll
-    for (int v = 0; v < 4; v++) {
-      s[0] += (double)ah[b][v] * (double)x[b][v];
-      s[1] += (double)d[b][v] * (double)x[b][v];
-      s[2] += (double)wh[b][v] * (double)x[b][v];
-    }
-#pragma unroll
-  for (int k = 0; k < 3; k++) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) s[k] += __shfl_xor(s[k], off);
-    if (t.lane == 0) red[t.wave][k] = s[k];
-  }
-  __syncthreads();
-  if (threadIdx.x < 3) {
-    double sum = 0.0;
-    for (int w = 0; w < RP / 32; w++) sum += red[w][threadIdx.x];
-    partials[(int64_t)blockIdx.x * 3 + threadIdx.x] = sum;
-  }
+  fit_sums<RP>(t, x, ah, d, wh, red, partials + (int64_t)blockIdx.x * 3);
 }
 
 // out[k] = sum of the workgroups' k-th sums, in a fixed order
@@ -194,16 +220,19 @@ static void fit_dispatch(int r, F&& f) {
   else f(std::integral_constant<int, 256>{});
 }
 
+constexpr int FIT_STEPS_MAX = 256;  // per launch: 256 steps are about a millisecond per 4,096 rows at r = 256
+bool fit_loss_with_steps(int64_t n, int n_steps) { return n_steps >= 1 && n_steps <= FIT_STEPS_MAX && 4 * fit_loss_parts(n) <= HOST_WORDS; }
+
 int launch_fit_steps(int64_t n, int r, float* W, const float* G, const float* AH, float eps, int n_steps,
-                     float* WHH) {
-  // (a launch of many steps would keep the device from everything else for long: 256 steps are about a
-  // millisecond per 4,096 rows at r = 256)
-  for (int done = 0; done < n_steps; done += 256) {
-    const int now = n_steps - done < 256 ? n_steps - done : 256;
+                     float* WHH, double* sums) {
+  const dim3 grid((unsigned)ceil_div(n, FIT_ROWS));
+  // (a launch of many steps would keep the device from everything else for long)
+  for (int done = 0; done < n_steps; done += FIT_STEPS_MAX) {
+    const int now = n_steps - done < FIT_STEPS_MAX ? n_steps - done : FIT_STEPS_MAX;
     fit_dispatch(r, [&](auto rp) {
       constexpr int RP = decltype(rp)::value;
-      hipLaunchKernelGGL(k_fit_steps<RP>, dim3((unsigned)ceil_div(n, FIT_ROWS)), dim3(2 * RP), 0, stream(), W, G,
-                         AH, eps, n, r, now, WHH);
+      if (sums) hipLaunchKernelGGL((k_fit_steps<RP, true>), grid, dim3(2 * RP), 0, stream(), W, G, AH, eps, n, r, now, WHH, sums);
+      else hipLaunchKernelGGL((k_fit_steps<RP, false>), grid, dim3(2 * RP), 0, stream(), W, G, AH, eps, n, r, now, WHH, sums);
     });
     DN_LAUNCH_CHECK();
   }

@@ -39,7 +39,9 @@ int fuw_launch_h(int wgs, const fused_plan& f, const int64_t* colptr, int r, con
 int fuw_launch_w(int wgs, int64_t n, int r, const int* n_base, const float* N, float* W, float eps, const float* gh,
                  float* gpart);
 
-// Whole runs in one workgroup's LDS (fused_small.hip): steps, or the two sums of the loss.
+// Whole runs in one workgroup's LDS (fused_small.hip): steps, then (loss: pinned, or NULL) the two sums of the loss
+// and the ticks of wall_clock64() that the steps took; FUSED_SMALL_STEPS at most where these are asked for.
+constexpr int FUSED_SMALL_STEPS = 1024;
 bool fused_small_fits(int64_t n, int64_t m, int64_t nnz, int r);
 int fused_small_launch(const dnpeff_csr* S, int r, float* W, float* H, float eps, int steps, double* loss);
 

@@ -4,7 +4,8 @@
 // At this size an iteration as launches (fused.hip) is three kernels of 3 to 5 us that wait for each other, and the loss
 // four more.  One workgroup of 16 waves that never leaves its LDS takes 9 us per iteration at 48 x 907 with 3,072
 // entries and r = 8, bound by the issue of its vector instructions (H update 4 us, A H^T and H^T H 3, the rest of W's
-// update and six barriers 2): ten iterations and the loss 126 us with the host's waits, 165 as launches.
+// update and six barriers 2): ten iterations and the loss 117 us with the host's wait, 131 with a launch of its own for the loss
+// and a wait in between, 165 as launches.
 // Rows of the factors lie in LDS with their components padded to a multiple of four; lane (l % 16, l / 16) takes
 // row l % 16 of a tile and its components 4 (l / 16) .. + 3, as the fp32 matrix instructions want their operands (see
 // fused.hip).  An entry is its value and the byte offset of the row that it multiplies.
@@ -26,7 +27,8 @@ static int64_t fs_bytes(int64_t n, int64_t m, int64_t nnz, int r) {
 
 // (A column is one chain of multiply-adds: no more than 128 rows.)  Where one compute unit is slower than the launches
 // the sizes are left to them: they take 145 to 160 us for ten iterations and the loss up to 128 rows, one workgroup some 47 + 0.050
-// m + 0.37 n + 0.0073 nnz (500 matrices of even and of Zipf columns, 6 us off on average).  One workgroup / launches: 63 / 149
+// m + 0.37 n + 0.0073 nnz (500 matrices of even and of Zipf columns, 6 us off on average; with the loss in a launch of its
+// own, 14 us less in the steps').  One workgroup / launches: 63 / 149
 // at 8 x 40, 131 / 168 at 48 x 368 with 3,072 entries, 125 / 150 at 64 x 1000 with 1,280, 147 / 149 with 3,200; past the line
 // 193 / 153 at 128 x 1000 with 6,400, 233 / 150 at 87 x 2966 with 435, 314 / 149 at 128 x 4000 with 2,560.
 bool fused_small_fits(int64_t n, int64_t m, int64_t nnz, int r) {
@@ -40,7 +42,7 @@ struct fs_args {
   const float *vals, *tvals;
   float *W, *H;
   float eps;
-  double* loss;  // (or NULL) <A H^T, W>, <W^T W, H^T H> after the steps
+  double* loss;  // (or NULL) <A H^T, W>, <W^T W, H^T H> after the steps, and the ticks that these took
 };
 
 // The sum over the 16 lanes of a DPP row, in all of them.
@@ -53,6 +55,7 @@ __device__ inline float fs_row_sum(float x) {
 }
 
 __global__ void __launch_bounds__(FS_THREADS) k_fs_steps(fs_args p) {
+  const long long start = wall_clock64();
   extern __shared__ __align__(16) char lds[];
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, l16 = lane & 15, g = lane >> 4;
   const int n = p.n, m = p.m, nnz = p.nnz, r = p.r, ld = (r + 3) / 4 * 4, quads = ld / 4;
@@ -202,6 +205,7 @@ __global__ void __launch_bounds__(FS_THREADS) k_fs_steps(fs_args p) {
     store(W, p.W, n);
   }
   if (p.loss) {
+    if (tid == 0) p.loss[2] = (double)(wall_clock64() - start);
     gram(H, m);
     product();
     __syncthreads();
@@ -238,7 +242,7 @@ int fused_small_launch(const dnpeff_csr* S, int r, float* W, float* H, float eps
   const int bytes = (int)fs_bytes(S->n_rows, S->n_cols, S->nnz, r);
   DN_HIP(hipFuncSetAttribute((const void*)k_fs_steps, hipFuncAttributeMaxDynamicSharedMemorySize, (int)FS_LDS));
   do {  // (a launch of very many steps would keep a compute unit for long)
-    p.steps = std::min(steps, 1024);
+    p.steps = std::min(steps, FUSED_SMALL_STEPS);
     hipLaunchKernelGGL(k_fs_steps, dim3(1), dim3(FS_THREADS), (size_t)bytes, stream(), p);
     DN_LAUNCH_CHECK();
     steps -= p.steps;

@@ -7,6 +7,7 @@ to ~0 make an element-wise relative error meaningless."""
 
 import numpy as np
 import pytest
+import scipy.sparse as sp
 
 import npeff_ref_amd as d
 from conftest import random_csr
@@ -506,3 +507,58 @@ def test_two_contexts_of_different_rank_on_one_matrix():
     big.close()
     small.close()
     A.close()
+
+
+@pytest.mark.parametrize("n,m,per_row,r,steps", [(48, 900, 40, 8, 10), (1, 40, 5, 3, 1), (48, 900, 40, 8, 1030),
+                                                 (300, 20000, 90, 24, 3), (90, 3000, 60, 130, 2)])
+def test_nmf_step_loss_is_a_step_and_a_loss(n, m, per_row, r, steps):
+    """Steps and loss in one launch (small matrices, up to 1024 steps), or one after the other."""
+    rng = np.random.default_rng(n + r)
+    cols = np.stack([rng.choice(m, per_row, replace=False) for _ in range(n)]).astype(np.int32)
+    vals = rng.lognormal(-1, 1, cols.shape).astype(np.float32)
+    got = []
+    for together in (False, True):
+        A = d.Csr.from_pef(cols, vals, m)
+        nmf = d.MuNmf(A, d.MuNmfParams(rank=r, max_iters=steps, log_every=steps))
+        nmf.initialize()
+        if together:
+            (done, loss, ms), = nmf.run(log=lambda s: None)
+            assert done == steps and 0.0 < ms < 1e3
+        else:
+            nmf.step(steps)
+            loss = nmf.computeUncachedLoss()
+        again = nmf.computeUncachedLoss()
+        nmf.step(1)
+        got.append((loss, again, nmf.computeUncachedLoss(), nmf.loadWToHostSync(), nmf.loadHToHostSync()))
+        nmf.close()
+        A.close()
+    for a, b in zip(*got):  # (one row: the model is exact, and the sum under the root may end below zero in both)
+        np.testing.assert_array_equal(a, b)
+
+
+@pytest.mark.parametrize("n,r,steps", [(1, 1, 1), (100, 20, 25), (33, 250, 256), (33, 100, 257), (2048, 64, 2), (2049, 33, 2),
+                                       (60, 300, 3)])
+def test_fit_step_loss_is_a_step_and_a_loss(n, r, steps):
+    """Sums from the launch of the steps (2048 rows and 256 steps at most, rank 256 at most) or from one of their own."""
+    rng = np.random.default_rng(n + r)
+    m = 2000
+    cols = np.stack([rng.choice(m, 20, replace=False) for _ in range(n)]).astype(np.int32)
+    A = d.Csr.from_pef(cols, rng.lognormal(-1, 1, cols.shape).astype(np.float32), m)
+    Hd = rng.random((r, m), dtype=np.float32) * (rng.random((r, m)) < 0.05)
+    Hs = sp.csr_matrix(Hd)
+    H = d.Csr.from_host(Hs.indptr, Hs.indices, Hs.data, m)
+    got = []
+    for together in (False, True):
+        fit = d.Learner(A, H, d.LearnerParams(max_iters=steps, log_every_n_steps=steps))
+        if together:
+            (done, ref, true, ms), = fit.Run(log=lambda s: None)
+            assert done == steps and 0.0 < ms < 1e3
+            losses = (ref, true)
+        else:
+            fit.initialize()
+            fit.step(steps)
+            losses = fit.losses()
+        got.append((losses, fit.losses(), fit.GetOnHost_W()))
+        fit.close()
+    for a, b in zip(*got):
+        assert np.array_equal(a, b)
