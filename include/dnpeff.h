@@ -332,8 +332,7 @@ int dnpeff_nmf_update_H(dnpeff_nmf* nmf);
  * device_contexts1.h:337-354) through the same trace identity. */
 int dnpeff_nmf_loss(dnpeff_nmf* nmf, double* out);
 /* dnpeff_nmf_step and dnpeff_nmf_loss of what it leaves, in one call, and in *steps_ms the time of the
- * steps alone (the figure that nmf1.h:186-200 logs): their time on the device where steps and
- * loss are one launch, the host's clock around them otherwise. */
+ * steps alone, by the device's clock (the figure that nmf1.h:186-200 logs). */
 int dnpeff_nmf_step_loss(dnpeff_nmf* nmf, int n_steps, double* loss, double* steps_ms);
 
 /* The three terms of the loss: ||A||^2, <H,(W^T W)H>, <W^T A,H>. */

@@ -906,15 +906,25 @@ static int ticks_to_ms(double ticks, double* ms) {
   return 0;
 }
 
-// steps(), the host's clock on it (nothing else in hand before and after), then loss()
+namespace dn {
+__global__ void __launch_bounds__(64) k_stamp(unsigned long long* out) {
+  if (threadIdx.x == 0) *out = (unsigned long long)wall_clock64();
+}
+}  // namespace dn
+
+// steps(), then loss(), which waits for the stream; the steps lie between two stamps of the device's clock.  (The host's clock
+// asks for a wait in between: the four launches of a loss of the fused step then start on an idle device, one by one.  Ten
+// iterations at 512 x 431 k, r = 16, and a loss: 547 us, 552 with the wait.)
 template <class Steps, class Loss>
 static int steps_then_loss(Steps steps, Loss loss, double* ms) {
-  DN_TRY(dnpeff_sync());
-  const auto t0 = std::chrono::steady_clock::now();
+  unsigned long long* stamps = nullptr;
+  DN_TRY(host_stamps(&stamps));
+  hipLaunchKernelGGL(k_stamp, dim3(1), dim3(64), 0, stream(), stamps);
   DN_TRY(steps());
-  DN_TRY(dnpeff_sync());
-  *ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
-  return loss();
+  hipLaunchKernelGGL(k_stamp, dim3(1), dim3(64), 0, stream(), stamps + 1);
+  DN_LAUNCH_CHECK();
+  DN_TRY(loss());
+  return ticks_to_ms((double)(stamps[1] - stamps[0]), ms);
 }
 
 DN_API int dnpeff_nmf_step_loss(dnpeff_nmf* h, int n_steps, double* loss, double* steps_ms) {

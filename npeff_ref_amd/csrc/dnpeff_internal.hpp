@@ -80,6 +80,8 @@ hipError_t copy_down_parts(const copy_part* parts, int n_parts);
 inline hipError_t copy_down_parts(std::initializer_list<copy_part> parts) { return copy_down_parts(parts.begin(), (int)parts.size()); }
 constexpr int HOST_WORDS = 512;
 int host_words(unsigned long long** out);  // HOST_WORDS pinned words of the calling thread
+constexpr int HOST_STAMPS = 2;
+int host_stamps(unsigned long long** out);  // HOST_STAMPS more, for the clock around calls that use those
 
 // One of the pinned buffers that short copies go through, for a kernel that writes a call's results there.  p() is NULL
 // where none could be had.  Whoever gives it back has waited for what writes to it.

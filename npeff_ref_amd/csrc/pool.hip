@@ -525,9 +525,14 @@ hipError_t copy_down(void* dst_host, const void* src_dev, size_t bytes) {
 int host_words(unsigned long long** out) {
   static thread_local unsigned long long* words = nullptr;
   if (!words) {
-    DN_HIP(hipHostMalloc((void**)&words, HOST_WORDS * sizeof(unsigned long long), hipHostMallocDefault));
+    DN_HIP(hipHostMalloc((void**)&words, (HOST_WORDS + HOST_STAMPS) * sizeof(unsigned long long), hipHostMallocDefault));
   }
   *out = words;
+  return 0;
+}
+int host_stamps(unsigned long long** out) {
+  DN_TRY(host_words(out));
+  *out += HOST_WORDS;
   return 0;
 }
 
