@@ -198,13 +198,14 @@ __device__ inline void topk_sweep(const float* __restrict__ xr, int64_t count, F
       const int64_t b = base + 1024 * u;
       if (VEC4) {
         const int64_t i = b + 4 * t;
-        const float4 q = *reinterpret_cast<const float4*>(xr + (i < count ? i : 0));
+        typedef float f4 __attribute__((ext_vector_type(4)));
+        const f4 q = __builtin_nontemporal_load(reinterpret_cast<const f4*>(xr + (i < count ? i : 0)));
         v[u][0] = q.x; v[u][1] = q.y; v[u][2] = q.z; v[u][3] = q.w;
       } else {
 #pragma unroll
         for (int e = 0; e < 4; e++) {
           const int64_t i = b + t + 256 * e;
-          v[u][e] = xr[i < count ? i : 0];
+          v[u][e] = __builtin_nontemporal_load(xr + (i < count ? i : 0));
         }
       }
     }
