@@ -30,7 +30,8 @@ __device__ inline float bcast_f(float v, int src_lane) {
 // Any rank: lane l holds components l + 64 t; every entry is applied by the whole wave.
 template <int VPL>
 struct GatherDword {
-  static constexpr int UNR = VPL <= 2 ? 8 : VPL <= 4 ? 4 : 2, FEW = UNR;
+  // (runs of hundreds of entries are a chain of trips: A H^T of 43 x 3022, rank 55, 37 -> 30 us with twice as many in flight)
+  static constexpr int FEW = VPL <= 2 ? 8 : VPL <= 4 ? 4 : 2, UNR = 2 * FEW;
   float acc[VPL];
   bool ok[VPL];
   int lane;
@@ -831,7 +832,7 @@ __global__ void __launch_bounds__(256)
 }
 
 // Short and medium columns (at most SPMM_T_LONG entries), rank a multiple of 4: a wave owns
-// SPMM_T_COLS consecutive columns and each of its 64/LPR lane groups walks whole columns on its
+// `cols` consecutive columns (at most SPMM_T_COLS) and each of its 64/LPR lane groups walks whole columns on its
 // own, so that a wave works on several columns at once, no cross-lane reduction is needed and
 // the column offsets of all its columns come from one coalesced load.  A group reads up to LPR
 // (row, value) pairs of its column with one load, hands them out with lane shuffles inside the
@@ -846,7 +847,7 @@ template <int LPR, int T, bool FULL, bool SMALL, bool PAST>
 __global__ void __launch_bounds__(256)
     k_spmm_t_grouped(const int64_t* __restrict__ colptr, const int32_t* __restrict__ rowind,
                      const float* __restrict__ tvals, int64_t m, int r, int n_slices,
-                     const float* __restrict__ W, float* __restrict__ Tout) {
+                     const float* __restrict__ W, float* __restrict__ Tout, int cols) {
   constexpr int G = 64 / LPR;
   constexpr int UNR = T >= 4 ? 1 : T == 2 ? 2 : 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
@@ -856,16 +857,16 @@ __global__ void __launch_bounds__(256)
   const int slice = blockIdx.x % n_slices;
   W += slice * (4 * LPR * T);
   Tout += slice * (4 * LPR * T);
-  const int64_t j0 = ((int64_t)(blockIdx.x / n_slices) * 4 + wave) * SPMM_T_COLS;
+  const int64_t j0 = ((int64_t)(blockIdx.x / n_slices) * 4 + wave) * cols;
   if (j0 >= m) return;
   bool ok[T];
 #pragma unroll
   for (int t = 0; t < T; t++) ok[t] = FULL || 4 * (sub + LPR * t) < r;
   const unsigned r4 = 4u * (unsigned)r, sub16 = 16u * (unsigned)sub;
 
-  // colptr[j0 + lane] for lane <= SPMM_T_COLS, as two 32-bit halves for the shuffles
+  // colptr[j0 + lane] for lane <= cols, as two 32-bit halves for the shuffles
   const int64_t jc = j0 + lane < m ? j0 + lane : m;
-  const int64_t cp = lane <= SPMM_T_COLS ? colptr[jc] : 0;
+  const int64_t cp = lane <= cols ? colptr[jc] : 0;
   const int cp_lo = (int)(uint32_t)(cp & 0xffffffffLL), cp_hi = (int)(cp >> 32);
 
   // The (row, value) pairs of a round's columns are requested one round ahead, so that their
@@ -877,7 +878,7 @@ __global__ void __launch_bounds__(256)
     p0 = ((int64_t)__shfl(cp_hi, jl & 63) << 32) | (uint32_t)__shfl(cp_lo, jl & 63);
     const int64_t p1 =
         ((int64_t)__shfl(cp_hi, (jl + 1) & 63) << 32) | (uint32_t)__shfl(cp_lo, (jl + 1) & 63);
-    active = jl < SPMM_T_COLS && j < m && (p1 - p0) <= SPMM_T_LONG;  // longer: k_spmm_t_long
+    active = jl < cols && j < m && (p1 - p0) <= SPMM_T_LONG;  // longer: k_spmm_t_long
     len = active ? (int)(p1 - p0) : 0;
     e_i = 0;
     e_v = 0.0f;
@@ -892,7 +893,7 @@ __global__ void __launch_bounds__(256)
   float nx_v;
   request(0, nx_p0, nx_len, nx_active, nx_i, nx_v);
 
-  for (int round = 0; round * G < SPMM_T_COLS; round++) {
+  for (int round = 0; round * G < cols; round++) {
     const int64_t j = j0 + round * G + grp;
     const int64_t p0 = nx_p0;
     const int len = nx_len;
@@ -1798,14 +1799,19 @@ static int launch_spmm_t_sparse(const dnpeff_csr* A, int r, const float* W_nr, f
   const bool grouped = aligned && r % 4 == 0 && slice_ok;
   const bool w_small = (double)A->n_rows * r * 4.0 < 4.0e9;  // 32-bit offsets into W
   if (grouped) {
-    dim3 gg((unsigned)(ceil_div(m, 4 * SPMM_T_COLS) * n_slices));
     const int w4 = width / 4;
+    // Fewer columns per wave where 32 leave fewer than 32 workgroups per CU: a wave's columns are one chain of trips.
+    // 32 / now, us: 111 / 92 at 200k columns with 22 entries each, rank 128, 101 / 64 at 60k, rank 100, 19 / 8 at 20k, rank
+    // 100; the same (0.98 to 1.01) at 600k and 1.5M.  Lines of 2, 8 and 16 workgroups are behind by up to 1.2.
+    int cols = SPMM_T_COLS;
+    while (cols > 4 && cols > 64 / w4 && ceil_div(m, 4 * cols) * n_slices < 32 * n_cus()) cols /= 2;
+    dim3 gg((unsigned)(ceil_div(m, 4 * cols) * n_slices));
     // Slices of a large W stay in the L2s, and a T that the memory-side cache does not hold goes past both: an
     // iteration at 20 000 x 211 M, rank 256, tiles of 768 MiB, 667.5 -> 662.8 ms.
     const bool past = n_slices > 1 && m * r * (int64_t)sizeof(float) > ((int64_t)256 << 20);
 #define DN_GROUPED3(LPR, T_, FULL, SMALL, PAST)                                                      \
   hipLaunchKernelGGL((k_spmm_t_grouped<LPR, T_, FULL, SMALL, PAST>), gg, block, 0, stream(), colptr, \
-                     A->rowind, A->tvals, m, r, n_slices, W_nr, T)
+                     A->rowind, A->tvals, m, r, n_slices, W_nr, T, cols)
 #define DN_GROUPED2(LPR, T_, FULL, SMALL)              \
   do {                                                 \
     if (past) DN_GROUPED3(LPR, T_, FULL, SMALL, true); \

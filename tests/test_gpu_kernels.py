@@ -280,6 +280,39 @@ def test_spmm_t_component_slices(slices, r, tune):
     A.close()
 
 
+@pytest.mark.parametrize("r", [4, 16, 20, 36, 64, 100, 128, 260])
+def test_spmm_t_columns_per_wave(r):
+    """Waves with 32 columns (1.1 million of them), with 4 to 16 (parts of them, down to one), and columns of up to 70
+    entries: a column is the same sum, bit for bit, and right."""
+    rng = np.random.default_rng(r)
+    n, m = 70, 1_100_000
+    at = rng.integers(0, n * m, 900_000)
+    at = np.unique(np.concatenate([at, (np.arange(n)[:, None] * m + np.arange(0, 300, 7)).ravel()]))
+    rp = np.searchsorted(at, np.arange(n + 1) * m).astype(np.int64)
+    ci, va = (at % m).astype(np.int32), rng.random(at.size, dtype=np.float32)
+    W = rng.random((n, r), dtype=np.float32)
+    A = d.Csr.from_host(rp, ci, va, m)
+    dW, dT = d.DeviceArray.from_numpy(W), d.DeviceArray((m, r))
+    d.op_spmm_t(A, r, dW, dT)
+    T = dT.numpy()
+    for c0, c1 in ((0, m), (0, 1), (3, 130), (0, 4097), (100_000, 300_001), (m - 700_000, m)):
+        part = d.DeviceArray((c1 - c0, r))
+        d.binding._check(d.lib.dnpeff_op_spmm_t_tile(A._h, r, dW.ptr, c0, c1, part.ptr))
+        assert np.array_equal(part.numpy(), T[c0:c1]), (c0, c1)
+    want = sp.csr_matrix((va.astype(np.float64), ci, rp), (n, m))[:, :5000].T @ W.astype(np.float64)
+    assert np.abs(T[:5000] - want).max() <= 1e-6 * np.abs(want).max()  # (70 terms of one sign: 70 roundings at most)
+    A.close()
+
+
+@pytest.mark.parametrize("rows,r", [(1, 33), (31, 55), (32, 55), (33, 126), (257, 37), (3022, 55), (9001, 127), (5000, 130), (700, 333)])
+def test_gram_of_ranks_that_four_does_not_divide(rows, r):
+    rng = np.random.default_rng(rows + r)
+    X = rng.random((rows, r), dtype=np.float32)
+    G = d.DeviceArray((r, r))
+    d.op_gram(d.DeviceArray.from_numpy(X), G)
+    assert _rel(G.numpy(), X.astype(np.float64).T @ X.astype(np.float64)) < TOL
+
+
 def test_spmm_t_more_columns_than_one_pass_of_the_grid():
     """36M columns: more (column, slice) work items than workgroups in the capped grid, so every
     workgroup walks several column groups; columns without entries must come out as zeros."""
