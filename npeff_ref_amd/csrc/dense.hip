@@ -107,9 +107,39 @@ struct GramPipe {
   int r, ld, kb;
   int64_t k1;  // number of rows of X
   float4 stage[GRAM_STAGES][NVEC];
+  // Not VEC4: number threadIdx.x + THREADS (4 q + i) of a tile, single loads as far ahead; where it goes in the slot,
+  // or -1.  (Loaded when they were stored, seven trips per tile: 3022 rows, rank 55, 33 us, now 25.)
+  int place[VEC4 ? 1 : NVEC][4];
+
+  __device__ inline void init() {
+    if constexpr (!VEC4) {
+#pragma unroll
+      for (int q = 0; q < NVEC; q++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          const int e = threadIdx.x + THREADS * (4 * q + i);
+          place[q][i] = e < kb * r ? e / r * ld + gram_lds_col(e % r) : -1;
+        }
+    }
+  }
 
   __device__ inline void fetch(int st, int64_t kt) {
-    if (!VEC4) return;
+    if constexpr (!VEC4) {
+      const int64_t left = (k1 - kt) * r;
+      const float* p = X + kt * r;
+#pragma unroll
+      for (int q = 0; q < NVEC; q++) {
+        float v[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          const int e = threadIdx.x + THREADS * (4 * q + i);
+          const bool ok = place[q][i] >= 0 && e < left;
+          v[i] = ok ? p[e] : 0.0f;
+        }
+        stage[st][q] = make_float4(v[0], v[1], v[2], v[3]);
+      }
+      return;
+    }
     const int r4 = r >> 2;
 #pragma unroll
     for (int q = 0; q < NVEC; q++) {
@@ -136,10 +166,12 @@ struct GramPipe {
         }
       }
     } else {
-      for (int e = threadIdx.x; e < kb * r; e += THREADS) {
-        const int64_t row = kt + e / r;
-        const int c = e % r;
-        slot[(e / r) * ld + gram_lds_col(c)] = row < k1 ? X[row * (int64_t)r + c] : 0.0f;
+#pragma unroll
+      for (int q = 0; q < NVEC; q++) {
+        const float v[4] = {stage[st][q].x, stage[st][q].y, stage[st][q].z, stage[st][q].w};
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+          if (place[q][i] >= 0) slot[place[q][i]] = v[i];
       }
     }
   }
@@ -208,6 +240,7 @@ __device__ inline void gram_stream(const float* __restrict__ X, int r, int kb, i
   GramPipe<NW, VEC4> pipe;
   const int ld = 128 * ((r + 127) / 128);
   pipe.X = X; pipe.r = r; pipe.ld = ld; pipe.kb = kb; pipe.k1 = rows;
+  pipe.init();
   const int64_t all_tiles = (rows + kb - 1) / kb;
   const int64_t n_tiles = all_tiles > slice ? (all_tiles - slice + n_slices - 1) / n_slices : 0;
   const int64_t k0 = (int64_t)slice * kb;         // first row of this slice's tile 0
@@ -361,7 +394,14 @@ __global__ void __launch_bounds__(256)
   const int64_t stride = (int64_t)n_pairs * 1024;
   const float* p = partials + e;
   double s = 0.0;
-  for (int64_t sl = 0; sl < slices; sl++) s += (double)p[sl * stride];
+  constexpr int U = 16;  // (slices under way: 77 of them 21 us one by one, now 5)
+  for (int64_t sl = 0; sl < slices; sl += U) {
+    float v[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) v[u] = p[(sl + u < slices ? sl + u : sl) * stride];
+#pragma unroll
+    for (int u = 0; u < U; u++) s += sl + u < slices ? (double)v[u] : 0.0;
+  }
   G[(int64_t)a * r + b] = (float)s;
   G[(int64_t)b * r + a] = (float)s;
 }
@@ -525,10 +565,23 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
   const int c0 = blockIdx.y * CW;
   const int kpad = 8 * nsteps;
 
-  for (int idx = threadIdx.x; idx < kpad * CW; idx += 256) {
-    const int k = idx / CW, c = idx % CW, gc = c0 + c;
-    const float v = (k < r && gc < r) ? G[(int64_t)k * r + gc] : 0.0f;
-    g_lds[(k * 32 + (c & 31)) * NB + (c >> 5)] = v;
+  // (sixteen numbers of a thread under way: of few rows this chain of trips was a third of the kernel; 3022 rows, rank 55: 21 ->
+  // 15 us)
+  constexpr int UG = 16;
+  for (int i0 = threadIdx.x; i0 < kpad * CW; i0 += UG * 256) {
+    float v[UG];
+#pragma unroll
+    for (int u = 0; u < UG; u++) {
+      const int idx = i0 + 256 * u, k = idx / CW, gc = c0 + idx % CW;
+      const bool ok = k < r && gc < r;  // (k < r: within the chunk too)
+      v[u] = G[ok ? (int64_t)k * r + gc : 0];
+      v[u] = ok ? v[u] : 0.0f;
+    }
+#pragma unroll
+    for (int u = 0; u < UG; u++) {
+      const int idx = i0 + 256 * u, k = idx / CW, c = idx % CW;
+      if (idx < kpad * CW) g_lds[(k * 32 + (c & 31)) * NB + (c >> 5)] = v[u];
+    }
   }
   __syncthreads();
 
