@@ -1548,6 +1548,18 @@ static int launch_xg_mu_nb(int64_t rows, int r, const float* X, const float* G, 
 #undef DN_XG
 }
 
+// Chunks of as many columns as keep their part of G in 128 KB of LDS, narrower where that leaves CUs without work: a wave of few
+// rows is one chain of matrix instructions (128 columns of r = 128: 256 of them, 7 us).  Every sum keeps its order.  The last rows
+// at 300 x 30k, r = 128: 18 -> 7.5 us.
+static int launch_xg_mu_chunks(int64_t rows, int r, const float* X, const float* G, const float* num, float eps, float* out,
+                               float* D_out) {
+  int nb = r <= 256 ? 4 : r <= 512 ? 2 : 1;
+  while (nb > 1 && ceil_div(rows, 128) * ceil_div(r, 32 * nb) < n_cus()) nb /= 2;
+  if (nb == 4) return launch_xg_mu_nb<4>(rows, r, X, G, num, eps, out, D_out);
+  if (nb == 2) return launch_xg_mu_nb<2>(rows, r, X, G, num, eps, out, D_out);
+  return launch_xg_mu_nb<1>(rows, r, X, G, num, eps, out, D_out);
+}
+
 // ---------------------------------------------------------------------------
 // The same update for r = 128 that also accumulates the Gram matrix of its OUTPUT, so that the
 // next A-side update does not have to read the new factor again: out = X * num / (X G + eps),
@@ -2071,7 +2083,7 @@ int launch_xg_mu_gram(int64_t rows, const float* X, const float* G, const float*
   const int64_t head = tiles * tile_rows;
   if (head < rows) {
     const int64_t off = head * r;
-    DN_TRY(launch_xg_mu_nb<4>(rows - head, r, X + off, G, num + off, eps, out + off, nullptr));
+    DN_TRY(launch_xg_mu_chunks(rows - head, r, X + off, G, num + off, eps, out + off, nullptr));
     DN_TRY(launch_gram(rows - head, r, out + off, G_tmp, gram_ws));
     hipLaunchKernelGGL(k_add_inplace, dim3(r * r / 256), dim3(256), 0, stream(), Gout, G_tmp, r * r);
     DN_LAUNCH_CHECK();
@@ -2119,8 +2131,8 @@ int launch_xg_mu(int64_t rows, int r, const float* X, const float* G, const floa
     }
     if (head == rows) return 0;
     const int64_t off = head * r;
-    return launch_xg_mu_nb<4>(rows - head, r, X + off, G, num + off, eps, out + off,
-                              D_out ? D_out + off : nullptr);
+    return launch_xg_mu_chunks(rows - head, r, X + off, G, num + off, eps, out + off,
+                               D_out ? D_out + off : nullptr);
   }
   if (r > 128 && r % 128 == 0 && aligned && ((uintptr_t)G % 16) == 0 &&
       (rows >= 256 || (rows_there >= ceil_div(rows, 128) * 128 && use_split_bf16())) &&
@@ -2129,10 +2141,7 @@ int launch_xg_mu(int64_t rows, int r, const float* X, const float* G, const floa
       return launch_xg_mu_tile_b16(rows, r, X, G, num, eps, out, D_out, rows_there);
     return launch_xg_mu_tile(rows, r, X, G, num, eps, out, D_out);
   }
-  // widest column chunk whose slice of G fits 128 KB of LDS
-  if (r <= 256) return launch_xg_mu_nb<4>(rows, r, X, G, num, eps, out, D_out);
-  if (r <= 512) return launch_xg_mu_nb<2>(rows, r, X, G, num, eps, out, D_out);
-  return launch_xg_mu_nb<1>(rows, r, X, G, num, eps, out, D_out);
+  return launch_xg_mu_chunks(rows, r, X, G, num, eps, out, D_out);
 }
 
 // ---------------------------------------------------------------------------

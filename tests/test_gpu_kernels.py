@@ -131,6 +131,22 @@ def test_xg_mu(rows, r):
     assert np.array_equal(dnum.numpy(), out1)
 
 
+@pytest.mark.parametrize("r", [5, 50, 100, 130, 300])
+def test_xg_mu_chunks_of_columns(r):
+    """Few rows take narrower chunks of columns than many: the same bits."""
+    rng = np.random.default_rng(r)
+    rows, eps = 33_000, 1e-6
+    X, num = rng.random((rows, r), dtype=np.float32), rng.random((rows, r), dtype=np.float32)
+    G = d.DeviceArray.from_numpy((X[:500].T @ X[:500]).astype(np.float32))
+    outs = []
+    for n in (rows, 5000, 129, 1):
+        out = d.DeviceArray((n, r))
+        d.op_xg_mu(d.DeviceArray.from_numpy(X[:n]), G, d.DeviceArray.from_numpy(num[:n]), eps, out)
+        outs.append(out.numpy())
+    for o in outs[1:]:
+        assert np.array_equal(o, outs[0][:len(o)])
+
+
 @pytest.mark.parametrize("rows,r", [(128, 256), (4100, 256), (40000, 256), (3000, 512), (700, 1024), (1001, 384),
                                     (400000, 256)])
 def test_xg_mu_tiles_with_two_and_three_workgroups_per_cu(rows, r, tune):
