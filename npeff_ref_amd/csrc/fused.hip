@@ -954,6 +954,11 @@ int fused_tiles_build(dnpeff_csr* S, int r) {
   // entries, r = 90: 57 against 63 ms; at r = 20 smaller tiles are the better ones, 16.4 against 18.6).
   int64_t most = 16 * tc;
   if (r > FUSED_NARROW_RANK && r <= FUSED_MAX_RANK) most = std::max<int64_t>(most, S->nnz / (16 * (int64_t)n_cus()));
+  // Above rank 128 (A^T W alone, a wave per eighth of a tile's columns) as few as 64 where the tiles leave compute units without
+  // work: ten iterations at 119 x 5.2k, rank 460, 2.40 -> 2.30 ms, 60 x 6k, rank 256, 1.62 -> 1.53.  Everywhere it costs
+  // 1 to 2 % from 150 x 159k and 200 x 46k on.
+  if (r > FUSED_MAX_RANK && S->n_cols < (int64_t)tc * 2 * n_cus())
+    most = std::max<int64_t>(64, std::min<int64_t>(most, S->nnz / (8 * (int64_t)n_cus())));
   return fused_tiles_make(S, tc, most, r > FUSED_MAX_RANK ? SPMM_T_LONG : INT64_MAX, false);
 }
 
