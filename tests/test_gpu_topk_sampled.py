@@ -73,10 +73,11 @@ def test_threshold_and_largest_entry_close_together(count, k, kind):
 
 
 @pytest.mark.parametrize("kind,n,count,k", [("lognormal", 2, 600_000, 65_536), ("lognormal", 1, 700_000, 262_100),
-                                            ("lognormal", 3, 600_001, 300_000), ("few", 2, 524_288, 5000),
+                                            ("lognormal", 10, 600_001, 38_482), ("lognormal", 1, 700_000, 524_280),
+                                            ("lognormal", 1, 700_000, 524_288), ("lognormal", 3, 600_001, 300_000), ("few", 2, 524_288, 5000),
                                             ("hidden", 1, 600_000, 900), ("uniform", 1, 9, 1)])
 def test_results_for_the_host_equal_those_on_the_device(kind, n, count, k):
-    """One pinned buffer holds them (the second case just), or not, or the sample's threshold does not serve."""
+    """One pinned buffer holds them (the second case just), or two (the fourth just), or not, or the sample's threshold does not serve."""
     x = d.DeviceArray.from_numpy(_values(kind, n, count, np.random.default_rng(k)))
     on_dev = [d.DeviceArray((n, k)), d.DeviceArray((n, k), np.int32), d.DeviceArray((n,))]
     d.binding._check(d.lib.dnpeff_topk_rows(n, count, k, x.ptr, *(a.ptr for a in on_dev)))
