@@ -631,7 +631,8 @@ struct topk_down {
   copy_part parts[3];
   int n_parts;
   pinned_buf pinned[BUFS];
-  std::vector<copy_part> of[BUFS];  // what goes through which
+  copy_part of[BUFS][3];  // what goes through which: of each array one piece at most
+  int n_of[BUFS] = {};
   bool queued = false;
 
   // Where two pinned buffers hold them, they go there behind the last kernel, before it is known whether that served;
@@ -647,7 +648,7 @@ struct topk_down {
           used = 0;
         }
         const size_t left = parts[q].bytes - off, room = (pinned_buf::BYTES - used) / 16 * 16, n = left < room ? left : room;
-        of[b].push_back({(char*)parts[q].dst + off, (const char*)parts[q].src + off, n});
+        of[b][n_of[b]++] = {(char*)parts[q].dst + off, (const char*)parts[q].src + off, n};
         used += gather_room(n);
         off += n;
       }
@@ -655,7 +656,7 @@ struct topk_down {
       pinned[i].take();
       if (!pinned[i].p()) return 0;
     }
-    for (int i = 0; i <= b; i++) DN_HIP(gather_queue(of[i].data(), (int)of[i].size(), pinned[i].p()));
+    for (int i = 0; i <= b; i++) DN_HIP(gather_queue(of[i], n_of[i], pinned[i].p()));
     queued = true;
     constexpr size_t PAGE = 4096;
     for (int q = 0; q < n_parts; q++) {
@@ -666,7 +667,7 @@ struct topk_down {
     return 0;
   }
   void take() {
-    for (int i = 0; i < BUFS; i++) gather_take(of[i].data(), (int)of[i].size(), pinned[i].p());
+    for (int i = 0; i < BUFS; i++) gather_take(of[i], n_of[i], pinned[i].p());
   }
 };
 
@@ -859,7 +860,7 @@ DN_API int dnpeff_topk_rows_host(int64_t n_rows, int64_t count, int64_t k, const
   DN_TRY(idx.alloc((int64_t)n));
   if (norms_host) DN_TRY(norms.alloc(n_rows));
   topk_down down{{{vals_host, vals.p, 4 * n}, {idx_host, idx.p, 4 * n}, {norms_host, norms.p, 4 * (size_t)n_rows}},
-                 norms_host ? 3 : 2, {}, {}};
+                 norms_host ? 3 : 2};
   DN_TRY(topk_of_rows(n_rows, count, k, x, vals.p, idx.p, norms.p, &down));
   if (n_rows == 0) return 0;
   if (down.queued) down.take();
