@@ -2,7 +2,7 @@
 //
 // W <- W * (A H^T) / (W (H H^T) + eps) works row by row, so a workgroup that holds 16 rows of W and
 // of A H^T and the whole of G = H H^T can do every step of the call without touching memory in
-// between: at r = 256 its registers hold G (32 columns per wave, 128 registers a lane), the 16 rows of W
+// between: at r = 256 its registers hold G (16 columns per wave, 64 registers a lane), the 16 rows of W
 // lie in LDS as the A operand of the next step (two buffers: one barrier per step) and, with A H^T, in
 // registers in the accumulator layout for the update itself.  fp32 matrix cores, as the rows are too
 // few for the split-operand kernels: 2,000 rows are 125 workgroups.  Bound by the matrix cores of the CUs
@@ -20,14 +20,18 @@ typedef float acc4 __attribute__((ext_vector_type(4)));
 constexpr int FIT_ROWS = 16;
 
 // G in registers and the product of a workgroup's 16 rows (in LDS) with it.  RP: the rank padded to a
-// multiple of 32; wave w owns columns 32 w .. 32 w + 31 as two blocks of 16.  Lane (i = l % 16,
+// multiple of 32; wave w owns columns 16 w .. 16 w + 15.  Lane (i = l % 16,
 // kg = l / 16) reads X[row i][16 q + 4 kg .. + 3] with one 16-byte LDS read and step s of the
 // group contracts component 16 q + 4 kg + s against the same row of G.
+//
+// A step is a chain (matrix instructions, division, LDS, barrier), so that half as many columns per wave, on twice as many
+// waves, make it shorter where few waves have the chip: 25 steps and the loss at 100 x 20, the whole fit, 61 -> 54 us, 489 x
+// 64 102 -> 90, 200 x 128 96 -> 91, 2000 x 256 (bound by the matrix cores) 265 -> 264.
 template <int RP>
 struct FitTile {
   static constexpr int LD = RP + 4;  // floats per row of X in LDS
-  static constexpr int Q = RP / 16;
-  float g[Q][2][4];
+  static constexpr int Q = RP / 16, WAVES = RP / 16;
+  float g[Q][4];
   int lane, wave, kg, l16;
 
   __device__ inline void init(const float* __restrict__ G, int r) {
@@ -38,20 +42,18 @@ struct FitTile {
 #pragma unroll
     for (int q = 0; q < Q; q++)
 #pragma unroll
-      for (int b = 0; b < 2; b++)
-#pragma unroll
-        for (int s = 0; s < 4; s++) {
-          const int k = 16 * q + 4 * kg + s, c = col(b);
-          const bool ok = k < r && c < r;
-          const float v = G[ok ? (int64_t)k * r + c : 0];
-          g[q][b][s] = ok ? v : 0.0f;
-        }
+      for (int s = 0; s < 4; s++) {
+        const int k = 16 * q + 4 * kg + s;
+        const bool ok = k < r && col() < r;
+        const float v = G[ok ? (int64_t)k * r + col() : 0];
+        g[q][s] = ok ? v : 0.0f;
+      }
   }
-  __device__ inline int col(int b) const { return 32 * wave + 16 * b + l16; }
+  __device__ inline int col() const { return 16 * wave + l16; }
   __device__ inline int row(int v) const { return 4 * kg + v; }  // of accumulator register v
 
-  __device__ inline void product(const float* buf, acc4 (&d)[2]) const {
-    d[0] = d[1] = acc4{0.0f, 0.0f, 0.0f, 0.0f};
+  __device__ inline acc4 product(const float* buf) const {
+    acc4 d = acc4{0.0f, 0.0f, 0.0f, 0.0f};
     const float* pa = buf + l16 * LD + 4 * kg;
 #pragma unroll
     for (int q = 0; q < Q; q++) {
@@ -59,26 +61,24 @@ struct FitTile {
 #pragma unroll
       for (int s = 0; s < 4; s++) {
         const float as = s == 0 ? a.x : s == 1 ? a.y : s == 2 ? a.z : a.w;
-#pragma unroll
-        for (int b = 0; b < 2; b++) d[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(as, g[q][b][s], d[b], 0, 0, 0);
+        d = __builtin_amdgcn_mfma_f32_16x16x4f32(as, g[q][s], d, 0, 0, 0);
       }
     }
+    return d;
   }
 };
 
 // <A H^T, W>, <W G, W> and <WHH, W> of a lane's entries, in fp64: to the workgroup's three sums.
 template <int RP>
-__device__ inline void fit_sums(const FitTile<RP>& t, const float (&x)[2][4], const float (&ah)[2][4], const acc4 (&d)[2],
-                                const acc4 (&wh)[2], double (&red)[RP / 32][3], double* __restrict__ out) {
+__device__ inline void fit_sums(const FitTile<RP>& t, const float (&x)[4], const float (&ah)[4], const acc4& d, const acc4& wh,
+                                double (&red)[FitTile<RP>::WAVES][3], double* __restrict__ out) {
   double s[3] = {0.0, 0.0, 0.0};
 #pragma unroll
-  for (int b = 0; b < 2; b++)
-#pragma unroll
-    for (int v = 0; v < 4; v++) {
-      s[0] += (double)ah[b][v] * (double)x[b][v];
-      s[1] += (double)d[b][v] * (double)x[b][v];
-      s[2] += (double)wh[b][v] * (double)x[b][v];
-    }
+  for (int v = 0; v < 4; v++) {
+    s[0] += (double)ah[v] * (double)x[v];
+    s[1] += (double)d[v] * (double)x[v];
+    s[2] += (double)wh[v] * (double)x[v];
+  }
 #pragma unroll
   for (int k = 0; k < 3; k++) {
 #pragma unroll
@@ -88,7 +88,7 @@ __device__ inline void fit_sums(const FitTile<RP>& t, const float (&x)[2][4], co
   __syncthreads();
   if (threadIdx.x < 3) {
     double sum = 0.0;
-    for (int w = 0; w < RP / 32; w++) sum += red[w][threadIdx.x];
+    for (int w = 0; w < FitTile<RP>::WAVES; w++) sum += red[w][threadIdx.x];
     out[threadIdx.x] = sum;
   }
 }
@@ -98,7 +98,7 @@ __device__ inline void fit_sums(const FitTile<RP>& t, const float (&x)[2][4], co
 // what the loss reads is at hand here, and a launch and a wait between the two are saved (a fit of 100 x 20 in 25 steps: 64 us,
 // 86 before).
 template <int RP, bool LOSS>
-__global__ void __launch_bounds__(2 * RP)
+__global__ void __launch_bounds__(4 * RP)
     k_fit_steps(float* __restrict__ W, const float* __restrict__ G, const float* __restrict__ AH, float eps,
                 int64_t n, int r, int n_steps, float* __restrict__ WHH, double* __restrict__ sums) {
   using T = FitTile<RP>;
@@ -107,58 +107,47 @@ __global__ void __launch_bounds__(2 * RP)
   T t;
   t.init(G, r);
   const int64_t row0 = (int64_t)blockIdx.x * FIT_ROWS;
-  float x[2][4], ah[2][4];
-  bool ok[2][4];
-  int64_t at[2][4];
+  float x[4], ah[4];
+  bool ok[4];
+  int64_t at[4];
 #pragma unroll
-  for (int b = 0; b < 2; b++)
+  for (int v = 0; v < 4; v++) {
+    ok[v] = row0 + t.row(v) < n && t.col() < r;
+    at[v] = ok[v] ? (row0 + t.row(v)) * r + t.col() : 0;
+    x[v] = W[at[v]];
+    ah[v] = AH[at[v]];
+  }
 #pragma unroll
-    for (int v = 0; v < 4; v++) {
-      ok[b][v] = row0 + t.row(v) < n && t.col(b) < r;
-      at[b][v] = ok[b][v] ? (row0 + t.row(v)) * r + t.col(b) : 0;
-      x[b][v] = W[at[b][v]];
-      ah[b][v] = AH[at[b][v]];
-    }
-#pragma unroll
-  for (int b = 0; b < 2; b++)
-#pragma unroll
-    for (int v = 0; v < 4; v++) {
-      if (!ok[b][v]) x[b][v] = 0.0f;  // (rows and columns of the padding stay zero)
-      buf[0][t.row(v) * T::LD + t.col(b)] = x[b][v];
-    }
+  for (int v = 0; v < 4; v++) {
+    if (!ok[v]) x[v] = 0.0f;  // (rows and columns of the padding stay zero)
+    buf[0][t.row(v) * T::LD + t.col()] = x[v];
+  }
   __syncthreads();
-  acc4 d[2];
+  acc4 d;
   for (int s = 0; s < n_steps; s++) {
-    t.product(buf[s & 1], d);
+    d = t.product(buf[s & 1]);
 #pragma unroll
-    for (int b = 0; b < 2; b++)
-#pragma unroll
-      for (int v = 0; v < 4; v++) {
-        const float q = ah[b][v] / (d[b][v] + eps);
-        x[b][v] = ok[b][v] ? x[b][v] * q : 0.0f;
-        buf[(s + 1) & 1][t.row(v) * T::LD + t.col(b)] = x[b][v];
-      }
+    for (int v = 0; v < 4; v++) {
+      const float q = ah[v] / (d[v] + eps);
+      x[v] = ok[v] ? x[v] * q : 0.0f;
+      buf[(s + 1) & 1][t.row(v) * T::LD + t.col()] = x[v];
+    }
     __syncthreads();  // (the buffer just read is written again one barrier from here)
   }
 #pragma unroll
-  for (int b = 0; b < 2; b++)
-#pragma unroll
-    for (int v = 0; v < 4; v++)
-      if (ok[b][v]) {
-        W[at[b][v]] = x[b][v];
-        WHH[at[b][v]] = d[b][v];
-      }
+  for (int v = 0; v < 4; v++)
+    if (ok[v]) {
+      W[at[v]] = x[v];
+      WHH[at[v]] = d[v];
+    }
   if constexpr (LOSS) {
-    __shared__ double red[RP / 32][3];
+    __shared__ double red[T::WAVES][3];
     const long long ticks = wall_clock64() - start;
     double* out = sums + (int64_t)blockIdx.x * 4;
-    acc4 now[2];
-    t.product(buf[n_steps & 1], now);
+    const acc4 now = t.product(buf[n_steps & 1]);
 #pragma unroll
-    for (int b = 0; b < 2; b++)
-#pragma unroll
-      for (int v = 0; v < 4; v++)
-        if (!ok[b][v]) ah[b][v] = d[b][v] = 0.0f;
+    for (int v = 0; v < 4; v++)
+      if (!ok[v]) ah[v] = d[v] = 0.0f;
     fit_sums<RP>(t, x, ah, now, d, red, out);
     if (threadIdx.x == 0) out[3] = (double)ticks;
   }
@@ -166,32 +155,29 @@ __global__ void __launch_bounds__(2 * RP)
 
 // <A H^T, W>, <W G, W> and (where WHH is given) <WHH, W> of a workgroup's rows, in fp64.
 template <int RP>
-__global__ void __launch_bounds__(2 * RP)
+__global__ void __launch_bounds__(4 * RP)
     k_fit_loss(const float* __restrict__ W, const float* __restrict__ G, const float* __restrict__ AH,
                const float* __restrict__ WHH, int64_t n, int r, double* __restrict__ partials) {
   using T = FitTile<RP>;
   __shared__ __align__(16) float buf[FIT_ROWS * T::LD];
-  __shared__ double red[RP / 32][3];
+  __shared__ double red[T::WAVES][3];
   T t;
   t.init(G, r);
   const int64_t row0 = (int64_t)blockIdx.x * FIT_ROWS;
-  float x[2][4], ah[2][4];
-  acc4 wh[2];
+  float x[4], ah[4];
+  acc4 wh;
 #pragma unroll
-  for (int b = 0; b < 2; b++)
-#pragma unroll
-    for (int v = 0; v < 4; v++) {
-      const bool ok = row0 + t.row(v) < n && t.col(b) < r;
-      const int64_t at = ok ? (row0 + t.row(v)) * r + t.col(b) : 0;
-      const float w = W[at], a = AH[at], h = WHH ? WHH[at] : 0.0f;
-      x[b][v] = ok ? w : 0.0f;
-      ah[b][v] = ok ? a : 0.0f;
-      wh[b][v] = ok ? h : 0.0f;
-      buf[t.row(v) * T::LD + t.col(b)] = x[b][v];
-    }
+  for (int v = 0; v < 4; v++) {
+    const bool ok = row0 + t.row(v) < n && t.col() < r;
+    const int64_t at = ok ? (row0 + t.row(v)) * r + t.col() : 0;
+    const float w = W[at], a = AH[at], h = WHH ? WHH[at] : 0.0f;
+    x[v] = ok ? w : 0.0f;
+    ah[v] = ok ? a : 0.0f;
+    wh[v] = ok ? h : 0.0f;
+    buf[t.row(v) * T::LD + t.col()] = x[v];
+  }
   __syncthreads();
-  acc4 d[2];
-  t.product(buf, d);
+  const acc4 d = t.product(buf);
   fit_sums<RP>(t, x, ah, d, wh, red, partials + (int64_t)blockIdx.x * 3);
 }
 
@@ -231,8 +217,8 @@ int launch_fit_steps(int64_t n, int r, float* W, const float* G, const float* AH
     const int now = n_steps - done < FIT_STEPS_MAX ? n_steps - done : FIT_STEPS_MAX;
     fit_dispatch(r, [&](auto rp) {
       constexpr int RP = decltype(rp)::value;
-      if (sums) hipLaunchKernelGGL((k_fit_steps<RP, true>), grid, dim3(2 * RP), 0, stream(), W, G, AH, eps, n, r, now, WHH, sums);
-      else hipLaunchKernelGGL((k_fit_steps<RP, false>), grid, dim3(2 * RP), 0, stream(), W, G, AH, eps, n, r, now, WHH, sums);
+      if (sums) hipLaunchKernelGGL((k_fit_steps<RP, true>), grid, dim3(4 * RP), 0, stream(), W, G, AH, eps, n, r, now, WHH, sums);
+      else hipLaunchKernelGGL((k_fit_steps<RP, false>), grid, dim3(4 * RP), 0, stream(), W, G, AH, eps, n, r, now, WHH, sums);
     });
     DN_LAUNCH_CHECK();
   }
@@ -243,7 +229,7 @@ int launch_fit_loss(int64_t n, int r, const float* W, const float* G, const floa
                     double* partials, double* out3) {
   fit_dispatch(r, [&](auto rp) {
     constexpr int RP = decltype(rp)::value;
-    hipLaunchKernelGGL(k_fit_loss<RP>, dim3((unsigned)ceil_div(n, FIT_ROWS)), dim3(2 * RP), 0, stream(), W, G, AH,
+    hipLaunchKernelGGL(k_fit_loss<RP>, dim3((unsigned)ceil_div(n, FIT_ROWS)), dim3(4 * RP), 0, stream(), W, G, AH,
                        WHH, n, r, partials);
   });
   if (out3) hipLaunchKernelGGL(k_fit_loss_sum, dim3(1), dim3(192), 0, stream(), partials, fit_loss_parts(n), out3);
