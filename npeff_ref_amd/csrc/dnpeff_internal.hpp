@@ -88,6 +88,7 @@ int host_stamps(unsigned long long** out);  // HOST_STAMPS more, for the clock a
 class pinned_buf {
  public:
   static constexpr size_t BYTES = (size_t)2 << 20;
+  static constexpr int EVENTS = 4;
   pinned_buf() = default;
   pinned_buf(const pinned_buf&) = delete;
   pinned_buf& operator=(const pinned_buf&) = delete;
@@ -98,12 +99,13 @@ class pinned_buf {
 
  private:
   char* p_ = nullptr;
-  hipEvent_t done_[2] = {};
+  hipEvent_t done_[EVENTS] = {};
   int dev_ = 0;
 };
 // Short arrays down through such a buffer: a kernel writes them side by side, each (whole words) in gather_room bytes, and
 // after a wait for the library stream they are taken from there.
 inline size_t gather_room(size_t bytes) { return (bytes + 15) / 16 * 16; }
+void fetch_pages(void* p, size_t bytes);  // of memory that the device's results go to, ahead of the copy
 hipError_t gather_queue(const copy_part* parts, int n_parts, char* buf);
 void gather_take(const copy_part* parts, int n_parts, const char* buf);
 

@@ -658,12 +658,7 @@ struct topk_down {
     }
     for (int i = 0; i <= b; i++) DN_HIP(gather_queue(of[i], n_of[i], pinned[i].p()));
     queued = true;
-    constexpr size_t PAGE = 4096;
-    for (int q = 0; q < n_parts; q++) {
-      volatile char* to = (volatile char*)parts[q].dst;
-      for (size_t at = 0; at < parts[q].bytes; at += PAGE) to[at] = 0;
-      to[parts[q].bytes - 1] = 0;
-    }
+    for (int q = 0; q < n_parts; q++) fetch_pages(parts[q].dst, parts[q].bytes);
     return 0;
   }
   void take() {
