@@ -456,6 +456,86 @@ __global__ void __launch_bounds__(256) k_topk_threshold(unsigned* __restrict__ h
     for (int i = t; i < TOPK_BINS; i += 256) h[i] = 0;
 }
 
+// Both levels of a row of few chunks by one workgroup: what five launches (the start, two histograms and their bins) else take.
+// 64 rows of 20,000: 72 -> 48 us a call, 1 of 16,000 71 -> 42, 3 of 1,000,000 (489 chunks) 73 -> 55, 40 of 700,000 86 -> 74. Past
+// 512 chunks it falls behind: 20 of 60,000 (938) 66 us against 54, 5 of 4,000,000 (1954) 174 against 147.
+constexpr int TOPK_SHORT = 512;
+__global__ void __launch_bounds__(1024)
+    k_topk_short(const float* __restrict__ x, int64_t count, int64_t stride, int64_t chunks, unsigned target,
+                 TopkRow* __restrict__ rows, int* __restrict__ buckets, int nb) {
+  static_assert(TOPK_BINS == 2 * 1024, "a thread has two bins");
+  __shared__ unsigned h[TOPK_BINS];
+  __shared__ unsigned part[16];
+  __shared__ uint32_t most[16], found_bin, found_need;
+  const int row = blockIdx.x, t = threadIdx.x, wave = t >> 6, lane = t & 63;
+  for (int i = t; i < nb; i += 1024) buckets[(int64_t)row * nb + i] = 0;
+  const float* xr = x + (int64_t)row * count;
+  uint32_t bin = 0, thr = 0, top = 0;
+  unsigned need = target;
+  for (int level = 0; level < 2; level++) {
+    h[t] = h[t + 1024] = 0;
+    __syncthreads();
+    constexpr int U = 8;
+    for (int64_t c = wave; c < chunks; c += 16 * U) {
+      float v[U];
+      bool ok[U];
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        const int64_t i = (c + 16 * u) * stride + lane;
+        ok[u] = c + 16 * u < chunks && i < count;
+        v[u] = xr[ok[u] ? i : 0];
+      }
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        const uint32_t key = sort_key(v[u]);
+        if (level) ok[u] = ok[u] && (key >> 21) == bin;
+        else top = ok[u] ? max(top, key) : top;
+        if (ok[u]) atomicAdd(&h[level ? (key >> 10) & (TOPK_BINS - 1) : key >> 21], 1u);
+      }
+    }
+    if (level == 0) {
+#pragma unroll
+      for (int off = 32; off > 0; off >>= 1) top = max(top, (uint32_t)__shfl_xor((int)top, off));
+      if (lane == 0) most[wave] = top;
+    }
+    __syncthreads();
+    // the bin from the top where the entries reach the target: thread t has bins 2047 - 2 t and the one below
+    const int first = TOPK_BINS - 1 - 2 * t;
+    const unsigned c0 = h[first], c1 = h[first - 1];
+    unsigned incl = c0 + c1;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const unsigned up = __shfl_up(incl, off);
+      if (lane >= off) incl += up;
+    }
+    if (lane == 63) part[wave] = incl;
+    __syncthreads();
+    unsigned total = 0, above = incl - (c0 + c1);
+    for (int w = 0; w < 16; w++) {
+      if (w < wave) above += part[w];
+      total += part[w];
+    }
+    if (above < need && above + c0 + c1 >= need) {
+      const int b = above + c0 < need;
+      found_bin = (uint32_t)(first - b);
+      found_need = need - above - (b ? c0 : 0u);
+    }
+    __syncthreads();
+    const bool all = total < need;  // (fewer entries than the target: everything is a candidate)
+    if (level == 0) {
+      bin = all ? 0u : found_bin;
+      need = all ? need : found_need;
+    } else {
+      thr = all ? 0u : (bin << 21) | (found_bin << 10);
+    }
+    __syncthreads();
+  }
+  if (t == 0) {
+    for (int w = 0; w < 16; w++) top = max(top, most[w]);
+    rows[row] = TopkRow{bin, thr, top, need, 0ull};
+  }
+}
+
 // Entries from the threshold up and the sum of squares.  Bound by the read of the row (2 rows of
 // 110 M: 156 us, 5.6 TB/s; a barrier and a shared buffer per 1024 entries: 200 us).
 __global__ void __launch_bounds__(256)
@@ -690,7 +770,6 @@ static int topk_by_sample(int64_t n_rows, int64_t count, int64_t k, const float*
   dbuf<double> sq;
   const dim3 gc = blocks(count, 4096);
   DN_TRY(rows.alloc(n_rows));
-  DN_TRY(hist.alloc(n_rows * TOPK_BINS));
   DN_TRY(cand.alloc(n_rows * cap));
   DN_TRY(sorted.alloc(n_rows * cap));
   DN_TRY(starts.alloc(n_rows * plan.buckets()));
@@ -699,12 +778,17 @@ static int topk_by_sample(int64_t n_rows, int64_t count, int64_t k, const float*
   unsigned long long* failed = nullptr;
   DN_TRY(host_words(&failed));
   *failed = 0;
-  hipLaunchKernelGGL(k_topk_row_init, dim3((unsigned)n_rows), dim3(1024), 0, st, rows.p, plan.target, hist.p, plan.buckets(), starts.p);
   const dim3 gs = blocks(chunks, TOPK_SAMPLE_EACH), gr((unsigned)n_rows), gp = blocks(cap, 256);
-  hipLaunchKernelGGL(k_topk_sample<0>, gs, dim3(TOPK_SAMPLE_WAVES * 64), 0, st, x, count, stride, chunks, rows.p, hist.p);
-  hipLaunchKernelGGL(k_topk_threshold<0>, gr, block, 0, st, hist.p, rows.p);
-  hipLaunchKernelGGL(k_topk_sample<1>, gs, dim3(TOPK_SAMPLE_WAVES * 64), 0, st, x, count, stride, chunks, rows.p, hist.p);
-  hipLaunchKernelGGL(k_topk_threshold<1>, gr, block, 0, st, hist.p, rows.p);
+  if (chunks <= TOPK_SHORT) {
+    hipLaunchKernelGGL(k_topk_short, gr, dim3(1024), 0, st, x, count, stride, chunks, plan.target, rows.p, starts.p, plan.buckets());
+  } else {
+    DN_TRY(hist.alloc(n_rows * TOPK_BINS));
+    hipLaunchKernelGGL(k_topk_row_init, gr, dim3(1024), 0, st, rows.p, plan.target, hist.p, plan.buckets(), starts.p);
+    hipLaunchKernelGGL(k_topk_sample<0>, gs, dim3(TOPK_SAMPLE_WAVES * 64), 0, st, x, count, stride, chunks, rows.p, hist.p);
+    hipLaunchKernelGGL(k_topk_threshold<0>, gr, block, 0, st, hist.p, rows.p);
+    hipLaunchKernelGGL(k_topk_sample<1>, gs, dim3(TOPK_SAMPLE_WAVES * 64), 0, st, x, count, stride, chunks, rows.p, hist.p);
+    hipLaunchKernelGGL(k_topk_threshold<1>, gr, block, 0, st, hist.p, rows.p);
+  }
   hipLaunchKernelGGL(k_topk_collect, gc, block, 0, st, x, count, rows.p, cand.p, cap, log_nb, above, starts.p, place.p, sq.p);
   hipLaunchKernelGGL(k_topk_bucket_scan, gr, dim3(TOPK_SCAN), 0, st, rows.p, cap, k, plan.buckets(), starts.p, sq.p, (int)gc.x,
                      norms, failed);
