@@ -2397,7 +2397,8 @@ __global__ void __launch_bounds__(256)
   for (int off = 32; off > 0; off >>= 1) t += __shfl_xor(t, off);
   if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = t;
   __syncthreads();
-  if (threadIdx.x == 0) out[blockIdx.x] = ((sh[0] + sh[1]) + sh[2]) + sh[3];
+  if (threadIdx.x == 0)
+    __hip_atomic_store(out + blockIdx.x, ((sh[0] + sh[1]) + sh[2]) + sh[3], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 DN_API int dnpeff_op_dot(int64_t count, const float* x, const float* y, double* out_host) {
@@ -2407,9 +2408,10 @@ DN_API int dnpeff_op_dot(int64_t count, const float* x, const float* y, double* 
   DN_TRY(host_words(&words));
   double* part = reinterpret_cast<double*>(words);
   const int wgs = (int)std::max<int64_t>(1, std::min<int64_t>(HOST_WORDS, ceil_div(count, 4096)));
+  std::fill(words, words + wgs, WORD_NONE);  // (no sum: a NaN that no fp32 number makes)
   hipLaunchKernelGGL(k_dot_host, dim3((unsigned)wgs), dim3(256), 0, stream(), count, x, y, part);
   DN_LAUNCH_CHECK();
-  DN_HIP(hipStreamSynchronize(stream()));
+  DN_HIP(wait_words(words, wgs, stream()));  // (with the stream 4 us more: 4 components of 6 M 270 -> 259 us)
   double sum = 0.0;
   for (int i = 0; i < wgs; i++) sum += part[i];
   *out_host = sum;

@@ -80,6 +80,10 @@ hipError_t copy_down_parts(const copy_part* parts, int n_parts);
 inline hipError_t copy_down_parts(std::initializer_list<copy_part> parts) { return copy_down_parts(parts.begin(), (int)parts.size()); }
 constexpr int HOST_WORDS = 512;
 int host_words(unsigned long long** out);  // HOST_WORDS pinned words of the calling thread
+// Words that a kernel on its way writes (at system scope; WORD_NONE before): waited for by themselves for a while, then with
+// the whole stream.  What else the kernel writes is not there yet.
+constexpr unsigned long long WORD_NONE = ~0ull;
+hipError_t wait_words(const unsigned long long* words, int n, hipStream_t st);
 constexpr int HOST_STAMPS = 2;
 int host_stamps(unsigned long long** out);  // HOST_STAMPS more, for the clock around calls that use those
 

@@ -9,7 +9,6 @@
 
 #include <algorithm>
 #include <cctype>
-#include <chrono>
 #include <cstdarg>
 #include <cstring>
 #include <memory>
@@ -545,7 +544,7 @@ __global__ void __launch_bounds__(256)
 // four: 7.9).
 constexpr int THR_KEEP = 1024;  // notes per workgroup: 8 KB of LDS, 8 MB on the device
 constexpr int THR_STEP = 2;     // tiles per step
-constexpr unsigned long long THR_FITS = 1ull << 40, THR_NONE = ~0ull;  // (no word yet)
+constexpr unsigned long long THR_FITS = 1ull << 40;
 
 template <bool VEC4, bool BY_CUT>
 __global__ void __launch_bounds__(256)
@@ -2008,17 +2007,6 @@ struct threshold_found {
     if (st) (void)hipStreamSynchronize(st);
   }
 };
-
-// A word that a kernel on its way writes to pinned memory: waited for by itself for a while, then with the whole stream.
-static hipError_t wait_word(const unsigned long long* word, hipStream_t st) {
-  const auto written = [&] { return __atomic_load_n(word, __ATOMIC_ACQUIRE) != THR_NONE; };
-  const auto until = std::chrono::steady_clock::now() + std::chrono::milliseconds(1);
-  while (!written() && std::chrono::steady_clock::now() < until) {
-  }
-  if (written()) return hipSuccess;
-  const hipError_t e = hipStreamSynchronize(st);
-  return e != hipSuccess || written() ? e : hipErrorUnknown;
-}
 }  // namespace dn
 
 DN_API int dnpeff_op_threshold_compact(int64_t count, const float* x, float divisor, float threshold,
@@ -2067,7 +2055,7 @@ DN_API int dnpeff_threshold_find(int64_t count, const float* x, float divisor, f
     DN_TRY(notes.alloc((int64_t)runs.wgs * THR_KEEP));
     unsigned long long* word = nullptr;
     DN_TRY(host_words(&word));
-    *word = THR_NONE;
+    *word = WORD_NONE;
     F->pinned.take();
     constexpr int ROOM = (int)(pinned_buf::BYTES / 8);
     hipStream_t st = F->st = stream();
@@ -2082,7 +2070,7 @@ DN_API int dnpeff_threshold_find(int64_t count, const float* x, float divisor, f
     DN_LAUNCH_CHECK();
     // (the finds are still on their way: the caller makes room for them meanwhile.  4 components of 6 M: 283 -> 277 us, a first time
     // 331 -> 309)
-    DN_HIP(wait_word(word, st));
+    DN_HIP(wait_words(word, 1, st));
     F->n = (int64_t)(*word & (THR_FITS - 1));
     F->at_hand = (*word & THR_FITS) != 0;
     if (!F->at_hand) {

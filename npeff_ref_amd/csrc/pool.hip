@@ -575,6 +575,19 @@ int host_words(unsigned long long** out) {
   *out = words;
   return 0;
 }
+hipError_t wait_words(const unsigned long long* words, int n, hipStream_t st) {
+  const auto until = std::chrono::steady_clock::now() + std::chrono::milliseconds(1);
+  int i = 0;
+  auto here = [&] {
+    while (i < n && __atomic_load_n(words + i, __ATOMIC_ACQUIRE) != WORD_NONE) i++;
+    return i == n;
+  };
+  while (!here() && std::chrono::steady_clock::now() < until) {
+  }
+  if (i == n) return hipSuccess;
+  const hipError_t e = hipStreamSynchronize(st);
+  return e != hipSuccess || here() ? e : hipErrorUnknown;
+}
 int host_stamps(unsigned long long** out) {
   DN_TRY(host_words(out));
   *out += HOST_WORDS;
