@@ -27,11 +27,10 @@ __device__ inline float bcast_f(float v, int src_lane) {
 // Gatherers: acc += sum_{p in [p0, p1)} val[p] * X[idx[p], :], then store(dst).
 // ---------------------------------------------------------------------------
 
-// Any rank: lane l holds components l + 64 t; every entry is applied by the whole wave.
-template <int VPL>
+// Any rank: lane l holds components l + 64 t; every entry is applied by the whole wave.  MANY: gather_many().
+template <int VPL, bool MANY>
 struct GatherDword {
-  // (runs of hundreds of entries are a chain of trips: A H^T of 43 x 3022, rank 55, 37 -> 30 us with twice as many in flight)
-  static constexpr int FEW = VPL <= 2 ? 8 : VPL <= 4 ? 4 : 2, UNR = 2 * FEW;
+  static constexpr int FEW = VPL <= 2 ? 8 : VPL <= 4 ? 4 : 2, UNR = MANY ? 2 * FEW : FEW;
   float acc[VPL];
   bool ok[VPL];
   int lane;
@@ -1409,9 +1408,21 @@ struct TypeTag {
   using type = T;
 };
 
+// GatherDword's steps in a launch of `wgs` workgroups that gathers from `rows` rows of `width` components: twice as many gathers of
+// a wave in flight where its chain of trips is the bound, which is where few waves have the chip or the L2s hold most of the
+// rows.  More waves than that, and rows from the fabric, and the requests only push each other's lines out.  A H^T, us, small steps /
+// large ones: 43 rows of 500 entries, 3022 columns, rank 99 40 / 37, rank 510 135 / 108; 300 rows of 2000, 300k columns, rank 250
+// 120 / 101; 1000 rows of 1000, 8000 columns, rank 250 90 / 74; past the line 700 rows of 4000, 60k columns, rank 126 106 /
+// 124, 400 rows of them, rank 250 132 / 157, rank 510 345 / 382, 2000 rows of 75, 20k columns, rank 997 71 / 82.  In workgroups
+// per CU the two meet at 3 to 4 up to 64 components, at 3 to 4 up to 128 (60k columns; 300k columns: 2), at 2 up to 512 and at 1 above.
+static bool gather_many(int width, int64_t rows, int64_t wgs) {
+  const int per_cu = width <= 64 ? 4 : width <= 128 ? 3 : width <= 512 ? 2 : 1;
+  return rows * width <= (int64_t)5 << 20 || wgs <= (int64_t)per_cu * n_cus();
+}
+
 // Calls f(TypeTag<Gatherer>) with the gatherer that fits rank r and the alignment of X.
 template <class F>
-static int dispatch_gather(int r, bool aligned16, F&& f) {
+static int dispatch_gather(int r, bool aligned16, bool many, F&& f) {
   if (r % 4 == 0 && aligned16) {
     const int r4 = r / 4;
     if (r4 == 4) return f(TypeTag<GatherVec4<4, 1, true>>{});
@@ -1429,13 +1440,17 @@ static int dispatch_gather(int r, bool aligned16, F&& f) {
     if (r4 <= 128) return f(TypeTag<GatherVec4<64, 2>>{});
     return f(TypeTag<GatherVec4<64, 4>>{});
   }
-  switch (vpl_for(r)) {
-    case 1: return f(TypeTag<GatherDword<1>>{});
-    case 2: return f(TypeTag<GatherDword<2>>{});
-    case 4: return f(TypeTag<GatherDword<4>>{});
-    case 8: return f(TypeTag<GatherDword<8>>{});
-    default: return f(TypeTag<GatherDword<16>>{});
-  }
+  auto by_width = [&](auto large) {
+    constexpr bool MANY = decltype(large)::value;
+    switch (vpl_for(r)) {
+      case 1: return f(TypeTag<GatherDword<1, MANY>>{});
+      case 2: return f(TypeTag<GatherDword<2, MANY>>{});
+      case 4: return f(TypeTag<GatherDword<4, MANY>>{});
+      case 8: return f(TypeTag<GatherDword<8, MANY>>{});
+      default: return f(TypeTag<GatherDword<16, MANY>>{});
+    }
+  };
+  return many ? by_width(std::true_type{}) : by_width(std::false_type{});
 }
 
 __global__ void k_sweep_clear(int* progress) { progress[threadIdx.x] = 0; }
@@ -1633,7 +1648,7 @@ int launch_spmm_n(const dnpeff_csr* A_full, int r, const float* H_mr, int part) 
     if (A->n_plain > 0 && (part == 0 || (part == 1) == plain_early)) {
       const int64_t row_groups = ceil_div(A->n_rows, 4);
       dim3 grid((unsigned)(row_groups * A->n_plain)), block(256);
-      dispatch_gather(r, aligned, [&](auto tag) {
+      dispatch_gather(r, aligned, gather_many(r, A->n_cols, grid.x), [&](auto tag) {
         using GT = typename decltype(tag)::type;
         hipLaunchKernelGGL((k_spmm_n_panel<GT>), grid, block, 0, stream(), A->seg, A->pcol,
                            A->pval, A->n_rows, row_groups, A->n_panels, A->panel_ids, slots, r, H_mr,
@@ -1674,7 +1689,7 @@ int launch_spmm_n(const dnpeff_csr* A_full, int r, const float* H_mr, int part) 
     return 0;
   }
   const size_t lds = sizeof(float) * 4 * (size_t)r;
-  dispatch_gather(r, ((uintptr_t)H_mr % 16) == 0, [&](auto tag) {
+  dispatch_gather(r, ((uintptr_t)H_mr % 16) == 0, gather_many(r, A->n_cols, grid.x), [&](auto tag) {
     using GT = typename decltype(tag)::type;
     hipLaunchKernelGGL((k_spmm_n<GT>), grid, block, lds, stream(), A->rowptr, A->colind, A->vals,
                        A->chunk_base, A->n_rows, r, H_mr, partials);
@@ -1844,7 +1859,7 @@ static int launch_spmm_t_sparse(const dnpeff_csr* A, int r, const float* W_nr, f
 #undef DN_GROUPED2
 #undef DN_GROUPED
   }
-  dispatch_gather(width, aligned, [&](auto tag) {
+  dispatch_gather(width, aligned, gather_many(width, A->n_rows, (l1 - l0) * n_slices), [&](auto tag) {
     using GT = typename decltype(tag)::type;
     if (!grouped)
       hipLaunchKernelGGL((k_spmm_t_short<GT>), grid, block, 0, stream(), colptr, A->rowind, A->tvals,
@@ -2059,7 +2074,7 @@ DN_API int dnpeff_op_spmm_n_variant(dnpeff_csr* A_full, int r, const float* H_mr
   if (variant == 1) {
     if (A->n_rows > 0) {
       dim3 grid((unsigned)ceil_div(A->n_rows, 4)), block(256);
-      dispatch_gather(r, aligned, [&](auto tag) {
+      dispatch_gather(r, aligned, gather_many(r, A->n_cols, grid.x), [&](auto tag) {
         using GT = typename decltype(tag)::type;
         hipLaunchKernelGGL((k_spmm_n_rowwave<GT>), grid, block, 0, stream(), A->rowptr, A->colind,
                            A->vals, A->n_rows, r, H_mr, N_nr);
@@ -2074,7 +2089,7 @@ DN_API int dnpeff_op_spmm_n_variant(dnpeff_csr* A_full, int r, const float* H_mr
       DN_TRY(carry.alloc(n_shares * 2 * (int64_t)r));
       DN_CHECK(ceil_div(n_shares, 4) < ((int64_t)1 << 24), "too many shares for one launch");
       dim3 grid((unsigned)ceil_div(n_shares, 4)), block(256);
-      dispatch_gather(r, aligned, [&](auto tag) {
+      dispatch_gather(r, aligned, gather_many(r, A->n_cols, grid.x), [&](auto tag) {
         using GT = typename decltype(tag)::type;
         hipLaunchKernelGGL((k_spmm_n_merge<GT>), grid, block, 0, stream(), A->rowptr, A->colind, A->vals,
                            A->n_rows, n_shares, r, H_mr, N_nr, carry.p);
@@ -2093,7 +2108,7 @@ DN_API int dnpeff_op_spmm_n_variant(dnpeff_csr* A_full, int r, const float* H_mr
       DN_CHECK(A->n_chunks < (int64_t)INT32_MAX, "too many work chunks");
       dim3 grid((unsigned)A->n_chunks), block(256);
       const size_t lds = sizeof(float) * 4 * (size_t)r;
-      dispatch_gather(r, ((uintptr_t)H_mr % 16) == 0, [&](auto tag) {
+      dispatch_gather(r, ((uintptr_t)H_mr % 16) == 0, gather_many(r, A->n_cols, grid.x), [&](auto tag) {
         using GT = typename decltype(tag)::type;
         hipLaunchKernelGGL((k_spmm_n<GT>), grid, block, lds, stream(), A->rowptr, A->colind, A->vals,
                            A->chunk_base, A->n_rows, r, H_mr, A->partials);

@@ -16,13 +16,17 @@ def _chain(acc, a, h):
     return (np.float64(a) * h.astype(np.float64) + acc.astype(np.float64)).astype(np.float32)
 
 
+@pytest.mark.parametrize("large", [False, True])  # on either side of the line between the two lengths of a step (gather_many)
 @pytest.mark.parametrize("r", [3, 50, 63, 126, 250, 510, 1001])
-def test_runs_of_every_length_keep_the_order_of_their_sum(r):
+def test_runs_of_every_length_keep_the_order_of_their_sum(r, large):
     lens = [0, 1, 2, 3, 4, 5, 7, 8, 9, 12, 15, 16, 17, 31, 33, 47, 48, 63, 64, 65, 79, 80, 95, 127, 128, 200]
     m = 300
+    if large:  # more than 20 MB of rows to gather from, more than four workgroups per CU
+        m = (5 << 20) // r + 1
+        lens += [0] * (4 * 4 * d.device_info()[2])
     rng = np.random.default_rng(r)
     rowptr = np.concatenate(([0], np.cumsum(lens))).astype(np.int64)
-    cols = np.concatenate([rng.permutation(m)[:n] for n in lens]).astype(np.int32)
+    cols = np.concatenate([rng.permutation(m)[:n] for n in lens if n]).astype(np.int32)
     vals = rng.random(len(cols), dtype=np.float32)
     H = rng.random((m, r), dtype=np.float32)
     A = d.Csr.from_host(rowptr, cols, vals, m)
