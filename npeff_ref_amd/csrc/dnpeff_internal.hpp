@@ -33,10 +33,12 @@ bool side_stream_pending();
 
 }  // namespace dn
 
+// (An error is reported once: hipGetLastError() would hand it to the next launch check as well.)
 #define DN_HIP(expr)                                                                 \
   do {                                                                               \
     hipError_t dn_e_ = (expr);                                                       \
     if (dn_e_ != hipSuccess) {                                                       \
+      (void)hipGetLastError();                                                       \
       dn::set_error("%s failed: %s (%s:%d)", #expr, hipGetErrorString(dn_e_), __FILE__, \
                     __LINE__);                                                       \
       return 1;                                                                      \

@@ -111,6 +111,7 @@ int device_alloc(void** out, size_t bytes, bool* reused) {
     e = hipMalloc(out, size);
   }
   if (e != hipSuccess) {
+    (void)hipGetLastError();  // (reported here: not by the next launch of whoever does without the block)
     set_error("hipMalloc of %zu bytes failed: %s", size, hipGetErrorString(e));
     return 1;
   }

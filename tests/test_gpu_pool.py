@@ -2,6 +2,7 @@
 
 import ctypes as C
 
+import numpy as np
 import pytest
 
 import npeff_ref_amd as d
@@ -34,3 +35,16 @@ def test_nothing_large_is_kept_on_a_full_device():
     assert _device_free() >= left - (64 << 20)
     fill.free()
     d.release_cached()
+
+
+def test_a_refused_allocation_is_reported_once():
+    """The next call launches kernels and succeeds, whoever asked for the memory."""
+    x = d.DeviceArray.from_numpy(np.arange(6, dtype=np.float32).reshape(3, 2))
+    with pytest.raises(d.DnpeffError, match="out of memory"):
+        d.DeviceArray((1 << 44,))
+    G = d.DeviceArray((2, 2))
+    d.binding.op_gram(x, G)
+    assert np.array_equal(G.numpy(), [[20, 26], [26, 35]])
+    with pytest.raises(d.DnpeffError, match="out of memory"):
+        d.DeviceArray((1 << 44,))
+    assert d.op_dot(x, x) == 55
