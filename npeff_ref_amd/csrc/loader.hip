@@ -2182,12 +2182,10 @@ static int transpose_by_ranges(const dnpeff_csr* A, int64_t* colptr, int32_t* ro
   dbuf<uint32_t> at;
   dbuf<int> count;
   dbuf<int64_t> base;
-  if (at.alloc((ranges + 1) * n)) {  // (no room: row by row)
+  if (at.alloc((ranges + 1) * n) || count.alloc(ranges + 1) || base.alloc(ranges + 1)) {  // (no room: row by row)
     clear_error();
     return 0;
   }
-  DN_TRY(count.alloc(ranges + 1));
-  DN_TRY(base.alloc(ranges + 1));
   const int64_t per_row = std::max<int64_t>(1, std::min<int64_t>(64, A->nnz / n / 1024));
   DN_HIP(hipMemsetAsync(count, 0, sizeof(int), st));  // (its first element: whether columns are out of order)
   hipLaunchKernelGGL(k_range_starts, dim3((unsigned)n, (unsigned)per_row), dim3(256), 0, st, A->rowptr, A->colind, n, ranges,
