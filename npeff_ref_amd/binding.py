@@ -5,6 +5,7 @@ from __future__ import annotations
 import ctypes as C
 import math
 import os
+import time
 from dataclasses import dataclass
 from typing import Callable, Optional
 
@@ -647,7 +648,9 @@ class MuNmf:
 
     def run(self, log: Callable[[str], None] = print):
         """MuNmf::run (nmf1.h:152-205): W-update, H-update; every log_every steps the loss and
-        the mean ms/step of the window, loss time excluded.  Returns [(step, loss, ms_per_step)]."""
+        the mean ms/step of the window by the device's clock, loss time excluded (include/dnpeff.h,
+        dnpeff_nmf_step_loss).  Returns [(step, loss, ms_per_step)].  Where step or computeUncachedLoss
+        is not this class's own, every window goes through them, by the host's clock."""
         if not self._initialized:
             self.initialize()
         p = self.params
@@ -659,11 +662,15 @@ class MuNmf:
                 run = min(run, p.log_every - done % p.log_every)
             done += run
             if p.log_every > 0 and done % p.log_every == 0:
-                loss, steps_ms = _f64(0), _f64(0)
-                _check(lib.dnpeff_nmf_step_loss(self._h, run, C.byref(loss), C.byref(steps_ms)))
-                ms = steps_ms.value / p.log_every
-                log(f"step {done}: {loss.value:g} [{ms:g} ms/step]")
-                history.append((done, loss.value, ms))
+                if _replaced(self, _MUNMF_OWN):
+                    ms = _timed_ms(self.step, run) / p.log_every
+                    loss = self.computeUncachedLoss()
+                else:
+                    out, steps_ms = _f64(0), _f64(0)
+                    _check(lib.dnpeff_nmf_step_loss(self._h, run, C.byref(out), C.byref(steps_ms)))
+                    loss, ms = out.value, steps_ms.value / p.log_every
+                log(f"step {done}: {loss:g} [{ms:g} ms/step]")
+                history.append((done, loss, ms))
             else:
                 self.step(run)
         sync()
@@ -769,7 +776,9 @@ class Learner:
         return a.value, b.value
 
     def Run(self, log: Callable[[str], None] = print):
-        """RunSecondStage (nmf_sparse_H.h:298-340); the first stage ran in the constructor."""
+        """RunSecondStage (nmf_sparse_H.h:298-340); the first stage was queued by the constructor.  Returns
+        [(step, reference loss, true loss, ms_per_step)]; times, and a step or losses of a subclass, as in
+        MuNmf.run."""
         if not self._initialized:
             self.initialize()
         p = self.params
@@ -782,11 +791,15 @@ class Learner:
                 run = min(run, every - done % every)
             done += run
             if every > 0 and done % every == 0:
-                ref_loss, true_loss, steps_ms = _f64(0), _f64(0), _f64(0)
-                _check(lib.dnpeff_fit_step_loss(self._h, run, C.byref(ref_loss), C.byref(true_loss), C.byref(steps_ms)))
-                ms = steps_ms.value / every
-                log(f"step {done}: {ref_loss.value:g} [{ms:g} ms/step]")
-                history.append((done, ref_loss.value, true_loss.value, ms))
+                if _replaced(self, _LEARNER_OWN):
+                    ms = _timed_ms(self.step, run) / every
+                    ref_loss, true_loss = self.losses()
+                else:
+                    ref, true, steps_ms = _f64(0), _f64(0), _f64(0)
+                    _check(lib.dnpeff_fit_step_loss(self._h, run, C.byref(ref), C.byref(true), C.byref(steps_ms)))
+                    ref_loss, true_loss, ms = ref.value, true.value, steps_ms.value / every
+                log(f"step {done}: {ref_loss:g} [{ms:g} ms/step]")
+                history.append((done, ref_loss, true_loss, ms))
             else:
                 self.step(run)
         sync()
@@ -814,3 +827,21 @@ class Learner:
             self.close()
         except Exception:
             pass
+
+
+# What run() and Run() may leave out for one call of the library that does both.
+_MUNMF_OWN = {"step": MuNmf.step, "computeUncachedLoss": MuNmf.computeUncachedLoss}
+_LEARNER_OWN = {"step": Learner.step, "losses": Learner.losses}
+
+
+def _replaced(obj, own) -> bool:
+    """Whether one of these methods is another one: of a subclass, of the object, or put into the class."""
+    return any(getattr(getattr(obj, name), "__func__", None) is not f for name, f in own.items())
+
+
+def _timed_ms(step, n_steps: int) -> float:
+    sync()
+    t0 = time.perf_counter()
+    step(n_steps)
+    sync()
+    return (time.perf_counter() - t0) * 1e3
