@@ -5,7 +5,8 @@
  * non-zero status on failure; dnpeff_last_error() then holds a message.  The
  * reference aborts the process on every error (print + bare `throw;`,
  * cc/cuda_d_npeff/src/cuda/cuda_statuses.h:15-38); hosts that want that
- * behaviour turn a non-zero status into message + abort.
+ * behaviour turn a non-zero status into message + abort.  After a non-zero status
+ * the contents of a call's outputs are undefined: a part of a copy may have arrived.
  *
  * Storage conventions
  *   - A is CSR with 64-bit row offsets and 32-bit column ids.

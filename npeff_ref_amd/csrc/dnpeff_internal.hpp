@@ -111,7 +111,6 @@ class pinned_buf {
 // Short arrays down through such a buffer: a kernel writes them side by side, each (whole words) in gather_room bytes, and
 // after a wait for the library stream they are taken from there.
 inline size_t gather_room(size_t bytes) { return (bytes + 15) / 16 * 16; }
-void fetch_pages(void* p, size_t bytes);  // of memory that the device's results go to, ahead of the copy
 hipError_t gather_queue(const copy_part* parts, int n_parts, char* buf);
 void gather_take(const copy_part* parts, int n_parts, const char* buf);
 

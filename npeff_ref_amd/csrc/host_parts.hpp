@@ -1,6 +1,7 @@
 // Parts of the copies between host and device that need no GPU.
 #pragma once
 
+#include <cstddef>
 #include <map>
 #include <mutex>
 #include <thread>
@@ -23,6 +24,17 @@ void run_shares(int n, Work&& work, Spawn&& spawn) {
   work(0);
   for (int t = made; t < n; t++) work(t);
   for (int t = 1; t < made; t++) helpers[t].join();
+}
+
+// The pages of memory that a copy is about to write: fetched while the piece is on its way, not by the copy.  Into new arrays,
+// 131 MB: 3.4 -> 2.9 ms, 16 MB 0.83 -> 0.53, 3 MB 0.74 -> 0.51, 512 KB 120 -> 97 us; into memory that is there, the same.
+// What the memory holds stays: the copy may still fail.  (A byte of each page is written as it is, in one instruction: a load of its own
+// would map the page of zeros first, and the compiler makes a load of an atomic that changes nothing.)
+inline void fetch_pages(void* p, std::size_t bytes) {
+  constexpr std::size_t PAGE = 4096;
+  char* to = static_cast<char*>(p);
+  for (std::size_t at = 0; at < bytes; at += PAGE) asm volatile("lock orb $0, %0" : "+m"(to[at]));
+  if (bytes) asm volatile("lock orb $0, %0" : "+m"(to[bytes - 1]));
 }
 
 // Objects that wait for their next use on the device they belong to.

@@ -2,6 +2,7 @@
 // column retention, transposed CSR, ||A||^2.  Integer results are bit-exact
 // with the reference's host code; see include/dnpeff.h for the citations.
 #include "dnpeff_internal.hpp"
+#include "host_parts.hpp"
 #include "scan.hpp"
 
 #include <cmath>

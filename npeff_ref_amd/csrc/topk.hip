@@ -22,6 +22,7 @@
 // predicate scan) are the candidates.  Everything but the norm is integer work; nothing depends on
 // scheduling.
 #include "dnpeff_internal.hpp"
+#include "host_parts.hpp"
 #include "scan.hpp"
 #include "topk_buckets.hpp"
 

@@ -58,3 +58,28 @@ int main() {
   CHECK(!idle.take(0, &x));
 }
 """)
+
+
+@pytest.mark.parametrize("first, n", [(0, 1), (0, 4096), (1, 4096), (4095, 2), (17, 8192), (5000, 100_000), (4096, 0)])
+def test_fetched_pages_are_there_and_hold_what_they_held(tmp_path, first, n):
+    _run(tmp_path, """
+#include <cstring>
+#include <sys/mman.h>
+int main() {
+  const size_t first = %d, n = %d, page = 4096, pages = 40;
+  char* p = (char*)mmap(nullptr, pages * page, PROT_READ | PROT_WRITE, MAP_PRIVATE | MAP_ANONYMOUS, -1, 0);
+  CHECK(p != (char*)MAP_FAILED);
+  madvise(p, pages * page, MADV_NOHUGEPAGE);
+  dn::fetch_pages(p + first, n);
+  unsigned char there[pages];
+  CHECK(mincore(p, pages * page, there) == 0);
+  for (size_t q = 0; q < pages; q++) {
+    const bool of_range = n && q >= first / page && q <= (first + n - 1) / page;
+    CHECK((there[q] & 1) == of_range);
+  }
+  for (size_t i = 0; i < pages * page; i++) CHECK(p[i] == 0);
+  for (size_t i = 0; i < pages * page; i++) p[i] = (char)(i * 31 + 7);
+  dn::fetch_pages(p + first, n);
+  for (size_t i = 0; i < pages * page; i++) CHECK(p[i] == (char)(i * 31 + 7));
+}
+""" % (first, n))
