@@ -308,20 +308,8 @@ class DeviceArray:
             pass
 
 
-class _Scratch:
-    """A device buffer for results of one call that only the library writes (no waits)."""
-
-    def __init__(self, nbytes: int):
-        self.ptr = C.c_void_p()
-        _check(lib.dnpeff_scratch_malloc(nbytes, C.byref(self.ptr)))
-
-    def __del__(self):
-        if self.ptr:
-            lib.dnpeff_scratch_free(self.ptr)
-
-
 def _scratch_numpy(*parts):
-    """The first elements of several scratch buffers, [(buffer, shape, dtype)], in one download."""
+    """The first elements of several device buffers, [(buffer with its ptr, shape, dtype)], in one download."""
     out = [np.empty(shape, dtype=dtype) for _, shape, dtype in parts]
     n = len(parts)
     _check(

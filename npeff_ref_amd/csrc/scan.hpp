@@ -93,8 +93,6 @@ __global__ void __launch_bounds__(SCAN_BLOCK)
   }
 }
 
-static __global__ void k_set_one_i64(int64_t* p, int64_t v) { *p = v; }
-
 // The stream is not waited for.  total (or NULL): a pinned word for the sum of all.
 template <class F, class OutT>
 static int exclusive_scan(F f, int64_t n, OutT* out, int64_t* total = nullptr) {
