@@ -333,7 +333,11 @@ int dnpeff_nmf_update_H(dnpeff_nmf* nmf);
  * device_contexts1.h:337-354) through the same trace identity. */
 int dnpeff_nmf_loss(dnpeff_nmf* nmf, double* out);
 /* dnpeff_nmf_step and dnpeff_nmf_loss of what it leaves, in one call, and in *steps_ms the time of the
- * steps alone, by the device's clock (the figure that nmf1.h:186-200 logs). */
+ * steps alone, by the device's clock: from a stamp queued before them to one behind them, with the launches and
+ * the host's work in between.  Where steps and loss are one launch (runs in one workgroup, up to 1024 steps;
+ * dnpeff_fit_step_loss up to 2048 examples, 256 components and 256 steps) it is the time that the slowest
+ * workgroup spends on them inside it, without the launch.  The reference (nmf1.h:186-200) and the executables
+ * log the host's clock around the steps and a wait, which is more by launch and wait: 5 to 20 us a window. */
 int dnpeff_nmf_step_loss(dnpeff_nmf* nmf, int n_steps, double* loss, double* steps_ms);
 
 /* The three terms of the loss: ||A||^2, <H,(W^T W)H>, <W^T A,H>. */
@@ -398,7 +402,8 @@ int dnpeff_nmf_destroy(dnpeff_nmf* nmf);
 /* Stage 1: H H^T (r x r) and A H^T (n x r) from sparse A [n, m] and sparse H
  * [r, m], plus ||A||^2.  Replaces Learner::RunFirstStage
  * (cc/cuda_d_npeff/src/nmf/sparse2/nmf_sparse_H.h:157-292;
- * cuda/ops/spsp_matmul.h:95-131).  A and H may be destroyed afterwards. */
+ * cuda/ops/spsp_matmul.h:95-131).  A and H may be destroyed afterwards.  Returns without waiting for
+ * the kernels of the products: should they fail, the next call that waits reports it. */
 int dnpeff_fit_create(dnpeff_csr* A, dnpeff_csr* H, float eps, int64_t seed, dnpeff_fit** out);
 
 /* W ~ U[0,1) from the seed / caller-chosen W [n, r] row-major. */

@@ -301,7 +301,7 @@ __device__ inline void fu_gram_out(const V& v, float* __restrict__ lds, float* _
 //
 // Which shares left a carry for a column (fu_cut_by) one thread per column finds before the entries are gathered, not every
 // lane that updates a part of it: two quotients a lane were up to a tenth of the vector instructions (ten iterations at
-// 512 x 431k, r = 16: 567 -> 558 us, 777 x 862k, r = 50: 2805 -> 2786, a job at 300 x 146k, r = 20: 4.33 -> 4.21 ms.  At
+// 512 x 431k, r = 16: 561 -> 554 us, 777 x 862k, r = 50: 2801 -> 2781, a job at 300 x 146k, r = 20: 4.26 -> 4.19 ms.  At
 // ranks above 64 the kernel has no two registers for it: 27.4 -> 27.6 ms at 1000 x 3.4M, r = 128).
 // ---------------------------------------------------------------------------
 template <int Q, int R, int JB, bool TOTALS, bool PAST>

@@ -1181,8 +1181,8 @@ __global__ void __launch_bounds__(256)
 // adds them one after the other in lane order, the same way in every run.  The sums are fp64 because
 // ds_add_f64 takes 9 / 13 / 23 cycles of a CU for 16 / 32 / 64 lanes at random components where ds_add_f32
 // takes 2.7 per lane (43 / 85 / 170): with fp32 sums the LDS was taken 98 % of the time.
-// Bound by the random sectors that miss the L2s: A H^T of 65.5 M entries with 256 x 22M at 1 % takes
-// 0.88 ms, 50 M sectors of 64 bytes at 3.5 TB/s (1.60 with four pairs per slot, whose second half was read
+// Bound by the random lines that miss the L2s: A H^T of 65.5 M entries with 256 x 22M at 1 % takes
+// 0.88 ms, 49 M lines of 128 bytes at 7.2 TB/s (1.60 with four pairs per slot, whose second half was read
 // only where it was needed, one round trip later).
 //
 // H H^T (CUTS) has an order to use: rows that hold their columns in ascending order are cut at the same
@@ -1191,7 +1191,8 @@ __global__ void __launch_bounds__(256)
 // in its L2.  Only components from the row's own up are added, its own in a register (every lane meets
 // there).  256 rows of 220 k entries, 22M columns: 0.56 ms with 14 M misses (1.07 with 61 M when the rows ran
 // side by side in chunks of equal length on all XCDs, which is what `across` still does for rows in
-// another order or of uneven parts); what is left is the L2s' line rate and the rest of long columns.
+// another order or of uneven parts); what is left is trips to the L2s (80 % hits; the L1s wait for them 71 % of the
+// cycles, the L2s' channels take 0.43 requests a cycle, LDS is active for 20 %) and the rest of long columns.
 // ---------------------------------------------------------------------------
 constexpr int SPSP_PAIRS = 6;
 constexpr int SPSP_XCDS = 8;
@@ -1332,7 +1333,7 @@ __global__ void __launch_bounds__(256)
     j = colind[at];
     a = vals[at];
   };
-  // CUTS, where the L2s hold the slots and their line rate is the bound: two lanes ask for a slot together, half each,
+  // CUTS, where the L2s hold the slots and the L1s' trips to them are the bound: two lanes ask for a slot together, half each,
   // first the even one's and then the odd one's, and change halves when they are there.  (Half the lines per instruction:
   // H H^T 618 -> 559 us; A H^T, whose slots are not in the L2s, 882 -> 922.)
   const bool odd = lane & 1;

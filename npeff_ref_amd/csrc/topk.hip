@@ -538,7 +538,7 @@ __global__ void __launch_bounds__(1024)
 }
 
 // Entries from the threshold up and the sum of squares.  Bound by the read of the row (2 rows of
-// 110 M: 156 us, 5.6 TB/s; a barrier and a shared buffer per 1024 entries: 200 us).
+// 110 M: 145 to 154 us, 5.7 to 6.1 TB/s; a barrier and a shared buffer per 1024 entries: 200 us).
 __global__ void __launch_bounds__(256)
     k_topk_collect(const float* __restrict__ x, int64_t count, TopkRow* __restrict__ rows, uint64_t* __restrict__ cand,
                    int64_t cap, int log_nb, int above, int* __restrict__ buckets, unsigned* __restrict__ place,
