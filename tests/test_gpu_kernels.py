@@ -569,7 +569,7 @@ def test_threshold_compact_bit_exact(n, div, thr):
     (1, 1.0, 0), (3, 0.0, 0), (4095, 0.5, 1), (4 * 1024 * 1024 + 1029, 0.02, 0), (4 * 1024 * 1024 + 1029, 0.02, 3),
     (262144, 1.0, 0),       # the last that the pinned buffer holds: 256 runs, 1024 finds each
     (262145, 1.0, 0),       # one more
-    (9_000_000, 0.001, 0),  # runs of nine tiles: two steps of four and one tile over
+    (9_000_000, 0.001, 0),  # runs of nine tiles: four steps of two and one tile over
     (9_000_000, -1.0, 0),   # all finds in few runs: more than a run's notes, less than the buffer
     (2_500_000, 0.3, 0),    # more than the buffer, staged down
 ])
