@@ -2405,7 +2405,7 @@ DN_API int dnpeff_op_dot(int64_t count, const float* x, const float* y, double* 
   clear_error();
   DN_CHECK(out_host != nullptr, "out is NULL");
   unsigned long long* words = nullptr;
-  DN_TRY(host_words(&words));
+  DN_TRY(host_waited_words(&words));
   double* part = reinterpret_cast<double*>(words);
   const int wgs = (int)std::max<int64_t>(1, std::min<int64_t>(HOST_WORDS, ceil_div(count, 4096)));
   std::fill(words, words + wgs, WORD_NONE);  // (no sum: a NaN that no fp32 number makes)

@@ -85,6 +85,9 @@ int host_words(unsigned long long** out);  // HOST_WORDS pinned words of the cal
 // Words that a kernel on its way writes (at system scope; WORD_NONE before): waited for by themselves for a while, then with
 // the whole stream.  What else the kernel writes is not there yet.
 constexpr unsigned long long WORD_NONE = ~0ull;
+// HOST_WORDS more, for these alone: a call that gave up (for want of memory, say) may have left a kernel behind that still writes to
+// the others, in the stream's order but not in that of the host, which marks these before its launch.
+int host_waited_words(unsigned long long** out);
 hipError_t wait_words(const unsigned long long* words, int n, hipStream_t st);
 constexpr int HOST_STAMPS = 2;
 int host_stamps(unsigned long long** out);  // HOST_STAMPS more, for the clock around calls that use those

@@ -2055,7 +2055,7 @@ DN_API int dnpeff_threshold_find(int64_t count, const float* x, float divisor, f
     DN_TRY(counts.alloc(runs.wgs));
     DN_TRY(notes.alloc((int64_t)runs.wgs * THR_KEEP));
     unsigned long long* word = nullptr;
-    DN_TRY(host_words(&word));
+    DN_TRY(host_waited_words(&word));
     *word = WORD_NONE;
     F->pinned.take();
     constexpr int ROOM = (int)(pinned_buf::BYTES / 8);

@@ -562,9 +562,14 @@ hipError_t copy_down(void* dst_host, const void* src_dev, size_t bytes) {
 int host_words(unsigned long long** out) {
   static thread_local unsigned long long* words = nullptr;
   if (!words) {
-    DN_HIP(hipHostMalloc((void**)&words, (HOST_WORDS + HOST_STAMPS) * sizeof(unsigned long long), hipHostMallocDefault));
+    DN_HIP(hipHostMalloc((void**)&words, (2 * HOST_WORDS + HOST_STAMPS) * sizeof(unsigned long long), hipHostMallocDefault));
   }
   *out = words;
+  return 0;
+}
+int host_waited_words(unsigned long long** out) {
+  DN_TRY(host_words(out));
+  *out += HOST_WORDS;
   return 0;
 }
 hipError_t wait_words(const unsigned long long* words, int n, hipStream_t st) {
@@ -582,7 +587,7 @@ hipError_t wait_words(const unsigned long long* words, int n, hipStream_t st) {
 }
 int host_stamps(unsigned long long** out) {
   DN_TRY(host_words(out));
-  *out += HOST_WORDS;
+  *out += 2 * HOST_WORDS;
   return 0;
 }
 
