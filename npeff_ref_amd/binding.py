@@ -642,6 +642,9 @@ class MuNmf:
         if not self._initialized:
             self.initialize()
         p = self.params
+        # (not those of a subclass, of the object, or put into the class)
+        cls, of_self = type(self), self.__dict__
+        own = (cls.step, cls.computeUncachedLoss) == _MUNMF_OWN and "step" not in of_self and "computeUncachedLoss" not in of_self
         history = []
         done = 0
         while done < p.max_iters:  # the steps up to the next logged one in one call
@@ -650,7 +653,7 @@ class MuNmf:
                 run = min(run, p.log_every - done % p.log_every)
             done += run
             if p.log_every > 0 and done % p.log_every == 0:
-                if _replaced(self, _MUNMF_OWN):
+                if not own:
                     ms = _timed_ms(self.step, run) / p.log_every
                     loss = self.computeUncachedLoss()
                 else:
@@ -770,6 +773,8 @@ class Learner:
         if not self._initialized:
             self.initialize()
         p = self.params
+        cls, of_self = type(self), self.__dict__
+        own = (cls.step, cls.losses) == _LEARNER_OWN and "step" not in of_self and "losses" not in of_self
         history = []
         every = p.log_every_n_steps
         done = 0
@@ -779,7 +784,7 @@ class Learner:
                 run = min(run, every - done % every)
             done += run
             if every > 0 and done % every == 0:
-                if _replaced(self, _LEARNER_OWN):
+                if not own:
                     ms = _timed_ms(self.step, run) / every
                     ref_loss, true_loss = self.losses()
                 else:
@@ -818,13 +823,8 @@ class Learner:
 
 
 # What run() and Run() may leave out for one call of the library that does both.
-_MUNMF_OWN = {"step": MuNmf.step, "computeUncachedLoss": MuNmf.computeUncachedLoss}
-_LEARNER_OWN = {"step": Learner.step, "losses": Learner.losses}
-
-
-def _replaced(obj, own) -> bool:
-    """Whether one of these methods is another one: of a subclass, of the object, or put into the class."""
-    return any(getattr(getattr(obj, name), "__func__", None) is not f for name, f in own.items())
+_MUNMF_OWN = MuNmf.step, MuNmf.computeUncachedLoss
+_LEARNER_OWN = Learner.step, Learner.losses
 
 
 def _timed_ms(step, n_steps: int) -> float:

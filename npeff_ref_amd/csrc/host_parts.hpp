@@ -33,8 +33,8 @@ void run_shares(int n, Work&& work, Spawn&& spawn) {
 inline void fetch_pages(void* p, std::size_t bytes) {
   constexpr std::size_t PAGE = 4096;
   char* to = static_cast<char*>(p);
-  for (std::size_t at = 0; at < bytes; at += PAGE) asm volatile("lock orb $0, %0" : "+m"(to[at]));
-  if (bytes) asm volatile("lock orb $0, %0" : "+m"(to[bytes - 1]));
+  for (std::size_t at = 0; at < bytes; at += PAGE) asm volatile("orb $0, %0" : "+m"(to[at]));
+  if (bytes) asm volatile("orb $0, %0" : "+m"(to[bytes - 1]));
 }
 
 // Objects that wait for their next use on the device they belong to.
