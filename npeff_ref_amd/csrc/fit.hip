@@ -27,8 +27,8 @@ constexpr int FIT_ROWS = 16;
 // A step is a chain (matrix instructions, division, LDS, barrier), so that half as many columns per wave, on twice as many
 // waves, make it shorter where few waves have the chip: 25 steps and the loss at 100 x 20, the whole fit, 61 -> 54 us, 489 x
 // 64 102 -> 90, 200 x 128 96 -> 91, 2000 x 256 (bound by the matrix cores) 265 -> 264.  One step of many rows: 50,000 x 50 5.0 -> 4.6
-// us, x 128 14.6 -> 14.4, x 180 42.9 -> 32.9, x 256 54.4 -> 54.6; ranks 65 to 96, whose six waves leave two SIMDs with one
-// each, 10.2 -> 10.6 (20,000 rows 4.2 -> 4.4, 4000 1.33 -> 1.24).
+// us, x 128 14.6 -> 14.4, x 180 42.9 -> 32.9, x 256 54.4 -> 54.6; 50,000 x 90 (six waves for three) 10.2 -> 10.6, 20,000
+// rows 4.2 -> 4.4, 4000 1.33 -> 1.24.
 template <int RP>
 struct FitTile {
   static constexpr int LD = RP + 4;  // floats per row of X in LDS
